@@ -443,7 +443,13 @@ static bool fast_path_enabled() {
 
 // products go to the direct-to-LDS kernel of their element type when their shape allows it
 template <typename T, bool A_KS, bool B_KS, bool WG, int EPI>
-static int run_gemm(const GemmArgs &g, int max_rows, int tiles_generic, hipStream_t st, int kid) {
+static int run_gemm(const GemmArgs &g, int max_rows, int tiles_generic, hipStream_t st, int kid, void *ws = nullptr, size_t ws_bytes = 0) {
+    if constexpr (!WG && !A_KS) {
+        if (fast_path_enabled()) {
+            const int rc = launch_gemm_skinny(g, sizeof(T) == 2 ? MOLE_BF16 : MOLE_F32, B_KS, EPI, max_rows, ws, ws_bytes, st, kid);
+            if (rc != -100) return rc;
+        }
+    }
     if constexpr (sizeof(T) == 2) {
         if (fast_path_enabled()) {
             const int rc = launch_gemm256(g, A_KS, B_KS, WG, EPI, max_rows, st, kid);
@@ -464,7 +470,7 @@ static int run_gemm(const GemmArgs &g, int max_rows, int tiles_generic, hipStrea
 template <typename T>
 static int ffn_fwd_t(const void *xd, const int32_t *offsets, const int32_t *kept, int E, int max_rows, int M, int F,
                      const void *w1, const void *b1, const void *w2, const void *b2, void *h, void *a, void *out,
-                     hipStream_t st) {
+                     void *ws, size_t ws_bytes, hipStream_t st) {
     const int m_tiles = max_rows / TBM + E;  // every expert may end in a partial tile
     GemmArgs g{};
     g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles;
@@ -475,14 +481,14 @@ static int ffn_fwd_t(const void *xd, const int32_t *offsets, const int32_t *kept
     // out = a . w2 + b2   (w2 [F,M]: K-strided)
     g.A = a; g.lda = F; g.B = w2; g.ldb = M; g.strideB = (long)F * M; g.N = M; g.K = F;
     g.C = out; g.C2 = nullptr; g.ldc = M; g.bias = b2;
-    return run_gemm<T, false, true, false, EPI_BIAS>(g, max_rows, m_tiles * ceil_div(M, TBN), st, MOLE_K_FFN_FWD2);
+    return run_gemm<T, false, true, false, EPI_BIAS>(g, max_rows, m_tiles * ceil_div(M, TBN), st, MOLE_K_FFN_FWD2, ws, ws_bytes);
 }
 
 template <typename T>
 static int ffn_bwd_t(const void *go, const void *xd, const void *h, const void *a, const int32_t *offsets,
                      const int32_t *kept, int E, int max_rows, int M, int F, const void *w1, const void *w2, void *t,
                      void *g_w1, void *g_b1, void *g_w2, void *g_b2, void *gx, int accumulate, int gelu_bwd,
-                     hipStream_t st) {
+                     void *ws, size_t ws_bytes, hipStream_t st) {
     const int m_tiles = max_rows / TBM + E;
     GemmArgs g{};
     g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles;
@@ -523,7 +529,7 @@ static int ffn_bwd_t(const void *go, const void *xd, const void *h, const void *
     // gx = t . w1                  (w1 [F,M]: K = F strided)
     if (gx != nullptr) {
         g.A = t; g.lda = F; g.B = w1; g.ldb = M; g.strideB = (long)F * M; g.N = M; g.K = F; g.C = gx; g.ldc = M;
-        if (int rc = run_gemm<T, false, true, false, EPI_STORE>(g, max_rows, m_tiles * ceil_div(M, TBN), st, MOLE_K_FFN_GX)) return rc;
+        if (int rc = run_gemm<T, false, true, false, EPI_STORE>(g, max_rows, m_tiles * ceil_div(M, TBN), st, MOLE_K_FFN_GX, ws, ws_bytes)) return rc;
     }
     return 0;
 }
@@ -541,33 +547,56 @@ static bool al16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 using namespace mole;
 
-extern "C" int mole_ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
-                            int max_rows, int M, int F, const void *w1, const void *b1, const void *w2, const void *b2,
-                            void *h, void *a, void *out, mole_stream_t stream) {
+extern "C" size_t mole_ffn_workspace_bytes(int dtype, int E, int max_rows, int M, int F) {
+    if (E <= 0 || max_rows <= 0 || M <= 0 || F <= 0) return 0;
+    return gemm_skinny_workspace_bytes(E, max_rows, M, F, dtype);
+}
+
+extern "C" int mole_ffn_fwd_ws(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
+                               int max_rows, int M, int F, const void *w1, const void *b1, const void *w2, const void *b2,
+                               void *h, void *a, void *out, void *workspace, size_t workspace_bytes, mole_stream_t stream) {
     if (int rc = check_ffn("mole_ffn_fwd", dtype, E, max_rows, M, F)) return rc;
     if (max_rows == 0) return 0;
     MOLE_REQUIRE(xd && offsets && kept_rows && w1 && b1 && w2 && b2 && h && a && out, "mole_ffn_fwd: null pointer");
-    MOLE_REQUIRE(al16(xd) && al16(w1) && al16(w2) && al16(h) && al16(a) && al16(out), "mole_ffn_fwd: buffers must be 16-byte aligned");
+    MOLE_REQUIRE(al16(xd) && al16(w1) && al16(w2) && al16(h) && al16(a) && al16(out) && al16(workspace),
+                 "mole_ffn_fwd: buffers must be 16-byte aligned");
     if (dtype == MOLE_BF16)
-        return ffn_fwd_t<bf16_t>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, (hipStream_t)stream);
-    return ffn_fwd_t<float>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, (hipStream_t)stream);
+        return ffn_fwd_t<bf16_t>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes,
+                                 (hipStream_t)stream);
+    return ffn_fwd_t<float>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes,
+                            (hipStream_t)stream);
+}
+
+extern "C" int mole_ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
+                            int max_rows, int M, int F, const void *w1, const void *b1, const void *w2, const void *b2,
+                            void *h, void *a, void *out, mole_stream_t stream) {
+    return mole_ffn_fwd_ws(xd, dtype, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, nullptr, 0, stream);
+}
+
+extern "C" int mole_ffn_bwd_ws(const void *go, const void *xd, const void *h, const void *a, int dtype,
+                               const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, int M, int F,
+                               const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2, void *g_b2,
+                               void *gx, int accumulate, int gelu_bwd, void *workspace, size_t workspace_bytes,
+                               mole_stream_t stream) {
+    if (int rc = check_ffn("mole_ffn_bwd", dtype, E, max_rows, M, F)) return rc;
+    MOLE_REQUIRE(gelu_bwd == MOLE_GELU_BWD_TANH || gelu_bwd == MOLE_GELU_BWD_EXACT, "mole_ffn_bwd: bad gelu_bwd %d", gelu_bwd);
+    MOLE_REQUIRE(offsets && kept_rows && w1 && w2 && g_w1 && g_b1 && g_w2 && g_b2, "mole_ffn_bwd: null pointer");
+    MOLE_REQUIRE(max_rows == 0 || (go && xd && h && a && t), "mole_ffn_bwd: null activation pointer");
+    MOLE_REQUIRE(al16(go) && al16(xd) && al16(h) && al16(a) && al16(t) && al16(w1) && al16(w2) && al16(gx) && al16(workspace),
+                 "mole_ffn_bwd: buffers must be 16-byte aligned");
+    if (dtype == MOLE_BF16)
+        return ffn_bwd_t<bf16_t>(go, xd, h, a, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2,
+                                 gx, accumulate, gelu_bwd, workspace, workspace_bytes, (hipStream_t)stream);
+    return ffn_bwd_t<float>(go, xd, h, a, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx,
+                            accumulate, gelu_bwd, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 extern "C" int mole_ffn_bwd(const void *go, const void *xd, const void *h, const void *a, int dtype,
                             const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, int M, int F,
                             const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2, void *g_b2,
                             void *gx, int accumulate, int gelu_bwd, mole_stream_t stream) {
-    if (int rc = check_ffn("mole_ffn_bwd", dtype, E, max_rows, M, F)) return rc;
-    MOLE_REQUIRE(gelu_bwd == MOLE_GELU_BWD_TANH || gelu_bwd == MOLE_GELU_BWD_EXACT, "mole_ffn_bwd: bad gelu_bwd %d", gelu_bwd);
-    MOLE_REQUIRE(offsets && kept_rows && w1 && w2 && g_w1 && g_b1 && g_w2 && g_b2, "mole_ffn_bwd: null pointer");
-    MOLE_REQUIRE(max_rows == 0 || (go && xd && h && a && t), "mole_ffn_bwd: null activation pointer");
-    MOLE_REQUIRE(al16(go) && al16(xd) && al16(h) && al16(a) && al16(t) && al16(w1) && al16(w2) && al16(gx),
-                 "mole_ffn_bwd: buffers must be 16-byte aligned");
-    if (dtype == MOLE_BF16)
-        return ffn_bwd_t<bf16_t>(go, xd, h, a, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2,
-                                 gx, accumulate, gelu_bwd, (hipStream_t)stream);
-    return ffn_bwd_t<float>(go, xd, h, a, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx,
-                            accumulate, gelu_bwd, (hipStream_t)stream);
+    return mole_ffn_bwd_ws(go, xd, h, a, dtype, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx,
+                           accumulate, gelu_bwd, nullptr, 0, stream);
 }
 
 extern "C" int mole_gemm_nt(const void *a, const void *b, int dtype, int rows, int N, int K, float *c,

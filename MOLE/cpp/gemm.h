@@ -60,6 +60,64 @@ __device__ __forceinline__ float d_gelu_exact(float x) {
     return cdf + x * e * 0.39894228040143267794f;
 }
 
+// ---- activation math for a bf16 result -----------------------------------------------------------
+// On this chip every VALU instruction of an epilogue takes issue time from the MFMAs of the wave that
+// shares its SIMD, and exp / rcp run at a quarter of the plain rate, so the three functions are evaluated
+// as clamped odd polynomials: f(x) = v q(v^2), v = clamp(x / c, -1, 1), fitted (near-minimax, Lawson
+// iteration) to erf(x / sqrt 2) and to the odd parts of the two GELU derivatives.  Beyond the clamp the
+// functions are constant to within the stated error.  Absolute errors in fp32 Horner evaluation:
+// erf 5.8e-5, derivatives 1.8e-4 - an order of magnitude below the bf16 rounding of the result.
+// gelu(x) = x (1/2 + 1/2 erf(x / sqrt 2)).  The fit of erf(x / sqrt 2) is v q(v^2) in v = clamp(x / 4, -1, 1); with every
+// coefficient scaled by a power of two (c_k / (8 * 16^k): exact in binary floating point, the Horner steps round as
+// before) the same polynomial is evaluated in v = clamp(x, -4, 4) itself and delivers 1/2 erf directly:
+// clamp, square, eight FMAs, one FMA for the 1/2 and the product with x - twelve instructions, no scaling of x, no
+// separate x / 2.  Beyond the clamp erf is +-1 to within the fit's error, so x (1/2 +- 1/2) is x or 0 as it should be.
+__device__ __forceinline__ float fast_gelu_erf(float x) {
+    constexpr float c[9] = {3.19138169f / 8.0f,
+                            -8.50055408f / (8.0f * 16.0f),
+                            20.229044f / (8.0f * 256.0f),
+                            -37.1561737f / (8.0f * 4096.0f),
+                            51.8556824f / (8.0f * 65536.0f),
+                            -52.8050575f / (8.0f * 1048576.0f),
+                            36.4542885f / (8.0f * 16777216.0f),
+                            -15.039053f / (8.0f * 268435456.0f),
+                            2.77038407f / (8.0f * 4294967296.0f)};
+    const float v = __builtin_amdgcn_fmed3f(x, -4.0f, 4.0f);
+    const float t = v * v;
+    float q = c[8];
+#pragma unroll
+    for (int k = 7; k >= 0; --k) q = fmaf(q, t, c[k]);
+    return x * fmaf(v, q, 0.5f);
+}
+// The two GELU derivatives share the clamp (4.5) and the degree, so the variant is a choice of coefficients,
+// made once per tile, not a branch per element: tanh form = what the reference's backward multiplies by
+// (MOLE/cpp/gelu.cu:3-14), exact form = Phi(x) + x phi(x).  d(x) = 1/2 + v q(v^2), v = clamp(x / 4.5, -1, 1); as above
+// the polynomial is evaluated in v = clamp(x, -4.5, 4.5) with the coefficients divided by 4.5^(2k+1) (in double
+// precision, then rounded once: 4.5 is not a power of two).
+struct DGeluCoef {
+    float c[10];
+    __device__ __forceinline__ void select(bool tanh_form) {
+        constexpr double ct[10] = {3.58895016, -24.237009, 110.279869, -345.395355, 772.538513,
+                                   -1226.4845, 1338.11902, -946.521179, 388.703674, -70.0920258};
+        constexpr double ce[10] = {3.58931732, -24.1413288, 108.150215, -329.418243, 711.674683,
+                                   -1091.27979, 1154.8053, -796.700195, 320.776367, -56.9563408};
+        double s = 1.0 / 4.5;
+#pragma unroll
+        for (int i = 0; i < 10; ++i) {
+            c[i] = (float)((tanh_form ? ct[i] : ce[i]) * s);
+            s *= 1.0 / (4.5 * 4.5);
+        }
+    }
+    __device__ __forceinline__ float operator()(float x) const {
+        const float v = __builtin_amdgcn_fmed3f(x, -4.5f, 4.5f);
+        const float t = v * v;
+        float q = c[9];
+#pragma unroll
+        for (int k = 8; k >= 0; --k) q = fmaf(q, t, c[k]);
+        return fmaf(v, q, 0.5f);
+    }
+};
+
 enum { EPI_STORE = 0, EPI_BIAS = 1, EPI_BIAS_GELU = 2, EPI_DGELU = 3, EPI_WGRAD = 4, EPI_F32 = 5,
        EPI_NONE = 6 /* measurement only: the K loop runs, nothing is stored; EPI_NONE + 1..4: the K loop without
                        its operand loads / its fragment reads / its barriers / all three */ };
@@ -86,6 +144,9 @@ struct GemmArgs {
     int colsum_side;        //   over the expert's rows: 1 = the m-side operand (A), 2 = the n-side operand (B)
     int wg_expert_major;    // weight gradients, 256-wide kernel: all (m-tile, n-tile) blocks of an expert on one XCD
     int m_fastest_from;     //   ... for experts with at least this many m-tiles (of the class); the others n-tile first
+    float *part;            // few-row kernel: fp32 partial results [ksplit][part_rows][N] when the contraction is split over blocks
+    long part_rows;
+    int ksplit;
     int m_fastest;          // row-ragged products, 256-wide kernel: number an expert's tiles m-tile first (see gemm256.hip)
 };
 
@@ -94,6 +155,9 @@ struct GemmArgs {
 // meet its alignment requirements; the caller then uses the generic kernel.
 int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid);
 bool gemm256_sums_operand(const GemmArgs &g, int kid);
+// Few rows per expert (gemm_skinny.hip): weights streamed straight into fragments; -100 when the shape is not its.
+int launch_gemm_skinny(const GemmArgs &g, int dtype, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
+size_t gemm_skinny_workspace_bytes(int E, int max_rows, int N, int K, int dtype);
 // fp32 tiles with direct-to-LDS loads (gemm_f32.hip); -100 as above.
 int launch_gemm_f32(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid);
 bool gemm_f32_sums_operand(const GemmArgs &g);

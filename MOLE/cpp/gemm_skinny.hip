@@ -1,0 +1,450 @@
+// Row-ragged products of experts with few rows (decode batches, short training batches): the expert's weights are
+// read once, straight from memory into MFMA fragments, and everything else is arranged around keeping those loads
+// in flight.
+//
+// With a handful of rows per expert a product is a stream over its weights (2 x 16.8 MB for an expert of 2048 x 8192),
+// and the big-tile kernels have too few blocks to pull it: a contraction over 8192 with 2048 result columns is 8 tiles
+// of 256 columns per active expert, each a serial walk over 8192 of K by one CU (about 60 GB/s a CU).  Here the waves of
+// a block split the contraction, and blocks split it further (ksplit) where the result is too narrow to give every CU a
+// block; partial results meet in LDS, or as fp32 planes in a workspace that skinny_reduce_kernel adds up in plane order
+// (deterministic, no atomics).
+//
+// Tokens take the MFMA's B side (16 rows), weights its A side (16 result columns), so a lane ends up with 4 consecutive
+// columns of one row.  A lane supplies EPC = 16 bytes worth of consecutive k (8 bf16: one 16x16x32 MFMA; 4 fp32: four
+// 16x16x4 MFMAs, one per component), lane group l / 16 the k-run l / 16 of a 64-byte step.
+//   KC  (weights [N][K], h = xd.w1^T and t = go.w2^T): a 16-byte load per lane is a fragment as it comes.
+//   KS  (weights [K][N], out = a.w2 and gx = t.w1): a lane loads EPC rows of EPC consecutive columns and transposes
+//       the EPC x EPC block in registers (bf16: byte permutes; fp32: a renaming); fragment j is then column EPC i + j
+//       of the tile's 16 EPC columns for lane i, and a row's results are EPC consecutive columns per lane.
+// No LDS on the way in, no barrier before the partial sums meet.
+#include "gemm.h"
+
+namespace mole {
+
+typedef float sk_f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int SK_WAVES = 8, SK_THREADS = 64 * SK_WAVES;
+constexpr int SK_NA = 4;             // KC: 16-column fragments per block (64 result columns)
+
+template <typename T> struct SkElem;
+template <> struct SkElem<bf16_t> { static constexpr int EPC = 8; };
+template <> struct SkElem<float> { static constexpr int EPC = 4; };
+
+template <typename T> __device__ __forceinline__ sk_f32x4 sk_mma(uint4 w, uint4 x, sk_f32x4 acc) {
+    if constexpr (sizeof(T) == 2) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), acc, 0, 0, 0);
+    } else {
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w.x), __uint_as_float(x.x), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w.y), __uint_as_float(x.y), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w.z), __uint_as_float(x.z), acc, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w.w), __uint_as_float(x.w), acc, 0, 0, 0);
+    }
+}
+
+// q[kk] = EPC consecutive columns of k-row kk; f[j] = the EPC k of column j
+__device__ __forceinline__ void sk_transpose(const uint4 (&q)[8], uint4 (&f)[8]) {
+    const uint32_t w[8][4] = {{q[0].x, q[0].y, q[0].z, q[0].w}, {q[1].x, q[1].y, q[1].z, q[1].w},
+                              {q[2].x, q[2].y, q[2].z, q[2].w}, {q[3].x, q[3].y, q[3].z, q[3].w},
+                              {q[4].x, q[4].y, q[4].z, q[4].w}, {q[5].x, q[5].y, q[5].z, q[5].w},
+                              {q[6].x, q[6].y, q[6].z, q[6].w}, {q[7].x, q[7].y, q[7].z, q[7].w}};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+        f[j] = make_uint4(__builtin_amdgcn_perm(w[1][j >> 1], w[0][j >> 1], sel), __builtin_amdgcn_perm(w[3][j >> 1], w[2][j >> 1], sel),
+                          __builtin_amdgcn_perm(w[5][j >> 1], w[4][j >> 1], sel), __builtin_amdgcn_perm(w[7][j >> 1], w[6][j >> 1], sel));
+    }
+}
+__device__ __forceinline__ void sk_transpose(const uint4 (&q)[4], uint4 (&f)[4]) {
+    f[0] = make_uint4(q[0].x, q[1].x, q[2].x, q[3].x);
+    f[1] = make_uint4(q[0].y, q[1].y, q[2].y, q[3].y);
+    f[2] = make_uint4(q[0].z, q[1].z, q[2].z, q[3].z);
+    f[3] = make_uint4(q[0].w, q[1].w, q[2].w, q[3].w);
+}
+
+// The `target`-th group of at most RG rows, counted over the experts in order: its expert, its number within the expert,
+// the expert's rows and first row.  Every wave looks it up for itself (rows and offsets of 256 experts per pass come in
+// one go); false when there are fewer groups.
+template <int RG>
+__device__ __forceinline__ bool sk_find_group(const GemmArgs &g, int target, int &e, int &grp, int &rows, long &row0) {
+    const int lane = threadIdx.x & 63;
+    int run = 0;
+    for (int base = 0; base < g.E; base += 4 * WAVE) {
+        int r[4], o[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int ee = min(base + c * WAVE + lane, g.E - 1);
+            r[c] = g.kept[ee];
+            o[c] = g.offsets[ee];
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (base + c * WAVE >= g.E) break;
+            const int cnt = base + c * WAVE + lane < g.E ? (r[c] + RG - 1) / RG : 0;
+            int incl = cnt;
+            for (int d = 1; d < WAVE; d <<= 1) {
+                const int y = __shfl_up(incl, d, WAVE);
+                if (lane >= d) incl += y;
+            }
+            const unsigned long long hit = __ballot(run + incl > target);
+            if (hit) {
+                const int src = __ffsll(hit) - 1;
+                e = __builtin_amdgcn_readfirstlane(base + c * WAVE + src);
+                grp = __builtin_amdgcn_readfirstlane(target - (run + __shfl(incl - cnt, src, WAVE)));
+                rows = __builtin_amdgcn_readfirstlane(__shfl(r[c], src, WAVE));
+                row0 = __builtin_amdgcn_readfirstlane(__shfl(o[c], src, WAVE));
+                return true;
+            }
+            run += __shfl(incl, WAVE - 1, WAVE);
+        }
+    }
+    return false;
+}
+
+template <typename T> __device__ __forceinline__ void sk_store4(T *p, const float (&v)[4]) {
+    if constexpr (sizeof(T) == 2) {
+        typedef __bf16 bf16x4_ __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<uint2 *>(p) = __builtin_bit_cast(uint2, bf16x4_{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]});
+    } else {
+        *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+}
+template <typename T> __device__ __forceinline__ void sk_load4(const T *p, float (&v)[4]) {
+    if constexpr (sizeof(T) == 2) {
+        const uint2 u = *reinterpret_cast<const uint2 *>(p);
+        v[0] = __uint_as_float(u.x << 16); v[1] = __uint_as_float(u.x & 0xffff0000u);
+        v[2] = __uint_as_float(u.y << 16); v[3] = __uint_as_float(u.y & 0xffff0000u);
+    } else {
+        const float4 u = *reinterpret_cast<const float4 *>(p);
+        v[0] = u.x; v[1] = u.y; v[2] = u.z; v[3] = u.w;
+    }
+}
+
+// Four consecutive columns n .. n+3 (all inside the result: N is a multiple of 4) of row `row` of expert e.
+template <typename T, int EPI>
+__device__ __forceinline__ void sk_epilogue4(const GemmArgs &g, int e, long row, int n, float (&v)[4]) {
+    if constexpr (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU) {
+        float b[4];
+        sk_load4<T>((const T *)g.bias + (long)e * g.N + n, b);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += b[j];
+    }
+    const long at = row * g.ldc + n;
+    if constexpr (EPI == EPI_DGELU) {
+        float h[4];
+        sk_load4<T>((const T *)g.H + at, h);
+        if constexpr (sizeof(T) == 2) {
+            DGeluCoef d;
+            d.select(g.gelu_bwd == MOLE_GELU_BWD_TANH);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] *= d(h[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] *= g.gelu_bwd == MOLE_GELU_BWD_TANH ? d_gelu_tanh(h[j]) : d_gelu_exact(h[j]);
+        }
+    }
+    if constexpr (EPI == EPI_BIAS_GELU) {
+        if (g.C != nullptr) sk_store4<T>((T *)g.C + at, v);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = sizeof(T) == 2 ? fast_gelu_erf(v[j]) : gelu_erf(v[j]);
+        sk_store4<T>((T *)g.C2 + at, v);
+    } else {
+        sk_store4<T>((T *)g.C + at, v);
+    }
+}
+
+// ---- weights [N][K] ---------------------------------------------------------------------------------------------
+// A block owns 64 result columns of one group of up to 16 MB rows; its eight waves split the contraction.  A wave has the
+// weights of two steps (eight loads of 1 KiB) in flight and waits for them before it asks for more: sixteen waves to a
+// CU, out of step with each other, keep the memory busier than eight waves with two rounds in flight each (the
+// registers allow one or the other; 256 experts of eight rows, 2048 -> 1024: 215 against 250 us, 1.07 GB of weights).
+template <typename T, int MB, int EPI>
+__device__ __forceinline__ void skinny_kc_run(const GemmArgs &g, sk_f32x4 (&red)[SK_WAVES][SK_NA][WAVE], int e, int rows, long row0,
+                                              int m0, int n0) {
+    constexpr int EPC = SkElem<T>::EPC, KSTEP = 4 * EPC, NA = SK_NA, U = 2;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i16 = lane & 15, kg = lane >> 4;
+    const int steps = (g.K + KSTEP - 1) / KSTEP;
+    const int s_lo = wave * steps / SK_WAVES, s_hi = (wave + 1) * steps / SK_WAVES;
+    const T *wp[NA], *xp[MB];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) wp[a] = (const T *)g.B + (long)e * g.strideB + (long)min(n0 + 16 * a + i16, g.N - 1) * g.ldb;
+#pragma unroll
+    for (int b = 0; b < MB; ++b) xp[b] = (const T *)g.A + (row0 + min(m0 + 16 * b + i16, rows - 1)) * g.lda;
+    sk_f32x4 acc[NA][MB];
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int b = 0; b < MB; ++b) acc[a][b] = sk_f32x4{0.f, 0.f, 0.f, 0.f};
+    uint4 w[U][NA], x[U][MB];
+    // steps past the wave's share repeat its last one; they, and k past the contraction's end, are masked to zero
+    auto fetch = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = min(min(s + u, s_hi - 1) * KSTEP + kg * EPC, g.K - EPC);
+#pragma unroll
+            for (int a = 0; a < NA; ++a) w[u][a] = *reinterpret_cast<const uint4 *>(wp[a] + k);
+#pragma unroll
+            for (int b = 0; b < MB; ++b) x[u][b] = *reinterpret_cast<const uint4 *>(xp[b] + k);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto use = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t keep = (s + u < s_hi && (s + u) * KSTEP + kg * EPC < g.K) ? 0xffffffffu : 0u;
+#pragma unroll
+            for (int b = 0; b < MB; ++b) {
+                const uint4 xv = make_uint4(x[u][b].x & keep, x[u][b].y & keep, x[u][b].z & keep, x[u][b].w & keep);
+#pragma unroll
+                for (int a = 0; a < NA; ++a) acc[a][b] = sk_mma<T>(w[u][a], xv, acc[a][b]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int s = s_lo; s < s_hi; s += U) {
+        fetch(s);
+        use(s);
+    }
+    // per 16-row block the waves' partial tiles meet in LDS; wave a adds up 16-column cell a in wave order
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+        if (b > 0) __syncthreads();
+#pragma unroll
+        for (int a = 0; a < NA; ++a) red[wave][a][lane] = acc[a][b];
+        __syncthreads();
+        const int m = m0 + 16 * b + i16, n = n0 + 16 * wave + 4 * kg;
+        if (wave < NA && m < rows && n < g.N) {
+            sk_f32x4 s = red[0][wave][lane];
+#pragma unroll
+            for (int q = 1; q < SK_WAVES; ++q) s += red[q][wave][lane];
+            float v[4] = {s[0], s[1], s[2], s[3]};
+            sk_epilogue4<T, EPI>(g, e, row0 + m, n, v);
+        }
+    }
+}
+
+// MB: 16-row blocks of a group; a group with fewer live ones runs the code for those
+template <typename T, int MB, int EPI>
+__global__ __launch_bounds__(SK_THREADS, 4) void skinny_kc_kernel(const GemmArgs g) {
+    __shared__ __align__(16) sk_f32x4 red[SK_WAVES][SK_NA][WAVE];
+    const int chunks = (g.N + 16 * SK_NA - 1) / (16 * SK_NA);
+    int e, grp, rows;
+    long row0;
+    if (!sk_find_group<16 * MB>(g, blockIdx.x / chunks, e, grp, rows, row0)) return;
+    const int n0 = (blockIdx.x % chunks) * (16 * SK_NA), m0 = grp * (16 * MB), live = rows - m0;
+    if (MB == 1 || live <= 16) skinny_kc_run<T, 1, EPI>(g, red, e, rows, row0, m0, n0);
+    else skinny_kc_run<T, MB, EPI>(g, red, e, rows, row0, m0, n0);
+}
+
+// ---- weights [K][N] ---------------------------------------------------------------------------------------------
+// A block owns 16 EPC result columns (256 bytes of a weight row) of one group of up to 16 MB rows and 1 / ksplit of the
+// contraction, which its eight waves split again; a wave has the weights of one step (EPC loads of 1 KiB) in flight.
+template <typename T, int MB, int EPI>
+__device__ __forceinline__ void skinny_ks_run(const GemmArgs &g, sk_f32x4 (&red)[SK_WAVES][SkElem<T>::EPC][WAVE], int e, int rows,
+                                              long row0, int m0, int n0, int split) {
+    constexpr int EPC = SkElem<T>::EPC, KSTEP = 4 * EPC;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i16 = lane & 15, kg = lane >> 4;
+    const int steps = (g.K + KSTEP - 1) / KSTEP, parts = g.ksplit * SK_WAVES, part = split * SK_WAVES + wave;
+    const int s_lo = (int)((long)part * steps / parts), s_hi = (int)((long)(part + 1) * steps / parts);
+    const T *wp = (const T *)g.B + (long)e * g.strideB + min(n0 + i16 * EPC, g.N - EPC);
+    const T *xp[MB];
+#pragma unroll
+    for (int b = 0; b < MB; ++b) xp[b] = (const T *)g.A + (row0 + min(m0 + 16 * b + i16, rows - 1)) * g.lda;
+    sk_f32x4 acc[EPC][MB];
+#pragma unroll
+    for (int j = 0; j < EPC; ++j)
+#pragma unroll
+        for (int b = 0; b < MB; ++b) acc[j][b] = sk_f32x4{0.f, 0.f, 0.f, 0.f};
+    uint4 w[EPC], x[MB];
+    auto fetch = [&](int s) __attribute__((always_inline)) {
+        const int k = min(s * KSTEP + kg * EPC, g.K - EPC);
+        const T *wk = wp + (long)k * g.ldb;
+#pragma unroll
+        for (int q = 0; q < EPC; ++q) w[q] = *reinterpret_cast<const uint4 *>(wk + (long)q * g.ldb);
+#pragma unroll
+        for (int b = 0; b < MB; ++b) x[b] = *reinterpret_cast<const uint4 *>(xp[b] + k);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto use = [&](int s) __attribute__((always_inline)) {
+        const uint32_t keep = s * KSTEP + kg * EPC < g.K ? 0xffffffffu : 0u;
+        uint4 f[EPC];
+        sk_transpose(w, f);
+#pragma unroll
+        for (int b = 0; b < MB; ++b) {
+            const uint4 xv = make_uint4(x[b].x & keep, x[b].y & keep, x[b].z & keep, x[b].w & keep);
+#pragma unroll
+            for (int j = 0; j < EPC; ++j) acc[j][b] = sk_mma<T>(f[j], xv, acc[j][b]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int s = s_lo; s < s_hi; ++s) {
+        fetch(s);
+        use(s);
+    }
+    // acc[j][b][r] of lane (i16, kg) is row m0 + 16 b + i16, column n0 + EPC (4 kg + r) + j.  Per 16-row block the waves'
+    // partial tiles meet in LDS; a thread adds up four consecutive columns (j = 4 q .. 4 q + 3) of one lane and r.
+    constexpr int QJ = EPC / 4;          // quadruples of columns per (lane, r)
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+        if (b > 0) __syncthreads();
+#pragma unroll
+        for (int j = 0; j < EPC; ++j) red[wave][j][lane] = acc[j][b];
+        __syncthreads();
+        const int r = wave & 3;
+        const int m = m0 + 16 * b + i16;
+        if (wave < 4 * QJ && m < rows) {
+            const int q = wave >> 2;
+            const int n = n0 + EPC * (4 * kg + r) + 4 * q;
+            if (n < g.N) {
+                float v[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float s = red[0][4 * q + j][lane][r];
+#pragma unroll
+                    for (int ww = 1; ww < SK_WAVES; ++ww) s += red[ww][4 * q + j][lane][r];
+                    v[j] = s;
+                }
+                if (g.ksplit == 1) {
+                    sk_epilogue4<T, EPI>(g, e, row0 + m, n, v);
+                } else {
+                    if (EPI == EPI_BIAS && split == 0) {
+                        float bv[4];
+                        sk_load4<T>((const T *)g.bias + (long)e * g.N + n, bv);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) v[j] += bv[j];
+                    }
+                    *reinterpret_cast<float4 *>(g.part + ((long)split * g.part_rows + row0 + m) * g.N + n) = make_float4(v[0], v[1], v[2], v[3]);
+                }
+            }
+        }
+    }
+}
+
+template <typename T, int MB, int EPI>
+__global__ __launch_bounds__(SK_THREADS, 4) void skinny_ks_kernel(const GemmArgs g) {
+    constexpr int BN = 16 * SkElem<T>::EPC;
+    __shared__ __align__(16) sk_f32x4 red[SK_WAVES][SkElem<T>::EPC][WAVE];
+    const int chunks = (g.N + BN - 1) / BN;
+    int e, grp, rows;
+    long row0;
+    const int per_group = chunks * g.ksplit;
+    if (!sk_find_group<16 * MB>(g, blockIdx.x / per_group, e, grp, rows, row0)) return;
+    const int in_group = blockIdx.x % per_group;
+    const int n0 = (in_group % chunks) * BN, split = in_group / chunks, m0 = grp * (16 * MB), live = rows - m0;
+    if (MB == 1 || live <= 16) skinny_ks_run<T, 1, EPI>(g, red, e, rows, row0, m0, n0, split);
+    else skinny_ks_run<T, MB, EPI>(g, red, e, rows, row0, m0, n0, split);
+}
+
+// out[row][n] = sum over the planes of part[plane][row][n] (the bias is in plane 0), rows of every expert
+template <typename T>
+__global__ __launch_bounds__(256) void skinny_reduce_kernel(const float *__restrict__ part, long part_rows, int N, int ksplit, T *__restrict__ out) {
+    const long row = blockIdx.y;
+    const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
+    if (n >= N) return;
+    const float *p = part + row * N + n;
+    const long plane = part_rows * N;
+    float4 s = *reinterpret_cast<const float4 *>(p);
+    for (int k = 1; k < ksplit; k += 4) {
+        float4 t[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) t[u] = *reinterpret_cast<const float4 *>(p + (long)min(k + u, ksplit - 1) * plane);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (k + u < ksplit) { s.x += t[u].x; s.y += t[u].y; s.z += t[u].z; s.w += t[u].w; }
+    }
+    float v[4] = {s.x, s.y, s.z, s.w};
+    sk_store4<T>(out + row * N + n, v);
+}
+
+// ---- which products come here, and how they are cut ------------------------------------------------------------
+// avg: rows of an expert if the rows spread evenly; tiles: blocks the big-tile kernel of the type would have.
+struct SkinnyPlan { int mb, ksplit, groups; };
+static bool skinny_plan(int dtype, bool b_ks, int E, int max_rows, int N, int K, SkinnyPlan &p) {
+    if (max_rows <= 0) return false;
+    const bool bf16 = dtype == MOLE_BF16;
+    const int epc = bf16 ? 8 : 4;
+    const int active = E < max_rows ? E : max_rows;
+    const int avg = ceil_div(max_rows, active);
+    // bf16: with a CU's worth of tiles or more (192 of 256) the 256-column tiles of gemm256.hip stream the weights as
+    // fast or faster (16 experts of 1024 -> 4096, 61 rows: 27 against 30 us); with fewer they leave CUs without work
+    // (2 rows of 64 experts, 2048 -> 8192: h 24 against 17.5 us, out 66 against 13).  KC stops at 24 rows per expert,
+    // where the token loads, one per four weight loads and 16 rows, begin to cost (8 experts of 512 -> 2048, 600 rows:
+    // 18 against 14 us); KS, eight weight loads each, at 64 (16 x 1024 -> 4096, 400 / 800 / 1600 rows: 39 / 50 / 79
+    // against 55 / 61 / 75 us).
+    // fp32: the 64 x 128 tiles of gemm_f32.hip walk the whole contraction in one block, however few rows there are
+    // (out at 16 x 1024 -> 4096: 128 us from 2 to 800 rows); 244 / 400 / 800 / 1600 rows: 59 / 75 / 102 / 157 against
+    // 127 / 127 / 128 / 137 us.  KC: 244 / 400 rows 69 / 84 against 75 / 78 us.
+    bool takes;
+    if (bf16) {
+        const long tiles = (long)active * ceil_div(avg, 256) * ceil_div(N, 256);
+        takes = tiles < 192 && avg <= (b_ks ? 64 : 24);
+    } else {
+        takes = avg <= (b_ks ? 64 : 20);
+    }
+    if (!takes) return false;
+    // rows per group: KC shares a block's weight loads among 32 rows once experts hold more than eight; KS in bf16 has
+    // eight accumulators per 16 rows and runs better on more waves (groups of 16 re-read the weights out of the caches)
+    p.mb = b_ks ? (bf16 ? 1 : 2) : (avg > 8 ? 2 : 1);
+    p.groups = active + max_rows / (16 * p.mb);
+    // KS: about two blocks of eight waves per CU, every wave with at least two steps
+    const int blocks = active * ceil_div(avg, 16 * p.mb) * ceil_div(N, 16 * epc);
+    int ks = b_ks ? ceil_div(512, blocks) : 1;
+    const int most = ceil_div(K, 4 * epc) / (2 * SK_WAVES);
+    if (ks > most) ks = most;
+    if (ks > 16) ks = 16;
+    p.ksplit = ks < 1 ? 1 : ks;
+    return true;
+}
+
+size_t gemm_skinny_workspace_bytes(int E, int max_rows, int N, int K, int dtype) {
+    SkinnyPlan p;
+    if (!skinny_plan(dtype, true, E, max_rows, N, K, p)) return 0;
+    return p.ksplit > 1 ? (size_t)p.ksplit * max_rows * N * sizeof(float) : 0;
+}
+
+template <typename T, int MB>
+static int launch_kc(const GemmArgs &g, int epi, int groups, hipStream_t st, int kid) {
+    const dim3 grid((unsigned)(groups * ceil_div(g.N, 16 * SK_NA)));
+    if (epi == EPI_BIAS_GELU) timed_launch(kid, skinny_kc_kernel<T, MB, EPI_BIAS_GELU>, grid, dim3(SK_THREADS), 0, st, g);
+    else if (epi == EPI_DGELU) timed_launch(kid, skinny_kc_kernel<T, MB, EPI_DGELU>, grid, dim3(SK_THREADS), 0, st, g);
+    else return -100;
+    MOLE_LAUNCH_CHECK();
+    return 0;
+}
+
+template <typename T, int MB>
+static int launch_ks(const GemmArgs &g, int epi, int groups, int max_rows, hipStream_t st, int kid) {
+    const dim3 grid((unsigned)(groups * ceil_div(g.N, 16 * SkElem<T>::EPC) * g.ksplit));
+    if (epi == EPI_BIAS) timed_launch(kid, skinny_ks_kernel<T, MB, EPI_BIAS>, grid, dim3(SK_THREADS), 0, st, g);
+    else if (epi == EPI_STORE) timed_launch(kid, skinny_ks_kernel<T, MB, EPI_STORE>, grid, dim3(SK_THREADS), 0, st, g);
+    else return -100;
+    MOLE_LAUNCH_CHECK();
+    if (g.ksplit > 1) {
+        hipLaunchKernelGGL(skinny_reduce_kernel<T>, dim3(ceil_div(g.N, 1024), max_rows), dim3(256), 0, st, g.part, g.part_rows, g.N, g.ksplit, (T *)g.C);
+        MOLE_LAUNCH_CHECK();
+    }
+    return 0;
+}
+
+int launch_gemm_skinny(const GemmArgs &g0, int dtype, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid) {
+    GemmArgs g = g0;
+    const int epc = dtype == MOLE_BF16 ? 8 : 4;
+    SkinnyPlan p;
+    if (g.offsets == nullptr || g.kept == nullptr || !skinny_plan(dtype, b_ks, g.E, max_rows, g.N, g.K, p)) return -100;
+    if (g.K % epc || g.N % epc || g.lda % epc || g.ldb % epc || g.ldc % epc || g.strideB % epc) return -100;
+    g.ksplit = 1;
+    if (p.ksplit > 1 && ws != nullptr && ws_bytes >= (size_t)p.ksplit * max_rows * g.N * sizeof(float)) {
+        g.ksplit = p.ksplit;
+        g.part = (float *)ws;
+        g.part_rows = max_rows;
+    }
+    if (dtype == MOLE_BF16) {
+        if (b_ks) return launch_ks<bf16_t, 1>(g, epi, p.groups, max_rows, st, kid);
+        return p.mb == 1 ? launch_kc<bf16_t, 1>(g, epi, p.groups, st, kid) : launch_kc<bf16_t, 2>(g, epi, p.groups, st, kid);
+    }
+    if (b_ks) return launch_ks<float, 2>(g, epi, p.groups, max_rows, st, kid);
+    return p.mb == 1 ? launch_kc<float, 1>(g, epi, p.groups, st, kid) : launch_kc<float, 2>(g, epi, p.groups, st, kid);
+}
+
+}  // namespace mole

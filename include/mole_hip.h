@@ -237,6 +237,20 @@ int mole_ffn_bwd(const void *go, const void *xd, const void *h, const void *a, i
                  const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, int M, int F,
                  const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2,
                  void *g_b2, void *gx, int accumulate, int gelu_bwd, mole_stream_t stream);
+/* The same two calls with a workspace.  With few rows per expert the two products whose contraction runs over F are
+ * narrow (M columns) and long; given mole_ffn_workspace_bytes() bytes (0: none needed) the library splits the
+ * contraction over several blocks and adds the fp32 partial results in a fixed order.  A smaller or NULL workspace is
+ * allowed: the contraction is then not split. */
+size_t mole_ffn_workspace_bytes(int dtype, int E, int max_rows, int M, int F);
+int mole_ffn_fwd_ws(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
+                    int max_rows, int M, int F, const void *w1, const void *b1, const void *w2,
+                    const void *b2, void *h, void *a, void *out, void *workspace, size_t workspace_bytes,
+                    mole_stream_t stream);
+int mole_ffn_bwd_ws(const void *go, const void *xd, const void *h, const void *a, int dtype,
+                    const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, int M, int F,
+                    const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2,
+                    void *g_b2, void *gx, int accumulate, int gelu_bwd, void *workspace, size_t workspace_bytes,
+                    mole_stream_t stream);
 
 /* Plain GEMMs on the same tiles, used by the gate: c[rows,N] = a[rows,K] . b[N,K]^T  (fp32 out). */
 int mole_gemm_nt(const void *a, const void *b, int dtype, int rows, int N, int K, float *c,

@@ -55,6 +55,10 @@ _SIGNATURES = {
     "mole_ffn_fwd": (c_int, [_P, c_int, _P, _P, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P, _P]),
     "mole_ffn_bwd": (c_int, [_P, _P, _P, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P,
                              _P, c_int, c_int, _P]),
+    "mole_ffn_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
+    "mole_ffn_fwd_ws": (c_int, [_P, c_int, _P, _P, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P, _P, c_size_t, _P]),
+    "mole_ffn_bwd_ws": (c_int, [_P, _P, _P, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P,
+                                _P, c_int, c_int, _P, c_size_t, _P]),
     "mole_gemm_nt": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P]),
     "mole_gemm_nn": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P]),
     "mole_gemm_tn": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P]),

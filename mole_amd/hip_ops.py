@@ -336,20 +336,28 @@ def zero_pad_rows(buf: torch.Tensor, kept_rows: torch.Tensor, offsets: torch.Ten
             "mole_zero_pad_rows")
 
 
+def _ffn_workspace(xd, E, max_rows, M, F):
+    """(tensor or None, bytes): scratch for the products that the library splits over blocks when experts have few rows."""
+    nbytes = L.lib().mole_ffn_workspace_bytes(L.dtype_code(xd.dtype), int(E), int(max_rows), int(M), int(F))
+    return (torch.empty(nbytes, dtype=torch.uint8, device=xd.device) if nbytes else None), nbytes
+
+
 def ffn_fwd_into(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out) -> None:
     """mole_ffn_fwd on caller-provided buffers.  Weights may be tensors or raw device addresses
     (slot-pool pointers); offsets/kept_rows may be views starting at the first expert of a chunk."""
-    L.check(L.lib().mole_ffn_fwd(L.ptr(xd), L.dtype_code(xd.dtype), L.ptr(offsets), L.ptr(kept_rows), int(E), int(max_rows),
-                                 int(M), int(F), L.ptr(w1), L.ptr(b1), L.ptr(w2), L.ptr(b2), L.ptr(h), L.ptr(a), L.ptr(out),
-                                 L.stream()), "mole_ffn_fwd")
+    ws, nbytes = _ffn_workspace(xd, E, max_rows, M, F)
+    L.check(L.lib().mole_ffn_fwd_ws(L.ptr(xd), L.dtype_code(xd.dtype), L.ptr(offsets), L.ptr(kept_rows), int(E), int(max_rows),
+                                    int(M), int(F), L.ptr(w1), L.ptr(b1), L.ptr(w2), L.ptr(b2), L.ptr(h), L.ptr(a), L.ptr(out),
+                                    L.ptr(ws), nbytes, L.stream()), "mole_ffn_fwd")
 
 
 def ffn_bwd_into(go, xd, h, a, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx,
                  accumulate: bool, gelu_bwd: int) -> None:
-    L.check(L.lib().mole_ffn_bwd(L.ptr(go), L.ptr(xd), L.ptr(h), L.ptr(a), L.dtype_code(xd.dtype), L.ptr(offsets),
-                                 L.ptr(kept_rows), int(E), int(max_rows), int(M), int(F), L.ptr(w1), L.ptr(w2), L.ptr(t),
-                                 L.ptr(g_w1), L.ptr(g_b1), L.ptr(g_w2), L.ptr(g_b2), L.ptr(gx), int(accumulate),
-                                 int(gelu_bwd), L.stream()), "mole_ffn_bwd")
+    ws, nbytes = _ffn_workspace(xd, E, max_rows, M, F) if gx is not None else (None, 0)
+    L.check(L.lib().mole_ffn_bwd_ws(L.ptr(go), L.ptr(xd), L.ptr(h), L.ptr(a), L.dtype_code(xd.dtype), L.ptr(offsets),
+                                    L.ptr(kept_rows), int(E), int(max_rows), int(M), int(F), L.ptr(w1), L.ptr(w2), L.ptr(t),
+                                    L.ptr(g_w1), L.ptr(g_b1), L.ptr(g_w2), L.ptr(g_b2), L.ptr(gx), int(accumulate),
+                                    int(gelu_bwd), L.ptr(ws), nbytes, L.stream()), "mole_ffn_bwd")
 
 
 def ffn_fwd(xd, offsets, kept_rows, w1, b1, w2, b2, max_rows: Optional[int] = None):

@@ -342,3 +342,43 @@ def test_fused_activation_math_on_a_dense_grid(dtype):
         worst = float((err - half_ulp(d64, slack)).max())
         print(f"fused GELU' ({variant}) {dtype}: worst error beyond rounding {worst:.2e}", flush=True)
         assert bool((err <= bound).all()), f"GELU' ({variant}) off by {float((err / bound).max()):.2f}x its bound"
+
+
+# Experts of few rows: the streamed-weight kernels.  Rows around their 16-row blocks and 32-row groups, widths that end
+# inside a step of the contraction, a 64- or 128-column tile, and contractions short and long enough to be split over
+# blocks or not.  The tolerance is the one of every FFN test (fp32 sums of bf16 / fp32 products in another order).
+FEW_ROWS = [
+    (1, 64, 128, [1], 0),
+    (4, 520, 1416, [1, 0, 15, 16], 0),
+    (5, 136, 2056, [17, 1, 0, 31, 3], 2),
+    (3, 264, 4096, [33, 16, 5], 1),
+    (6, 1032, 520, [0, 2, 40, 1, 0, 64], 0),
+    (70, 64, 1032, [(5 * e) % 9 for e in range(70)], 0),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("E,M,Fd,rows,gap", FEW_ROWS)
+def test_ffn_few_rows_matches_oracle(E, M, Fd, rows, gap, dtype):
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"ffn few rows E={E} M={M} F={Fd} rows={rows} gap={gap} {dtype}", flush=True)
+    d = _make(E, M, Fd, rows, dtype, seed=E + M + Fd, pad_between=gap)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off = torch.from_numpy(d["off"]).cuda(); n = torch.from_numpy(d["n"]).cuda()
+    w_out, w_h, w_gx, w_gw1, w_gb1, w_gw2, w_gb2 = _oracle_fwd_bwd(d, "tanh")
+    mask = torch.zeros(max(d["R"], 1), dtype=torch.bool)
+    for e in range(E):
+        mask[int(d["off"][e]):int(d["off"][e]) + int(d["n"][e])] = True
+    t = tol(dtype)
+    out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+    g = [torch.full_like(c[k], 9.0) for k in ("w1", "b1", "w2", "b2")]
+    gx = H.ffn_bwd(c["go"], c["xd"], h, a, off, n, c["w1"], c["w2"], *g)
+    for got, want in ((h, w_h), (a, torch.nn.functional.gelu(w_h)), (out, w_out), (gx, w_gx)):
+        assert rel_err(got.cpu()[mask], want[mask]) < t
+    for got, want in zip(g, (w_gw1, w_gb1, w_gw2, w_gb2)):
+        assert rel_err(got, want) < t
+    # without a workspace the contraction is not split over blocks: the same result to rounding
+    out2, h2, a2 = torch.empty_like(out), torch.empty_like(h), torch.empty_like(a)
+    L.check(L.lib().mole_ffn_fwd(L.ptr(c["xd"]), L.dtype_code(dtype), L.ptr(off), L.ptr(n), E, d["R"], M, Fd, L.ptr(c["w1"]),
+                                 L.ptr(c["b1"]), L.ptr(c["w2"]), L.ptr(c["b2"]), L.ptr(h2), L.ptr(a2), L.ptr(out2), L.stream()), "ffn")
+    assert torch.equal(h2.cpu()[mask], h.cpu()[mask]) and rel_err(out2.cpu()[mask], w_out[mask]) < t
