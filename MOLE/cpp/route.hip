@@ -4,14 +4,14 @@
 // Replaces tutel's extract_critical (called at MOLE/moe/layer.py:445-446) and the softmax half of
 // MOLETopk.forward (MOLE/utils/Ugate.py:13).
 //
-// Four launches, all on the caller's stream:
-//   route_topk      64 tokens per block (16 per wave).  A group of G lanes (G = pow2 >= E, at most 64) owns one
-//                   token and holds VPL = ceil(E/G) scores per lane; k rounds of a shuffle arg-max
-//                   with the (score desc, index asc) order.  Then, per choice j, the rank of each
-//                   token among the block's earlier tokens with the same expert: wave ballot +
-//                   popcount over the block's 64 tokens.
+// Up to four launches, all on the caller's stream:
+//   route_tokens    64 tokens per block of 16 waves.  A group of 16 lanes (64 beyond 256 experts) owns one token and holds
+//                   its scores in registers - softmaxed on the spot when it is given logits; k rounds of a lane-pattern
+//                   arg-max with the (score desc, index asc) order.  Then wave j ranks choice j: a token's rank is the
+//                   number of the block's earlier tokens with the same expert, from one ballot per bit of the index.
 //   route_scan      one wave per (choice, expert): exclusive prefix over the blocks' histograms.
-//   route_finish    one block: per-expert totals, capacity, kept rows, row offsets, l_aux.
+//   route_finish    one block: per-expert totals, capacity, kept rows, row offsets, l_aux; for small problems also the scan
+//                   and the last stage.  A single block of tokens does all of it itself.
 //   route_finalize  loc = base(choice, expert) + block prefix + in-block rank; row = offset + loc.
 #include "common.h"
 
@@ -24,8 +24,7 @@
 namespace mole {
 
 constexpr int RT_THREADS = 256;
-constexpr int RT_TOKENS = 64;   // tokens per block: 16 per wave in the top-k phase; a choice is ranked by one wave over all 64
-constexpr int RT_WTOK = RT_TOKENS / 4;
+constexpr int RT_TOKENS = 64;   // tokens per block of route_tokens; a choice is ranked by one wave over all 64
 constexpr float FP32_EPS = 1.1920928955078125e-07f;
 
 // A load that is always issued (the caller clamps the address to something valid) and gives +0 where the value
@@ -73,6 +72,20 @@ template <typename T, typename Op> __device__ __forceinline__ T group_reduce(T x
     return x;
 }
 
+// Rank of the lane among the valid lanes below it that hold the same expert, and how many valid lanes hold it: one ballot
+// per bit of the expert index.  (A loop over the distinct experts present is a serial chain of up to 64 ballots and
+// lane reads.)
+__device__ __forceinline__ int rank_in_wave(int e, bool valid, int E, int &same) {
+    uint64_t m = __ballot(valid);
+    for (int b = 0; (1 << b) < E; ++b) {
+        const bool bit = (e >> b) & 1;
+        const uint64_t bal = __ballot(valid && bit);
+        m &= bit ? bal : ~bal;
+    }
+    same = __popcll(m);
+    return __popcll(m & ((1ull << (threadIdx.x & 63)) - 1ull));
+}
+
 // What a block does once the top-k of its BT tokens (BT <= 64) lies in LDS - s_idx / s_graw [k][BT]: expert and raw
 // gate value of every choice, s_col [4][E]: the four waves' column sums of the block's scores: the block's column sums
 // out, gate values and indices out, then each choice's in-block ranks and per-expert histogram.  Four waves.
@@ -103,109 +116,20 @@ __device__ __forceinline__ void topk_block_tail(int BT, int S, int E, int k, int
     }
 
     // ---- in-block ranks per choice (lane = token; wave w takes choices w, w + 4, ...) ------
-    // Each wave works on a histogram of its own, so the choices proceed side by side without block barriers
-    // (the loop over distinct experts is a serial chain of ballots: with one wave doing all k choices it was the
-    // longest part of the kernel at top-8).
-    const uint64_t lt_mask = (1ull << lane) - 1ull;
+    // Each wave works on a histogram of its own, so the choices proceed side by side without block barriers.
     int *my_hist = s_hist + w * E;
     const int ctoken = tok0 + lane;
     const bool cv = lane < BT && ctoken < S;
     for (int j = w; j < k; j += RT_THREADS / WAVE) {
         for (int e = lane; e < E; e += WAVE) my_hist[e] = 0;
         const int e = cv ? s_idx[j * BT + lane] : -1;
-        int rank = 0;
-        uint64_t remaining = __ballot(cv);
-        while (remaining) {
-            const int leader = __ffsll((unsigned long long)remaining) - 1;
-            const int e0 = __shfl(e, leader, WAVE);
-            const uint64_t m = __ballot(cv && e == e0);
-            if (cv && e == e0) rank = __popcll(m & lt_mask);
-            if (lane == leader) my_hist[e0] = __popcll(m);
-            remaining &= ~m;
-        }
+        int same;
+        const int rank = rank_in_wave(e, cv, E, same);
+        if (cv && rank == 0) my_hist[e] = same;
         if (cv) lrank[(size_t)j * S + ctoken] = rank;
         // (the histogram is written and read by this wave only: program order is enough)
         for (int e2 = lane; e2 < E; e2 += WAVE) hist[((size_t)j * E + e2) * nb + b] = my_hist[e2];
     }
-}
-
-template <int VPL>
-__global__ __launch_bounds__(RT_THREADS) void route_topk_kernel(
-    const float *__restrict__ scores, int S, int E, int k, int logG, int normalize,
-    int32_t *__restrict__ idx, int32_t *__restrict__ lrank, float *__restrict__ gates,
-    int32_t *__restrict__ hist /* [k][E][nb] */, float *__restrict__ colsum /* [nb][E] */, int nb) {
-    extern __shared__ char smem[];
-    int *s_idx = (int *)smem;                          // [k][64]
-    float *s_graw = (float *)(s_idx + k * RT_TOKENS);  // [k][64]
-    int *s_hist = (int *)(s_graw + k * RT_TOKENS);     // [4][E]: one histogram per wave
-    float *s_col = (float *)(s_hist + 4 * E);          // [4][E]
-
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int b = blockIdx.x, tok0 = b * RT_TOKENS;
-    const int G = 1 << logG;
-    const int tpw = 64 >> logG;  // tokens a wave handles per pass
-    const int g = lane & (G - 1), tg = lane >> logG;
-
-    // ---- phase A: top-k of every token (wave w owns tokens 16w .. 16w+15 of the block) ----------
-    float colacc[VPL];
-#pragma unroll
-    for (int r = 0; r < VPL; ++r) colacc[r] = 0.f;
-
-    // the scores of the wave's next token(s) are fetched while the current ones go through their k rounds
-    float nxt[VPL];
-#pragma unroll
-    for (int r = 0; r < VPL; ++r) nxt[r] = 0.f;
-    auto fetch = [&](int it) __attribute__((always_inline)) {
-        const int tok = min(tok0 + w * RT_WTOK + it * tpw + tg, S - 1);
-#pragma unroll
-        for (int r = 0; r < VPL; ++r) nxt[r] = scores[(size_t)tok * E + min(g + (r << logG), E - 1)];
-    };
-    if (S > 0) fetch(0);
-    for (int it = 0; it * tpw < RT_WTOK; ++it) {
-        const int tw = it * tpw + tg;                  // token within the wave's 16
-        const int tl = w * RT_WTOK + tw;
-        const int token = tok0 + tl;
-        const bool tv = tw < RT_WTOK && token < S;
-        uint32_t key[VPL];
-#pragma unroll
-        for (int r = 0; r < VPL; ++r) {
-            const bool ok = tv && g + (r << logG) < E;
-            const float sv = __uint_as_float(__float_as_uint(nxt[r]) & (ok ? 0xffffffffu : 0u));
-            colacc[r] += sv;
-            key[r] = ok ? topk_key(sv) : 0u;
-        }
-        if (S > 0 && (it + 1) * tpw < RT_WTOK) fetch(it + 1);
-        for (int j = 0; j < k; ++j) {
-            // the best score of the token, then the lowest expert index among those that hold it
-            uint32_t best = key[0];
-#pragma unroll
-            for (int r = 1; r < VPL; ++r) best = max(best, key[r]);
-            const uint32_t top = group_reduce(best, logG, [](uint32_t a, uint32_t c) { return max(a, c); });
-            int cand = INT_MAX;
-#pragma unroll
-            for (int r = VPL - 1; r >= 0; --r)
-                if (key[r] == top) cand = g + (r << logG);             // ends on the lane's lowest such expert
-            if (top == 0u) cand = INT_MAX;                             // nothing available (a token past the end)
-            const int bi = group_reduce(cand, logG, [](int a, int c) { return min(a, c); });
-            const bool mine = bi != INT_MAX && (bi & (G - 1)) == g;
-#pragma unroll
-            for (int r = 0; r < VPL; ++r)
-                if (mine && (bi >> logG) == r) key[r] = 0u;
-            if (g == 0 && tv) {
-                s_idx[j * RT_TOKENS + tl] = bi;
-                s_graw[j * RT_TOKENS + tl] = topk_unkey(top);
-            }
-        }
-    }
-    // column sums of the scores (for l_aux): fold the token groups of a wave, then the 4 waves
-#pragma unroll
-    for (int r = 0; r < VPL; ++r) {
-        float c = colacc[r];
-        for (int m = G; m < WAVE; m <<= 1) c += __shfl_xor(c, m, WAVE);
-        const int e = g + (r << logG);
-        if (tg == 0 && e < E) s_col[w * E + e] = c;
-    }
-    topk_block_tail(RT_TOKENS, S, E, k, normalize, s_idx, s_graw, s_hist, s_col, idx, lrank, gates, hist, colsum, nb);
 }
 
 // one wave per (choice, expert) pair: exclusive prefix over blocks, total into counts
@@ -267,115 +191,159 @@ __global__ __launch_bounds__(256) void route_scan_kernel(int32_t *__restrict__ h
 
 constexpr int FIN_THREADS = 1024;
 
-// scan_hist != NULL: the block first does the work of route_scan_kernel itself (small problems: one launch
-// less), its 16 waves taking the pairs in turn.
-__global__ __launch_bounds__(FIN_THREADS) void route_finish_kernel(
-    int32_t *__restrict__ counts, const float *__restrict__ colsum, int nb, int S, int E, int k,
-    int cf_sign, int cap_bound, int alignment, int layout, int32_t *__restrict__ basej,
-    int32_t *__restrict__ kept_rows, int32_t *__restrict__ offsets, int32_t *__restrict__ capacity,
-    float *__restrict__ l_aux, int32_t *__restrict__ scan_hist) {
-    __shared__ int s_n[MOLE_MAX_EXPERTS];
-    __shared__ int s_red[FIN_THREADS];
-    __shared__ float s_fred[FIN_THREADS];
-    const int tid = threadIdx.x;
-    if (scan_hist != nullptr) {
-        for (int pair = tid >> 6; pair < k * E; pair += FIN_THREADS / 64) scan_pair(scan_hist, nb, pair, counts);
-        __threadfence_block();
-        __syncthreads();
-    }
-    // only the first min(E, FIN_THREADS) threads hold data: the block-wide reductions and the scan below run over
-    // the next power of two, not over all 1024 threads (fewer barrier rounds for small gates)
-    int P = 1;
-    while (P < E && P < FIN_THREADS) P <<= 1;
-    int lmax = 0;
-    for (int e = tid; e < E; e += FIN_THREADS) {
-        int tot = 0;
-        for (int j = 0; j < k; ++j) {
-            basej[j * E + e] = tot;
-            tot += counts[j * E + e];
-        }
-        s_n[e] = tot;
-        lmax = max(lmax, tot);
-    }
-    s_red[tid] = lmax;
-    __syncthreads();
-    for (int d = P / 2; d >= 1; d >>= 1) {
-        if (tid < d) s_red[tid] = max(s_red[tid], s_red[tid + d]);
-        __syncthreads();
-    }
-    int cap = cf_sign > 0 ? cap_bound : s_red[0];
-    if (cf_sign < 0) cap = min(cap, cap_bound);
-    const int rem = cap % alignment;
-    if (rem > 0) cap += alignment - rem;
-    __syncthreads();
+// What the end of the routing needs and produces.
+struct RouteEnd {
+    int S, E, k, cf_sign, cap_bound, alignment, layout;
+    int32_t *counts, *kept_rows, *offsets, *capacity;
+    float *l_aux;
+    int32_t *idx, *loc, *row;          // loc: in-block ranks in, locations out
+};
 
-    // kept rows, then their exclusive prefix (chunk per thread + Hillis-Steele over the chunks)
-    const int chunk = (E + FIN_THREADS - 1) / FIN_THREADS;
-    const int lo = min(tid * chunk, E), hi = min(lo + chunk, E);
-    int csum = 0;
-    for (int e = lo; e < hi; ++e) {
-        const int n = min(s_n[e], cap);
-        s_n[e] = n;
-        kept_rows[e] = n;
-        csum += n;
-    }
-    s_red[tid] = csum;
+// block-wide reductions of FIN_THREADS threads: lane patterns inside a wave, 16 values in LDS between the waves
+__device__ __forceinline__ int block_max(int v, int *s16) {
+    v = group_reduce(v, 6, [](int a, int c) { return max(a, c); });
+    if ((threadIdx.x & 63) == 0) s16[threadIdx.x >> 6] = v;
     __syncthreads();
-    for (int d = 1; d < P; d <<= 1) {
-        const int y = tid >= d ? s_red[tid - d] : 0;
-        __syncthreads();
-        s_red[tid] += y;
-        __syncthreads();
+    int m = s16[0];
+#pragma unroll
+    for (int w = 1; w < FIN_THREADS / WAVE; ++w) m = max(m, s16[w]);
+    __syncthreads();
+    return m;
+}
+__device__ __forceinline__ float block_sum(float v, float *s16) {
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) s16[threadIdx.x >> 6] = v;
+    __syncthreads();
+    float m = s16[0];
+#pragma unroll
+    for (int w = 1; w < FIN_THREADS / WAVE; ++w) m += s16[w];
+    __syncthreads();
+    return m;
+}
+__device__ __forceinline__ int block_inclusive(int v, int *s16) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int d = 1; d < WAVE; d <<= 1) {
+        const int y = __shfl_up(v, d, WAVE);
+        if (lane >= d) v += y;
     }
-    if (layout == MOLE_LAYOUT_RAGGED) {
-        int run = s_red[tid] - csum;
-        for (int e = lo; e < hi; ++e) {
-            offsets[e] = run;
-            run += s_n[e];
+    if (lane == WAVE - 1) s16[w] = v;
+    __syncthreads();
+    for (int q = 0; q < w; ++q) v += s16[q];
+    __syncthreads();
+    return v;
+}
+
+// Counts -> capacity, kept rows, offsets, l_aux.  Thread e owns expert e (E <= FIN_THREADS).  cnt: [k][E] totals (global or
+// LDS), replaced by base(choice, expert), the rows of the expert's earlier choices; me: the column sum of the scores of
+// the thread's expert.  Returns the capacity; s_off[e] = first row of expert e.
+__device__ __forceinline__ int finish_counts(const RouteEnd &r, int *cnt, float me, int *s_off, int *s16) {
+    const int e = threadIdx.x, E = r.E;
+    int tot = 0, first = 0;
+    if (e < E) {
+        for (int j = 0; j < r.k; ++j) {
+            const int c = cnt[j * E + e];
+            if (j == 0) first = c;
+            r.counts[j * E + e] = c;
+            cnt[j * E + e] = tot;
+            tot += c;
         }
-        if (tid == P - 1) offsets[E] = s_red[tid];
+    }
+    int cap = r.cap_bound;
+    if (r.cf_sign <= 0) {              // uniform: the largest load, which only capacity factors <= 0 ask for
+        cap = block_max(tot, s16);
+        if (r.cf_sign < 0) cap = min(cap, r.cap_bound);
+    }
+    const int rem = cap % r.alignment;
+    if (rem > 0) cap += r.alignment - rem;
+    const int n = min(tot, cap);
+    if (e < E) r.kept_rows[e] = n;
+    if (r.layout == MOLE_LAYOUT_RAGGED) {
+        const int incl = block_inclusive(n, s16);
+        if (e < E) { r.offsets[e] = incl - n; s_off[e] = incl - n; }
+        if (e == E - 1) r.offsets[E] = incl;
     } else {
-        for (int e = lo; e < hi; ++e) offsets[e] = e * cap;
-        if (tid == 0) offsets[E] = E * cap;
+        if (e < E) { r.offsets[e] = e * cap; s_off[e] = e * cap; }
+        if (e == 0) r.offsets[E] = E * cap;
     }
-    if (tid == 0) capacity[0] = cap;
+    if (e == 0) r.capacity[0] = cap;
+    if (r.l_aux != nullptr) {          // uniform over the grid
+        const float sum = block_sum(e < E ? me * (float)first : 0.f, (float *)s16);
+        if (e == 0) r.l_aux[0] = r.S > 0 ? sum * ((float)E / ((float)r.S * (float)r.S)) : 0.f;
+    }
+    __syncthreads();
+    return cap;
+}
 
-    if (l_aux != nullptr) {
-        // me[e] = sum over blocks of the partial column sums, in a fixed order: thread (g, e) adds
-        // blocks g, g+groups, ...; thread e then adds the groups in order
-        __syncthreads();
-        const int groups = FIN_THREADS / E > 0 ? FIN_THREADS / E : 1;
-        if (tid < groups * E && E <= FIN_THREADS) {
+// One block.  scan_hist == NULL: counts holds the totals already (route_scan ran).  Otherwise the block scans the
+// histograms itself: a thread per (choice, expert) where few blocks of tokens were counted (all its loads are in
+// flight at once), a wave per pair otherwise.  last: it also writes locations and rows (small problems: a launch less).
+// (256 experts, top-8, 256 tokens: 2048 pairs of four counts took a wave each and 197 us; by threads, last stage
+// included, 15 us.)
+constexpr int FIN_FEW = 32;            // blocks of tokens up to which a thread scans a pair on its own
+__global__ __launch_bounds__(FIN_THREADS) void route_finish_kernel(const RouteEnd r, const float *__restrict__ colsum, int nb_col,
+                                                                   int32_t *__restrict__ basej, int32_t *scan_hist, int nb, int bt,
+                                                                   int last) {
+    __shared__ int s_off[FIN_THREADS];
+    __shared__ int s16[FIN_THREADS / WAVE];
+    __shared__ float s_fred[FIN_THREADS];
+    const int tid = threadIdx.x, E = r.E, npairs = r.k * E;
+    // column sums of the scores: thread (g, e) adds blocks g, g + groups, ... in order, thread e then the groups in order
+    float me = 0.f;
+    if (r.l_aux != nullptr) {
+        const int groups = FIN_THREADS / E;
+        if (tid < groups * E) {
             const int e = tid % E, gq = tid / E;
-            float me = 0.f;
-            for (int b0 = gq; b0 < nb; b0 += 8 * groups) {       // 8 loads in flight, added in block order
+            for (int b0 = gq; b0 < nb_col; b0 += 8 * groups) {
                 float t[8];
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
                     const int b = b0 + u * groups;
-                    t[u] = load_or_zero(colsum + (size_t)min(b, nb - 1) * E + e, b < nb);
+                    t[u] = load_or_zero(colsum + (size_t)min(b, nb_col - 1) * E + e, b < nb_col);
                 }
 #pragma unroll
                 for (int u = 0; u < 8; ++u)
-                    if (b0 + u * groups < nb) me += t[u];
+                    if (b0 + u * groups < nb_col) me += t[u];
             }
-            s_fred[tid] = me;
         }
-        __syncthreads();
-        float acc = 0.f;
-        if (tid < E) {
-            float me = 0.f;
-            for (int gq = 0; gq < groups; ++gq) me += s_fred[gq * E + tid];
-            acc = me * (float)counts[tid];
+        s_fred[tid] = me;
+    }
+    if (scan_hist != nullptr) {
+        if (nb <= FIN_FEW) {
+            for (int pair = tid; pair < npairs; pair += FIN_THREADS) {
+                int32_t *h = scan_hist + (size_t)pair * nb;
+                int carry = 0;
+                for (int b0 = 0; b0 < nb; b0 += 8) {
+                    int v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = load_or_zero(h + min(b0 + u, nb - 1), b0 + u < nb);
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (b0 + u < nb) { h[b0 + u] = carry; carry += v[u]; }
+                }
+                basej[pair] = carry;
+            }
+        } else {
+            for (int pair = tid >> 6; pair < npairs; pair += FIN_THREADS / 64) scan_pair(scan_hist, nb, pair, basej);
         }
-        __syncthreads();
-        s_fred[tid] = acc;
-        __syncthreads();
-        for (int d = P / 2; d >= 1; d >>= 1) {
-            if (tid < d) s_fred[tid] += s_fred[tid + d];
-            __syncthreads();
-        }
-        if (tid == 0) l_aux[0] = S > 0 ? s_fred[0] * ((float)E / ((float)S * (float)S)) : 0.f;
+    } else {
+        for (int pair = tid; pair < npairs; pair += FIN_THREADS) basej[pair] = r.counts[pair];
+    }
+    __threadfence_block();
+    __syncthreads();
+    if (r.l_aux != nullptr && tid < E) {
+        const int groups = FIN_THREADS / E;
+        me = s_fred[tid];
+        for (int gq = 1; gq < groups; ++gq) me += s_fred[gq * E + tid];
+    }
+    const int cap = finish_counts(r, basej, me, s_off, s16);
+    if (!last) return;
+    __threadfence_block();
+    for (int p = tid; p < r.k * r.S; p += FIN_THREADS) {
+        const int j = p / r.S, i = p % r.S;
+        const int e = r.idx[p];
+        const int l = basej[j * E + e] + scan_hist[((size_t)j * E + e) * nb + i / bt] + r.loc[p];
+        r.loc[p] = l;
+        r.row[p] = l < cap ? s_off[e] + l : -1;
     }
 }
 
@@ -394,6 +362,165 @@ __global__ __launch_bounds__(256) void route_finalize_kernel(
     row[p] = l < capacity[0] ? offsets[e] + l : -1;
 }
 
+// ---- the tokens' own part ------------------------------------------------------------------------------------------
+// 64 tokens per block of 16 waves.  2^LOGG lanes own a token and hold VPL scores each (lane g: experts g, g + G, ...); with
+// 16 lanes per token all 64 tokens go through their rounds at once.  (Four waves on 64 tokens, 16 tokens a wave, four at a
+// time, spent four times the latency of a round: 256 experts, top-8: 42 us for 256 tokens and 58 for 32768, now 9 and 27.)
+// logits != 0: `in` holds logits (without bias if one is given) and the block starts with the softmax (the sums in the order of gate_fwd_kernel's), writing
+// scores.  nb == 1: the block has seen all tokens and goes on to the end of the routing by itself.
+template <int VPL, int LOGG>
+__global__ __launch_bounds__(FIN_THREADS) void route_tokens_kernel(const float *__restrict__ in, const float *__restrict__ bias,
+                                                                   int logits, int normalize,
+                                                                   float *__restrict__ scores, float *__restrict__ gates,
+                                                                   int32_t *__restrict__ hist /* [k][E][nb] */,
+                                                                   float *__restrict__ colsum /* [nb][E] */, int nb, const RouteEnd r) {
+    constexpr int G = 1 << LOGG, TPP = FIN_THREADS >> LOGG, PASSES = RT_TOKENS > TPP ? RT_TOKENS / TPP : 1;
+    constexpr int WAVES = FIN_THREADS / WAVE;
+    extern __shared__ __align__(16) char smem[];
+    const int S = r.S, E = r.E, k = r.k;
+    int *s_idx = (int *)smem;                          // [k][64]
+    float *s_graw = (float *)(s_idx + k * RT_TOKENS);  // [k][64]
+    int *s_hist = (int *)(s_graw + k * RT_TOKENS);     // [k][E]
+    float *s_col = (float *)(s_hist + k * E);          // [16][E]
+    __shared__ int s_off[FIN_THREADS];
+    __shared__ int s16[WAVES];
+
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int b = blockIdx.x, tok0 = b * RT_TOKENS;
+    const int g = lane & (G - 1);
+    for (int i = tid; i < k * E; i += FIN_THREADS) s_hist[i] = 0;
+    float colacc[VPL];
+#pragma unroll
+    for (int q = 0; q < VPL; ++q) colacc[q] = 0.f;
+    for (int pass = 0; pass < PASSES; ++pass) {
+        const int tl = pass * TPP + (tid >> LOGG);
+        const int token = tok0 + tl;
+        const bool tv = tl < RT_TOKENS && token < S;
+        float v[VPL];
+#pragma unroll
+        for (int q = 0; q < VPL; ++q) v[q] = 0.f;
+        if (S > 0) {
+#pragma unroll
+            for (int q = 0; q < VPL; ++q) v[q] = in[(size_t)min(token, S - 1) * E + min(g + (q << LOGG), E - 1)];
+        }
+        if (logits) {
+            float mx = -INFINITY;
+#pragma unroll
+            for (int q = 0; q < VPL; ++q) {
+                if (bias) v[q] += bias[min(g + (q << LOGG), E - 1)];
+                v[q] = g + (q << LOGG) < E ? v[q] : -INFINITY;
+                mx = fmaxf(mx, v[q]);
+            }
+            for (int m = G / 2; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, WAVE));
+            float sum = 0.f;
+#pragma unroll
+            for (int q = 0; q < VPL; ++q) v[q] = g + (q << LOGG) < E ? expf(v[q] - mx) : 0.f;
+            // the sums of the kernels that do the softmax alone, term for term: up to 64 experts gate_fwd_kernel's, beyond
+            // softmax_fwd_kernel's, whose wave holds experts l, l + 64, .. in lane l (four of them are lane g's here)
+            if constexpr (LOGG == 4 && VPL > 4) {
+                float part[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    part[c] = 0.f;
+#pragma unroll
+                    for (int q = c; q < VPL; q += 4) part[c] += v[q];
+                    part[c] = group_reduce(part[c], 4, [](float a, float d) { return a + d; });
+                }
+                sum = (part[0] + part[1]) + (part[2] + part[3]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < VPL; ++q) sum += v[q];
+                if constexpr (LOGG == 4) {
+                    for (int m = 8; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, WAVE);
+                } else {
+                    sum = group_reduce(sum, LOGG, [](float a, float d) { return a + d; });
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < VPL; ++q) {
+                const int e = g + (q << LOGG);
+                v[q] = v[q] / sum;
+                if (tv && e < E) scores[(size_t)token * E + e] = v[q];
+            }
+        }
+        uint32_t key[VPL];
+#pragma unroll
+        for (int q = 0; q < VPL; ++q) {
+            const bool ok = tv && g + (q << LOGG) < E;
+            const float sv = __uint_as_float(__float_as_uint(v[q]) & (ok ? 0xffffffffu : 0u));
+            colacc[q] += sv;
+            key[q] = ok ? topk_key(sv) : 0u;
+        }
+        for (int j = 0; j < k; ++j) {
+            // the best score of the token, then the lowest expert index among those that hold it
+            uint32_t best = key[0];
+#pragma unroll
+            for (int q = 1; q < VPL; ++q) best = max(best, key[q]);
+            const uint32_t top = group_reduce(best, LOGG, [](uint32_t a, uint32_t c) { return max(a, c); });
+            int cand = INT_MAX;
+#pragma unroll
+            for (int q = VPL - 1; q >= 0; --q)
+                if (key[q] == top) cand = g + (q << LOGG);             // ends on the lane's lowest such expert
+            if (top == 0u) cand = INT_MAX;                             // nothing available (a token past the end)
+            const int bi = group_reduce(cand, LOGG, [](int a, int c) { return min(a, c); });
+            const bool mine = bi != INT_MAX && (bi & (G - 1)) == g;
+#pragma unroll
+            for (int q = 0; q < VPL; ++q)
+                if (mine && (bi >> LOGG) == q) key[q] = 0u;
+            if (g == 0 && tv) {
+                s_idx[j * RT_TOKENS + tl] = bi;
+                s_graw[j * RT_TOKENS + tl] = topk_unkey(top);
+            }
+        }
+    }
+    // column sums of the scores (for l_aux): the tokens of a wave, then (below) the waves in order
+#pragma unroll
+    for (int q = 0; q < VPL; ++q) {
+        float c = colacc[q];
+        for (int m = G; m < WAVE; m <<= 1) c += __shfl_xor(c, m, WAVE);
+        const int e = g + (q << LOGG);
+        if (lane < G && e < E) s_col[w * E + e] = c;
+    }
+    __syncthreads();
+    float me = 0.f;
+    if (tid < E) {
+        for (int q = 0; q < WAVES; ++q) me += s_col[q * E + tid];
+        if (nb > 1) colsum[(size_t)b * E + tid] = me;
+    }
+    // gate values and indices out: thread t < 64 is token t
+    if (tid < RT_TOKENS && tok0 + tid < S) {
+        float denom = 0.f;
+        for (int j = 0; j < k; ++j) denom += s_graw[j * RT_TOKENS + tid];  // left to right, fp32
+        const float den = denom < FP32_EPS ? FP32_EPS : denom;
+        for (int j = 0; j < k; ++j) {
+            float gv = s_graw[j * RT_TOKENS + tid];
+            if (k > 1 && normalize) gv = gv / den;
+            gates[(size_t)j * S + tok0 + tid] = gv;
+            r.idx[(size_t)j * S + tok0 + tid] = s_idx[j * RT_TOKENS + tid];
+        }
+    }
+    // in-block ranks: wave j ranks choice j (k <= 16 = the number of waves), lane = token
+    const int token = tok0 + lane;
+    const bool cv = w < k && token < S;
+    const int my_e = cv ? s_idx[w * RT_TOKENS + lane] : 0;
+    int same;
+    const int rank = rank_in_wave(my_e, cv, E, same);
+    if (cv && rank == 0) s_hist[w * E + my_e] = same;
+    if (nb > 1) {
+        if (cv) r.loc[(size_t)w * S + token] = rank;
+        if (w < k)                     // written and read by this wave: program order is enough
+            for (int e = lane; e < E; e += WAVE) hist[((size_t)w * E + e) * nb + b] = s_hist[w * E + e];
+        return;
+    }
+    __syncthreads();
+    const int cap = finish_counts(r, s_hist, me, s_off, s16);
+    if (cv) {
+        const int l = s_hist[w * E + my_e] + rank;
+        r.loc[(size_t)w * S + token] = l;
+        r.row[(size_t)w * S + token] = l < cap ? s_off[my_e] + l : -1;
+    }
+}
+
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 }  // namespace mole
@@ -407,60 +534,79 @@ extern "C" size_t mole_route_workspace_bytes(int S, int E, int k) {
            align256(nb * E * sizeof(float)) + align256((size_t)COLSUM_SLICES * E * sizeof(float));
 }
 
-// Lanes per token (as a power of two) of the kernels that give a group of lanes a token's E values, each lane holding
-// E / lanes of them: 16 lanes at most, more only where a lane would otherwise hold more than 16 values.  A group's
-// reductions act on all the wave's groups at once, so in the top-k, whose rounds are chains of reductions, small groups
-// with many values per lane cost fewer instructions per token than the whole wave on one token (top-8 of 256 scores for 32768 tokens: 106 us with 64 lanes per token,
-// 83 with 32, 72 with 16; top-2 of 64 for 8192: 33.6 / 29.5 / 25.8 us).
-static int lane_group_log2(int E) {
-    int logG = 0;
-    while ((1 << logG) < E && logG < 4) ++logG;
-    while (ceil_div(E, 1 << logG) > 16 && logG < 6) ++logG;
-    return logG;
-}
-
-// The stages of the routing behind the per-block top-k: scan of the histograms over blocks, counts / capacity /
-// offsets / l_aux, then locations and destination rows.  bt: tokens per histogram block.
-static int route_after_topk(int32_t *hist, int32_t *basej, float *colsum, float *colpart, int nb, int bt, int S, int E, int k,
-                            double capacity_factor, int alignment, int layout, const int32_t *idx, int32_t *loc,
-                            int32_t *row, int32_t *counts, int32_t *kept_rows, int32_t *offsets, int32_t *capacity,
-                            float *l_aux, hipStream_t st) {
-    const int npairs = k * E;
-    const bool scan_in_finish = (long long)npairs * nb <= 8192;    // small enough for one block: saves a launch
+// The stages of the routing behind the tokens' own: scan of the histograms over blocks, counts / capacity / offsets /
+// l_aux, then locations and destination rows.  nb blocks of bt tokens each were counted.
+static int route_after_topk(const RouteEnd &r, int32_t *hist, int32_t *basej, float *colsum, float *colpart, int nb, int bt,
+                            hipStream_t st) {
+    const int npairs = r.k * r.E;
+    // small enough for the finishing block (saves a launch): a thread per pair up to FIN_FEW blocks of tokens and 2^16
+    // counts, a wave per pair up to 2^13 counts
+    const bool scan_in_finish = (long long)npairs * nb <= (nb <= FIN_FEW ? 65536 : 8192);
+    const bool last_in_finish = scan_in_finish && (long long)r.k * r.S <= 4 * FIN_THREADS;
     if (!scan_in_finish) {
         const int scan_blocks = ceil_div(npairs, 4);
-        hipLaunchKernelGGL(route_scan_kernel, dim3(scan_blocks + COLSUM_SLICES * ceil_div(E, 256)), dim3(256), 0, st, hist,
-                           nb, npairs, counts, scan_blocks, colsum, E, colpart);
+        hipLaunchKernelGGL(route_scan_kernel, dim3(scan_blocks + COLSUM_SLICES * ceil_div(r.E, 256)), dim3(256), 0, st, hist,
+                           nb, npairs, r.counts, scan_blocks, colsum, r.E, colpart);
         MOLE_LAUNCH_CHECK();
     }
-
-    const int spe = (S + E - 1) / E;
-    const int cf_sign = capacity_factor > 0. ? 1 : (capacity_factor < 0. ? -1 : 0);
-    // int(cf * spe) of the Python reference: the product is taken in double precision
-    const double prod = (capacity_factor < 0. ? -capacity_factor : capacity_factor) * (double)spe;
-    const int cap_bound = k * (int)prod;
     // (when the scan kernel ran, it also folded the column sums: the finish then adds its COLSUM_SLICES rows)
-    hipLaunchKernelGGL(route_finish_kernel, dim3(1), dim3(FIN_THREADS), 0, st, counts,
-                       scan_in_finish ? colsum : colpart, scan_in_finish ? nb : min(nb, COLSUM_SLICES), S, E, k, cf_sign,
-                       cap_bound, alignment, layout, basej, kept_rows, offsets, capacity, l_aux,
-                       scan_in_finish ? hist : (int32_t *)nullptr);
+    hipLaunchKernelGGL(route_finish_kernel, dim3(1), dim3(FIN_THREADS), 0, st, r, scan_in_finish ? colsum : colpart,
+                       scan_in_finish ? nb : min(nb, COLSUM_SLICES), basej, scan_in_finish ? hist : (int32_t *)nullptr, nb, bt,
+                       (int)last_in_finish);
     MOLE_LAUNCH_CHECK();
-
-    if (S > 0) {
-        const size_t n = (size_t)k * S;
-        hipLaunchKernelGGL(route_finalize_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, idx, hist,
-                           basej, offsets, capacity, S, E, k, nb, bt, loc, row);
+    if (r.S > 0 && !last_in_finish) {
+        const size_t n = (size_t)r.k * r.S;
+        hipLaunchKernelGGL(route_finalize_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, r.idx, hist,
+                           basej, r.offsets, r.capacity, r.S, r.E, r.k, nb, bt, r.loc, r.row);
         MOLE_LAUNCH_CHECK();
     }
     return 0;
 }
 
-template <int VPL>
-static void launch_topk(const float *scores, int S, int E, int k, int logG, int normalize, int32_t *idx,
-                        int32_t *loc, float *gates, int32_t *hist, float *colsum, int nb, hipStream_t st) {
-    const size_t lds = (size_t)k * RT_TOKENS * 8 + (size_t)E * 4 * 4 + (size_t)E * 4 * 4;
-    hipLaunchKernelGGL(route_topk_kernel<VPL>, dim3(nb), dim3(RT_THREADS), lds, st, scores, S, E, k, logG,
-                       normalize, idx, loc, gates, hist, colsum, nb);
+static RouteEnd route_end(int S, int E, int k, double capacity_factor, int alignment, int layout, int32_t *idx, int32_t *loc,
+                          int32_t *row, int32_t *counts, int32_t *kept_rows, int32_t *offsets, int32_t *capacity, float *l_aux) {
+    const int spe = (S + E - 1) / E;
+    const int cf_sign = capacity_factor > 0. ? 1 : (capacity_factor < 0. ? -1 : 0);
+    // int(cf * spe) of the Python reference: the product is taken in double precision
+    const double prod = (capacity_factor < 0. ? -capacity_factor : capacity_factor) * (double)spe;
+    return RouteEnd{S, E, k, cf_sign, k * (int)prod, alignment, layout, counts, kept_rows, offsets, capacity, l_aux, idx, loc, row};
+}
+
+template <int VPL, int LOGG>
+static int launch_tokens(const float *in, const float *bias, int logits, int normalize, float *scores, float *gates, int32_t *hist, float *colsum,
+                         int nb, const RouteEnd &r, hipStream_t st) {
+    const size_t lds = (size_t)r.k * RT_TOKENS * 8 + (size_t)r.k * r.E * 4 + (size_t)(FIN_THREADS / WAVE) * r.E * 4;
+    auto kern = route_tokens_kernel<VPL, LOGG>;
+    if (lds > 48 * 1024)               // hundreds of experts and a long top-k: beyond the default limit together with the static part
+        MOLE_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kern, dim3(nb), dim3(FIN_THREADS), lds, st, in, bias, logits, normalize, scores, gates, hist, colsum, nb, r);
+    MOLE_LAUNCH_CHECK();
+    return 0;
+}
+
+// The whole routing of scores (or of logits, to which bias is added if given and whose softmax then goes to `scores`).
+static int route_from(const float *in, const float *bias, int logits, int normalize, float *scores, float *gates, const RouteEnd &r, void *workspace,
+                      hipStream_t st) {
+    const int nb = ceil_div(r.S > 0 ? r.S : 1, RT_TOKENS);
+    char *ws = (char *)workspace;
+    int32_t *hist = (int32_t *)ws;
+    ws += align256((size_t)nb * r.k * r.E * sizeof(int32_t));
+    int32_t *basej = (int32_t *)ws;
+    ws += align256((size_t)r.k * r.E * sizeof(int32_t));
+    float *colsum = (float *)ws;
+    ws += align256((size_t)nb * r.E * sizeof(float));
+    float *colpart = (float *)ws;
+    // 16 lanes per token; beyond 256 experts a lane would hold more than 16 values, so the whole wave takes a token
+    const int vpl = ceil_div(r.E, 16);
+    int rc;
+    if (vpl <= 1) rc = launch_tokens<1, 4>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
+    else if (vpl <= 2) rc = launch_tokens<2, 4>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
+    else if (vpl <= 4) rc = launch_tokens<4, 4>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
+    else if (vpl <= 8) rc = launch_tokens<8, 4>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
+    else if (vpl <= 16) rc = launch_tokens<16, 4>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
+    else rc = launch_tokens<16, 6>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
+    if (rc || nb == 1) return rc;
+    return route_after_topk(r, hist, basej, colsum, colpart, nb, RT_TOKENS, st);
 }
 
 extern "C" int mole_route(const float *scores, int S, int E, int k, double capacity_factor, int normalize_gate,
@@ -482,27 +628,8 @@ extern "C" int mole_route(const float *scores, int S, int E, int k, double capac
     }
     hipStream_t st = (hipStream_t)stream;
     ScopedTiming timing(MOLE_K_ROUTE, st);
-    const int nb = ceil_div(S > 0 ? S : 1, RT_TOKENS);
-    char *ws = (char *)workspace;
-    int32_t *hist = (int32_t *)ws;
-    ws += align256((size_t)nb * k * E * sizeof(int32_t));
-    int32_t *basej = (int32_t *)ws;
-    ws += align256((size_t)k * E * sizeof(int32_t));
-    float *colsum = (float *)ws;
-    ws += align256((size_t)nb * E * sizeof(float));
-    float *colpart = (float *)ws;
-
-    const int logG = lane_group_log2(E);
-    const int vpl = ceil_div(E, 1 << logG);
-    if (vpl <= 1) launch_topk<1>(scores, S, E, k, logG, normalize_gate, idx, loc, gates, hist, colsum, nb, st);
-    else if (vpl <= 2) launch_topk<2>(scores, S, E, k, logG, normalize_gate, idx, loc, gates, hist, colsum, nb, st);
-    else if (vpl <= 4) launch_topk<4>(scores, S, E, k, logG, normalize_gate, idx, loc, gates, hist, colsum, nb, st);
-    else if (vpl <= 8) launch_topk<8>(scores, S, E, k, logG, normalize_gate, idx, loc, gates, hist, colsum, nb, st);
-    else launch_topk<16>(scores, S, E, k, logG, normalize_gate, idx, loc, gates, hist, colsum, nb, st);
-    MOLE_LAUNCH_CHECK();
-
-    return route_after_topk(hist, basej, colsum, colpart, nb, RT_TOKENS, S, E, k, capacity_factor, alignment, layout, idx, loc,
-                            row, counts, kept_rows, offsets, capacity, l_aux, st);
+    const RouteEnd r = route_end(S, E, k, capacity_factor, alignment, layout, idx, loc, row, counts, kept_rows, offsets, capacity, l_aux);
+    return route_from(scores, nullptr, 0, normalize_gate, nullptr, gates, r, workspace, st);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -562,7 +689,7 @@ extern "C" int mole_route_static(const float *scores, int S, int E, int k, doubl
 // ---------------------------------------------------------------------------------------------
 namespace mole {
 
-// One group of G lanes per token (same mapping as route_topk), VPL values per lane.
+// One group of G lanes per token, VPL values per lane.
 template <int VPL>
 __global__ __launch_bounds__(256) void softmax_fwd_kernel(const float *__restrict__ logits,
                                                           const float *__restrict__ bias, int S, int E, int logG,
@@ -760,7 +887,7 @@ typedef float gate_f32x4 __attribute__((ext_vector_type(4)));
 // fall into distinct banks).  A wave stages and reads its own rows only.
 // ROUTE: the block goes on to the first stage of the routing for its 16 TG tokens - top-k, gate values, in-block
 // ranks and per-expert histograms, the block's column sums for l_aux - while a token's scores are still in the 16
-// lanes that formed them (the layout route_topk_kernel works in: lane j of the group holds experts j, 16 + j, ...).
+// lanes that formed them (the layout route_tokens_kernel works in: lane j of the group holds experts j, 16 + j, ...).
 // The scores are written out as well (the backward needs them) but not read back: one kernel and 4 S E bytes less.
 struct GateRoute {
     int k, normalize, nb;
@@ -913,7 +1040,7 @@ __global__ __launch_bounds__(256) void gate_fwd_kernel(const bf16_t *__restrict_
             if (token < S && e < E) scores[(size_t)token * E + e] = v[g];
         }
         if constexpr (ROUTE) {
-            // the k rounds of route_topk_kernel on the token's scores (the same keys, the same tie rule)
+            // the k rounds of route_tokens_kernel on the token's scores (the same keys, the same tie rule)
             uint32_t key[EG];
 #pragma unroll
             for (int g = 0; g < EG; ++g) {
@@ -959,6 +1086,84 @@ __global__ __launch_bounds__(256) void gate_fwd_kernel(const bf16_t *__restrict_
     }
 }
 
+// ---- logits alone, for few tokens ------------------------------------------------------------------------------------
+// A block owns 16 TG tokens x 16 experts; its four waves take a quarter of the model dimension each, in the order of
+// gate_fwd_kernel (whose logits these equal bit for bit where it applies: bf16, M a multiple of 128).  One block per
+// 16-expert group instead of one that reads all of Wg: 512 KB of Wg for one token is then 4 blocks' work side by side
+// instead of one block's 20 us, and 256 tokens x 256 experts x 2048 are 256 blocks (10 us; one 256 x 256 tile: 54).
+// Fragments come straight from memory; k past the end is masked to zero on the token side.
+template <typename T, int TG>
+__global__ __launch_bounds__(256) void gate_logits_kernel(const T *__restrict__ x, const float *__restrict__ wg,
+                                                          const float *__restrict__ bias, int S, int E, int M,
+                                                          float *__restrict__ logits) {
+    constexpr int EPC = 16 / sizeof(T), KSTEP = 4 * EPC, U = TG == 1 ? 8 : 4;
+    __shared__ float part[4][16 * TG][17];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, kq = lane >> 4;
+    const int tok0 = blockIdx.x * 16 * TG, e0 = blockIdx.y * 16;
+    const int steps = (M + KSTEP - 1) / KSTEP, s_lo = wave * steps / 4, s_hi = (wave + 1) * steps / 4;
+    const T *xp[TG];
+#pragma unroll
+    for (int t = 0; t < TG; ++t) xp[t] = x + (size_t)min(tok0 + 16 * t + r16, S - 1) * M;
+    const float *wp = wg + (size_t)min(e0 + r16, E - 1) * M;
+    gate_f32x4 acc[TG];
+#pragma unroll
+    for (int t = 0; t < TG; ++t) acc[t] = gate_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = s_lo; s < s_hi; s += U) {
+        uint4 a[TG][U];
+        float4 w[U][EPC / 4];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = min(min(s + u, s_hi - 1) * KSTEP + kq * EPC, M - EPC);
+#pragma unroll
+            for (int t = 0; t < TG; ++t) a[t][u] = *reinterpret_cast<const uint4 *>(xp[t] + k);
+#pragma unroll
+            for (int h = 0; h < EPC / 4; ++h) w[u][h] = *reinterpret_cast<const float4 *>(wp + k + 4 * h);
+        }
+        __builtin_amdgcn_sched_barrier(0);       // all loads of the round first
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t keep = (s + u < s_hi && (s + u) * KSTEP + kq * EPC < M) ? 0xffffffffu : 0u;
+#pragma unroll
+            for (int t = 0; t < TG; ++t) {
+                const uint4 v = make_uint4(a[t][u].x & keep, a[t][u].y & keep, a[t][u].z & keep, a[t][u].w & keep);
+                if constexpr (sizeof(T) == 2) {
+                    const float4 w0 = w[u][0], w1 = w[u][EPC / 4 - 1];
+                    const gate_bf16x8 b = {(bf16_t)w0.x, (bf16_t)w0.y, (bf16_t)w0.z, (bf16_t)w0.w,
+                                           (bf16_t)w1.x, (bf16_t)w1.y, (bf16_t)w1.z, (bf16_t)w1.w};
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gate_bf16x8, v), b, acc[t], 0, 0, 0);
+                } else {
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.x), w[u][0].x, acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.y), w[u][0].y, acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.z), w[u][0].z, acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.w), w[u][0].w, acc[t], 0, 0, 0);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < TG; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[wave][16 * t + 4 * kq + r][r16] = acc[t][r];
+    __syncthreads();
+    const int e = e0 + (threadIdx.x & 15);
+#pragma unroll
+    for (int t = 0; t < TG; ++t) {
+        const int tl = 16 * t + (threadIdx.x >> 4);
+        if (tok0 + tl < S && e < E)
+            logits[(size_t)(tok0 + tl) * E + e] = part[0][tl][e - e0] + part[1][tl][e - e0] + part[2][tl][e - e0] + part[3][tl][e - e0] + (bias ? bias[e] : 0.f);
+    }
+}
+
+// Wg in the operand type of the GEMM path
+__global__ __launch_bounds__(256) void f32_to_bf16_kernel(const float *__restrict__ in, bf16_t *__restrict__ out, size_t n4) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    const float4 v = reinterpret_cast<const float4 *>(in)[i];
+    typedef __bf16 bf16x4_ __attribute__((ext_vector_type(4)));
+    reinterpret_cast<uint2 *>(out)[i] = __builtin_bit_cast(uint2, bf16x4_{(bf16_t)v.x, (bf16_t)v.y, (bf16_t)v.z, (bf16_t)v.w});
+}
+
 }  // namespace mole
 
 #define MOLE_VPL_DISPATCH(vpl, KERNEL, grid, st, ...)                                              \
@@ -991,11 +1196,35 @@ static constexpr unsigned GATE_STAGE_LDS = 4 * 32 * (4 * 64 + 16);
 // tokens per block of the fused gate + routing kernels (TG = 2)
 static constexpr int GATE_ROUTE_TOKENS = 32;
 
-extern "C" size_t mole_gate_route_workspace_bytes(int S, int E, int k) {
-    if (S < 0 || E <= 0 || k <= 0) return 0;
+static size_t gate_route_fused_bytes(int S, int E, int k) {
     const size_t nb = (size_t)ceil_div(S > 0 ? S : 1, GATE_ROUTE_TOKENS);
     return align256(nb * k * E * sizeof(int32_t)) + align256((size_t)k * E * sizeof(int32_t)) +
            align256(nb * E * sizeof(float)) + align256((size_t)COLSUM_SLICES * E * sizeof(float));
+}
+
+// How the gate and the routing of a call run.
+//   FUSED   the gate kernel does the tokens' part of the routing as well: bf16, gates of up to 64 experts, many tokens
+//           (a block of 32 tokens reads all of Wg, so with few tokens few blocks read it one after the other:
+//           1 token, 64 experts of 2048: 21 + 17 + 4 us in three kernels against 4 + 7 us)
+//   FEW     logits by 16 x 16 tiles, then softmax and routing: up to 2048 tokens (2048 blocks at 256 experts; beyond, the
+//           re-reads of x and Wg by the tiles cost more than the GEMM's tiles)
+//   SCORES  fp32, up to 32 experts: mole_gate_fwd's wave per token, then the routing of the scores
+//   GEMM    logits on the grouped-GEMM tiles, then softmax and routing
+enum { GR_FUSED, GR_FEW, GR_SCORES, GR_GEMM };
+static int gate_route_path(int dtype, int S, int E, int M) {
+    if (dtype == MOLE_BF16 && M % 128 == 0 && E <= 64 && S > RT_TOKENS) return GR_FUSED;
+    if (S <= 2048) return GR_FEW;
+    return dtype == MOLE_F32 && E <= 32 ? GR_SCORES : GR_GEMM;
+}
+
+extern "C" size_t mole_gate_route_workspace_bytes(int dtype, int S, int E, int M, int k) {
+    if (S < 0 || E <= 0 || M <= 0 || k <= 0) return 0;
+    const int path = gate_route_path(dtype, S, E, M);
+    if (path == GR_FUSED) return gate_route_fused_bytes(S, E, k);
+    size_t n = mole_route_workspace_bytes(S, E, k);
+    if (path != GR_SCORES) n += align256((size_t)S * E * sizeof(float));
+    if (path == GR_GEMM && dtype == MOLE_BF16) n += align256((size_t)E * M * sizeof(bf16_t));
+    return n;
 }
 
 extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M,
@@ -1003,22 +1232,60 @@ extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const 
                                int32_t *idx, int32_t *loc, float *gates, int32_t *row, int32_t *counts,
                                int32_t *kept_rows, int32_t *offsets, int32_t *capacity, float *l_aux, void *workspace,
                                size_t workspace_bytes, mole_stream_t stream) {
-    MOLE_REQUIRE(dtype == MOLE_BF16 && S >= 1 && E >= 1 && E <= 64 && M >= 128 && M % 128 == 0,
-                 "mole_gate_route: needs bf16 tokens, M a multiple of 128 and at most 64 experts (S=%d E=%d M=%d dtype=%d); "
-                 "other shapes: mole_gate_fwd (or mole_gemm_nt + mole_softmax_fwd), then mole_route", S, E, M, dtype);
+    MOLE_REQUIRE(dtype == MOLE_BF16 || dtype == MOLE_F32, "mole_gate_route: bad dtype %d", dtype);
+    const int epc = dtype == MOLE_BF16 ? 8 : 4;
+    MOLE_REQUIRE(S >= 1 && E >= 1 && E <= MOLE_MAX_EXPERTS && M >= epc && M % epc == 0,
+                 "mole_gate_route: needs S >= 1, 1 <= E <= %d and M a multiple of %d (S=%d E=%d M=%d dtype=%d)", MOLE_MAX_EXPERTS,
+                 epc, S, E, M, dtype);
     MOLE_REQUIRE(k >= 1 && k <= MOLE_MAX_TOPK && k <= E, "mole_gate_route: need 1 <= k <= min(E, %d) (k=%d E=%d)", MOLE_MAX_TOPK, k, E);
     MOLE_REQUIRE(alignment >= 1, "mole_gate_route: alignment must be >= 1");
     MOLE_REQUIRE(layout == MOLE_LAYOUT_PADDED || layout == MOLE_LAYOUT_RAGGED, "mole_gate_route: bad layout %d", layout);
     MOLE_REQUIRE(x && wg && scores && idx && loc && gates && row && counts && kept_rows && offsets && capacity && workspace,
                  "mole_gate_route: null pointer");
+    MOLE_REQUIRE((((uintptr_t)x | (uintptr_t)wg) & 15) == 0, "mole_gate_route: x and wg must be 16-byte aligned");
     MOLE_REQUIRE((long long)S * k < INT_MAX, "mole_gate_route: S*k too large");
-    if (workspace_bytes < mole_gate_route_workspace_bytes(S, E, k)) {
-        set_error("mole_gate_route: workspace of %zu bytes, need %zu", workspace_bytes, mole_gate_route_workspace_bytes(S, E, k));
+    const size_t need = mole_gate_route_workspace_bytes(dtype, S, E, M, k);
+    if (workspace_bytes < need) {
+        set_error("mole_gate_route: workspace of %zu bytes, need %zu", workspace_bytes, need);
         return MOLE_E_WORKSPACE;
     }
     hipStream_t st = (hipStream_t)stream;
-    const int nb = ceil_div(S, GATE_ROUTE_TOKENS);
+    const RouteEnd r = route_end(S, E, k, capacity_factor, alignment, layout, idx, loc, row, counts, kept_rows, offsets, capacity, l_aux);
+    const int path = gate_route_path(dtype, S, E, M);
     char *ws = (char *)workspace;
+    if (path != GR_FUSED) {
+        void *route_ws = ws;
+        ws += mole_route_workspace_bytes(S, E, k);
+        if (path == GR_SCORES) {
+            if (int rc = mole_gate_fwd(x, dtype, wg, logit_bias, S, E, M, scores, stream)) return rc;
+            ScopedTiming timing(MOLE_K_ROUTE, st);
+            return route_from(scores, nullptr, 0, normalize_gate, nullptr, gates, r, route_ws, st);
+        }
+        float *logits = (float *)ws;
+        ws += align256((size_t)S * E * sizeof(float));
+        if (path == GR_FEW) {
+            const int tg = S <= 512 ? 1 : 2;           // Wg is read once for 16 or 32 tokens
+            const dim3 grid(ceil_div(S, 16 * tg), ceil_div(E, 16));
+#define MOLE_GL(T, TG) timed_launch(MOLE_K_GATE_FWD, gate_logits_kernel<T, TG>, grid, dim3(256), 0, st, (const T *)x, wg, logit_bias, S, E, M, logits)
+            if (dtype == MOLE_BF16) { if (tg == 1) MOLE_GL(bf16_t, 1); else MOLE_GL(bf16_t, 2); }
+            else { if (tg == 1) MOLE_GL(float, 1); else MOLE_GL(float, 2); }
+#undef MOLE_GL
+            MOLE_LAUNCH_CHECK();
+            ScopedTiming timing(MOLE_K_ROUTE, st);
+            return route_from(logits, nullptr, 1, normalize_gate, scores, gates, r, route_ws, st);
+        }
+        const void *w = wg;
+        if (dtype == MOLE_BF16) {
+            const size_t n4 = (size_t)E * M / 4;
+            hipLaunchKernelGGL(f32_to_bf16_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, wg, (bf16_t *)ws, n4);
+            MOLE_LAUNCH_CHECK();
+            w = ws;
+        }
+        if (int rc = mole_gemm_nt(x, w, dtype, S, E, M, logits, stream)) return rc;
+        ScopedTiming timing(MOLE_K_ROUTE, st);
+        return route_from(logits, logit_bias, 1, normalize_gate, scores, gates, r, route_ws, st);
+    }
+    const int nb = ceil_div(S, GATE_ROUTE_TOKENS);
     int32_t *hist = (int32_t *)ws;
     ws += align256((size_t)nb * k * E * sizeof(int32_t));
     int32_t *basej = (int32_t *)ws;
@@ -1040,8 +1307,7 @@ extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const 
                      E, M, scores, rt);
     MOLE_LAUNCH_CHECK();
     ScopedTiming timing(MOLE_K_ROUTE, st);
-    return route_after_topk(hist, basej, colsum, colpart, nb, GATE_ROUTE_TOKENS, S, E, k, capacity_factor, alignment, layout, idx,
-                            loc, row, counts, kept_rows, offsets, capacity, l_aux, st);
+    return route_after_topk(r, hist, basej, colsum, colpart, nb, GATE_ROUTE_TOKENS, st);
 }
 
 extern "C" int mole_gate_fwd(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M,

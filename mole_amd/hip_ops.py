@@ -202,15 +202,15 @@ def route(scores: torch.Tensor, top_k: int, capacity_factor: float = 1.0, normal
 
 def gate_route_fused(x: torch.Tensor, wg: torch.Tensor) -> bool:
     """Whether gate_route() takes (x, wg) in its one-call form."""
-    return (x.dtype == torch.bfloat16 and wg.dtype == torch.float32 and wg.shape[0] <= 64 and x.shape[1] % 128 == 0
-            and x.shape[0] >= 1)
+    return (wg.dtype == torch.float32 and x.dtype in (torch.bfloat16, torch.float32) and wg.shape[0] <= L.MAX_EXPERTS
+            and x.shape[1] % (8 if x.dtype == torch.bfloat16 else 4) == 0 and x.shape[0] >= 1)
 
 
 def gate_route(x: torch.Tensor, wg: torch.Tensor, logit_bias: Optional[torch.Tensor], top_k: int,
                capacity_factor: float = 1.0, normalize_gate: bool = True, alignment: int = 1,
                layout: int = L.LAYOUT_RAGGED):
-    """(scores, Route) = (gate_fwd(x, wg, logit_bias), route(scores, ...)): for small gates on bf16 tokens one call whose
-    gate kernel also does the routing's first stage (mole_gate_route), otherwise the two calls."""
+    """(scores, Route) = (gate_fwd(x, wg, logit_bias), route(scores, ...)) in one call of the library (mole_gate_route,
+    which says how the kernels of the two are joined for the shape), otherwise the two calls."""
     _dev(x), _dev(wg)
     if not gate_route_fused(x, wg):
         scores = gate_fwd(x, wg, logit_bias)
@@ -229,7 +229,7 @@ def gate_route(x: torch.Tensor, wg: torch.Tensor, logit_bias: Optional[torch.Ten
     offsets = meta[k * E + E:k * E + 2 * E + 1]
     cap = meta[k * E + 2 * E + 1:]
     l_aux = torch.empty(1, dtype=torch.float32, device=dev)
-    nbytes = L.lib().mole_gate_route_workspace_bytes(S, E, k)
+    nbytes = L.lib().mole_gate_route_workspace_bytes(L.dtype_code(x.dtype), S, E, M, k)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     L.check(L.lib().mole_gate_route(L.ptr(x), L.dtype_code(x.dtype), L.ptr(wg), L.ptr(logit_bias), S, E, M, k,
                                     float(capacity_factor), int(normalize_gate), int(alignment), int(layout), L.ptr(scores),

@@ -230,3 +230,32 @@ def test_gate_and_route_in_one_call(S, E, M, k, cf, bias, normalize, ragged):
         np.testing.assert_array_equal(a[name], b[name], err_msg=name)
     assert a["capacity"] == b["capacity"]
     assert abs(a["l_aux"] - b["l_aux"]) <= 1e-5 * max(1.0, abs(b["l_aux"]))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("S,E,M,k,cf,bias,ragged", [
+    (1, 5, 128, 1, 0.0, False, True), (64, 17, 520, 4, 1.0, True, True), (65, 200, 264, 8, 0.0, False, False),
+    (513, 16, 136, 4, 1.25, True, True), (2048, 256, 512, 8, 0.0, False, True), (2049, 70, 264, 2, 1.0, True, True),
+    (300, 257, 128, 2, 0.0, True, True), (40, 1024, 256, 16, 0.5, False, True), (5000, 31, 72, 3, -0.5, True, False),
+])
+def test_gate_and_route_other_shapes(S, E, M, k, cf, bias, ragged, dtype):
+    """mole_gate_route beyond the small bf16 gates: few tokens (around 64, where one block does the whole routing, and
+    2048, the last size on the tiles), widths that are not whole steps, more experts than 16 or 64 lanes hold one of.
+    The scores against the oracle's gate; the routing against mole_route of the same scores, bit for bit."""
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"gate_route other S={S} E={E} M={M} k={k} cf={cf} bias={bias} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(S * 3 + E)
+    x = torch.randn(S, M, generator=g).to(dtype)
+    wg = torch.randn(E, M, generator=g) * 0.05
+    wg[E - 1] = wg[0]
+    lb = torch.randn(E, generator=g) * 0.5 if bias else None
+    layout = L.LAYOUT_RAGGED if ragged else L.LAYOUT_PADDED
+    scores, r = H.gate_route(x.cuda(), wg.cuda(), lb.cuda() if bias else None, k, cf, True, 1, layout)
+    want = O.gate_scores(x.float(), wg.to(dtype).float(), lb)
+    assert rel_err(scores.cpu(), want) < 1e-5
+    r2 = H.route(scores, k, cf, True, 1, layout)
+    a, b = crit_to_numpy(r), crit_to_numpy(r2)
+    for name in ("idx", "loc", "gates", "row", "counts", "kept", "offsets"):
+        np.testing.assert_array_equal(a[name], b[name], err_msg=name)
+    assert a["capacity"] == b["capacity"]
+    assert abs(a["l_aux"] - b["l_aux"]) <= 1e-5 * max(1.0, abs(b["l_aux"]))
