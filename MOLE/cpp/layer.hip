@@ -1,0 +1,136 @@
+// The layer's forward and backward as one call each: gate, routing, dispatch, grouped FFN and combine (and their
+// gradients) enqueued back to back from native code on buffers the caller laid out.
+//
+// Replaces the sequence of MOLEModule.forward (MOLE/moe/layer.py:440-462) and its autograd.  The kernels are those of
+// the separate entry points, which these two call; what goes away is the host's work between them - a tensor
+// allocation per intermediate, a foreign call with its argument conversion per step - which for short batches took
+// longer than the kernels (61 tokens, 16 experts of 1024 -> 4096: 95 us of host time for 75 us of kernels).
+#include "common.h"
+
+namespace mole {
+
+static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// out [ro][co] in T = in [r][c] fp32, zeros beyond
+template <typename T>
+__global__ __launch_bounds__(256) void pad_convert_kernel(const float *__restrict__ in, int r, int c, T *__restrict__ out, int ro, int co) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (size_t)ro * co) return;
+    const int y = (int)(i / co), x = (int)(i % co);
+    out[i] = y < r && x < c ? from_f32<T>(in[(size_t)y * c + x]) : from_f32<T>(0.f);
+}
+template <typename T>
+__global__ __launch_bounds__(256) void to_f32_kernel(const T *__restrict__ in, float *__restrict__ out, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) out[i] = to_f32(in[i]);
+}
+static int pad_convert(const float *in, int r, int c, void *out, int ro, int co, int dtype, hipStream_t st) {
+    const dim3 grid((unsigned)(((size_t)ro * co + 255) / 256));
+    if (dtype == MOLE_BF16) hipLaunchKernelGGL(pad_convert_kernel<bf16_t>, grid, dim3(256), 0, st, in, r, c, (bf16_t *)out, ro, co);
+    else hipLaunchKernelGGL(pad_convert_kernel<float>, grid, dim3(256), 0, st, in, r, c, (float *)out, ro, co);
+    MOLE_LAUNCH_CHECK();
+    return 0;
+}
+
+// Scratch of the backward's gate part, and which way its two products go.
+struct GateBwdPlan {
+    bool fold;           // dlogits . Wg inside the dispatch backward (up to 32 experts)
+    bool wgrad_kernel;   // dlogits^T . x on the gate's own kernel, otherwise on the grouped-GEMM tiles
+    int e_pad;           // experts rounded up to the tiles' granule
+    size_t dgates, dl_t, wg_t, dx_add, wgrad, total;     // bytes
+};
+static GateBwdPlan gate_bwd_plan(const mole_layer &L) {
+    GateBwdPlan p{};
+    const size_t es = L.dtype == MOLE_BF16 ? 2 : 4;
+    const int epc = L.dtype == MOLE_BF16 ? 8 : 4;
+    p.fold = L.E <= 32;
+    p.wgrad_kernel = (L.dtype == MOLE_BF16 && L.E <= 256 && L.M % 64 == 0) || L.E <= 32;
+    p.e_pad = (L.E + epc - 1) / epc * epc;
+    p.dgates = L.E > 256 ? up256((size_t)L.k * L.S * 4) : 0;
+    p.dl_t = p.fold && p.wgrad_kernel ? 0 : up256((size_t)L.S * p.e_pad * es);
+    p.wg_t = p.fold ? 0 : up256((size_t)p.e_pad * L.M * es);
+    p.dx_add = p.fold ? 0 : up256((size_t)L.S * L.M * es);
+    p.wgrad = up256(p.wgrad_kernel ? mole_gate_wgrad_workspace_bytes(L.S, L.E, L.M) : (size_t)p.e_pad * L.M * es);
+    p.total = p.dgates + p.dl_t + p.wg_t + p.dx_add + p.wgrad;
+    return p;
+}
+
+}  // namespace mole
+
+using namespace mole;
+
+extern "C" size_t mole_layer_workspace_bytes(const mole_layer *L, int backward) {
+    if (L == nullptr || L->S <= 0 || L->E <= 0) return 0;
+    const size_t ffn = mole_ffn_workspace_bytes(L->dtype, L->E, L->rows, L->M, L->F);
+    const size_t other = backward ? gate_bwd_plan(*L).total : mole_gate_route_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
+    return ffn > other ? ffn : other;        // the two are never in use at the same time
+}
+
+static int check_layer(const char *fn, const mole_layer *L, mole_stream_t) {
+    MOLE_REQUIRE(L != nullptr, "%s: null argument block", fn);
+    MOLE_REQUIRE(L->S >= 1 && L->rows >= 1 && L->E >= 1 && L->F >= 1, "%s: bad sizes S=%d rows=%d E=%d F=%d", fn, L->S, L->rows, L->E, L->F);
+    MOLE_REQUIRE(L->x && L->wg && L->scores && L->gates && L->idx && L->row && L->counts && L->kept_rows && L->offsets && L->xd &&
+                     L->h && L->a && L->out && L->workspace, "%s: null pointer", fn);
+    return 0;
+}
+
+extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream) {
+    if (int rc = check_layer("mole_layer_fwd", L, stream)) return rc;
+    const size_t need = mole_layer_workspace_bytes(L, 0);
+    if (L->workspace_bytes < need) {
+        set_error("mole_layer_fwd: workspace of %zu bytes, need %zu", L->workspace_bytes, need);
+        return MOLE_E_WORKSPACE;
+    }
+    if (int rc = mole_gate_route(L->x, L->dtype, L->wg, L->logit_bias, L->S, L->E, L->M, L->k, L->capacity_factor, L->normalize_gate, 1,
+                                 L->layout, L->scores, L->idx, L->loc, L->gates, L->row, L->counts, L->kept_rows, L->offsets,
+                                 L->capacity, L->l_aux, L->workspace, L->workspace_bytes, stream)) return rc;
+    if (int rc = mole_dispatch_fwd(L->x, L->dtype, L->row, L->S, L->M, L->k, L->xd, stream)) return rc;
+    if (int rc = mole_ffn_fwd_ws(L->xd, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, L->M, L->F, L->w1, L->b1, L->w2, L->b2, L->h,
+                                 L->a, L->out, L->workspace, L->workspace_bytes, stream)) return rc;
+    return mole_combine_fwd(L->out, L->dtype, L->row, L->gates, L->S, L->M, L->k, y, stream);
+}
+
+extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mole_stream_t stream) {
+    if (int rc = check_layer("mole_layer_bwd", L, stream)) return rc;
+    MOLE_REQUIRE(G && G->dy && G->dlogits && G->d_o && G->t && G->gxd && G->dx && G->dwg, "mole_layer_bwd: null gradient pointer");
+    const size_t need = mole_layer_workspace_bytes(L, 1);
+    if (L->workspace_bytes < need) {
+        set_error("mole_layer_bwd: workspace of %zu bytes, need %zu", L->workspace_bytes, need);
+        return MOLE_E_WORKSPACE;
+    }
+    const GateBwdPlan p = gate_bwd_plan(*L);
+    hipStream_t st = (hipStream_t)stream;
+    char *ws = (char *)L->workspace;
+    const int32_t *counts0 = G->d_l_aux ? L->counts : nullptr;
+    if (p.dgates == 0) {
+        if (int rc = mole_combine_bwd_gate(G->dy, L->out, L->dtype, L->row, L->gates, L->S, L->M, L->k, G->d_o, L->scores, L->idx, L->E,
+                                           L->normalize_gate, 1, counts0, G->d_l_aux, G->dlogits, stream)) return rc;
+    } else {
+        float *dgates = (float *)ws;
+        if (int rc = mole_combine_bwd(G->dy, L->out, L->dtype, L->row, L->gates, L->S, L->M, L->k, G->d_o, dgates, stream)) return rc;
+        if (int rc = mole_gate_bwd(dgates, L->scores, L->idx, L->S, L->E, L->k, L->normalize_gate, 1, counts0, G->d_l_aux, G->dlogits,
+                                   stream)) return rc;
+    }
+    // (the FFN's scratch takes the place of dgates and makes room for the gate's products, in stream order)
+    if (int rc = mole_ffn_bwd_ws(G->d_o, L->xd, L->h, L->a, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, L->M, L->F, L->w1, L->w2,
+                                 G->t, G->g_w1, G->g_b1, G->g_w2, G->g_b2, G->gxd, G->accumulate, G->gelu_bwd, L->workspace,
+                                 L->workspace_bytes, stream)) return rc;
+    char *dl_t = ws + p.dgates, *wg_t = dl_t + p.dl_t, *dx_add = wg_t + p.wg_t, *wgrad = dx_add + p.dx_add;
+    if (p.dl_t)
+        if (int rc = pad_convert(G->dlogits, L->S, L->E, dl_t, L->S, p.e_pad, L->dtype, st)) return rc;
+    if (p.fold) {
+        if (int rc = mole_dispatch_bwd(G->gxd, L->dtype, L->row, L->S, L->M, L->k, G->dlogits, L->wg, L->E, nullptr, G->dx, stream)) return rc;
+    } else {
+        if (int rc = pad_convert(L->wg, L->E, L->M, wg_t, p.e_pad, L->M, L->dtype, st)) return rc;
+        if (int rc = mole_gemm_nn(dl_t, wg_t, L->dtype, L->S, L->M, p.e_pad, dx_add, stream)) return rc;
+        if (int rc = mole_dispatch_bwd(G->gxd, L->dtype, L->row, L->S, L->M, L->k, nullptr, nullptr, 0, dx_add, G->dx, stream)) return rc;
+    }
+    if (p.wgrad_kernel) return mole_gate_wgrad(G->dlogits, L->x, L->dtype, L->S, L->E, L->M, G->dwg, wgrad, p.wgrad, stream);
+    if (int rc = mole_gemm_tn(dl_t, L->x, L->dtype, L->S, p.e_pad, L->M, wgrad, stream)) return rc;
+    const size_t n = (size_t)L->E * L->M;
+    const dim3 grid((unsigned)((n + 255) / 256));
+    if (L->dtype == MOLE_BF16) hipLaunchKernelGGL(to_f32_kernel<bf16_t>, grid, dim3(256), 0, st, (const bf16_t *)wgrad, G->dwg, n);
+    else hipLaunchKernelGGL(to_f32_kernel<float>, grid, dim3(256), 0, st, (const float *)wgrad, G->dwg, n);
+    MOLE_LAUNCH_CHECK();
+    return 0;
+}

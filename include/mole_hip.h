@@ -253,6 +253,41 @@ int mole_ffn_bwd_ws(const void *go, const void *xd, const void *h, const void *a
                     void *g_b2, void *gx, int accumulate, int gelu_bwd, void *workspace, size_t workspace_bytes,
                     mole_stream_t stream);
 
+/* ------------------------------------------------------------------------------------------
+ * The layer in one call each way: gate, routing, dispatch, grouped FFN, combine (MOLE/moe/layer.py:440-462) and their
+ * gradients, enqueued on the caller's stream.  The argument block names every buffer; the buffers, their shapes and
+ * what they hold are those of the separate entry points above (x [S,M], wg [E,M] fp32, logit_bias [E] or NULL, xd and out
+ * [rows,M], h and a [rows,F], rows >= 1 a bound of the kept rows: S*k, the capacity's bound, or E*C in the padded layout).
+ * S >= 1.  workspace of mole_layer_workspace_bytes(L, backward) bytes, which reads the sizes of the block only.
+ * mole_layer_fwd fills scores .. l_aux, xd, h, a, out and y [S,M]; mole_layer_bwd reads them again (the same block) and
+ * fills dx, dwg [E,M] fp32 and the expert gradients; dlogits [S,E] fp32, d_o and gxd [rows,M], t [rows,F] are scratch of the
+ * caller's; d_l_aux: NULL or the gradient of l_aux. */
+typedef struct mole_layer {
+    int32_t dtype, S, M, E, k, F, rows, layout, normalize_gate;
+    double capacity_factor;
+    const void *x;
+    const float *wg, *logit_bias;
+    const void *w1, *b1, *w2, *b2;
+    float *scores, *gates, *l_aux;
+    int32_t *idx, *loc, *row, *counts, *kept_rows, *offsets, *capacity;
+    void *xd, *h, *a, *out;
+    void *workspace;
+    size_t workspace_bytes;
+} mole_layer;
+typedef struct mole_layer_grads {
+    int32_t accumulate, gelu_bwd;
+    const void *dy;
+    const float *d_l_aux;
+    float *dlogits;
+    void *d_o, *t, *gxd;
+    void *g_w1, *g_b1, *g_w2, *g_b2;
+    void *dx;
+    float *dwg;
+} mole_layer_grads;
+size_t mole_layer_workspace_bytes(const mole_layer *layer, int backward);
+int mole_layer_fwd(const mole_layer *layer, void *y, mole_stream_t stream);
+int mole_layer_bwd(const mole_layer *layer, const mole_layer_grads *grads, mole_stream_t stream);
+
 /* Plain GEMMs on the same tiles, used by the gate: c[rows,N] = a[rows,K] . b[N,K]^T  (fp32 out). */
 int mole_gemm_nt(const void *a, const void *b, int dtype, int rows, int N, int K, float *c,
                  mole_stream_t stream);

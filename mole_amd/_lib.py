@@ -22,6 +22,23 @@ KERNEL_IDS = ("ffn_fwd1", "ffn_fwd2", "ffn_gw2", "ffn_da", "ffn_gw1", "ffn_gx", 
               "combine_fwd", "combine_bwd", "route", "gemm_nt", "adam", "gate_fwd", "gate_bwd", "gate_wgrad", "probe")
 
 _P = c_void_p
+
+
+class LayerArgs(ctypes.Structure):
+    """mole_layer of include/mole_hip.h."""
+    _fields_ = ([(n, c_int32) for n in ("dtype", "S", "M", "E", "k", "F", "rows", "layout", "normalize_gate")]
+                + [("capacity_factor", c_double)]
+                + [(n, c_void_p) for n in ("x", "wg", "logit_bias", "w1", "b1", "w2", "b2", "scores", "gates", "l_aux", "idx", "loc",
+                                           "row", "counts", "kept_rows", "offsets", "capacity", "xd", "h", "a", "out", "workspace")]
+                + [("workspace_bytes", c_size_t)])
+
+
+class LayerGrads(ctypes.Structure):
+    """mole_layer_grads of include/mole_hip.h."""
+    _fields_ = ([("accumulate", c_int32), ("gelu_bwd", c_int32)]
+                + [(n, c_void_p) for n in ("dy", "d_l_aux", "dlogits", "d_o", "t", "gxd", "g_w1", "g_b1", "g_w2", "g_b2", "dx", "dwg")])
+
+
 _SIGNATURES = {
     "mole_version": (c_int, []),
     "mole_last_error_string": (c_char_p, []),
@@ -59,6 +76,9 @@ _SIGNATURES = {
     "mole_ffn_fwd_ws": (c_int, [_P, c_int, _P, _P, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P, _P, c_size_t, _P]),
     "mole_ffn_bwd_ws": (c_int, [_P, _P, _P, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P,
                                 _P, c_int, c_int, _P, c_size_t, _P]),
+    "mole_layer_workspace_bytes": (c_size_t, [POINTER(LayerArgs), c_int]),
+    "mole_layer_fwd": (c_int, [POINTER(LayerArgs), _P, _P]),
+    "mole_layer_bwd": (c_int, [POINTER(LayerArgs), POINTER(LayerGrads), _P]),
     "mole_gemm_nt": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P]),
     "mole_gemm_nn": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P]),
     "mole_gemm_tn": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P]),

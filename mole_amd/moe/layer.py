@@ -7,8 +7,12 @@ Constructor and forward keep the reference's names, argument order and defaults
 Two execution shapes, same results:
   * fused (default): one autograd node over the ragged, expert-contiguous layout.  Nothing is
     padded, nothing is read back to the host, every step is a kernel of libmole_hip.so.
-  * reference_layout=True: the reference's literal call sequence - extract_critical, fast_encode
-    into a zero-padded [E, C, M], BatchFusedFWD.apply over all E*C rows, fast_decode.
+    With all experts on the GPU that is one native call each way (mole_layer_fwd / mole_layer_bwd).
+  * reference_layout=True: the reference's padded layout, expert e's rows at e*C of an [E, C, M] buffer.  With all experts on
+    the GPU and a capacity known on the host (capacity_factor > 0) the same two native calls, which compute the kept rows
+    only; otherwise the reference's literal call sequence - extract_critical, fast_encode into a zero-padded [E, C, M],
+    BatchFusedFWD.apply over all E*C rows, fast_decode - with the same results (a padding row is zero and meets a zero
+    gradient).
 
 New, optional keyword arguments (all defaulting to the reference's behaviour): dtype,
 normalize_gate, gelu_bwd ("tanh" = the derivative the reference compiles, MOLE/cpp/define.hpp:6;
@@ -101,6 +105,40 @@ class _FusedMoE(torch.autograd.Function):
         return dx, dwg, torch.zeros_like(m.dummy_param), None, None, None
 
 
+class _LayerFn(torch.autograd.Function):
+    """_FusedMoE for experts that all live on the GPU: the same steps, each direction one call of the library on buffers
+    laid out by a LayerPlan."""
+
+    @staticmethod
+    def forward(ctx, x, wg, dummy_param, module, plan, time_it):
+        m = module
+        ctx.set_materialize_grads(False)
+        l_aux = torch.empty((), dtype=torch.float32, device=x.device)
+        y, route, act = plan.forward(x, wg, m.gate[0].logit_bias, [g[0] for g in m.MOLECore.gpu], l_aux)
+        m._route = (plan, route)
+        ctx.m, ctx.plan, ctx.time_it = m, plan, time_it
+        ctx.save_for_backward(x, wg, route, act)
+        return y, l_aux
+
+    @staticmethod
+    def backward(ctx, dy, d_l_aux):
+        m = ctx.m
+        x, wg, route, act = ctx.saved_tensors
+        if dy is None:            # only l_aux was used
+            dy = torch.zeros_like(x)
+        if ctx.time_it:
+            UATimer.track_bwd_start(m.moe_id)
+        if d_l_aux is not None and d_l_aux.dtype != torch.float32:
+            d_l_aux = d_l_aux.float()
+        core_ = m.MOLECore
+        dx, dwg = ctx.plan.backward(dy.contiguous(), d_l_aux, x, wg, [g[0] for g in core_.gpu], route, act,
+                                    [g[1] for g in core_.gpu], core_.acc_step > 1)
+        core_.step += 1
+        if ctx.time_it:
+            UATimer.track_bwd_end(m.moe_id)
+        return dx, dwg, None, None, None, None
+
+
 class MOLEModule(torch.nn.Module):
     _instance = []
     _fwdgaps = []
@@ -128,6 +166,7 @@ class MOLEModule(torch.nn.Module):
         self.device = torch.device(f"cuda:{self.local_rank}")
         self.param_dtype = dtype
         self.normalize_gate = normalize_gate
+        self._granule = 8 if dtype == torch.bfloat16 else 4       # elements of a 16-byte piece
         self.reference_layout = reference_layout
 
         core.create_UniMem(self.local_rank, pool_size, dtype, [[ffn_dim, embed_dim], [ffn_dim], [ffn_dim, embed_dim],
@@ -198,8 +237,49 @@ class MOLEModule(torch.nn.Module):
         self.global_prefetch = False
         self.grad_use_pool, self.mome_use_pool, self.vari_use_pool = pool_for_extra
         self.l_aux = None
+        self._route = None           # (plan, buffer) of the last one-call forward, or the Route of another
+        self._plans = {}             # LayerPlan per (tokens, capacity factor, ...): sizes only, no device memory
         self.moe_id = len(MOLEModule._instance)
         MOLEModule._instance.append(self)
+
+    # ---- results of the last forward besides its output ---------------------------------------
+    @property
+    def last_route(self):
+        """The Route of the last forward pass."""
+        r = self._route
+        return r[0].route(r[1]) if isinstance(r, tuple) else r
+
+    @last_route.setter
+    def last_route(self, r):
+        self._route = r
+
+    @property
+    def l_aux(self):
+        """The load-balancing loss of the last forward pass."""
+        if self._l_aux is None and isinstance(self.__dict__.get("_route"), tuple):
+            self._l_aux = self.last_route.l_aux.view(())
+        return self._l_aux
+
+    @l_aux.setter
+    def l_aux(self, v):
+        self._l_aux = v
+
+    def _plan(self, S, capacity_factor, wg):
+        """The LayerPlan of a forward pass over S tokens, or None when it takes the step-by-step path (experts offloaded, no
+        tokens, a gate in another dtype, a padded capacity that only the device knows)."""
+        if (self.d_experts or not self.s_experts or S < 1 or wg.dtype != torch.float32 or not wg.is_contiguous()
+                or self.embed_dim % self._granule or self.ffn_dim % self._granule or (self.reference_layout and capacity_factor <= 0)):
+            return None
+        key = (S, capacity_factor, self.topk, self.normalize_gate, self.reference_layout)
+        plan = self._plans.get(key)
+        if plan is None:
+            if len(self._plans) >= 64:
+                self._plans.clear()
+            plan = self._plans[key] = H.LayerPlan(
+                self.param_dtype, S, self.embed_dim, self.total_experts, min(self.topk, self.total_experts), self.ffn_dim,
+                capacity_factor, L.LAYOUT_PADDED if self.reference_layout else L.LAYOUT_RAGGED, self.normalize_gate,
+                self.MOLECore.gelu_bwd)
+        return plan
 
     # ---- prefetch API (layer.py:138-180) -----------------------------------------------------
     def dummy_fetch(self, batch_size):
@@ -255,7 +335,16 @@ class MOLEModule(torch.nn.Module):
             resized_input = resized_input.to(self.param_dtype)
         resized_input = resized_input.contiguous()
 
-        if self.reference_layout:
+        gate = self.gate[0]
+        wg = gate.linear.weight
+        plan = self._plan(resized_input.shape[0], float(capacity_factor), wg)
+        if plan is not None:
+            if torch.is_grad_enabled():
+                expert_output, self.l_aux = _LayerFn.apply(resized_input, wg, self.dummy_param, self, plan, bool(time_it))
+            else:
+                expert_output, route, _ = plan.forward(resized_input, wg, gate.logit_bias, [g[0] for g in self.MOLECore.gpu])
+                self._route, self.l_aux = (plan, route), None
+        elif self.reference_layout:
             scores = self.gate[0](resized_input)
             crit, l_aux = tutel_fast_dispatcher.extract_critical(
                 scores, top_k=self.topk, capacity_factor=capacity_factor, normalize_gate=self.normalize_gate)
@@ -264,8 +353,7 @@ class MOLEModule(torch.nn.Module):
             experts_output = BatchFusedFWD.apply(dispatched_input, self, self.dummy_param, time_it, prefetch)
             expert_output = tutel_fast_dispatcher.fast_decode(data=experts_output, critial_data=crit)
         else:
-            expert_output, self.l_aux = _FusedMoE.apply(resized_input, self.gate[0].linear.weight, self.dummy_param,
-                                                        self, float(capacity_factor), bool(time_it))
+            expert_output, self.l_aux = _FusedMoE.apply(resized_input, wg, self.dummy_param, self, float(capacity_factor), bool(time_it))
 
         expert_output = expert_output.reshape(original_shape)
         out = expert_output.to(original_dtype)

@@ -545,3 +545,19 @@ def test_resident_experts_halve_the_traffic_and_follow_weight_updates(dtype):
     layers[0].FC2_B_CPU.all_tensors.mul_(2.0)
     y_after = layers[0](x, capacity_factor=0.0).detach()
     assert rel_err(y_after, 2.0 * y_before.float()) < (1e-5 if dtype == torch.float32 else 2e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("S,M,E,k,Fd,cf,padded", [(5, 64, 33, 2, 128, 0.0, False), (130, 72, 40, 2, 136, 1.25, True),
+                                                  (90, 64, 260, 3, 64, 0.0, False)])
+def test_layer_one_call_gate_paths(S, M, E, k, Fd, cf, padded, dtype):
+    """The native layer call where the gate's backward leaves the small-gate kernels: more than 32 experts (its products on
+    the GEMM tiles, experts padded to their granule), more than 256 (the gate gradients in a kernel of their own), with
+    and without the load-balancing loss; forward under no_grad gives the bits of the forward that autograd records."""
+    print(f"layer gate paths S={S} M={M} E={E} k={k} F={Fd} cf={cf} padded={padded} {dtype}", flush=True)
+    m, x, ref = _build(S, M, E, k, Fd, dtype, reference_layout=padded, seed=S)
+    res = _run_and_compare(m, x, ref, k, cf, dtype, aux_w=25.0)
+    assert m.last_route.kept_rows.shape == (E,)
+    with torch.no_grad():
+        y = m(x, capacity_factor=cf)
+    assert torch.equal(y, res.extras["y_gpu"]) and abs(float(m.l_aux) - res.crit.l_aux) < 1e-4 * max(1.0, res.crit.l_aux)
