@@ -503,7 +503,7 @@ static int ffn_bwd_t(const void *go, const void *xd, const void *h, const void *
     gw2.A = a; gw2.lda = F; gw2.B = go; gw2.ldb = M; gw2.M = F; gw2.N = M; gw2.C = g_w2; gw2.ldc = M; gw2.strideC = (long)F * M;
     bool fused_sums = false;
     if constexpr (sizeof(T) == 2)
-        fused_sums = fast_path_enabled() && gemm256_sums_operand(gw2, MOLE_K_FFN_GW2) && gemm256_sums_operand(gw2, MOLE_K_FFN_GW1);
+        fused_sums = fast_path_enabled() && gemm256_sums_operand(gw2);
     else
         fused_sums = fast_path_enabled() && gemm_f32_sums_operand(gw2);
     // g_w2[e] = a^T . go          (contract over the expert's rows); g_b2 = sum go

@@ -154,7 +154,7 @@ struct GemmArgs {
 // 256x256 bf16 tiles with direct-to-LDS loads (gemm256.hip).  Returns -100 when the shape does not
 // meet its alignment requirements; the caller then uses the generic kernel.
 int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid);
-bool gemm256_sums_operand(const GemmArgs &g, int kid);
+bool gemm256_sums_operand(const GemmArgs &g);
 // Few rows per expert (gemm_skinny.hip): weights streamed straight into fragments; -100 when the shape is not its.
 int launch_gemm_skinny(const GemmArgs &g, int dtype, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
 size_t gemm_skinny_workspace_bytes(int E, int max_rows, int N, int K, int dtype);

@@ -2,8 +2,8 @@
 //
 // A block of 8 waves (2 wave rows x 4 wave columns, two waves per SIMD) owns a BM (m) x 256 (n) output tile, BM =
 // 256 or up to 320; a wave covers BM/2 rows and 64 columns (BM/64 x 2 MFMA 32x32x16 blocks, fp32 accumulators).
-// One block per CU.  (A build with -DMOLE_TUNING also carries the four-wave shapes and launch orders that were
-// measured against this one and lost.)
+// One block per CU.  Launches too small to give most CUs such a tile run 128 x 128 tiles of four waves, two blocks to a
+// CU.  (A build with -DMOLE_TUNING also reads the launch orders that were measured against these and lost.)
 // Operand tiles go from HBM/L2 straight into LDS (global_load_lds_dwordx4, no staging registers)
 // through a ring of stages of 32 of K, several stages of loads in flight while one is consumed: with
 // a single stage of look-ahead the loop ran at the memory latency, not at the MFMA rate.  One
@@ -27,37 +27,38 @@ namespace mole {
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int Q_BN = 256, Q_BK = 32;
-constexpr int Q_N_OPERAND = Q_BN * Q_BK * 2;   // bytes of the n-side tile of one stage
+constexpr int Q_BK = 32;
 
-// Geometry of a BM x 256 tile of TMB 32-row m-blocks computed by 4 WM waves: WM wave rows of TMB/WM m-blocks
-// each, 4 wave columns of 64 columns each.  WM = 2 puts two waves on every SIMD: while one waits for
+// Geometry of a BM x BN tile of TMB 32-row m-blocks computed by WM x WN waves: WM wave rows of TMB/WM m-blocks
+// each, WN wave columns of 64 columns each.  Eight waves put two on every SIMD: while one waits for
 // the memory pipeline to accept a load or for a barrier, the other issues MFMAs.
-template <int TMB, int WM> struct Tile {
-    static constexpr int NW = 4 * WM, THREADS = 64 * NW, TMW = TMB / WM;
-    static constexpr int BM = TMB * 32;
+template <int TMB, int WM, int WN> struct Tile {
+    static constexpr int NW = WM * WN, THREADS = 64 * NW, TMW = TMB / WM;
+    static constexpr int BM = TMB * 32, BN = 64 * WN;
     static constexpr int M_ROWS = (BM + 16 * NW - 1) / (16 * NW) * (16 * NW);   // rows the waves' loads cover
-    static constexpr int M_OPERAND = M_ROWS * Q_BK * 2;
-    static constexpr int STAGE = M_OPERAND + Q_N_OPERAND;
-    static constexpr int NSTAGE = TMB >= 8 ? 4 : 3;
+    static constexpr int M_OPERAND = M_ROWS * Q_BK * 2, N_OPERAND = BN * Q_BK * 2;   // bytes of one stage
+    static constexpr int STAGE = M_OPERAND + N_OPERAND;
+    static constexpr bool WHOLE_CU = TMB >= 8 && WN == 4;
+    static constexpr int LDS_BUDGET = TMB >= 4 ? 80 * 1024 : 40 * 1024;   // two or four blocks per CU
+    static constexpr int NSTAGE = WHOLE_CU ? 4 : (LDS_BUDGET / STAGE < 6 ? LDS_BUDGET / STAGE : 6);
     static constexpr int SLABS = NW * TMW * 32 * 128;                // the waves' epilogue staging areas
     static constexpr int LDS_BYTES = NSTAGE * STAGE > SLABS ? NSTAGE * STAGE : SLABS;
-    static constexpr int BLOCKS_PER_CU = TMB >= 8 ? 1 : 2;
+    static constexpr int WAVES_PER_SIMD = TMB >= 4 ? 2 : 4;
 };
 
 // One stage of the operand ring for a tile of which the first TMC 32-row blocks are live.  Of a K-contiguous
 // m-side tile only the 64-row groups that hold live blocks are fetched and stored, so a light tile has
 // smaller stages and its ring, in the same LDS, is deeper: light tiles do little arithmetic per stage and
 // run at the memory latency divided by the stages in flight.
-template <int TMB, int WM, bool M_KS, int TMC> struct Stage {
-    typedef Tile<TMB, WM> TL;
+template <int TMB, int WM, int WN, bool M_KS, int TMC> struct Stage {
+    typedef Tile<TMB, WM, WN> TL;
     static constexpr int RPL = 16 * TL::NW;                                       // rows (or 16-byte slot groups) one load of every wave covers
     static_assert(!M_KS || TL::BM % RPL == 0, "a K-strided m-side tile must be whole load rounds wide");
     static constexpr int LM = M_KS ? TL::BM / RPL : (TMC * 32 + RPL - 1) / RPL;  // m-side loads per wave
-    static constexpr int LN = Q_BN / RPL;
+    static constexpr int LN = TL::BN / RPL;
     static constexpr int L = LM + LN;                                             // loads per wave
     static constexpr int M_OPERAND = LM * RPL * Q_BK * 2;
-    static constexpr int BYTES = M_OPERAND + Q_N_OPERAND;
+    static constexpr int BYTES = M_OPERAND + TL::N_OPERAND;
     static constexpr int FIT = TL::NSTAGE * TL::STAGE / BYTES;
     static constexpr int NSTAGE = FIT > 6 ? 6 : FIT;
 };
@@ -145,15 +146,15 @@ template <int P, int NP, int N> constexpr int part_lo() { return P * N / NP; }
 
 // The fragments one wave needs for a k-sub-step: its TMCW m-blocks (blocks wm*TMCW .. of the tile, of which
 // the tile's first TMC are fetched) and its two 32-column n-blocks.
-template <int TMB, int WM, bool M_KS, bool N_KS, int TMC, int TMCW> struct Frags {
-    typedef Tile<TMB, WM> TL;
+template <int TMB, int WM, int WN, bool M_KS, bool N_KS, int TMC, int TMCW> struct Frags {
+    typedef Tile<TMB, WM, WN> TL;
     static constexpr int NR = TMCW ? TMCW + 2 : 0;
     bf16x8 m[TMCW ? TMCW : 1], n[2];
     // the fragment reads of a k-sub-step, n-side first, dealt to NP parts
     template <int P, int NP> __device__ __forceinline__ void read_part(const char *stage, int wm, int wn, int kk) {
 #pragma unroll
         for (int r = part_lo<P, NP, NR>(); r < part_lo<P + 1, NP, NR>(); ++r) {
-            if (r < 2) n[r] = frag<N_KS, Q_BN>(stage + Stage<TMB, WM, M_KS, TMC>::M_OPERAND, wn * 2 + r, kk);
+            if (r < 2) n[r] = frag<N_KS, TL::BN>(stage + Stage<TMB, WM, WN, M_KS, TMC>::M_OPERAND, wn * 2 + r, kk);
             else m[r - 2] = frag<M_KS, TL::BM>(stage, wm * TMCW + r - 2, kk);
         }
     }
@@ -185,12 +186,12 @@ template <int TMB, int WM, bool M_KS, bool N_KS, int TMC, int TMCW> struct Frags
 // fixed for the whole K loop.  Stages are fetched in order; past the last one the last is fetched again,
 // harmlessly: it keeps the number of loads per stage, which the vmcnt arithmetic of the loop relies on.
 // Of a K-contiguous m-side tile only the 64-row groups that hold live 32-row blocks (the first TMC) are fetched.
-template <int TMB, int WM, bool M_KS, bool N_KS, bool WG, int TMC> struct Feeder {
-    typedef Tile<TMB, WM> TL;
-    typedef Stage<TMB, WM, M_KS, TMC> SG;
+template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool WG, int TMC> struct Feeder {
+    typedef Tile<TMB, WM, WN> TL;
+    typedef Stage<TMB, WM, WN, M_KS, TMC> SG;
     static constexpr int LM = SG::LM, L = SG::L;
     Off<TL::M_ROWS, TL::NW, M_KS> om, cm;
-    Off<Q_BN, TL::NW, N_KS> on, cn;
+    Off<TL::BN, TL::NW, N_KS> on, cn;
     const char *bm, *bn;
     long step_m, step_n;
     uint32_t lds_w;      // LDS address of ring buffer 0 + this wave's 1 KiB lane
@@ -272,14 +273,14 @@ template <int B, int L, int X> __device__ __forceinline__ void wait_stages_behin
 // BIAS: the accumulators start from the bias of their columns instead of zero (bias_raw: the 8 x 4 columns a lane
 // holds, fetched before the operand loads and therefore landed when the first stage has), so that the epilogue adds
 // nothing.
-template <int TMB, int WM, bool M_KS, bool N_KS, bool WG, int TMC, int TMCW, int SUM, int PART = 0, bool BIAS = false>
+template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool WG, int TMC, int TMCW, int SUM, int PART = 0, bool BIAS = false>
 __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, int m_ext, const bf16_t *Np, long ldn,
                                           int n0, int n_ext, int k_ext, char *smem, int wave, int wm, int wn,
-                                          f32x16 (&acc)[Tile<TMB, WM>::TMW][2], f32x16 &sums, const uint2 (&bias_raw)[8]) {
-    typedef Tile<TMB, WM> TL;
-    typedef Stage<TMB, WM, M_KS, TMC> SG;
+                                          f32x16 (&acc)[Tile<TMB, WM, WN>::TMW][2], f32x16 &sums, const uint2 (&bias_raw)[8]) {
+    typedef Tile<TMB, WM, WN> TL;
+    typedef Stage<TMB, WM, WN, M_KS, TMC> SG;
     constexpr int AHEAD = SG::NSTAGE - 1, NP = 4;
-    typedef Feeder<TMB, WM, M_KS, N_KS, WG, TMC> FD;
+    typedef Feeder<TMB, WM, WN, M_KS, N_KS, WG, TMC> FD;
     constexpr int L = FD::L, LH = L / 2;      // loads per wave per stage; the halves are LH and L - LH
     const int nk = __builtin_amdgcn_readfirstlane((k_ext + Q_BK - 1) / Q_BK);
     if (nk == 0) return;
@@ -289,7 +290,7 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
         if (WG && s == nk - 1 && (k_ext & (Q_BK - 1))) {
             char *b = smem + buf * SG::BYTES;
             zero_k_tail<TL::BM, TL::THREADS>(b, k_ext & (Q_BK - 1));
-            zero_k_tail<Q_BN, TL::THREADS>(b + SG::M_OPERAND, k_ext & (Q_BK - 1));
+            zero_k_tail<TL::BN, TL::THREADS>(b + SG::M_OPERAND, k_ext & (Q_BK - 1));
             __syncthreads();
         }
     };
@@ -327,7 +328,7 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
         }
     }
     fix_tail(0, 0);
-    Frags<TMB, WM, M_KS, N_KS, TMC, TMCW> f0, f1;
+    Frags<TMB, WM, WN, M_KS, N_KS, TMC, TMCW> f0, f1;
     f0.read(smem, wm, wn, 0);
     if constexpr (NO_READS) f1.read(smem, wm, wn, 1);
     int cur_b = 0;                    // ring buffer of stage s
@@ -391,8 +392,8 @@ template <int EPI> __device__ __forceinline__ void load_bias(const GemmArgs &g, 
 // per lane out, 8 rows per store instruction.  The pre-activation that GELU' needs comes in the same way,
 // in the opposite direction.  TMCW is a compile-time bound so that the work of different cells can be
 // interleaved.  live: the wave's live rows.
-template <int TMB, int WM, bool WG, int EPI, int TMC>
-__device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<TMB, WM>::TMW][2], char *smem, int lane, int wave,
+template <int TMB, int WM, int WN, bool WG, int EPI, int TMC>
+__device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<TMB, WM, WN>::TMW][2], char *smem, int lane, int wave,
                                          int wn, int e, long row0, int m0, int n0, int m_ext, int live,
                                          const uint2 (&bias_raw)[8]) {
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
@@ -403,7 +404,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<T
     long crow0 = row0;
     if constexpr (WG) { crow0 = 0; Cb += (long)e * g.strideC; }
     const int nw0 = n0 + wn * 64;                   // first column of this wave's slab
-    char *slab = smem + wave * (Tile<TMB, WM>::TMW * 32 * 128);
+    char *slab = smem + wave * (Tile<TMB, WM, WN>::TMW * 32 * 128);
     const int jr = lane >> 3, jc = lane & 7;        // row-in-group / 16-byte column of the wide accesses
     const bool col_ok = nw0 + jc * 8 < g.N;
 
@@ -614,11 +615,11 @@ __device__ __forceinline__ void store_sums(const GemmArgs &g, const f32x16 &sums
 
 // Row-ragged (!WG): C[rows_e, N] = Mop[rows_e, K] . Nop_e ; Mop K-contiguous, Nop_e [N,K] or (N_KS) [K,N].
 // Weight gradient (WG): C_e[M, N] = sum_{r in rows_e} Mop[r, M]^T . Nop[r, N], both K-strided.
-template <int TMB, int WM, bool N_KS, bool WG, int EPI>
-__global__ __launch_bounds__((Tile<TMB, WM>::THREADS), (Tile<TMB, WM>::BLOCKS_PER_CU)) void gemm256_kernel(const GemmArgs g) {
-    typedef Tile<TMB, WM> TL;
+template <int TMB, int WM, int WN, bool N_KS, bool WG, int EPI>
+__global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::WAVES_PER_SIMD)) void gemm256_kernel(const GemmArgs g) {
+    typedef Tile<TMB, WM, WN> TL;
     constexpr bool M_KS = WG;
-    constexpr int Q_BM = TL::BM, TMW = TL::TMW;
+    constexpr int Q_BM = TL::BM, Q_BN = TL::BN, TMW = TL::TMW;
     extern __shared__ __align__(16) char smem[];
     // ---- which tile am I?  Blocks are dealt round-robin to the 8 XCDs (block b runs on XCD b mod 8):
     //      give each XCD a contiguous range of the REAL tiles, so that neighbours share operands in
@@ -821,8 +822,9 @@ __global__ __launch_bounds__((Tile<TMB, WM>::THREADS), (Tile<TMB, WM>::BLOCKS_PE
             if (g.accumulate) return;
             typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
             bf16_t *Cz = (bf16_t *)g.C + (long)e * g.strideC;
-            const int col = n0 + (lane & 31) * 8;
-            for (int r = wave * 2 + (lane >> 5); r < Q_BM; r += 2 * TL::NW) {
+            constexpr int LPR = Q_BN / 8, RPW = WAVE / LPR;        // lanes per row piece, rows per wave and store
+            const int col = n0 + (lane % LPR) * 8;
+            for (int r = wave * RPW + lane / LPR; r < Q_BM; r += RPW * TL::NW) {
                 const int m = m0 + r;
                 if (m < m_ext && col < g.N)
                     __builtin_nontemporal_store(u32x4{0u, 0u, 0u, 0u}, reinterpret_cast<u32x4 *>(Cz + (long)m * g.ldc + col));
@@ -855,14 +857,14 @@ __global__ __launch_bounds__((Tile<TMB, WM>::THREADS), (Tile<TMB, WM>::BLOCKS_PE
     const int live = min(tile_h, m_ext - m0);
     const int tmc = (live + 31) >> 5;
     const int wu = __builtin_amdgcn_readfirstlane(wave);
-    const int wm = WM == 1 ? 0 : wu >> 2, wn = wu & 3;     // wave row / wave column
+    const int wm = wu / WN, wn = wu % WN;     // wave row / wave column
     uint2 bias_raw[8];
     load_bias<EPI>(g, e, n0, lane, wn, bias_raw);
     // Operand sums ride along in the weight-gradient blocks that see the whole operand once: one n-tile
     // of every m-tile for the m-side, one m-tile of every n-tile for the n-side.  These blocks run the
     // full tile shape (blocks past the operand's end repeat its last row and are not stored).
     int sum_side = 0;
-    if constexpr (WG && WM == 2 && TMW == 4) {
+    if constexpr (WG && WM == 2 && TMW <= WN) {
         if (g.colsum != nullptr && ((g.colsum_side == 1 && nt == sum_nt) || (g.colsum_side == 2 && mt == sum_mt))) sum_side = g.colsum_side;
     }
     // The live blocks are dealt evenly to the wave rows: c to each (the last row may find fewer live).
@@ -874,37 +876,31 @@ __global__ __launch_bounds__((Tile<TMB, WM>::THREADS), (Tile<TMB, WM>::BLOCKS_PE
     for (int q = 0; q < 16; ++q) sums[q] = 0.f;
 #define MOLE_RUN_TILE_SUM(C, SUM)                                                                                         \
     {                                                                                                                     \
-        main_loop<TMB, WM, M_KS, N_KS, WG, WM *(C), (C), SUM, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw); \
+        main_loop<TMB, WM, WN, M_KS, N_KS, WG, WM *(C), (C), SUM, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw); \
         if constexpr (SUM != 0) store_sums<SUM, (C)>(g, sums, e, m0, n0, m_ext, wm, wn, lane);                            \
-        epilogue<TMB, WM, WG, EPI, (C)>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, bias_raw);      \
+        epilogue<TMB, WM, WN, WG, EPI, (C)>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, bias_raw);      \
     }
 #define MOLE_RUN_TILE(C) MOLE_RUN_TILE_SUM(C, 0)
-    if constexpr (WG && WM == 2 && TMW == 4) {
+    if constexpr (WG && WM == 2 && TMW <= WN) {
         if (sum_side == 1) { MOLE_RUN_TILE_SUM(TMW, 1) return; }
         if (sum_side == 2) { MOLE_RUN_TILE_SUM(TMW, 2) return; }
     }
-    if constexpr (WM == 1) {
-        if (c > TMB / 2) MOLE_RUN_TILE(TMB)
-        else if (c > TMB / 4) MOLE_RUN_TILE(TMB / 2)
-        else MOLE_RUN_TILE(TMB / 4)
-    } else {
-        if (c >= TMW) MOLE_RUN_TILE(TMW)
-        else if (TMW > 4 && c == 4) MOLE_RUN_TILE(TMW > 4 ? 4 : 1)
-        else if (c == 3) MOLE_RUN_TILE(3)
-        else if (c == 2) MOLE_RUN_TILE(2)
-        else MOLE_RUN_TILE(1)
-    }
+    if (c >= TMW) MOLE_RUN_TILE(TMW)
+    else if (TMW > 4 && c == 4) MOLE_RUN_TILE(TMW > 4 ? 4 : 1)
+    else if (TMW > 3 && c == 3) MOLE_RUN_TILE(TMW > 3 ? 3 : 1)
+    else if (TMW > 2 && c == 2) MOLE_RUN_TILE(TMW > 2 ? 2 : 1)
+    else MOLE_RUN_TILE(1)
 #undef MOLE_RUN_TILE
 #undef MOLE_RUN_TILE_SUM
 }
 
-template <int TMB, int WM, bool N_KS, bool WG, int EPI>
+template <int TMB, int WM, int WN, bool N_KS, bool WG, int EPI>
 static int launch256(GemmArgs g, int tiles, hipStream_t st, int kid) {
-    typedef Tile<TMB, WM> TL;
+    typedef Tile<TMB, WM, WN> TL;
     if (tiles <= 0) return 0;
     g.n_blocks = tiles;
     const int grid = (tiles + 7) & ~7;
-    auto kern = gemm256_kernel<TMB, WM, N_KS, WG, EPI>;
+    auto kern = gemm256_kernel<TMB, WM, WN, N_KS, WG, EPI>;
     static bool attr_done = false;
     if (!attr_done) {
         MOLE_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS_BYTES));
@@ -918,7 +914,7 @@ static int launch256(GemmArgs g, int tiles, hipStream_t st, int kid) {
 // Launch options and their defaults; a -DMOLE_TUNING build reads them from the environment
 // (MOLE_MFAST: bit mask of the products that number an expert's tiles m-tile first within groups of MOLE_MFAST_G
 // n-tiles, MOLE_MFAST_FROM: m-tiles an expert needs for that order, MOLE_WG_EMAJOR: expert count from which a weight gradient keeps an expert's blocks on one XCD,
-// MOLE_TMB: 4 | 8 = four-wave tiles of 128 | 256 rows, 16 = the 256-row eight-wave tile for every product,
+// MOLE_TMB: 128 = the 128 x 128 tile, 16 = the 256-row one, for every row-ragged product,
 // MOLE_NO_SUMS: bias gradients from their own kernel).
 #ifdef MOLE_TUNING
 static int env_int(const char *name, int dflt) { const char *v = getenv(name); return v ? atoi(v) : dflt; }
@@ -937,18 +933,18 @@ static int forced_tile() { return 0; }
 static bool sums_off() { return false; }
 #endif
 
-template <int TMB, int WM>
+template <int TMB, int WM, int WN>
 static int dispatch256(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid) {
-    constexpr int BM = Tile<TMB, WM>::BM;
-    const int n_tiles = ceil_div(g.N, Q_BN);
-    if constexpr (TMB != 10) {
+    constexpr int BM = Tile<TMB, WM, WN>::BM;
+    const int n_tiles = ceil_div(g.N, (Tile<TMB, WM, WN>::BN));
+    if constexpr (TMB == 8) {
         if (wg) {
             GemmArgs gw = g;
             gw.wg_expert_major = g.E >= wg_emajor_from();
             // whole (expert, m-tile) units per XCD, or whole experts
             const int tiles = gw.wg_expert_major ? 8 * ceil_div(g.E, 8) * ceil_div(g.M, BM) * n_tiles
                                                  : 8 * ceil_div(g.E * ceil_div(g.M, BM), 8) * n_tiles;
-            if (epi == EPI_WGRAD) return launch256<TMB, WM, true, true, EPI_WGRAD>(gw, tiles, st, kid);
+            if (epi == EPI_WGRAD) return launch256<TMB, WM, WN, true, true, EPI_WGRAD>(gw, tiles, st, kid);
             return -100;
         }
     }
@@ -962,22 +958,22 @@ static int dispatch256(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_r
     if (wg) return -100;
     if (!b_ks) {
         if constexpr (TMB != 10) {
-            if (epi == EPI_DGELU) return launch256<TMB, WM, false, false, EPI_DGELU>(gg, tiles, st, kid);
-            if (epi == EPI_BIAS_GELU) return launch256<TMB, WM, false, false, EPI_BIAS_GELU>(gg, tiles, st, kid);
-            if (epi == EPI_F32) return launch256<TMB, WM, false, false, EPI_F32>(gg, tiles, st, kid);
-            if (epi == EPI_NONE) return launch256<TMB, WM, false, false, EPI_NONE>(gg, tiles, st, kid);
+            if (epi == EPI_DGELU) return launch256<TMB, WM, WN, false, false, EPI_DGELU>(gg, tiles, st, kid);
+            if (epi == EPI_BIAS_GELU) return launch256<TMB, WM, WN, false, false, EPI_BIAS_GELU>(gg, tiles, st, kid);
+            if constexpr (TMB == 8) if (epi == EPI_F32) return launch256<TMB, WM, WN, false, false, EPI_F32>(gg, tiles, st, kid);
+            if constexpr (TMB == 8) if (epi == EPI_NONE) return launch256<TMB, WM, WN, false, false, EPI_NONE>(gg, tiles, st, kid);
 #ifdef MOLE_TUNING
-            if constexpr (TMB == 8 && WM == 2) {     // the loop's parts are probed at the default tile shape only
-                if (epi == EPI_NONE + 1) return launch256<TMB, WM, false, false, EPI_NONE + 1>(gg, tiles, st, kid);
-                if (epi == EPI_NONE + 2) return launch256<TMB, WM, false, false, EPI_NONE + 2>(gg, tiles, st, kid);
-                if (epi == EPI_NONE + 3) return launch256<TMB, WM, false, false, EPI_NONE + 3>(gg, tiles, st, kid);
-                if (epi == EPI_NONE + 4) return launch256<TMB, WM, false, false, EPI_NONE + 4>(gg, tiles, st, kid);
+            if constexpr (TMB == 8 && WM == 2 && WN == 4) {     // the loop's parts are probed at the default tile shape only
+                if (epi == EPI_NONE + 1) return launch256<TMB, WM, WN, false, false, EPI_NONE + 1>(gg, tiles, st, kid);
+                if (epi == EPI_NONE + 2) return launch256<TMB, WM, WN, false, false, EPI_NONE + 2>(gg, tiles, st, kid);
+                if (epi == EPI_NONE + 3) return launch256<TMB, WM, WN, false, false, EPI_NONE + 3>(gg, tiles, st, kid);
+                if (epi == EPI_NONE + 4) return launch256<TMB, WM, WN, false, false, EPI_NONE + 4>(gg, tiles, st, kid);
             }
 #endif
         }
     } else {
-        if (epi == EPI_BIAS) return launch256<TMB, WM, true, false, EPI_BIAS>(gg, tiles, st, kid);
-        if (epi == EPI_STORE) return launch256<TMB, WM, true, false, EPI_STORE>(gg, tiles, st, kid);
+        if (epi == EPI_BIAS) return launch256<TMB, WM, WN, true, false, EPI_BIAS>(gg, tiles, st, kid);
+        if (epi == EPI_STORE) return launch256<TMB, WM, WN, true, false, EPI_STORE>(gg, tiles, st, kid);
     }
     return -100;
 }
@@ -990,19 +986,29 @@ static int dispatch256(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_r
 // remainder tiles, numbered last, fill the final round, which measured better than the even split
 // (t = (go.w2^T) gelu'(h): 213 against 219 us) - and h = xd.w1^T + b1 with the GELU epilogue would spill at
 // the 160 accumulators of the larger tile.
-static int tile_blocks_for(int kid) {
+// 128 x 128 tiles of four waves, two blocks to a CU, where the large tiles would leave half of the CUs without one: a
+// row-ragged product is then a few long serial walks over K.  16 experts of 256 rows, 512 -> 1024: h 20.9 -> 14.7 us, out
+// 30.0 -> 16.9; 8 experts of 256 rows, 1024 -> 4096: out 99 -> 54 us.  With a tile for half of the CUs or more the two are
+// even (32 experts of 125 rows, 1024 -> 2048: out 51.7 against 51.2 us, h 44 against 47) and beyond the large tile's
+// fewer operand bytes per flop win (16 experts of 375 rows, 1024 -> 4096: h 83 against 109 us).
+enum { TILE_256, TILE_320, TILE_128 };
+static int tile_for(const GemmArgs &g, bool wg, bool b_ks, int max_rows, int kid) {
     const int forced = forced_tile();
-    if (forced == 4 || forced == 8 || forced == 16) return forced;
-    return (kid == MOLE_K_FFN_FWD2 || kid == MOLE_K_FFN_GX) ? 20 : 16;
+    if (forced == 128) return TILE_128;
+    const bool tall = kid == MOLE_K_FFN_FWD2 || kid == MOLE_K_FFN_GX;
+    if (!wg && g.offsets != nullptr && forced == 0) {
+        const int active = g.E < max_rows ? g.E : max_rows;
+        const int avg = active > 0 ? ceil_div(max_rows, active) : 0;          // rows of an expert if they spread evenly
+        const long tiles = (long)active * ceil_div(avg, tall ? 320 : 256) * ceil_div(g.N, 256);
+        if (tiles < 112) return TILE_128;
+    }
+    return tall && b_ks && !wg ? TILE_320 : TILE_256;
 }
 
-// Whether the weight-gradient launch for g will also produce the operand sums asked for in g.colsum
-// (the eight-wave 256-row tile does; the tuning variants and the generic kernel do not).
-bool gemm256_sums_operand(const GemmArgs &g, int kid) {
+// Whether the weight-gradient launch for g will also produce the operand sums asked for in g.colsum.
+bool gemm256_sums_operand(const GemmArgs &g) {
     if (g.lda % 8 || g.ldb % 8 || g.ldc % 8 || g.N % 8 || g.M % 8) return false;
-    const int tmb = tile_blocks_for(kid);
-    if (sums_off()) return false;
-    return tmb == 16 || tmb == 20;
+    return !sums_off();
 }
 
 int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid) {
@@ -1010,13 +1016,10 @@ int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, in
     if (g.lda % 8 || g.ldb % 8 || g.ldc % 8 || g.N % 8) return -100;
     if (!wg && (a_ks || g.K % Q_BK)) return -100;
     if (wg && (!a_ks || !b_ks || g.M % 8)) return -100;
-    const int tmb = tile_blocks_for(kid);
-#ifdef MOLE_TUNING
-    if (tmb == 4) return dispatch256<4, 1>(g, b_ks, wg, epi, max_rows, st, kid);
-    if (tmb == 8) return dispatch256<8, 1>(g, b_ks, wg, epi, max_rows, st, kid);
-#endif
-    if (tmb == 20 && !wg && b_ks) return dispatch256<10, 2>(g, b_ks, wg, epi, max_rows, st, kid);   // up to 320 rows, eight waves
-    return dispatch256<8, 2>(g, b_ks, wg, epi, max_rows, st, kid);                                  // 256 rows, eight waves
+    const int tile = tile_for(g, wg, b_ks, max_rows, kid);
+    if (tile == TILE_128) return dispatch256<4, 2, 2>(g, b_ks, wg, epi, max_rows, st, kid);
+    if (tile == TILE_320) return dispatch256<10, 2, 4>(g, b_ks, wg, epi, max_rows, st, kid);
+    return dispatch256<8, 2, 4>(g, b_ks, wg, epi, max_rows, st, kid);
 }
 
 }  // namespace mole
