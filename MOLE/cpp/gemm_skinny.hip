@@ -336,25 +336,37 @@ __global__ __launch_bounds__(SK_THREADS, 4) void skinny_ks_kernel(const GemmArgs
     else skinny_ks_run<T, MB, EPI>(g, red, e, rows, row0, m0, n0, split);
 }
 
-// out[row][n] = sum over the planes of part[plane][row][n] (the bias is in plane 0), rows of every expert
+// out[row][n] = sum over the planes of part[plane][row][n] (the bias is in plane 0), for the rows of the launch's experts
+// only: the rows between them belong to experts of other launches (offloaded experts run in chunks).
+constexpr int SK_RED_ROWS = 4;
 template <typename T>
-__global__ __launch_bounds__(256) void skinny_reduce_kernel(const float *__restrict__ part, long part_rows, int N, int ksplit, T *__restrict__ out) {
-    const long row = blockIdx.y;
+__global__ __launch_bounds__(256) void skinny_reduce_kernel(const GemmArgs g) {
+    int e, grp, rows;
+    long row0;
+    if (!sk_find_group<SK_RED_ROWS>(g, blockIdx.y, e, grp, rows, row0)) return;
     const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
-    if (n >= N) return;
-    const float *p = part + row * N + n;
-    const long plane = part_rows * N;
-    float4 s = *reinterpret_cast<const float4 *>(p);
-    for (int k = 1; k < ksplit; k += 4) {
-        float4 t[4];
+    if (n >= g.N) return;
+    const long plane = g.part_rows * g.N;
+    const int m0 = grp * SK_RED_ROWS;
+    float4 s[SK_RED_ROWS];
+    const float *p[SK_RED_ROWS];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) t[u] = *reinterpret_cast<const float4 *>(p + (long)min(k + u, ksplit - 1) * plane);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (k + u < ksplit) { s.x += t[u].x; s.y += t[u].y; s.z += t[u].z; s.w += t[u].w; }
+    for (int i = 0; i < SK_RED_ROWS; ++i) {            // (rows past the expert's end repeat its last one and are not stored)
+        p[i] = g.part + (row0 + min(m0 + i, rows - 1)) * g.N + n;
+        s[i] = *reinterpret_cast<const float4 *>(p[i]);
     }
-    float v[4] = {s.x, s.y, s.z, s.w};
-    sk_store4<T>(out + row * N + n, v);
+    for (int k = 1; k < g.ksplit; ++k) {
+        float4 t[SK_RED_ROWS];
+#pragma unroll
+        for (int i = 0; i < SK_RED_ROWS; ++i) t[i] = *reinterpret_cast<const float4 *>(p[i] + (long)k * plane);
+#pragma unroll
+        for (int i = 0; i < SK_RED_ROWS; ++i) { s[i].x += t[i].x; s[i].y += t[i].y; s[i].z += t[i].z; s[i].w += t[i].w; }
+    }
+#pragma unroll
+    for (int i = 0; i < SK_RED_ROWS; ++i) {
+        float v[4] = {s[i].x, s[i].y, s[i].z, s[i].w};
+        if (m0 + i < rows) sk_store4<T>((T *)g.C + (row0 + m0 + i) * g.ldc + n, v);
+    }
 }
 
 // ---- which products come here, and how they are cut ------------------------------------------------------------
@@ -421,7 +433,7 @@ static int launch_ks(const GemmArgs &g, int epi, int groups, int max_rows, hipSt
     else return -100;
     MOLE_LAUNCH_CHECK();
     if (g.ksplit > 1) {
-        hipLaunchKernelGGL(skinny_reduce_kernel<T>, dim3(ceil_div(g.N, 1024), max_rows), dim3(256), 0, st, g.part, g.part_rows, g.N, g.ksplit, (T *)g.C);
+        hipLaunchKernelGGL(skinny_reduce_kernel<T>, dim3(ceil_div(g.N, 1024), (g.E < max_rows ? g.E : max_rows) + max_rows / SK_RED_ROWS), dim3(256), 0, st, g);
         MOLE_LAUNCH_CHECK();
     }
     return 0;

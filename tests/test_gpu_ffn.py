@@ -382,3 +382,30 @@ def test_ffn_few_rows_matches_oracle(E, M, Fd, rows, gap, dtype):
     L.check(L.lib().mole_ffn_fwd(L.ptr(c["xd"]), L.dtype_code(dtype), L.ptr(off), L.ptr(n), E, d["R"], M, Fd, L.ptr(c["w1"]),
                                  L.ptr(c["b1"]), L.ptr(c["w2"]), L.ptr(c["b2"]), L.ptr(h2), L.ptr(a2), L.ptr(out2), L.stream()), "ffn")
     assert torch.equal(h2.cpu()[mask], h.cpu()[mask]) and rel_err(out2.cpu()[mask], w_out[mask]) < t
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_ffn_few_rows_leaves_other_experts_rows_alone(dtype):
+    """A launch over some of the experts (offloaded experts run in chunks) with its contraction split over blocks: rows of
+    experts outside the launch keep what they hold, in the forward's out and in the backward's gx."""
+    from mole_amd import hip_ops as H
+    E, M, Fd, rows = 4, 256, 4096, [3, 5, 2, 6]
+    print(f"ffn few rows, chunk {dtype}", flush=True)
+    d = _make(E, M, Fd, rows, dtype, seed=3)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off = torch.from_numpy(d["off"]).cuda(); n = torch.from_numpy(d["n"]).cuda()
+    R = d["R"]
+    h, a = (torch.empty(R, Fd, dtype=dtype, device="cuda") for _ in range(2))
+    t = torch.empty_like(h)
+    out, gx = (torch.full((R, M), 7.0, dtype=dtype, device="cuda") for _ in range(2))
+    w_out, _, w_gx, *_ = _oracle_fwd_bwd(d, "tanh")
+    junk = torch.full((64 * R * M,), float("nan"), device="cuda")      # what the workspace's memory may hold
+    del junk
+    lo, hi = int(d["off"][1]), int(d["off"][3])
+    ws = [c[k][1:3] for k in ("w1", "b1", "w2", "b2")]
+    H.ffn_fwd_into(c["xd"], off[1:], n[1:], 2, R, M, Fd, *ws, h, a, out)
+    g = [torch.empty_like(w) for w in ws]
+    H.ffn_bwd_into(c["go"], c["xd"], h, a, off[1:], n[1:], 2, R, M, Fd, ws[0], ws[2], t, *g, gx, False, 0)
+    assert rel_err(out.cpu()[lo:hi], w_out[lo:hi]) < tol(dtype) and rel_err(gx.cpu()[lo:hi], w_gx[lo:hi]) < tol(dtype)
+    for buf in (out, gx):
+        assert float((torch.cat([buf[:lo], buf[hi:]]) - 7.0).abs().max()) == 0.0
