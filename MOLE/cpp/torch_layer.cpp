@@ -1,0 +1,211 @@
+// The layer as one autograd node in C++: allocation of a call's buffers, the argument block of mole_layer_fwd /
+// mole_layer_bwd, and the node autograd records.  Built into mole_torch.so beside libmole_hip.so, which it calls through the
+// C ABI; there is no GPU code here.
+//
+// Why it exists: with the same two calls made from Python a training step of a small layer spent 250 us on the host, 50 of
+// them in the library.  The rest was an autograd.Function and its context in Python, tensor allocations through the
+// interpreter and argument blocks through ctypes, half of it on autograd's own thread.
+#include <torch/extension.h>
+#include <c10/hip/HIPStream.h>
+
+#include <atomic>
+
+#include "mole_hip.h"
+
+namespace {
+
+using torch::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+void check(int rc, const char *what) {
+    TORCH_CHECK(rc == 0, what, " failed (code ", rc, "): ", mole_last_error_string());
+}
+int64_t up256(int64_t v) { return (v + 255) & ~(int64_t)255; }
+
+// Passes a layer has been through backward, shared with the Python side (MOLECore.step)
+struct Counter {
+    std::atomic<int64_t> value;
+    explicit Counter(int64_t v) : value(v) {}
+};
+
+// Sizes of one layer call, shared by every call of the same shape: the kept rows' bound, and where each intermediate lies
+// in the three buffers of a call - route (scores and routing, kept for the backward), act (xd, h, a, out and the forward's
+// scratch) and grad (the backward's temporaries and scratch).  Holds no device memory.
+struct Plan {
+    mole_layer head{};
+    at::ScalarType dtype;
+    int gelu_bwd;
+    enum { SCORES, GATES, L_AUX, IDX, LOC, ROW, COUNTS, KEPT, OFFSETS, CAPACITY, N_ROUTE };
+    enum { XD, H, A, OUT, ACT_WS, N_ACT };
+    enum { D_O, T, GXD, DLOGITS, GRAD_WS, N_GRAD };
+    int64_t route_off[N_ROUTE], act_off[N_ACT], grad_off[N_GRAD];
+    int64_t route_bytes, act_bytes, grad_bytes, ws_fwd, ws_bwd;
+
+    template <int N> static int64_t carve(const int64_t (&bytes)[N], int64_t (&off)[N]) {
+        int64_t at = 0;
+        for (int i = 0; i < N; ++i) {
+            off[i] = at;
+            at += up256(bytes[i]);
+        }
+        return at;
+    }
+
+    Plan(int dtype_code, int64_t S, int64_t M, int64_t E, int64_t k, int64_t F, double cf, int layout, bool normalize, int gelu)
+        : dtype(dtype_code == MOLE_BF16 ? at::kBFloat16 : at::kFloat), gelu_bwd(gelu) {
+        TORCH_CHECK(S >= 1 && M >= 1 && E >= 1 && k >= 1 && F >= 1 && S * k < (1ll << 31), "bad layer sizes");
+        const int64_t es = dtype_code == MOLE_BF16 ? 2 : 4;
+        int64_t rows = S * k;
+        if (cf > 0) {
+            // the reference's integer: k * int(cf * ceil(S / E)), the product in double precision
+            const int64_t cap = k * (int64_t)(cf * (double)((S + E - 1) / E));
+            rows = layout == MOLE_LAYOUT_PADDED ? E * cap : std::min(rows, E * cap);
+        }
+        rows = std::max<int64_t>(rows, 1);
+        TORCH_CHECK(rows < (1ll << 31), "too many rows");
+        head.dtype = dtype_code; head.S = (int)S; head.M = (int)M; head.E = (int)E; head.k = (int)k; head.F = (int)F;
+        head.rows = (int)rows; head.layout = layout; head.normalize_gate = normalize; head.capacity_factor = cf;
+        ws_fwd = (int64_t)mole_layer_workspace_bytes(&head, 0);
+        ws_bwd = (int64_t)mole_layer_workspace_bytes(&head, 1);
+        route_bytes = carve({S * E * 4, k * S * 4, 4, k * S * 4, k * S * 4, k * S * 4, k * E * 4, E * 4, (E + 1) * 4, 4}, route_off);
+        act_bytes = carve({rows * M * es, rows * F * es, rows * F * es, rows * M * es, ws_fwd}, act_off);
+        grad_bytes = carve({rows * M * es, rows * F * es, rows * M * es, S * E * 4, ws_bwd}, grad_off);
+    }
+    std::vector<int64_t> route_offsets() const { return {route_off, route_off + N_ROUTE}; }
+};
+
+// What a backward pass needs beside the saved tensors: kept by the node until it is released.
+struct Call : torch::CustomClassHolder {
+    std::shared_ptr<Plan> plan;
+    std::shared_ptr<Counter> counter;
+    std::optional<Tensor> bias;
+    std::vector<Tensor> weights, grads;      // w1, b1, w2, b2 of all experts and their gradient buffers
+    bool accumulate = false;
+    Tensor route;                            // forward's result for the caller
+};
+
+void check_tensor(const Tensor &t, const char *name) {
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous(), "mole_amd: ", name, " must be a contiguous tensor on the GPU (there is no CPU path)");
+}
+
+mole_layer arguments(const Call &c, const Tensor &x, const Tensor &wg, char *route, char *act, char *ws, int64_t ws_bytes) {
+    const Plan &p = *c.plan;
+    mole_layer L = p.head;
+    L.x = x.data_ptr();
+    L.wg = wg.data_ptr<float>();
+    L.logit_bias = c.bias.has_value() ? c.bias->data_ptr<float>() : nullptr;
+    L.w1 = c.weights[0].data_ptr(); L.b1 = c.weights[1].data_ptr(); L.w2 = c.weights[2].data_ptr(); L.b2 = c.weights[3].data_ptr();
+    L.scores = (float *)(route + p.route_off[Plan::SCORES]);
+    L.gates = (float *)(route + p.route_off[Plan::GATES]);
+    L.l_aux = (float *)(route + p.route_off[Plan::L_AUX]);
+    L.idx = (int32_t *)(route + p.route_off[Plan::IDX]);
+    L.loc = (int32_t *)(route + p.route_off[Plan::LOC]);
+    L.row = (int32_t *)(route + p.route_off[Plan::ROW]);
+    L.counts = (int32_t *)(route + p.route_off[Plan::COUNTS]);
+    L.kept_rows = (int32_t *)(route + p.route_off[Plan::KEPT]);
+    L.offsets = (int32_t *)(route + p.route_off[Plan::OFFSETS]);
+    L.capacity = (int32_t *)(route + p.route_off[Plan::CAPACITY]);
+    L.xd = act + p.act_off[Plan::XD]; L.h = act + p.act_off[Plan::H]; L.a = act + p.act_off[Plan::A]; L.out = act + p.act_off[Plan::OUT];
+    L.workspace = ws;
+    L.workspace_bytes = (size_t)ws_bytes;
+    return L;
+}
+
+void *current_stream(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+
+// (y, act); c.route is set.  l_aux: where the loss term goes, or undefined (it then stays inside route).
+std::pair<Tensor, Tensor> run_forward(Call &c, const Tensor &x, const Tensor &wg, const Tensor &l_aux) {
+    const Plan &p = *c.plan;
+    check_tensor(x, "x");
+    check_tensor(wg, "the gate's weight");
+    TORCH_CHECK(x.dim() == 2 && x.size(0) == p.head.S && x.size(1) == p.head.M && x.scalar_type() == p.dtype &&
+                    wg.dim() == 2 && wg.size(0) == p.head.E && wg.size(1) == p.head.M && wg.scalar_type() == at::kFloat,
+                "mole_amd: the layer's input or gate does not have the planned shape or type");
+    const auto bytes = x.options().dtype(at::kByte);
+    c.route = at::empty({p.route_bytes}, bytes);
+    Tensor act = at::empty({p.act_bytes}, bytes), y = at::empty({p.head.S, p.head.M}, x.options());
+    char *a = (char *)act.data_ptr();
+    mole_layer L = arguments(c, x, wg, (char *)c.route.data_ptr(), a, a + p.act_off[Plan::ACT_WS], p.ws_fwd);
+    if (l_aux.defined()) L.l_aux = l_aux.data_ptr<float>();
+    check(mole_layer_fwd(&L, y.data_ptr(), current_stream(x)), "mole_layer_fwd");
+    return {y, act};
+}
+
+struct LayerFn : torch::autograd::Function<LayerFn> {
+    // dummy: an empty parameter that makes autograd record the node although x need not require a gradient
+    static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &wg, const Tensor &dummy, c10::intrusive_ptr<Call> c) {
+        (void)dummy;
+        ctx->set_materialize_grads(false);
+        Tensor l_aux = at::empty({}, x.options().dtype(at::kFloat));
+        auto [y, act] = run_forward(*c, x, wg, l_aux);
+        ctx->save_for_backward({x, wg, c->route, act});
+        ctx->saved_data["call"] = c10::IValue::make_capsule(std::move(c));
+        return {y, l_aux};
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list g) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &wg = saved[1], &route = saved[2], &act = saved[3];
+        auto c = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
+        const Plan &p = *c->plan;
+        Tensor dy = g[0].defined() ? g[0].contiguous() : at::zeros_like(x);      // (undefined: only l_aux was used)
+        Tensor d_aux = g[1].defined() ? g[1].to(at::kFloat).contiguous() : Tensor();
+        TORCH_CHECK(dy.scalar_type() == p.dtype && dy.numel() == x.numel(), "mole_amd: the output's gradient has another shape or type");
+        Tensor tmp = at::empty({p.grad_bytes}, x.options().dtype(at::kByte));
+        Tensor dx = at::empty({p.head.S, p.head.M}, x.options()), dwg = at::empty({p.head.E, p.head.M}, wg.options());
+        char *t = (char *)tmp.data_ptr();
+        mole_layer L = arguments(*c, x, wg, (char *)route.data_ptr(), (char *)act.data_ptr(), t + p.grad_off[Plan::GRAD_WS], p.ws_bwd);
+        mole_layer_grads G{};
+        G.accumulate = c->accumulate;
+        G.gelu_bwd = p.gelu_bwd;
+        G.dy = dy.data_ptr();
+        G.d_l_aux = d_aux.defined() ? d_aux.data_ptr<float>() : nullptr;
+        G.dlogits = (float *)(t + p.grad_off[Plan::DLOGITS]);
+        G.d_o = t + p.grad_off[Plan::D_O]; G.t = t + p.grad_off[Plan::T]; G.gxd = t + p.grad_off[Plan::GXD];
+        G.g_w1 = c->grads[0].data_ptr(); G.g_b1 = c->grads[1].data_ptr(); G.g_w2 = c->grads[2].data_ptr(); G.g_b2 = c->grads[3].data_ptr();
+        G.dx = dx.data_ptr();
+        G.dwg = dwg.data_ptr<float>();
+        check(mole_layer_bwd(&L, &G, current_stream(x)), "mole_layer_bwd");
+        c->counter->value += 1;
+        return {dx, dwg, Tensor(), Tensor()};
+    }
+};
+
+// (y, l_aux or None, route)
+std::tuple<Tensor, std::optional<Tensor>, Tensor> layer(const Tensor &x, const Tensor &wg, const Tensor &dummy, std::optional<Tensor> bias,
+                                                        std::vector<Tensor> weights, std::vector<Tensor> grads,
+                                                        std::shared_ptr<Plan> plan, bool accumulate, std::shared_ptr<Counter> counter) {
+    TORCH_CHECK(weights.size() == 4 && grads.size() == 4, "mole_amd: four parameter and four gradient tensors");
+    auto c = c10::make_intrusive<Call>();
+    c->plan = std::move(plan);
+    c->counter = std::move(counter);
+    c->bias = std::move(bias);
+    c->weights = std::move(weights);
+    c->grads = std::move(grads);
+    c->accumulate = accumulate;
+    if (!at::GradMode::is_enabled()) {
+        auto ya = run_forward(*c, x, wg, Tensor());
+        return {ya.first, std::nullopt, c->route};
+    }
+    auto out = LayerFn::apply(x, wg, dummy, c);
+    return {out[0], out[1], c->route};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    py::class_<Counter, std::shared_ptr<Counter>>(m, "Counter")
+        .def(py::init<int64_t>())
+        .def_property("value", [](const Counter &c) { return c.value.load(); }, [](Counter &c, int64_t v) { c.value = v; })
+        .def(py::pickle([](const Counter &c) { return py::make_tuple(c.value.load()); },
+                        [](py::tuple t) { return std::make_shared<Counter>(t[0].cast<int64_t>()); }));
+    py::class_<Plan, std::shared_ptr<Plan>>(m, "Plan")
+        .def(py::init<int, int64_t, int64_t, int64_t, int64_t, int64_t, double, int, bool, int>())
+        .def("route_offsets", &Plan::route_offsets)
+        .def(py::pickle([](const Plan &p) { return py::make_tuple(p.head.dtype, p.head.S, p.head.M, p.head.E, p.head.k, p.head.F,
+                                                                  p.head.capacity_factor, p.head.layout, p.head.normalize_gate, p.gelu_bwd); },
+                        [](py::tuple t) { return std::make_shared<Plan>(t[0].cast<int>(), t[1].cast<int64_t>(), t[2].cast<int64_t>(),
+                                              t[3].cast<int64_t>(), t[4].cast<int64_t>(), t[5].cast<int64_t>(), t[6].cast<double>(),
+                                              t[7].cast<int>(), t[8].cast<int>() != 0, t[9].cast<int>()); }));
+    m.def("layer", &layer, py::call_guard<py::gil_scoped_release>());
+}

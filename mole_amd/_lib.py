@@ -7,6 +7,8 @@ holds is the one the library binds to.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from ctypes import POINTER, c_char_p, c_double, c_float, c_int, c_int32, c_int64, c_size_t, c_uint64, c_void_p
 
@@ -22,23 +24,6 @@ KERNEL_IDS = ("ffn_fwd1", "ffn_fwd2", "ffn_gw2", "ffn_da", "ffn_gw1", "ffn_gx", 
               "combine_fwd", "combine_bwd", "route", "gemm_nt", "adam", "gate_fwd", "gate_bwd", "gate_wgrad", "probe")
 
 _P = c_void_p
-
-
-class LayerArgs(ctypes.Structure):
-    """mole_layer of include/mole_hip.h."""
-    _fields_ = ([(n, c_int32) for n in ("dtype", "S", "M", "E", "k", "F", "rows", "layout", "normalize_gate")]
-                + [("capacity_factor", c_double)]
-                + [(n, c_void_p) for n in ("x", "wg", "logit_bias", "w1", "b1", "w2", "b2", "scores", "gates", "l_aux", "idx", "loc",
-                                           "row", "counts", "kept_rows", "offsets", "capacity", "xd", "h", "a", "out", "workspace")]
-                + [("workspace_bytes", c_size_t)])
-
-
-class LayerGrads(ctypes.Structure):
-    """mole_layer_grads of include/mole_hip.h."""
-    _fields_ = ([("accumulate", c_int32), ("gelu_bwd", c_int32)]
-                + [(n, c_void_p) for n in ("dy", "d_l_aux", "dlogits", "d_o", "t", "gxd", "g_w1", "g_b1", "g_w2", "g_b2", "dx", "dwg")])
-
-
 _SIGNATURES = {
     "mole_version": (c_int, []),
     "mole_last_error_string": (c_char_p, []),
@@ -76,9 +61,9 @@ _SIGNATURES = {
     "mole_ffn_fwd_ws": (c_int, [_P, c_int, _P, _P, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P, _P, c_size_t, _P]),
     "mole_ffn_bwd_ws": (c_int, [_P, _P, _P, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P,
                                 _P, c_int, c_int, _P, c_size_t, _P]),
-    "mole_layer_workspace_bytes": (c_size_t, [POINTER(LayerArgs), c_int]),
-    "mole_layer_fwd": (c_int, [POINTER(LayerArgs), _P, _P]),
-    "mole_layer_bwd": (c_int, [POINTER(LayerArgs), POINTER(LayerGrads), _P]),
+    "mole_layer_workspace_bytes": (c_size_t, [_P, c_int]),
+    "mole_layer_fwd": (c_int, [_P, _P, _P]),
+    "mole_layer_bwd": (c_int, [_P, _P, _P]),
     "mole_gemm_nt": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P]),
     "mole_gemm_nn": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P]),
     "mole_gemm_tn": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P]),
@@ -133,6 +118,24 @@ def lib() -> ctypes.CDLL:
             fn.restype, fn.argtypes = res, args
         _lib = handle
     return _lib
+
+
+TORCH_LIB_PATH = os.path.join(os.path.dirname(LIB_PATH), "mole_torch.so")
+_native = None
+
+
+def native():
+    """The layer's autograd node in C++ (MOLE/cpp/torch_layer.cpp); like the library it is the only implementation."""
+    global _native
+    if _native is None:
+        if not os.path.exists(TORCH_LIB_PATH):
+            raise RuntimeError(f"{TORCH_LIB_PATH} is missing: build it with `python -m mole_amd.build` (needs hipcc, no GPU).")
+        lib()
+        loader = importlib.machinery.ExtensionFileLoader("mole_torch", TORCH_LIB_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("mole_torch", loader))
+        loader.exec_module(module)
+        _native = module
+    return _native
 
 
 def last_error() -> str:

@@ -414,7 +414,8 @@ class MOLECore:
         self.adv_adam = bool(adv_adam)
         self.adam = None            # set_adam(): (beta1, beta2, t, lr, lam, eps, adamW)
         self.hybrid_adam_count = d_experts
-        self.use_pool, self.acc_step, self.step = bool(use_pool), int(acc_step), int(step)
+        self.use_pool, self.acc_step = bool(use_pool), int(acc_step)
+        self.passes = L.native().Counter(int(step))    # backward passes so far: the native layer node counts them too
         self.device, self.moe_id, self.total_experts = device, moe_id, total_experts
         self.s_experts, self.d_experts, self.ebatch_size = s_experts, d_experts, max(int(ebatch_size), 1)
         self.world_size, self.act_name = world_size, act_name
@@ -435,6 +436,14 @@ class MOLECore:
         # decided once per pass, by the first prefetch for it or by the forward itself, and carried to its backward.
         self._home_fwd = None       # decision for the coming forward pass (valid while experts are prefetched for it)
         self._home_pass = None      # decision of the last forward pass: its backward and the prefetches for it use it
+
+    @property
+    def step(self) -> int:
+        return self.passes.value
+
+    @step.setter
+    def step(self, v: int):
+        self.passes.value = int(v)
 
     # the reference's counters of experts prefetched so far (define.hpp:352-353)
     @property

@@ -427,86 +427,25 @@ def adam_step(p, g, m, v, beta1: float, beta2: float, t: int, lr: float, lam: fl
 
 
 # ---- the layer in one call each way (mole_layer_fwd / mole_layer_bwd) ---------------------------------------------
-def _carve(parts):
-    """({name: offset}, total) of named byte counts laid out one after the other on 256-byte boundaries."""
-    offs, at = {}, 0
-    for name, nbytes in parts:
-        offs[name] = at
-        at += (nbytes + 255) & ~255
-    return offs, at
-
-
 class LayerPlan:
-    """Sizes of one layer call, shared by every call of the same shape: the kept rows' bound, and where each intermediate
-    lies in the three buffers of a call - `route` (scores and routing, kept for the backward), `act` (xd, h, a, out and the
-    forward's scratch) and `grad` (the backward's temporaries and scratch)."""
+    """Sizes of one layer call, shared by every call of the same shape (the native Plan); route() gives the routing in a
+    call's `route` buffer as tensors."""
 
     def __init__(self, dtype, S, M, E, k, F, capacity_factor, layout, normalize_gate, gelu_bwd):
-        es = 2 if dtype == torch.bfloat16 else 4
-        self.S, self.M, self.E, self.k, self.F, self.layout, self.normalize_gate = S, M, E, k, F, layout, normalize_gate
-        self.capacity_factor, self.gelu_bwd, self.dtype = capacity_factor, gelu_bwd, dtype
-        rows = S * k
-        if capacity_factor > 0:
-            cap = k * int(capacity_factor * ((S + E - 1) // E))
-            rows = E * cap if layout == L.LAYOUT_PADDED else min(rows, E * cap)
-        self.rows = rows = max(rows, 1)
-        self.head = (L.dtype_code(dtype), S, M, E, k, F, rows, layout, int(normalize_gate), capacity_factor)
-        probe = L.LayerArgs(*self.head)
-        self.route_off, self.route_bytes = _carve((("scores", S * E * 4), ("gates", k * S * 4), ("l_aux", 4), ("idx", k * S * 4),
-                                                   ("loc", k * S * 4), ("row", k * S * 4), ("counts", k * E * 4), ("kept", E * 4),
-                                                   ("offsets", (E + 1) * 4), ("capacity", 4)))
-        self.ws_fwd = L.lib().mole_layer_workspace_bytes(probe, 0)
-        self.act_off, self.act_bytes = _carve((("xd", rows * M * es), ("h", rows * F * es), ("a", rows * F * es),
-                                               ("out", rows * M * es), ("ws", self.ws_fwd)))
-        self.ws_bwd = L.lib().mole_layer_workspace_bytes(probe, 1)
-        self.grad_off, self.grad_bytes = _carve((("d_o", rows * M * es), ("t", rows * F * es), ("gxd", rows * M * es),
-                                                 ("dlogits", S * E * 4), ("ws", self.ws_bwd)))
+        self.S, self.E, self.k, self.layout, self.normalize_gate = S, E, k, layout, normalize_gate
+        self.native = L.native().Plan(L.dtype_code(dtype), S, M, E, k, F, capacity_factor, layout, normalize_gate, gelu_bwd)
 
-    def route(self, buf: torch.Tensor) -> "Route":
-        """The routing result in a call's `route` buffer as tensors."""
-        def at(name, dt, *shape):
-            n = 1
+    def route(self, buf: torch.Tensor) -> Route:
+        offs = iter(self.native.route_offsets())
+
+        def take(dt, *shape):
+            o, n = next(offs), 1
             for d in shape:
                 n *= d
-            o = self.route_off[name]
             return buf[o:o + n * 4].view(dt).view(*shape)
-        S, E, k, i32 = self.S, self.E, self.k, torch.int32
-        return Route(S, E, k, self.layout, at("idx", i32, k, S), at("loc", i32, k, S), at("gates", torch.float32, k, S),
-                     at("row", i32, k, S), at("counts", i32, k, E), at("kept", i32, E), at("offsets", i32, E + 1),
-                     at("capacity", i32, 1), at("l_aux", torch.float32, 1), self.normalize_gate)
-
-    def _args(self, x, wg, logit_bias, weights, route, act, l_aux, ws, ws_bytes):
-        r, a, ro, ao = route.data_ptr(), act.data_ptr(), self.route_off, self.act_off
-        w1, b1, w2, b2 = weights
-        return L.LayerArgs(*self.head, x.data_ptr(), wg.data_ptr(), None if logit_bias is None else logit_bias.data_ptr(),
-                           w1.data_ptr(), b1.data_ptr(), w2.data_ptr(), b2.data_ptr(), r + ro["scores"], r + ro["gates"],
-                           r + ro["l_aux"] if l_aux is None else l_aux.data_ptr(), r + ro["idx"], r + ro["loc"], r + ro["row"],
-                           r + ro["counts"], r + ro["kept"], r + ro["offsets"], r + ro["capacity"], a + ao["xd"], a + ao["h"],
-                           a + ao["a"], a + ao["out"], ws, ws_bytes)
-
-    def forward(self, x, wg, logit_bias, weights, l_aux=None):
-        """(y, route, act): everything of a forward pass.  l_aux: a tensor of its own for the loss (else inside route)."""
-        _dev(x), _dev(wg)
-        dev = x.device
-        route = torch.empty(self.route_bytes, dtype=torch.uint8, device=dev)
-        act = torch.empty(self.act_bytes, dtype=torch.uint8, device=dev)
-        y = torch.empty(self.S, self.M, dtype=self.dtype, device=dev)
-        args = self._args(x, wg, logit_bias, weights, route, act, l_aux, act.data_ptr() + self.act_off["ws"], self.ws_fwd)
-        L.check(L.lib().mole_layer_fwd(args, y.data_ptr(), L.stream()), "mole_layer_fwd")
-        return y, route, act
-
-    def backward(self, dy, d_l_aux, x, wg, weights, route, act, grads, accumulate):
-        """(dx, dwg); the expert gradients go to `grads`."""
-        _dev(dy)
-        dev = x.device
-        tmp = torch.empty(self.grad_bytes, dtype=torch.uint8, device=dev)
-        dx = torch.empty(self.S, self.M, dtype=self.dtype, device=dev)
-        dwg = torch.empty(self.E, self.M, dtype=torch.float32, device=dev)
-        t, go = tmp.data_ptr(), self.grad_off
-        args = self._args(x, wg, None, weights, route, act, None, t + go["ws"], self.ws_bwd)
-        gw1, gb1, gw2, gb2 = grads
-        out = L.LayerGrads(int(accumulate), self.gelu_bwd, dy.data_ptr(), None if d_l_aux is None else d_l_aux.data_ptr(),
-                           t + go["dlogits"], t + go["d_o"], t + go["t"], t + go["gxd"], gw1.data_ptr(), gb1.data_ptr(),
-                           gw2.data_ptr(), gb2.data_ptr(), dx.data_ptr(), dwg.data_ptr())
-        L.check(L.lib().mole_layer_bwd(args, out, L.stream()), "mole_layer_bwd")
-        return dx, dwg
+        S, E, k, i32, f32 = self.S, self.E, self.k, torch.int32, torch.float32
+        take(f32, S, E)                                     # the scores
+        gates, l_aux = take(f32, k, S), take(f32, 1)
+        idx, loc, row = take(i32, k, S), take(i32, k, S), take(i32, k, S)
+        counts, kept, offsets, capacity = take(i32, k, E), take(i32, E), take(i32, E + 1), take(i32, 1)
+        return Route(S, E, k, self.layout, idx, loc, gates, row, counts, kept, offsets, capacity, l_aux, self.normalize_gate)

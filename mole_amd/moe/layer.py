@@ -7,9 +7,10 @@ Constructor and forward keep the reference's names, argument order and defaults
 Two execution shapes, same results:
   * fused (default): one autograd node over the ragged, expert-contiguous layout.  Nothing is
     padded, nothing is read back to the host, every step is a kernel of libmole_hip.so.
-    With all experts on the GPU that is one native call each way (mole_layer_fwd / mole_layer_bwd).
+    With all experts on the GPU that is one native autograd node (MOLE/cpp/torch_layer.cpp) with one library call each
+    way (mole_layer_fwd / mole_layer_bwd).
   * reference_layout=True: the reference's padded layout, expert e's rows at e*C of an [E, C, M] buffer.  With all experts on
-    the GPU and a capacity known on the host (capacity_factor > 0) the same two native calls, which compute the kept rows
+    the GPU and a capacity known on the host (capacity_factor > 0) the same node, which computes the kept rows
     only; otherwise the reference's literal call sequence - extract_critical, fast_encode into a zero-padded [E, C, M],
     BatchFusedFWD.apply over all E*C rows, fast_decode - with the same results (a padding row is zero and meets a zero
     gradient).
@@ -103,40 +104,6 @@ class _FusedMoE(torch.autograd.Function):
         if ctx.time_it:
             UATimer.track_bwd_end(m.moe_id)
         return dx, dwg, torch.zeros_like(m.dummy_param), None, None, None
-
-
-class _LayerFn(torch.autograd.Function):
-    """_FusedMoE for experts that all live on the GPU: the same steps, each direction one call of the library on buffers
-    laid out by a LayerPlan."""
-
-    @staticmethod
-    def forward(ctx, x, wg, dummy_param, module, plan, time_it):
-        m = module
-        ctx.set_materialize_grads(False)
-        l_aux = torch.empty((), dtype=torch.float32, device=x.device)
-        y, route, act = plan.forward(x, wg, m.gate[0].logit_bias, [g[0] for g in m.MOLECore.gpu], l_aux)
-        m._route = (plan, route)
-        ctx.m, ctx.plan, ctx.time_it = m, plan, time_it
-        ctx.save_for_backward(x, wg, route, act)
-        return y, l_aux
-
-    @staticmethod
-    def backward(ctx, dy, d_l_aux):
-        m = ctx.m
-        x, wg, route, act = ctx.saved_tensors
-        if dy is None:            # only l_aux was used
-            dy = torch.zeros_like(x)
-        if ctx.time_it:
-            UATimer.track_bwd_start(m.moe_id)
-        if d_l_aux is not None and d_l_aux.dtype != torch.float32:
-            d_l_aux = d_l_aux.float()
-        core_ = m.MOLECore
-        dx, dwg = ctx.plan.backward(dy.contiguous(), d_l_aux, x, wg, [g[0] for g in core_.gpu], route, act,
-                                    [g[1] for g in core_.gpu], core_.acc_step > 1)
-        core_.step += 1
-        if ctx.time_it:
-            UATimer.track_bwd_end(m.moe_id)
-        return dx, dwg, None, None, None, None
 
 
 class MOLEModule(torch.nn.Module):
@@ -266,7 +233,7 @@ class MOLEModule(torch.nn.Module):
 
     def _plan(self, S, capacity_factor, wg):
         """The LayerPlan of a forward pass over S tokens, or None when it takes the step-by-step path (experts offloaded, no
-        tokens, a gate in another dtype, a padded capacity that only the device knows)."""
+        tokens, a gate in another dtype, a padded capacity that only the device knows; a profiled pass also does)."""
         if (self.d_experts or not self.s_experts or S < 1 or wg.dtype != torch.float32 or not wg.is_contiguous()
                 or self.embed_dim % self._granule or self.ffn_dim % self._granule or (self.reference_layout and capacity_factor <= 0)):
             return None
@@ -337,13 +304,14 @@ class MOLEModule(torch.nn.Module):
 
         gate = self.gate[0]
         wg = gate.linear.weight
-        plan = self._plan(resized_input.shape[0], float(capacity_factor), wg)
+        plan = None if time_it else self._plan(resized_input.shape[0], float(capacity_factor), wg)
         if plan is not None:
-            if torch.is_grad_enabled():
-                expert_output, self.l_aux = _LayerFn.apply(resized_input, wg, self.dummy_param, self, plan, bool(time_it))
-            else:
-                expert_output, route, _ = plan.forward(resized_input, wg, gate.logit_bias, [g[0] for g in self.MOLECore.gpu])
-                self._route, self.l_aux = (plan, route), None
+            core_ = self.MOLECore
+            expert_output, l_aux, route = L.native().layer(
+                resized_input, wg, self.dummy_param, gate.logit_bias, [g[0] for g in core_.gpu], [g[1] for g in core_.gpu],
+                plan.native, core_.acc_step > 1, core_.passes)
+            self.__dict__["_route"] = (plan, route)
+            self.__dict__["_l_aux"] = l_aux
         elif self.reference_layout:
             scores = self.gate[0](resized_input)
             crit, l_aux = tutel_fast_dispatcher.extract_critical(
