@@ -79,12 +79,12 @@ template <int TMB, int WM, int WN, bool M_KS, int TMC> struct Stage {
 // of a ragged contraction has fewer than 32).
 template <int ROWS, int NW> struct OffKC {
     uint32_t off[ROWS / (16 * NW)];
-    __device__ __forceinline__ void init(long ld, int r_left) {
+    __device__ __forceinline__ void init(long ld, int r_left, int k_left) {
         const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
         for (int i = 0; i < ROWS / (16 * NW); ++i) {
             const int row = (NW * i + w) * 16 + (lane >> 2);
-            const int c = (lane & 3) ^ swz4(row);
+            const int c = min((lane & 3) ^ swz4(row), (k_left >> 3) - 1);     // (k_left is a multiple of 8)
             off[i] = (uint32_t)(min(row, r_left - 1) * ld * 2 + c * 16);
         }
     }
@@ -110,7 +110,14 @@ template <int ROWS, int NW> struct OffKS {
 template <int ROWS, int NW, bool KS> struct Off;
 template <int ROWS, int NW> struct Off<ROWS, NW, false> : OffKC<ROWS, NW> {};
 template <int ROWS, int NW> struct Off<ROWS, NW, true> : OffKS<ROWS, NW> {};
-// zero the k-rows [k_valid, 32) of a K-strided tile (the last, partial stage of a weight gradient)
+// zero the chunks of k from k_valid (a multiple of 8) on of a K-contiguous tile
+template <int ROWS, int THREADS> __device__ __forceinline__ void zero_kc_tail(char *lds, int k_valid) {
+    for (int idx = threadIdx.x; idx < ROWS * 4; idx += THREADS) {
+        const int row = idx >> 2, c = idx & 3;
+        if (c * 8 >= k_valid) *reinterpret_cast<uint4 *>(lds + row * 64 + ((c ^ swz4(row)) << 4)) = make_uint4(0, 0, 0, 0);
+    }
+}
+// zero the k-rows [k_valid, 32) of a K-strided tile (the last, partial stage of a ragged contraction)
 template <int ROWS, int THREADS> __device__ __forceinline__ void zero_k_tail(char *lds, int k_valid) {
     for (int idx = threadIdx.x; idx < (Q_BK - k_valid) * (ROWS / 8); idx += THREADS)
         *reinterpret_cast<uint4 *>(lds + k_valid * (ROWS * 2) + idx * 16) = make_uint4(0, 0, 0, 0);
@@ -186,7 +193,9 @@ template <int TMB, int WM, int WN, bool M_KS, bool N_KS, int TMC, int TMCW> stru
 // fixed for the whole K loop.  Stages are fetched in order; past the last one the last is fetched again,
 // harmlessly: it keeps the number of loads per stage, which the vmcnt arithmetic of the loop relies on.
 // Of a K-contiguous m-side tile only the 64-row groups that hold live 32-row blocks (the first TMC) are fetched.
-template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool WG, int TMC> struct Feeder {
+// KT: the contraction may end inside a stage (weight gradients always may; row-ragged products when K is not a multiple of
+// 32).  The last stage's loads are then clamped to what exists and main_loop zeroes what lies past it.
+template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC> struct Feeder {
     typedef Tile<TMB, WM, WN> TL;
     typedef Stage<TMB, WM, WN, M_KS, TMC> SG;
     static constexpr int LM = SG::LM, L = SG::L;
@@ -199,10 +208,10 @@ template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool WG, int TMC> struc
     bool ragged_k;
     __device__ __forceinline__ void init(const bf16_t *Mp, long ldm, int m0, int m_ext, const bf16_t *Np, long ldn, int n0,
                                          int n_ext, int k_ext, char *smem, int wave) {
-        if constexpr (M_KS) om.init(ldm, m_ext - m0, Q_BK); else om.init(ldm, m_ext - m0);
-        if constexpr (N_KS) on.init(ldn, n_ext - n0, Q_BK); else on.init(ldn, n_ext - n0);
-        ragged_k = WG && (k_ext & (Q_BK - 1));
-        if constexpr (WG) {   // last stage of a ragged contraction: k-rows past the end are clamped to the last one
+        om.init(ldm, m_ext - m0, Q_BK);
+        on.init(ldn, n_ext - n0, Q_BK);
+        ragged_k = KT && (k_ext & (Q_BK - 1));
+        if constexpr (KT) {   // last stage of a ragged contraction: k past the end is clamped to the last k-row / 16-byte piece
             cm.init(ldm, m_ext - m0, ragged_k ? (k_ext & (Q_BK - 1)) : Q_BK);
             cn.init(ldn, n_ext - n0, ragged_k ? (k_ext & (Q_BK - 1)) : Q_BK);
         }
@@ -216,16 +225,16 @@ template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool WG, int TMC> struc
     // loads [J0, J1) of stage s (the m-side tile's loads come first) into ring buffer buf
     template <int J0, int J1> __device__ __forceinline__ void issue(int s, int buf) {
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_w + buf * SG::BYTES);
-        const bool clamp_k = WG && ragged_k && s >= nk - 1;
+        const bool clamp_k = KT && ragged_k && s >= nk - 1;
 #pragma unroll
         for (int j = J0; j < J1; ++j) {
             if (j < LM) {
                 uint32_t o = om.off[j];
-                if constexpr (WG) o = clamp_k ? cm.off[j] : o;
+                if constexpr (KT) o = clamp_k ? cm.off[j] : o;
                 dma16s(bm, o, dst + j * (TL::NW * 1024));
             } else {
                 uint32_t o = on.off[j - LM];
-                if constexpr (WG) o = clamp_k ? cn.off[j - LM] : o;
+                if constexpr (KT) o = clamp_k ? cn.off[j - LM] : o;
                 dma16s(bn, o, dst + SG::M_OPERAND + (j - LM) * (TL::NW * 1024));
             }
         }
@@ -273,24 +282,26 @@ template <int B, int L, int X> __device__ __forceinline__ void wait_stages_behin
 // BIAS: the accumulators start from the bias of their columns instead of zero (bias_raw: the 8 x 4 columns a lane
 // holds, fetched before the operand loads and therefore landed when the first stage has), so that the epilogue adds
 // nothing.
-template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool WG, int TMC, int TMCW, int SUM, int PART = 0, bool BIAS = false>
+template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC, int TMCW, int SUM, int PART = 0, bool BIAS = false>
 __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, int m_ext, const bf16_t *Np, long ldn,
                                           int n0, int n_ext, int k_ext, char *smem, int wave, int wm, int wn,
                                           f32x16 (&acc)[Tile<TMB, WM, WN>::TMW][2], f32x16 &sums, const uint2 (&bias_raw)[8]) {
     typedef Tile<TMB, WM, WN> TL;
     typedef Stage<TMB, WM, WN, M_KS, TMC> SG;
     constexpr int AHEAD = SG::NSTAGE - 1, NP = 4;
-    typedef Feeder<TMB, WM, WN, M_KS, N_KS, WG, TMC> FD;
+    typedef Feeder<TMB, WM, WN, M_KS, N_KS, KT, TMC> FD;
     constexpr int L = FD::L, LH = L / 2;      // loads per wave per stage; the halves are LH and L - LH
     const int nk = __builtin_amdgcn_readfirstlane((k_ext + Q_BK - 1) / Q_BK);
     if (nk == 0) return;
     FD fd;
     fd.init(Mp, ldm, m0, m_ext, Np, ldn, n0, n_ext, k_ext, smem, wave);
     auto fix_tail = [&](int s, int buf) __attribute__((always_inline)) {   // ragged contraction: zero what lies past it in the last stage
-        if (WG && s == nk - 1 && (k_ext & (Q_BK - 1))) {
+        if (KT && s == nk - 1 && (k_ext & (Q_BK - 1))) {
             char *b = smem + buf * SG::BYTES;
-            zero_k_tail<TL::BM, TL::THREADS>(b, k_ext & (Q_BK - 1));
-            zero_k_tail<TL::BN, TL::THREADS>(b + SG::M_OPERAND, k_ext & (Q_BK - 1));
+            if constexpr (M_KS) zero_k_tail<TL::BM, TL::THREADS>(b, k_ext & (Q_BK - 1));
+            else zero_kc_tail<SG::M_OPERAND / 64, TL::THREADS>(b, k_ext & (Q_BK - 1));
+            if constexpr (N_KS) zero_k_tail<TL::BN, TL::THREADS>(b + SG::M_OPERAND, k_ext & (Q_BK - 1));
+            else zero_kc_tail<TL::BN, TL::THREADS>(b + SG::M_OPERAND, k_ext & (Q_BK - 1));
             __syncthreads();
         }
     };
@@ -615,7 +626,7 @@ __device__ __forceinline__ void store_sums(const GemmArgs &g, const f32x16 &sums
 
 // Row-ragged (!WG): C[rows_e, N] = Mop[rows_e, K] . Nop_e ; Mop K-contiguous, Nop_e [N,K] or (N_KS) [K,N].
 // Weight gradient (WG): C_e[M, N] = sum_{r in rows_e} Mop[r, M]^T . Nop[r, N], both K-strided.
-template <int TMB, int WM, int WN, bool N_KS, bool WG, int EPI>
+template <int TMB, int WM, int WN, bool N_KS, bool WG, bool KT, int EPI>
 __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::WAVES_PER_SIMD)) void gemm256_kernel(const GemmArgs g) {
     typedef Tile<TMB, WM, WN> TL;
     constexpr bool M_KS = WG;
@@ -876,7 +887,7 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
     for (int q = 0; q < 16; ++q) sums[q] = 0.f;
 #define MOLE_RUN_TILE_SUM(C, SUM)                                                                                         \
     {                                                                                                                     \
-        main_loop<TMB, WM, WN, M_KS, N_KS, WG, WM *(C), (C), SUM, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw); \
+        main_loop<TMB, WM, WN, M_KS, N_KS, KT, WM *(C), (C), SUM, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw); \
         if constexpr (SUM != 0) store_sums<SUM, (C)>(g, sums, e, m0, n0, m_ext, wm, wn, lane);                            \
         epilogue<TMB, WM, WN, WG, EPI, (C)>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, bias_raw);      \
     }
@@ -894,13 +905,13 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
 #undef MOLE_RUN_TILE_SUM
 }
 
-template <int TMB, int WM, int WN, bool N_KS, bool WG, int EPI>
-static int launch256(GemmArgs g, int tiles, hipStream_t st, int kid) {
+template <int TMB, int WM, int WN, bool N_KS, bool WG, bool KT, int EPI>
+static int launch256_kt(GemmArgs g, int tiles, hipStream_t st, int kid) {
     typedef Tile<TMB, WM, WN> TL;
     if (tiles <= 0) return 0;
     g.n_blocks = tiles;
     const int grid = (tiles + 7) & ~7;
-    auto kern = gemm256_kernel<TMB, WM, WN, N_KS, WG, EPI>;
+    auto kern = gemm256_kernel<TMB, WM, WN, N_KS, WG, KT, EPI>;
     static bool attr_done = false;
     if (!attr_done) {
         MOLE_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS_BYTES));
@@ -909,6 +920,15 @@ static int launch256(GemmArgs g, int tiles, hipStream_t st, int kid) {
     timed_launch(kid, kern, dim3(grid), dim3(TL::THREADS), TL::LDS_BYTES, st, g);
     MOLE_LAUNCH_CHECK();
     return 0;
+}
+
+// (the weight gradients' contraction is always ragged; the others have a kernel of their own for a K that is not whole
+// stages, so that whole-stage ones carry no clamped offsets)
+template <int TMB, int WM, int WN, bool N_KS, bool WG, int EPI>
+static int launch256(const GemmArgs &g, int tiles, hipStream_t st, int kid) {
+    if constexpr (WG) return launch256_kt<TMB, WM, WN, N_KS, WG, true, EPI>(g, tiles, st, kid);
+    else if constexpr (EPI >= EPI_NONE) return launch256_kt<TMB, WM, WN, N_KS, WG, false, EPI>(g, tiles, st, kid);
+    else return g.K % Q_BK ? launch256_kt<TMB, WM, WN, N_KS, WG, true, EPI>(g, tiles, st, kid) : launch256_kt<TMB, WM, WN, N_KS, WG, false, EPI>(g, tiles, st, kid);
 }
 
 // Launch options and their defaults; a -DMOLE_TUNING build reads them from the environment
@@ -1012,9 +1032,9 @@ bool gemm256_sums_operand(const GemmArgs &g) {
 }
 
 int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid) {
-    // alignment the direct-to-LDS path relies on: 16-byte rows, whole stages of K for row-ragged products
+    // alignment the direct-to-LDS path relies on: 16-byte rows and pieces of K
     if (g.lda % 8 || g.ldb % 8 || g.ldc % 8 || g.N % 8) return -100;
-    if (!wg && (a_ks || g.K % Q_BK)) return -100;
+    if (!wg && (a_ks || g.K % 8)) return -100;
     if (wg && (!a_ks || !b_ks || g.M % 8)) return -100;
     const int tile = tile_for(g, wg, b_ks, max_rows, kid);
     if (tile == TILE_128) return dispatch256<4, 2, 2>(g, b_ks, wg, epi, max_rows, st, kid);

@@ -409,3 +409,29 @@ def test_ffn_few_rows_leaves_other_experts_rows_alone(dtype):
     assert rel_err(out.cpu()[lo:hi], w_out[lo:hi]) < tol(dtype) and rel_err(gx.cpu()[lo:hi], w_gx[lo:hi]) < tol(dtype)
     for buf in (out, gx):
         assert float((torch.cat([buf[:lo], buf[hi:]]) - 7.0).abs().max()) == 0.0
+
+
+# bf16 contractions that end inside a 32-wide stage of the direct-to-LDS kernel: one short stage only, every remainder of 8,
+# one and several stages before it; 128-row, 256-row and 320-row tiles (few experts, many rows, many experts).
+@pytest.mark.parametrize("E,M,Fd,rows,gap", [
+    (2, 8, 24, [300, 70], 0), (3, 40, 72, [129, 200, 31], 1), (2, 136, 520, [600, 257], 0), (4, 104, 1112, [90, 128, 0, 65], 0),
+    (30, 264, 2088, [60 + (37 * e) % 90 for e in range(30)], 0), (40, 72, 1048, [300 + (29 * e) % 100 for e in range(40)], 0),
+])
+def test_ffn_contraction_ends_inside_a_stage(E, M, Fd, rows, gap):
+    from mole_amd import hip_ops as H
+    dtype = torch.bfloat16
+    print(f"ffn K tail E={E} M={M} F={Fd} rows={rows[:4]}", flush=True)
+    d = _make(E, M, Fd, rows, dtype, seed=M + Fd, pad_between=gap)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off = torch.from_numpy(d["off"]).cuda(); n = torch.from_numpy(d["n"]).cuda()
+    w_out, w_h, w_gx, *w_g = _oracle_fwd_bwd(d, "tanh")
+    mask = torch.zeros(d["R"], dtype=torch.bool)
+    for e in range(E):
+        mask[int(d["off"][e]):int(d["off"][e]) + int(d["n"][e])] = True
+    out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+    g = [torch.full_like(c[k], 9.0) for k in ("w1", "b1", "w2", "b2")]
+    gx = H.ffn_bwd(c["go"], c["xd"], h, a, off, n, c["w1"], c["w2"], *g)
+    for got, want in ((h, w_h), (out, w_out), (gx, w_gx)):
+        assert rel_err(got.cpu()[mask], want[mask]) < tol(dtype)
+    for got, want in zip(g, w_g):
+        assert rel_err(got, want) < tol(dtype)
