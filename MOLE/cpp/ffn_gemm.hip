@@ -452,7 +452,7 @@ static int run_gemm(const GemmArgs &g, int max_rows, int tiles_generic, hipStrea
     }
     if constexpr (sizeof(T) == 2) {
         if (fast_path_enabled()) {
-            const int rc = launch_gemm256(g, A_KS, B_KS, WG, EPI, max_rows, st, kid);
+            const int rc = launch_gemm256(g, A_KS, B_KS, WG, EPI, max_rows, ws, ws_bytes, st, kid);
             if (rc != -100) return rc;
         }
     } else {
@@ -470,10 +470,10 @@ static int run_gemm(const GemmArgs &g, int max_rows, int tiles_generic, hipStrea
 template <typename T>
 static int ffn_fwd_t(const void *xd, const int32_t *offsets, const int32_t *kept, int E, int max_rows, int M, int F,
                      const void *w1, const void *b1, const void *w2, const void *b2, void *h, void *a, void *out,
-                     void *ws, size_t ws_bytes, hipStream_t st) {
+                     void *ws, size_t ws_bytes, int est_rows, hipStream_t st) {
     const int m_tiles = max_rows / TBM + E;  // every expert may end in a partial tile
     GemmArgs g{};
-    g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles;
+    g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles; g.est_rows = est_rows;
     // h = xd . w1^T + b1, a = gelu(h)
     g.A = xd; g.lda = M; g.B = w1; g.ldb = M; g.strideB = (long)F * M; g.N = F; g.K = M;
     g.C = h; g.C2 = a; g.ldc = F; g.bias = b1;
@@ -488,10 +488,10 @@ template <typename T>
 static int ffn_bwd_t(const void *go, const void *xd, const void *h, const void *a, const int32_t *offsets,
                      const int32_t *kept, int E, int max_rows, int M, int F, const void *w1, const void *w2, void *t,
                      void *g_w1, void *g_b1, void *g_w2, void *g_b2, void *gx, int accumulate, int gelu_bwd,
-                     void *ws, size_t ws_bytes, hipStream_t st) {
+                     void *ws, size_t ws_bytes, int est_rows, hipStream_t st) {
     const int m_tiles = max_rows / TBM + E;
     GemmArgs g{};
-    g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles;
+    g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles; g.est_rows = est_rows;
     g.accumulate = accumulate; g.gelu_bwd = gelu_bwd;
     const int wg_tiles = E * ceil_div(F, TBM) * ceil_div(M, TBN);
     // The bias gradients are sums of go and of t over every expert's rows: go and t are operands of the two
@@ -528,7 +528,7 @@ static int ffn_bwd_t(const void *go, const void *xd, const void *h, const void *
     g.colsum = nullptr; g.colsum_side = 0;
     // gx = t . w1                  (w1 [F,M]: K = F strided)
     if (gx != nullptr) {
-        g.A = t; g.lda = F; g.B = w1; g.ldb = M; g.strideB = (long)F * M; g.N = M; g.K = F; g.C = gx; g.ldc = M;
+        g.A = t; g.lda = F; g.B = w1; g.ldb = M; g.strideB = (long)F * M; g.N = M; g.K = F; g.C = gx; g.ldc = M; g.bias = nullptr;
         if (int rc = run_gemm<T, false, true, false, EPI_STORE>(g, max_rows, m_tiles * ceil_div(M, TBN), st, MOLE_K_FFN_GX, ws, ws_bytes)) return rc;
     }
     return 0;
@@ -547,24 +547,55 @@ static bool al16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 using namespace mole;
 
-extern "C" size_t mole_ffn_workspace_bytes(int dtype, int E, int max_rows, int M, int F) {
+namespace mole {
+
+size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, int F) {
     if (E <= 0 || max_rows <= 0 || M <= 0 || F <= 0) return 0;
-    return gemm_skinny_workspace_bytes(E, max_rows, M, F, dtype);
+    int ks = gemm_skinny_ksplit(E, est_rows, M, F, dtype);
+    if (ks == 0 && dtype == MOLE_BF16) ks = gemm256_ksplit(E, est_rows, M, F);
+    return ks > 1 ? (size_t)ks * max_rows * M * sizeof(float) : 0;
 }
 
-extern "C" int mole_ffn_fwd_ws(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
-                               int max_rows, int M, int F, const void *w1, const void *b1, const void *w2, const void *b2,
-                               void *h, void *a, void *out, void *workspace, size_t workspace_bytes, mole_stream_t stream) {
+int ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, int est_rows, int M, int F,
+            const void *w1, const void *b1, const void *w2, const void *b2, void *h, void *a, void *out, void *workspace,
+            size_t workspace_bytes, hipStream_t st) {
     if (int rc = check_ffn("mole_ffn_fwd", dtype, E, max_rows, M, F)) return rc;
     if (max_rows == 0) return 0;
     MOLE_REQUIRE(xd && offsets && kept_rows && w1 && b1 && w2 && b2 && h && a && out, "mole_ffn_fwd: null pointer");
     MOLE_REQUIRE(al16(xd) && al16(w1) && al16(w2) && al16(h) && al16(a) && al16(out) && al16(workspace),
                  "mole_ffn_fwd: buffers must be 16-byte aligned");
     if (dtype == MOLE_BF16)
-        return ffn_fwd_t<bf16_t>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes,
-                                 (hipStream_t)stream);
-    return ffn_fwd_t<float>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes,
-                            (hipStream_t)stream);
+        return ffn_fwd_t<bf16_t>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes, est_rows, st);
+    return ffn_fwd_t<float>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes, est_rows, st);
+}
+
+int ffn_bwd(const void *go, const void *xd, const void *h, const void *a, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
+            int max_rows, int est_rows, int M, int F, const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2, void *g_b2,
+            void *gx, int accumulate, int gelu_bwd, void *workspace, size_t workspace_bytes, hipStream_t st) {
+    if (int rc = check_ffn("mole_ffn_bwd", dtype, E, max_rows, M, F)) return rc;
+    MOLE_REQUIRE(gelu_bwd == MOLE_GELU_BWD_TANH || gelu_bwd == MOLE_GELU_BWD_EXACT, "mole_ffn_bwd: bad gelu_bwd %d", gelu_bwd);
+    MOLE_REQUIRE(offsets && kept_rows && w1 && w2 && g_w1 && g_b1 && g_w2 && g_b2, "mole_ffn_bwd: null pointer");
+    MOLE_REQUIRE(max_rows == 0 || (go && xd && h && a && t), "mole_ffn_bwd: null activation pointer");
+    MOLE_REQUIRE(al16(go) && al16(xd) && al16(h) && al16(a) && al16(t) && al16(w1) && al16(w2) && al16(gx) && al16(workspace),
+                 "mole_ffn_bwd: buffers must be 16-byte aligned");
+    if (dtype == MOLE_BF16)
+        return ffn_bwd_t<bf16_t>(go, xd, h, a, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx, accumulate,
+                                 gelu_bwd, workspace, workspace_bytes, est_rows, st);
+    return ffn_bwd_t<float>(go, xd, h, a, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx, accumulate, gelu_bwd,
+                            workspace, workspace_bytes, est_rows, st);
+}
+
+}  // namespace mole
+
+extern "C" size_t mole_ffn_workspace_bytes(int dtype, int E, int max_rows, int M, int F) {
+    return ffn_workspace_bytes(dtype, E, max_rows, max_rows, M, F);
+}
+
+extern "C" int mole_ffn_fwd_ws(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
+                               int max_rows, int M, int F, const void *w1, const void *b1, const void *w2, const void *b2,
+                               void *h, void *a, void *out, void *workspace, size_t workspace_bytes, mole_stream_t stream) {
+    return ffn_fwd(xd, dtype, offsets, kept_rows, E, max_rows, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes,
+                   (hipStream_t)stream);
 }
 
 extern "C" int mole_ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
@@ -578,17 +609,8 @@ extern "C" int mole_ffn_bwd_ws(const void *go, const void *xd, const void *h, co
                                const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2, void *g_b2,
                                void *gx, int accumulate, int gelu_bwd, void *workspace, size_t workspace_bytes,
                                mole_stream_t stream) {
-    if (int rc = check_ffn("mole_ffn_bwd", dtype, E, max_rows, M, F)) return rc;
-    MOLE_REQUIRE(gelu_bwd == MOLE_GELU_BWD_TANH || gelu_bwd == MOLE_GELU_BWD_EXACT, "mole_ffn_bwd: bad gelu_bwd %d", gelu_bwd);
-    MOLE_REQUIRE(offsets && kept_rows && w1 && w2 && g_w1 && g_b1 && g_w2 && g_b2, "mole_ffn_bwd: null pointer");
-    MOLE_REQUIRE(max_rows == 0 || (go && xd && h && a && t), "mole_ffn_bwd: null activation pointer");
-    MOLE_REQUIRE(al16(go) && al16(xd) && al16(h) && al16(a) && al16(t) && al16(w1) && al16(w2) && al16(gx) && al16(workspace),
-                 "mole_ffn_bwd: buffers must be 16-byte aligned");
-    if (dtype == MOLE_BF16)
-        return ffn_bwd_t<bf16_t>(go, xd, h, a, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2,
-                                 gx, accumulate, gelu_bwd, workspace, workspace_bytes, (hipStream_t)stream);
-    return ffn_bwd_t<float>(go, xd, h, a, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx,
-                            accumulate, gelu_bwd, workspace, workspace_bytes, (hipStream_t)stream);
+    return ffn_bwd(go, xd, h, a, dtype, offsets, kept_rows, E, max_rows, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx, accumulate,
+                   gelu_bwd, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 extern "C" int mole_ffn_bwd(const void *go, const void *xd, const void *h, const void *a, int dtype,
@@ -606,7 +628,7 @@ extern "C" int mole_gemm_nt(const void *a, const void *b, int dtype, int rows, i
     if (rows == 0) return 0;
     MOLE_REQUIRE(a && b && c && al16(a) && al16(b), "mole_gemm_nt: null or misaligned pointer");
     GemmArgs g{};
-    g.single_rows = rows; g.E = 1;
+    g.single_rows = rows; g.E = 1; g.est_rows = rows;
     g.A = a; g.lda = K; g.B = b; g.ldb = K; g.N = N; g.K = K; g.C = c; g.ldc = N;
     const int tiles = ceil_div(rows, TBM) * ceil_div(N, TBN);
     if (dtype == MOLE_BF16) return run_gemm<bf16_t, false, false, false, EPI_F32>(g, rows, tiles, (hipStream_t)stream, MOLE_K_GEMM_NT);
@@ -621,7 +643,7 @@ extern "C" int mole_gemm_nn(const void *a, const void *b, int dtype, int rows, i
     if (rows == 0) return 0;
     MOLE_REQUIRE(a && b && c && al16(a) && al16(b) && al16(c), "mole_gemm_nn: null or misaligned pointer");
     GemmArgs g{};
-    g.single_rows = rows; g.E = 1;
+    g.single_rows = rows; g.E = 1; g.est_rows = rows;
     g.A = a; g.lda = K; g.B = b; g.ldb = N; g.N = N; g.K = K; g.C = c; g.ldc = N;
     const int tiles = ceil_div(rows, TBM) * ceil_div(N, TBN);
     if (dtype == MOLE_BF16) return run_gemm<bf16_t, false, true, false, EPI_STORE>(g, rows, tiles, (hipStream_t)stream, MOLE_K_GEMM_NT);
@@ -635,7 +657,7 @@ extern "C" int mole_gemm_tn(const void *a, const void *b, int dtype, int rows, i
     MOLE_REQUIRE(rows >= 0 && N > 0 && Mo > 0 && Mo % epc == 0 && N % epc == 0, "mole_gemm_tn: bad sizes rows=%d Mo=%d N=%d", rows, Mo, N);
     MOLE_REQUIRE(c && al16(c) && (rows == 0 || (a && b && al16(a) && al16(b))), "mole_gemm_tn: null or misaligned pointer");
     GemmArgs g{};
-    g.single_rows = rows; g.E = 1;      // one group whose contraction runs over all rows (zero rows: c = 0)
+    g.single_rows = rows; g.E = 1; g.est_rows = rows;      // one group whose contraction runs over all rows (zero rows: c = 0)
     g.A = a; g.lda = Mo; g.B = b; g.ldb = N; g.M = Mo; g.N = N; g.C = c; g.ldc = N; g.strideC = (long)Mo * N;
     const int tiles = ceil_div(Mo, TBM) * ceil_div(N, TBN);
     if (dtype == MOLE_BF16) return launch_gemm<bf16_t, true, true, true, TBM, TBN, EPI_WGRAD>(g, tiles, (hipStream_t)stream, MOLE_K_GEMM_NT);

@@ -119,7 +119,8 @@ struct DGeluCoef {
 };
 
 enum { EPI_STORE = 0, EPI_BIAS = 1, EPI_BIAS_GELU = 2, EPI_DGELU = 3, EPI_WGRAD = 4, EPI_F32 = 5,
-       EPI_NONE = 6 /* measurement only: the K loop runs, nothing is stored; EPI_NONE + 1..4: the K loop without
+       EPI_PART = 6 /* one plane of a contraction split over blocks: fp32 into GemmArgs.part */,
+       EPI_NONE = 7 /* measurement only: the K loop runs, nothing is stored; EPI_NONE + 1..4: the K loop without
                        its operand loads / its fragment reads / its barriers / all three */ };
 
 struct GemmArgs {
@@ -144,20 +145,25 @@ struct GemmArgs {
     int colsum_side;        //   over the expert's rows: 1 = the m-side operand (A), 2 = the n-side operand (B)
     int wg_expert_major;    // weight gradients, 256-wide kernel: all (m-tile, n-tile) blocks of an expert on one XCD
     int m_fastest_from;     //   ... for experts with at least this many m-tiles (of the class); the others n-tile first
-    float *part;            // few-row kernel: fp32 partial results [ksplit][part_rows][N] when the contraction is split over blocks
+    float *part;            // fp32 partial results [ksplit][part_rows][N] of a contraction split over blocks
     long part_rows;
     int ksplit;
+    int est_rows;           // host's estimate of the rows of all experts together (no more than the launch's bound)
     int m_fastest;          // row-ragged products, 256-wide kernel: number an expert's tiles m-tile first (see gemm256.hip)
 };
 
 
 // 256x256 bf16 tiles with direct-to-LDS loads (gemm256.hip).  Returns -100 when the shape does not
 // meet its alignment requirements; the caller then uses the generic kernel.
-int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid);
+int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
+// planes a K = F product of est_rows rows over E experts would be split into, given the workspace (1: none)
+int gemm256_ksplit(int E, int est_rows, int N, int K);
+// out = sum of the planes (+ bias), for the rows of g's experts (gemm_skinny.hip)
+int launch_plane_reduce(const GemmArgs &g, int dtype, int max_rows, hipStream_t st);
 bool gemm256_sums_operand(const GemmArgs &g);
 // Few rows per expert (gemm_skinny.hip): weights streamed straight into fragments; -100 when the shape is not its.
 int launch_gemm_skinny(const GemmArgs &g, int dtype, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
-size_t gemm_skinny_workspace_bytes(int E, int max_rows, int N, int K, int dtype);
+int gemm_skinny_ksplit(int E, int est_rows, int N, int K, int dtype);    // 0: not its shape
 // fp32 tiles with direct-to-LDS loads (gemm_f32.hip); -100 as above.
 int launch_gemm_f32(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid);
 bool gemm_f32_sums_operand(const GemmArgs &g);

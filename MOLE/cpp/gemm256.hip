@@ -406,7 +406,7 @@ template <int EPI> __device__ __forceinline__ void load_bias(const GemmArgs &g, 
 template <int TMB, int WM, int WN, bool WG, int EPI, int TMC>
 __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<TMB, WM, WN>::TMW][2], char *smem, int lane, int wave,
                                          int wn, int e, long row0, int m0, int n0, int m_ext, int live,
-                                         const uint2 (&bias_raw)[8]) {
+                                         const uint2 (&bias_raw)[8], int split_k) {
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     __syncthreads();
     if constexpr (TMC == 0) return;
@@ -543,6 +543,28 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<T
             }
         return;
     }
+    if constexpr (EPI == EPI_PART) {
+        // fp32, 32 columns (128 bytes) of a row at a time through the slab: results straight from the accumulators would be
+        // 32-byte pieces of 32 rows per store.  Ordinary stores: the reduction reads them next.
+#pragma unroll
+        for (int tn = 0; tn < 2; ++tn) {
+            float *dst = g.part + ((long)split_k * g.part_rows + crow0 + m0) * g.N + nw0 + tn * 32;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int tm = 0; tm < TMC; ++tm) {
+                    const int row = tm * 32 + lm;
+                    *reinterpret_cast<float4 *>(slab + row * 128 + (((2 * q + h) ^ ((row >> 1) & 7)) << 4)) =
+                        make_float4(acc[tm][tn][4 * q], acc[tm][tn][4 * q + 1], acc[tm][tn][4 * q + 2], acc[tm][tn][4 * q + 3]);
+                }
+            // (the slab is this wave's own: program order is enough)
+#pragma unroll
+            for (int it = 0; it < TMC * 4; ++it)
+                if (it * 8 + jr < live && nw0 + tn * 32 + jc * 4 < g.N)
+                    *reinterpret_cast<uint4 *>(dst + (long)(it * 8 + jr) * g.N + jc * 4) = *reinterpret_cast<const uint4 *>(wide_cell(it));
+        }
+        return;
+    }
     if constexpr (EPI == EPI_DGELU) fill((const bf16_t *)g.H);
     if constexpr (EPI == EPI_WGRAD) { if (g.accumulate) fill(Cb); }
 
@@ -639,6 +661,9 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n_tiles = (g.N + Q_BN - 1) / Q_BN;
     int sum_nt = 0, sum_mt = 0;   // weight gradients: the n-tile / m-tile whose block also sums the m-side / n-side operand
+    // a contraction split over blocks: the planes of an m-tile's n-tiles are numbered like more n-tiles
+    const int n_units = EPI == EPI_PART ? n_tiles * g.ksplit : n_tiles;
+    int split_k = 0;
     int e, mt, nt, m_ext, k_ext, tile_h = Q_BM;   // tile_h: rows of this tile's m-tiles (row-ragged products cut experts evenly)
     long row0;  // first row of the expert
     if constexpr (!WG) {
@@ -697,8 +722,8 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
             n_l += tiles_of(r) - hv;
         }
         for (int d = WAVE / 2; d >= 1; d >>= 1) { n_h += __shfl_xor(n_h, d, WAVE); n_l += __shfl_xor(n_l, d, WAVE); }
-        if ((n_h + n_l) * n_tiles > 16 * 256) { split = false; n_h += n_l; n_l = 0; }
-        const int total_h = n_h * n_tiles, total_l = n_l * n_tiles;
+        if ((n_h + n_l) * n_units > 16 * 256) { split = false; n_h += n_l; n_l = 0; }
+        const int total_h = n_h * n_units, total_l = n_l * n_units;
         const int per_h = (total_h + 7) >> 3, per_l = (total_l + 7) >> 3;
         const int slot = blockIdx.x >> 3, xcd = blockIdx.x & 7;
         const bool heavy = slot < per_h;
@@ -717,8 +742,8 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
         // rows, 1024 -> 4096: +6 and +3 us), so those keep n-tile first.
         const bool mf = g.m_fastest != 0;
         const int unit = mf ? n_tiles : 1;       // tiles per counted m-tile
-        const int target = mf ? t : t / n_tiles;
-        nt = t % n_tiles;
+        const int target = mf ? t : t / n_units;
+        nt = t % n_units;
         // the expert whose running count (of the class) passes `target`
         int run = 0, found = -1, before = 0, cnt_found = 1;
         for (int base = 0; base < nE && found < 0; base += WAVE) {
@@ -778,6 +803,10 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
             row0 = single ? 0 : ((found >> 6) < RC ? ov : g.offsets[e]);
         }
         k_ext = g.K;
+        if constexpr (EPI == EPI_PART) {
+            split_k = nt / n_tiles;
+            nt %= n_tiles;
+        }
     } else {
         // The contraction length differs from expert to expert, so experts are not handed to XCDs in
         // contiguous ranges: the (expert, m-tile) units are dealt round-robin over the 8 XCDs, which gives
@@ -856,6 +885,14 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
     }
     const bf16_t *Mp = (const bf16_t *)g.A + row0 * g.lda;
     const bf16_t *Np = WG ? (const bf16_t *)g.B + row0 * g.ldb : (const bf16_t *)g.B + (long)e * g.strideB;
+    if constexpr (EPI == EPI_PART) {           // this block's whole stages of the contraction (the last plane has the ragged end)
+        split_k = __builtin_amdgcn_readfirstlane(split_k);
+        const int stages = (k_ext + Q_BK - 1) / Q_BK;
+        const int k_lo = split_k * stages / g.ksplit * Q_BK, k_hi = min((split_k + 1) * stages / g.ksplit * Q_BK, k_ext);
+        Mp += k_lo;
+        Np += N_KS ? (long)k_lo * g.ldb : (long)k_lo;
+        k_ext = k_hi - k_lo;
+    }
 
     f32x16 acc[TMW][2];
 #pragma unroll
@@ -889,7 +926,7 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
     {                                                                                                                     \
         main_loop<TMB, WM, WN, M_KS, N_KS, KT, WM *(C), (C), SUM, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw); \
         if constexpr (SUM != 0) store_sums<SUM, (C)>(g, sums, e, m0, n0, m_ext, wm, wn, lane);                            \
-        epilogue<TMB, WM, WN, WG, EPI, (C)>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, bias_raw);      \
+        epilogue<TMB, WM, WN, WG, EPI, (C)>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, bias_raw, split_k);      \
     }
 #define MOLE_RUN_TILE(C) MOLE_RUN_TILE_SUM(C, 0)
     if constexpr (WG && WM == 2 && TMW <= WN) {
@@ -934,7 +971,6 @@ static int launch256(const GemmArgs &g, int tiles, hipStream_t st, int kid) {
 // Launch options and their defaults; a -DMOLE_TUNING build reads them from the environment
 // (MOLE_MFAST: bit mask of the products that number an expert's tiles m-tile first within groups of MOLE_MFAST_G
 // n-tiles, MOLE_MFAST_FROM: m-tiles an expert needs for that order, MOLE_WG_EMAJOR: expert count from which a weight gradient keeps an expert's blocks on one XCD,
-// MOLE_TMB: 128 = the 128 x 128 tile, 16 = the 256-row one, for every row-ragged product,
 // MOLE_NO_SUMS: bias gradients from their own kernel).
 #ifdef MOLE_TUNING
 static int env_int(const char *name, int dflt) { const char *v = getenv(name); return v ? atoi(v) : dflt; }
@@ -942,14 +978,12 @@ static int m_fastest_mask() { static const int v = env_int("MOLE_MFAST", 9); ret
 static int m_fastest_group() { static const int v = env_int("MOLE_MFAST_G", 8); return v > 0 ? v : 1; }
 static int m_fastest_from() { static const int v = env_int("MOLE_MFAST_FROM", 8); return v; }
 static int wg_emajor_from() { static const int v = env_int("MOLE_WG_EMAJOR", 128); return v; }
-static int forced_tile() { static const int v = env_int("MOLE_TMB", 0); return v; }
 static bool sums_off() { static const bool v = getenv("MOLE_NO_SUMS") != nullptr; return v; }
 #else
 static int m_fastest_mask() { return 9; }        // h = xd.w1^T + b1 and t = (go.w2^T) gelu'(h)
 static int m_fastest_group() { return 8; }
 static int m_fastest_from() { return 8; }
 static int wg_emajor_from() { return 128; }
-static int forced_tile() { return 0; }
 static bool sums_off() { return false; }
 #endif
 
@@ -974,7 +1008,8 @@ static int dispatch256(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_r
     gg.m_fastest = ((m_fastest_mask() >> kid) & 1) ? m_fastest_group() : 0;
     gg.m_fastest_from = m_fastest_from();
     // (+ 16: the heavy and the light tiles of an XCD are rounded up to whole slots separately)
-    const int tiles = (((rows_bound / BM + (g.offsets ? g.E : 1)) * n_tiles + 7) & ~7) + 16;
+    const int m_bound = rows_bound / BM + (g.offsets ? min(g.E, rows_bound) : 1);
+    const int tiles = ((m_bound * n_tiles * (epi == EPI_PART ? g.ksplit : 1) + 7) & ~7) + 16;
     if (wg) return -100;
     if (!b_ks) {
         if constexpr (TMB != 10) {
@@ -994,36 +1029,64 @@ static int dispatch256(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_r
     } else {
         if (epi == EPI_BIAS) return launch256<TMB, WM, WN, true, false, EPI_BIAS>(gg, tiles, st, kid);
         if (epi == EPI_STORE) return launch256<TMB, WM, WN, true, false, EPI_STORE>(gg, tiles, st, kid);
+        if (epi == EPI_PART) return launch256<TMB, WM, WN, true, false, EPI_PART>(gg, tiles, st, kid);
     }
     return -100;
 }
 
 // Tile configuration.  Eight waves (two per SIMD hide each other's waits; one fetch of the n-side tile
-// serves all rows of the tile) for every product.  256-row tiles by default; tiles of up to 320 rows, an
-// expert's rows split evenly over them, for the two K = F products (out = a.w2 + b2 and gx = t.w1): one tile
-// is a whole round there, and with a capacity factor of 1.25 no expert then needs more m-tiles than the
-// average one, so the launch stays one round.  The K = M products run four rounds anyway; their short
+// serves all rows of the tile) for every product of some size.  256-row tiles by default; tiles of up to 320 rows, an
+// expert's rows split evenly over them, for the two K = F products (out = a.w2 + b2 and gx = t.w1) where they need fewer
+// rounds of tiles: with about 1024 rows an expert and a capacity factor of 1.25 they are one round where 256-row tiles
+// are two (16 experts, 1024 -> 4096: 126 against 163 us).  Where the rounds are the same the smaller tile is the faster
+// (6 experts of 1333 rows, 1088 -> 4352: 86 against 108 us).  The K = M products run several rounds anyway; their short
 // remainder tiles, numbered last, fill the final round, which measured better than the even split
 // (t = (go.w2^T) gelu'(h): 213 against 219 us) - and h = xd.w1^T + b1 with the GELU epilogue would spill at
 // the 160 accumulators of the larger tile.
-// 128 x 128 tiles of four waves, two blocks to a CU, where the large tiles would leave half of the CUs without one: a
-// row-ragged product is then a few long serial walks over K.  16 experts of 256 rows, 512 -> 1024: h 20.9 -> 14.7 us, out
-// 30.0 -> 16.9; 8 experts of 256 rows, 1024 -> 4096: out 99 -> 54 us.  With a tile for half of the CUs or more the two are
-// even (32 experts of 125 rows, 1024 -> 2048: out 51.7 against 51.2 us, h 44 against 47) and beyond the large tile's
-// fewer operand bytes per flop win (16 experts of 375 rows, 1024 -> 4096: h 83 against 109 us).
+//
+// Launches whose large tiles do not fill the chip once:
+//   * K = F products with a long contraction split it over blocks (planes of fp32 partial results in the caller's workspace,
+//     added by plane_reduce_kernel) as often as the tiles fit the chip, four times at most: every further plane costs its
+//     write and its read.  out, reduction included: 16 experts of 375 rows, 1024 -> 4096: 81 -> 68 us in two planes; of 125
+//     rows: 79 -> 46 in four; 8 experts of 250 rows, 2048 -> 8192: 184 -> 103 in four.
+//   * the others run 128 x 128 tiles of four waves, two blocks to a CU, up to 112 large tiles (16 experts of 256 rows,
+//     512 -> 1024: h 20.9 -> 14.7 us, out 26 -> 14); with more, their operand bytes per flop cost more than the idle CUs
+//     (16 experts of 375 rows, 1024 -> 4096: h 109 against 83 us).  Their K = F products are split as well while the tiles
+//     leave CUs idle (8 experts of 194 rows, 512 -> 2048: out 25 -> 16 us).
 enum { TILE_256, TILE_320, TILE_128 };
-static int tile_for(const GemmArgs &g, bool wg, bool b_ks, int max_rows, int kid) {
-    const int forced = forced_tile();
-    if (forced == 128) return TILE_128;
-    const bool tall = kid == MOLE_K_FFN_FWD2 || kid == MOLE_K_FFN_GX;
-    if (!wg && g.offsets != nullptr && forced == 0) {
-        const int active = g.E < max_rows ? g.E : max_rows;
-        const int avg = active > 0 ? ceil_div(max_rows, active) : 0;          // rows of an expert if they spread evenly
-        const long tiles = (long)active * ceil_div(avg, tall ? 320 : 256) * ceil_div(g.N, 256);
-        if (tiles < 112) return TILE_128;
+struct TilePlan { int tile, ksplit; };
+static TilePlan tile_plan(int E, int est_rows, int N, int K, bool tall) {
+    TilePlan p{TILE_256, 1};
+    const int active = E < est_rows ? E : est_rows;
+    if (active <= 0) return p;
+    // rows of an expert if they spread evenly, and of a fuller one (two standard deviations of a random routing)
+    const int avg = ceil_div(est_rows, active);
+    int full = avg;
+    while ((full - avg) * (full - avg) < 4 * avg) ++full;
+    const int n_tiles = ceil_div(N, 256), c256 = ceil_div(full, 256), c320 = ceil_div(full, 320);
+    const long t256 = (long)active * c256 * n_tiles, t320 = (long)active * c320 * n_tiles;
+    const bool few = (long)active * ceil_div(avg, 256) * n_tiles < 112;
+    if (!tall) {
+        if (few) p.tile = TILE_128;
+        return p;
     }
-    return tall && b_ks && !wg ? TILE_320 : TILE_256;
+    p.tile = (t256 + 255) / 256 > (t320 + 255) / 256 ? TILE_320 : TILE_256;
+    if (K >= 3072 || (K >= 2048 && full <= 192)) {
+        const long fit = 256 / t320;
+        if (fit >= 2) {
+            p.ksplit = fit < 4 ? (int)fit : 4;
+            p.tile = c256 > c320 ? TILE_320 : TILE_256;
+        }
+    } else if (few) {
+        p.tile = TILE_128;
+        const long t128 = (long)active * ceil_div(full, 128) * ceil_div(N, 128);
+        const long fit = 256 / t128, most = K / 512;
+        p.ksplit = (int)(fit < most ? fit : most);
+        p.ksplit = p.ksplit < 1 ? 1 : (p.ksplit > 4 ? 4 : p.ksplit);
+    }
+    return p;
 }
+int gemm256_ksplit(int E, int est_rows, int N, int K) { return tile_plan(E, est_rows, N, K, true).ksplit; }
 
 // Whether the weight-gradient launch for g will also produce the operand sums asked for in g.colsum.
 bool gemm256_sums_operand(const GemmArgs &g) {
@@ -1031,15 +1094,26 @@ bool gemm256_sums_operand(const GemmArgs &g) {
     return !sums_off();
 }
 
-int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid) {
+int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid) {
     // alignment the direct-to-LDS path relies on: 16-byte rows and pieces of K
     if (g.lda % 8 || g.ldb % 8 || g.ldc % 8 || g.N % 8) return -100;
     if (!wg && (a_ks || g.K % 8)) return -100;
     if (wg && (!a_ks || !b_ks || g.M % 8)) return -100;
-    const int tile = tile_for(g, wg, b_ks, max_rows, kid);
-    if (tile == TILE_128) return dispatch256<4, 2, 2>(g, b_ks, wg, epi, max_rows, st, kid);
-    if (tile == TILE_320) return dispatch256<10, 2, 4>(g, b_ks, wg, epi, max_rows, st, kid);
-    return dispatch256<8, 2, 4>(g, b_ks, wg, epi, max_rows, st, kid);
+    TilePlan p{TILE_256, 1};
+    if (!wg && g.offsets != nullptr && epi < EPI_NONE) p = tile_plan(g.E, g.est_rows, g.N, g.K, b_ks);
+    GemmArgs gp = g;
+    gp.ksplit = 1;
+    if (p.ksplit > 1 && b_ks && ws != nullptr && ws_bytes >= (size_t)p.ksplit * max_rows * g.N * sizeof(float)) {
+        gp.ksplit = p.ksplit;
+        gp.part = (float *)ws;
+        gp.part_rows = max_rows;
+        epi = EPI_PART;
+    }
+    int rc;
+    if (p.tile == TILE_128) rc = dispatch256<4, 2, 2>(gp, b_ks, wg, epi, max_rows, st, kid);
+    else if (p.tile == TILE_320) rc = dispatch256<10, 2, 4>(gp, b_ks, wg, epi, max_rows, st, kid);
+    else rc = dispatch256<8, 2, 4>(gp, b_ks, wg, epi, max_rows, st, kid);
+    return rc != 0 || gp.ksplit == 1 ? rc : launch_plane_reduce(gp, MOLE_BF16, max_rows, st);
 }
 
 }  // namespace mole

@@ -6,7 +6,7 @@
 // and the big-tile kernels have too few blocks to pull it: a contraction over 8192 with 2048 result columns is 8 tiles
 // of 256 columns per active expert, each a serial walk over 8192 of K by one CU (about 60 GB/s a CU).  Here the waves of
 // a block split the contraction, and blocks split it further (ksplit) where the result is too narrow to give every CU a
-// block; partial results meet in LDS, or as fp32 planes in a workspace that skinny_reduce_kernel adds up in plane order
+// block; partial results meet in LDS, or as fp32 planes in a workspace that plane_reduce_kernel adds up in plane order
 // (deterministic, no atomics).
 //
 // Tokens take the MFMA's B side (16 rows), weights its A side (16 result columns), so a lane ends up with 4 consecutive
@@ -308,12 +308,6 @@ __device__ __forceinline__ void skinny_ks_run(const GemmArgs &g, sk_f32x4 (&red)
                 if (g.ksplit == 1) {
                     sk_epilogue4<T, EPI>(g, e, row0 + m, n, v);
                 } else {
-                    if (EPI == EPI_BIAS && split == 0) {
-                        float bv[4];
-                        sk_load4<T>((const T *)g.bias + (long)e * g.N + n, bv);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) v[j] += bv[j];
-                    }
                     *reinterpret_cast<float4 *>(g.part + ((long)split * g.part_rows + row0 + m) * g.N + n) = make_float4(v[0], v[1], v[2], v[3]);
                 }
             }
@@ -336,48 +330,50 @@ __global__ __launch_bounds__(SK_THREADS, 4) void skinny_ks_kernel(const GemmArgs
     else skinny_ks_run<T, MB, EPI>(g, red, e, rows, row0, m0, n0, split);
 }
 
-// out[row][n] = sum over the planes of part[plane][row][n] (the bias is in plane 0), for the rows of the launch's experts
+// out[row][n] = bias[n] + sum over the planes of part[plane][row][n], for the rows of the launch's experts
 // only: the rows between them belong to experts of other launches (offloaded experts run in chunks).
-constexpr int SK_RED_ROWS = 4;
+constexpr int RED_ROWS = 4;
 template <typename T>
-__global__ __launch_bounds__(256) void skinny_reduce_kernel(const GemmArgs g) {
+__global__ __launch_bounds__(256) void plane_reduce_kernel(const GemmArgs g) {
     int e, grp, rows;
     long row0;
-    if (!sk_find_group<SK_RED_ROWS>(g, blockIdx.y, e, grp, rows, row0)) return;
+    if (!sk_find_group<RED_ROWS>(g, blockIdx.y, e, grp, rows, row0)) return;
     const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (n >= g.N) return;
     const long plane = g.part_rows * g.N;
-    const int m0 = grp * SK_RED_ROWS;
-    float4 s[SK_RED_ROWS];
-    const float *p[SK_RED_ROWS];
+    const int m0 = grp * RED_ROWS;
+    float4 s[RED_ROWS];
+    const float *p[RED_ROWS];
 #pragma unroll
-    for (int i = 0; i < SK_RED_ROWS; ++i) {            // (rows past the expert's end repeat its last one and are not stored)
+    for (int i = 0; i < RED_ROWS; ++i) {            // (rows past the expert's end repeat its last one and are not stored)
         p[i] = g.part + (row0 + min(m0 + i, rows - 1)) * g.N + n;
         s[i] = *reinterpret_cast<const float4 *>(p[i]);
     }
     for (int k = 1; k < g.ksplit; ++k) {
-        float4 t[SK_RED_ROWS];
+        float4 t[RED_ROWS];
 #pragma unroll
-        for (int i = 0; i < SK_RED_ROWS; ++i) t[i] = *reinterpret_cast<const float4 *>(p[i] + (long)k * plane);
+        for (int i = 0; i < RED_ROWS; ++i) t[i] = *reinterpret_cast<const float4 *>(p[i] + (long)k * plane);
 #pragma unroll
-        for (int i = 0; i < SK_RED_ROWS; ++i) { s[i].x += t[i].x; s[i].y += t[i].y; s[i].z += t[i].z; s[i].w += t[i].w; }
+        for (int i = 0; i < RED_ROWS; ++i) { s[i].x += t[i].x; s[i].y += t[i].y; s[i].z += t[i].z; s[i].w += t[i].w; }
     }
+    float b[4] = {0.f, 0.f, 0.f, 0.f};
+    if (g.bias != nullptr) sk_load4<T>((const T *)g.bias + (long)e * g.N + n, b);
 #pragma unroll
-    for (int i = 0; i < SK_RED_ROWS; ++i) {
-        float v[4] = {s[i].x, s[i].y, s[i].z, s[i].w};
+    for (int i = 0; i < RED_ROWS; ++i) {
+        float v[4] = {s[i].x + b[0], s[i].y + b[1], s[i].z + b[2], s[i].w + b[3]};
         if (m0 + i < rows) sk_store4<T>((T *)g.C + (row0 + m0 + i) * g.ldc + n, v);
     }
 }
 
 // ---- which products come here, and how they are cut ------------------------------------------------------------
 // avg: rows of an expert if the rows spread evenly; tiles: blocks the big-tile kernel of the type would have.
-struct SkinnyPlan { int mb, ksplit, groups; };
-static bool skinny_plan(int dtype, bool b_ks, int E, int max_rows, int N, int K, SkinnyPlan &p) {
-    if (max_rows <= 0) return false;
+struct SkinnyPlan { int mb, ksplit; };
+static bool skinny_plan(int dtype, bool b_ks, int E, int est_rows, int N, int K, SkinnyPlan &p) {
+    if (est_rows <= 0) return false;
     const bool bf16 = dtype == MOLE_BF16;
     const int epc = bf16 ? 8 : 4;
-    const int active = E < max_rows ? E : max_rows;
-    const int avg = ceil_div(max_rows, active);
+    const int active = E < est_rows ? E : est_rows;
+    const int avg = ceil_div(est_rows, active);
     // bf16: with a CU's worth of tiles or more (192 of 256) the 256-column tiles of gemm256.hip stream the weights as
     // fast or faster (16 experts of 1024 -> 4096, 61 rows: 27 against 30 us); with fewer they leave CUs without work
     // (2 rows of 64 experts, 2048 -> 8192: h 24 against 17.5 us, out 66 against 13).  KC stops at 24 rows per expert,
@@ -398,7 +394,6 @@ static bool skinny_plan(int dtype, bool b_ks, int E, int max_rows, int N, int K,
     // rows per group: KC shares a block's weight loads among 32 rows once experts hold more than eight; KS in bf16 has
     // eight accumulators per 16 rows and runs better on more waves (groups of 16 re-read the weights out of the caches)
     p.mb = b_ks ? (bf16 ? 1 : 2) : (avg > 8 ? 2 : 1);
-    p.groups = active + max_rows / (16 * p.mb);
     // KS: about two blocks of eight waves per CU, every wave with at least two steps
     const int blocks = active * ceil_div(avg, 16 * p.mb) * ceil_div(N, 16 * epc);
     int ks = b_ks ? ceil_div(512, blocks) : 1;
@@ -409,10 +404,17 @@ static bool skinny_plan(int dtype, bool b_ks, int E, int max_rows, int N, int K,
     return true;
 }
 
-size_t gemm_skinny_workspace_bytes(int E, int max_rows, int N, int K, int dtype) {
+int gemm_skinny_ksplit(int E, int est_rows, int N, int K, int dtype) {
     SkinnyPlan p;
-    if (!skinny_plan(dtype, true, E, max_rows, N, K, p)) return 0;
-    return p.ksplit > 1 ? (size_t)p.ksplit * max_rows * N * sizeof(float) : 0;
+    return skinny_plan(dtype, true, E, est_rows, N, K, p) ? p.ksplit : 0;
+}
+
+int launch_plane_reduce(const GemmArgs &g, int dtype, int max_rows, hipStream_t st) {
+    const dim3 grid(ceil_div(g.N, 1024), (g.E < max_rows ? g.E : max_rows) + max_rows / RED_ROWS);
+    if (dtype == MOLE_BF16) hipLaunchKernelGGL(plane_reduce_kernel<bf16_t>, grid, dim3(256), 0, st, g);
+    else hipLaunchKernelGGL(plane_reduce_kernel<float>, grid, dim3(256), 0, st, g);
+    MOLE_LAUNCH_CHECK();
+    return 0;
 }
 
 template <typename T, int MB>
@@ -432,10 +434,7 @@ static int launch_ks(const GemmArgs &g, int epi, int groups, int max_rows, hipSt
     else if (epi == EPI_STORE) timed_launch(kid, skinny_ks_kernel<T, MB, EPI_STORE>, grid, dim3(SK_THREADS), 0, st, g);
     else return -100;
     MOLE_LAUNCH_CHECK();
-    if (g.ksplit > 1) {
-        hipLaunchKernelGGL(skinny_reduce_kernel<T>, dim3(ceil_div(g.N, 1024), (g.E < max_rows ? g.E : max_rows) + max_rows / SK_RED_ROWS), dim3(256), 0, st, g);
-        MOLE_LAUNCH_CHECK();
-    }
+    if (g.ksplit > 1) return launch_plane_reduce(g, sizeof(T) == 2 ? MOLE_BF16 : MOLE_F32, max_rows, st);
     return 0;
 }
 
@@ -443,7 +442,8 @@ int launch_gemm_skinny(const GemmArgs &g0, int dtype, bool b_ks, int epi, int ma
     GemmArgs g = g0;
     const int epc = dtype == MOLE_BF16 ? 8 : 4;
     SkinnyPlan p;
-    if (g.offsets == nullptr || g.kept == nullptr || !skinny_plan(dtype, b_ks, g.E, max_rows, g.N, g.K, p)) return -100;
+    if (max_rows <= 0 || g.offsets == nullptr || g.kept == nullptr || !skinny_plan(dtype, b_ks, g.E, g.est_rows, g.N, g.K, p)) return -100;
+    const int groups = (g.E < max_rows ? g.E : max_rows) + max_rows / (16 * p.mb);     // as many as max_rows rows can need
     if (g.K % epc || g.N % epc || g.lda % epc || g.ldb % epc || g.ldc % epc || g.strideB % epc) return -100;
     g.ksplit = 1;
     if (p.ksplit > 1 && ws != nullptr && ws_bytes >= (size_t)p.ksplit * max_rows * g.N * sizeof(float)) {
@@ -452,11 +452,11 @@ int launch_gemm_skinny(const GemmArgs &g0, int dtype, bool b_ks, int epi, int ma
         g.part_rows = max_rows;
     }
     if (dtype == MOLE_BF16) {
-        if (b_ks) return launch_ks<bf16_t, 1>(g, epi, p.groups, max_rows, st, kid);
-        return p.mb == 1 ? launch_kc<bf16_t, 1>(g, epi, p.groups, st, kid) : launch_kc<bf16_t, 2>(g, epi, p.groups, st, kid);
+        if (b_ks) return launch_ks<bf16_t, 1>(g, epi, groups, max_rows, st, kid);
+        return p.mb == 1 ? launch_kc<bf16_t, 1>(g, epi, groups, st, kid) : launch_kc<bf16_t, 2>(g, epi, groups, st, kid);
     }
-    if (b_ks) return launch_ks<float, 2>(g, epi, p.groups, max_rows, st, kid);
-    return p.mb == 1 ? launch_kc<float, 1>(g, epi, p.groups, st, kid) : launch_kc<float, 2>(g, epi, p.groups, st, kid);
+    if (b_ks) return launch_ks<float, 2>(g, epi, groups, max_rows, st, kid);
+    return p.mb == 1 ? launch_kc<float, 1>(g, epi, groups, st, kid) : launch_kc<float, 2>(g, epi, groups, st, kid);
 }
 
 }  // namespace mole

@@ -9,6 +9,10 @@
 
 namespace mole {
 
+// rows the experts hold in all likelihood: every pair, or the capacity's bound where that is less (the padded layout's
+// buffers have a row for every slot)
+static int est_rows(const mole_layer &L) { return L.rows < L.S * L.k ? L.rows : L.S * L.k; }
+
 static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // out [ro][co] in T = in [r][c] fp32, zeros beyond
@@ -61,7 +65,7 @@ using namespace mole;
 
 extern "C" size_t mole_layer_workspace_bytes(const mole_layer *L, int backward) {
     if (L == nullptr || L->S <= 0 || L->E <= 0) return 0;
-    const size_t ffn = mole_ffn_workspace_bytes(L->dtype, L->E, L->rows, L->M, L->F);
+    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
     const size_t other = backward ? gate_bwd_plan(*L).total : mole_gate_route_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
     return ffn > other ? ffn : other;        // the two are never in use at the same time
 }
@@ -85,8 +89,8 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
                                  L->layout, L->scores, L->idx, L->loc, L->gates, L->row, L->counts, L->kept_rows, L->offsets,
                                  L->capacity, L->l_aux, L->workspace, L->workspace_bytes, stream)) return rc;
     if (int rc = mole_dispatch_fwd(L->x, L->dtype, L->row, L->S, L->M, L->k, L->xd, stream)) return rc;
-    if (int rc = mole_ffn_fwd_ws(L->xd, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, L->M, L->F, L->w1, L->b1, L->w2, L->b2, L->h,
-                                 L->a, L->out, L->workspace, L->workspace_bytes, stream)) return rc;
+    if (int rc = ffn_fwd(L->xd, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, est_rows(*L), L->M, L->F, L->w1, L->b1, L->w2, L->b2, L->h,
+                                 L->a, L->out, L->workspace, L->workspace_bytes, (hipStream_t)stream)) return rc;
     return mole_combine_fwd(L->out, L->dtype, L->row, L->gates, L->S, L->M, L->k, y, stream);
 }
 
@@ -112,9 +116,9 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
                                    stream)) return rc;
     }
     // (the FFN's scratch takes the place of dgates and makes room for the gate's products, in stream order)
-    if (int rc = mole_ffn_bwd_ws(G->d_o, L->xd, L->h, L->a, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, L->M, L->F, L->w1, L->w2,
+    if (int rc = ffn_bwd(G->d_o, L->xd, L->h, L->a, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, est_rows(*L), L->M, L->F, L->w1, L->w2,
                                  G->t, G->g_w1, G->g_b1, G->g_w2, G->g_b2, G->gxd, G->accumulate, G->gelu_bwd, L->workspace,
-                                 L->workspace_bytes, stream)) return rc;
+                                 L->workspace_bytes, st)) return rc;
     char *dl_t = ws + p.dgates, *wg_t = dl_t + p.dl_t, *dx_add = wg_t + p.wg_t, *wgrad = dx_add + p.dx_add;
     if (p.dl_t)
         if (int rc = pad_convert(G->dlogits, L->S, L->E, dl_t, L->S, p.e_pad, L->dtype, st)) return rc;

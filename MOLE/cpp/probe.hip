@@ -77,7 +77,7 @@ extern "C" int mole_probe_kloop_part(const void *a, const void *b, const int32_t
     GemmArgs g{};
     g.offsets = offsets; g.kept = kept_rows; g.E = E;
     g.A = a; g.lda = K; g.B = b; g.ldb = K; g.strideB = (long)N * K; g.N = N; g.K = K; g.C = sink; g.ldc = N;
-    const int rc = launch_gemm256(g, false, false, false, EPI_NONE + part, max_rows, (hipStream_t)stream, MOLE_K_PROBE);
+    const int rc = launch_gemm256(g, false, false, false, EPI_NONE + part, max_rows, nullptr, 0, (hipStream_t)stream, MOLE_K_PROBE);
     MOLE_REQUIRE(rc != -100, "mole_probe_kloop: shape not taken by the 256-wide kernel");
     return rc;
 }

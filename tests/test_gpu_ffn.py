@@ -435,3 +435,32 @@ def test_ffn_contraction_ends_inside_a_stage(E, M, Fd, rows, gap):
         assert rel_err(got.cpu()[mask], want[mask]) < tol(dtype)
     for got, want in zip(g, w_g):
         assert rel_err(got, want) < tol(dtype)
+
+
+# K = F products whose contraction is split into planes: 256- and 320-row tiles in two to four planes, 128 x 128 tiles in two to
+# four, planes of unequal and of ragged length, columns that are not whole tiles, an expert with no rows; the two results
+# with a workspace (split) and without one.
+@pytest.mark.parametrize("E,M,Fd,rows,gap", [
+    (3, 264, 3080, [330, 0, 200], 2), (4, 1032, 3104, [375, 370, 380, 20], 0), (30, 520, 2056, [100 + (7 * e) % 50 for e in range(30)], 0),
+    (4, 72, 2088, [200, 130, 90, 300], 1), (2, 520, 1064, [129, 250], 0),
+])
+def test_ffn_split_contraction(E, M, Fd, rows, gap):
+    from mole_amd import hip_ops as H, _lib as L
+    dtype = torch.bfloat16
+    print(f"ffn planes E={E} M={M} F={Fd} rows={rows[:4]}", flush=True)
+    d = _make(E, M, Fd, rows, dtype, seed=M + Fd, pad_between=gap)
+    assert L.lib().mole_ffn_workspace_bytes(L.dtype_code(dtype), E, d["R"], M, Fd) > 0
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off = torch.from_numpy(d["off"]).cuda(); n = torch.from_numpy(d["n"]).cuda()
+    w_out, _, w_gx, *_ = _oracle_fwd_bwd(d, "tanh")
+    mask = torch.zeros(d["R"], dtype=torch.bool)
+    for e in range(E):
+        mask[int(d["off"][e]):int(d["off"][e]) + int(d["n"][e])] = True
+    out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+    g = [torch.empty_like(c[k]) for k in ("w1", "b1", "w2", "b2")]
+    gx = H.ffn_bwd(c["go"], c["xd"], h, a, off, n, c["w1"], c["w2"], *g)
+    assert rel_err(out.cpu()[mask], w_out[mask]) < tol(dtype) and rel_err(gx.cpu()[mask], w_gx[mask]) < tol(dtype)
+    out2, h2, a2 = torch.empty_like(out), torch.empty_like(h), torch.empty_like(a)
+    L.check(L.lib().mole_ffn_fwd(L.ptr(c["xd"]), L.dtype_code(dtype), L.ptr(off), L.ptr(n), E, d["R"], M, Fd, L.ptr(c["w1"]),
+                                 L.ptr(c["b1"]), L.ptr(c["w2"]), L.ptr(c["b2"]), L.ptr(h2), L.ptr(a2), L.ptr(out2), L.stream()), "ffn")
+    assert rel_err(out2.cpu()[mask], w_out[mask]) < tol(dtype)
