@@ -457,7 +457,7 @@ static int run_gemm(const GemmArgs &g, int max_rows, int tiles_generic, hipStrea
         }
     } else {
         if (fast_path_enabled()) {
-            const int rc = launch_gemm_f32(g, A_KS, B_KS, WG, EPI, max_rows, st, kid);
+            const int rc = launch_gemm_f32(g, A_KS, B_KS, WG, EPI, max_rows, ws, ws_bytes, st, kid);
             if (rc != -100) return rc;
         }
     }
@@ -552,7 +552,7 @@ namespace mole {
 size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, int F) {
     if (E <= 0 || max_rows <= 0 || M <= 0 || F <= 0) return 0;
     int ks = gemm_skinny_ksplit(E, est_rows, M, F, dtype);
-    if (ks == 0 && dtype == MOLE_BF16) ks = gemm256_ksplit(E, est_rows, M, F);
+    if (ks == 0) ks = dtype == MOLE_BF16 ? gemm256_ksplit(E, est_rows, M, F) : gemm_f32_ksplit(E, est_rows, M, F);
     return ks > 1 ? (size_t)ks * max_rows * M * sizeof(float) : 0;
 }
 

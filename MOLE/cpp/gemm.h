@@ -165,7 +165,8 @@ bool gemm256_sums_operand(const GemmArgs &g);
 int launch_gemm_skinny(const GemmArgs &g, int dtype, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
 int gemm_skinny_ksplit(int E, int est_rows, int N, int K, int dtype);    // 0: not its shape
 // fp32 tiles with direct-to-LDS loads (gemm_f32.hip); -100 as above.
-int launch_gemm_f32(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid);
+int launch_gemm_f32(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
+int gemm_f32_ksplit(int E, int est_rows, int N, int K);
 bool gemm_f32_sums_operand(const GemmArgs &g);
 
 }  // namespace mole

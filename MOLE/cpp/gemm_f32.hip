@@ -123,7 +123,9 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
     //      takes a contiguous range of the real tiles, so that neighbours share operands in its L2.  For row-ragged
     //      products the number of real tiles is only known here (the grid is sized for the worst case).
     const int n_tiles = (g.N + BN - 1) / BN;
-    int e, mt, nt, m_ext, k_ext;
+    // a contraction split over blocks: the planes of an m-tile's n-tiles are numbered like more n-tiles
+    const int n_units = EPI == EPI_PART ? n_tiles * g.ksplit : n_tiles;
+    int e, mt, nt, m_ext, k_ext, split_k = 0;
     long row0;
     if constexpr (!WG) {
         const bool single = g.offsets == nullptr;
@@ -131,13 +133,13 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
         int part = 0;
         for (int ee = lane; ee < nE; ee += WAVE) part += ((single ? g.single_rows : g.kept[ee]) + BM - 1) / BM;
         for (int d = WAVE / 2; d >= 1; d >>= 1) part += __shfl_xor(part, d, WAVE);
-        const int total = part * n_tiles;
+        const int total = part * n_units;
         const int per_xcd = (total + 7) >> 3;
         const int slot = blockIdx.x >> 3;
         const int t = (blockIdx.x & 7) * per_xcd + slot;
         if (slot >= per_xcd || t >= total) return;
-        const int mtg = t / n_tiles;
-        nt = t % n_tiles;
+        const int mtg = t / n_units;
+        nt = t % n_units;
         int run = 0, found = -1, fmt = 0;
         for (int base = 0; base < nE && found < 0; base += WAVE) {
             const int ee = base + lane;
@@ -160,6 +162,10 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
         m_ext = single ? g.single_rows : g.kept[e];
         row0 = single ? 0 : g.offsets[e];
         k_ext = g.K;
+        if constexpr (EPI == EPI_PART) {
+            split_k = nt / n_tiles;
+            nt %= n_tiles;
+        }
     } else {
         const int t = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
         if (t >= g.n_blocks) return;
@@ -181,6 +187,14 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
     const int m0 = mt * BM, n0 = nt * BN;
     const float *Mp = (const float *)g.A + row0 * g.lda;
     const float *Np = WG ? (const float *)g.B + row0 * g.ldb : (const float *)g.B + (long)e * g.strideB;
+    if constexpr (EPI == EPI_PART) {           // this block's stages of the contraction (which is whole stages)
+        split_k = __builtin_amdgcn_readfirstlane(split_k);
+        const int stages = k_ext / F_BK;
+        const int k_lo = split_k * stages / g.ksplit * F_BK;
+        k_ext = (split_k + 1) * stages / g.ksplit * F_BK - k_lo;
+        Mp += k_lo;
+        Np += N_KS ? (long)k_lo * g.ldb : (long)k_lo;
+    }
     const int wm = wave >> 1, wn = wave & 1;
 
     f32x16 acc[TMW][TNW];
@@ -355,8 +369,9 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
     // ---- epilogue.  acc[tm][tn][q] = C[m, n] with i = 8 (q / 4) + 4 (lane / 32) + q % 4 the row inside the m-block and
     //      lane % 32 the column inside the n-block; a K-strided side interleaves the wave's blocks (row 2 i + tm).
     const int lr = lane & 31, h = lane >> 5;
-    float *Cb = (float *)g.C;
-    long crow0 = row0;
+    float *Cb = EPI == EPI_PART ? g.part : (float *)g.C;
+    const long ldc = EPI == EPI_PART ? (long)g.N : g.ldc;
+    long crow0 = EPI == EPI_PART ? split_k * g.part_rows + row0 : row0;
     if constexpr (WG) { crow0 = 0; Cb += (long)e * g.strideC; }
     constexpr bool PAIR = N_KS && TNW == 2;         // a lane holds two adjacent columns: 8-byte accesses
     int ncol[TNW];
@@ -384,11 +399,11 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
                 for (int q = 0; q < 16; ++q) {
                     const long r = crow0 + min(row_of(tm, q), m_ext - 1);
                     if constexpr (PAIR) {
-                        const float2 t = *reinterpret_cast<const float2 *>(src + r * g.ldc + min(ncol[0], g.N - 2));
+                        const float2 t = *reinterpret_cast<const float2 *>(src + r * ldc + min(ncol[0], g.N - 2));
                         old[q][0] = t.x; old[q][1] = t.y;
                     } else {
 #pragma unroll
-                        for (int tn = 0; tn < TNW; ++tn) old[q][tn] = src[r * g.ldc + min(ncol[tn], g.N - 1)];
+                        for (int tn = 0; tn < TNW; ++tn) old[q][tn] = src[r * ldc + min(ncol[tn], g.N - 1)];
                     }
                 }
             }
@@ -414,7 +429,7 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
                     if (g.accumulate) v[tn] += old[q][tn];
                 }
             }
-            float *dst = Cb + (crow0 + m) * g.ldc;
+            float *dst = Cb + (crow0 + m) * ldc;
             // The weight gradients (which nothing reads before the optimizer) leave with non-temporal stores: -2 us on
             // 8 x 2048 x 512.  For h, a and t it measured neutral to worse: the launches that follow read them.
             constexpr bool STREAM = EPI == EPI_WGRAD;
@@ -429,14 +444,14 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
             if constexpr (PAIR) {
                 if (ncol[0] < g.N) {
                     put2(dst + ncol[0], v[0], v[1]);
-                    if constexpr (EPI == EPI_BIAS_GELU) put2((float *)g.C2 + (crow0 + m) * g.ldc + ncol[0], v2[0], v2[1]);
+                    if constexpr (EPI == EPI_BIAS_GELU) put2((float *)g.C2 + (crow0 + m) * ldc + ncol[0], v2[0], v2[1]);
                 }
             } else {
 #pragma unroll
                 for (int tn = 0; tn < TNW; ++tn) {
                     if (ncol[tn] >= g.N) continue;
                     put(dst + ncol[tn], v[tn]);
-                    if constexpr (EPI == EPI_BIAS_GELU) put((float *)g.C2 + (crow0 + m) * g.ldc + ncol[tn], v2[tn]);
+                    if constexpr (EPI == EPI_BIAS_GELU) put((float *)g.C2 + (crow0 + m) * ldc + ncol[tn], v2[tn]);
                 }
             }
         }
@@ -479,6 +494,7 @@ int dispatch_f32(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_rows, h
     } else {
         if (epi == EPI_BIAS) return launch_f32<BM, BN, NSTAGE, BPC, false, true, false, EPI_BIAS>(g, tiles, st, kid);
         if (epi == EPI_STORE) return launch_f32<BM, BN, NSTAGE, BPC, false, true, false, EPI_STORE>(g, tiles, st, kid);
+        if (epi == EPI_PART) return launch_f32<BM, BN, NSTAGE, BPC, false, true, false, EPI_PART>(g, tiles * g.ksplit, st, kid);
     }
     return -100;
 }
@@ -501,7 +517,30 @@ bool gemm_f32_sums_operand(const GemmArgs &g) {
     return !(g.lda % 4 || g.ldb % 4 || g.ldc % 4 || g.N % 4 || g.N < 4 || g.M % 4 || g.M < 4);
 }
 
-int launch_gemm_f32(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid) {
+// The K = F products are narrow and long: their tiles, each a serial walk over K at the matrix pipes' rate, do not divide
+// evenly among the 256 CUs.  A CU works off its blocks one after the other (two side by side share the pipes), so a
+// launch takes ceil(tiles / 256) walks; split into p planes of partial results it takes ceil(p tiles / 256) / p, plus
+// the planes' way through memory and the reduction's launch.  The fewest microseconds win, by the walk's 0.55 us per
+// stage and a plane's traffic at 5 TB/s.
+static int plan_ksplit(int E, int est_rows, int N, int K) {
+    const int active = E < est_rows ? E : est_rows;
+    if (active <= 0 || K % F_BK) return 1;
+    const int avg = ceil_div(est_rows, active);
+    const long tiles = (long)active * ceil_div(avg, 64) * ceil_div(N, 128);
+    const double walk = K / F_BK * 0.55, plane = 2.0 * est_rows * N * sizeof(float) / 5.0e6;
+    int best = 1;
+    double least = (double)((tiles + 255) / 256) * walk;
+    for (int p = 2; p <= 4 && K / p >= 16 * F_BK; ++p) {
+        const double us = (double)((p * tiles + 255) / 256) / p * walk + p * plane + 6.0;
+        if (us < least) { least = us; best = p; }
+    }
+    return best;
+}
+int gemm_f32_ksplit(int E, int est_rows, int N, int K) { return plan_ksplit(E, est_rows, N, K); }
+
+int launch_gemm_f32(const GemmArgs &g0, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid) {
+    GemmArgs g = g0;
+    g.ksplit = 1;
     // what the direct-to-LDS path relies on: 16-byte rows, whole stages of K for row-ragged products
     if (g.lda % 4 || g.ldb % 4 || g.ldc % 4 || g.N % 4 || g.N < 4) return -100;
     if (!wg && (a_ks || g.K <= 0 || g.K % F_BK)) return -100;
@@ -509,6 +548,16 @@ int launch_gemm_f32(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, i
     if (wg) return dispatch_f32<128, 128, 4, 2>(g, b_ks, wg, epi, max_rows, st, kid);
     const int rows = g.offsets ? max_rows : g.single_rows;
     const long tiles = (long)ceil_div(rows, 64) * ceil_div(g.N, 128);
+    if (b_ks && g.offsets != nullptr && ws != nullptr) {
+        const int p = plan_ksplit(g.E, g.est_rows, g.N, g.K);
+        if (p > 1 && ws_bytes >= (size_t)p * max_rows * g.N * sizeof(float)) {
+            g.ksplit = p;
+            g.part = (float *)ws;
+            g.part_rows = max_rows;
+            const int rc = dispatch_f32<64, 128, 4, 2>(g, b_ks, wg, EPI_PART, max_rows, st, kid);
+            return rc != 0 ? rc : launch_plane_reduce(g, MOLE_F32, max_rows, st);
+        }
+    }
     if (tiles >= 4 * 256) return dispatch_f32<64, 128, 3, 4>(g, b_ks, wg, epi, max_rows, st, kid);
     return dispatch_f32<64, 128, 4, 2>(g, b_ks, wg, epi, max_rows, st, kid);
 }

@@ -464,3 +464,31 @@ def test_ffn_split_contraction(E, M, Fd, rows, gap):
     L.check(L.lib().mole_ffn_fwd(L.ptr(c["xd"]), L.dtype_code(dtype), L.ptr(off), L.ptr(n), E, d["R"], M, Fd, L.ptr(c["w1"]),
                                  L.ptr(c["b1"]), L.ptr(c["w2"]), L.ptr(c["b2"]), L.ptr(h2), L.ptr(a2), L.ptr(out2), L.stream()), "ffn")
     assert rel_err(out2.cpu()[mask], w_out[mask]) < tol(dtype)
+
+
+# The same in fp32: 64 x 128 tiles in two to four planes of equal and of unequal length, columns that are not whole tiles,
+# an expert with no rows, gaps between the experts.  Without a workspace the same products run in one piece; sums of the
+# same fp32 terms in another order differ by a few rounding errors of the partial sums, far inside the tolerance.
+@pytest.mark.parametrize("E,M,Fd,rows,gap", [
+    (1, 132, 2064, [70], 0), (8, 512, 2048, [190 + e for e in range(8)], 2), (3, 68, 1040, [100, 0, 129], 1), (5, 260, 784, [65, 80, 193, 64, 90], 0),
+])
+def test_ffn_split_contraction_fp32(E, M, Fd, rows, gap):
+    from mole_amd import hip_ops as H, _lib as L
+    dtype = torch.float32
+    print(f"ffn fp32 planes E={E} M={M} F={Fd} rows={rows[:4]}", flush=True)
+    d = _make(E, M, Fd, rows, dtype, seed=M + Fd, pad_between=gap)
+    assert L.lib().mole_ffn_workspace_bytes(L.dtype_code(dtype), E, d["R"], M, Fd) > 0
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off = torch.from_numpy(d["off"]).cuda(); n = torch.from_numpy(d["n"]).cuda()
+    w_out, _, w_gx, *_ = _oracle_fwd_bwd(d, "tanh")
+    mask = torch.zeros(d["R"], dtype=torch.bool)
+    for e in range(E):
+        mask[int(d["off"][e]):int(d["off"][e]) + int(d["n"][e])] = True
+    out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+    g = [torch.empty_like(c[k]) for k in ("w1", "b1", "w2", "b2")]
+    gx = H.ffn_bwd(c["go"], c["xd"], h, a, off, n, c["w1"], c["w2"], *g)
+    assert rel_err(out.cpu()[mask], w_out[mask]) < tol(dtype) and rel_err(gx.cpu()[mask], w_gx[mask]) < tol(dtype)
+    out2, h2, a2 = torch.empty_like(out), torch.empty_like(h), torch.empty_like(a)
+    L.check(L.lib().mole_ffn_fwd(L.ptr(c["xd"]), L.dtype_code(dtype), L.ptr(off), L.ptr(n), E, d["R"], M, Fd, L.ptr(c["w1"]),
+                                 L.ptr(c["b1"]), L.ptr(c["w2"]), L.ptr(c["b2"]), L.ptr(h2), L.ptr(a2), L.ptr(out2), L.stream()), "ffn")
+    assert torch.equal(h2.cpu()[mask], h.cpu()[mask]) and rel_err(out2.cpu()[mask], w_out[mask]) < tol(dtype)
