@@ -812,10 +812,9 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
         // contiguous ranges: the (expert, m-tile) units are dealt round-robin over the 8 XCDs, which gives
         // every XCD the same share of every expert; the n-tiles of a unit stay together (they share the
         // m-side operand in that XCD's L2).
-        // With hundreds of experts of similar size that spread is not needed, and it costs traffic: the m-tiles of
-        // an expert on different XCDs each fetch the expert's rows of the n-side operand into their own L2 (3x the
-        // operands' bytes at 256 experts, which made the launch HBM-bound).  Then (wg_expert_major) the experts are
-        // dealt round-robin instead, all blocks of one expert on one XCD.
+        // With hundreds of experts of many rows that spread costs more traffic than it is worth: the m-tiles of an expert
+        // on different XCDs each fetch the expert's rows of the n-side operand into their own L2.  Then (wg_expert_major)
+        // the experts are dealt round-robin instead, all blocks of one expert on one XCD.
         const int m_tiles = (g.M + Q_BM - 1) / Q_BM;
         const int slot = blockIdx.x >> 3;
         if (g.wg_expert_major) {
@@ -970,20 +969,18 @@ static int launch256(const GemmArgs &g, int tiles, hipStream_t st, int kid) {
 
 // Launch options and their defaults; a -DMOLE_TUNING build reads them from the environment
 // (MOLE_MFAST: bit mask of the products that number an expert's tiles m-tile first within groups of MOLE_MFAST_G
-// n-tiles, MOLE_MFAST_FROM: m-tiles an expert needs for that order, MOLE_WG_EMAJOR: expert count from which a weight gradient keeps an expert's blocks on one XCD,
+// n-tiles, MOLE_MFAST_FROM: m-tiles an expert needs for that order,
 // MOLE_NO_SUMS: bias gradients from their own kernel).
 #ifdef MOLE_TUNING
 static int env_int(const char *name, int dflt) { const char *v = getenv(name); return v ? atoi(v) : dflt; }
 static int m_fastest_mask() { static const int v = env_int("MOLE_MFAST", 9); return v; }
 static int m_fastest_group() { static const int v = env_int("MOLE_MFAST_G", 8); return v > 0 ? v : 1; }
 static int m_fastest_from() { static const int v = env_int("MOLE_MFAST_FROM", 8); return v; }
-static int wg_emajor_from() { static const int v = env_int("MOLE_WG_EMAJOR", 128); return v; }
 static bool sums_off() { static const bool v = getenv("MOLE_NO_SUMS") != nullptr; return v; }
 #else
 static int m_fastest_mask() { return 9; }        // h = xd.w1^T + b1 and t = (go.w2^T) gelu'(h)
 static int m_fastest_group() { return 8; }
 static int m_fastest_from() { return 8; }
-static int wg_emajor_from() { return 128; }
 static bool sums_off() { return false; }
 #endif
 
@@ -991,10 +988,13 @@ template <int TMB, int WM, int WN>
 static int dispatch256(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid) {
     constexpr int BM = Tile<TMB, WM, WN>::BM;
     const int n_tiles = ceil_div(g.N, (Tile<TMB, WM, WN>::BN));
-    if constexpr (TMB == 8) {
+    if constexpr (TMB == 8 || TMB == 4) {
         if (wg) {
+            // All blocks of an expert on one XCD from 128 experts of 768 rows on: 256 experts of 2048 x 1024, 1024 rows each,
+            // the training step 8624 against 8788 us.  With fewer rows it gains nothing (256 rows each: 482 against 486 us a
+            // product) and loses under skewed loads, where a few XCDs get the large experts (Zipf(1.2): 755 against 516 us).
             GemmArgs gw = g;
-            gw.wg_expert_major = g.E >= wg_emajor_from();
+            gw.wg_expert_major = g.E >= 128 && g.est_rows / g.E >= 768;
             // whole (expert, m-tile) units per XCD, or whole experts
             const int tiles = gw.wg_expert_major ? 8 * ceil_div(g.E, 8) * ceil_div(g.M, BM) * n_tiles
                                                  : 8 * ceil_div(g.E * ceil_div(g.M, BM), 8) * n_tiles;
@@ -1086,6 +1086,16 @@ static TilePlan tile_plan(int E, int est_rows, int N, int K, bool tall) {
     }
     return p;
 }
+// Weight gradients.  A CU pair of 128 x 128 blocks does 0.6-0.65 of the work of a 256 x 256 block in half the time of one
+// (its operands cross LDS once per 128 rows instead of 256: 16 experts of 1024 x 4096, 512 rows each, 109 against 88 us),
+// but wastes less where the large tiles do not fit the matrix or the last round of them is nearly empty: a round of
+// 256 large tiles costs what 768 small ones do.  128 x 128 against 256 x 256: 16 experts of 520 x 1416, 128 rows, 17 / 22 us;
+// 512 x 512, 1000 rows, 20 / 30; 4 of 512 x 2048, 500 rows, 13 / 19; 63 of 384 x 1536, 344 rows, 55 / 58; on the other
+// side of the line 8 experts of 1024 x 3072, 500 rows, 44 / 41; 123 of 256 x 512, 325 rows, 29 / 27.
+static int wgrad_tile(int E, int M, int N) {
+    const long t256 = (long)E * ceil_div(M, 256) * ceil_div(N, 256), t128 = (long)E * ceil_div(M, 128) * ceil_div(N, 128);
+    return t128 < 768 * ((t256 + 255) / 256) ? TILE_128 : TILE_256;
+}
 int gemm256_ksplit(int E, int est_rows, int N, int K) { return tile_plan(E, est_rows, N, K, true).ksplit; }
 
 // Whether the weight-gradient launch for g will also produce the operand sums asked for in g.colsum.
@@ -1101,6 +1111,7 @@ int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, in
     if (wg && (!a_ks || !b_ks || g.M % 8)) return -100;
     TilePlan p{TILE_256, 1};
     if (!wg && g.offsets != nullptr && epi < EPI_NONE) p = tile_plan(g.E, g.est_rows, g.N, g.K, b_ks);
+    if (wg && epi == EPI_WGRAD) p.tile = wgrad_tile(g.E, g.M, g.N);
     GemmArgs gp = g;
     gp.ksplit = 1;
     if (p.ksplit > 1 && b_ks && ws != nullptr && ws_bytes >= (size_t)p.ksplit * max_rows * g.N * sizeof(float)) {

@@ -492,3 +492,24 @@ def test_ffn_split_contraction_fp32(E, M, Fd, rows, gap):
     L.check(L.lib().mole_ffn_fwd(L.ptr(c["xd"]), L.dtype_code(dtype), L.ptr(off), L.ptr(n), E, d["R"], M, Fd, L.ptr(c["w1"]),
                                  L.ptr(c["b1"]), L.ptr(c["w2"]), L.ptr(c["b2"]), L.ptr(h2), L.ptr(a2), L.ptr(out2), L.stream()), "ffn")
     assert torch.equal(h2.cpu()[mask], h.cpu()[mask]) and rel_err(out2.cpu()[mask], w_out[mask]) < tol(dtype)
+
+
+# bf16 weight gradients by 128 x 128 tiles: widths below, at and just past a tile's edge, contractions of less than one
+# stage up to several rings of stages, experts without rows, written and added to what is there.
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("E,M,Fd,rows,gap", [
+    (1, 8, 8, [1], 0), (3, 128, 128, [31, 0, 33], 0), (2, 136, 264, [64, 250], 1), (5, 520, 1416, [128, 97, 1, 0, 161], 2), (33, 72, 120, [(13 * e) % 70 for e in range(33)], 0),
+])
+def test_ffn_weight_gradients_by_small_tiles(E, M, Fd, rows, gap, accumulate):
+    from mole_amd import hip_ops as H
+    dtype = torch.bfloat16
+    print(f"ffn weight gradients E={E} M={M} F={Fd} rows={rows[:5]} accumulate={accumulate}", flush=True)
+    d = _make(E, M, Fd, rows, dtype, seed=E + M + Fd, pad_between=gap)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off = torch.from_numpy(d["off"]).cuda(); n = torch.from_numpy(d["n"]).cuda()
+    *_, w_gw1, w_gb1, w_gw2, w_gb2 = _oracle_fwd_bwd(d, "tanh")
+    out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+    g = [torch.full_like(c[k], 0.5) for k in ("w1", "b1", "w2", "b2")]
+    H.ffn_bwd(c["go"], c["xd"], h, a, off, n, c["w1"], c["w2"], *g, accumulate=accumulate)
+    for got, want in zip(g, (w_gw1, w_gb1, w_gw2, w_gb2)):
+        assert rel_err(got, want + 0.5 if accumulate else want) < tol(dtype)
