@@ -148,6 +148,7 @@ struct GemmArgs {
     float *part;            // fp32 partial results [ksplit][part_rows][N] of a contraction split over blocks
     long part_rows;
     int ksplit;
+    int once;               // row-ragged products with K-strided weights: see weights_pass_by()
     int est_rows;           // host's estimate of the rows of all experts together (no more than the launch's bound)
     int m_fastest;          // row-ragged products, 256-wide kernel: number an expert's tiles m-tile first (see gemm256.hip)
 };

@@ -195,7 +195,8 @@ template <int TMB, int WM, int WN, bool M_KS, bool N_KS, int TMC, int TMCW> stru
 // Of a K-contiguous m-side tile only the 64-row groups that hold live 32-row blocks (the first TMC) are fetched.
 // KT: the contraction may end inside a stage (weight gradients always may; row-ragged products when K is not a multiple of
 // 32).  The last stage's loads are then clamped to what exists and main_loop zeroes what lies past it.
-template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC> struct Feeder {
+// ONCE: no other tile reads this tile's n-side panel (the weights of an expert with a single m-tile).
+template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC, bool ONCE> struct Feeder {
     typedef Tile<TMB, WM, WN> TL;
     typedef Stage<TMB, WM, WN, M_KS, TMC> SG;
     static constexpr int LM = SG::LM, L = SG::L;
@@ -235,7 +236,8 @@ template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC> struc
             } else {
                 uint32_t o = on.off[j - LM];
                 if constexpr (KT) o = clamp_k ? cn.off[j - LM] : o;
-                dma16s(bn, o, dst + SG::M_OPERAND + (j - LM) * (TL::NW * 1024));
+                if constexpr (ONCE) dma16s_nt(bn, o, dst + SG::M_OPERAND + (j - LM) * (TL::NW * 1024));
+                else dma16s(bn, o, dst + SG::M_OPERAND + (j - LM) * (TL::NW * 1024));
             }
         }
         if (J1 == L && s + 1 < nk) { bm += step_m; bn += step_n; }
@@ -282,14 +284,14 @@ template <int B, int L, int X> __device__ __forceinline__ void wait_stages_behin
 // BIAS: the accumulators start from the bias of their columns instead of zero (bias_raw: the 8 x 4 columns a lane
 // holds, fetched before the operand loads and therefore landed when the first stage has), so that the epilogue adds
 // nothing.
-template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC, int TMCW, int SUM, int PART = 0, bool BIAS = false>
+template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC, int TMCW, int SUM, bool ONCE = false, int PART = 0, bool BIAS = false>
 __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, int m_ext, const bf16_t *Np, long ldn,
                                           int n0, int n_ext, int k_ext, char *smem, int wave, int wm, int wn,
                                           f32x16 (&acc)[Tile<TMB, WM, WN>::TMW][2], f32x16 &sums, const uint2 (&bias_raw)[8]) {
     typedef Tile<TMB, WM, WN> TL;
     typedef Stage<TMB, WM, WN, M_KS, TMC> SG;
     constexpr int AHEAD = SG::NSTAGE - 1, NP = 4;
-    typedef Feeder<TMB, WM, WN, M_KS, N_KS, KT, TMC> FD;
+    typedef Feeder<TMB, WM, WN, M_KS, N_KS, KT, TMC, ONCE> FD;
     constexpr int L = FD::L, LH = L / 2;      // loads per wave per stage; the halves are LH and L - LH
     const int nk = __builtin_amdgcn_readfirstlane((k_ext + Q_BK - 1) / Q_BK);
     if (nk == 0) return;
@@ -921,16 +923,23 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
     f32x16 sums;
 #pragma unroll
     for (int q = 0; q < 16; ++q) sums[q] = 0.f;
-#define MOLE_RUN_TILE_SUM(C, SUM)                                                                                         \
+#define MOLE_RUN_TILE_AS(C, SUM, ONCE)                                                                                         \
     {                                                                                                                     \
-        main_loop<TMB, WM, WN, M_KS, N_KS, KT, WM *(C), (C), SUM, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw); \
+        main_loop<TMB, WM, WN, M_KS, N_KS, KT, WM *(C), (C), SUM, ONCE, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw); \
         if constexpr (SUM != 0) store_sums<SUM, (C)>(g, sums, e, m0, n0, m_ext, wm, wn, lane);                            \
         epilogue<TMB, WM, WN, WG, EPI, (C)>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, bias_raw, split_k);      \
     }
-#define MOLE_RUN_TILE(C) MOLE_RUN_TILE_SUM(C, 0)
+#define MOLE_RUN_TILE_SUM(C, SUM) MOLE_RUN_TILE_AS(C, SUM, false)
+#define MOLE_RUN_TILE(C) MOLE_RUN_TILE_AS(C, 0, false)
     if constexpr (WG && WM == 2 && TMW <= WN) {
         if (sum_side == 1) { MOLE_RUN_TILE_SUM(TMW, 1) return; }
         if (sum_side == 2) { MOLE_RUN_TILE_SUM(TMW, 2) return; }
+    }
+    if constexpr (N_KS && !WG && TMB >= 8) {
+        // The only m-tile of an expert with few rows: its weights pass by once, and the launch is their stream.  (256 experts
+        // of 1024 -> 2048 with 8 rows each, 1.07 GB: 197 -> 180 us; 149 of 1536 -> 1536, 17 rows: 143 -> 133.)
+        if (g.once && m_ext <= 64) { MOLE_RUN_TILE_AS(1, 0, true) return; }
+        if (g.once && m_ext <= 128) { MOLE_RUN_TILE_AS(2, 0, true) return; }
     }
     if (c >= TMW) MOLE_RUN_TILE(TMW)
     else if (TMW > 4 && c == 4) MOLE_RUN_TILE(TMW > 4 ? 4 : 1)
@@ -939,6 +948,7 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
     else MOLE_RUN_TILE(1)
 #undef MOLE_RUN_TILE
 #undef MOLE_RUN_TILE_SUM
+#undef MOLE_RUN_TILE_AS
 }
 
 template <int TMB, int WM, int WN, bool N_KS, bool WG, bool KT, int EPI>

@@ -119,6 +119,20 @@ template <typename T> __device__ __forceinline__ void sk_load4(const T *p, float
     }
 }
 
+// 16 bytes of a weight.  ONCE: no other block reads them, so they leave no copy behind (non-temporal): a plain stream of
+// 1 GB runs at 6.4 instead of 5.8 TB/s that way on this chip.  Only for KS, whose loads cover whole 128-byte lines: a KC
+// load takes 64 bytes of a row and the next one the other half of the line, which a non-temporal load has let go of by
+// then (123 experts of 448 -> 1344, fp32, 2 rows each: KS 59 -> 53 us, KC 57 -> 80).
+template <bool ONCE> __device__ __forceinline__ uint4 sk_weight(const void *p) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    if constexpr (ONCE) {
+        const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
+        return make_uint4(v[0], v[1], v[2], v[3]);
+    } else {
+        return *reinterpret_cast<const uint4 *>(p);
+    }
+}
+
 // Four consecutive columns n .. n+3 (all inside the result: N is a multiple of 4) of row `row` of expert e.
 template <typename T, int EPI>
 __device__ __forceinline__ void sk_epilogue4(const GemmArgs &g, int e, long row, int n, float (&v)[4]) {
@@ -239,7 +253,7 @@ __global__ __launch_bounds__(SK_THREADS, 4) void skinny_kc_kernel(const GemmArgs
 // ---- weights [K][N] ---------------------------------------------------------------------------------------------
 // A block owns 16 EPC result columns (256 bytes of a weight row) of one group of up to 16 MB rows and 1 / ksplit of the
 // contraction, which its eight waves split again; a wave has the weights of one step (EPC loads of 1 KiB) in flight.
-template <typename T, int MB, int EPI>
+template <typename T, int MB, bool ONCE, int EPI>
 __device__ __forceinline__ void skinny_ks_run(const GemmArgs &g, sk_f32x4 (&red)[SK_WAVES][SkElem<T>::EPC][WAVE], int e, int rows,
                                               long row0, int m0, int n0, int split) {
     constexpr int EPC = SkElem<T>::EPC, KSTEP = 4 * EPC;
@@ -261,7 +275,7 @@ __device__ __forceinline__ void skinny_ks_run(const GemmArgs &g, sk_f32x4 (&red)
         const int k = min(s * KSTEP + kg * EPC, g.K - EPC);
         const T *wk = wp + (long)k * g.ldb;
 #pragma unroll
-        for (int q = 0; q < EPC; ++q) w[q] = *reinterpret_cast<const uint4 *>(wk + (long)q * g.ldb);
+        for (int q = 0; q < EPC; ++q) w[q] = sk_weight<ONCE>(wk + (long)q * g.ldb);
 #pragma unroll
         for (int b = 0; b < MB; ++b) x[b] = *reinterpret_cast<const uint4 *>(xp[b] + k);
         __builtin_amdgcn_sched_barrier(0);
@@ -326,8 +340,9 @@ __global__ __launch_bounds__(SK_THREADS, 4) void skinny_ks_kernel(const GemmArgs
     if (!sk_find_group<16 * MB>(g, blockIdx.x / per_group, e, grp, rows, row0)) return;
     const int in_group = blockIdx.x % per_group;
     const int n0 = (in_group % chunks) * BN, split = in_group / chunks, m0 = grp * (16 * MB), live = rows - m0;
-    if (MB == 1 || live <= 16) skinny_ks_run<T, 1, EPI>(g, red, e, rows, row0, m0, n0, split);
-    else skinny_ks_run<T, MB, EPI>(g, red, e, rows, row0, m0, n0, split);
+    if (rows <= 16 && g.once) skinny_ks_run<T, 1, true, EPI>(g, red, e, rows, row0, m0, n0, split);
+    else if (MB == 1 || live <= 16) skinny_ks_run<T, 1, false, EPI>(g, red, e, rows, row0, m0, n0, split);
+    else skinny_ks_run<T, MB, false, EPI>(g, red, e, rows, row0, m0, n0, split);
 }
 
 // out[row][n] = bias[n] + sum over the planes of part[plane][row][n], for the rows of the launch's experts

@@ -90,7 +90,7 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
                                  L->capacity, L->l_aux, L->workspace, L->workspace_bytes, stream)) return rc;
     if (int rc = mole_dispatch_fwd(L->x, L->dtype, L->row, L->S, L->M, L->k, L->xd, stream)) return rc;
     if (int rc = ffn_fwd(L->xd, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, est_rows(*L), L->M, L->F, L->w1, L->b1, L->w2, L->b2, L->h,
-                                 L->a, L->out, L->workspace, L->workspace_bytes, (hipStream_t)stream)) return rc;
+                                 L->a, L->out, L->workspace, L->workspace_bytes, L->forward_only, (hipStream_t)stream)) return rc;
     return mole_combine_fwd(L->out, L->dtype, L->row, L->gates, L->S, L->M, L->k, y, stream);
 }
 

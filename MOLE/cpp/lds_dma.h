@@ -22,6 +22,10 @@ __device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_off) {
 __device__ __forceinline__ void dma16s(const void *sbase, uint32_t voff, uint32_t lds_off) {
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_off) : "memory");
 }
+// The same for data that no other block reads: non-temporal, leaving no copy behind in the caches.
+__device__ __forceinline__ void dma16s_nt(const void *sbase, uint32_t voff, uint32_t lds_off) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(sbase), "s"(lds_off) : "memory");
+}
 __device__ __forceinline__ const char *uniform_ptr(const void *p) {   // tell the compiler the pointer is wave-uniform
     const uint64_t v = (uint64_t)p;
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));

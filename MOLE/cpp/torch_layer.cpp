@@ -127,6 +127,7 @@ std::pair<Tensor, Tensor> run_forward(Call &c, const Tensor &x, const Tensor &wg
     char *a = (char *)act.data_ptr();
     mole_layer L = arguments(c, x, wg, (char *)c.route.data_ptr(), a, a + p.act_off[Plan::ACT_WS], p.ws_fwd);
     if (l_aux.defined()) L.l_aux = l_aux.data_ptr<float>();
+    else L.forward_only = 1;
     check(mole_layer_fwd(&L, y.data_ptr(), current_stream(x)), "mole_layer_fwd");
     return {y, act};
 }

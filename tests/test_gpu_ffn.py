@@ -513,3 +513,19 @@ def test_ffn_weight_gradients_by_small_tiles(E, M, Fd, rows, gap, accumulate):
     H.ffn_bwd(c["go"], c["xd"], h, a, off, n, c["w1"], c["w2"], *g, accumulate=accumulate)
     for got, want in zip(g, (w_gw1, w_gb1, w_gw2, w_gb2)):
         assert rel_err(got, want + 0.5 if accumulate else want) < tol(dtype)
+
+
+# K-strided weights read past the caches: experts with one m-tile of one or two live row blocks per wave, with more rows (the
+# ordinary loads) and with none, in a forward pass that no backward follows.  The loads' cache policy changes no result.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("E,M,k,S", [(200, 128, 1, 61), (200, 256, 2, 3000), (2, 1024, 1, 5), (3, 64, 1, 300)])
+def test_forward_only_weights_leave_no_copy(E, M, k, S, dtype):
+    from mole_amd.moe.layer import MOLEModule
+    print(f"forward only E={E} M={M} k={k} S={S} {dtype}", flush=True)
+    MOLEModule.reset_instances()
+    m = MOLEModule(0, E, M, 192, -1, k, 4, {"local_rank": 0, "world_size": 1, "rank": 0}, "gelu", 1, False, False, dtype=dtype)
+    x = torch.randn(S, M, generator=torch.Generator().manual_seed(S)).to(dtype).cuda()
+    y = m(x, capacity_factor=0.0).detach()            # recorded: the general policy
+    with torch.no_grad():
+        assert torch.equal(m(x, capacity_factor=0.0), y)
+    MOLEModule.reset_instances()
