@@ -212,17 +212,17 @@ __global__ __launch_bounds__(PM_THREADS) void dispatch_bwd_kernel(const T *__res
     }
 }
 
-// dispatch backward with the gate's input gradient folded in, for small gates (E <= 32): a thread
+// fp32 dispatch backward with the gate's input gradient folded in, for small gates (E <= 32): a thread
 // owns 4 columns and keeps its 4 x E slice of Wg in registers; the block walks db_tokens tokens (8 or 32), whose
 // row indices and dlogits are block-uniform (scalar loads).  Larger gates use the kernel above.
 constexpr int DB_TOKENS = 32;   // tokens per block when there are enough of them to fill the chip several times over
 constexpr int DB_TOKENS_FEW = 8;   // otherwise: more, shorter blocks (4096 x 512 fp32 tokens: 10.5 against 22 us)
-template <typename T, int EB>
-__global__ __launch_bounds__(256) void dispatch_bwd_gate_kernel(const T *__restrict__ dxd,
+template <int EB>
+__global__ __launch_bounds__(256) void dispatch_bwd_gate_kernel(const float *__restrict__ dxd,
                                                                 const int32_t *__restrict__ row, int S, int M, int k,
                                                                 const float *__restrict__ dlogits,
                                                                 const float *__restrict__ wg, int E,
-                                                                T *__restrict__ dx, int db_tokens) {
+                                                                float *__restrict__ dx, int db_tokens) {
     const int m = (blockIdx.y * 256 + threadIdx.x) * 4;
     if (m >= M) return;
     float w[EB][4];
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(256) void dispatch_bwd_gate_kernel(const T *__restr
     // Eight tokens per batch; the first choice's row gathers of the next batch are in flight while the
     // current batch is finished: one token at a time, or one batch at a time, runs at the memory latency.
     constexpr int U = 8;
-    typedef typename std::conditional<sizeof(T) == 2, uint2, float4>::type Raw;
+    typedef float4 Raw;
     // (every load is issued unconditionally from a clamped address; what must not count - a token past the
     // block's end, a dropped pair - is masked when it is added: loads under a condition are waited for one by one)
     auto gather = [&](Raw (&v)[U], uint32_t (&ok)[U], int ib, int j) __attribute__((always_inline)) {
@@ -251,16 +251,10 @@ __global__ __launch_bounds__(256) void dispatch_bwd_gate_kernel(const T *__restr
     auto add = [&](float (&acc)[U][4], const Raw (&v)[U], const uint32_t (&ok)[U]) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if constexpr (sizeof(T) == 2) {
-                const uint32_t x = v[u].x & ok[u], y = v[u].y & ok[u];
-                acc[u][0] += __uint_as_float(x << 16); acc[u][1] += __uint_as_float(x & 0xffff0000u);
-                acc[u][2] += __uint_as_float(y << 16); acc[u][3] += __uint_as_float(y & 0xffff0000u);
-            } else {
-                acc[u][0] += __uint_as_float(__float_as_uint(v[u].x) & ok[u]);
-                acc[u][1] += __uint_as_float(__float_as_uint(v[u].y) & ok[u]);
-                acc[u][2] += __uint_as_float(__float_as_uint(v[u].z) & ok[u]);
-                acc[u][3] += __uint_as_float(__float_as_uint(v[u].w) & ok[u]);
-            }
+            acc[u][0] += __uint_as_float(__float_as_uint(v[u].x) & ok[u]);
+            acc[u][1] += __uint_as_float(__float_as_uint(v[u].y) & ok[u]);
+            acc[u][2] += __uint_as_float(__float_as_uint(v[u].z) & ok[u]);
+            acc[u][3] += __uint_as_float(__float_as_uint(v[u].w) & ok[u]);
         }
     };
     auto finish = [&](const Raw (&first)[U], const uint32_t (&first_ok)[U], int ib) __attribute__((always_inline)) {
@@ -285,15 +279,7 @@ __global__ __launch_bounds__(256) void dispatch_bwd_gate_kernel(const T *__restr
 #pragma unroll
                 for (int q = 0; q < 4; ++q) acc[u][q] += d * w[e][q];
             }
-            if constexpr (sizeof(T) == 2) {
-                const bf16_t b0 = (bf16_t)acc[u][0], b1 = (bf16_t)acc[u][1], b2 = (bf16_t)acc[u][2], b3 = (bf16_t)acc[u][3];
-                uint2 o;
-                o.x = (uint32_t)__builtin_bit_cast(uint16_t, b0) | ((uint32_t)__builtin_bit_cast(uint16_t, b1) << 16);
-                o.y = (uint32_t)__builtin_bit_cast(uint16_t, b2) | ((uint32_t)__builtin_bit_cast(uint16_t, b3) << 16);
-                *reinterpret_cast<uint2 *>(dx + (size_t)i * M + m) = o;
-            } else {
-                *reinterpret_cast<float4 *>(dx + (size_t)i * M + m) = make_float4(acc[u][0], acc[u][1], acc[u][2], acc[u][3]);
-            }
+            *reinterpret_cast<float4 *>(dx + (size_t)i * M + m) = make_float4(acc[u][0], acc[u][1], acc[u][2], acc[u][3]);
         }
     };
     Raw va[U], vb[U];
@@ -318,11 +304,18 @@ __global__ __launch_bounds__(256) void dispatch_bwd_gate_kernel(const T *__restr
 // source rows, adds and stores 16 bytes.  The first-choice gathers and the gradients of a group of tokens are issued one
 // group ahead (two groups ahead: 14.7 against 14.3 us; all four groups' up front: 16.1, the weights' loads queue behind them).
 constexpr int DM_TOKENS = 64;                 // tokens per block: four groups of 16 (32: +5 %, 16: +20 % at 16384 x 1024)
+// Blocks of 16 tokens where 64 leave CUs without one, and a choice's gathers of four tokens in flight together: 2048 x 512,
+// 16 experts, top-2: 15.0 -> 5.1 us; 513 x 520, top-4 (on the fp32 kernel above before): 12.4 -> 8.4.
+constexpr int DM_TOKENS_FEW = 16, DM_FEW_BLOCKS = 192;
 constexpr int DM_COLS = 128;                  // columns per wave
 constexpr int DM_ROW = DM_COLS + 4;           // floats per token row of the LDS buffer: 4 rows apart = 16 banks apart
 typedef __bf16 perm_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float perm_f32x4 __attribute__((ext_vector_type(4)));
-template <bool E8>   // E8: E is a multiple of 8, a lane's 8 gradients are two 16-byte loads
+// E8: E is a multiple of 8, a lane's 8 gradients are two 16-byte loads.  TOK: tokens per block.  M is a multiple of 8: the
+// last wave's columns past it read the row's last ones and are not stored.  SPLIT: gradients and weights enter as the sum of
+// three bf16 numbers each (24 bits; six products, what is left out is below 2^-23 of a term), which keeps the gate's part at
+// fp32 accuracy before it is rounded to bf16: widths that are not whole 128-column pieces take it.
+template <bool E8, int TOK, bool SPLIT>
 __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_t *__restrict__ dxd,
                                                                      const int32_t *__restrict__ row, int S, int M, int k,
                                                                      const float *__restrict__ dlogits,
@@ -332,29 +325,31 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, kq = lane >> 4;
     const int col0 = (blockIdx.y * 8 + wave) * DM_COLS;      // this wave's first column
-    if (col0 >= M) return;                                   // M is a multiple of 128: whole waves drop out
+    if (col0 >= M) return;                                   // (no barrier below)
     float *buf = s_t[wave];
     const int tsel = lane >> 4, c8 = (lane & 15) * 8;        // row-major side: token within a quartet, first of 8 columns
+    const bool col_ok = col0 + c8 < M;
+    const int at = min(col0 + c8, M - 8);
     // the first-choice source rows of the 4 tokens this lane finishes in a group (tokens tok0 + 4 u + tsel)
     // (loads are unconditional, from clamped addresses, and what must not count is masked where it is used: a
     // load under a condition would make the compiler wait for all loads in flight at every such place)
-    // (the first-choice rows of the block's 64 tokens come with one load, lane l holding token l's, and are handed
+    // (the first-choice rows of the block's tokens come with one load, lane l holding token l's, and are handed
     // round between lanes: the gathers' addresses then wait for no load of their own)
-    static_assert(DM_TOKENS == WAVE, "one first-choice row per lane");
-    const int my_row = row[min((int)blockIdx.x * DM_TOKENS + lane, S - 1)];
+    static_assert(TOK <= WAVE, "one first-choice row per lane");
+    const int my_row = row[min((int)blockIdx.x * TOK + lane, S - 1)];
     auto gather = [&](uint4 (&v)[4], uint32_t (&ok)[4], int tok0) __attribute__((always_inline)) {
         int r[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) r[u] = __shfl(my_row, (tok0 - (int)blockIdx.x * DM_TOKENS + 4 * u + tsel) & (WAVE - 1), WAVE);
+        for (int u = 0; u < 4; ++u) r[u] = __shfl(my_row, (tok0 - (int)blockIdx.x * TOK + 4 * u + tsel) & (WAVE - 1), WAVE);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             ok[u] = (tok0 + 4 * u + tsel < S && r[u] >= 0) ? 0xffffffffu : 0u;
-            v[u] = *reinterpret_cast<const uint4 *>(dxd + (size_t)(r[u] & (int)ok[u]) * M + col0 + c8);
+            v[u] = *reinterpret_cast<const uint4 *>(dxd + (size_t)(r[u] & (int)ok[u]) * M + at);
         }
     };
     uint4 src[4];
     uint32_t src_ok[4];
-    gather(src, src_ok, blockIdx.x * DM_TOKENS);
+    gather(src, src_ok, blockIdx.x * TOK);
     // A fragment of a group of 16 tokens: dlogits[tok0 + r16][8 kq .. 8 kq + 7], fetched one group ahead like the rows
     // (fetched where it is used, the product waited for it in every group: 15.0 -> 14.2 us at 16384 x 1024)
     auto load_d = [&](float (&d)[8], int tok0) __attribute__((always_inline)) {
@@ -369,12 +364,19 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
         }
     };
     float d[8];
-    load_d(d, blockIdx.x * DM_TOKENS);
+    load_d(d, blockIdx.x * TOK);
     // B fragments: Wg[8 kq + i][col0 + 16 cb + r16], i = 0..7, for the wave's 8 column blocks.  Fetched row by row
     // with 16-byte loads (a lane takes 4 columns of the 8 experts of one group) and turned by way of the LDS
     // buffer, [expert group][column] with a group's 8 experts as one bf16x8 entry: picking them out of global
     // memory one float at a time took longer than the rest of the kernel.  Two expert groups per pass.
-    perm_bf16x8 bfrag[8];
+    constexpr int P = SPLIT ? 3 : 1;
+    perm_bf16x8 bfrag[P][8];
+    // the value rounded to bf16, of which the remainder stays behind for the next part
+    auto part_of = [](float &v) __attribute__((always_inline)) {
+        const bf16_t b = (bf16_t)v;
+        v -= (float)b;
+        return b;
+    };
     {
         perm_bf16x8 *wt = reinterpret_cast<perm_bf16x8 *>(buf);      // [2][DM_COLS]
         const int c4 = (lane & 31) * 4, half = lane >> 5;
@@ -384,83 +386,114 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
             const int eg = 2 * pass + half;
             float4 w[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) w[i] = *reinterpret_cast<const float4 *>(wg + (size_t)min(8 * eg + i, E - 1) * M + col0 + c4);
+            for (int i = 0; i < 8; ++i) w[i] = *reinterpret_cast<const float4 *>(wg + (size_t)min(8 * eg + i, E - 1) * M + min(col0 + c4, M - 4));
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 if (8 * eg + i >= E) w[i] = make_float4(0.f, 0.f, 0.f, 0.f);
             perm_bf16x8 *dst = wt + half * DM_COLS + c4;
-            dst[0] = perm_bf16x8{(bf16_t)w[0].x, (bf16_t)w[1].x, (bf16_t)w[2].x, (bf16_t)w[3].x,
-                                 (bf16_t)w[4].x, (bf16_t)w[5].x, (bf16_t)w[6].x, (bf16_t)w[7].x};
-            dst[1] = perm_bf16x8{(bf16_t)w[0].y, (bf16_t)w[1].y, (bf16_t)w[2].y, (bf16_t)w[3].y,
-                                 (bf16_t)w[4].y, (bf16_t)w[5].y, (bf16_t)w[6].y, (bf16_t)w[7].y};
-            dst[2] = perm_bf16x8{(bf16_t)w[0].z, (bf16_t)w[1].z, (bf16_t)w[2].z, (bf16_t)w[3].z,
-                                 (bf16_t)w[4].z, (bf16_t)w[5].z, (bf16_t)w[6].z, (bf16_t)w[7].z};
-            dst[3] = perm_bf16x8{(bf16_t)w[0].w, (bf16_t)w[1].w, (bf16_t)w[2].w, (bf16_t)w[3].w,
-                                 (bf16_t)w[4].w, (bf16_t)w[5].w, (bf16_t)w[6].w, (bf16_t)w[7].w};
-            // the lanes whose expert group (kq) this pass staged pick up their fragments
-            if ((kq >> 1) == pass) {
 #pragma unroll
-                for (int cb = 0; cb < 8; ++cb) bfrag[cb] = wt[(kq & 1) * DM_COLS + 16 * cb + r16];
+            for (int p = 0; p < P; ++p) {
+                perm_bf16x8 t[4];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    t[0][i] = part_of(w[i].x); t[1][i] = part_of(w[i].y);
+                    t[2][i] = part_of(w[i].z); t[3][i] = part_of(w[i].w);
+                }
+#pragma unroll
+                for (int c = 0; c < 4; ++c) dst[c] = t[c];
+                // the lanes whose expert group (kq) this pass staged pick up their fragments
+                if ((kq >> 1) == pass) {
+#pragma unroll
+                    for (int cb = 0; cb < 8; ++cb) bfrag[p][cb] = wt[(kq & 1) * DM_COLS + 16 * cb + r16];
+                }
             }
         }
         if (8 * kq >= E) {        // expert groups past the gate's size contribute nothing
             const bf16_t z = (bf16_t)0.0f;
 #pragma unroll
-            for (int cb = 0; cb < 8; ++cb) bfrag[cb] = perm_bf16x8{z, z, z, z, z, z, z, z};
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (int cb = 0; cb < 8; ++cb) bfrag[p][cb] = perm_bf16x8{z, z, z, z, z, z, z, z};
         }
     }
 #pragma unroll
-    for (int g0 = 0; g0 < DM_TOKENS; g0 += 16) {
-        const int tok0 = blockIdx.x * DM_TOKENS + g0;
+    for (int g0 = 0; g0 < TOK; g0 += 16) {
+        const int tok0 = blockIdx.x * TOK + g0;
+        if (tok0 >= S) return;
         uint4 nxt[4];
         uint32_t nxt_ok[4];
         float d_nxt[8];
-        if (g0 + 16 < DM_TOKENS) {
+        if (g0 + 16 < TOK) {
             gather(nxt, nxt_ok, tok0 + 16);
             load_d(d_nxt, tok0 + 16);
         }
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             if (tok0 + r16 >= S || 8 * kq + i >= E) d[i] = 0.f;
-        const perm_bf16x8 afrag = {(bf16_t)d[0], (bf16_t)d[1], (bf16_t)d[2], (bf16_t)d[3],
-                                   (bf16_t)d[4], (bf16_t)d[5], (bf16_t)d[6], (bf16_t)d[7]};
+        perm_bf16x8 afrag[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) afrag[p][i] = part_of(d[i]);
         // product tiles into LDS.  The gate's weights go into the first operand slot, so the four results of a lane
         // are four consecutive columns of one token (acc[r] = column 16 cb + 4 kq + r of token r16) and leave with
         // one 16-byte LDS write (a quarter wave's 16 rows are 16 banks-of-four apart: see DM_ROW)
 #pragma unroll
         for (int cb = 0; cb < 8; ++cb) {
-            const perm_f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfrag[cb], afrag, perm_f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            perm_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int order = P - 1; order >= 0; --order)       // the smallest products first
+#pragma unroll
+                for (int p = 0; p <= order; ++p)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfrag[p][cb], afrag[order - p], acc, 0, 0, 0);
             *reinterpret_cast<perm_f32x4 *>(buf + r16 * DM_ROW + 16 * cb + 4 * kq) = acc;
         }
         // (a wave's LDS buffer is written and read by that wave only: program order is enough)
+        float acc[4][8];
+        Vec<bf16_t> v;
+        float f[8];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const int tl = 4 * u + tsel, t = tok0 + tl;
+            const int tl = 4 * u + tsel;
             const float4 p0 = *reinterpret_cast<const float4 *>(buf + tl * DM_ROW + c8);
             const float4 p1 = *reinterpret_cast<const float4 *>(buf + tl * DM_ROW + c8 + 4);
-            float acc[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-            Vec<bf16_t> v;
-            float f[8];
+            acc[u][0] = p0.x; acc[u][1] = p0.y; acc[u][2] = p0.z; acc[u][3] = p0.w;
+            acc[u][4] = p1.x; acc[u][5] = p1.y; acc[u][6] = p1.z; acc[u][7] = p1.w;
             v.raw = src[u];
             v.mask(src_ok[u]);
             v.unpack(f);
 #pragma unroll
-            for (int q = 0; q < 8; ++q) acc[q] += f[q];
-            for (int j = 1; j < k; ++j) {
-                const int r = row[(size_t)j * S + min(t, S - 1)];
-                const uint32_t ok = (t < S && r >= 0) ? 0xffffffffu : 0u;
-                v.load(dxd + (size_t)(r & (int)ok) * M + col0 + c8);
-                v.mask(ok);
+            for (int q = 0; q < 8; ++q) acc[u][q] += f[q];
+        }
+        for (int j = 1; j < k; ++j) {          // a choice's four gathers are in flight together
+            uint4 more[4];
+            uint32_t ok[4];
+            int r[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) r[u] = row[(size_t)j * S + min(tok0 + 4 * u + tsel, S - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                ok[u] = (tok0 + 4 * u + tsel < S && r[u] >= 0) ? 0xffffffffu : 0u;
+                more[u] = *reinterpret_cast<const uint4 *>(dxd + (size_t)(r[u] & (int)ok[u]) * M + at);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                v.raw = more[u];
+                v.mask(ok[u]);
                 v.unpack(f);
 #pragma unroll
-                for (int q = 0; q < 8; ++q) acc[q] += f[q];
-            }
-            if (t < S) {
-                v.pack(acc);
-                v.store(dx + (size_t)t * M + col0 + c8);
+                for (int q = 0; q < 8; ++q) acc[u][q] += f[q];
             }
         }
-        if (g0 + 16 < DM_TOKENS) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int t = tok0 + 4 * u + tsel;
+            if (t < S && col_ok) {
+                v.pack(acc[u]);
+                v.store(dx + (size_t)t * M + at);
+            }
+        }
+        if (g0 + 16 < TOK) {
 #pragma unroll
             for (int u = 0; u < 4; ++u) { src[u] = nxt[u]; src_ok[u] = nxt_ok[u]; }
 #pragma unroll
@@ -1039,14 +1072,18 @@ extern "C" int mole_dispatch_bwd(const void *dxd, int dtype, const int32_t *row,
     MOLE_REQUIRE(dlogits == nullptr || (wg != nullptr && E >= 1 && aligned16(wg) && M % 4 == 0),
                  "mole_dispatch_bwd: dlogits given without a valid wg/E");
     MOLE_REQUIRE(dx_add == nullptr || aligned16(dx_add), "mole_dispatch_bwd: misaligned dx_add");
-    if (dlogits != nullptr && dx_add == nullptr && E <= 32 && M % DM_COLS == 0 && dtype == MOLE_BF16) {
-        const dim3 grid(ceil_div(S, DM_TOKENS), ceil_div(M, 8 * DM_COLS));
-        if (E % 8 == 0 && ((uintptr_t)dlogits & 15) == 0)
-            timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_mfma_kernel<true>, grid, dim3(512), 0, (hipStream_t)stream,
-                         (const bf16_t *)dxd, row, S, M, k, dlogits, wg, E, (bf16_t *)dx);
-        else
-            timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_mfma_kernel<false>, grid, dim3(512), 0, (hipStream_t)stream,
-                         (const bf16_t *)dxd, row, S, M, k, dlogits, wg, E, (bf16_t *)dx);
+    if (dlogits != nullptr && dx_add == nullptr && E <= 32 && dtype == MOLE_BF16) {
+        const int tok = (long)ceil_div(S, DM_TOKENS) * ceil_div(M, 8 * DM_COLS) < DM_FEW_BLOCKS ? DM_TOKENS_FEW : DM_TOKENS;
+        const dim3 grid(ceil_div(S, tok), ceil_div(M, 8 * DM_COLS));
+        const bool e8 = E % 8 == 0 && ((uintptr_t)dlogits & 15) == 0;
+        const bool split = M % DM_COLS != 0;
+#define MOLE_DM_(E8, TOK, SPLIT) timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_mfma_kernel<E8, TOK, SPLIT>, grid, dim3(512), 0, (hipStream_t)stream, \
+                                              (const bf16_t *)dxd, row, S, M, k, dlogits, wg, E, (bf16_t *)dx)
+#define MOLE_DM(E8, TOK) if (split) MOLE_DM_(E8, TOK, true); else MOLE_DM_(E8, TOK, false)
+        if (tok == DM_TOKENS) { if (e8) { MOLE_DM(true, DM_TOKENS); } else { MOLE_DM(false, DM_TOKENS); } }
+        else { if (e8) { MOLE_DM(true, DM_TOKENS_FEW); } else { MOLE_DM(false, DM_TOKENS_FEW); } }
+#undef MOLE_DM
+#undef MOLE_DM_
         MOLE_LAUNCH_CHECK();
         return 0;
     }
@@ -1054,12 +1091,8 @@ extern "C" int mole_dispatch_bwd(const void *dxd, int dtype, const int32_t *row,
         const int db_tokens = (long)ceil_div(S, DB_TOKENS) * ceil_div(M, 1024) < 1024 ? DB_TOKENS_FEW : DB_TOKENS;
         const dim3 grid(ceil_div(S, db_tokens), ceil_div(M, 1024));
         hipStream_t st = (hipStream_t)stream;
-#define MOLE_DB(T, EB) timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_kernel<T, EB>, grid, dim3(256), 0, st, (const T *)dxd, row, S, M, k, dlogits, wg, E, (T *)dx, db_tokens)
-        if (dtype == MOLE_BF16) {
-            if (E <= 8) MOLE_DB(bf16_t, 8); else if (E <= 16) MOLE_DB(bf16_t, 16); else MOLE_DB(bf16_t, 32);
-        } else {
-            if (E <= 8) MOLE_DB(float, 8); else if (E <= 16) MOLE_DB(float, 16); else MOLE_DB(float, 32);
-        }
+#define MOLE_DB(EB) timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_kernel<EB>, grid, dim3(256), 0, st, (const float *)dxd, row, S, M, k, dlogits, wg, E, (float *)dx, db_tokens)
+        if (E <= 8) MOLE_DB(8); else if (E <= 16) MOLE_DB(16); else MOLE_DB(32);
 #undef MOLE_DB
         MOLE_LAUNCH_CHECK();
         return 0;

@@ -166,3 +166,29 @@ def test_combine_bwd_with_the_gate_backward_in_its_tail(S, M, E, k, cf, normaliz
     want_s = H.gate_bwd(dgates, scores, r.idx, normalize, False, **kw)
     _, got_s = H.combine_bwd_gate(dy, o, r.row, r.gates, scores, r.idx, normalize, False, **kw)
     assert rel_err(got_s, want_s) < 1e-5
+
+
+# bf16 widths that end inside a wave's 128 columns (the gate product there in three bf16 parts per operand), few tokens (16 per
+# block) and many (64), tokens past the last group, gates of whole and ragged groups of eight.  With no rows to gather dx is
+# the gate product alone: bf16 rounding of the result plus what the split leaves out, below 2^-23 of every term, with fp32 sums
+# of six products of at most 32 terms.
+@pytest.mark.parametrize("S,E,k,M", [(1, 8, 1, 8), (17, 3, 3, 72), (63, 32, 8, 136), (513, 16, 4, 520), (2000, 9, 1, 1032), (12500, 24, 2, 72), (7000, 32, 2, 2888)])
+def test_dispatch_bwd_with_gate_bf16_ragged_widths(S, E, k, M):
+    from mole_amd import hip_ops as H
+    print(f"dispatch_bwd+gate ragged S={S} E={E} k={k} M={M}", flush=True)
+    g = torch.Generator().manual_seed(S + M)
+    dlog, wg = torch.randn(S, E, generator=g), torch.randn(E, M, generator=g)
+    row = torch.full((k, S), -1, dtype=torch.int32)
+    dxd = torch.randn(S * k, M, generator=g).bfloat16()
+    got = H.dispatch_bwd(dxd.cuda(), row.cuda(), dlog.cuda(), wg.cuda()).double().cpu()
+    want, terms = dlog.double() @ wg.double(), dlog.double().abs() @ wg.double().abs()
+    left_out = 2.0 ** -23 + 6 * 32 * 2.0 ** -24 if M % 128 else 2.0 ** -7       # (whole pieces: operands rounded to bf16)
+    assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + left_out * terms).all())
+    # and with rows: every token's k source rows on top, some dropped
+    row = torch.randperm(S * k, generator=g).view(k, S).int()
+    row[:, ::5] = -1
+    got = H.dispatch_bwd(dxd.cuda(), row.cuda(), dlog.cuda(), wg.cuda()).double().cpu()
+    for j in range(k):
+        src = torch.where(row[j] >= 0, row[j], 0).long()
+        want = want + dxd[src].double() * (row[j] >= 0).double()[:, None]
+    assert rel_err(got, want) < tol(torch.bfloat16)
