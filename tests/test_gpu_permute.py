@@ -192,3 +192,17 @@ def test_dispatch_bwd_with_gate_bf16_ragged_widths(S, E, k, M):
         src = torch.where(row[j] >= 0, row[j], 0).long()
         want = want + dxd[src].double() * (row[j] >= 0).double()[:, None]
     assert rel_err(got, want) < tol(torch.bfloat16)
+
+
+# The gate's weight gradient where its blocks take 16 tokens (few of them) and 64, around the batch of eight.  fp32 sums of up
+# to 12300 terms (2^-24 sqrt(12300) = 7e-6 at worst); the matrix cores' variant splits dlogits in two parts (2^-17 = 8e-6).
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("S,E,M", [(1, 3, 72), (15, 8, 520), (17, 16, 8), (513, 32, 520), (12300, 8, 72), (6200, 9, 1032)])
+def test_gate_wgrad_short_blocks(S, E, M, dtype):
+    from mole_amd import hip_ops as H
+    print(f"gate_wgrad S={S} E={E} M={M} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(S + M)
+    dl, x = torch.randn(S, E, generator=g), torch.randn(S, M, generator=g).to(dtype)
+    want = dl.double().t() @ x.double()
+    got = H.gate_wgrad(dl.cuda(), x.cuda()).double().cpu()
+    assert float((got - want).norm() / want.norm()) < 2e-5
