@@ -569,7 +569,9 @@ static RouteEnd route_end(int S, int E, int k, double capacity_factor, int align
     const int cf_sign = capacity_factor > 0. ? 1 : (capacity_factor < 0. ? -1 : 0);
     // int(cf * spe) of the Python reference: the product is taken in double precision
     const double prod = (capacity_factor < 0. ? -capacity_factor : capacity_factor) * (double)spe;
-    return RouteEnd{S, E, k, cf_sign, k * (int)prod, alignment, layout, counts, kept_rows, offsets, capacity, l_aux, idx, loc, row};
+    // (held to what leaves room for the alignment in 32 bits: a factor that overflowed them made the capacity negative)
+    const int limit = (INT_MAX - alignment) / k;
+    return RouteEnd{S, E, k, cf_sign, k * (prod < (double)limit ? (int)prod : limit), alignment, layout, counts, kept_rows, offsets, capacity, l_aux, idx, loc, row};
 }
 
 template <int VPL, int LOGG>

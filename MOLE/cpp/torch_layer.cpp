@@ -8,7 +8,9 @@
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <atomic>
+#include <limits>
 
 #include "mole_hip.h"
 
@@ -57,8 +59,11 @@ struct Plan {
         const int64_t es = dtype_code == MOLE_BF16 ? 2 : 4;
         int64_t rows = S * k;
         if (cf > 0) {
-            // the reference's integer: k * int(cf * ceil(S / E)), the product in double precision
-            const int64_t cap = k * (int64_t)(cf * (double)((S + E - 1) / E));
+            // the reference's integer: k * int(cf * ceil(S / E)), the product in double precision.  A factor whose product
+            // no int64 holds would come out of the conversion negative, and the buffers a row long: 2^31 per choice is
+            // more than the S k rows there are (and more than the padded layout takes)
+            TORCH_CHECK(cf <= std::numeric_limits<double>::max(), "the capacity factor must be finite");
+            const int64_t cap = k * (int64_t)std::min(cf * (double)((S + E - 1) / E), 2147483648.0);
             rows = layout == MOLE_LAYOUT_PADDED ? E * cap : std::min(rows, E * cap);
         }
         rows = std::max<int64_t>(rows, 1);
@@ -203,6 +208,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     py::class_<Plan, std::shared_ptr<Plan>>(m, "Plan")
         .def(py::init<int, int64_t, int64_t, int64_t, int64_t, int64_t, double, int, bool, int>())
         .def("route_offsets", &Plan::route_offsets)
+        .def_property_readonly("rows", [](const Plan &p) { return p.head.rows; })
         .def(py::pickle([](const Plan &p) { return py::make_tuple(p.head.dtype, p.head.S, p.head.M, p.head.E, p.head.k, p.head.F,
                                                                   p.head.capacity_factor, p.head.layout, p.head.normalize_gate, p.gelu_bwd); },
                         [](py::tuple t) { return std::make_shared<Plan>(t[0].cast<int>(), t[1].cast<int64_t>(), t[2].cast<int64_t>(),

@@ -235,7 +235,7 @@ class MOLEModule(torch.nn.Module):
         """The LayerPlan of a forward pass over S tokens, or None when it takes the step-by-step path (experts offloaded, no
         tokens, a gate in another dtype, a padded capacity that only the device knows; a profiled pass also does)."""
         if (self.d_experts or not self.s_experts or S < 1 or wg.dtype != torch.float32 or not wg.is_contiguous()
-                or self.embed_dim % self._granule or self.ffn_dim % self._granule or (self.reference_layout and capacity_factor <= 0)):
+                or self.embed_dim % self._granule or self.ffn_dim % self._granule or (self.reference_layout and not capacity_factor > 0)):
             return None
         key = (S, capacity_factor, self.topk, self.normalize_gate, self.reference_layout)
         plan = self._plans.get(key)

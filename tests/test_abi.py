@@ -149,3 +149,16 @@ def test_every_entry_point_rejects_bad_arguments_on_the_host():
         assert rc < 0, f"{name}: expected a library error code, got {rc}"
         msg = L.last_error()
         assert name in msg, f"{name}: message does not name the entry point: {msg!r}"
+
+
+@pytest.mark.parametrize("cf", [0.0, -0.5, 0.25, 1.25, 1e9, 1e19, 1e300])
+def test_layer_plan_rows_hold_every_kept_pair(cf):
+    """64 tokens, top-2 of 4 experts: min(S k, E k int(cf ceil(S / E))) rows, also where no integer holds the product."""
+    from mole_amd import _lib as L
+    from mole_amd import hip_ops as H
+    import torch
+    plan = lambda f: H.LayerPlan(torch.bfloat16, 64, 128, 4, 2, 256, f, L.LAYOUT_RAGGED, True, 0)
+    want = 128 if cf <= 0 else min(128, 4 * 2 * int(cf * 16))
+    assert plan(cf).native.rows == want
+    with pytest.raises(RuntimeError, match="finite"):
+        plan(float("inf"))
