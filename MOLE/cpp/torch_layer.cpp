@@ -189,7 +189,8 @@ std::tuple<Tensor, std::optional<Tensor>, Tensor> layer(const Tensor &x, const T
     c->weights = std::move(weights);
     c->grads = std::move(grads);
     c->accumulate = accumulate;
-    if (!at::GradMode::is_enabled()) {
+    // (no_grad leaves forward-mode derivatives on: an input that carries a tangent goes through the node, which refuses it)
+    if (!at::GradMode::is_enabled() && !x._fw_grad(0).defined() && !wg._fw_grad(0).defined()) {
         auto ya = run_forward(*c, x, wg, Tensor());
         return {ya.first, std::nullopt, c->route};
     }

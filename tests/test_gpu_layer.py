@@ -561,3 +561,12 @@ def test_layer_one_call_gate_paths(S, M, E, k, Fd, cf, padded, dtype):
     with torch.no_grad():
         y = m(x, capacity_factor=cf)
     assert torch.equal(y, res.extras["y_gpu"]) and abs(float(m.l_aux) - res.crit.l_aux) < 1e-4 * max(1.0, res.crit.l_aux)
+
+
+def test_layer_refuses_forward_mode_tangents():
+    """The layer has no forward-mode derivative: a tangent is an error under no_grad too, not silently dropped."""
+    import torch.autograd.forward_ad as fwAD
+    m, x, _ = _build(16, 64, 4, 2, 128, torch.float32)
+    for grad in (True, False):
+        with torch.set_grad_enabled(grad), fwAD.dual_level(), pytest.raises(RuntimeError, match="jvp|forward"):
+            m(fwAD.make_dual(x, torch.ones_like(x)), capacity_factor=0.0)
