@@ -86,6 +86,8 @@ struct Call : torch::CustomClassHolder {
     std::optional<Tensor> bias;
     std::vector<Tensor> weights, grads;      // w1, b1, w2, b2 of all experts and their gradient buffers
     bool accumulate = false;
+    std::vector<int64_t> dummy_sizes;        // the marker parameter: its gradient is a tensor of zeros, never left out
+    at::TensorOptions dummy_options;
     Tensor route;                            // forward's result for the caller
 };
 
@@ -140,7 +142,8 @@ std::pair<Tensor, Tensor> run_forward(Call &c, const Tensor &x, const Tensor &wg
 struct LayerFn : torch::autograd::Function<LayerFn> {
     // dummy: an empty parameter that makes autograd record the node although x need not require a gradient
     static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &wg, const Tensor &dummy, c10::intrusive_ptr<Call> c) {
-        (void)dummy;
+        c->dummy_sizes = dummy.sizes().vec();
+        c->dummy_options = dummy.options();
         ctx->set_materialize_grads(false);
         Tensor l_aux = at::empty({}, x.options().dtype(at::kFloat));
         auto [y, act] = run_forward(*c, x, wg, l_aux);
@@ -173,7 +176,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         G.dwg = dwg.data_ptr<float>();
         check(mole_layer_bwd(&L, &G, current_stream(x)), "mole_layer_bwd");
         c->counter->value += 1;
-        return {dx, dwg, Tensor(), Tensor()};
+        return {dx, dwg, at::zeros(c->dummy_sizes, c->dummy_options), Tensor()};
     }
 };
 

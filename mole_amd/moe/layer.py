@@ -237,7 +237,7 @@ class MOLEModule(torch.nn.Module):
         if (self.d_experts or not self.s_experts or S < 1 or wg.dtype != torch.float32 or not wg.is_contiguous()
                 or self.embed_dim % self._granule or self.ffn_dim % self._granule or (self.reference_layout and not capacity_factor > 0)):
             return None
-        key = (S, capacity_factor, self.topk, self.normalize_gate, self.reference_layout)
+        key = (S, capacity_factor, self.topk, self.normalize_gate, self.reference_layout, self.MOLECore.gelu_bwd)
         plan = self._plans.get(key)
         if plan is None:
             if len(self._plans) >= 64:

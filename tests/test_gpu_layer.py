@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+from mole_amd import _lib as L
 from oracle import moe_oracle as O
 from tests.util import expert_rel_err, rel_err, row_rel_err, tol
 
@@ -570,3 +571,18 @@ def test_layer_refuses_forward_mode_tangents():
     for grad in (True, False):
         with torch.set_grad_enabled(grad), fwAD.dual_level(), pytest.raises(RuntimeError, match="jvp|forward"):
             m(fwAD.make_dual(x, torch.ones_like(x)), capacity_factor=0.0)
+
+
+@pytest.mark.parametrize("padded", [False, True])
+def test_layer_marker_parameter_and_changed_gelu_derivative(padded):
+    """The empty parameter that makes autograd record the layer gets its (empty) gradient, as every parameter does; the
+    GELU derivative is the one set when the pass runs, for a shape that has been seen with the other one too."""
+    m, x, _ = _build(33, 64, 4, 2, 128, torch.float32, reference_layout=padded)
+    other = next(v for v in (L.GELU_BWD_TANH, L.GELU_BWD_EXACT) if v != m.MOLECore.gelu_bwd)
+    grads = []
+    for mode in (m.MOLECore.gelu_bwd, other):
+        m.MOLECore.gelu_bwd = mode
+        m(x, capacity_factor=2.0).sum().backward()
+        grads.append(m.FC1_W_GPU.grad_tensors.clone())
+        assert m.dummy_param.grad is not None and m.dummy_param.grad.shape == m.dummy_param.shape
+    assert not torch.equal(grads[0], grads[1])
