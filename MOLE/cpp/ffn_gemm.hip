@@ -329,7 +329,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kernel(const GemmArgs g) {
                     ((T *)Cb)[off] = from_f32<T>(v + bias);
                 } else if constexpr (EPI == EPI_BIAS_GELU) {
                     v += bias;
-                    ((T *)Cb)[off] = from_f32<T>(v);
+                    if (Cb != nullptr) ((T *)Cb)[off] = from_f32<T>(v);
                     ((T *)g.C2)[off] = from_f32<T>(gelu_erf(v));
                 } else if constexpr (EPI == EPI_DGELU) {
                     const float hv = hv16[i];
@@ -487,7 +487,9 @@ static int ffn_fwd_t(const void *xd, const int32_t *offsets, const int32_t *kept
     g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles; g.est_rows = est_rows;
     // h = xd . w1^T + b1, a = gelu(h)
     g.A = xd; g.lda = M; g.B = w1; g.ldb = M; g.strideB = (long)F * M; g.N = F; g.K = M;
-    g.C = h; g.C2 = a; g.ldc = F; g.bias = b1;
+    // (h is for the backward pass alone: a store of R F elements and a turn through LDS less where none follows; 6002 rows,
+    // 16 experts, 1024 -> 4096: the pass 188.4 -> 183.0 us, and 49 MB less memory)
+    g.C = forward_only ? nullptr : h; g.C2 = a; g.ldc = F; g.bias = b1;
     if (int rc = run_gemm<T, false, false, false, EPI_BIAS_GELU>(g, max_rows, m_tiles * ceil_div(F, TBN), st, MOLE_K_FFN_FWD1)) return rc;
     // out = a . w2 + b2   (w2 [F,M]: K-strided)
     g.A = a; g.lda = F; g.B = w2; g.ldb = M; g.strideB = (long)F * M; g.N = M; g.K = F;
@@ -574,7 +576,7 @@ int ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *ke
             size_t workspace_bytes, int forward_only, hipStream_t st) {
     if (int rc = check_ffn("mole_ffn_fwd", dtype, E, max_rows, M, F)) return rc;
     if (max_rows == 0) return 0;
-    MOLE_REQUIRE(xd && offsets && kept_rows && w1 && b1 && w2 && b2 && h && a && out, "mole_ffn_fwd: null pointer");
+    MOLE_REQUIRE(xd && offsets && kept_rows && w1 && b1 && w2 && b2 && (h || forward_only) && a && out, "mole_ffn_fwd: null pointer");
     MOLE_REQUIRE(al16(xd) && al16(w1) && al16(w2) && al16(h) && al16(a) && al16(out) && al16(workspace),
                  "mole_ffn_fwd: buffers must be 16-byte aligned");
     if (dtype == MOLE_BF16)

@@ -125,7 +125,7 @@ enum { EPI_STORE = 0, EPI_BIAS = 1, EPI_BIAS_GELU = 2, EPI_DGELU = 3, EPI_WGRAD 
 
 struct GemmArgs {
     const void *A, *B;      // operands (see A_KS / B_KS for their layout)
-    void *C, *C2;           // outputs; C2 = gelu(h) for EPI_BIAS_GELU
+    void *C, *C2;           // outputs; C2 = gelu(h) for EPI_BIAS_GELU, whose C may be null (h is then not stored)
     const void *bias;       // [E][N] for EPI_BIAS*, else unused
     const void *H;          // [rows][N] pre-activation for EPI_DGELU
     const int32_t *offsets; // [E] first row of every expert (NULL: one group starting at row 0)

@@ -572,10 +572,14 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<T
 
     DGeluCoef dgelu;
     if constexpr (EPI == EPI_DGELU) dgelu.select(g.gelu_bwd == MOLE_GELU_BWD_TANH);
-    // pass 0 writes C; for EPI_BIAS_GELU pass 1 writes C2 = gelu(h)
+    // pass 0 writes C; for EPI_BIAS_GELU pass 1 writes C2 = gelu(h), and without a C (no backward pass will ask for h)
+    // there is no pass 0
     constexpr int PASSES = EPI == EPI_BIAS_GELU ? 2 : 1;
 #pragma unroll
     for (int pass = 0; pass < PASSES; ++pass) {
+        if constexpr (EPI == EPI_BIAS_GELU) {
+            if (pass == 0 && g.C == nullptr) continue;
+        }
 #pragma unroll
         for (int tn = 0; tn < 2; ++tn) {
 #pragma unroll

@@ -373,6 +373,7 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
     const long ldc = EPI == EPI_PART ? (long)g.N : g.ldc;
     long crow0 = EPI == EPI_PART ? split_k * g.part_rows + row0 : row0;
     if constexpr (WG) { crow0 = 0; Cb += (long)e * g.strideC; }
+    const bool store = EPI != EPI_BIAS_GELU || g.C != nullptr;      // h is left out where no backward pass will ask for it
     constexpr bool PAIR = N_KS && TNW == 2;         // a lane holds two adjacent columns: 8-byte accesses
     int ncol[TNW];
     float bias[TNW];
@@ -443,14 +444,14 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
             };
             if constexpr (PAIR) {
                 if (ncol[0] < g.N) {
-                    put2(dst + ncol[0], v[0], v[1]);
+                    if (store) put2(dst + ncol[0], v[0], v[1]);
                     if constexpr (EPI == EPI_BIAS_GELU) put2((float *)g.C2 + (crow0 + m) * ldc + ncol[0], v2[0], v2[1]);
                 }
             } else {
 #pragma unroll
                 for (int tn = 0; tn < TNW; ++tn) {
                     if (ncol[tn] >= g.N) continue;
-                    put(dst + ncol[tn], v[tn]);
+                    if (store) put(dst + ncol[tn], v[tn]);
                     if constexpr (EPI == EPI_BIAS_GELU) put((float *)g.C2 + (crow0 + m) * ldc + ncol[tn], v2[tn]);
                 }
             }

@@ -74,7 +74,7 @@ static int check_layer(const char *fn, const mole_layer *L, mole_stream_t) {
     MOLE_REQUIRE(L != nullptr, "%s: null argument block", fn);
     MOLE_REQUIRE(L->S >= 1 && L->rows >= 1 && L->E >= 1 && L->F >= 1, "%s: bad sizes S=%d rows=%d E=%d F=%d", fn, L->S, L->rows, L->E, L->F);
     MOLE_REQUIRE(L->x && L->wg && L->scores && L->gates && L->idx && L->row && L->counts && L->kept_rows && L->offsets && L->xd &&
-                     L->h && L->a && L->out && L->workspace, "%s: null pointer", fn);
+                     (L->h || L->forward_only) && L->a && L->out && L->workspace, "%s: null pointer", fn);
     return 0;
 }
 
@@ -96,6 +96,7 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
 
 extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mole_stream_t stream) {
     if (int rc = check_layer("mole_layer_bwd", L, stream)) return rc;
+    MOLE_REQUIRE(!L->forward_only, "mole_layer_bwd: the forward pass was a forward_only one");
     MOLE_REQUIRE(G && G->dy && G->dlogits && G->d_o && G->t && G->gxd && G->dx && G->dwg, "mole_layer_bwd: null gradient pointer");
     const size_t need = mole_layer_workspace_bytes(L, 1);
     if (L->workspace_bytes < need) {

@@ -39,7 +39,7 @@ struct Plan {
     at::ScalarType dtype;
     int gelu_bwd;
     enum { SCORES, GATES, L_AUX, IDX, LOC, ROW, COUNTS, KEPT, OFFSETS, CAPACITY, N_ROUTE };
-    enum { XD, H, A, OUT, ACT_WS, N_ACT };
+    enum { XD, A, OUT, ACT_WS, H, N_ACT };       // (h last: a pass without autograd leaves it out)
     enum { D_O, T, GXD, DLOGITS, GRAD_WS, N_GRAD };
     int64_t route_off[N_ROUTE], act_off[N_ACT], grad_off[N_GRAD];
     int64_t route_bytes, act_bytes, grad_bytes, ws_fwd, ws_bwd;
@@ -73,7 +73,7 @@ struct Plan {
         ws_fwd = (int64_t)mole_layer_workspace_bytes(&head, 0);
         ws_bwd = (int64_t)mole_layer_workspace_bytes(&head, 1);
         route_bytes = carve({S * E * 4, k * S * 4, 4, k * S * 4, k * S * 4, k * S * 4, k * E * 4, E * 4, (E + 1) * 4, 4}, route_off);
-        act_bytes = carve({rows * M * es, rows * F * es, rows * F * es, rows * M * es, ws_fwd}, act_off);
+        act_bytes = carve({rows * M * es, rows * F * es, rows * M * es, ws_fwd, rows * F * es}, act_off);
         grad_bytes = carve({rows * M * es, rows * F * es, rows * M * es, S * E * 4, ws_bwd}, grad_off);
     }
     std::vector<int64_t> route_offsets() const { return {route_off, route_off + N_ROUTE}; }
@@ -130,11 +130,14 @@ std::pair<Tensor, Tensor> run_forward(Call &c, const Tensor &x, const Tensor &wg
                 "mole_amd: the layer's input or gate does not have the planned shape or type");
     const auto bytes = x.options().dtype(at::kByte);
     c.route = at::empty({p.route_bytes}, bytes);
-    Tensor act = at::empty({p.act_bytes}, bytes), y = at::empty({p.head.S, p.head.M}, x.options());
+    Tensor act = at::empty({l_aux.defined() ? p.act_bytes : p.act_off[Plan::H]}, bytes), y = at::empty({p.head.S, p.head.M}, x.options());
     char *a = (char *)act.data_ptr();
     mole_layer L = arguments(c, x, wg, (char *)c.route.data_ptr(), a, a + p.act_off[Plan::ACT_WS], p.ws_fwd);
     if (l_aux.defined()) L.l_aux = l_aux.data_ptr<float>();
-    else L.forward_only = 1;
+    else {
+        L.forward_only = 1;
+        L.h = nullptr;
+    }
     check(mole_layer_fwd(&L, y.data_ptr(), current_stream(x)), "mole_layer_fwd");
     return {y, act};
 }

@@ -586,3 +586,19 @@ def test_layer_marker_parameter_and_changed_gelu_derivative(padded):
         grads.append(m.FC1_W_GPU.grad_tensors.clone())
         assert m.dummy_param.grad is not None and m.dummy_param.grad.shape == m.dummy_param.shape
     assert not torch.equal(grads[0], grads[1])
+
+
+@pytest.mark.parametrize("S,M,E,k,Fd,dtype", [
+    (16387, 256, 4, 1, 1024, torch.bfloat16),       # 256-row tiles with a remainder
+    (16387, 264, 4, 1, 1032, torch.bfloat16),       # the same, contraction and columns ending inside a tile
+    (1003, 256, 4, 1, 520, torch.bfloat16),         # 128 x 128 tiles
+    (33, 128, 8, 2, 256, torch.bfloat16),           # few rows
+    (33, 128, 8, 2, 256, torch.float32), (1003, 128, 4, 1, 264, torch.float32), (8200, 256, 4, 2, 1024, torch.float32),
+    (90, 68, 4, 2, 132, torch.float32)])            # widths that no tiled kernel takes
+def test_forward_without_autograd_gives_the_same_bits(S, M, E, k, Fd, dtype):
+    """Under no_grad the pre-activation is not stored; the output has the bits of the pass that stores it."""
+    print(f"no_grad forward S={S} M={M} E={E} k={k} F={Fd} {dtype}", flush=True)
+    m, x, _ = _build(S, M, E, k, Fd, dtype)
+    y = m(x, capacity_factor=0.0).detach()
+    with torch.no_grad():
+        assert torch.equal(m(x, capacity_factor=0.0), y)
