@@ -411,7 +411,7 @@ static bool skinny_plan(int dtype, bool b_ks, int E, int est_rows, int N, int K,
         takes = tiles < 192 && avg <= (b_ks ? 64 : 24);
         // every group of 16 rows reads the expert's weights again, from memory where they are more than the 256 MB last-level
         // cache holds: there the tiles take what is more than one group (14 experts of 2304 -> 4608, 56 rows: out 169 us
-        // against 76; 20 of 2264 -> 9056, 20 rows: 304 against 153)
+        // against 58, planes added; 20 of 2264 -> 9056, 20 rows: 304 against 153)
         if (b_ks && avg > 16 && (size_t)active * N * K * sizeof(bf16_t) > (size_t)256 << 20) takes = false;
     } else {
         takes = avg <= (b_ks ? 64 : 20);
