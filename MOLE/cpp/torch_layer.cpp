@@ -38,7 +38,7 @@ struct Plan {
     mole_layer head{};
     at::ScalarType dtype;
     int gelu_bwd;
-    enum { SCORES, GATES, L_AUX, IDX, LOC, ROW, COUNTS, KEPT, OFFSETS, CAPACITY, N_ROUTE };
+    enum { SCORES, GATES, IDX, LOC, ROW, COUNTS, KEPT, OFFSETS, CAPACITY, N_ROUTE };
     enum { XD, A, OUT, ACT_WS, H, N_ACT };       // (h last: a pass without autograd leaves it out)
     enum { D_O, T, GXD, DLOGITS, GRAD_WS, N_GRAD };
     int64_t route_off[N_ROUTE], act_off[N_ACT], grad_off[N_GRAD];
@@ -72,7 +72,7 @@ struct Plan {
         head.rows = (int)rows; head.layout = layout; head.normalize_gate = normalize; head.capacity_factor = cf;
         ws_fwd = (int64_t)mole_layer_workspace_bytes(&head, 0);
         ws_bwd = (int64_t)mole_layer_workspace_bytes(&head, 1);
-        route_bytes = carve({S * E * 4, k * S * 4, 4, k * S * 4, k * S * 4, k * S * 4, k * E * 4, E * 4, (E + 1) * 4, 4}, route_off);
+        route_bytes = carve({S * E * 4, k * S * 4, k * S * 4, k * S * 4, k * S * 4, k * E * 4, E * 4, (E + 1) * 4, 4}, route_off);
         act_bytes = carve({rows * M * es, rows * F * es, rows * M * es, ws_fwd, rows * F * es}, act_off);
         grad_bytes = carve({rows * M * es, rows * F * es, rows * M * es, S * E * 4, ws_bwd}, grad_off);
     }
@@ -104,7 +104,6 @@ mole_layer arguments(const Call &c, const Tensor &x, const Tensor &wg, char *rou
     L.w1 = c.weights[0].data_ptr(); L.b1 = c.weights[1].data_ptr(); L.w2 = c.weights[2].data_ptr(); L.b2 = c.weights[3].data_ptr();
     L.scores = (float *)(route + p.route_off[Plan::SCORES]);
     L.gates = (float *)(route + p.route_off[Plan::GATES]);
-    L.l_aux = (float *)(route + p.route_off[Plan::L_AUX]);
     L.idx = (int32_t *)(route + p.route_off[Plan::IDX]);
     L.loc = (int32_t *)(route + p.route_off[Plan::LOC]);
     L.row = (int32_t *)(route + p.route_off[Plan::ROW]);
@@ -120,8 +119,12 @@ mole_layer arguments(const Call &c, const Tensor &x, const Tensor &wg, char *rou
 
 void *current_stream(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
-// (y, act); c.route is set.  l_aux: where the loss term goes, or undefined (it then stays inside route).
-std::pair<Tensor, Tensor> run_forward(Call &c, const Tensor &x, const Tensor &wg, const Tensor &l_aux) {
+// y, the intermediates the backward reads, and the loss term, a tensor of its own: callers keep it, and part of a larger
+// buffer would keep all of that.  c.route is set.
+struct Outputs {
+    Tensor y, act, l_aux;
+};
+Outputs run_forward(Call &c, const Tensor &x, const Tensor &wg, bool forward_only) {
     const Plan &p = *c.plan;
     check_tensor(x, "x");
     check_tensor(wg, "the gate's weight");
@@ -130,16 +133,17 @@ std::pair<Tensor, Tensor> run_forward(Call &c, const Tensor &x, const Tensor &wg
                 "mole_amd: the layer's input or gate does not have the planned shape or type");
     const auto bytes = x.options().dtype(at::kByte);
     c.route = at::empty({p.route_bytes}, bytes);
-    Tensor act = at::empty({l_aux.defined() ? p.act_bytes : p.act_off[Plan::H]}, bytes), y = at::empty({p.head.S, p.head.M}, x.options());
+    Tensor act = at::empty({forward_only ? p.act_off[Plan::H] : p.act_bytes}, bytes), y = at::empty({p.head.S, p.head.M}, x.options());
+    Tensor l_aux = at::empty({}, x.options().dtype(at::kFloat));
     char *a = (char *)act.data_ptr();
     mole_layer L = arguments(c, x, wg, (char *)c.route.data_ptr(), a, a + p.act_off[Plan::ACT_WS], p.ws_fwd);
-    if (l_aux.defined()) L.l_aux = l_aux.data_ptr<float>();
-    else {
+    L.l_aux = l_aux.data_ptr<float>();
+    if (forward_only) {
         L.forward_only = 1;
         L.h = nullptr;
     }
     check(mole_layer_fwd(&L, y.data_ptr(), current_stream(x)), "mole_layer_fwd");
-    return {y, act};
+    return {y, act, l_aux};
 }
 
 struct LayerFn : torch::autograd::Function<LayerFn> {
@@ -148,8 +152,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         c->dummy_sizes = dummy.sizes().vec();
         c->dummy_options = dummy.options();
         ctx->set_materialize_grads(false);
-        Tensor l_aux = at::empty({}, x.options().dtype(at::kFloat));
-        auto [y, act] = run_forward(*c, x, wg, l_aux);
+        auto [y, act, l_aux] = run_forward(*c, x, wg, false);
         ctx->save_for_backward({x, wg, c->route, act});
         ctx->saved_data["call"] = c10::IValue::make_capsule(std::move(c));
         return {y, l_aux};
@@ -183,10 +186,10 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     }
 };
 
-// (y, l_aux or None, route)
-std::tuple<Tensor, std::optional<Tensor>, Tensor> layer(const Tensor &x, const Tensor &wg, const Tensor &dummy, std::optional<Tensor> bias,
-                                                        std::vector<Tensor> weights, std::vector<Tensor> grads,
-                                                        std::shared_ptr<Plan> plan, bool accumulate, std::shared_ptr<Counter> counter) {
+// (y, l_aux, route, l_aux without its graph)
+std::tuple<Tensor, Tensor, Tensor, Tensor> layer(const Tensor &x, const Tensor &wg, const Tensor &dummy, std::optional<Tensor> bias,
+                                                 std::vector<Tensor> weights, std::vector<Tensor> grads, std::shared_ptr<Plan> plan,
+                                                 bool accumulate, std::shared_ptr<Counter> counter) {
     TORCH_CHECK(weights.size() == 4 && grads.size() == 4, "mole_amd: four parameter and four gradient tensors");
     auto c = c10::make_intrusive<Call>();
     c->plan = std::move(plan);
@@ -197,11 +200,11 @@ std::tuple<Tensor, std::optional<Tensor>, Tensor> layer(const Tensor &x, const T
     c->accumulate = accumulate;
     // (no_grad leaves forward-mode derivatives on: an input that carries a tangent goes through the node, which refuses it)
     if (!at::GradMode::is_enabled() && !x._fw_grad(0).defined() && !wg._fw_grad(0).defined()) {
-        auto ya = run_forward(*c, x, wg, Tensor());
-        return {ya.first, std::nullopt, c->route};
+        auto r = run_forward(*c, x, wg, true);
+        return {r.y, r.l_aux, c->route, r.l_aux};
     }
     auto out = LayerFn::apply(x, wg, dummy, c);
-    return {out[0], out[1], c->route};
+    return {out[0], out[1], c->route, out[1].detach()};
 }
 
 }  // namespace

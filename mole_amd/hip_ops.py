@@ -429,13 +429,13 @@ def adam_step(p, g, m, v, beta1: float, beta2: float, t: int, lr: float, lam: fl
 # ---- the layer in one call each way (mole_layer_fwd / mole_layer_bwd) ---------------------------------------------
 class LayerPlan:
     """Sizes of one layer call, shared by every call of the same shape (the native Plan); route() gives the routing in a
-    call's `route` buffer as tensors."""
+    call's `route` buffer, and the loss term beside it, as tensors."""
 
     def __init__(self, dtype, S, M, E, k, F, capacity_factor, layout, normalize_gate, gelu_bwd):
         self.S, self.E, self.k, self.layout, self.normalize_gate = S, E, k, layout, normalize_gate
         self.native = L.native().Plan(L.dtype_code(dtype), S, M, E, k, F, capacity_factor, layout, normalize_gate, gelu_bwd)
 
-    def route(self, buf: torch.Tensor) -> Route:
+    def route(self, buf: torch.Tensor, l_aux: torch.Tensor) -> Route:
         offs = iter(self.native.route_offsets())
 
         def take(dt, *shape):
@@ -445,7 +445,8 @@ class LayerPlan:
             return buf[o:o + n * 4].view(dt).view(*shape)
         S, E, k, i32, f32 = self.S, self.E, self.k, torch.int32, torch.float32
         take(f32, S, E)                                     # the scores
-        gates, l_aux = take(f32, k, S), take(f32, 1)
+        gates = take(f32, k, S)
         idx, loc, row = take(i32, k, S), take(i32, k, S), take(i32, k, S)
         counts, kept, offsets, capacity = take(i32, k, E), take(i32, E), take(i32, E + 1), take(i32, 1)
-        return Route(S, E, k, self.layout, idx, loc, gates, row, counts, kept, offsets, capacity, l_aux, self.normalize_gate)
+        return Route(S, E, k, self.layout, idx, loc, gates, row, counts, kept, offsets, capacity, l_aux.view(1),
+                     self.normalize_gate)

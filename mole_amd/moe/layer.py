@@ -204,7 +204,7 @@ class MOLEModule(torch.nn.Module):
         self.global_prefetch = False
         self.grad_use_pool, self.mome_use_pool, self.vari_use_pool = pool_for_extra
         self.l_aux = None
-        self._route = None           # (plan, buffer) of the last one-call forward, or the Route of another
+        self._route = None           # (plan, buffer, l_aux) of the last one-call forward, or the Route of another
         self._plans = {}             # LayerPlan per (tokens, capacity factor, ...): sizes only, no device memory
         self.moe_id = len(MOLEModule._instance)
         MOLEModule._instance.append(self)
@@ -214,22 +214,11 @@ class MOLEModule(torch.nn.Module):
     def last_route(self):
         """The Route of the last forward pass."""
         r = self._route
-        return r[0].route(r[1]) if isinstance(r, tuple) else r
+        return r[0].route(*r[1:]) if isinstance(r, tuple) else r
 
     @last_route.setter
     def last_route(self, r):
         self._route = r
-
-    @property
-    def l_aux(self):
-        """The load-balancing loss of the last forward pass."""
-        if self._l_aux is None and isinstance(self.__dict__.get("_route"), tuple):
-            self._l_aux = self.last_route.l_aux.view(())
-        return self._l_aux
-
-    @l_aux.setter
-    def l_aux(self, v):
-        self._l_aux = v
 
     def _plan(self, S, capacity_factor, wg):
         """The LayerPlan of a forward pass over S tokens, or None when it takes the step-by-step path (experts offloaded, no
@@ -307,11 +296,11 @@ class MOLEModule(torch.nn.Module):
         plan = None if time_it else self._plan(resized_input.shape[0], float(capacity_factor), wg)
         if plan is not None:
             core_ = self.MOLECore
-            expert_output, l_aux, route = L.native().layer(
+            expert_output, l_aux, route, l_aux_value = L.native().layer(
                 resized_input, wg, self.dummy_param, gate.logit_bias, [g[0] for g in core_.gpu], [g[1] for g in core_.gpu],
                 plan.native, core_.acc_step > 1, core_.passes)
-            self.__dict__["_route"] = (plan, route)
-            self.__dict__["_l_aux"] = l_aux
+            self.__dict__["_route"] = (plan, route, l_aux_value)
+            self.__dict__["l_aux"] = l_aux
         elif self.reference_layout:
             scores = self.gate[0](resized_input)
             crit, l_aux = tutel_fast_dispatcher.extract_critical(

@@ -602,3 +602,23 @@ def test_forward_without_autograd_gives_the_same_bits(S, M, E, k, Fd, dtype):
     y = m(x, capacity_factor=0.0).detach()
     with torch.no_grad():
         assert torch.equal(m(x, capacity_factor=0.0), y)
+
+
+@pytest.mark.parametrize("padded", [False, True])
+def test_last_route_holds_the_loss_term(padded):
+    """last_route.l_aux is the l_aux of the pass, recorded by autograd or not, whatever the memory held before; both are
+    small tensors of their own, and an l_aux that the caller has let go of stays away."""
+    from mole_amd.utils import Ugate
+    m, x, _ = _build(200, 64, 8, 2, 128, torch.bfloat16, reference_layout=padded)
+    for grad in (True, False, True):
+        fill = [torch.full((n,), float("nan"), device="cuda") for n in (1 << 8, 1 << 12, 1 << 16, 1 << 20)]
+        del fill
+        with torch.set_grad_enabled(grad):
+            m(x, capacity_factor=1.0)
+        r = m.last_route
+        want = O.extract_critical(Ugate.gate_scores(x, m.gate[0].linear.weight).cpu(), 2, 1.0).l_aux
+        assert abs(float(m.l_aux.detach()) - want) < 1e-4 * max(1.0, want)
+        assert torch.equal(r.l_aux, m.l_aux.detach().view(1)) and not r.l_aux.requires_grad and m.l_aux.requires_grad == grad
+        assert m.l_aux.untyped_storage().nbytes() == 4
+        m.l_aux = None
+        assert m.l_aux is None
