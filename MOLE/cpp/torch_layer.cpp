@@ -6,6 +6,7 @@
 // them in the library.  The rest was an autograd.Function and its context in Python, tensor allocations through the
 // interpreter and argument blocks through ctypes, half of it on autograd's own thread.
 #include <torch/extension.h>
+#include <ATen/TracerMode.h>
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
@@ -191,6 +192,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> layer(const Tensor &x, const Tensor &
                                                  std::vector<Tensor> weights, std::vector<Tensor> grads, std::shared_ptr<Plan> plan,
                                                  bool accumulate, std::shared_ptr<Counter> counter) {
     TORCH_CHECK(weights.size() == 4 && grads.size() == 4, "mole_amd: four parameter and four gradient tensors");
+    // (a trace would record the allocations and none of the kernels: its replays would return memory nothing has written)
+    TORCH_CHECK(!at::tracer::impl::is_dispatch_enabled(), "mole_amd: the layer cannot be traced by torch.jit.trace");
     auto c = c10::make_intrusive<Call>();
     c->plan = std::move(plan);
     c->counter = std::move(counter);

@@ -622,3 +622,13 @@ def test_last_route_holds_the_loss_term(padded):
         assert m.l_aux.untyped_storage().nbytes() == 4
         m.l_aux = None
         assert m.l_aux is None
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_layer_refuses_to_be_traced(grad):
+    """The native node's kernels leave nothing in a trace: tracing is an error, not a function of unwritten memory."""
+    m, x, _ = _build(16, 64, 4, 2, 128, torch.float32)
+    with torch.set_grad_enabled(grad), pytest.raises(RuntimeError):
+        torch.jit.trace(lambda t: m(t, capacity_factor=0.0), (x,), check_trace=False)
+    with torch.set_grad_enabled(grad):
+        assert bool(m(x, capacity_factor=0.0).isfinite().all())       # and untraced calls go on
