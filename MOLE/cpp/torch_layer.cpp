@@ -33,14 +33,16 @@ struct Counter {
 };
 
 // Sizes of one layer call, shared by every call of the same shape: the kept rows' bound, and where each intermediate lies
-// in the three buffers of a call - route (scores and routing, kept for the backward), act (xd, h, a, out and the forward's
-// scratch) and grad (the backward's temporaries and scratch).  Holds no device memory.
+// in the buffers of a call - route (the routing, which the layer also keeps as last_route), act (xd, a, out, scores and h, kept
+// for the backward) and grad (the backward's temporaries and scratch).  The forward's scratch is no part of what is kept: it
+// has a buffer of its own, or in a pass without autograd, which keeps nothing and stores no h, the place of h.  Holds no
+// device memory.
 struct Plan {
     mole_layer head{};
     at::ScalarType dtype;
     int gelu_bwd;
-    enum { SCORES, GATES, IDX, LOC, ROW, COUNTS, KEPT, OFFSETS, CAPACITY, N_ROUTE };
-    enum { XD, A, OUT, ACT_WS, H, N_ACT };       // (h last: a pass without autograd leaves it out)
+    enum { GATES, IDX, LOC, ROW, COUNTS, KEPT, OFFSETS, CAPACITY, N_ROUTE };
+    enum { XD, A, OUT, SCORES, H, N_ACT };
     enum { D_O, T, GXD, DLOGITS, GRAD_WS, N_GRAD };
     int64_t route_off[N_ROUTE], act_off[N_ACT], grad_off[N_GRAD];
     int64_t route_bytes, act_bytes, grad_bytes, ws_fwd, ws_bwd;
@@ -73,8 +75,8 @@ struct Plan {
         head.rows = (int)rows; head.layout = layout; head.normalize_gate = normalize; head.capacity_factor = cf;
         ws_fwd = (int64_t)mole_layer_workspace_bytes(&head, 0);
         ws_bwd = (int64_t)mole_layer_workspace_bytes(&head, 1);
-        route_bytes = carve({S * E * 4, k * S * 4, k * S * 4, k * S * 4, k * S * 4, k * E * 4, E * 4, (E + 1) * 4, 4}, route_off);
-        act_bytes = carve({rows * M * es, rows * F * es, rows * M * es, ws_fwd, rows * F * es}, act_off);
+        route_bytes = carve({k * S * 4, k * S * 4, k * S * 4, k * S * 4, k * E * 4, E * 4, (E + 1) * 4, 4}, route_off);
+        act_bytes = carve({rows * M * es, rows * F * es, rows * M * es, S * E * 4, rows * F * es}, act_off);
         grad_bytes = carve({rows * M * es, rows * F * es, rows * M * es, S * E * 4, ws_bwd}, grad_off);
     }
     std::vector<int64_t> route_offsets() const { return {route_off, route_off + N_ROUTE}; }
@@ -103,7 +105,7 @@ mole_layer arguments(const Call &c, const Tensor &x, const Tensor &wg, char *rou
     L.wg = wg.data_ptr<float>();
     L.logit_bias = c.bias.has_value() ? c.bias->data_ptr<float>() : nullptr;
     L.w1 = c.weights[0].data_ptr(); L.b1 = c.weights[1].data_ptr(); L.w2 = c.weights[2].data_ptr(); L.b2 = c.weights[3].data_ptr();
-    L.scores = (float *)(route + p.route_off[Plan::SCORES]);
+    L.scores = (float *)(act + p.act_off[Plan::SCORES]);
     L.gates = (float *)(route + p.route_off[Plan::GATES]);
     L.idx = (int32_t *)(route + p.route_off[Plan::IDX]);
     L.loc = (int32_t *)(route + p.route_off[Plan::LOC]);
@@ -134,10 +136,12 @@ Outputs run_forward(Call &c, const Tensor &x, const Tensor &wg, bool forward_onl
                 "mole_amd: the layer's input or gate does not have the planned shape or type");
     const auto bytes = x.options().dtype(at::kByte);
     c.route = at::empty({p.route_bytes}, bytes);
-    Tensor act = at::empty({forward_only ? p.act_off[Plan::H] : p.act_bytes}, bytes), y = at::empty({p.head.S, p.head.M}, x.options());
+    Tensor act = at::empty({forward_only ? p.act_off[Plan::H] + p.ws_fwd : p.act_bytes}, bytes), y = at::empty({p.head.S, p.head.M}, x.options());
     Tensor l_aux = at::empty({}, x.options().dtype(at::kFloat));
+    Tensor ws;
+    if (!forward_only) ws = at::empty({p.ws_fwd}, bytes);       // (released on return, for later work of this stream)
     char *a = (char *)act.data_ptr();
-    mole_layer L = arguments(c, x, wg, (char *)c.route.data_ptr(), a, a + p.act_off[Plan::ACT_WS], p.ws_fwd);
+    mole_layer L = arguments(c, x, wg, (char *)c.route.data_ptr(), a, forward_only ? a + p.act_off[Plan::H] : (char *)ws.data_ptr(), p.ws_fwd);
     L.l_aux = l_aux.data_ptr<float>();
     if (forward_only) {
         L.forward_only = 1;

@@ -444,7 +444,6 @@ class LayerPlan:
                 n *= d
             return buf[o:o + n * 4].view(dt).view(*shape)
         S, E, k, i32, f32 = self.S, self.E, self.k, torch.int32, torch.float32
-        take(f32, S, E)                                     # the scores
         gates = take(f32, k, S)
         idx, loc, row = take(i32, k, S), take(i32, k, S), take(i32, k, S)
         counts, kept, offsets, capacity = take(i32, k, E), take(i32, E), take(i32, E + 1), take(i32, 1)

@@ -632,3 +632,22 @@ def test_layer_refuses_to_be_traced(grad):
         torch.jit.trace(lambda t: m(t, capacity_factor=0.0), (x,), check_trace=False)
     with torch.set_grad_enabled(grad):
         assert bool(m(x, capacity_factor=0.0).isfinite().all())       # and untraced calls go on
+
+
+@pytest.mark.parametrize("S,M,E,k,Fd,padded", [(1000, 256, 8, 2, 3072, False), (300, 512, 4, 1, 2048, False), (40, 256, 16, 2, 2048, True),
+                                               (5000, 64, 64, 2, 64, False)])
+def test_recorded_pass_keeps_what_its_backward_reads(S, M, E, k, Fd, padded):
+    """Between forward and backward a pass holds its input, the gate's weight, the scores, the routing and the four row
+    buffers, and no scratch: neither the split contractions' planes nor the routing's workspace.  last_route keeps the
+    routing alone (k (3 S + E) numbers and the gate values), not the scores.  (Buffers begin at multiples of 256 bytes.)"""
+    m, x, _ = _build(S, M, E, k, Fd, torch.bfloat16, reference_layout=padded)
+    cf = 1.0 if padded else 0.0
+    rows = E * k * int(cf * -(-S // E)) if padded else S * k
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (kept.append(t.nbytes), t)[1], lambda t: t):
+        y = m(x, capacity_factor=cf)
+    route = 4 * (4 * k * S + k * E + 2 * E + 2)
+    want = x.nbytes + 4 * E * M + route + 4 * S * E + 2 * rows * (2 * M + 2 * Fd)
+    assert want <= sum(kept) <= want + 32 * 256
+    assert m.last_route.row.untyped_storage().nbytes() <= route + 16 * 256
+    y.sum().backward()
