@@ -37,6 +37,12 @@ from ..utils.Uparam import CPUHostBatchedParameter, GPUHostBatchedParameter, Uni
 from . import fast_dispatch as tutel_fast_dispatcher
 
 
+def _is_plain(gate):
+    """Whether calling the gate is what the fused paths compute from its weight and bias, and nothing else would notice."""
+    return (type(gate) is Ugate.MOLETopk and "forward" not in gate.__dict__ and not torch.nn.modules.module._has_any_global_hook()
+            and not (gate._forward_hooks or gate._forward_pre_hooks or gate._backward_hooks or gate._backward_pre_hooks))
+
+
 class pfetchbwd(torch.autograd.Function):
     """Identity on the layer input whose backward - which runs once this layer's own backward is
     done - starts the previous layer's backward prefetch (the counterpart of layer.py:464-472; the
@@ -220,9 +226,13 @@ class MOLEModule(torch.nn.Module):
     def last_route(self, r):
         self._route = r
 
-    def _plan(self, S, capacity_factor, wg):
+    def _plan(self, S, capacity_factor, gate):
         """The LayerPlan of a forward pass over S tokens, or None when it takes the step-by-step path (experts offloaded, no
-        tokens, a gate in another dtype, a padded capacity that only the device knows; a profiled pass also does)."""
+        tokens, a gate in another dtype, a padded capacity that only the device knows; a profiled pass also does).  The
+        padded layout calls the gate as a module: a gate of another kind and one with hooks are called there still."""
+        if self.reference_layout and not _is_plain(gate):
+            return None
+        wg = gate.linear.weight
         if (self.d_experts or not self.s_experts or S < 1 or wg.dtype != torch.float32 or not wg.is_contiguous()
                 or self.embed_dim % self._granule or self.ffn_dim % self._granule or (self.reference_layout and not capacity_factor > 0)):
             return None
@@ -292,17 +302,16 @@ class MOLEModule(torch.nn.Module):
         resized_input = resized_input.contiguous()
 
         gate = self.gate[0]
-        wg = gate.linear.weight
-        plan = None if time_it else self._plan(resized_input.shape[0], float(capacity_factor), wg)
+        plan = None if time_it else self._plan(resized_input.shape[0], float(capacity_factor), gate)
         if plan is not None:
             core_ = self.MOLECore
             expert_output, l_aux, route, l_aux_value = L.native().layer(
-                resized_input, wg, self.dummy_param, gate.logit_bias, [g[0] for g in core_.gpu], [g[1] for g in core_.gpu],
+                resized_input, gate.linear.weight, self.dummy_param, gate.logit_bias, [g[0] for g in core_.gpu], [g[1] for g in core_.gpu],
                 plan.native, core_.acc_step > 1, core_.passes)
             self.__dict__["_route"] = (plan, route, l_aux_value)
             self.__dict__["l_aux"] = l_aux
         elif self.reference_layout:
-            scores = self.gate[0](resized_input)
+            scores = gate(resized_input)
             crit, l_aux = tutel_fast_dispatcher.extract_critical(
                 scores, top_k=self.topk, capacity_factor=capacity_factor, normalize_gate=self.normalize_gate)
             self.l_aux = l_aux
@@ -310,7 +319,8 @@ class MOLEModule(torch.nn.Module):
             experts_output = BatchFusedFWD.apply(dispatched_input, self, self.dummy_param, time_it, prefetch)
             expert_output = tutel_fast_dispatcher.fast_decode(data=experts_output, critial_data=crit)
         else:
-            expert_output, self.l_aux = _FusedMoE.apply(resized_input, wg, self.dummy_param, self, float(capacity_factor), bool(time_it))
+            expert_output, self.l_aux = _FusedMoE.apply(resized_input, gate.linear.weight, self.dummy_param, self, float(capacity_factor),
+                                                        bool(time_it))
 
         expert_output = expert_output.reshape(original_shape)
         out = expert_output.to(original_dtype)

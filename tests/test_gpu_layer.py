@@ -651,3 +651,39 @@ def test_recorded_pass_keeps_what_its_backward_reads(S, M, E, k, Fd, padded):
     assert want <= sum(kept) <= want + 32 * 256
     assert m.last_route.row.untyped_storage().nbytes() <= route + 16 * 256
     y.sum().backward()
+
+
+@pytest.mark.parametrize("kind", ["hook", "backward hook", "other module", "own forward"])
+def test_padded_layout_calls_the_gate(kind):
+    """The padded layout takes its scores from self.gate[0] as a module: hooks on it run, and a gate of another kind (with no
+    `linear` of its own) or with a forward of its own decides the routing."""
+    S, M, E, k, cf = 60, 64, 4, 1, 4.0
+    m, x, _ = _build(S, M, E, k, 128, torch.float32, reference_layout=True)
+    x.requires_grad_(True)
+    gate, seen = m.gate[0], []
+    w = gate.linear.weight
+    worst_first = lambda t: torch.softmax(-(t @ w.t()), dim=1)
+    want = gate(x.detach()).argmax(dim=1) if "hook" in kind else worst_first(x.detach()).argmax(dim=1)
+    if kind == "hook":
+        gate.register_forward_hook(lambda mod, args, out: seen.append(out.shape))
+    elif kind == "backward hook":
+        gate.register_full_backward_hook(lambda mod, gi, go: seen.append(go[0].shape))
+    elif kind == "own forward":
+        gate.forward = worst_first
+    else:
+        class Gate(torch.nn.Module):
+            def forward(self, t):
+                return worst_first(t)
+        m.gate[0] = Gate()
+    y = m(x, capacity_factor=cf)
+    y.sum().backward()
+    if "hook" in kind:
+        assert seen == [(S, E)]
+    # all experts but the chosen one silenced in the second product: the output names the expert
+    with torch.no_grad():
+        for e in range(E):
+            m.FC2_W_GPU.all_tensors[e].zero_()
+            m.FC2_B_GPU.all_tensors[e].fill_(float(e))
+        got = m(x, capacity_factor=cf)[:, 0]
+    score = (gate(x.detach()) if "hook" in kind else worst_first(x.detach())).max(dim=1).values
+    assert torch.allclose(got, want.float() * score, rtol=1e-5, atol=1e-6)
