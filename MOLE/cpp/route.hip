@@ -1244,7 +1244,11 @@ extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const 
     MOLE_REQUIRE(layout == MOLE_LAYOUT_PADDED || layout == MOLE_LAYOUT_RAGGED, "mole_gate_route: bad layout %d", layout);
     MOLE_REQUIRE(x && wg && scores && idx && loc && gates && row && counts && kept_rows && offsets && capacity && workspace,
                  "mole_gate_route: null pointer");
-    MOLE_REQUIRE((((uintptr_t)x | (uintptr_t)wg) & 15) == 0, "mole_gate_route: x and wg must be 16-byte aligned");
+    // (fp32 as in the entry points it joins; bf16 kernels read the fp32 weights, and small gates the tokens, at any alignment
+    // of their elements: a gate's weight may be a view into a flat parameter buffer)
+    const bool any_x = dtype == MOLE_BF16 && E <= 64 && M % 128 == 0, any_wg = dtype == MOLE_BF16;
+    MOLE_REQUIRE((any_x || ((uintptr_t)x & 15) == 0) && (any_wg || ((uintptr_t)wg & 15) == 0),
+                 "mole_gate_route: x and wg must be 16-byte aligned");
     MOLE_REQUIRE((long long)S * k < INT_MAX, "mole_gate_route: S*k too large");
     const size_t need = mole_gate_route_workspace_bytes(dtype, S, E, M, k);
     if (workspace_bytes < need) {

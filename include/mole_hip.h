@@ -150,7 +150,8 @@ int mole_route(const float *scores, int S, int E, int k, double capacity_factor,
 
 /* mole_gate_fwd (or mole_gemm_nt + mole_softmax_fwd) and mole_route in one call: MOLETopk.forward followed by
  * extract_critical (MOLE/utils/Ugate.py:11-14, MOLE/moe/layer.py:442-446).  Any S >= 1, E and k as in mole_route, M a
- * multiple of 8 (bf16) or 4 (fp32), x and wg 16-byte aligned.  Arguments and results are those of the two calls; scores
+ * multiple of 8 (bf16) or 4 (fp32), x and wg 16-byte aligned (bf16: wg in any case as it comes; x as well if E <= 64 and M is
+ * a multiple of 128).  Arguments and results are those of the two calls; scores
  * [S,E] is an output here.  Small gates on many bf16 tokens run as one kernel up to the per-token part of the routing
  * (the scores are routed in the lanes that formed them), few tokens on 16 x 16 tiles of the logits followed by one
  * kernel that does the softmax and, up to 64 tokens, the whole routing.  Against the two calls the scores and every

@@ -687,3 +687,29 @@ def test_padded_layout_calls_the_gate(kind):
         got = m(x, capacity_factor=cf)[:, 0]
     score = (gate(x.detach()) if "hook" in kind else worst_first(x.detach())).max(dim=1).values
     assert torch.allclose(got, want.float() * score, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("S,M,E,train", [(5, 128, 8, False), (200, 128, 8, False), (50, 136, 70, False), (2100, 72, 300, False),
+                                         (2100, 128, 33, True), (60, 264, 40, True)])
+def test_gate_weight_inside_a_flat_buffer(S, M, E, train):
+    """bf16 layers take a gate weight that starts anywhere in a buffer of fp32 values (a view into flat parameters): on every
+    way the gate and the routing can go, and in training where the gate's input gradient is a product of its own."""
+    print(f"gate weight in a flat buffer S={S} M={M} E={E} train={train}", flush=True)
+    m, x, _ = _build(S, M, E, 2, 64, torch.bfloat16)
+    w = m.gate[0].linear.weight.detach().clone()
+    flat = torch.zeros(w.numel() + 4, device="cuda")
+    got = []
+    for at in (0, 1, 2, 3):
+        view = flat[at:at + w.numel()].view(w.shape)
+        view.copy_(w)
+        m.gate[0].linear.weight = torch.nn.Parameter(view)
+        assert view.data_ptr() % 16 == 4 * at
+        xx = x.clone().requires_grad_(train)
+        with torch.set_grad_enabled(train):
+            y = m(xx, capacity_factor=0.0)
+        if train:
+            y.sum().backward()
+        got.append([y.detach()] + ([xx.grad, m.gate[0].linear.weight.grad] if train else []))
+    for other in got[1:]:
+        for a, b in zip(other, got[0]):
+            assert torch.equal(a, b)
