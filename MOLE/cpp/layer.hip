@@ -66,7 +66,7 @@ using namespace mole;
 extern "C" size_t mole_layer_workspace_bytes(const mole_layer *L, int backward) {
     if (L == nullptr || L->S <= 0 || L->E <= 0) return 0;
     const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
-    const size_t other = backward ? gate_bwd_plan(*L).total : mole_gate_route_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
+    const size_t other = backward ? gate_bwd_plan(*L).total : mole_gate_route_shape_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
     return ffn > other ? ffn : other;        // the two are never in use at the same time
 }
 

@@ -15,6 +15,7 @@
 //   route_finalize  loc = base(choice, expert) + block prefix + in-block rank; row = offset + loc.
 #include "common.h"
 
+#include <algorithm>
 #include <limits.h>
 #include <math.h>
 
@@ -1219,7 +1220,7 @@ static int gate_route_path(int dtype, int S, int E, int M) {
     return dtype == MOLE_F32 && E <= 32 ? GR_SCORES : GR_GEMM;
 }
 
-extern "C" size_t mole_gate_route_workspace_bytes(int dtype, int S, int E, int M, int k) {
+extern "C" size_t mole_gate_route_shape_workspace_bytes(int dtype, int S, int E, int M, int k) {
     if (S < 0 || E <= 0 || M <= 0 || k <= 0) return 0;
     const int path = gate_route_path(dtype, S, E, M);
     if (path == GR_FUSED) return gate_route_fused_bytes(S, E, k);
@@ -1227,6 +1228,12 @@ extern "C" size_t mole_gate_route_workspace_bytes(int dtype, int S, int E, int M
     if (path != GR_SCORES) n += align256((size_t)S * E * sizeof(float));
     if (path == GR_GEMM && dtype == MOLE_BF16) n += align256((size_t)E * M * sizeof(bf16_t));
     return n;
+}
+
+extern "C" size_t mole_gate_route_workspace_bytes(int S, int E, int k) {
+    if (S < 0 || E <= 0 || k <= 0) return 0;
+    return S > RT_TOKENS ? gate_route_fused_bytes(S, E, k)
+                         : std::max(gate_route_fused_bytes(S, E, k), mole_gate_route_shape_workspace_bytes(MOLE_BF16, S, E, 128, k));
 }
 
 extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M,
@@ -1250,7 +1257,7 @@ extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const 
     MOLE_REQUIRE((any_x || ((uintptr_t)x & 15) == 0) && (any_wg || ((uintptr_t)wg & 15) == 0),
                  "mole_gate_route: x and wg must be 16-byte aligned");
     MOLE_REQUIRE((long long)S * k < INT_MAX, "mole_gate_route: S*k too large");
-    const size_t need = mole_gate_route_workspace_bytes(dtype, S, E, M, k);
+    const size_t need = mole_gate_route_shape_workspace_bytes(dtype, S, E, M, k);
     if (workspace_bytes < need) {
         set_error("mole_gate_route: workspace of %zu bytes, need %zu", workspace_bytes, need);
         return MOLE_E_WORKSPACE;

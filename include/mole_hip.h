@@ -157,7 +157,9 @@ int mole_route(const float *scores, int S, int E, int k, double capacity_factor,
  * kernel that does the softmax and, up to 64 tokens, the whole routing.  Against the two calls the scores and every
  * routing result are equal bit for bit where both run the same order of sums (bf16, M a multiple of 128, E <= 64);
  * l_aux, and elsewhere the scores, to rounding. */
-size_t mole_gate_route_workspace_bytes(int dtype, int S, int E, int M, int k);
+size_t mole_gate_route_shape_workspace_bytes(int dtype, int S, int E, int M, int k);
+/* ... the same for bf16, E <= 64 and M a multiple of 128, whatever M is */
+size_t mole_gate_route_workspace_bytes(int S, int E, int k);
 int mole_gate_route(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M, int k,
                     double capacity_factor, int normalize_gate, int alignment, int layout, float *scores,
                     int32_t *idx, int32_t *loc, float *gates, int32_t *row, int32_t *counts, int32_t *kept_rows,

@@ -42,7 +42,8 @@ _SIGNATURES = {
     "mole_route_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
     "mole_route": (c_int, [_P, c_int, c_int, c_int, c_double, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P, _P,
                            _P, _P, c_size_t, _P]),
-    "mole_gate_route_workspace_bytes": (c_size_t, [c_int] * 5),
+    "mole_gate_route_shape_workspace_bytes": (c_size_t, [c_int] * 5),
+    "mole_gate_route_workspace_bytes": (c_size_t, [c_int] * 3),
     "mole_gate_route": (c_int, [_P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_double, c_int, c_int, c_int, _P, _P, _P, _P, _P,
                                 _P, _P, _P, _P, _P, _P, c_size_t, _P]),
     "mole_route_static_max_bytes": (c_size_t, []),

@@ -229,7 +229,7 @@ def gate_route(x: torch.Tensor, wg: torch.Tensor, logit_bias: Optional[torch.Ten
     offsets = meta[k * E + E:k * E + 2 * E + 1]
     cap = meta[k * E + 2 * E + 1:]
     l_aux = torch.empty(1, dtype=torch.float32, device=dev)
-    nbytes = L.lib().mole_gate_route_workspace_bytes(L.dtype_code(x.dtype), S, E, M, k)
+    nbytes = L.lib().mole_gate_route_shape_workspace_bytes(L.dtype_code(x.dtype), S, E, M, k)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     L.check(L.lib().mole_gate_route(L.ptr(x), L.dtype_code(x.dtype), L.ptr(wg), L.ptr(logit_bias), S, E, M, k,
                                     float(capacity_factor), int(normalize_gate), int(alignment), int(layout), L.ptr(scores),

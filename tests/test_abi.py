@@ -162,3 +162,20 @@ def test_layer_plan_rows_hold_every_kept_pair(cf):
     assert plan(cf).native.rows == want
     with pytest.raises(RuntimeError, match="finite"):
         plan(float("inf"))
+
+
+def test_gate_route_workspace_of_three_sizes():
+    """mole_gate_route_workspace_bytes(S, E, k), as programs built against its first declaration call it, covers every call
+    it is for: bf16, up to 64 experts, a width that is a multiple of 128."""
+    import torch
+    from mole_amd import _lib as L
+    lib = L.lib()
+    decl = re.search(r"mole_gate_route_workspace_bytes\(([^)]*)\)", open(os.path.join(ROOT, "include", "mole_hip.h")).read()).group(1)
+    assert [a.split()[-1] for a in decl.split(",")] == ["S", "E", "k"]
+    bf16 = L.dtype_code(torch.bfloat16)
+    for S in (1, 31, 32, 63, 64, 65, 2048, 2049, 40000):
+        for E in (1, 2, 33, 64):
+            for k in (1, min(E, 8)):
+                have = lib.mole_gate_route_workspace_bytes(S, E, k)
+                assert all(have >= lib.mole_gate_route_shape_workspace_bytes(bf16, S, E, M, k) > 0 for M in (128, 1024, 8192))
+    assert lib.mole_gate_route_workspace_bytes(-1, 4, 1) == 0 and lib.mole_gate_route_workspace_bytes(4, 0, 1) == 0
