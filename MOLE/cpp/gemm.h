@@ -66,7 +66,9 @@ __device__ __forceinline__ float d_gelu_exact(float x) {
 // as clamped odd polynomials: f(x) = v q(v^2), v = clamp(x / c, -1, 1), fitted (near-minimax, Lawson
 // iteration) to erf(x / sqrt 2) and to the odd parts of the two GELU derivatives.  Beyond the clamp the
 // functions are constant to within the stated error.  Absolute errors in fp32 Horner evaluation:
-// erf 5.8e-5, derivatives 1.8e-4 - an order of magnitude below the bf16 rounding of the result.
+// erf 5.8e-5, derivatives 1.8e-4 - an order of magnitude below the bf16 rounding of the result, except where the result
+// itself is small (gelu(-4) = -1.3e-4).  Products whose contraction is not whole stages of 32 keep the closed forms above on
+// every kernel: their loops leave the time for it, and such layers have had that accuracy from the first.
 // gelu(x) = x (1/2 + 1/2 erf(x / sqrt 2)).  The fit of erf(x / sqrt 2) is v q(v^2) in v = clamp(x / 4, -1, 1); with every
 // coefficient scaled by a power of two (c_k / (8 * 16^k): exact in binary floating point, the Horner steps round as
 // before) the same polynomial is evaluated in v = clamp(x, -4, 4) itself and delivers 1/2 erf directly:

@@ -405,7 +405,8 @@ template <int EPI> __device__ __forceinline__ void load_bias(const GemmArgs &g, 
 // per lane out, 8 rows per store instruction.  The pre-activation that GELU' needs comes in the same way,
 // in the opposite direction.  TMCW is a compile-time bound so that the work of different cells can be
 // interleaved.  live: the wave's live rows.
-template <int TMB, int WM, int WN, bool WG, int EPI, int TMC>
+// CLOSED: GELU and its derivatives by their closed forms instead of the fitted polynomials (see gemm.h).
+template <int TMB, int WM, int WN, bool WG, int EPI, int TMC, bool CLOSED>
 __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<TMB, WM, WN>::TMW][2], char *smem, int lane, int wave,
                                          int wn, int e, long row0, int m0, int n0, int m_ext, int live,
                                          const uint2 (&bias_raw)[8], int split_k) {
@@ -595,13 +596,14 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<T
                     if constexpr (EPI == EPI_BIAS_GELU) {
                         if (pass == 1) {
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) v[j] = fast_gelu_erf(v[j]);
+                            for (int j = 0; j < 4; ++j) v[j] = CLOSED ? gelu_erf(v[j]) : fast_gelu_erf(v[j]);
                         }
                     } else if constexpr (EPI == EPI_DGELU) {
                         float hv[4];
                         unpack4(*reinterpret_cast<const uint2 *>(cell), hv);
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) v[j] *= dgelu(hv[j]);
+                        for (int j = 0; j < 4; ++j)
+                            v[j] *= !CLOSED ? dgelu(hv[j]) : g.gelu_bwd == MOLE_GELU_BWD_TANH ? d_gelu_tanh(hv[j]) : d_gelu_exact(hv[j]);
                     } else if constexpr (EPI == EPI_WGRAD) {
                         if (g.accumulate) {
                             float old[4];
@@ -931,7 +933,7 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
     {                                                                                                                     \
         main_loop<TMB, WM, WN, M_KS, N_KS, KT, WM *(C), (C), SUM, ONCE, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw); \
         if constexpr (SUM != 0) store_sums<SUM, (C)>(g, sums, e, m0, n0, m_ext, wm, wn, lane);                            \
-        epilogue<TMB, WM, WN, WG, EPI, (C)>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, bias_raw, split_k);      \
+        epilogue<TMB, WM, WN, WG, EPI, (C), KT && !WG>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, bias_raw, split_k);      \
     }
 #define MOLE_RUN_TILE_SUM(C, SUM) MOLE_RUN_TILE_AS(C, SUM, false)
 #define MOLE_RUN_TILE(C) MOLE_RUN_TILE_AS(C, 0, false)

@@ -143,10 +143,11 @@ __device__ __forceinline__ void sk_epilogue4(const GemmArgs &g, int e, long row,
         for (int j = 0; j < 4; ++j) v[j] += b[j];
     }
     const long at = row * g.ldc + n;
+    const bool fitted = sizeof(T) == 2 && g.K % 32 == 0;      // (the fitted polynomials or the closed forms: see gemm.h)
     if constexpr (EPI == EPI_DGELU) {
         float h[4];
         sk_load4<T>((const T *)g.H + at, h);
-        if constexpr (sizeof(T) == 2) {
+        if (fitted) {
             DGeluCoef d;
             d.select(g.gelu_bwd == MOLE_GELU_BWD_TANH);
 #pragma unroll
@@ -159,7 +160,7 @@ __device__ __forceinline__ void sk_epilogue4(const GemmArgs &g, int e, long row,
     if constexpr (EPI == EPI_BIAS_GELU) {
         if (g.C != nullptr) sk_store4<T>((T *)g.C + at, v);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = sizeof(T) == 2 ? fast_gelu_erf(v[j]) : gelu_erf(v[j]);
+        for (int j = 0; j < 4; ++j) v[j] = fitted ? fast_gelu_erf(v[j]) : gelu_erf(v[j]);
         sk_store4<T>((T *)g.C2 + at, v);
     } else {
         sk_store4<T>((T *)g.C + at, v);

@@ -529,3 +529,51 @@ def test_forward_only_weights_leave_no_copy(E, M, k, S, dtype):
     with torch.no_grad():
         assert torch.equal(m(x, capacity_factor=0.0), y)
     MOLEModule.reset_instances()
+
+
+# bf16 widths that are multiples of 8 but not of 32: the activation by the closed forms on every kernel that takes them - 256 x
+# 256 tiles (many rows and columns), 128 x 128 tiles, few rows - on every bf16 value of magnitude 2^-14 .. 8.  Error of the
+# closed form 2e-6 of max(1, |h|) as in fp32 (erf and exp to a few units of fp32, amplified at most by |h|), and the result's
+# rounding; -inf gives what 0 * inf gives, a NaN stays one in the derivative too.
+@pytest.mark.parametrize("M,Fd,per", [(72, 29992, 1 << 20), (72, 264, 1 << 20), (200, 264, 7)])
+def test_activation_at_ragged_widths_is_the_closed_form(M, Fd, per):
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"closed-form activation M={M} F={Fd} rows per expert {per}", flush=True)
+    dtype, grid = torch.bfloat16, _bf16_grid()
+    rows = (grid.numel() + M - 1) // M
+    vals = torch.zeros(rows * M)
+    vals[:grid.numel()] = grid
+    xd = vals.view(rows, M).to(dtype).cuda()
+    n = [min(per, rows - lo) for lo in range(0, rows, per)]
+    E = len(n)
+    off = torch.tensor([0] + n).cumsum(0).int().cuda()
+    n = torch.tensor(n).int().cuda()
+    w1, w2 = (torch.zeros(E, Fd, M, dtype=dtype, device="cuda") for _ in range(2))
+    w1[:, torch.arange(Fd), torch.arange(Fd) % M] = 1.0          # h[r, f] = xd[r, f mod M]
+    w2[:, :, 0] = 1.0                                             # (go . w2^T)[r, f] = go[r, 0]
+    b1, b2 = torch.zeros(E, Fd, dtype=dtype, device="cuda"), torch.zeros(E, M, dtype=dtype, device="cuda")
+    go = torch.zeros(rows, M, dtype=dtype, device="cuda")
+    go[:, 0] = 1.0
+    out, h, a = H.ffn_fwd(xd, off, n, w1, b1, w2, b2)
+    assert torch.equal(h, xd[:, torch.arange(Fd) % M])
+    assert torch.equal(a[:, :M].repeat(1, Fd // M + 1)[:, :Fd], a)
+    h64 = h[:, :M].double().cpu()
+
+    def check(got, want, what):
+        slack = 2e-6 * h64.abs().clamp(min=1.0)
+        half_ulp = torch.pow(2.0, torch.floor(torch.log2((want.abs() + slack).clamp(min=2.0 ** -126))) - 8)
+        err = (got[:, :M].double().cpu() - want).abs()
+        assert bool((err <= slack + half_ulp).all()), f"{what}: {float((err / (slack + half_ulp)).max()):.1f}x its bound"
+
+    check(a, 0.5 * h64 * (1.0 + torch.erf(h64 / 2.0 ** 0.5)), "GELU")
+    g = [torch.empty_like(v) for v in (w1, b1, w2, b2)]
+    t = torch.empty(rows, Fd, dtype=dtype, device="cuda")
+    for fn, code in ((O.d_gelu_tanh, L.GELU_BWD_TANH), (O.d_gelu_exact, L.GELU_BWD_EXACT)):
+        H.ffn_bwd_into(go, xd, h, a, off, n, E, rows, M, Fd, w1, w2, t, *g, None, False, code)
+        assert torch.equal(t[:, :M].repeat(1, Fd // M + 1)[:, :Fd], t)
+        check(t, fn(h64), "GELU'")
+    b1[:, 0], b1[:, 1] = -float("inf"), float("nan")
+    out, h, a = H.ffn_fwd(xd, off, n, w1, b1, w2, b2)
+    assert bool(a[:, :2].isnan().all()) and bool(a[:, 2:].isfinite().all())
+    H.ffn_bwd_into(go, xd, h, a, off, n, E, rows, M, Fd, w1, w2, t, *g, None, False, L.GELU_BWD_TANH)
+    assert bool(t[:, :2].isnan().all()) and bool(t[:, 2:].isfinite().all())
