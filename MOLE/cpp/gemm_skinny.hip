@@ -41,6 +41,10 @@ template <typename T> __device__ __forceinline__ sk_f32x4 sk_mma(uint4 w, uint4 
     }
 }
 
+__device__ __forceinline__ void sk_mask(uint4 &v, uint32_t keep) {
+    v = make_uint4(v.x & keep, v.y & keep, v.z & keep, v.w & keep);
+}
+
 // q[kk] = EPC consecutive columns of k-row kk; f[j] = the EPC k of column j
 __device__ __forceinline__ void sk_transpose(const uint4 (&q)[8], uint4 (&f)[8]) {
     const uint32_t w[8][4] = {{q[0].x, q[0].y, q[0].z, q[0].w}, {q[1].x, q[1].y, q[1].z, q[1].w},
@@ -191,7 +195,8 @@ __device__ __forceinline__ void skinny_kc_run(const GemmArgs &g, sk_f32x4 (&red)
 #pragma unroll
         for (int b = 0; b < MB; ++b) acc[a][b] = sk_f32x4{0.f, 0.f, 0.f, 0.f};
     uint4 w[U][NA], x[U][MB];
-    // steps past the wave's share repeat its last one; they, and k past the contraction's end, are masked to zero
+    // (steps past the wave's share repeat its last one and are not multiplied; of a step that the contraction ends in, the lanes
+    // past its end are masked on both sides: a weight that is no number times zero would be none)
     auto fetch = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -206,13 +211,18 @@ __device__ __forceinline__ void skinny_kc_run(const GemmArgs &g, sk_f32x4 (&red)
     auto use = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const uint32_t keep = (s + u < s_hi && (s + u) * KSTEP + kg * EPC < g.K) ? 0xffffffffu : 0u;
+            if (s + u >= s_hi) break;
+            if ((s + u + 1) * KSTEP > g.K) {
+                const uint32_t keep = (s + u) * KSTEP + kg * EPC < g.K ? 0xffffffffu : 0u;
 #pragma unroll
-            for (int b = 0; b < MB; ++b) {
-                const uint4 xv = make_uint4(x[u][b].x & keep, x[u][b].y & keep, x[u][b].z & keep, x[u][b].w & keep);
+                for (int a = 0; a < NA; ++a) sk_mask(w[u][a], keep);
 #pragma unroll
-                for (int a = 0; a < NA; ++a) acc[a][b] = sk_mma<T>(w[u][a], xv, acc[a][b]);
+                for (int b = 0; b < MB; ++b) sk_mask(x[u][b], keep);
             }
+#pragma unroll
+            for (int b = 0; b < MB; ++b)
+#pragma unroll
+                for (int a = 0; a < NA; ++a) acc[a][b] = sk_mma<T>(w[u][a], x[u][b], acc[a][b]);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -282,15 +292,19 @@ __device__ __forceinline__ void skinny_ks_run(const GemmArgs &g, sk_f32x4 (&red)
         __builtin_amdgcn_sched_barrier(0);
     };
     auto use = [&](int s) __attribute__((always_inline)) {
-        const uint32_t keep = s * KSTEP + kg * EPC < g.K ? 0xffffffffu : 0u;
+        if ((s + 1) * KSTEP > g.K) {       // the step that the contraction ends in: as for the other layout
+            const uint32_t keep = s * KSTEP + kg * EPC < g.K ? 0xffffffffu : 0u;
+#pragma unroll
+            for (int q = 0; q < EPC; ++q) sk_mask(w[q], keep);
+#pragma unroll
+            for (int b = 0; b < MB; ++b) sk_mask(x[b], keep);
+        }
         uint4 f[EPC];
         sk_transpose(w, f);
 #pragma unroll
-        for (int b = 0; b < MB; ++b) {
-            const uint4 xv = make_uint4(x[b].x & keep, x[b].y & keep, x[b].z & keep, x[b].w & keep);
+        for (int b = 0; b < MB; ++b)
 #pragma unroll
-            for (int j = 0; j < EPC; ++j) acc[j][b] = sk_mma<T>(f[j], xv, acc[j][b]);
-        }
+            for (int j = 0; j < EPC; ++j) acc[j][b] = sk_mma<T>(f[j], x[b], acc[j][b]);
         __builtin_amdgcn_sched_barrier(0);
     };
     for (int s = s_lo; s < s_hi; ++s) {

@@ -577,3 +577,48 @@ def test_activation_at_ragged_widths_is_the_closed_form(M, Fd, per):
     assert bool(a[:, :2].isnan().all()) and bool(a[:, 2:].isfinite().all())
     H.ffn_bwd_into(go, xd, h, a, off, n, E, rows, M, Fd, w1, w2, t, *g, None, False, L.GELU_BWD_TANH)
     assert bool(t[:, :2].isnan().all()) and bool(t[:, 2:].isfinite().all())
+
+
+def _same_class(got, want):
+    """the same numbers, infinities of the same sign and NaNs in the same places (finite values are compared elsewhere)"""
+    got, want = got.double().cpu(), want.double().cpu()
+    code = lambda t: torch.where(t.isnan(), 3.0, torch.where(t.isposinf(), 1.0, torch.where(t.isneginf(), 2.0, 0.0)))
+    return bool((code(got) == code(want)).all())
+
+
+# Few-row products with an infinite weight: every row of the expert gets what fp32 arithmetic gives, an infinity of the right sign
+# where the terms are one infinity and finite numbers.  Contractions of odd numbers of steps, ending inside a step, shorter
+# than the waves of a block; the weight in the last piece of the contraction, in its last step and in its middle.  (Rows are
+# kept from zero; the other column's term is finite.)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("E,M,Fd,rows", [(1, 520, 776, [9]), (4, 264, 520, [12, 12, 1, 0]), (2, 768, 2064, [3, 40]), (3, 96, 1544, [5, 24, 17])])
+def test_ffn_few_rows_with_infinite_weights(E, M, Fd, rows, dtype):
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"few rows, infinite weights E={E} M={M} F={Fd} {dtype}", flush=True)
+    d = _make(E, M, Fd, rows, dtype, seed=M)
+    for name in ("xd", "go"):
+        d[name] = torch.where(d[name].abs() < 0.1, torch.full_like(d[name], 0.1), d[name])
+    off, n = torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda()
+    g = [torch.empty_like(d[q]).cuda() for q in ("w1", "b1", "w2", "b2")]
+    owner = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))
+    inf, R = float("inf"), d["R"]
+    c = {q: (v.cuda() if torch.is_tensor(v) else v) for q, v in d.items()}
+    for at in (lambda K: K - 1, lambda K: K - 9, lambda K: K // 2):
+        for sign in (inf, -inf):
+            w1, w2 = d["w1"].clone(), d["w2"].clone()
+            w1[:, 5, at(M)], w2[:, at(Fd), 7] = sign, sign
+            # h = xd.w1^T, and through the second product a finite activation on the infinite weight
+            _, h, a = H.ffn_fwd(c["xd"], off, n, w1.cuda(), c["b1"], c["w2"], c["b2"])
+            want = torch.einsum("rm,rfm->rf", d["xd"].double(), w1.double()[owner]) + d["b1"].double()[owner]
+            assert _same_class(h, want)
+            out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], w2.cuda(), c["b2"])
+            want = torch.einsum("rf,rfm->rm", a.double().cpu(), w2.double()[owner]) + d["b2"].double()[owner]
+            assert _same_class(out, want)
+            # t = (go.w2^T) gelu'(h), gx = t.w1 with t finite
+            t, gx = torch.empty(R, Fd, dtype=dtype, device="cuda"), torch.empty(R, M, dtype=dtype, device="cuda")
+            H.ffn_bwd_into(c["go"], c["xd"], h, a, off, n, E, R, M, Fd, c["w1"], w2.cuda(), t, *g, None, False, L.GELU_BWD_EXACT)
+            want = torch.einsum("rm,rfm->rf", d["go"].double(), w2.double()[owner]) * O.d_gelu_exact(h.double().cpu())
+            assert _same_class(t, want)
+            H.ffn_bwd_into(c["go"], c["xd"], h, a, off, n, E, R, M, Fd, w1.cuda(), c["w2"], t, *g, gx, False, L.GELU_BWD_EXACT)
+            want = torch.einsum("rf,rfm->rm", t.double().cpu(), w1.double()[owner])
+            assert _same_class(gx, want)
