@@ -219,17 +219,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> layer(const Tensor &x, const Tensor &
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     py::class_<Counter, std::shared_ptr<Counter>>(m, "Counter")
         .def(py::init<int64_t>())
-        .def_property("value", [](const Counter &c) { return c.value.load(); }, [](Counter &c, int64_t v) { c.value = v; })
-        .def(py::pickle([](const Counter &c) { return py::make_tuple(c.value.load()); },
-                        [](py::tuple t) { return std::make_shared<Counter>(t[0].cast<int64_t>()); }));
+        .def_property("value", [](const Counter &c) { return c.value.load(); }, [](Counter &c, int64_t v) { c.value = v; });
     py::class_<Plan, std::shared_ptr<Plan>>(m, "Plan")
         .def(py::init<int, int64_t, int64_t, int64_t, int64_t, int64_t, double, int, bool, int>())
         .def("route_offsets", &Plan::route_offsets)
-        .def_property_readonly("rows", [](const Plan &p) { return p.head.rows; })
-        .def(py::pickle([](const Plan &p) { return py::make_tuple(p.head.dtype, p.head.S, p.head.M, p.head.E, p.head.k, p.head.F,
-                                                                  p.head.capacity_factor, p.head.layout, p.head.normalize_gate, p.gelu_bwd); },
-                        [](py::tuple t) { return std::make_shared<Plan>(t[0].cast<int>(), t[1].cast<int64_t>(), t[2].cast<int64_t>(),
-                                              t[3].cast<int64_t>(), t[4].cast<int64_t>(), t[5].cast<int64_t>(), t[6].cast<double>(),
-                                              t[7].cast<int>(), t[8].cast<int>() != 0, t[9].cast<int>()); }));
+        .def_property_readonly("rows", [](const Plan &p) { return p.head.rows; });
     m.def("layer", &layer, py::call_guard<py::gil_scoped_release>());
 }

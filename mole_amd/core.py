@@ -445,6 +445,17 @@ class MOLECore:
     def step(self, v: int):
         self.passes.value = int(v)
 
+    # (pickled with the count itself: the native counter's type has no importable name)
+    def __getstate__(self):
+        state = dict(self.__dict__)
+        state["step"] = state.pop("passes").value
+        return state
+
+    def __setstate__(self, state):
+        state = dict(state)
+        self.passes = L.native().Counter(state.pop("step"))
+        self.__dict__.update(state)
+
     # the reference's counters of experts prefetched so far (define.hpp:352-353)
     @property
     def fwd_base(self) -> int:

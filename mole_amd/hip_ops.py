@@ -434,6 +434,10 @@ class LayerPlan:
     def __init__(self, dtype, S, M, E, k, F, capacity_factor, layout, normalize_gate, gelu_bwd):
         self.S, self.E, self.k, self.layout, self.normalize_gate = S, E, k, layout, normalize_gate
         self.native = L.native().Plan(L.dtype_code(dtype), S, M, E, k, F, capacity_factor, layout, normalize_gate, gelu_bwd)
+        self._sizes = (dtype, S, M, E, k, F, capacity_factor, layout, normalize_gate, gelu_bwd)
+
+    def __reduce__(self):        # (the native plan's type has no importable name: a copy is made from the sizes)
+        return LayerPlan, self._sizes
 
     def route(self, buf: torch.Tensor, l_aux: torch.Tensor) -> Route:
         offs = iter(self.native.route_offsets())

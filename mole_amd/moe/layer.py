@@ -215,6 +215,12 @@ class MOLEModule(torch.nn.Module):
         self.moe_id = len(MOLEModule._instance)
         MOLEModule._instance.append(self)
 
+    def __setstate__(self, state):       # a layer pickled with its last routing as a plain attribute has no plans
+        super().__setstate__(state)
+        self.__dict__.setdefault("_route", self.__dict__.pop("last_route", None))
+        self.__dict__.setdefault("_plans", {})
+        self.__dict__.setdefault("_granule", 8 if self.param_dtype == torch.bfloat16 else 4)
+
     # ---- results of the last forward besides its output ---------------------------------------
     @property
     def last_route(self):

@@ -179,3 +179,33 @@ def test_gate_route_workspace_of_three_sizes():
                 have = lib.mole_gate_route_workspace_bytes(S, E, k)
                 assert all(have >= lib.mole_gate_route_shape_workspace_bytes(bf16, S, E, M, k) > 0 for M in (128, 1024, 8192))
     assert lib.mole_gate_route_workspace_bytes(-1, 4, 1) == 0 and lib.mole_gate_route_workspace_bytes(4, 0, 1) == 0
+
+
+def test_core_and_plans_travel_through_pickle(tmp_path):
+    """Copies and pickles of a layer's core and of its plans, read by a process that has loaded neither library; a state that
+    holds the number of passes as plain integer (as these do) is also what earlier cores were pickled with."""
+    import copy
+    import pickle
+    import subprocess
+    import sys
+    import torch
+    from mole_amd import _lib as L, core, hip_ops as H
+    from mole_amd.moe.layer import MOLEModule
+    c = core.MOLECore(False, False, False, False, 4, 0, 4, 1, "gelu", False, 2, 5, 0, 0, 4)
+    plan = H.LayerPlan(torch.bfloat16, 64, 128, 4, 2, 256, 1.25, L.LAYOUT_PADDED, True, 1)
+    assert type(c.__getstate__()["step"]) is int
+    d = copy.deepcopy(c)
+    c.step += 1
+    assert (c.step, d.step) == (6, 5)
+    path = tmp_path / "state.pkl"
+    path.write_bytes(pickle.dumps((c, plan)))
+    code = ("import pickle, sys; c, p = pickle.load(open(sys.argv[1], 'rb'))\n"
+            "c.step += 1; print(c.step, c.acc_step, c.passes.value, p.native.rows, p.native.route_offsets() == p.__reduce__()[0](*p.__reduce__()[1]).native.route_offsets())")
+    r = subprocess.run([sys.executable, "-c", code, str(path)], capture_output=True, text=True, cwd=ROOT)
+    assert r.returncode == 0, r.stderr
+    assert r.stdout.split() == ["7", "2", "7", str(plan.native.rows), "True"]
+    # a layer whose state has its last routing as a plain attribute, and no plans
+    m = MOLEModule.__new__(MOLEModule)
+    torch.nn.Module.__init__(m)
+    m.__setstate__(dict(m.__dict__, param_dtype=torch.bfloat16, last_route="route"))
+    assert m.last_route == "route" and m._plans == {} and m._granule == 8
