@@ -1094,7 +1094,8 @@ __global__ __launch_bounds__(256) void gate_fwd_kernel(const bf16_t *__restrict_
 // gate_fwd_kernel (whose logits these equal bit for bit where it applies: bf16, M a multiple of 128).  One block per
 // 16-expert group instead of one that reads all of Wg: 512 KB of Wg for one token is then 4 blocks' work side by side
 // instead of one block's 20 us, and 256 tokens x 256 experts x 2048 are 256 blocks (10 us; one 256 x 256 tile: 54).
-// Fragments come straight from memory; k past the end is masked to zero on the token side.
+// Fragments come straight from memory.  Steps past a wave's share repeat its last one and are not multiplied; of a step
+// that M ends in, the lanes past the end are zero on both sides (an infinite weight times zero would be NaN).
 template <typename T, int TG>
 __global__ __launch_bounds__(256) void gate_logits_kernel(const T *__restrict__ x, const float *__restrict__ wg,
                                                           const float *__restrict__ bias, int S, int E, int M,
@@ -1126,10 +1127,16 @@ __global__ __launch_bounds__(256) void gate_logits_kernel(const T *__restrict__ 
         __builtin_amdgcn_sched_barrier(0);       // all loads of the round first
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const uint32_t keep = (s + u < s_hi && (s + u) * KSTEP + kq * EPC < M) ? 0xffffffffu : 0u;
+            if (s + u >= s_hi) break;
+            if ((s + u + 1) * KSTEP > M && (s + u) * KSTEP + kq * EPC >= M) {
+#pragma unroll
+                for (int t = 0; t < TG; ++t) a[t][u] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+                for (int h = 0; h < EPC / 4; ++h) w[u][h] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
 #pragma unroll
             for (int t = 0; t < TG; ++t) {
-                const uint4 v = make_uint4(a[t][u].x & keep, a[t][u].y & keep, a[t][u].z & keep, a[t][u].w & keep);
+                const uint4 v = a[t][u];
                 if constexpr (sizeof(T) == 2) {
                     const float4 w0 = w[u][0], w1 = w[u][EPC / 4 - 1];
                     const gate_bf16x8 b = {(bf16_t)w0.x, (bf16_t)w0.y, (bf16_t)w0.z, (bf16_t)w0.w,

@@ -259,3 +259,24 @@ def test_gate_and_route_other_shapes(S, E, M, k, cf, bias, ragged, dtype):
         np.testing.assert_array_equal(a[name], b[name], err_msg=name)
     assert a["capacity"] == b["capacity"]
     assert abs(a["l_aux"] - b["l_aux"]) <= 1e-5 * max(1.0, abs(b["l_aux"]))
+
+
+# An infinite weight in the logits' 16 x 16 tiles: its expert's logit is an infinity, of the sign that the (positive) tokens
+# leave it, and -inf takes the expert out of the softmax.  Widths of fewer steps than the four waves take in a round, whole and
+# ragged; the weight in the last piece, in the last step and in the middle.  Tolerance as for the finite scores above.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("S,E,M", [(1, 5, 72), (65, 17, 128), (300, 40, 264), (513, 9, 520), (2048, 8, 512)])
+def test_gate_logits_with_an_infinite_weight(S, E, M, dtype):
+    from mole_amd import hip_ops as H
+    print(f"gate logits, infinite weight S={S} E={E} M={M} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(S + M)
+    x = (torch.rand(S, M, generator=g) + 0.1).to(dtype)
+    for at in (M - 1, M - 9, M // 2):
+        wg = torch.randn(E, M, generator=g) * 0.05
+        wg[2, at] = float("-inf")
+        scores, _ = H.gate_route(x.cuda(), wg.cuda(), None, 2, 0.0, True, 1)
+        want = torch.softmax(x.double() @ wg.to(dtype).double().t(), 1)
+        assert bool((scores[:, 2] == 0).all()) and rel_err(scores.cpu(), want) < 1e-5
+        wg[2, at] = float("inf")       # inf - inf in the softmax of every token
+        scores, _ = H.gate_route(x.cuda(), wg.cuda(), None, 2, 0.0, True, 1)
+        assert bool(scores[:, 2].isnan().all())
