@@ -446,6 +446,12 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
 #pragma unroll
                 for (int p = 0; p <= order; ++p)
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfrag[p][cb], afrag[order - p], acc, 0, 0, 0);
+            if constexpr (SPLIT) {
+                // the parts of an infinity are the infinity and NaN: where the leading product is not finite, it is the result
+                const perm_f32x4 lead = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfrag[0][cb], afrag[0], perm_f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[r] = fabsf(lead[r]) < INFINITY ? acc[r] : lead[r];
+            }
             *reinterpret_cast<perm_f32x4 *>(buf + r16 * DM_ROW + 16 * cb + 4 * kq) = acc;
         }
         // (a wave's LDS buffer is written and read by that wave only: program order is enough)

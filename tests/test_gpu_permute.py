@@ -206,3 +206,32 @@ def test_gate_wgrad_short_blocks(S, E, M, dtype):
     want = dl.double().t() @ x.double()
     got = H.gate_wgrad(dl.cuda(), x.cuda()).double().cpu()
     assert float((got - want).norm() / want.norm()) < 2e-5
+
+
+# The gate's share of dx at ragged bf16 widths with infinite operands: a weight, and a gradient, each +-inf, give infinities of
+# the sign that the (non-zero) other operand leaves them, a NaN gives NaN, and the columns and tokens beside them stay finite.
+@pytest.mark.parametrize("S,E,k,M", [(17, 3, 1, 72), (513, 16, 2, 520), (7000, 32, 1, 2888)])
+def test_dispatch_bwd_with_gate_ragged_widths_not_finite(S, E, k, M):
+    from mole_amd import hip_ops as H
+    print(f"dispatch_bwd+gate not finite S={S} E={E} k={k} M={M}", flush=True)
+    g = torch.Generator().manual_seed(S + M)
+    away = lambda t: torch.where(t.abs() < 0.1, torch.full_like(t, 0.1), t)
+    dlog, wg = away(torch.randn(S, E, generator=g)), away(torch.randn(E, M, generator=g))
+    for t in (dlog, wg):
+        t[:, -1] = t[:, -1].bfloat16().float()          # (values whose remainder is zero)
+    row = torch.full((k, S), -1, dtype=torch.int32)
+    dxd = torch.randn(S * k, M, generator=g).bfloat16()
+    for bad in (float("inf"), float("-inf"), float("nan")):
+        for which in (0, 1):
+            d, w = dlog.clone(), wg.clone()
+            if which:
+                w[E - 1, 5], w[0, M - 1] = bad, bad
+            else:
+                d[S // 2, 1], d[S - 1, E - 1] = bad, bad
+            got = H.dispatch_bwd(dxd.cuda(), row.cuda(), d.cuda(), w.cuda()).double().cpu()
+            want = d.double() @ w.double()
+            assert torch.equal(got.isnan(), want.isnan())
+            assert torch.equal(got.isposinf(), want.isposinf()) and torch.equal(got.isneginf(), want.isneginf())
+            fin = want.isfinite()
+            terms = dlog.double().abs() @ wg.double().abs()
+            assert bool(((got - want).abs()[fin] <= (2.0 ** -8 * want.abs() + (2.0 ** -23 + 6 * 32 * 2.0 ** -24) * terms)[fin]).all())
