@@ -367,8 +367,9 @@ template <typename T>
 __global__ __launch_bounds__(256) void plane_reduce_kernel(const GemmArgs g) {
     int e, grp, rows;
     long row0;
-    if (!sk_find_group<RED_ROWS>(g, blockIdx.y, e, grp, rows, row0)) return;
-    const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
+    const int chunks = (g.N + 1023) / 1024;
+    if (!sk_find_group<RED_ROWS>(g, blockIdx.x / chunks, e, grp, rows, row0)) return;
+    const int n = (blockIdx.x % chunks * 256 + threadIdx.x) * 4;
     if (n >= g.N) return;
     const long plane = g.part_rows * g.N;
     const int m0 = grp * RED_ROWS;
@@ -451,7 +452,8 @@ int gemm_skinny_ksplit(int E, int est_rows, int N, int K, int dtype) {
 }
 
 int launch_plane_reduce(const GemmArgs &g, int dtype, int max_rows, hipStream_t st) {
-    const dim3 grid(ceil_div(g.N, 1024), (g.E < max_rows ? g.E : max_rows) + max_rows / RED_ROWS);
+    // (the row groups are counted in x: y ends at 65535 blocks, which 262144 rows of a narrow layer reach)
+    const dim3 grid((unsigned)((g.E < max_rows ? g.E : max_rows) + max_rows / RED_ROWS) * (unsigned)ceil_div(g.N, 1024));
     if (dtype == MOLE_BF16) hipLaunchKernelGGL(plane_reduce_kernel<bf16_t>, grid, dim3(256), 0, st, g);
     else hipLaunchKernelGGL(plane_reduce_kernel<float>, grid, dim3(256), 0, st, g);
     MOLE_LAUNCH_CHECK();

@@ -622,3 +622,24 @@ def test_ffn_few_rows_with_infinite_weights(E, M, Fd, rows, dtype):
             H.ffn_bwd_into(c["go"], c["xd"], h, a, off, n, E, R, M, Fd, w1.cuda(), c["w2"], t, *g, gx, False, L.GELU_BWD_EXACT)
             want = torch.einsum("rf,rfm->rm", t.double().cpu(), w1.double()[owner])
             assert _same_class(gx, want)
+
+
+def test_ffn_split_contraction_of_more_than_2_to_18_rows():
+    """The reduction of a split contraction has a block for every four rows: more of them than a grid has in y.  fp32, rows of
+    eight columns; out against torch's fp32 products of the same activations (two orders of 1024 terms: 2^-24 sqrt(1024) of
+    the terms' norm each)."""
+    from mole_amd import hip_ops as H, _lib as L
+    E, per, M, Fd = 4, 70000, 8, 1024
+    R = E * per
+    assert L.lib().mole_ffn_workspace_bytes(L.MOLE_F32, E, R, M, Fd) >= 2 * R * M * 4 and R / 4 > 65535
+    print(f"split contraction, {R} rows", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    new = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    xd, w1, b1, w2, b2 = new(R, M), new(E, Fd, M), new(E, Fd), new(E, Fd, M), new(E, M)
+    off = torch.arange(E + 1, dtype=torch.int32, device="cuda") * per
+    n = torch.full((E,), per, dtype=torch.int32, device="cuda")
+    out, _, a = H.ffn_fwd(xd, off, n, w1, b1, w2, b2)
+    for e in range(E):
+        ae, got = a[e * per:(e + 1) * per], out[e * per:(e + 1) * per]
+        terms = (ae.norm(dim=1, keepdim=True) * w2[e].abs().max()) + b2[e].abs().max()
+        assert bool(((got - (ae @ w2[e] + b2[e])).abs() <= 4 * 2.0 ** -24 * 32 * terms).all())
