@@ -568,6 +568,7 @@ size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, 
     if (E <= 0 || max_rows <= 0 || M <= 0 || F <= 0) return 0;
     int ks = gemm_skinny_ksplit(E, est_rows, M, F, dtype);
     if (ks == 0) ks = dtype == MOLE_BF16 ? gemm256_ksplit(E, est_rows, M, F) : gemm_f32_ksplit(E, est_rows, M, F);
+    ks = planes_allowed(ks, max_rows, est_rows, M);
     return ks > 1 ? (size_t)ks * max_rows * M * sizeof(float) : 0;
 }
 

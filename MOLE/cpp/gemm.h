@@ -164,6 +164,14 @@ int gemm256_ksplit(int E, int est_rows, int N, int K);
 // out = sum of the planes (+ bias), for the rows of g's experts (gemm_skinny.hip)
 int launch_plane_reduce(const GemmArgs &g, int dtype, int max_rows, hipStream_t st);
 bool gemm256_sums_operand(const GemmArgs &g);
+// Planes of a split that asks for ks.  A plane has a row for every row of the launch's buffers, also where few of them are
+// used: the padded layout holds E C rows however few are routed (1 token, top-2 of 256 experts, capacity factor 2,
+// 2048 -> 4096: 1024 rows for 2, 67 MB in eight planes).  Beyond four times the rows that can be used, 32 MB in all.
+inline int planes_allowed(int ks, int max_rows, int est_rows, int N) {
+    if (max_rows <= 4ll * est_rows) return ks;
+    const long long fit = (32ll << 20) / ((long long)max_rows * N * (long long)sizeof(float));
+    return fit < 2 ? 1 : (ks < fit ? ks : (int)fit);
+}
 // Few rows per expert (gemm_skinny.hip): weights streamed straight into fragments; -100 when the shape is not its.
 int launch_gemm_skinny(const GemmArgs &g, int dtype, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
 int gemm_skinny_ksplit(int E, int est_rows, int N, int K, int dtype);    // 0: not its shape

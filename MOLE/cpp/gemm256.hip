@@ -1127,6 +1127,7 @@ int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, in
     if (wg && (!a_ks || !b_ks || g.M % 8)) return -100;
     TilePlan p{TILE_256, 1};
     if (!wg && g.offsets != nullptr && epi < EPI_NONE) p = tile_plan(g.E, g.est_rows, g.N, g.K, b_ks);
+    p.ksplit = planes_allowed(p.ksplit, max_rows, g.est_rows, g.N);
     if (wg && epi == EPI_WGRAD) p.tile = wgrad_tile(g.E, g.M, g.N);
     GemmArgs gp = g;
     gp.ksplit = 1;

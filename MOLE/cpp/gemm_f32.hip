@@ -550,7 +550,7 @@ int launch_gemm_f32(const GemmArgs &g0, bool a_ks, bool b_ks, bool wg, int epi, 
     const int rows = g.offsets ? max_rows : g.single_rows;
     const long tiles = (long)ceil_div(rows, 64) * ceil_div(g.N, 128);
     if (b_ks && g.offsets != nullptr && ws != nullptr) {
-        const int p = plan_ksplit(g.E, g.est_rows, g.N, g.K);
+        const int p = planes_allowed(plan_ksplit(g.E, g.est_rows, g.N, g.K), max_rows, g.est_rows, g.N);
         if (p > 1 && ws_bytes >= (size_t)p * max_rows * g.N * sizeof(float)) {
             g.ksplit = p;
             g.part = (float *)ws;

@@ -489,6 +489,7 @@ int launch_gemm_skinny(const GemmArgs &g0, int dtype, bool b_ks, int epi, int ma
     const int groups = (g.E < max_rows ? g.E : max_rows) + max_rows / (16 * p.mb);     // as many as max_rows rows can need
     if (g.K % epc || g.N % epc || g.lda % epc || g.ldb % epc || g.ldc % epc || g.strideB % epc) return -100;
     g.ksplit = 1;
+    p.ksplit = planes_allowed(p.ksplit, max_rows, g.est_rows, g.N);
     if (p.ksplit > 1 && ws != nullptr && ws_bytes >= (size_t)p.ksplit * max_rows * g.N * sizeof(float)) {
         g.ksplit = p.ksplit;
         g.part = (float *)ws;

@@ -209,3 +209,26 @@ def test_core_and_plans_travel_through_pickle(tmp_path):
     torch.nn.Module.__init__(m)
     m.__setstate__(dict(m.__dict__, param_dtype=torch.bfloat16, last_route="route"))
     assert m.last_route == "route" and m._plans == {} and m._granule == 8
+
+
+def test_planes_of_a_padded_layout_stay_bounded():
+    """Scratch of the layer's split contractions where the padded layout has many more slots than rows: 32 MB of planes at most
+    (or none), beside the few bytes of the gate; as many as the ragged layout's where the slots are near the rows."""
+    import struct
+    from mole_amd import _lib as L
+    import ctypes
+    lib = L.lib()
+
+    def workspace(S, M, E, k, F, rows, layout, backward=0):
+        block = ctypes.create_string_buffer(struct.pack("10id", L.MOLE_BF16, S, M, E, k, F, rows, layout, 1, 0, 1.0), 512)
+        return lib.mole_layer_workspace_bytes(ctypes.cast(block, ctypes.c_void_p), backward)
+
+    def gate(S, M, E, k):
+        return lib.mole_gate_route_shape_workspace_bytes(L.MOLE_BF16, S, E, M, k)
+
+    assert gate(1, 2048, 256, 2) < 1 << 20
+    assert 1 << 20 < workspace(1, 2048, 256, 2, 4096, 1024, L.LAYOUT_PADDED) <= 32 << 20        # eight planes: 67 MB
+    assert workspace(4096, 512, 64, 2, 2048, 524288, L.LAYOUT_PADDED) <= max(32 << 20, gate(4096, 512, 64, 2))   # two: 2.1 GB
+    assert workspace(1, 8192, 256, 2, 4096, 4096, L.LAYOUT_PADDED) <= 1 << 20                   # not one plane fits
+    ragged, padded = workspace(3001, 1024, 16, 2, 4096, 6002, L.LAYOUT_RAGGED), workspace(3001, 1024, 16, 2, 4096, 7520, L.LAYOUT_PADDED)
+    assert ragged > 32 << 20 and ragged * 7520 == padded * 6002
