@@ -418,9 +418,10 @@ static bool skinny_plan(int dtype, bool b_ks, int E, int est_rows, int N, int K,
     // where the token loads, one per four weight loads and 16 rows, begin to cost (8 experts of 512 -> 2048, 600 rows:
     // 18 against 14 us); KS, eight weight loads each, at 64 (16 x 1024 -> 4096, 400 / 800 / 1600 rows: 39 / 50 / 79
     // against 55 / 61 / 75 us).
-    // fp32: the 64 x 128 tiles of gemm_f32.hip walk the whole contraction in one block, however few rows there are
-    // (out at 16 x 1024 -> 4096: 128 us from 2 to 800 rows); 244 / 400 / 800 / 1600 rows: 59 / 75 / 102 / 157 against
-    // 127 / 127 / 128 / 137 us.  KC: 244 / 400 rows 69 / 84 against 75 / 78 us.
+    // fp32: the 64 x 128 tiles of gemm_f32.hip, with their planes, from 48 rows per expert on, where also evenly spread rows
+    // need more than one group of 32 and the fuller experts of a skewed routing many, each reading the weights again
+    // (16 experts of 1024 -> 4096, forward pass, tiles / here: 800 rows 190 / 225 us, skewed 295 / 318; 960 rows 302 / 329;
+    // 640 rows here 204, skewed 277).  KC: 244 / 400 rows 69 / 84 against 75 / 78 us.
     bool takes;
     if (bf16) {
         const long tiles = (long)active * ceil_div(avg, 256) * ceil_div(N, 256);
@@ -430,7 +431,7 @@ static bool skinny_plan(int dtype, bool b_ks, int E, int est_rows, int N, int K,
         // against 58, planes added; 20 of 2264 -> 9056, 20 rows: 304 against 153)
         if (b_ks && avg > 16 && (size_t)active * N * K * sizeof(bf16_t) > (size_t)256 << 20) takes = false;
     } else {
-        takes = avg <= (b_ks ? 64 : 20);
+        takes = avg <= (b_ks ? 48 : 20);
     }
     if (!takes) return false;
     // rows per group: KC shares a block's weight loads among 32 rows once experts hold more than eight; KS in bf16 has

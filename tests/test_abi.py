@@ -232,3 +232,11 @@ def test_planes_of_a_padded_layout_stay_bounded():
     assert workspace(1, 8192, 256, 2, 4096, 4096, L.LAYOUT_PADDED) <= 1 << 20                   # not one plane fits
     ragged, padded = workspace(3001, 1024, 16, 2, 4096, 6002, L.LAYOUT_RAGGED), workspace(3001, 1024, 16, 2, 4096, 7520, L.LAYOUT_PADDED)
     assert ragged > 32 << 20 and ragged * 7520 == padded * 6002
+
+
+def test_fp32_products_leave_the_few_row_kernel_at_48_rows():
+    """Beyond 48 rows per expert the tiles with split contractions are the faster ones; the few-row kernel has blocks enough
+    there without a split, and no workspace."""
+    from mole_amd import _lib as L
+    ws = lambda rows: L.lib().mole_ffn_workspace_bytes(L.MOLE_F32, 16, rows, 1024, 4096)
+    assert ws(16 * 48) == 0 and ws(16 * 48 + 1) > 0
