@@ -33,16 +33,16 @@ struct Counter {
 };
 
 // Sizes of one layer call, shared by every call of the same shape: the kept rows' bound, and where each intermediate lies
-// in the buffers of a call - route (the routing, which the layer also keeps as last_route), act (xd, a, out, scores and h, kept
-// for the backward) and grad (the backward's temporaries and scratch).  The forward's scratch is no part of what is kept: it
-// has a buffer of its own, or in a pass without autograd, which keeps nothing and stores no h, the place of h.  Holds no
-// device memory.
+// in the buffers of a call - route (the routing, which the layer also keeps as last_route), act (xd, a, out and h, kept for
+// the backward, as the scores are) and grad (the backward's temporaries and scratch).  The forward's scratch is no part of what
+// is kept: it has a buffer of its own, or in a pass without autograd, which keeps nothing and stores no h, the place of h.
+// Holds no device memory.
 struct Plan {
     mole_layer head{};
     at::ScalarType dtype;
     int gelu_bwd;
     enum { GATES, IDX, LOC, ROW, COUNTS, KEPT, OFFSETS, CAPACITY, N_ROUTE };
-    enum { XD, A, OUT, SCORES, H, N_ACT };
+    enum { XD, A, OUT, H, N_ACT };
     enum { D_O, T, GXD, DLOGITS, GRAD_WS, N_GRAD };
     int64_t route_off[N_ROUTE], act_off[N_ACT], grad_off[N_GRAD];
     int64_t route_bytes, act_bytes, grad_bytes, ws_fwd, ws_bwd;
@@ -76,7 +76,7 @@ struct Plan {
         ws_fwd = (int64_t)mole_layer_workspace_bytes(&head, 0);
         ws_bwd = (int64_t)mole_layer_workspace_bytes(&head, 1);
         route_bytes = carve({k * S * 4, k * S * 4, k * S * 4, k * S * 4, k * E * 4, E * 4, (E + 1) * 4, 4}, route_off);
-        act_bytes = carve({rows * M * es, rows * F * es, rows * M * es, S * E * 4, rows * F * es}, act_off);
+        act_bytes = carve({rows * M * es, rows * F * es, rows * M * es, rows * F * es}, act_off);
         grad_bytes = carve({rows * M * es, rows * F * es, rows * M * es, S * E * 4, ws_bwd}, grad_off);
     }
     std::vector<int64_t> route_offsets() const { return {route_off, route_off + N_ROUTE}; }
@@ -91,21 +91,34 @@ struct Call : torch::CustomClassHolder {
     bool accumulate = false;
     std::vector<int64_t> dummy_sizes;        // the marker parameter: its gradient is a tensor of zeros, never left out
     at::TensorOptions dummy_options;
-    Tensor route;                            // forward's result for the caller
+    Tensor route;                            // the routing: a result for the caller as well
 };
 
 void check_tensor(const Tensor &t, const char *name) {
     TORCH_CHECK(t.is_cuda() && t.is_contiguous(), "mole_amd: ", name, " must be a contiguous tensor on the GPU (there is no CPU path)");
 }
 
-mole_layer arguments(const Call &c, const Tensor &x, const Tensor &wg, char *route, char *act, char *ws, int64_t ws_bytes) {
+void check_input(const Plan &p, const Tensor &x, const Tensor &wg) {
+    check_tensor(x, "x");
+    check_tensor(wg, "the gate's weight");
+    TORCH_CHECK(x.dim() == 2 && x.size(0) == p.head.S && x.size(1) == p.head.M && x.scalar_type() == p.dtype &&
+                    wg.dim() == 2 && wg.size(0) == p.head.E && wg.size(1) == p.head.M && wg.scalar_type() == at::kFloat,
+                "mole_amd: the layer's input or gate does not have the planned shape or type");
+}
+void check_saved(const Tensor &t, at::ScalarType dtype, int64_t numel, const char *name) {
+    check_tensor(t, name);
+    TORCH_CHECK(t.scalar_type() == dtype && t.numel() == numel, "mole_amd: ", name, " came back in another shape or type than they were saved in");
+}
+
+mole_layer arguments(const Call &c, const Tensor &x, const Tensor &wg, const Tensor &scores, char *act, char *ws, int64_t ws_bytes) {
     const Plan &p = *c.plan;
+    char *route = (char *)c.route.data_ptr();
     mole_layer L = p.head;
     L.x = x.data_ptr();
     L.wg = wg.data_ptr<float>();
     L.logit_bias = c.bias.has_value() ? c.bias->data_ptr<float>() : nullptr;
     L.w1 = c.weights[0].data_ptr(); L.b1 = c.weights[1].data_ptr(); L.w2 = c.weights[2].data_ptr(); L.b2 = c.weights[3].data_ptr();
-    L.scores = (float *)(act + p.act_off[Plan::SCORES]);
+    L.scores = scores.data_ptr<float>();
     L.gates = (float *)(route + p.route_off[Plan::GATES]);
     L.idx = (int32_t *)(route + p.route_off[Plan::IDX]);
     L.loc = (int32_t *)(route + p.route_off[Plan::LOC]);
@@ -122,33 +135,31 @@ mole_layer arguments(const Call &c, const Tensor &x, const Tensor &wg, char *rou
 
 void *current_stream(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
-// y, the intermediates the backward reads, and the loss term, a tensor of its own: callers keep it, and part of a larger
-// buffer would keep all of that.  c.route is set.
+// y, the scores and intermediates the backward reads, and the loss term, a tensor of its own: callers keep it, and part of a
+// larger buffer would keep all of that.  c.route is set.
 struct Outputs {
-    Tensor y, act, l_aux;
+    Tensor y, scores, act, l_aux;
 };
 Outputs run_forward(Call &c, const Tensor &x, const Tensor &wg, bool forward_only) {
     const Plan &p = *c.plan;
-    check_tensor(x, "x");
-    check_tensor(wg, "the gate's weight");
-    TORCH_CHECK(x.dim() == 2 && x.size(0) == p.head.S && x.size(1) == p.head.M && x.scalar_type() == p.dtype &&
-                    wg.dim() == 2 && wg.size(0) == p.head.E && wg.size(1) == p.head.M && wg.scalar_type() == at::kFloat,
-                "mole_amd: the layer's input or gate does not have the planned shape or type");
+    check_input(p, x, wg);
     const auto bytes = x.options().dtype(at::kByte);
     c.route = at::empty({p.route_bytes}, bytes);
-    Tensor act = at::empty({forward_only ? p.act_off[Plan::H] + p.ws_fwd : p.act_bytes}, bytes), y = at::empty({p.head.S, p.head.M}, x.options());
-    Tensor l_aux = at::empty({}, x.options().dtype(at::kFloat));
+    // (act in the layer's own type: hooks on saved tensors may convert it and back)
+    const int64_t es = x.element_size();
+    Tensor act = at::empty({(forward_only ? p.act_off[Plan::H] + p.ws_fwd : p.act_bytes) / es}, x.options()), y = at::empty({p.head.S, p.head.M}, x.options());
+    Tensor scores = at::empty({p.head.S, p.head.E}, x.options().dtype(at::kFloat)), l_aux = at::empty({}, scores.options());
     Tensor ws;
     if (!forward_only) ws = at::empty({p.ws_fwd}, bytes);       // (released on return, for later work of this stream)
     char *a = (char *)act.data_ptr();
-    mole_layer L = arguments(c, x, wg, (char *)c.route.data_ptr(), a, forward_only ? a + p.act_off[Plan::H] : (char *)ws.data_ptr(), p.ws_fwd);
+    mole_layer L = arguments(c, x, wg, scores, a, forward_only ? a + p.act_off[Plan::H] : (char *)ws.data_ptr(), p.ws_fwd);
     L.l_aux = l_aux.data_ptr<float>();
     if (forward_only) {
         L.forward_only = 1;
         L.h = nullptr;
     }
     check(mole_layer_fwd(&L, y.data_ptr(), current_stream(x)), "mole_layer_fwd");
-    return {y, act, l_aux};
+    return {y, scores, act, l_aux};
 }
 
 struct LayerFn : torch::autograd::Function<LayerFn> {
@@ -157,24 +168,28 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         c->dummy_sizes = dummy.sizes().vec();
         c->dummy_options = dummy.options();
         ctx->set_materialize_grads(false);
-        auto [y, act, l_aux] = run_forward(*c, x, wg, false);
-        ctx->save_for_backward({x, wg, c->route, act});
+        auto [y, scores, act, l_aux] = run_forward(*c, x, wg, false);
+        ctx->save_for_backward({x, wg, scores, act});
         ctx->saved_data["call"] = c10::IValue::make_capsule(std::move(c));
         return {y, l_aux};
     }
 
     static variable_list backward(AutogradContext *ctx, variable_list g) {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &x = saved[0], &wg = saved[1], &route = saved[2], &act = saved[3];
+        const Tensor &x = saved[0], &scores = saved[2], &act = saved[3], wg = saved[1].to(at::kFloat).contiguous();
         auto c = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
         const Plan &p = *c->plan;
+        // (what hooks on saved tensors hand back need not be what was saved)
+        check_input(p, x, wg);
+        check_saved(scores, at::kFloat, (int64_t)p.head.S * p.head.E, "the scores");
+        check_saved(act, p.dtype, p.act_bytes / x.element_size(), "the intermediates");
         Tensor dy = g[0].defined() ? g[0].contiguous() : at::zeros_like(x);      // (undefined: only l_aux was used)
         Tensor d_aux = g[1].defined() ? g[1].to(at::kFloat).contiguous() : Tensor();
         TORCH_CHECK(dy.scalar_type() == p.dtype && dy.numel() == x.numel(), "mole_amd: the output's gradient has another shape or type");
         Tensor tmp = at::empty({p.grad_bytes}, x.options().dtype(at::kByte));
         Tensor dx = at::empty({p.head.S, p.head.M}, x.options()), dwg = at::empty({p.head.E, p.head.M}, wg.options());
         char *t = (char *)tmp.data_ptr();
-        mole_layer L = arguments(*c, x, wg, (char *)route.data_ptr(), (char *)act.data_ptr(), t + p.grad_off[Plan::GRAD_WS], p.ws_bwd);
+        mole_layer L = arguments(*c, x, wg, scores, (char *)act.data_ptr(), t + p.grad_off[Plan::GRAD_WS], p.ws_bwd);
         mole_layer_grads G{};
         G.accumulate = c->accumulate;
         G.gelu_bwd = p.gelu_bwd;

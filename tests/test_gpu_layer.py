@@ -637,9 +637,9 @@ def test_layer_refuses_to_be_traced(grad):
 @pytest.mark.parametrize("S,M,E,k,Fd,padded", [(1000, 256, 8, 2, 3072, False), (300, 512, 4, 1, 2048, False), (40, 256, 16, 2, 2048, True),
                                                (5000, 64, 64, 2, 64, False)])
 def test_recorded_pass_keeps_what_its_backward_reads(S, M, E, k, Fd, padded):
-    """Between forward and backward a pass holds its input, the gate's weight, the scores, the routing and the four row
-    buffers, and no scratch: neither the split contractions' planes nor the routing's workspace.  last_route keeps the
-    routing alone (k (3 S + E) numbers and the gate values), not the scores.  (Buffers begin at multiples of 256 bytes.)"""
+    """Between forward and backward a pass saves its input, the gate's weight, the scores and the four row buffers, and no
+    scratch: neither the split contractions' planes nor the routing's workspace.  last_route keeps the routing alone
+    (k (3 S + E) numbers and the gate values), not the scores.  (Buffers begin at multiples of 256 bytes.)"""
     m, x, _ = _build(S, M, E, k, Fd, torch.bfloat16, reference_layout=padded)
     cf = 1.0 if padded else 0.0
     rows = E * k * int(cf * -(-S // E)) if padded else S * k
@@ -647,8 +647,8 @@ def test_recorded_pass_keeps_what_its_backward_reads(S, M, E, k, Fd, padded):
     with torch.autograd.graph.saved_tensors_hooks(lambda t: (kept.append(t.nbytes), t)[1], lambda t: t):
         y = m(x, capacity_factor=cf)
     route = 4 * (4 * k * S + k * E + 2 * E + 2)
-    want = x.nbytes + 4 * E * M + route + 4 * S * E + 2 * rows * (2 * M + 2 * Fd)
-    assert want <= sum(kept) <= want + 32 * 256
+    want = x.nbytes + 4 * E * M + 4 * S * E + 2 * rows * (2 * M + 2 * Fd)
+    assert want <= sum(kept) <= want + 4 * 256
     assert m.last_route.row.untyped_storage().nbytes() <= route + 16 * 256
     y.sum().backward()
 
@@ -713,3 +713,47 @@ def test_gate_weight_inside_a_flat_buffer(S, M, E, train):
     for other in got[1:]:
         for a, b in zip(other, got[0]):
             assert torch.equal(a, b)
+
+
+def _train_pass(m, x, dy, cf, aux=0.01, wrap=lambda f, t: f(t)):
+    """One recorded pass and its backward: y and every gradient, from gradients that begin at nothing."""
+    m.gate[0].linear.weight.grad = None
+    for t in (m.FC1_W_GPU, m.FC1_B_GPU, m.FC2_W_GPU, m.FC2_B_GPU):
+        t.grad_tensors.fill_(7.0)
+    xx = x.clone().requires_grad_(True)
+    y = wrap(lambda t: m(t, capacity_factor=cf), xx)
+    torch.autograd.backward([y, m.l_aux], [dy, torch.tensor(aux, device="cuda")])
+    return _results(m, xx, y)
+
+
+def _results(m, x, y):
+    grads = [t.grad_tensors.clone() for t in (m.FC1_W_GPU, m.FC1_B_GPU, m.FC2_W_GPU, m.FC2_B_GPU)]
+    return [y.detach().clone(), x.grad.clone(), m.gate[0].linear.weight.grad.clone()] + grads
+
+
+def _same(got, want):
+    return len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("padded", [False, True])
+def test_saved_tensors_may_be_converted_and_moved(padded, dtype):
+    """Hooks on saved tensors see the layer's input, weight, scores and intermediates in their own types: a conversion to a wider
+    type or a stay in host memory changes no bit of the backward; a type that is not changed back is an error."""
+    m, x, _ = _build(130, 64, 8, 2, 128, dtype, reference_layout=padded)
+    dy = torch.randn(x.shape, generator=torch.Generator().manual_seed(3)).to(dtype).cuda()
+    want = _train_pass(m, x, dy, 1.25)
+    seen = []
+
+    def widen(t):
+        seen.append(t.dtype)
+        return t.dtype, t.double()
+    with torch.autograd.graph.saved_tensors_hooks(widen, lambda p: p[1].to(p[0])):
+        assert _same(_train_pass(m, x, dy, 1.25), want)
+    assert seen and all(t.is_floating_point for t in seen)
+    with torch.autograd.graph.save_on_cpu():
+        assert _same(_train_pass(m, x, dy, 1.25), want)
+    for back in (lambda t: t.double(), lambda t: t.cpu(), lambda t: t.flatten()[:-1]):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, back), pytest.raises(RuntimeError, match="mole_amd"):
+            _train_pass(m, x, dy, 1.25)
+    assert _same(_train_pass(m, x, dy, 1.25), want)
