@@ -757,3 +757,55 @@ def test_saved_tensors_may_be_converted_and_moved(padded, dtype):
         with torch.autograd.graph.saved_tensors_hooks(lambda t: t, back), pytest.raises(RuntimeError, match="mole_amd"):
             _train_pass(m, x, dy, 1.25)
     assert _same(_train_pass(m, x, dy, 1.25), want)
+
+
+@pytest.mark.parametrize("padded", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_layer_under_checkpoint_retained_graphs_streams_and_threads(padded, dtype):
+    """The native node gives the same bits recomputed by torch.utils.checkpoint (both kinds), run through twice on a retained
+    graph, on a stream of its own, and from two threads with a layer each."""
+    import threading
+    from torch.utils.checkpoint import checkpoint
+    m, x, _ = _build(200, 128, 8, 2, 256, dtype, reference_layout=padded)
+    other = type(m)(0, 8, 128, 256, -1, 2, 4, {"local_rank": 0, "world_size": 1, "rank": 0}, "gelu", 1, False, False, dtype=dtype,
+                    reference_layout=padded)
+    with torch.no_grad():
+        other.gate[0].linear.weight.copy_(m.gate[0].linear.weight)
+        for a, b in ((other.FC1_W_GPU, m.FC1_W_GPU), (other.FC1_B_GPU, m.FC1_B_GPU), (other.FC2_W_GPU, m.FC2_W_GPU), (other.FC2_B_GPU, m.FC2_B_GPU)):
+            a.all_tensors.copy_(b.all_tensors)
+    dy = torch.randn(x.shape, generator=torch.Generator().manual_seed(3)).to(dtype).cuda()
+    want, plain = _train_pass(m, x, dy, 1.25), _train_pass(m, x, dy, 1.25, aux=0.0)
+    for reentrant in (False, True):        # (l_aux is no output of the checkpointed function: the loss leaves it out)
+        xx = x.clone().requires_grad_(True)
+        m.gate[0].linear.weight.grad = None
+        y = checkpoint(lambda t: m(t, capacity_factor=1.25), xx, use_reentrant=reentrant)
+        y.backward(dy)
+        assert _same(_results(m, xx, y), plain), f"checkpoint, reentrant={reentrant}"
+    xx = x.clone().requires_grad_(True)
+    m.gate[0].linear.weight.grad = None
+    y = m(xx, capacity_factor=1.25)
+    for times in (1, 2):
+        torch.autograd.backward([y, m.l_aux], [dy, torch.tensor(0.01, device="cuda")], retain_graph=times == 1)
+        got = _results(m, xx, y)
+        assert _same(got, [want[0]] + [times * t for t in want[1:3]] + want[3:]), f"backward {times}"
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = _train_pass(m, x, dy, 1.25)
+    torch.cuda.current_stream().wait_stream(side)
+    assert _same(got, want), "a stream of its own"
+    out = {}
+
+    def work(layer, key):
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.default_stream())
+        with torch.cuda.stream(stream):
+            out[key] = [_train_pass(layer, x, dy, 1.25) for _ in range(8)]
+        stream.synchronize()
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(layer, i)) for i, layer in enumerate((m, other))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert sorted(out) == [0, 1] and all(_same(got, want) for runs in out.values() for got in runs), "two threads"
