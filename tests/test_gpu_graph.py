@@ -57,3 +57,52 @@ def test_hot_path_replays_in_a_graph():
         torch.cuda.synchronize()
         for i, (got, exp) in enumerate(zip(outs, want)):
             assert torch.equal(got, exp), f"replay {rep}, output {i}"
+
+
+@pytest.mark.parametrize("padded", [False, True])
+@pytest.mark.parametrize("train", [False, True])
+def test_layer_replays_in_a_graph(padded, train):
+    """The layer through its module (one native call each way), forward alone and with its backward, captured and replayed on
+    new inputs, with eager passes between the replays."""
+    from mole_amd.moe.layer import MOLEModule
+    S, M, E, k, Fd, cf = 777, 256, 8, 2, 512, 1.25
+    MOLEModule.reset_instances()
+    m = MOLEModule(0, E, M, Fd, -1, k, 4, {"local_rank": 0, "world_size": 1, "rank": 0}, "gelu", 1, False, False, dtype=torch.bfloat16,
+                   reference_layout=padded)
+    g = torch.Generator().manual_seed(11)
+    new = lambda: torch.randn(S, M, generator=g).bfloat16().cuda()
+    x, dy, wg = new().requires_grad_(train), new(), m.gate[0].linear.weight
+    aux = torch.tensor(0.01, device="cuda")
+    stores = (m.FC1_W_GPU, m.FC1_B_GPU, m.FC2_W_GPU, m.FC2_B_GPU)
+
+    def step():
+        with torch.set_grad_enabled(train):
+            y = m(x, capacity_factor=cf)
+        if not train:
+            return [y, m.l_aux, m.last_route.row]
+        x.grad = wg.grad = None
+        torch.autograd.backward([y, m.l_aux], [dy, aux])
+        return [y.detach(), m.l_aux.detach(), x.grad, wg.grad] + [t.grad_tensors for t in stores]
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = step()
+    for rep in range(4):
+        with torch.no_grad():
+            x.copy_(new()), dy.copy_(new())
+        want = [t.clone() for t in step()]
+        torch.cuda.synchronize()
+        for t in stores:
+            t.grad_tensors.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        for i, (got, exp) in enumerate(zip(outs, want)):
+            assert torch.equal(got, exp), f"replay {rep}, output {i}"
+    MOLEModule.reset_instances()
