@@ -1096,11 +1096,15 @@ __global__ __launch_bounds__(256) void gate_fwd_kernel(const bf16_t *__restrict_
 // instead of one block's 20 us, and 256 tokens x 256 experts x 2048 are 256 blocks (10 us; one 256 x 256 tile: 54).
 // Fragments come straight from memory.  Steps past a wave's share repeat its last one and are not multiplied; of a step
 // that M ends in, the lanes past the end are zero on both sides (an infinite weight times zero would be NaN).
+// fp32: every step of a round and every component of its 16 bytes has sums of its own, added up in pairs at the end, as are
+// the waves'.  A single running sum per wave is a chain of M / 4 additions, which left the logits 1.9 (M = 256) to 3.6 times
+// (M = 4096) as far off as gate_fwd_f32_kernel's 64 lanes do, and with them the gate values; this way they are as close or
+// closer.
 template <typename T, int TG>
-__global__ __launch_bounds__(256) void gate_logits_kernel(const T *__restrict__ x, const float *__restrict__ wg,
+__global__ __launch_bounds__(256, 2) void gate_logits_kernel(const T *__restrict__ x, const float *__restrict__ wg,
                                                           const float *__restrict__ bias, int S, int E, int M,
                                                           float *__restrict__ logits) {
-    constexpr int EPC = 16 / sizeof(T), KSTEP = 4 * EPC, U = TG == 1 ? 8 : 4;
+    constexpr int EPC = 16 / sizeof(T), KSTEP = 4 * EPC, U = TG == 1 ? 8 : 4, NA = sizeof(T) == 2 ? 1 : 4 * U;
     __shared__ float part[4][16 * TG][17];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, kq = lane >> 4;
@@ -1110,9 +1114,11 @@ __global__ __launch_bounds__(256) void gate_logits_kernel(const T *__restrict__ 
 #pragma unroll
     for (int t = 0; t < TG; ++t) xp[t] = x + (size_t)min(tok0 + 16 * t + r16, S - 1) * M;
     const float *wp = wg + (size_t)min(e0 + r16, E - 1) * M;
-    gate_f32x4 acc[TG];
+    gate_f32x4 acc[TG][NA];
 #pragma unroll
-    for (int t = 0; t < TG; ++t) acc[t] = gate_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < TG; ++t)
+#pragma unroll
+        for (int i = 0; i < NA; ++i) acc[t][i] = gate_f32x4{0.f, 0.f, 0.f, 0.f};
     for (int s = s_lo; s < s_hi; s += U) {
         uint4 a[TG][U];
         float4 w[U][EPC / 4];
@@ -1141,27 +1147,34 @@ __global__ __launch_bounds__(256) void gate_logits_kernel(const T *__restrict__ 
                     const float4 w0 = w[u][0], w1 = w[u][EPC / 4 - 1];
                     const gate_bf16x8 b = {(bf16_t)w0.x, (bf16_t)w0.y, (bf16_t)w0.z, (bf16_t)w0.w,
                                            (bf16_t)w1.x, (bf16_t)w1.y, (bf16_t)w1.z, (bf16_t)w1.w};
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gate_bf16x8, v), b, acc[t], 0, 0, 0);
+                    acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gate_bf16x8, v), b, acc[t][0], 0, 0, 0);
                 } else {
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.x), w[u][0].x, acc[t], 0, 0, 0);
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.y), w[u][0].y, acc[t], 0, 0, 0);
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.z), w[u][0].z, acc[t], 0, 0, 0);
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.w), w[u][0].w, acc[t], 0, 0, 0);
+                    gate_f32x4 (&c)[NA] = acc[t];
+                    c[4 * u] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.x), w[u][0].x, c[4 * u], 0, 0, 0);
+                    c[4 * u + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.y), w[u][0].y, c[4 * u + 1], 0, 0, 0);
+                    c[4 * u + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.z), w[u][0].z, c[4 * u + 2], 0, 0, 0);
+                    c[4 * u + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(v.w), w[u][0].w, c[4 * u + 3], 0, 0, 0);
                 }
             }
         }
     }
 #pragma unroll
-    for (int t = 0; t < TG; ++t)
+    for (int t = 0; t < TG; ++t) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) part[wave][16 * t + 4 * kq + r][r16] = acc[t][r];
+        for (int half = NA / 2; half >= 1; half /= 2)
+#pragma unroll
+            for (int i = 0; i < half; ++i) acc[t][i] += acc[t][i + half];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[wave][16 * t + 4 * kq + r][r16] = acc[t][0][r];
+    }
     __syncthreads();
     const int e = e0 + (threadIdx.x & 15);
 #pragma unroll
     for (int t = 0; t < TG; ++t) {
         const int tl = 16 * t + (threadIdx.x >> 4);
-        if (tok0 + tl < S && e < E)
-            logits[(size_t)(tok0 + tl) * E + e] = part[0][tl][e - e0] + part[1][tl][e - e0] + part[2][tl][e - e0] + part[3][tl][e - e0] + (bias ? bias[e] : 0.f);
+        const float p0 = part[0][tl][e - e0], p1 = part[1][tl][e - e0], p2 = part[2][tl][e - e0], p3 = part[3][tl][e - e0];
+        const float sum = sizeof(T) == 2 ? p0 + p1 + p2 + p3 : (p0 + p1) + (p2 + p3);
+        if (tok0 + tl < S && e < E) logits[(size_t)(tok0 + tl) * E + e] = sum + (bias ? bias[e] : 0.f);
     }
 }
 
@@ -1284,7 +1297,9 @@ extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const 
         float *logits = (float *)ws;
         ws += align256((size_t)S * E * sizeof(float));
         if (path == GR_FEW) {
-            const int tg = S <= 512 ? 1 : 2;           // Wg is read once for 16 or 32 tokens
+            // Wg is read once for 16 or 32 tokens.  fp32 gates of one or two groups of experts have the blocks to spare
+            // (2048 tokens, 16 experts of 4096, with the routing: 32 us in 16s, 38 in 32s); wide ones do not (2000, 256 of 2048: 97 / 86).
+            const int tg = S <= 512 || (dtype == MOLE_F32 && E <= 32) ? 1 : 2;
             const dim3 grid(ceil_div(S, 16 * tg), ceil_div(E, 16));
 #define MOLE_GL(T, TG) timed_launch(MOLE_K_GATE_FWD, gate_logits_kernel<T, TG>, grid, dim3(256), 0, st, (const T *)x, wg, logit_bias, S, E, M, logits)
             if (dtype == MOLE_BF16) { if (tg == 1) MOLE_GL(bf16_t, 1); else MOLE_GL(bf16_t, 2); }

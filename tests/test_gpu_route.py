@@ -280,3 +280,21 @@ def test_gate_logits_with_an_infinite_weight(S, E, M, dtype):
         wg[2, at] = float("inf")       # inf - inf in the softmax of every token
         scores, _ = H.gate_route(x.cuda(), wg.cuda(), None, 2, 0.0, True, 1)
         assert bool(scores[:, 2].isnan().all())
+
+
+# fp32 gates of few tokens are as accurate as the kernel of many: logits (from the scores' logarithms) against 64 bits.  Every
+# running sum has M / 128 terms of deviation 4 / sqrt(M); roundings of 2^-24 of a partial sum leave such a sum off by
+# 2^-24 4 sqrt(M) / 128 / sqrt(6), all 128 by sqrt(128) times that, seven levels of pairs by 2^-24 4 sqrt(7 / 3) / 2 or less: 6e-7 at
+# M = 4096 with the softmax's own 4e-7 (its argument and value, rounded) beside it 7e-7 in the root mean square.  (One
+# running sum per wave: 2.4e-6.)
+@pytest.mark.parametrize("S,E,M", [(3, 8, 4096), (777, 32, 4100), (2048, 5, 4096), (600, 40, 4032)])
+def test_fp32_gate_logits_of_few_tokens_keep_their_accuracy(S, E, M):
+    from mole_amd import hip_ops as H
+    print(f"fp32 gate accuracy S={S} E={E} M={M}", flush=True)
+    g = torch.Generator().manual_seed(S + M)
+    x, wg = torch.randn(S, M, generator=g), torch.randn(E, M, generator=g) * (4.0 / M ** 0.5)
+    scores, _ = H.gate_route(x.cuda(), wg.cuda(), None, 1, 0.0, True, 1)
+    want = torch.log_softmax(x.double() @ wg.double().t(), 1)
+    near = want > -6.0                    # (the argument's rounding grows with its size)
+    err = (scores.cpu().double().log() - want)[near]
+    assert float(err.pow(2).mean().sqrt()) < 1e-6
