@@ -515,19 +515,38 @@ def test_ffn_weight_gradients_by_small_tiles(E, M, Fd, rows, gap, accumulate):
         assert rel_err(got, want + 0.5 if accumulate else want) < tol(dtype)
 
 
-# K-strided weights read past the caches: experts with one m-tile of one or two live row blocks per wave, with more rows (the
-# ordinary loads) and with none, in a forward pass that no backward follows.  The loads' cache policy changes no result.
+# K-strided weights read past the caches, in a forward pass that no backward follows: from 64 MB of weights of the experts that
+# can have rows, the recorded pass (256 MB) taking the ordinary loads.  Experts of a few rows on the kernel for them, of up
+# to 64 and up to 128 on the tiles, of more (ordinary loads there), and of none.  The loads' cache policy changes no result.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("E,M,k,S", [(200, 128, 1, 61), (200, 256, 2, 3000), (2, 1024, 1, 5), (3, 64, 1, 300)])
-def test_forward_only_weights_leave_no_copy(E, M, k, S, dtype):
+@pytest.mark.parametrize("E,M,Fd,k,S", [
+    (40, 1024, 1024, 1, 61), (40, 1024, 1024, 2, 120), (23, 512, 3264, 2, 33),      # few rows; the last of 67 / 134 MB
+    (60, 1024, 1024, 2, 900), (60, 1024, 1024, 2, 3000), (40, 1024, 1024, 2, 4000),  # bf16 tiles: up to 64 rows, up to 128, more
+    (9, 3072, 1280, 1, 301), (200, 128, 192, 1, 61), (2, 1024, 192, 1, 5), (3, 64, 192, 1, 300),      # and below the limit
+])
+def test_forward_only_weights_leave_no_copy(E, M, Fd, k, S, dtype):
     from mole_amd.moe.layer import MOLEModule
-    print(f"forward only E={E} M={M} k={k} S={S} {dtype}", flush=True)
+    print(f"forward only E={E} M={M} F={Fd} k={k} S={S} {dtype}", flush=True)
+    nbytes = E * M * Fd * dtype.itemsize
+    assert Fd == 192 or (64 << 20) <= nbytes < (256 << 20), "not the sizes this test is for"
     MOLEModule.reset_instances()
-    m = MOLEModule(0, E, M, 192, -1, k, 4, {"local_rank": 0, "world_size": 1, "rank": 0}, "gelu", 1, False, False, dtype=dtype)
+    m = MOLEModule(0, E, M, Fd, -1, k, 4, {"local_rank": 0, "world_size": 1, "rank": 0}, "gelu", 1, False, False, dtype=dtype)
     x = torch.randn(S, M, generator=torch.Generator().manual_seed(S)).to(dtype).cuda()
     y = m(x, capacity_factor=0.0).detach()            # recorded: the general policy
     with torch.no_grad():
         assert torch.equal(m(x, capacity_factor=0.0), y)
+    f = lambda t: t.detach().float().cpu()
+    r = m.last_route                                  # and against fp32 products of the experts that have rows
+    want = torch.zeros(S, M)
+    idx, gates, row = r.idx.cpu().long(), f(r.gates), r.row.cpu()
+    assert bool((row >= 0).all())
+    for e in idx.unique().tolist():
+        w1, b1, w2, b2 = (f(p.all_tensors[e]) for p in (m.FC1_W_GPU, m.FC1_B_GPU, m.FC2_W_GPU, m.FC2_B_GPU))
+        for j in range(k):
+            t = (idx[j] == e).nonzero()[:, 0]
+            a = torch.nn.functional.gelu(f(x[t.cuda()]) @ w1.t() + b1)
+            want[t] += gates[j, t, None] * (a @ w2 + b2)
+    assert rel_err(y, want) < tol(dtype)
     MOLEModule.reset_instances()
 
 
