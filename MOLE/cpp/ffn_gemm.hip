@@ -469,8 +469,10 @@ static int run_gemm(const GemmArgs &g, int max_rows, int tiles_generic, hipStrea
 
 // Whether a product's K-strided weights (out = a.w2, gx = t.w1), where one block each reads them, should leave no copy
 // behind in the caches, which makes the stream faster: if they are more than the 256 MB last-level cache holds, or, where no
-// backward pass reads them again soon, a quarter of it (the weights of a small layer stay there between calls: 9 experts of
-// 832 -> 2496, 24 rows, 42.0 against 42.6 us a forward pass).  In a training step with smaller ones the next product on the same matrix finds them there (16
+// backward pass reads them again soon, a quarter of it.  bf16 forward passes of layers that take turns, so that no weights wait
+// in a cache, without / with a copy left: 9 experts of 1024 -> 4096, 75 MB, 4 / 60 rows 59 / 75 against 60 / 77 us; 40 of 1024 ->
+// 1024, 84 MB, 70 / 83 against 71 / 85; 48 of 1536 -> 1536, 226 MB, 159 / 189 against 164 / 194.  (One layer called again and again
+// finds up to about 120 MB there: 40 of 1024 -> 1024 then takes 64 / 75 against 61 / 72.)  In a training step with smaller ones the next product on the same matrix finds them there (16
 // experts of 2048 x 4096 with 8 rows each: out 54 -> 48 us without a copy, but t = go.w2^T after it 44 -> 73).  Rows must be
 // whole 128-byte lines: two blocks share a line otherwise (60 experts of 2104 -> 6312, 28 rows: no gain).
 static int weights_pass_by(int E, int est_rows, int M, int F, size_t elem, int forward_only) {
@@ -566,7 +568,7 @@ namespace mole {
 
 size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, int F) {
     if (E <= 0 || max_rows <= 0 || M <= 0 || F <= 0) return 0;
-    int ks = gemm_skinny_ksplit(E, est_rows, M, F, dtype);
+    int ks = gemm_skinny_ksplit(E, max_rows, est_rows, M, F, dtype);
     if (ks == 0) ks = dtype == MOLE_BF16 ? gemm256_ksplit(E, est_rows, M, F) : gemm_f32_ksplit(E, est_rows, M, F);
     ks = planes_allowed(ks, max_rows, est_rows, M);
     return ks > 1 ? (size_t)ks * max_rows * M * sizeof(float) : 0;

@@ -174,7 +174,7 @@ inline int planes_allowed(int ks, int max_rows, int est_rows, int N) {
 }
 // Few rows per expert (gemm_skinny.hip): weights streamed straight into fragments; -100 when the shape is not its.
 int launch_gemm_skinny(const GemmArgs &g, int dtype, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
-int gemm_skinny_ksplit(int E, int est_rows, int N, int K, int dtype);    // 0: not its shape
+int gemm_skinny_ksplit(int E, int max_rows, int est_rows, int N, int K, int dtype);    // 0: not its shape
 // fp32 tiles with direct-to-LDS loads (gemm_f32.hip); -100 as above.
 int launch_gemm_f32(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
 int gemm_f32_ksplit(int E, int est_rows, int N, int K);

@@ -404,9 +404,10 @@ __global__ __launch_bounds__(256) void plane_reduce_kernel(const GemmArgs g) {
 }
 
 // ---- which products come here, and how they are cut ------------------------------------------------------------
-// avg: rows of an expert if the rows spread evenly; tiles: blocks the big-tile kernel of the type would have.
+// avg: rows of an expert if the rows spread evenly; tiles: blocks the big-tile kernel of the type would have; tiles_split:
+// whether those can split the contraction as they would, or have no need to.
 struct SkinnyPlan { int mb, ksplit; };
-static bool skinny_plan(int dtype, bool b_ks, int E, int est_rows, int N, int K, SkinnyPlan &p) {
+static bool skinny_plan(int dtype, bool b_ks, int E, int est_rows, int N, int K, bool tiles_split, SkinnyPlan &p) {
     if (est_rows <= 0) return false;
     const bool bf16 = dtype == MOLE_BF16;
     const int epc = bf16 ? 8 : 4;
@@ -416,8 +417,14 @@ static bool skinny_plan(int dtype, bool b_ks, int E, int est_rows, int N, int K,
     // fast or faster (16 experts of 1024 -> 4096, 61 rows: 27 against 30 us); with fewer they leave CUs without work
     // (2 rows of 64 experts, 2048 -> 8192: h 24 against 17.5 us, out 66 against 13).  KC stops at 24 rows per expert,
     // where the token loads, one per four weight loads and 16 rows, begin to cost (8 experts of 512 -> 2048, 600 rows:
-    // 18 against 14 us); KS, eight weight loads each, at 64 (16 x 1024 -> 4096, 400 / 800 / 1600 rows: 39 / 50 / 79
-    // against 55 / 61 / 75 us).
+    // 18 against 14 us).  KS, eight weight loads for every 16 rows, against tiles that split the contraction as well: with
+    // fewer than 32 tiles up to 64 rows per expert, below 48 up to 24, beyond up to 12 (and up to 64 where no workspace lets the
+    // tiles split).  Forward pass, weights in no cache, here / on tiles: 4 experts of 2048 -> 2048, 32 tiles, 20 / 40 / 60 rows
+    // 53 / 71 / 77 against 54 / 68 / 73 us; 20 of 512 -> 2048, 40 tiles, 20 / 40 / 60 rows 59 / 62 / 67 against 56 / 56 / 61, under Zipf
+    // loads 58 / 67 / 71 against 61 / 66 / 71; 32 of 768 -> 2304, 96 tiles, 9 / 16 / 40 / 60 rows 97 / 104 / 131 / 151 against 92 / 93 / 98 /
+    // 105, Zipf 80 / 91 / 116 / 127 against 77 / 88 / 114 / 113; 24 of 520 -> 1416, 72 tiles, 9 / 16 / 40 rows 53 / 61 / 77 against 52 /
+    // 54 / 61, Zipf 47 / 56 / 81 against 50 / 55 / 79.  (Weights in the caches: 2 of 2048 -> 8192, 16 tiles, 16 / 62 rows 55 / 60
+    // against 64 / 74.)
     // fp32: the 64 x 128 tiles of gemm_f32.hip, with their planes, from 48 rows per expert on, where also evenly spread rows
     // need more than one group of 32 and the fuller experts of a skewed routing many, each reading the weights again
     // (16 experts of 1024 -> 4096, forward pass, tiles / here: 800 rows 190 / 225 us, skewed 295 / 318; 960 rows 302 / 329;
@@ -425,10 +432,10 @@ static bool skinny_plan(int dtype, bool b_ks, int E, int est_rows, int N, int K,
     bool takes;
     if (bf16) {
         const long tiles = (long)active * ceil_div(avg, 256) * ceil_div(N, 256);
-        takes = tiles < 192 && avg <= (b_ks ? 64 : 24);
+        takes = tiles < 192 && avg <= (!b_ks ? 24 : tiles < 32 || !tiles_split ? 64 : tiles < 48 ? 24 : 12);
         // every group of 16 rows reads the expert's weights again, from memory where they are more than the 256 MB last-level
-        // cache holds: there the tiles take what is more than one group (14 experts of 2304 -> 4608, 56 rows: out 169 us
-        // against 58, planes added; 20 of 2264 -> 9056, 20 rows: 304 against 153)
+        // cache holds: there the tiles take what is more than one group (20 experts of 2264 -> 9056, 20 rows: out 304 us here
+        // against 153, planes added)
         if (b_ks && avg > 16 && (size_t)active * N * K * sizeof(bf16_t) > (size_t)256 << 20) takes = false;
     } else {
         takes = avg <= (b_ks ? 48 : 20);
@@ -447,9 +454,15 @@ static bool skinny_plan(int dtype, bool b_ks, int E, int est_rows, int N, int K,
     return true;
 }
 
-int gemm_skinny_ksplit(int E, int est_rows, int N, int K, int dtype) {
+static bool tiles_split(int dtype, int E, int max_rows, int est_rows, int N, int K, size_t ws_bytes) {
+    if (dtype != MOLE_BF16) return true;
+    const int ks = gemm256_ksplit(E, est_rows, N, K);
+    return ks <= 1 || (planes_allowed(ks, max_rows, est_rows, N) == ks && ws_bytes >= (size_t)ks * max_rows * N * sizeof(float));
+}
+
+int gemm_skinny_ksplit(int E, int max_rows, int est_rows, int N, int K, int dtype) {
     SkinnyPlan p;
-    return skinny_plan(dtype, true, E, est_rows, N, K, p) ? p.ksplit : 0;
+    return skinny_plan(dtype, true, E, est_rows, N, K, tiles_split(dtype, E, max_rows, est_rows, N, K, SIZE_MAX), p) ? p.ksplit : 0;
 }
 
 int launch_plane_reduce(const GemmArgs &g, int dtype, int max_rows, hipStream_t st) {
@@ -486,7 +499,9 @@ int launch_gemm_skinny(const GemmArgs &g0, int dtype, bool b_ks, int epi, int ma
     GemmArgs g = g0;
     const int epc = dtype == MOLE_BF16 ? 8 : 4;
     SkinnyPlan p;
-    if (max_rows <= 0 || g.offsets == nullptr || g.kept == nullptr || !skinny_plan(dtype, b_ks, g.E, g.est_rows, g.N, g.K, p)) return -100;
+    if (max_rows <= 0 || g.offsets == nullptr || g.kept == nullptr) return -100;
+    const bool split = !b_ks || tiles_split(dtype, g.E, max_rows, g.est_rows, g.N, g.K, ws != nullptr ? ws_bytes : 0);
+    if (!skinny_plan(dtype, b_ks, g.E, g.est_rows, g.N, g.K, split, p)) return -100;
     const int groups = (g.E < max_rows ? g.E : max_rows) + max_rows / (16 * p.mb);     // as many as max_rows rows can need
     if (g.K % epc || g.N % epc || g.lda % epc || g.ldb % epc || g.ldc % epc || g.strideB % epc) return -100;
     g.ksplit = 1;

@@ -486,7 +486,7 @@ def run_probes(args):
             try:
                 t = timed(lambda: L.check(L.lib().mole_probe_kloop_part(L.ptr(xa), L.ptr(wa), L.ptr(off), L.ptr(kept), E, S, F, M,
                                                                         part, L.ptr(sink), L.stream()), "mole_probe_kloop_part"), 20)
-            except RuntimeError:      # only the default tile shape has the variants (MOLE_TMB selects others)
+            except RuntimeError:      # the loop's parts are in a MOLE_TUNING build only
                 L.kernel_timing_enable(False)
                 continue
             cnt, ms = t["probe"]

@@ -22,8 +22,8 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-x", "hip",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-command-line-argument",
          "-I" + os.path.join(ROOT, "include"), "-I" + CPP]
-# MOLE_TUNING=1 in the environment of the build adds the tile shapes, launch orders and K-loop ablations that were
-# measured against the defaults (selected at run time by MOLE_TMB, MOLE_MFAST, ...: see MOLE/cpp/gemm256.hip)
+# MOLE_TUNING=1 in the environment of the build adds the launch orders and K-loop ablations that were measured against
+# the defaults (selected at run time by MOLE_MFAST, MOLE_GEMM, ...: see MOLE/cpp/gemm256.hip and ffn_gemm.hip)
 if os.environ.get("MOLE_TUNING"):
     FLAGS.append("-DMOLE_TUNING")
 

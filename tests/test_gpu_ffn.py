@@ -354,6 +354,10 @@ FEW_ROWS = [
     (3, 264, 4096, [33, 16, 5], 1),
     (6, 1032, 520, [0, 2, 40, 1, 0, 64], 0),
     (70, 64, 1032, [(5 * e) % 9 for e in range(70)], 0),
+    # where bf16's K-strided products change to tiles: below and from 32 and 48 tiles, at 24 / 12 rows an expert and one more;
+    # without a workspace, where the tiles could not split the contraction, they stay
+    (31, 64, 1032, [25 + e % 3 for e in range(31)], 0), (32, 64, 1032, [24 + (e % 3 - 1) for e in range(32)], 0),
+    (32, 64, 1032, [25] * 32, 1), (48, 64, 1032, [12] * 48, 0), (48, 72, 1032, [13 + 4 * (e % 3 - 1) for e in range(48)], 0),
 ]
 
 
