@@ -35,8 +35,8 @@ struct Counter {
 // Sizes of one layer call, shared by every call of the same shape: the kept rows' bound, and where each intermediate lies
 // in the buffers of a call - route (the routing, which the layer also keeps as last_route), act (xd, a, out and h, kept for
 // the backward, as the scores are) and grad (the backward's temporaries and scratch).  The forward's scratch is no part of what
-// is kept: it has a buffer of its own, or in a pass without autograd, which keeps nothing and stores no h, the place of h.
-// Holds no device memory.
+// is kept: it has a buffer of its own, or in a pass without autograd, which keeps nothing and stores no h, the place of h, with
+// the scores behind it (every allocation is a microsecond of the host's).  Holds no device memory.
 struct Plan {
     mole_layer head{};
     at::ScalarType dtype;
@@ -110,7 +110,7 @@ void check_saved(const Tensor &t, at::ScalarType dtype, int64_t numel, const cha
     TORCH_CHECK(t.scalar_type() == dtype && t.numel() == numel, "mole_amd: ", name, " came back in another shape or type than they were saved in");
 }
 
-mole_layer arguments(const Call &c, const Tensor &x, const Tensor &wg, const Tensor &scores, char *act, char *ws, int64_t ws_bytes) {
+mole_layer arguments(const Call &c, const Tensor &x, const Tensor &wg, void *scores, char *act, char *ws, int64_t ws_bytes) {
     const Plan &p = *c.plan;
     char *route = (char *)c.route.data_ptr();
     mole_layer L = p.head;
@@ -118,7 +118,7 @@ mole_layer arguments(const Call &c, const Tensor &x, const Tensor &wg, const Ten
     L.wg = wg.data_ptr<float>();
     L.logit_bias = c.bias.has_value() ? c.bias->data_ptr<float>() : nullptr;
     L.w1 = c.weights[0].data_ptr(); L.b1 = c.weights[1].data_ptr(); L.w2 = c.weights[2].data_ptr(); L.b2 = c.weights[3].data_ptr();
-    L.scores = scores.data_ptr<float>();
+    L.scores = (float *)scores;
     L.gates = (float *)(route + p.route_off[Plan::GATES]);
     L.idx = (int32_t *)(route + p.route_off[Plan::IDX]);
     L.loc = (int32_t *)(route + p.route_off[Plan::LOC]);
@@ -135,7 +135,7 @@ mole_layer arguments(const Call &c, const Tensor &x, const Tensor &wg, const Ten
 
 void *current_stream(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
-// y, the scores and intermediates the backward reads, and the loss term, a tensor of its own: callers keep it, and part of a
+// y, the scores and intermediates the backward reads (recorded passes), and the loss term, a tensor of its own: callers keep it, and part of a
 // larger buffer would keep all of that.  c.route is set.
 struct Outputs {
     Tensor y, scores, act, l_aux;
@@ -147,12 +147,17 @@ Outputs run_forward(Call &c, const Tensor &x, const Tensor &wg, bool forward_onl
     c.route = at::empty({p.route_bytes}, bytes);
     // (act in the layer's own type: hooks on saved tensors may convert it and back)
     const int64_t es = x.element_size();
-    Tensor act = at::empty({(forward_only ? p.act_off[Plan::H] + p.ws_fwd : p.act_bytes) / es}, x.options()), y = at::empty({p.head.S, p.head.M}, x.options());
-    Tensor scores = at::empty({p.head.S, p.head.E}, x.options().dtype(at::kFloat)), l_aux = at::empty({}, scores.options());
-    Tensor ws;
-    if (!forward_only) ws = at::empty({p.ws_fwd}, bytes);       // (released on return, for later work of this stream)
+    const int64_t only_scores = p.act_off[Plan::H] + up256(p.ws_fwd), only_bytes = only_scores + (int64_t)p.head.S * p.head.E * 4;
+    Tensor act = at::empty({(forward_only ? only_bytes : p.act_bytes) / es}, x.options()), y = at::empty({p.head.S, p.head.M}, x.options());
+    const auto f32 = x.options().dtype(at::kFloat);
+    Tensor scores, l_aux = at::empty({}, f32), ws;
+    if (!forward_only) {
+        scores = at::empty({p.head.S, p.head.E}, f32);
+        ws = at::empty({p.ws_fwd}, bytes);       // (released on return, for later work of this stream)
+    }
     char *a = (char *)act.data_ptr();
-    mole_layer L = arguments(c, x, wg, scores, a, forward_only ? a + p.act_off[Plan::H] : (char *)ws.data_ptr(), p.ws_fwd);
+    mole_layer L = arguments(c, x, wg, forward_only ? a + only_scores : scores.data_ptr(), a,
+                             forward_only ? a + p.act_off[Plan::H] : (char *)ws.data_ptr(), p.ws_fwd);
     L.l_aux = l_aux.data_ptr<float>();
     if (forward_only) {
         L.forward_only = 1;
@@ -189,7 +194,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
         Tensor tmp = at::empty({p.grad_bytes}, x.options().dtype(at::kByte));
         Tensor dx = at::empty({p.head.S, p.head.M}, x.options()), dwg = at::empty({p.head.E, p.head.M}, wg.options());
         char *t = (char *)tmp.data_ptr();
-        mole_layer L = arguments(*c, x, wg, scores, (char *)act.data_ptr(), t + p.grad_off[Plan::GRAD_WS], p.ws_bwd);
+        mole_layer L = arguments(*c, x, wg, scores.data_ptr(), (char *)act.data_ptr(), t + p.grad_off[Plan::GRAD_WS], p.ws_bwd);
         mole_layer_grads G{};
         G.accumulate = c->accumulate;
         G.gelu_bwd = p.gelu_bwd;

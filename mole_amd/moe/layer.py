@@ -302,7 +302,9 @@ class MOLEModule(torch.nn.Module):
             UATimer.track_fwd_start(self.moe_id)
         if prefetch:
             input_ = pfetchbwd.apply(input_, self)
-        resized_input = input_.reshape(-1, self.embed_dim)
+        # (tokens that come as [S, M] stay as they are: two views less on the host, and their nodes in the backward)
+        flat = input_.dim() == 2 and original_shape[1] == self.embed_dim
+        resized_input = input_ if flat else input_.reshape(-1, self.embed_dim)
         if resized_input.dtype != self.param_dtype:
             resized_input = resized_input.to(self.param_dtype)
         resized_input = resized_input.contiguous()
@@ -328,7 +330,8 @@ class MOLEModule(torch.nn.Module):
             expert_output, self.l_aux = _FusedMoE.apply(resized_input, gate.linear.weight, self.dummy_param, self, float(capacity_factor),
                                                         bool(time_it))
 
-        expert_output = expert_output.reshape(original_shape)
+        if not flat:
+            expert_output = expert_output.reshape(original_shape)
         out = expert_output.to(original_dtype)
         if time_it:
             UATimer.track_fwd_end(self.moe_id)
