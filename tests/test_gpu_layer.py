@@ -809,3 +809,31 @@ def test_layer_under_checkpoint_retained_graphs_streams_and_threads(padded, dtyp
     for t in threads:
         t.join()
     assert sorted(out) == [0, 1] and all(_same(got, want) for runs in out.values() for got in runs), "two threads"
+
+
+# Tokens in other shapes than [S, M] are the same tokens: outputs and gradients in the caller's shape, equal to the flat pass's.
+# (Rows of two tokens, three dimensions, one token without a dimension for it, every other row of a buffer, another type.)
+@pytest.mark.parametrize("form", ["rows of two", "three", "one", "strided", "fp32"])
+def test_layer_takes_tokens_in_other_shapes(form):
+    from mole_amd.moe.layer import MOLEModule
+    print(f"token shapes: {form}", flush=True)
+    S, M, E, Fd = (1 if form == "one" else 48), 128, 8, 256
+    MOLEModule.reset_instances()
+    m = MOLEModule(0, E, M, Fd, -1, 2, 4, {"local_rank": 0, "world_size": 1, "rank": 0}, "gelu", 1, False, False, dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(9)
+    x, dy = (torch.randn(S, M, generator=g).bfloat16().cuda() for _ in range(2))
+    flat = x.clone().requires_grad_(True)
+    y = m(flat, capacity_factor=0.0)
+    y.backward(dy)
+    shape = {"rows of two": (S // 2, 2 * M), "three": (6, S // 6, M), "one": (M,)}.get(form, (S, M))
+    if form == "strided":
+        other = torch.zeros(S, 2, M, dtype=x.dtype, device="cuda")[:, 1].copy_(x).requires_grad_(True)
+    else:
+        other = x.clone().view(shape).to(torch.float32 if form == "fp32" else x.dtype).requires_grad_(True)
+    got = m(other, capacity_factor=0.0)
+    assert got.shape == shape and got.dtype == other.dtype and torch.equal(got.view(S, M).to(y.dtype), y)
+    got.backward(dy.view(shape).to(got.dtype))
+    assert other.grad.shape == shape and torch.equal(other.grad.reshape(S, M).to(y.dtype), flat.grad)
+    with torch.no_grad():
+        assert torch.equal(m(other, capacity_factor=0.0).view(S, M).to(y.dtype), y)
+    MOLEModule.reset_instances()
