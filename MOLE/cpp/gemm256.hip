@@ -1,7 +1,7 @@
 // bf16 grouped GEMM for gfx950: the fast path of the six expert-FFN products.
 //
 // A block of 8 waves (2 wave rows x 4 wave columns, two waves per SIMD) owns a BM (m) x 256 (n) output tile, BM =
-// 256 or up to 320; a wave covers BM/2 rows and 64 columns (BM/64 x 2 MFMA 32x32x16 blocks, fp32 accumulators).
+// 256 or up to 320; a wave covers BM/2 rows and 64 columns (BM/32 x 4 MFMA 16x16x32 blocks, fp32 accumulators).
 // One block per CU.  Launches too small to give most CUs such a tile run 128 x 128 tiles of four waves, two blocks to a
 // CU.  (A build with -DMOLE_TUNING also reads the launch orders that were measured against these and lost.)
 // Operand tiles go from HBM/L2 straight into LDS (global_load_lds_dwordx4, no staging registers)
@@ -70,13 +70,15 @@ template <int TMB, int WM, int WN, bool M_KS, int TMC> struct Stage {
 // does not store - except along a ragged contraction length, which zero_k_tail() repairs.
 //
 // K-contiguous operand, element (r, k) at p[r*ld + k]: LDS [ROWS][4 x 16 B], the chunk index XORed
-// with swz4(row), chosen so that the 16 rows a ds_read_b128 pass touches (and any 8 aligned rows)
-// fall into distinct bank groups of the 64-bank LDS.
+// with swz16(row).  A fragment read has lane l at row l % 16, chunk l / 16; one pass of ds_read_b128 serves 16 lanes, either
+// 16 neighbours or (0-3, 12-15, 20-27) and its like, and with this swizzle both kinds fall into distinct bank groups of the
+// 64-bank LDS.
 // With NW waves, wave w's load i fills LDS bytes [(NW i + w)*1024, +1024) = rows 16(NW i + w) .. +16.
 // Per-lane byte offsets of the ROWS/(16 NW) loads a wave issues for one stage of an operand tile, relative to
 // the tile's first element at the stage's first k (what the scalar base points at).  r_left = rows of the
 // operand from the tile's first row on, k_left = k-rows from the stage's first k on (only the last stage
 // of a ragged contraction has fewer than 32).
+__device__ __forceinline__ int swz16(int row) { return ((row >> 3) & 1) | (((row >> 1) ^ (row >> 2)) & 2); }
 template <int ROWS, int NW> struct OffKC {
     uint32_t off[ROWS / (16 * NW)];
     __device__ __forceinline__ void init(long ld, int r_left, int k_left) {
@@ -84,14 +86,15 @@ template <int ROWS, int NW> struct OffKC {
 #pragma unroll
         for (int i = 0; i < ROWS / (16 * NW); ++i) {
             const int row = (NW * i + w) * 16 + (lane >> 2);
-            const int c = min((lane & 3) ^ swz4(row), (k_left >> 3) - 1);     // (k_left is a multiple of 8)
+            const int c = min((lane & 3) ^ swz16(row), (k_left >> 3) - 1);     // (k_left is a multiple of 8)
             off[i] = (uint32_t)(min(row, r_left - 1) * ld * 2 + c * 16);
         }
     }
 };
 // K-strided operand, element (r, k) at p[k*ld + r]: LDS [32 k][ROWS x 2 B] as it lies in HBM, the
-// 32-byte granule index XORed with (k & 3) << 1 (conflict-free transpose reads, see frag_ks).
+// 32-byte granule index XORed with swz_ks(k) (conflict-free transpose reads, see frag_ks).
 // A k-row has ROWS/8 slots of 16 bytes; a wave load of 1 KiB covers 512/ROWS k-rows.
+__device__ __forceinline__ int swz_ks(int k) { return ((k & 3) << 1) | ((k >> 3) & 1); }
 template <int ROWS, int NW> struct OffKS {
     uint32_t off[ROWS / (16 * NW)];
     __device__ __forceinline__ void init(long ld, int r_left, int k_left) {
@@ -102,7 +105,7 @@ template <int ROWS, int NW> struct OffKS {
         for (int i = 0; i < ROWS / (16 * NW); ++i) {
             const int kr = (NW * i + w) * KPL + lane / SPR;
             const int pc = lane % SPR;                                        // physical 16-byte slot in the k-row
-            const int c = ((((pc >> 1) ^ ((kr & 3) << 1)) << 1) | (pc & 1));  // logical 16-byte chunk
+            const int c = ((((pc >> 1) ^ swz_ks(kr)) << 1) | (pc & 1));  // logical 16-byte chunk
             off[i] = (uint32_t)(min(kr, k_left - 1) * ld * 2 + min(c * 8, r_left - 8) * 2);
         }
     }
@@ -114,7 +117,7 @@ template <int ROWS, int NW> struct Off<ROWS, NW, true> : OffKS<ROWS, NW> {};
 template <int ROWS, int THREADS> __device__ __forceinline__ void zero_kc_tail(char *lds, int k_valid) {
     for (int idx = threadIdx.x; idx < ROWS * 4; idx += THREADS) {
         const int row = idx >> 2, c = idx & 3;
-        if (c * 8 >= k_valid) *reinterpret_cast<uint4 *>(lds + row * 64 + ((c ^ swz4(row)) << 4)) = make_uint4(0, 0, 0, 0);
+        if (c * 8 >= k_valid) *reinterpret_cast<uint4 *>(lds + row * 64 + ((c ^ swz16(row)) << 4)) = make_uint4(0, 0, 0, 0);
     }
 }
 // zero the k-rows [k_valid, 32) of a K-strided tile (the last, partial stage of a ragged contraction)
@@ -123,20 +126,23 @@ template <int ROWS, int THREADS> __device__ __forceinline__ void zero_k_tail(cha
         *reinterpret_cast<uint4 *>(lds + k_valid * (ROWS * 2) + idx * 16) = make_uint4(0, 0, 0, 0);
 }
 
-// ---- MFMA fragments: 8 bf16 of k for row (lane % 32) of 32-row block tb, k-sub-step kk (16 of k) --
-__device__ __forceinline__ bf16x8 frag_kc(const char *lds, int tb, int kk) {
+// ---- MFMA fragments: 8 bf16 of k (8 (lane / 16) on) for row lane % 16 of 16-row block tb; one covers the stage's 32 of k --
+// v_mfma_f32_16x16x32_bf16 and not the 32x32x16 shape of the same rate: the chip runs matrix work against its power limit,
+// and per flop the smaller shape moves half of the accumulator bytes.  Back to back on random operands held in registers
+// (256 blocks of eight waves) it sustains 1985 TFLOP/s against 1665; on zeros both reach 2450-2490.
+__device__ __forceinline__ bf16x8 frag_kc(const char *lds, int tb) {
     const int lane = threadIdx.x & 63;
-    const int row = tb * 32 + (lane & 31);
-    const int chunk = (2 * kk + (lane >> 5)) ^ swz4(row);
-    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(lds + row * 64 + chunk * 16));
+    const int row = lane & 15;
+    const int chunk = (lane >> 4) ^ swz16(row);
+    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(lds + tb * 1024 + row * 64 + chunk * 16));
 }
 // ds_read_b64_tr_b16: in a group of 16 lanes, lane 4r+q supplies the address of 4 consecutive values
 // of k-row r, and lane i receives column i of that 4 x 16 block.  Two reads give 8 of k.
-template <int ROWS> __device__ __forceinline__ bf16x8 frag_ks(const char *lds, int tb, int kk) {
+template <int ROWS> __device__ __forceinline__ bf16x8 frag_ks(const char *lds, int tb) {
     const int lane = threadIdx.x & 63;
-    const int gq = lane >> 4, l = lane & 15;
-    const int k = 16 * kk + 8 * (gq >> 1) + (l >> 2);                   // + 4 for the second read
-    const int gran = (tb * 2 + (gq & 1)) ^ ((l >> 2) << 1);            // (k & 3) == l >> 2
+    const int l = lane & 15;
+    const int k = 8 * (lane >> 4) + (l >> 2);                           // + 4 for the second read
+    const int gran = tb ^ swz_ks(k);                                    // (the same for k + 4)
     const char *a0 = lds + k * (ROWS * 2) + gran * 32 + (l & 3) * 8;
     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(a0));
     const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(a0 + 4 * ROWS * 2));
@@ -144,45 +150,64 @@ template <int ROWS> __device__ __forceinline__ bf16x8 frag_ks(const char *lds, i
     const s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     return __builtin_bit_cast(bf16x8, v);
 }
-template <bool KS, int ROWS> __device__ __forceinline__ bf16x8 frag(const char *lds, int tb, int kk) {
-    if constexpr (KS) return frag_ks<ROWS>(lds, tb, kk); else return frag_kc(lds, tb, kk);
+template <bool KS, int ROWS> __device__ __forceinline__ bf16x8 frag(const char *lds, int tb) {
+    if constexpr (KS) return frag_ks<ROWS>(lds, tb); else return frag_kc(lds, tb);
 }
 
 // first index of part P when N items are dealt to NP consecutive parts
 template <int P, int NP, int N> constexpr int part_lo() { return P * N / NP; }
 
-// The fragments one wave needs for a k-sub-step: its TMCW m-blocks (blocks wm*TMCW .. of the tile, of which
-// the tile's first TMC are fetched) and its two 32-column n-blocks.
+// The fragments one wave needs for a stage: its 2 TMCW 16-row m-blocks (those from 2 wm TMCW on of the tile, of which
+// the tile's first 2 TMC are fetched) in two halves, and its four 16-column n-blocks.  A stage is consumed in two halves of
+// four parts: part P of half H multiplies n-block P with the TMCW m-blocks of half H.  The other half of the m-side is read
+// meanwhile, and in the second half the next stage's first: n-block P has been used for the last time after part P of that
+// half and is read again in the part that follows, so that the n-side needs no second set of registers.
 template <int TMB, int WM, int WN, bool M_KS, bool N_KS, int TMC, int TMCW> struct Frags {
     typedef Tile<TMB, WM, WN> TL;
-    static constexpr int NR = TMCW ? TMCW + 2 : 0;
-    bf16x8 m[TMCW ? TMCW : 1], n[2];
-    // the fragment reads of a k-sub-step, n-side first, dealt to NP parts
-    template <int P, int NP> __device__ __forceinline__ void read_part(const char *stage, int wm, int wn, int kk) {
+    bf16x8 m[2][TMCW ? TMCW : 1], n[4];
+    __device__ __forceinline__ void read_n(const char *stage, int wn, int j) {
+        n[j] = frag<N_KS, TL::BN>(stage + Stage<TMB, WM, WN, M_KS, TMC>::M_OPERAND, wn * 4 + j);
+    }
+    template <int H> __device__ __forceinline__ void read_m(const char *stage, int wm, int i) {
+        m[H][i] = frag<M_KS, TL::BM>(stage, wm * 2 * TMCW + H * TMCW + i);
+    }
+    // the reads that go with part P of half H (H 0: from the stage that is being consumed, H 1: from the next one).  The
+    // m-side goes into the first three parts, as the half that follows needs all of it at once.
+    template <int H, int P> __device__ __forceinline__ void read_part(const char *stage, int wm, int wn) {
+        if constexpr (TMCW > 0) {
+            if constexpr (H == 0 && P == 0) read_n(stage, wn, 3);
+            if constexpr (P < 3) {
 #pragma unroll
-        for (int r = part_lo<P, NP, NR>(); r < part_lo<P + 1, NP, NR>(); ++r) {
-            if (r < 2) n[r] = frag<N_KS, TL::BN>(stage + Stage<TMB, WM, WN, M_KS, TMC>::M_OPERAND, wn * 2 + r, kk);
-            else m[r - 2] = frag<M_KS, TL::BM>(stage, wm * TMCW + r - 2, kk);
+                for (int i = part_lo<P, 3, TMCW>(); i < part_lo<P + 1, 3, TMCW>(); ++i) read_m<1 - H>(stage, wm, i);
+            }
+            if constexpr (H == 1 && P > 0) read_n(stage, wn, P - 1);
         }
     }
-    __device__ __forceinline__ void read(const char *stage, int wm, int wn, int kk) { read_part<0, 1>(stage, wm, wn, kk); }
-    // the 2 TMCW MFMAs of a k-sub-step dealt to NP parts.  SUM: the last part adds one MFMA against a block of
-    // ones, which sums one operand block over k: of the m-side (SUM 1; wave column i takes the wave row's
-    // m-block i) or of the n-side (SUM 2; wave row j takes the wave column's n-block j).
-    template <int P, int NP, int SUM> __device__ __forceinline__ void mma_part(f32x16 (&acc)[TL::TMW][2], f32x16 &sums, int wm, int wn) const {
+    // what part 0 of half 0 finds already read
+    __device__ __forceinline__ void read_first(const char *stage, int wm, int wn) {
+        if constexpr (TMCW > 0) {
 #pragma unroll
-        for (int i = part_lo<P, NP, 2 * TMCW>(); i < part_lo<P + 1, NP, 2 * TMCW>(); ++i)
-            acc[i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(n[i & 1], m[i >> 1], acc[i >> 1][i & 1], 0, 0, 0);
-        if constexpr (SUM != 0 && P == NP - 1) {
+            for (int i = 0; i < TMCW; ++i) read_m<0>(stage, wm, i);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) read_n(stage, wn, j);
+        }
+    }
+    // the MFMAs of part P of half H.  SUM adds MFMAs against a block of ones, which sum an operand's blocks over k: of the
+    // m-side (SUM 1; wave column i takes the wave row's m-blocks 2 i and 2 i + 1) or of the n-side (SUM 2; wave row j takes
+    // the wave column's n-blocks 2 j and 2 j + 1).
+    template <int H, int P, int SUM> __device__ __forceinline__ void mma_part(f32x4 (&acc)[2 * TL::TMW][4], f32x4 (&sums)[2], int wm, int wn) const {
+#pragma unroll
+        for (int i = 0; i < TMCW; ++i)
+            acc[H * TMCW + i][P] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(n[P], m[H][i], acc[H * TMCW + i][P], 0, 0, 0);
+        if constexpr (SUM != 0) {
             const bf16_t one = (bf16_t)1.0f;
             const bf16x8 ones = {one, one, one, one, one, one, one, one};
-            if constexpr (SUM == 1) {
+            if constexpr (SUM == 1 && P == 3) {
 #pragma unroll
                 for (int i = 0; i < TMCW; ++i)
-                    if (wn == i) sums = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, m[i], sums, 0, 0, 0);
-            } else {
-                if (wm == 0) sums = __builtin_amdgcn_mfma_f32_32x32x16_bf16(n[0], ones, sums, 0, 0, 0);
-                else sums = __builtin_amdgcn_mfma_f32_32x32x16_bf16(n[1], ones, sums, 0, 0, 0);
+                    if (wn == (H * TMCW + i) >> 1) sums[i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, m[H][i], sums[i & 1], 0, 0, 0);
+            } else if constexpr (SUM == 2 && H == 0) {
+                if (wm == P >> 1) sums[P & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(n[P], ones, sums[P & 1], 0, 0, 0);
             }
         }
     }
@@ -281,13 +306,13 @@ template <int B, int L, int X> __device__ __forceinline__ void wait_stages_behin
 // still be in flight), then the barrier.
 // PART (measurement only, results are then meaningless): 1 leaves out the operand loads, 2 the fragment reads of the
 // loop (the first stage's fragments are used throughout), 3 the barriers, 4 all three.
-// BIAS: the accumulators start from the bias of their columns instead of zero (bias_raw: the 8 x 4 columns a lane
+// BIAS: the accumulators start from the bias of their columns instead of zero (bias_raw: the 4 x 4 columns a lane
 // holds, fetched before the operand loads and therefore landed when the first stage has), so that the epilogue adds
 // nothing.
 template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC, int TMCW, int SUM, bool ONCE = false, int PART = 0, bool BIAS = false>
 __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, int m_ext, const bf16_t *Np, long ldn,
                                           int n0, int n_ext, int k_ext, char *smem, int wave, int wm, int wn,
-                                          f32x16 (&acc)[Tile<TMB, WM, WN>::TMW][2], f32x16 &sums, const uint2 (&bias_raw)[8]) {
+                                          f32x4 (&acc)[2 * Tile<TMB, WM, WN>::TMW][4], f32x4 (&sums)[2], const uint2 (&bias_raw)[4]) {
     typedef Tile<TMB, WM, WN> TL;
     typedef Stage<TMB, WM, WN, M_KS, TMC> SG;
     constexpr int AHEAD = SG::NSTAGE - 1, NP = 4;
@@ -331,24 +356,28 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
     __builtin_amdgcn_s_barrier();
     if constexpr (BIAS) {
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
+        for (int c = 0; c < 4; ++c) {
             float b4[4];
             unpack4(bias_raw[c], b4);
 #pragma unroll
-            for (int tm = 0; tm < TMCW; ++tm)
+            for (int tm = 0; tm < 2 * TMCW; ++tm)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[tm][c >> 2][4 * (c & 3) + j] = b4[j];
+                for (int j = 0; j < 4; ++j) acc[tm][c][j] = b4[j];
         }
     }
     fix_tail(0, 0);
-    Frags<TMB, WM, WN, M_KS, N_KS, TMC, TMCW> f0, f1;
-    f0.read(smem, wm, wn, 0);
-    if constexpr (NO_READS) f1.read(smem, wm, wn, 1);
+    Frags<TMB, WM, WN, M_KS, N_KS, TMC, TMCW> fr;
+    fr.read_first(smem, wm, wn);
+    if constexpr (NO_READS) {
+        fr.template read_part<0, 0>(smem, wm, wn);
+        fr.template read_part<0, 1>(smem, wm, wn);
+        fr.template read_part<0, 2>(smem, wm, wn);
+    }
     int cur_b = 0;                    // ring buffer of stage s
-#define MOLE_HALF(ISSUE, P, J0, N, S_LOAD, BUF, FR, STAGE_PTR, KK, FM)                                    \
+#define MOLE_PART(ISSUE, H, P, J0, N, S_LOAD, BUF, STAGE_PTR)                                    \
         if constexpr (!NO_LOADS && (ISSUE)) fd.template issue<(J0) + part_lo<P, NP, (N)>(), (J0) + part_lo<P + 1, NP, (N)>()>(S_LOAD, BUF); \
-        if constexpr (!NO_READS) FR.template read_part<P, NP>(STAGE_PTR, wm, wn, KK);                       \
-        FM.template mma_part<P, NP, SUM>(acc, sums, wm, wn);                                              \
+        if constexpr (!NO_READS) fr.template read_part<H, P>(STAGE_PTR, wm, wn);                            \
+        fr.template mma_part<H, P, SUM>(acc, sums, wm, wn);                                               \
         __builtin_amdgcn_sched_barrier(0);
     // One iteration (stage s).  ISSUE: the first half issues the rest of stage s + AHEAD - 1, the second the first
     // loads of stage s + AHEAD; WAIT: the wait for stage s + 1.
@@ -359,18 +388,18 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
         const int fill_b = free_b == 0 ? SG::NSTAGE - 1 : free_b - 1;   /* takes the rest of stage s+AHEAD-1 */   \
         const char *cur = smem + cur_b * SG::BYTES;                                                       \
         const char *nxt = smem + nxt_b * SG::BYTES;                                                       \
-        MOLE_HALF(ISSUE, 0, SPLIT ? LH : 0, SPLIT ? L - LH : 0, s + AHEAD - 1, fill_b, f1, cur, 1, f0)    \
-        MOLE_HALF(ISSUE, 1, SPLIT ? LH : 0, SPLIT ? L - LH : 0, s + AHEAD - 1, fill_b, f1, cur, 1, f0)    \
-        MOLE_HALF(ISSUE, 2, SPLIT ? LH : 0, SPLIT ? L - LH : 0, s + AHEAD - 1, fill_b, f1, cur, 1, f0)    \
-        MOLE_HALF(ISSUE, 3, SPLIT ? LH : 0, SPLIT ? L - LH : 0, s + AHEAD - 1, fill_b, f1, cur, 1, f0)    \
+        MOLE_PART(ISSUE, 0, 0, SPLIT ? LH : 0, SPLIT ? L - LH : 0, s + AHEAD - 1, fill_b, cur)             \
+        MOLE_PART(ISSUE, 0, 1, SPLIT ? LH : 0, SPLIT ? L - LH : 0, s + AHEAD - 1, fill_b, cur)             \
+        MOLE_PART(ISSUE, 0, 2, SPLIT ? LH : 0, SPLIT ? L - LH : 0, s + AHEAD - 1, fill_b, cur)             \
+        MOLE_PART(ISSUE, 0, 3, SPLIT ? LH : 0, SPLIT ? L - LH : 0, s + AHEAD - 1, fill_b, cur)             \
         WAIT;                                                                                             \
         if constexpr (!NO_BARRIERS) __builtin_amdgcn_s_barrier();                                         \
         __builtin_amdgcn_sched_barrier(0);                                                                \
         fix_tail(s + 1, nxt_b);                                                                           \
-        MOLE_HALF(ISSUE, 0, 0, SPLIT ? LH : L, s + AHEAD, free_b, f0, nxt, 0, f1)                         \
-        MOLE_HALF(ISSUE, 1, 0, SPLIT ? LH : L, s + AHEAD, free_b, f0, nxt, 0, f1)                         \
-        MOLE_HALF(ISSUE, 2, 0, SPLIT ? LH : L, s + AHEAD, free_b, f0, nxt, 0, f1)                         \
-        MOLE_HALF(ISSUE, 3, 0, SPLIT ? LH : L, s + AHEAD, free_b, f0, nxt, 0, f1)                         \
+        MOLE_PART(ISSUE, 1, 0, 0, SPLIT ? LH : L, s + AHEAD, free_b, nxt)                                  \
+        MOLE_PART(ISSUE, 1, 1, 0, SPLIT ? LH : L, s + AHEAD, free_b, nxt)                                  \
+        MOLE_PART(ISSUE, 1, 2, 0, SPLIT ? LH : L, s + AHEAD, free_b, nxt)                                  \
+        MOLE_PART(ISSUE, 1, 3, 0, SPLIT ? LH : L, s + AHEAD, free_b, nxt)                                  \
         cur_b = nxt_b;                                                                                    \
     }
     int s = 0;
@@ -381,25 +410,25 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
     const bool extra = nk >= AHEAD;
     for (; s < nk; ++s) MOLE_ITER(false, (wait_stages_behind<AHEAD - 2, L, LX>(nk - 2 - s, extra)))
 #undef MOLE_ITER
-#undef MOLE_HALF
+#undef MOLE_PART
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));   // nothing may still be writing LDS when the block retires
 }
 
-// The bias of the 8 x 4 columns a lane holds results for, as raw bf16 quadruples; fetched before the K loop
+// The bias of the 4 x 4 columns a lane holds results for, as raw bf16 quadruples; fetched before the K loop
 // so that the epilogue does not wait for it (zero bits are 0.0 in bf16).
-template <int EPI> __device__ __forceinline__ void load_bias(const GemmArgs &g, int e, int n0, int lane, int wn, uint2 (&bias_raw)[8]) {
+template <int EPI> __device__ __forceinline__ void load_bias(const GemmArgs &g, int e, int n0, int lane, int wn, uint2 (&bias_raw)[4]) {
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
+    for (int c = 0; c < 4; ++c) {
         bias_raw[c] = make_uint2(0, 0);
         if constexpr (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU) {
-            const int n = n0 + wn * 64 + (c >> 2) * 32 + 8 * (c & 3) + 4 * (lane >> 5);
+            const int n = n0 + wn * 64 + 16 * c + 4 * (lane >> 4);
             if (n < g.N) bias_raw[c] = *reinterpret_cast<const uint2 *>((const bf16_t *)g.bias + (long)e * g.N + n);
         }
     }
 }
 
-// The epilogue of one wave, whose first TMCW 32-row blocks hold live rows.  acc[tm][tn][4q+j] = C[m, n] with
-// m = m0 + 32 tm + lane%32 (m0: the wave's first row) and n = n0 + 64 wn + 32 tn + 8 q + 4 (lane/32) + j.  A wave
+// The epilogue of one wave, whose first TMCW 32-row blocks hold live rows.  acc[tm][tn][j] = C[m, n] with
+// m = m0 + 16 tm + lane%16 (m0: the wave's first row) and n = n0 + 64 wn + 16 tn + 4 (lane/16) + j.  A wave
 // owns a (32 TMW) x 64 slab of the tile.  bf16 results go through the wave's own slab of LDS (the K loop is
 // done with it) so that global memory sees whole 128-byte rows: 8 bytes per lane into LDS, then 16 bytes
 // per lane out, 8 rows per store instruction.  The pre-activation that GELU' needs comes in the same way,
@@ -407,13 +436,13 @@ template <int EPI> __device__ __forceinline__ void load_bias(const GemmArgs &g, 
 // interleaved.  live: the wave's live rows.
 // CLOSED: GELU and its derivatives by their closed forms instead of the fitted polynomials (see gemm.h).
 template <int TMB, int WM, int WN, bool WG, int EPI, int TMC, bool CLOSED>
-__device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<TMB, WM, WN>::TMW][2], char *smem, int lane, int wave,
+__device__ __forceinline__ void epilogue(const GemmArgs &g, f32x4 (&acc)[2 * Tile<TMB, WM, WN>::TMW][4], char *smem, int lane, int wave,
                                          int wn, int e, long row0, int m0, int n0, int m_ext, int live,
-                                         const uint2 (&bias_raw)[8], int split_k) {
+                                         int split_k) {
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     __syncthreads();
     if constexpr (TMC == 0) return;
-    const int lm = lane & 31, h = lane >> 5;
+    const int lm = lane & 15, h = lane >> 4;
     bf16_t *Cb = (bf16_t *)g.C;
     long crow0 = row0;
     if constexpr (WG) { crow0 = 0; Cb += (long)e * g.strideC; }
@@ -422,12 +451,11 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<T
     const int jr = lane >> 3, jc = lane & 7;        // row-in-group / 16-byte column of the wide accesses
     const bool col_ok = nw0 + jc * 8 < g.N;
 
-    // 8-byte cell (row, chunk, half): chunk ^ (row >> 1) & 7 and half ^ (row >> 4) & 1 make the 32 rows
-    // one ds_write_b64 pass touches land in 32 distinct 8-byte bank groups
+    // 16-byte chunk of a row at chunk ^ (row >> 1) & 7: the 16 rows x 16 bytes one ds_write_b64 pass writes (a lane
+    // holds half of a chunk) land in 32 distinct 8-byte bank groups
     auto slab_at = [&](int row, int chunk, int half) -> char * {
-        return slab + row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4) + ((half ^ (row >> 4)) & 1) * 8;
+        return slab + row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4) + half * 8;
     };
-    // (a 16-byte access sees the two halves of a chunk swapped on rows with bit 4 set)
     // slab -> global: rows [0, live) of the slab, 128 bytes each
     // The large results - h, a, t and the weight gradients, 134-270 MB a launch, which no block of the same
     // launch reads - leave with non-temporal stores: ordinary stores let them push the operand panels of the
@@ -452,9 +480,6 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<T
     char *const wide0 = slab + jr * 128 + ((jc ^ (jr >> 1)) << 4);
     char *const wide1 = slab + jr * 128 + ((jc ^ (jr >> 1) ^ 4) << 4);
     auto wide_cell = [&](int it) -> char * { return ((it & 1) ? wide1 : wide0) + it * 1024; };
-    auto fix_it = [&](uint4 v, int it) -> uint4 {      // rows with bit 4 set (it & 2) hold their halves swapped
-        return (it & 2) ? make_uint4(v.z, v.w, v.x, v.y) : v;
-    };
     typedef __attribute__((address_space(1))) char gchar;
     auto flush = [&](bf16_t *dst) __attribute__((always_inline)) {
         typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -464,7 +489,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<T
             uint4 v[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i)
-                if (it0 + i < TMC * 4) v[i] = fix_it(*reinterpret_cast<const uint4 *>(wide_cell(it0 + i)), it0 + i);
+                if (it0 + i < TMC * 4) v[i] = *reinterpret_cast<const uint4 *>(wide_cell(it0 + i));
             auto put = [&](int i) __attribute__((always_inline)) {
                 gchar *p = gbase + (size_t)(it0 + i) * 8 * pitch + lane_off;
                 typedef __attribute__((address_space(1))) u32x4 g_u32x4;
@@ -510,7 +535,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<T
             }
 #pragma unroll
             for (int i = 0; i < 8; ++i)
-                if (it0 + i < TMC * 4) *reinterpret_cast<uint4 *>(wide_cell(it0 + i)) = fix_it(v[i], it0 + i);
+                if (it0 + i < TMC * 4) *reinterpret_cast<uint4 *>(wide_cell(it0 + i)) = v[i];
         }
     };
 
@@ -520,50 +545,46 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<T
         if (g.K < 0) {
             float s = 0.f;
 #pragma unroll
-            for (int tm = 0; tm < TMC; ++tm)
+            for (int tm = 0; tm < 2 * TMC; ++tm)
 #pragma unroll
-                for (int tn = 0; tn < 2; ++tn)
+                for (int tn = 0; tn < 4; ++tn)
 #pragma unroll
-                    for (int q = 0; q < 16; ++q) s += acc[tm][tn][q];
+                    for (int j = 0; j < 4; ++j) s += acc[tm][tn][j];
             ((float *)g.C)[threadIdx.x] = s;
         }
         return;
     }
     if constexpr (EPI == EPI_F32) {
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
+        for (int tn = 0; tn < 4; ++tn) {
+            const int n = nw0 + tn * 16 + 4 * h;
+            if (n >= g.N) continue;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int n = nw0 + tn * 32 + 8 * q + 4 * h;
-                if (n >= g.N) continue;
-#pragma unroll
-                for (int tm = 0; tm < TMC; ++tm) {
-                    const int m = m0 + tm * 32 + lm;
-                    if (m >= m_ext) continue;
-                    *reinterpret_cast<float4 *>((float *)g.C + (crow0 + m) * g.ldc + n) =
-                        make_float4(acc[tm][tn][4 * q], acc[tm][tn][4 * q + 1], acc[tm][tn][4 * q + 2], acc[tm][tn][4 * q + 3]);
-                }
+            for (int tm = 0; tm < 2 * TMC; ++tm) {
+                const int m = m0 + tm * 16 + lm;
+                if (m >= m_ext) continue;
+                *reinterpret_cast<f32x4 *>((float *)g.C + (crow0 + m) * g.ldc + n) = acc[tm][tn];
             }
+        }
         return;
     }
     if constexpr (EPI == EPI_PART) {
         // fp32, 32 columns (128 bytes) of a row at a time through the slab: results straight from the accumulators would be
         // 32-byte pieces of 32 rows per store.  Ordinary stores: the reduction reads them next.
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn) {
-            float *dst = g.part + ((long)split_k * g.part_rows + crow0 + m0) * g.N + nw0 + tn * 32;
+        for (int half = 0; half < 2; ++half) {
+            float *dst = g.part + ((long)split_k * g.part_rows + crow0 + m0) * g.N + nw0 + half * 32;
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int q = 0; q < 2; ++q)
 #pragma unroll
-                for (int tm = 0; tm < TMC; ++tm) {
-                    const int row = tm * 32 + lm;
-                    *reinterpret_cast<float4 *>(slab + row * 128 + (((2 * q + h) ^ ((row >> 1) & 7)) << 4)) =
-                        make_float4(acc[tm][tn][4 * q], acc[tm][tn][4 * q + 1], acc[tm][tn][4 * q + 2], acc[tm][tn][4 * q + 3]);
+                for (int tm = 0; tm < 2 * TMC; ++tm) {
+                    const int row = tm * 16 + lm;
+                    *reinterpret_cast<f32x4 *>(slab + row * 128 + (((4 * q + h) ^ ((row >> 1) & 7)) << 4)) = acc[tm][2 * half + q];
                 }
             // (the slab is this wave's own: program order is enough)
 #pragma unroll
             for (int it = 0; it < TMC * 4; ++it)
-                if (it * 8 + jr < live && nw0 + tn * 32 + jc * 4 < g.N)
+                if (it * 8 + jr < live && nw0 + half * 32 + jc * 4 < g.N)
                     *reinterpret_cast<uint4 *>(dst + (long)(it * 8 + jr) * g.N + jc * 4) = *reinterpret_cast<const uint4 *>(wide_cell(it));
         }
         return;
@@ -582,38 +603,34 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<T
             if (pass == 0 && g.C == nullptr) continue;
         }
 #pragma unroll
-        for (int tn = 0; tn < 2; ++tn) {
+        for (int tn = 0; tn < 4; ++tn) {
+            // (the bias is in the accumulators already: the K loop started from it)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int n = nw0 + tn * 32 + 8 * q + 4 * h;
-                (void)n;          // (the bias is in the accumulators already: the K loop started from it)
+            for (int tm = 0; tm < 2 * TMC; ++tm) {
+                char *cell = slab_at(tm * 16 + lm, tn * 2 + (h >> 1), h & 1);
+                float v[4];
 #pragma unroll
-                for (int tm = 0; tm < TMC; ++tm) {
-                    char *cell = slab_at(tm * 32 + lm, tn * 4 + q, h);
-                    float v[4];
+                for (int j = 0; j < 4; ++j) v[j] = acc[tm][tn][j];
+                if constexpr (EPI == EPI_BIAS_GELU) {
+                    if (pass == 1) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) v[j] = acc[tm][tn][4 * q + j];
-                    if constexpr (EPI == EPI_BIAS_GELU) {
-                        if (pass == 1) {
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) v[j] = CLOSED ? gelu_erf(v[j]) : fast_gelu_erf(v[j]);
-                        }
-                    } else if constexpr (EPI == EPI_DGELU) {
-                        float hv[4];
-                        unpack4(*reinterpret_cast<const uint2 *>(cell), hv);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            v[j] *= !CLOSED ? dgelu(hv[j]) : g.gelu_bwd == MOLE_GELU_BWD_TANH ? d_gelu_tanh(hv[j]) : d_gelu_exact(hv[j]);
-                    } else if constexpr (EPI == EPI_WGRAD) {
-                        if (g.accumulate) {
-                            float old[4];
-                            unpack4(*reinterpret_cast<const uint2 *>(cell), old);
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) v[j] += old[j];
-                        }
+                        for (int j = 0; j < 4; ++j) v[j] = CLOSED ? gelu_erf(v[j]) : fast_gelu_erf(v[j]);
                     }
-                    *reinterpret_cast<uint2 *>(cell) = pack4(v[0], v[1], v[2], v[3]);
+                } else if constexpr (EPI == EPI_DGELU) {
+                    float hv[4];
+                    unpack4(*reinterpret_cast<const uint2 *>(cell), hv);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        v[j] *= !CLOSED ? dgelu(hv[j]) : g.gelu_bwd == MOLE_GELU_BWD_TANH ? d_gelu_tanh(hv[j]) : d_gelu_exact(hv[j]);
+                } else if constexpr (EPI == EPI_WGRAD) {
+                    if (g.accumulate) {
+                        float old[4];
+                        unpack4(*reinterpret_cast<const uint2 *>(cell), old);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) v[j] += old[j];
+                    }
                 }
+                *reinterpret_cast<uint2 *>(cell) = pack4(v[0], v[1], v[2], v[3]);
             }
         }
         flush(pass == 0 ? Cb : (bf16_t *)g.C2);
@@ -621,35 +638,34 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, f32x16 (&acc)[Tile<T
 }
 
 // Writes the operand sums of a weight-gradient block (see Frags::mma_part): colsum[e][i] (+)= sum over the
-// expert's rows of operand column i.  SUM 1: every register of lane l < 32 holds the sum for row l of the wave's
-// summed m-block (block wn of wave row wm); SUM 2: register 4q+j of a lane holds the sum for column
-// 8q + 4 (lane/32) + j of the wave's summed n-block (block wm of wave column wn).
+// expert's rows of operand column i.  SUM 1: every register of lane l < 16 holds the sum for row l of the wave's two
+// summed m-blocks (blocks 2 wn and 2 wn + 1 of wave row wm); SUM 2: register j of a lane holds the sum for column
+// 4 (lane/16) + j of the wave's two summed n-blocks (blocks 2 wm and 2 wm + 1 of wave column wn).
 template <int SUM, int C>
-__device__ __forceinline__ void store_sums(const GemmArgs &g, const f32x16 &sums, int e, int m0, int n0, int m_ext, int wm,
+__device__ __forceinline__ void store_sums(const GemmArgs &g, const f32x4 (&sums)[2], int e, int m0, int n0, int m_ext, int wm,
                                            int wn, int lane) {
     bf16_t *out = (bf16_t *)g.colsum;
-    if constexpr (SUM == 1) {
-        const int m = m0 + (wm * C + wn) * 32 + (lane & 31);
-        if (lane < 32 && wn < C && m < m_ext) {
-            bf16_t *p = out + (long)e * g.M + m;
-            float v = sums[0];
-            if (g.accumulate) v += (float)*p;
-            *p = (bf16_t)v;
-        }
-    } else {
-        if ((lane & 31) == 0) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+    for (int b = 0; b < 2; ++b) {
+        if constexpr (SUM == 1) {
+            const int m = m0 + (wm * C + wn) * 32 + 16 * b + (lane & 15);
+            if (lane < 16 && wn < C && m < m_ext) {
+                bf16_t *p = out + (long)e * g.M + m;
+                float v = sums[b][0];
+                if (g.accumulate) v += (float)*p;
+                *p = (bf16_t)v;
+            }
+        } else if ((lane & 15) == 0) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int n = n0 + wn * 64 + wm * 32 + 8 * q + 4 * (lane >> 5) + j;
-                    if (n < g.N) {
-                        bf16_t *p = out + (long)e * g.N + n;
-                        float v = sums[4 * q + j];
-                        if (g.accumulate) v += (float)*p;
-                        *p = (bf16_t)v;
-                    }
+            for (int j = 0; j < 4; ++j) {
+                const int n = n0 + wn * 64 + wm * 32 + 16 * b + 4 * (lane >> 4) + j;
+                if (n < g.N) {
+                    bf16_t *p = out + (long)e * g.N + n;
+                    float v = sums[b][j];
+                    if (g.accumulate) v += (float)*p;
+                    *p = (bf16_t)v;
                 }
+            }
         }
     }
 }
@@ -901,19 +917,17 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
         k_ext = k_hi - k_lo;
     }
 
-    f32x16 acc[TMW][2];
+    f32x4 acc[2 * TMW][4];
 #pragma unroll
-    for (int i = 0; i < TMW; ++i)
+    for (int i = 0; i < 2 * TMW; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
+        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int live = min(tile_h, m_ext - m0);
     const int tmc = (live + 31) >> 5;
     const int wu = __builtin_amdgcn_readfirstlane(wave);
     const int wm = wu / WN, wn = wu % WN;     // wave row / wave column
-    uint2 bias_raw[8];
+    uint2 bias_raw[4];
     load_bias<EPI>(g, e, n0, lane, wn, bias_raw);
     // Operand sums ride along in the weight-gradient blocks that see the whole operand once: one n-tile
     // of every m-tile for the m-side, one m-tile of every n-tile for the n-side.  These blocks run the
@@ -926,14 +940,12 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
     const int c = sum_side ? TMW : (tmc + WM - 1) / WM;
     const int m0w = m0 + wm * c * 32, live_w = max(0, min(live - wm * c * 32, c * 32));
     // K loop and epilogue with C blocks per wave row
-    f32x16 sums;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) sums[q] = 0.f;
+    f32x4 sums[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #define MOLE_RUN_TILE_AS(C, SUM, ONCE)                                                                                         \
     {                                                                                                                     \
         main_loop<TMB, WM, WN, M_KS, N_KS, KT, WM *(C), (C), SUM, ONCE, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw); \
         if constexpr (SUM != 0) store_sums<SUM, (C)>(g, sums, e, m0, n0, m_ext, wm, wn, lane);                            \
-        epilogue<TMB, WM, WN, WG, EPI, (C), KT && !WG>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, bias_raw, split_k);      \
+        epilogue<TMB, WM, WN, WG, EPI, (C), KT && !WG>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, split_k);      \
     }
 #define MOLE_RUN_TILE_SUM(C, SUM) MOLE_RUN_TILE_AS(C, SUM, false)
 #define MOLE_RUN_TILE(C) MOLE_RUN_TILE_AS(C, 0, false)
