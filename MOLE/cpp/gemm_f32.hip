@@ -2,19 +2,29 @@
 // (MOLE/cpp/define.hpp:152-155 - fp32 is the only type its kernels are instantiated for; the products are
 // _BatchRecord::bffn_fwd / bffn_bwd, MOLE/cpp/core.cpp:344-356, 381-414).
 //
-// v_mfma_f32_32x32x2_f32 keeps a SIMD's matrix pipe busy for 64 cycles and consumes one register of each operand,
-// so the arithmetic leaves room for everything else - as long as something else is ready to issue.  The kernel is
-// therefore built for several independent blocks per CU rather than one large one: a block of 4 waves (2 x 2) owns a
-// BM x BN tile (64 x 128 for the row-ragged products, 128 x 128 for the weight gradients), its operand stages of 16
-// of K come from HBM/L2 straight into a ring of three or four LDS stages (global_load_lds_dwordx4, one barrier per
-// stage), and the fragments of stage s+1 are read into registers while the MFMAs of stage s run, the loads and reads
-// dealt out between the MFMAs.  Two to four blocks share a CU.
+// The products run on the bf16 matrix cores.  An fp32 number is the sum of three bf16 numbers (8 + 8 + 8 significand bits), so
+// a product is nine products of parts, of which the three smallest lie below 2^-24 of it: six of v_mfma_f32_32x32x16_bf16, which
+// takes 32 cycles for 16 of k, replace eight of v_mfma_f32_32x32x2_f32 of 64 each.  Nothing is lost by it: 16 of k are summed
+// before a rounding where there were two, and measured against 64 bits the errors are 0.75-0.9 of what fp32 operands gave (8
+// experts of 1000 rows, 512 -> 2048: h 4.05e-7 -> 3.4e-7, out 8.1e-7 -> 7.0e-7, weight gradients 5.6e-7 and 7.0e-7 -> 4.8e-7 and
+// 6.0e-7).  (Parts below 1.2e-38, the smallest normal number, may count as zero.)  The bf16 matrix cores round their sums down,
+// a bias of about 2^-26 a step that a sum over rows or columns would collect: one of a wave's two m-blocks is multiplied with its
+// sign changed, so that neighbouring blocks of rows err in opposite directions (bias gradients: 4.6e-7 with fp32 operands,
+// 8.4e-7 with one sign, 4.1e-7 with both).
+// Bound: the chip's power management, as in bf16 (1.76 GHz with the matrix pipes busy 0.61 of the cycles).  Same-box figures of
+// fp32 operands and of parts, us: 8 experts of 1000 rows, 512 -> 2048: h 163 -> 128, out 143 -> 116, t 165 -> 126, gx 142 -> 112,
+// the weight gradients 145 -> 102 each; 8 of 2000, 1024 -> 4096: 1042, 1008, 1047, 997, 1020 -> 797, 706, 783, 702, 715.
+//
+// A block of four waves owns a 128 x 128 tile (2 x 2 waves) or, where that suits the rows better, a 64 x 128 tile (1 x 4); two or
+// three blocks share a CU.  Operand stages of 16 of K come as fp32 from HBM/L2 straight into a ring of four LDS stages
+// (global_load_lds_dwordx4, one barrier per stage); the fragments of stage s + 1 are read and split while the MFMAs of
+// stage s run.
 //
 // LDS images (the 16-byte piece a lane's load fills is fixed by the hardware; which global address it fetches
 // is ours to choose, so any permutation of pieces is free):
 //   * K-contiguous operand -> [row][4 x 16 B], piece index XORed with swz4(row); a ds_read_b128 gives a lane four
-//     consecutive k of its row.  MFMA step (kk, j) therefore contracts k = 8 kk + j (lanes 0-31) and 8 kk + 4 + j
-//     (lanes 32-63) - any pairing of k is as good as any other as long as both operands use the same.
+//     consecutive k of its row: k = 8 kk + j (lanes 0-31) and 8 kk + 4 + j (lanes 32-63) for piece kk, j < 4 - any order
+//     of k is as good as any other as long as both operands use the same.
 //   * K-strided operand    -> [k][rows x 4 B] as it lies in HBM, the 16-byte piece index XORed with 8 on k-rows with
 //     bit 2 set (the two k-rows one MFMA step reads then fall into different banks).  A wave's two 32-row blocks are
 //     the even and the odd rows of its 64: one ds_read_b64 per step serves both.
@@ -31,7 +41,8 @@ constexpr int F_BK = 16;          // k per stage: 64 bytes of a K-contiguous row
 constexpr int F_THREADS = 256;    // 4 waves, 2 x 2
 
 template <int BM, int BN, int NSTAGE> struct FTile {
-    static constexpr int TMW = BM / 64, TNW = BN / 64;        // 32-row blocks per wave on either side
+    static constexpr int WM = BM / 64, WN = 4 / WM;           // waves along m and n
+    static constexpr int TMW = 2, TNW = BN / 32 / WN;         // 32-row blocks per wave on either side
     static constexpr int M_BYTES = BM * F_BK * 4, N_BYTES = BN * F_BK * 4, STAGE = M_BYTES + N_BYTES;
     static constexpr int LM = BM / 64, LN = BN / 64, L = LM + LN;   // 1-KiB loads per wave and stage
     static constexpr int LDS_BYTES = NSTAGE * STAGE;
@@ -110,11 +121,255 @@ template <int ROWS, bool KS, int NB> struct FFrag {
     }
 };
 
-template <int BM, int BN, int NSTAGE, int BPC, bool M_KS, bool N_KS, bool WG, int EPI>
-__global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs g) {
+// A fragment block (8 k of one row per lane) as three bf16 numbers a value: x = hi + mid + lo exactly, each the rounding of what
+// the ones before leave (8 + 8 + 8 significand bits are the 24 of fp32).  NEG: the parts of -x.  A remainder is taken with
+// plain additions on the unpacked parts, five instructions for a pair of values and a part: v_dot2_f32_bf16 would take three,
+// but it runs on the matrix pipe (5 of them behind each of 24 MFMAs of 32 x 32 x 16: 357 -> 669 us; additions, shifts, masks
+// and conversions: 331-379).
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+struct Planes {
+    u32x4 p[3];
+    template <bool NEG> __device__ __forceinline__ void split(const float (&x)[8]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float r0 = x[2 * i], r1 = x[2 * i + 1];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                uint32_t h;
+                if constexpr (NEG) asm("v_cvt_pk_bf16_f32 %0, -%1, -%2" : "=v"(h) : "v"(r0), "v"(r1));
+                else asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h) : "v"(r0), "v"(r1));
+                p[q][i] = h;
+                if (q < 2) {
+                    const float h0 = __uint_as_float(h << 16), h1 = __uint_as_float(h & 0xffff0000u);
+                    r0 = NEG ? r0 + h0 : r0 - h0;
+                    r1 = NEG ? r1 + h1 : r1 - h1;
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ bf16x8 part(int q) const { return __builtin_bit_cast(bf16x8, p[q]); }
+};
+// the six of the nine products of two triples that fp32 accuracy needs, the smallest first
+__device__ constexpr int SPLIT_M[6] = {0, 2, 1, 0, 1, 0}, SPLIT_N[6] = {2, 0, 1, 1, 0, 0};
+
+// The K loop of one tile: acc += the products of its nk stages.
+template <int BM, int BN, int NSTAGE, bool M_KS, bool N_KS, bool WG, bool SPLIT>
+__device__ __forceinline__ void f32_loop(const GemmArgs &g, const float *Mp, const float *Np, int m0, int n0, int m_ext, int k_ext, char *smem,
+                                         int wave, int wm, int wn, f32x16 (&acc)[FTile<BM, BN, NSTAGE>::TMW][FTile<BM, BN, NSTAGE>::TNW], int sum_side,
+                                         float (&psum)[4][2]) {
     typedef FTile<BM, BN, NSTAGE> TL;
     constexpr int F_NSTAGE = NSTAGE;
     constexpr int TMW = TL::TMW, TNW = TL::TNW, L = TL::L;
+    const int nk = (k_ext + F_BK - 1) / F_BK;
+    if (nk <= 0) return;
+    const int kl = k_ext - (nk - 1) * F_BK;     // k-rows of the last stage (a row-ragged product's K is whole stages)
+    FOff<BM, M_KS> om, cm;
+    FOff<BN, N_KS> on, cn;
+    om.init(g.lda, m_ext - m0, F_BK);
+    on.init(g.ldb, g.N - n0, F_BK);
+    if constexpr (WG) { cm.init(g.lda, m_ext - m0, kl); cn.init(g.ldb, g.N - n0, kl); }
+    const char *bm = uniform_ptr(M_KS ? Mp + m0 : Mp + (long)m0 * g.lda);
+    const char *bn = uniform_ptr(N_KS ? Np + n0 : Np + (long)n0 * g.ldb);
+    const long step_m = M_KS ? g.lda * (F_BK * 4) : F_BK * 4;
+    const long step_n = N_KS ? g.ldb * (F_BK * 4) : F_BK * 4;
+    const uint32_t lds_w = lds_offset_of(smem) + wave * 1024;
+    // load j of stage s (the m-side tile's loads come first) into ring buffer s mod NSTAGE; stages are issued in
+    // order, the bases advance after a stage's last load
+    auto issue_one = [&](int s, int j) __attribute__((always_inline)) {
+        const uint32_t dst = lds_w + (s % F_NSTAGE) * TL::STAGE;
+        const bool last = WG && s == nk - 1;
+        if (j < TL::LM) {
+            uint32_t o = om.off[j];
+            if constexpr (WG) o = last ? cm.off[j] : o;
+            dma16s(bm, o, dst + j * 4096);
+        } else {
+            uint32_t o = on.off[j - TL::LM];
+            if constexpr (WG) o = last ? cn.off[j - TL::LM] : o;
+            dma16s(bn, o, dst + TL::M_BYTES + (j - TL::LM) * 4096);
+        }
+        if (j == L - 1) { bm += step_m; bn += step_n; }
+    };
+    auto issue = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < L; ++j) issue_one(s, j);
+    };
+    // ragged contraction: zero the k-rows past its end in the last stage (both tiles are [k][rows] there)
+    auto zero_tail = [&](int buf) __attribute__((always_inline)) {
+        char *b = smem + buf * TL::STAGE;
+        for (int idx = threadIdx.x; idx < (F_BK - kl) * (BM / 4); idx += F_THREADS)
+            *reinterpret_cast<float4 *>(b + kl * (BM * 4) + idx * 16) = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int idx = threadIdx.x; idx < (F_BK - kl) * (BN / 4); idx += F_THREADS)
+            *reinterpret_cast<float4 *>(b + TL::M_BYTES + kl * (BN * 4) + idx * 16) = make_float4(0.f, 0.f, 0.f, 0.f);
+        __syncthreads();
+    };
+    uint32_t fm0, fm1, fn0, fn1;
+    FFrag<BM, M_KS, TMW>::offsets(wm * TMW, fm0, fm1);
+    FFrag<BN, N_KS, TNW>::offsets(wn * TNW, fn0, fn1);
+    FFrag<BM, M_KS, TMW> ma;
+    FFrag<BN, N_KS, TNW> na;
+
+#pragma unroll
+    for (int s = 0; s < F_NSTAGE - 1; ++s)
+        if (s < nk) issue(s);
+    if (F_NSTAGE == 4 && nk >= 3) __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * L));
+    else if (nk >= 2) __builtin_amdgcn_s_waitcnt(waitcnt_vm(L));
+    else __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+    __builtin_amdgcn_s_barrier();
+    if (WG && nk == 1 && kl < F_BK) zero_tail(0);
+    if constexpr (SPLIT) {
+        Planes pa[TMW + TNW], pb[TMW + TNW];
+        auto split_block = [&](Planes (&p)[TMW + TNW], int b) __attribute__((always_inline)) {      // m-blocks first
+            float x[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[i] = b < TMW ? ma.get(b, i >> 2, i & 3) : na.get(b - TMW, i >> 2, i & 3);
+            if (b < TMW && (b & 1)) p[b].template split<true>(x);
+            else p[b].template split<false>(x);
+            // (kept where it stands, among the MFMAs: left alone the compiler moves it to the use, a stage later)
+            asm volatile("" : "+v"(p[b].p[0]), "+v"(p[b].p[1]), "+v"(p[b].p[2]));
+        };
+        auto add_sums = [&]() __attribute__((always_inline)) {
+            if constexpr (WG) {
+                if (sum_side == 1) {
+#pragma unroll
+                    for (int b = 0; b < TMW; ++b)
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) psum[i & 3][b] += ma.get(b, i >> 2, i & 3);
+                } else if (sum_side == 2) {
+#pragma unroll
+                    for (int b = 0; b < TNW; ++b)
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) psum[i & 3][b] += na.get(b, i >> 2, i & 3);
+                }
+            }
+        };
+        ma.read(smem, fm0, fm1);
+        na.read(smem + TL::M_BYTES, fn0, fn1);
+#pragma unroll
+        for (int b = 0; b < TMW + TNW; ++b) split_block(pa, b);
+        add_sums();
+#define MOLE_SPLIT_STAGE(S, PC, PN, NEXT)                                                                   \
+        {                                                                                                   \
+            const int s_ = (S);                                                                             \
+            bool refill_ = false;                                                                           \
+            const int nb_ = (s_ + 1) % F_NSTAGE;                                                            \
+            if constexpr (NEXT) {                                                                           \
+                if (F_NSTAGE == 4 && s_ + 2 < nk) __builtin_amdgcn_s_waitcnt(waitcnt_vm(L));                \
+                else __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));                                             \
+                __builtin_amdgcn_s_barrier();                                                               \
+                refill_ = s_ + F_NSTAGE - 1 < nk;                                                           \
+                if (WG && s_ + 1 == nk - 1 && kl < F_BK) zero_tail(nb_);                                    \
+                ma.read(smem + nb_ * TL::STAGE, fm0, fm1);                                                  \
+                na.read(smem + nb_ * TL::STAGE + TL::M_BYTES, fn0, fn1);                                    \
+            }                                                                                               \
+            constexpr int CELLS_ = TMW * TNW;                                                               \
+            _Pragma("unroll") for (int grp = 0; grp < 2; ++grp) {                                           \
+                MOLE_SPLIT_MFMAS(PC, grp)                                                                   \
+                if constexpr (NEXT) {                                                                       \
+                    if (refill_) {                                                                          \
+                        _Pragma("unroll") for (int j = grp * L / 2; j < (grp + 1) * L / 2; ++j) issue_one(s_ + F_NSTAGE - 1, j); \
+                    }                                                                                       \
+                }                                                                                           \
+            }                                                                                               \
+            __builtin_amdgcn_sched_barrier(0);                                                              \
+            if constexpr (NEXT) {                                                                           \
+                _Pragma("unroll") for (int b = 0; b < TMW + TNW; ++b) split_block(PN, b);                   \
+            }                                                                                               \
+            _Pragma("unroll") for (int grp = 2; grp < 6; ++grp) { MOLE_SPLIT_MFMAS(PC, grp) }               \
+            if constexpr (NEXT) {                                                                           \
+                _Pragma("unroll") for (int u = 0; u < 4 * CELLS_; ++u) {                                    \
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                                        \
+                    __builtin_amdgcn_sched_group_barrier(0x2, (44 * (TMW + TNW)) / (4 * CELLS_), 0);        \
+                }                                                                                           \
+            }                                                                                               \
+            __builtin_amdgcn_sched_barrier(0);                                                              \
+            if constexpr (NEXT) add_sums();                                                                 \
+        }
+#define MOLE_SPLIT_MFMAS(PC, grp)                                                                           \
+        _Pragma("unroll") for (int cell_ = 0; cell_ < CELLS_; ++cell_) {                                    \
+            const int tm = cell_ / TNW, tn = cell_ % TNW;                                                   \
+            acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(PC[tm].part(SPLIT_M[grp]), PC[TMW + tn].part(SPLIT_N[grp]), acc[tm][tn], 0, 0, 0); \
+        }
+        int s = 0;
+        for (; s + 2 < nk; s += 2) {
+            MOLE_SPLIT_STAGE(s, pa, pb, true)
+            MOLE_SPLIT_STAGE(s + 1, pb, pa, true)
+        }
+        if (nk - s == 2) {
+            MOLE_SPLIT_STAGE(s, pa, pb, true)
+            MOLE_SPLIT_STAGE(s + 1, pb, pa, false)
+        } else {
+            MOLE_SPLIT_STAGE(s, pa, pb, false)
+        }
+#undef MOLE_SPLIT_STAGE
+#undef MOLE_SPLIT_MFMAS
+#pragma unroll
+        for (int j = 0; j < TNW; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[1][j][q] = -acc[1][j][q];
+        return;
+    }
+    FFrag<BM, M_KS, TMW> mb;
+    FFrag<BN, N_KS, TNW> nb;
+    ma.read(smem, fm0, fm1);
+    na.read(smem + TL::M_BYTES, fn0, fn1);
+
+    // One stage: the MFMAs of stage S on the fragments MC / NC.  With NEXT, first the hand-over to stage S + 1: wait
+    // until this wave's share of it has landed, barrier; then, dealt out between the MFMAs so that the matrix pipe
+    // always has the next one waiting, the loads that refill the buffer stage S - 1 has left and the fragment reads
+    // of stage S + 1 into MN / NN.  (A wave issues in order: eight loads and reads in a row right after the barrier
+    // left the pipe idle for a tenth of a 64 x 128 tile's stage.)  NEXT is a compile-time choice: were the fragment
+    // reads under a run-time condition, the compiler could not tell how many LDS reads are outstanding at the first
+    // MFMA and would wait for all of them, the ones just issued included.
+    // Order of a stage's MFMAs: two waves on a SIMD that each alternate between two accumulators run at 0.85 of the
+    // MFMA rate on this chip (measured with operands held in registers: one, three or four accumulators in turn, or
+    // one wave per SIMD, all reach the full rate), so a wave with two cells runs its eight steps on one cell, then
+    // on the other; with four cells they take turns.
+#define MOLE_F32_STAGE(S, MC, NC, MN, NN, NEXT)                                                             \
+    {                                                                                                   \
+        const int s_ = (S);                                                                             \
+        bool refill_ = false;                                                                           \
+        const int nb_ = (s_ + 1) % F_NSTAGE;                                                            \
+        if constexpr (NEXT) {                                                                           \
+            if (F_NSTAGE == 4 && s_ + 2 < nk) __builtin_amdgcn_s_waitcnt(waitcnt_vm(L));                \
+            else __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));                                             \
+            __builtin_amdgcn_s_barrier();                                                               \
+            refill_ = s_ + F_NSTAGE - 1 < nk;                                                           \
+            if (WG && s_ + 1 == nk - 1 && kl < F_BK) zero_tail(nb_);                                    \
+        }                                                                                               \
+        constexpr int CELLS_ = TMW * TNW, NM_ = 8 * CELLS_, G_ = NM_ / 8;                               \
+        _Pragma("unroll") for (int grp = 0; grp < 8; ++grp) {                                           \
+            _Pragma("unroll") for (int u = 0; u < G_; ++u) {                                            \
+                const int n_ = grp * G_ + u;                                                            \
+                const int cell_ = CELLS_ == 2 ? n_ / 8 : n_ % CELLS_, step_ = CELLS_ == 2 ? n_ % 8 : n_ / CELLS_; \
+                const int tm = cell_ / TNW, tn = cell_ % TNW, kk = step_ / 4, j = step_ % 4;            \
+                acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(MC.get(tm, kk, j), NC.get(tn, kk, j), acc[tm][tn], 0, 0, 0); \
+            }                                                                                           \
+            if constexpr (NEXT) {                                                                       \
+                if (grp < L && refill_) issue_one(s_ + F_NSTAGE - 1, grp);                              \
+                if (grp == 0) MN.read(smem + nb_ * TL::STAGE, fm0, fm1);                                \
+                if (grp == 1) NN.read(smem + nb_ * TL::STAGE + TL::M_BYTES, fn0, fn1);                  \
+            }                                                                                           \
+            __builtin_amdgcn_sched_barrier(0);                                                          \
+        }                                                                                               \
+    }
+    int s = 0;
+    for (; s + 2 < nk; s += 2) {
+        MOLE_F32_STAGE(s, ma, na, mb, nb, true)
+        MOLE_F32_STAGE(s + 1, mb, nb, ma, na, true)
+    }
+    if (nk - s == 2) {
+        MOLE_F32_STAGE(s, ma, na, mb, nb, true)
+        MOLE_F32_STAGE(s + 1, mb, nb, ma, na, false)
+    } else {
+        MOLE_F32_STAGE(s, ma, na, mb, nb, false)
+    }
+#undef MOLE_F32_STAGE
+}
+
+template <int BM, int BN, int NSTAGE, int BPC, bool M_KS, bool N_KS, bool WG, int EPI>
+__global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs g) {
+    typedef FTile<BM, BN, NSTAGE> TL;
+    constexpr int TMW = TL::TMW, TNW = TL::TNW;
     extern __shared__ __align__(16) char smem[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -195,7 +450,7 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
         Mp += k_lo;
         Np += N_KS ? (long)k_lo * g.ldb : (long)k_lo;
     }
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / TL::WN, wn = wave % TL::WN;
 
     f32x16 acc[TMW][TNW];
 #pragma unroll
@@ -216,134 +471,38 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
             if (g.colsum_side == 2 && mt == 0 && wm == 0) sum_side = 2;
         }
     }
-    constexpr int SB = TMW > TNW ? TMW : TNW;
+    constexpr int SB = 2;
     float psum[4][SB];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int b = 0; b < SB; ++b) psum[j][b] = 0.f;
 
-    const int nk = (k_ext + F_BK - 1) / F_BK;
-    if (nk > 0) {
-        const int kl = k_ext - (nk - 1) * F_BK;     // k-rows of the last stage (a row-ragged product's K is whole stages)
-        FOff<BM, M_KS> om, cm;
-        FOff<BN, N_KS> on, cn;
-        om.init(g.lda, m_ext - m0, F_BK);
-        on.init(g.ldb, g.N - n0, F_BK);
-        if constexpr (WG) { cm.init(g.lda, m_ext - m0, kl); cn.init(g.ldb, g.N - n0, kl); }
-        const char *bm = uniform_ptr(M_KS ? Mp + m0 : Mp + (long)m0 * g.lda);
-        const char *bn = uniform_ptr(N_KS ? Np + n0 : Np + (long)n0 * g.ldb);
-        const long step_m = M_KS ? g.lda * (F_BK * 4) : F_BK * 4;
-        const long step_n = N_KS ? g.ldb * (F_BK * 4) : F_BK * 4;
-        const uint32_t lds_w = lds_offset_of(smem) + wave * 1024;
-        // load j of stage s (the m-side tile's loads come first) into ring buffer s mod NSTAGE; stages are issued in
-        // order, the bases advance after a stage's last load
-        auto issue_one = [&](int s, int j) __attribute__((always_inline)) {
-            const uint32_t dst = lds_w + (s % F_NSTAGE) * TL::STAGE;
-            const bool last = WG && s == nk - 1;
-            if (j < TL::LM) {
-                uint32_t o = om.off[j];
-                if constexpr (WG) o = last ? cm.off[j] : o;
-                dma16s(bm, o, dst + j * 4096);
-            } else {
-                uint32_t o = on.off[j - TL::LM];
-                if constexpr (WG) o = last ? cn.off[j - TL::LM] : o;
-                dma16s(bn, o, dst + TL::M_BYTES + (j - TL::LM) * 4096);
-            }
-            if (j == L - 1) { bm += step_m; bn += step_n; }
-        };
-        auto issue = [&](int s) __attribute__((always_inline)) {
+    f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, true>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, sum_side, psum);
+    // An infinity, a NaN or a value within half a unit of bf16 of the overflow limit has no finite parts: its products with
+    // a part that is zero are NaN.  A tile with any result that is not finite is computed again with fp32 operands.
+    float poison = 0.f;
 #pragma unroll
-            for (int j = 0; j < L; ++j) issue_one(s, j);
-        };
-        // ragged contraction: zero the k-rows past its end in the last stage (both tiles are [k][rows] there)
-        auto zero_tail = [&](int buf) __attribute__((always_inline)) {
-            char *b = smem + buf * TL::STAGE;
-            for (int idx = threadIdx.x; idx < (F_BK - kl) * (BM / 4); idx += F_THREADS)
-                *reinterpret_cast<float4 *>(b + kl * (BM * 4) + idx * 16) = make_float4(0.f, 0.f, 0.f, 0.f);
-            for (int idx = threadIdx.x; idx < (F_BK - kl) * (BN / 4); idx += F_THREADS)
-                *reinterpret_cast<float4 *>(b + TL::M_BYTES + kl * (BN * 4) + idx * 16) = make_float4(0.f, 0.f, 0.f, 0.f);
-            __syncthreads();
-        };
-        uint32_t fm0, fm1, fn0, fn1;
-        FFrag<BM, M_KS, TMW>::offsets(wm * TMW, fm0, fm1);
-        FFrag<BN, N_KS, TNW>::offsets(wn * TNW, fn0, fn1);
-        FFrag<BM, M_KS, TMW> ma, mb;
-        FFrag<BN, N_KS, TNW> na, nb;
-
+    for (int i = 0; i < TMW; ++i)
 #pragma unroll
-        for (int s = 0; s < F_NSTAGE - 1; ++s)
-            if (s < nk) issue(s);
-        if (F_NSTAGE == 4 && nk >= 3) __builtin_amdgcn_s_waitcnt(waitcnt_vm(2 * L));
-        else if (nk >= 2) __builtin_amdgcn_s_waitcnt(waitcnt_vm(L));
-        else __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-        __builtin_amdgcn_s_barrier();
-        if (WG && nk == 1 && kl < F_BK) zero_tail(0);
-        ma.read(smem, fm0, fm1);
-        na.read(smem + TL::M_BYTES, fn0, fn1);
-
-        // One stage: the MFMAs of stage S on the fragments MC / NC.  With NEXT, first the hand-over to stage S + 1: wait
-        // until this wave's share of it has landed, barrier; then, dealt out between the MFMAs so that the matrix pipe
-        // always has the next one waiting, the loads that refill the buffer stage S - 1 has left and the fragment reads
-        // of stage S + 1 into MN / NN.  (A wave issues in order: eight loads and reads in a row right after the barrier
-        // left the pipe idle for a tenth of a 64 x 128 tile's stage.)  NEXT is a compile-time choice: were the fragment
-        // reads under a run-time condition, the compiler could not tell how many LDS reads are outstanding at the first
-        // MFMA and would wait for all of them, the ones just issued included.
-        // Order of a stage's MFMAs: two waves on a SIMD that each alternate between two accumulators run at 0.85 of the
-        // MFMA rate on this chip (measured with operands held in registers: one, three or four accumulators in turn, or
-        // one wave per SIMD, all reach the full rate), so a wave with two cells runs its eight steps on one cell, then
-        // on the other; with four cells they take turns.
-#define MOLE_F32_STAGE(S, MC, NC, MN, NN, NEXT)                                                             \
-        {                                                                                                   \
-            const int s_ = (S);                                                                             \
-            bool refill_ = false;                                                                           \
-            const int nb_ = (s_ + 1) % F_NSTAGE;                                                            \
-            if constexpr (NEXT) {                                                                           \
-                if (F_NSTAGE == 4 && s_ + 2 < nk) __builtin_amdgcn_s_waitcnt(waitcnt_vm(L));                \
-                else __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));                                             \
-                __builtin_amdgcn_s_barrier();                                                               \
-                refill_ = s_ + F_NSTAGE - 1 < nk;                                                           \
-                if (WG && s_ + 1 == nk - 1 && kl < F_BK) zero_tail(nb_);                                    \
-            }                                                                                               \
-            constexpr int CELLS_ = TMW * TNW, NM_ = 8 * CELLS_, G_ = NM_ / 8;                               \
-            _Pragma("unroll") for (int grp = 0; grp < 8; ++grp) {                                           \
-                _Pragma("unroll") for (int u = 0; u < G_; ++u) {                                            \
-                    const int n_ = grp * G_ + u;                                                            \
-                    const int cell_ = CELLS_ == 2 ? n_ / 8 : n_ % CELLS_, step_ = CELLS_ == 2 ? n_ % 8 : n_ / CELLS_; \
-                    const int tm = cell_ / TNW, tn = cell_ % TNW, kk = step_ / 4, j = step_ % 4;            \
-                    acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(MC.get(tm, kk, j), NC.get(tn, kk, j), acc[tm][tn], 0, 0, 0); \
-                }                                                                                           \
-                if constexpr (NEXT) {                                                                       \
-                    if (grp < L && refill_) issue_one(s_ + F_NSTAGE - 1, grp);                              \
-                    if (grp == 0) MN.read(smem + nb_ * TL::STAGE, fm0, fm1);                                \
-                    if (grp == 1) NN.read(smem + nb_ * TL::STAGE + TL::M_BYTES, fn0, fn1);                  \
-                }                                                                                           \
-                __builtin_amdgcn_sched_barrier(0);                                                          \
-            }                                                                                               \
-            if constexpr (WG) {                                                                             \
-                if (sum_side == 1) {                                                                        \
-                    _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                        \
-                    _Pragma("unroll") for (int j = 0; j < 4; ++j)                                           \
-                    _Pragma("unroll") for (int b = 0; b < TMW; ++b) psum[j][b] += MC.get(b, kk, j);         \
-                } else if (sum_side == 2) {                                                                 \
-                    _Pragma("unroll") for (int kk = 0; kk < 2; ++kk)                                        \
-                    _Pragma("unroll") for (int j = 0; j < 4; ++j)                                           \
-                    _Pragma("unroll") for (int b = 0; b < TNW; ++b) psum[j][b] += NC.get(b, kk, j);         \
-                }                                                                                           \
-            }                                                                                               \
-        }
-        int s = 0;
-        for (; s + 2 < nk; s += 2) {
-            MOLE_F32_STAGE(s, ma, na, mb, nb, true)
-            MOLE_F32_STAGE(s + 1, mb, nb, ma, na, true)
-        }
-        if (nk - s == 2) {
-            MOLE_F32_STAGE(s, ma, na, mb, nb, true)
-            MOLE_F32_STAGE(s + 1, mb, nb, ma, na, false)
-        } else {
-            MOLE_F32_STAGE(s, ma, na, mb, nb, false)
-        }
-#undef MOLE_F32_STAGE
+        for (int j = 0; j < TNW; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) poison = fmaf(acc[i][j][q], 0.f, poison);
+    int *flag = reinterpret_cast<int *>(smem);
+    __syncthreads();
+    const bool bad = __ballot(poison != 0.f) != 0;      // (NaN compares unequal)
+    if (lane == 0) flag[wave] = bad;
+    __syncthreads();
+    const bool redo = (flag[0] | flag[1] | flag[2] | flag[3]) != 0;
+    if (__builtin_amdgcn_readfirstlane(redo)) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TMW; ++i)
+#pragma unroll
+            for (int j = 0; j < TNW; ++j)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
+        f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, false>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, 0, psum);
     }
 
     if constexpr (WG) {
@@ -484,7 +643,8 @@ int dispatch_f32(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_rows, h
     const int n_tiles = ceil_div(g.N, BN);
     if (wg) {
         const int tiles = g.E * ceil_div(g.M, BM) * n_tiles;
-        if (epi == EPI_WGRAD) return launch_f32<BM, BN, NSTAGE, BPC, true, true, true, EPI_WGRAD>(g, tiles, st, kid);
+        if constexpr (BM == 128)
+            if (epi == EPI_WGRAD) return launch_f32<BM, BN, NSTAGE, BPC, true, true, true, EPI_WGRAD>(g, tiles, st, kid);
         return -100;
     }
     const int rows_bound = g.offsets ? max_rows : g.single_rows;
@@ -502,42 +662,40 @@ int dispatch_f32(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_rows, h
 
 }  // namespace
 
-// Tile shapes, from same-box sweeps on the reference's configuration (8 experts of about 1000 rows, M 512, F 2048) -
-// durations in us of h = xd.w1^T + b1 | t = (go.w2^T) gelu'(h) | out = a.w2 + b2 | gx = t.w1 | the weight gradients:
-//   128 x 128, 4 stages, 2 blocks per CU    153 | 150 |  -  |  -  | 126   (256 tiles of the two K = F products: one per CU)
-//    64 x 128, 4 stages, 2 blocks per CU     -  |  -  | 127 | 124 | 131
-//    64 x 128, 4 stages, 3 blocks per CU    155 | 145 |  -  |  -  | 131
-//    64 x 128, 3 stages, 4 blocks per CU    144 | 145 |  -  |  -  | 127
-//    64 x  64, 4 stages, 4 blocks per CU    154 | 163 | 128 | 127 |  -
-//    64 x  64, 3 stages, 5 blocks per CU    152 | 159 |  -  |  -  |  -
-//   128 x 128, 3 stages, 3 blocks per CU    176 | 171 |  -  |  -  | 125
-// Row-ragged products take 64 x 128 tiles: with enough of them for four blocks per CU the shallower ring, otherwise
-// two blocks per CU with the deeper one; weight gradients take 128 x 128.
 // Whether the weight-gradient launch for g also produces the operand sums asked for in g.colsum.
 bool gemm_f32_sums_operand(const GemmArgs &g) {
     return !(g.lda % 4 || g.ldb % 4 || g.ldc % 4 || g.N % 4 || g.N < 4 || g.M % 4 || g.M < 4);
 }
 
-// The K = F products are narrow and long: their tiles, each a serial walk over K at the matrix pipes' rate, do not divide
-// evenly among the 256 CUs.  A CU works off its blocks one after the other (two side by side share the pipes), so a
-// launch takes ceil(tiles / 256) walks; split into p planes of partial results it takes ceil(p tiles / 256) / p, plus
-// the planes' way through memory and the reduction's launch.  The fewest microseconds win, by the walk's 0.55 us per
-// stage and a plane's traffic at 5 TB/s.
-static int plan_ksplit(int E, int est_rows, int N, int K) {
+// Tile height and number of planes.  A CU works off its tiles one after the other (those that share it share the pipes), so a
+// launch takes ceil(tiles / 256) walks over K.  A stage of 16 of K costs 0.45 us on a 64 x 128 tile, by itself or with others,
+// and on a 128 x 128 tile, which splits a third fewer values per MFMA, 0.81 us where it has a CU to itself and 0.70 us else; the
+// epilogue comes on top.  Same-box figures, us, of h = xd.w1^T + b1 | out = a.w2 + b2 on 64- and on 128-row tiles:
+//   8 experts of 1000 rows, 512 -> 2048: 136 | 132 and 128 | 116;  8 of 2000, 1024 -> 4096: 887 | 837 and 797 | 706;
+//   16 of 60, 1024 -> 1024: 42 | 32 and 64 | 33;  8 of 194, 512 -> 2048: 40.5 | 38 and 45 | 38.5;  3 of 3000, 256 -> 256: 24 | 20 and 30 | 20.
+// The K = F products are narrow and long and may also be split over blocks into p planes of partial results, which costs the
+// planes' way through memory at 5 TB/s and the reduction's launch.
+static double f32_cost(int bm, int p, int E, int est_rows, int N, int K, bool heavy) {
     const int active = E < est_rows ? E : est_rows;
-    if (active <= 0 || K % F_BK) return 1;
-    const int avg = ceil_div(est_rows, active);
-    const long tiles = (long)active * ceil_div(avg, 64) * ceil_div(N, 128);
-    const double walk = K / F_BK * 0.55, plane = 2.0 * est_rows * N * sizeof(float) / 5.0e6;
+    const long tiles = (long)p * active * ceil_div(ceil_div(est_rows, active), bm) * ceil_div(N, 128), rounds = (tiles + 255) / 256;
+    const double stages = K / F_BK / (double)p, planes = p > 1 ? p * (2.0 * est_rows * N * sizeof(float) / 5.0e6) + 6.0 : 0.0;
+    if (bm == 64) return rounds * (0.45 * stages + (heavy ? 2.0 : 0.0)) + planes;
+    return rounds * ((rounds == 1 ? 0.81 : 0.70) * stages + (heavy ? (rounds == 1 ? 7.0 : 4.0) : 3.0)) + planes;
+}
+static int f32_tile(int p, int E, int est_rows, int N, int K, bool heavy) {
+    if (E <= 0 || est_rows <= 0 || N <= 64) return 64;      // (half of the columns or more are padding: 64 rows pad less)
+    return f32_cost(128, p, E, est_rows, N, K, heavy) < f32_cost(64, p, E, est_rows, N, K, heavy) ? 128 : 64;
+}
+int gemm_f32_ksplit(int E, int est_rows, int N, int K) {
+    if (E <= 0 || est_rows <= 0 || K % F_BK) return 1;
     int best = 1;
-    double least = (double)((tiles + 255) / 256) * walk;
-    for (int p = 2; p <= 4 && K / p >= 16 * F_BK; ++p) {
-        const double us = (double)((p * tiles + 255) / 256) / p * walk + p * plane + 6.0;
-        if (us < least) { least = us; best = p; }
+    double least = 0.0;
+    for (int p = 1; p <= 4 && (p == 1 || K / p >= 16 * F_BK); ++p) {
+        const double us = f32_cost(f32_tile(p, E, est_rows, N, K, false), p, E, est_rows, N, K, false);
+        if (p == 1 || us < least) { least = us; best = p; }
     }
     return best;
 }
-int gemm_f32_ksplit(int E, int est_rows, int N, int K) { return plan_ksplit(E, est_rows, N, K); }
 
 int launch_gemm_f32(const GemmArgs &g0, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid) {
     GemmArgs g = g0;
@@ -547,20 +705,20 @@ int launch_gemm_f32(const GemmArgs &g0, bool a_ks, bool b_ks, bool wg, int epi, 
     if (!wg && (a_ks || g.K <= 0 || g.K % F_BK)) return -100;
     if (wg && (!a_ks || !b_ks || g.M % 4 || g.M < 4)) return -100;
     if (wg) return dispatch_f32<128, 128, 4, 2>(g, b_ks, wg, epi, max_rows, st, kid);
-    const int rows = g.offsets ? max_rows : g.single_rows;
-    const long tiles = (long)ceil_div(rows, 64) * ceil_div(g.N, 128);
     if (b_ks && g.offsets != nullptr && ws != nullptr) {
-        const int p = planes_allowed(plan_ksplit(g.E, g.est_rows, g.N, g.K), max_rows, g.est_rows, g.N);
+        const int p = planes_allowed(gemm_f32_ksplit(g.E, g.est_rows, g.N, g.K), max_rows, g.est_rows, g.N);
         if (p > 1 && ws_bytes >= (size_t)p * max_rows * g.N * sizeof(float)) {
             g.ksplit = p;
             g.part = (float *)ws;
             g.part_rows = max_rows;
-            const int rc = dispatch_f32<64, 128, 4, 2>(g, b_ks, wg, EPI_PART, max_rows, st, kid);
-            return rc != 0 ? rc : launch_plane_reduce(g, MOLE_F32, max_rows, st);
         }
     }
-    if (tiles >= 4 * 256) return dispatch_f32<64, 128, 3, 4>(g, b_ks, wg, epi, max_rows, st, kid);
-    return dispatch_f32<64, 128, 4, 2>(g, b_ks, wg, epi, max_rows, st, kid);
+    const bool heavy = epi == EPI_BIAS_GELU || epi == EPI_DGELU;
+    const int e = g.ksplit > 1 ? (int)EPI_PART : epi;
+    const int rc = f32_tile(g.ksplit, g.E, g.est_rows, g.N, g.K, heavy) == 128
+                       ? dispatch_f32<128, 128, 4, 2>(g, b_ks, wg, e, max_rows, st, kid)
+                       : dispatch_f32<64, 128, 4, 3>(g, b_ks, wg, e, max_rows, st, kid);
+    return rc != 0 || g.ksplit == 1 ? rc : launch_plane_reduce(g, MOLE_F32, max_rows, st);
 }
 
 }  // namespace mole
