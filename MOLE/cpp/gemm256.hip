@@ -745,7 +745,8 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
             n_h += hv;
             n_l += tiles_of(r) - hv;
         }
-        for (int d = WAVE / 2; d >= 1; d >>= 1) { n_h += __shfl_xor(n_h, d, WAVE); n_l += __shfl_xor(n_l, d, WAVE); }
+        n_h = wave_total(wave_scan(n_h));
+        n_l = wave_total(wave_scan(n_l));
         if ((n_h + n_l) * n_units > 16 * 256) { split = false; n_h += n_l; n_l = 0; }
         const int total_h = n_h * n_units, total_l = n_l * n_units;
         const int per_h = (total_h + 7) >> 3, per_l = (total_l + 7) >> 3;
@@ -775,19 +776,15 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
             const int r = rows_at(ee);
             const int hv = heavy_of(r);
             const int cnt = (heavy ? hv : tiles_of(r) - hv) * unit;
-            int incl = cnt;
-            for (int d = 1; d < WAVE; d <<= 1) {
-                const int y = __shfl_up(incl, d, WAVE);
-                if (lane >= d) incl += y;
-            }
+            const int incl = wave_scan(cnt);
             const unsigned long long hit = __ballot(run + incl > target);
             if (hit) {
                 const int src = __ffsll(hit) - 1;
                 found = base + src;
-                before = run + __shfl(incl - cnt, src, WAVE);
-                cnt_found = __shfl(cnt, src, WAVE);
+                before = run + __builtin_amdgcn_readlane(incl - cnt, src);
+                cnt_found = __builtin_amdgcn_readlane(cnt, src);
             }
-            run += __shfl(incl, WAVE - 1, WAVE);
+            run += wave_total(incl);
         }
         if (found < 0) return;
         e = found;
@@ -796,7 +793,7 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
             int mv = 0;
 #pragma unroll
             for (int c = 0; c < RC; ++c)
-                if ((found >> 6) == c) mv = __shfl(rows_c[c], found & 63, WAVE);
+                if ((found >> 6) == c) mv = __builtin_amdgcn_readlane(rows_c[c], found & 63);
             m_ext = (found >> 6) < RC ? mv : rows_of(e);
         }
         int mt_class = target - before;
@@ -823,7 +820,7 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
             int ov = 0;
 #pragma unroll
             for (int c = 0; c < RC; ++c)
-                if ((found >> 6) == c) ov = __shfl(off_c[c], found & 63, WAVE);
+                if ((found >> 6) == c) ov = __builtin_amdgcn_readlane(off_c[c], found & 63);
             row0 = single ? 0 : ((found >> 6) < RC ? ov : g.offsets[e]);
         }
         k_ext = g.K;

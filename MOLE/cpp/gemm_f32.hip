@@ -387,8 +387,7 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
         const int nE = single ? 1 : g.E;
         int part = 0;
         for (int ee = lane; ee < nE; ee += WAVE) part += ((single ? g.single_rows : g.kept[ee]) + BM - 1) / BM;
-        for (int d = WAVE / 2; d >= 1; d >>= 1) part += __shfl_xor(part, d, WAVE);
-        const int total = part * n_units;
+        const int total = wave_total(wave_scan(part)) * n_units;
         const int per_xcd = (total + 7) >> 3;
         const int slot = blockIdx.x >> 3;
         const int t = (blockIdx.x & 7) * per_xcd + slot;
@@ -399,18 +398,14 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
         for (int base = 0; base < nE && found < 0; base += WAVE) {
             const int ee = base + lane;
             const int tiles = ee < nE ? ((single ? g.single_rows : g.kept[ee]) + BM - 1) / BM : 0;
-            int incl = tiles;
-            for (int d = 1; d < WAVE; d <<= 1) {
-                const int y = __shfl_up(incl, d, WAVE);
-                if (lane >= d) incl += y;
-            }
+            const int incl = wave_scan(tiles);
             const unsigned long long hit = __ballot(run + incl > mtg);
             if (hit) {
                 const int src = __ffsll(hit) - 1;
                 found = base + src;
-                fmt = mtg - (run + __shfl(incl - tiles, src, WAVE));
+                fmt = mtg - (run + __builtin_amdgcn_readlane(incl - tiles, src));
             }
-            run += __shfl(incl, WAVE - 1, WAVE);
+            run += wave_total(incl);
         }
         if (found < 0) return;
         e = found; mt = fmt;

@@ -84,21 +84,17 @@ __device__ __forceinline__ bool sk_find_group(const GemmArgs &g, int target, int
         for (int c = 0; c < 4; ++c) {
             if (base + c * WAVE >= g.E) break;
             const int cnt = base + c * WAVE + lane < g.E ? (r[c] + RG - 1) / RG : 0;
-            int incl = cnt;
-            for (int d = 1; d < WAVE; d <<= 1) {
-                const int y = __shfl_up(incl, d, WAVE);
-                if (lane >= d) incl += y;
-            }
+            const int incl = wave_scan(cnt);
             const unsigned long long hit = __ballot(run + incl > target);
             if (hit) {
                 const int src = __ffsll(hit) - 1;
                 e = __builtin_amdgcn_readfirstlane(base + c * WAVE + src);
-                grp = __builtin_amdgcn_readfirstlane(target - (run + __shfl(incl - cnt, src, WAVE)));
-                rows = __builtin_amdgcn_readfirstlane(__shfl(r[c], src, WAVE));
-                row0 = __builtin_amdgcn_readfirstlane(__shfl(o[c], src, WAVE));
+                grp = target - (run + __builtin_amdgcn_readlane(incl - cnt, src));
+                rows = __builtin_amdgcn_readlane(r[c], src);
+                row0 = __builtin_amdgcn_readlane(o[c], src);
                 return true;
             }
-            run += __shfl(incl, WAVE - 1, WAVE);
+            run += wave_total(incl);
         }
     }
     return false;

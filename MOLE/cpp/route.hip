@@ -148,13 +148,9 @@ __device__ __forceinline__ void scan_pair(int32_t *__restrict__ hist, int nb, in
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int bi = c0 + u * WAVE + lane;
-            int x = v[u];
-            for (int d = 1; d < WAVE; d <<= 1) {
-                const int y = __shfl_up(x, d, WAVE);
-                if (lane >= d) x += y;
-            }
+            const int x = wave_scan(v[u]);
             if (bi < nb) hist[(size_t)pair * nb + bi] = carry + x - v[u];
-            carry += __shfl(x, WAVE - 1, WAVE);
+            carry += wave_total(x);
         }
     }
     if (lane == 0) counts[pair] = carry;
@@ -223,10 +219,7 @@ __device__ __forceinline__ float block_sum(float v, float *s16) {
 }
 __device__ __forceinline__ int block_inclusive(int v, int *s16) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int d = 1; d < WAVE; d <<= 1) {
-        const int y = __shfl_up(v, d, WAVE);
-        if (lane >= d) v += y;
-    }
+    v = wave_scan(v);
     if (lane == WAVE - 1) s16[w] = v;
     __syncthreads();
     for (int q = 0; q < w; ++q) v += s16[q];
