@@ -126,6 +126,17 @@ enum { EPI_STORE = 0, EPI_BIAS = 1, EPI_BIAS_GELU = 2, EPI_DGELU = 3, EPI_WGRAD 
        EPI_NONE = 7 /* measurement only: the K loop runs, nothing is stored; EPI_NONE + 1..4: the K loop without
                        its operand loads / its fragment reads / its barriers / all three */ };
 
+// The combine behind out = a.w2 + b2, y[i] = sum over the k choices of gates[j][i] out[row[j][i]], for the reduction of a split
+// contraction to do on its way (layer.hip).  done: it has.
+struct CombineTail {
+    const int32_t *row, *idx;   // [k][S] row of a pair (-1: dropped), its expert
+    const float *gates;         // [k][S]
+    void *y;                    // [S][N]
+    int S, k;
+    bool keep_out;              // a backward pass will read out
+    bool done;
+};
+
 struct GemmArgs {
     const void *A, *B;      // operands (see A_KS / B_KS for their layout)
     void *C, *C2;           // outputs; C2 = gelu(h) for EPI_BIAS_GELU, whose C may be null (h is then not stored)
@@ -153,6 +164,7 @@ struct GemmArgs {
     int ksplit;
     int once;               // row-ragged products with K-strided weights: see weights_pass_by()
     int est_rows;           // host's estimate of the rows of all experts together (no more than the launch's bound)
+    CombineTail *tail;      // host side only: see CombineTail (null: none)
     int m_fastest;          // row-ragged products, 256-wide kernel: number an expert's tiles m-tile first (see gemm256.hip)
 };
 

@@ -5,7 +5,7 @@
 // the separate entry points, which these two call; what goes away is the host's work between them - a tensor
 // allocation per intermediate, a foreign call with its argument conversion per step - which for short batches took
 // longer than the kernels (61 tokens, 16 experts of 1024 -> 4096: 95 us of host time for 75 us of kernels).
-#include "common.h"
+#include "gemm.h"
 
 namespace mole {
 
@@ -89,8 +89,12 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
                                  L->layout, L->scores, L->idx, L->loc, L->gates, L->row, L->counts, L->kept_rows, L->offsets,
                                  L->capacity, L->l_aux, L->workspace, L->workspace_bytes, stream)) return rc;
     if (int rc = mole_dispatch_fwd(L->x, L->dtype, L->row, L->S, L->M, L->k, L->xd, stream)) return rc;
+    // (what the combine would refuse is left to it)
+    CombineTail tail{L->row, L->idx, L->gates, y, L->S, L->k, L->forward_only == 0, false};
+    const bool tail_ok = y != nullptr && ((uintptr_t)y & 15) == 0 && L->k >= 1 && L->k <= 16;
     if (int rc = ffn_fwd(L->xd, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, est_rows(*L), L->M, L->F, L->w1, L->b1, L->w2, L->b2, L->h,
-                                 L->a, L->out, L->workspace, L->workspace_bytes, L->forward_only, (hipStream_t)stream)) return rc;
+                                 L->a, L->out, L->workspace, L->workspace_bytes, L->forward_only, tail_ok ? &tail : nullptr, (hipStream_t)stream)) return rc;
+    if (tail.done) return 0;
     return mole_combine_fwd(L->out, L->dtype, L->row, L->gates, L->S, L->M, L->k, y, stream);
 }
 

@@ -837,3 +837,30 @@ def test_layer_takes_tokens_in_other_shapes(form):
     with torch.no_grad():
         assert torch.equal(m(other, capacity_factor=0.0).view(S, M).to(y.dtype), y)
     MOLEModule.reset_instances()
+
+
+# The combine inside the reduction of a split contraction: bit for bit what the reduction and the combine give one after the other,
+# for every bound on k that the kernel is built for, columns that are no whole block, one token and several; and the backward
+# pass finds the experts' outputs it reads.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("S,M,E,k,Fd,cf", [
+    (1, 512, 8, 1, 2048, 0.0), (3, 1032, 6, 2, 2064, 0.0), (40, 264, 9, 3, 2048, 0.0), (33, 256, 16, 8, 1024, 0.0),
+    (21, 136, 12, 11, 1024, 0.0), (300, 512, 8, 2, 2048, 0.0), (300, 512, 8, 2, 2048, 0.5),
+])
+def test_combine_in_the_reduction(S, M, E, k, Fd, cf, dtype):
+    from mole_amd import hip_ops as H
+    m, x, ref = _build(S, M, E, k, Fd, dtype, seed=S + k)
+    print(f"combine in the reduction S={S} M={M} E={E} k={k} F={Fd} cf={cf} {dtype}", flush=True)
+    assert L.lib().mole_ffn_workspace_bytes(L.dtype_code(dtype), E, S * k, M, Fd) > 0
+    with torch.no_grad():
+        y = m(x, capacity_factor=cf)
+        r = m.last_route
+        xd = H.dispatch_fwd(x, r.row, S * k)
+        out, _, _ = H.ffn_fwd(xd, r.offsets, r.kept_rows, m.FC1_W_GPU.all_tensors, m.FC1_B_GPU.all_tensors,
+                              m.FC2_W_GPU.all_tensors, m.FC2_B_GPU.all_tensors)
+        want = H.combine_fwd(out, r.row, r.gates)
+    if cf == 0.0:
+        assert torch.equal(y, want)
+    else:                                  # (fewer rows than S k: the layer may split the contraction otherwise)
+        assert int((r.row < 0).sum()) > 0 and rel_err(y.float().cpu(), want.float().cpu()) < tol(dtype)
+    _run_and_compare(m, x, ref, k, cf, dtype)
