@@ -24,7 +24,6 @@ namespace mole {
 typedef float sk_f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int SK_WAVES = 8, SK_THREADS = 64 * SK_WAVES;
-constexpr int SK_NA = 4;             // KC: 16-column fragments per block (64 result columns)
 
 template <typename T> struct SkElem;
 template <> struct SkElem<bf16_t> { static constexpr int EPC = 8; };
@@ -168,14 +167,14 @@ __device__ __forceinline__ void sk_epilogue4(const GemmArgs &g, int e, long row,
 }
 
 // ---- weights [N][K] ---------------------------------------------------------------------------------------------
-// A block owns 64 result columns of one group of up to 16 MB rows; its eight waves split the contraction.  A wave has the
-// weights of two steps (eight loads of 1 KiB) in flight and waits for them before it asks for more: sixteen waves to a
+// A block owns 16 NA result columns of one group of up to 16 MB rows; its eight waves split the contraction.  A wave has the
+// weights of 8 / NA steps (eight loads of 1 KiB) in flight and waits for them before it asks for more: sixteen waves to a
 // CU, out of step with each other, keep the memory busier than eight waves with two rounds in flight each (the
 // registers allow one or the other; 256 experts of eight rows, 2048 -> 1024: 215 against 250 us, 1.07 GB of weights).
-template <typename T, int MB, int EPI>
-__device__ __forceinline__ void skinny_kc_run(const GemmArgs &g, sk_f32x4 (&red)[SK_WAVES][SK_NA][WAVE], int e, int rows, long row0,
+template <typename T, int MB, int NA, int EPI>
+__device__ __forceinline__ void skinny_kc_run(const GemmArgs &g, sk_f32x4 (&red)[SK_WAVES][NA][WAVE], int e, int rows, long row0,
                                               int m0, int n0) {
-    constexpr int EPC = SkElem<T>::EPC, KSTEP = 4 * EPC, NA = SK_NA, U = 2;
+    constexpr int EPC = SkElem<T>::EPC, KSTEP = 4 * EPC, U = 8 / NA;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i16 = lane & 15, kg = lane >> 4;
     const int steps = (g.K + KSTEP - 1) / KSTEP;
@@ -245,16 +244,16 @@ __device__ __forceinline__ void skinny_kc_run(const GemmArgs &g, sk_f32x4 (&red)
 }
 
 // MB: 16-row blocks of a group; a group with fewer live ones runs the code for those
-template <typename T, int MB, int EPI>
+template <typename T, int MB, int NA, int EPI>
 __global__ __launch_bounds__(SK_THREADS, 4) void skinny_kc_kernel(const GemmArgs g) {
-    __shared__ __align__(16) sk_f32x4 red[SK_WAVES][SK_NA][WAVE];
-    const int chunks = (g.N + 16 * SK_NA - 1) / (16 * SK_NA);
+    __shared__ __align__(16) sk_f32x4 red[SK_WAVES][NA][WAVE];
+    const int chunks = (g.N + 16 * NA - 1) / (16 * NA);
     int e, grp, rows;
     long row0;
     if (!sk_find_group<16 * MB>(g, blockIdx.x / chunks, e, grp, rows, row0)) return;
-    const int n0 = (blockIdx.x % chunks) * (16 * SK_NA), m0 = grp * (16 * MB), live = rows - m0;
-    if (MB == 1 || live <= 16) skinny_kc_run<T, 1, EPI>(g, red, e, rows, row0, m0, n0);
-    else skinny_kc_run<T, MB, EPI>(g, red, e, rows, row0, m0, n0);
+    const int n0 = (blockIdx.x % chunks) * (16 * NA), m0 = grp * (16 * MB), live = rows - m0;
+    if (MB == 1 || live <= 16) skinny_kc_run<T, 1, NA, EPI>(g, red, e, rows, row0, m0, n0);
+    else skinny_kc_run<T, MB, NA, EPI>(g, red, e, rows, row0, m0, n0);
 }
 
 // ---- weights [K][N] ---------------------------------------------------------------------------------------------
@@ -551,14 +550,26 @@ int launch_plane_reduce(const GemmArgs &g, int dtype, int max_rows, hipStream_t 
     return 0;
 }
 
-template <typename T, int MB>
-static int launch_kc(const GemmArgs &g, int epi, int groups, hipStream_t st, int kid) {
-    const dim3 grid((unsigned)(groups * ceil_div(g.N, 16 * SK_NA)));
-    if (epi == EPI_BIAS_GELU) timed_launch(kid, skinny_kc_kernel<T, MB, EPI_BIAS_GELU>, grid, dim3(SK_THREADS), 0, st, g);
-    else if (epi == EPI_DGELU) timed_launch(kid, skinny_kc_kernel<T, MB, EPI_DGELU>, grid, dim3(SK_THREADS), 0, st, g);
+template <typename T, int MB, int NA>
+static int launch_kc_na(const GemmArgs &g, int epi, int groups, hipStream_t st, int kid) {
+    const dim3 grid((unsigned)(groups * ceil_div(g.N, 16 * NA)));
+    if (epi == EPI_BIAS_GELU) timed_launch(kid, skinny_kc_kernel<T, MB, NA, EPI_BIAS_GELU>, grid, dim3(SK_THREADS), 0, st, g);
+    else if (epi == EPI_DGELU) timed_launch(kid, skinny_kc_kernel<T, MB, NA, EPI_DGELU>, grid, dim3(SK_THREADS), 0, st, g);
     else return -100;
     MOLE_LAUNCH_CHECK();
     return 0;
+}
+// 32 columns a block instead of 64 where those give a CU no more than four blocks: two share a CU, so 64 columns leave half of
+// that room empty up to 512 blocks (forward passes, 64 / 32 columns: 1 token, 64 experts of 2048 -> 8192, 256 blocks of 64 columns,
+// 49.5 / 47.7 us; 8 tokens, 8 of 1024 -> 4096, 512 blocks, 39.6 / 37.8; fp32, 1 token, 64 blocks, 31.7 / 27.9, 16 tokens, 1024
+// blocks, 103.3 / 100.7; 2048 blocks 65.7 / 65.6).  Not with groups of 32 rows, whose token loads double (24 tokens, 4 of 4096 ->
+// 4096: 71 / 80 us).
+template <typename T, int MB>
+static int launch_kc(const GemmArgs &g, int epi, int groups, hipStream_t st, int kid) {
+    if constexpr (MB == 1) {
+        if ((long)(g.E < g.est_rows ? g.E : g.est_rows) * ceil_div(g.N, 64) <= 1024) return launch_kc_na<T, MB, 2>(g, epi, groups, st, kid);
+    }
+    return launch_kc_na<T, MB, 4>(g, epi, groups, st, kid);
 }
 
 template <typename T, int MB>

@@ -731,3 +731,21 @@ def test_ffn_fp32_tiles_with_infinite_and_largest_weights(E, M, Fd, rows):
     assert float((h.cpu().double() - want)[:, 5].norm() / want[:, 5].norm()) <= 2.0 ** -22
     rest = torch.arange(Fd) != 5
     assert float((h.cpu().double() - want)[:, rest].norm() / want[:, rest].norm()) <= 2.0 ** -24 * M ** 0.5
+
+
+# Few-row products with weights [N][K]: blocks of 32 columns (up to 1024 blocks of 64) and of 64, columns that end inside either,
+# contractions of fewer steps than a block's waves and of odd numbers of them.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("E,M,Fd,rows", [(1, 24, 40, [1]), (3, 264, 72, [2, 0, 7]), (2, 520, 1048, [8, 3]), (20, 136, 4096, [1 + e % 3 for e in range(20)])])
+def test_ffn_few_rows_by_block_width(E, M, Fd, rows, dtype):
+    from mole_amd import hip_ops as H
+    print(f"few rows, block widths E={E} M={M} F={Fd} {dtype}", flush=True)
+    d = _make(E, M, Fd, rows, dtype, seed=Fd)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off, n = torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda()
+    w_out, w_h, w_gx, *w_g = _oracle_fwd_bwd(d, "tanh")
+    out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+    g = [torch.empty_like(c[k]) for k in ("w1", "b1", "w2", "b2")]
+    gx = H.ffn_bwd(c["go"], c["xd"], h, a, off, n, c["w1"], c["w2"], *g)
+    for got, want in zip((out, h, gx, *g), (w_out, w_h, w_gx, *w_g)):
+        assert rel_err(got.float().cpu(), want) < tol(dtype)
