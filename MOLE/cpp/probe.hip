@@ -2,9 +2,9 @@
 // the product's K loop sustains without an epilogue.  Not part of the MoE path (no counterpart in the reference); the
 // benchmark script runs them so that the ceilings quoted beside the products' figures come from tracked code.
 //
-//   mole_probe_mfma   every wave issues v_mfma_f32_32x32x16_bf16 back to back on operands it holds in registers
-//                     (eight waves per block, one block per CU, 128 accumulator registers per lane: the product's
-//                     own register blocking), no memory traffic inside the loop.  Operands come from a caller
+//   mole_probe_mfma   every wave issues v_mfma_f32_16x16x32_bf16, the products' instruction, back to back on operands it
+//                     holds in registers (eight waves per block, one block per CU, 128 accumulator registers per lane:
+//                     the product's own register blocking), no memory traffic inside the loop.  Operands come from a caller
 //                     buffer: zeros show the published peak, random data what the chip sustains under load.
 //   mole_probe_kloop  the product kernel itself at a row-ragged shape (C = A . B^T, both K-contiguous, like
 //                     h = xd . w1^T) with the epilogue left out: prologue + K loop (LDS-DMA feed, fragment reads,
@@ -19,29 +19,27 @@ constexpr int PROBE_THREADS = 512;
 __global__ __launch_bounds__(PROBE_THREADS, 1) void probe_mfma_kernel(const uint4 *__restrict__ operands, int iters,
                                                                       float *__restrict__ sink) {
     extern __shared__ char smem[];     // sized by the launch so that one block fills a CU, as the product's does
-    f32x16 acc[4][2];
+    f32x4 acc[8][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 m[8], n[4];
 #pragma unroll
-            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
-    bf16x8 m[4], n[2];
+    for (int i = 0; i < 8; ++i) m[i] = __builtin_bit_cast(bf16x8, operands[i * PROBE_THREADS + threadIdx.x]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) m[i] = __builtin_bit_cast(bf16x8, operands[i * PROBE_THREADS + threadIdx.x]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) n[j] = __builtin_bit_cast(bf16x8, operands[(4 + j) * PROBE_THREADS + threadIdx.x]);
+    for (int j = 0; j < 4; ++j) n[j] = __builtin_bit_cast(bf16x8, operands[(8 + j) * PROBE_THREADS + threadIdx.x]);
     for (int it = 0; it < iters; ++it) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(n[j], m[i], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(n[j], m[i], acc[i][j], 0, 0, 0);
     }
     float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) s += acc[i][j][0];
+        for (int j = 0; j < 4; ++j) s += acc[i][j][0];
     if (iters < 0) smem[threadIdx.x] = 1;
     sink[(size_t)blockIdx.x * PROBE_THREADS + threadIdx.x] = s;
 }
@@ -50,7 +48,7 @@ __global__ __launch_bounds__(PROBE_THREADS, 1) void probe_mfma_kernel(const uint
 
 using namespace mole;
 
-extern "C" size_t mole_probe_mfma_operand_bytes(void) { return (size_t)6 * PROBE_THREADS * sizeof(uint4); }
+extern "C" size_t mole_probe_mfma_operand_bytes(void) { return (size_t)12 * PROBE_THREADS * sizeof(uint4); }
 
 extern "C" int mole_probe_mfma(const void *operands, int blocks, int iters, float *sink, double *flop_out,
                                mole_stream_t stream) {
@@ -64,8 +62,8 @@ extern "C" int mole_probe_mfma(const void *operands, int blocks, int iters, floa
     timed_launch(MOLE_K_PROBE, probe_mfma_kernel, dim3(blocks), dim3(PROBE_THREADS), lds, (hipStream_t)stream,
                  (const uint4 *)operands, iters, sink);
     MOLE_LAUNCH_CHECK();
-    // 8 MFMAs of 32 x 32 x 16 (2 x 16384 flop) per wave and iteration, 8 waves per block
-    if (flop_out) *flop_out = (double)blocks * 8.0 * iters * 8.0 * 32768.0;
+    // 32 MFMAs of 16 x 16 x 32 (2 x 8192 flop) per wave and iteration, 8 waves per block
+    if (flop_out) *flop_out = (double)blocks * 8.0 * iters * 32.0 * 16384.0;
     return 0;
 }
 

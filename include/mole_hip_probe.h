@@ -13,8 +13,8 @@ extern "C" {
 /* timing id (see mole_kernel_timing_read) under which every probe launch is timed */
 #define MOLE_K_PROBE MOLE_K_RESERVED_17
 
-/* mole_probe_mfma: `blocks` blocks of eight waves issue v_mfma_f32_32x32x16_bf16 back to
- * back for `iters` rounds of 8 on operands taken once from `operands` (mole_probe_mfma_operand_bytes() bytes: zeros
+/* mole_probe_mfma: `blocks` blocks of eight waves issue v_mfma_f32_16x16x32_bf16 back to
+ * back for `iters` rounds of 32 on operands taken once from `operands` (mole_probe_mfma_operand_bytes() bytes: zeros
  * show the published peak, random bf16 data what the chip sustains); sink: blocks * 512 floats; *flop_out: flop of
  * the launch.  mole_probe_kloop: the product kernel at the shape of h = xd . w1^T (a [rows,K], b [E,N,K], experts
  * by offsets / kept_rows) with its epilogue left out - prologue, K loop and launch only; sink: 512 floats.
