@@ -106,11 +106,13 @@ inline void timed_launch(int id, void (*kernel)(KArgs...), dim3 grid, dim3 block
 }
 
 struct CombineTail;     // gemm.h
+struct DispatchHead;
 // the FFN's entry points with the caller's estimate of the rows beside their bound (ffn_gemm.hip)
 size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, int F);
 int ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, int est_rows, int M, int F,
             const void *w1, const void *b1, const void *w2, const void *b2, void *h, void *a, void *out, void *workspace,
-            size_t workspace_bytes, int forward_only, CombineTail *tail, hipStream_t st);
+            size_t workspace_bytes, int forward_only, const DispatchHead *head, CombineTail *tail, hipStream_t st);     // head: xd is the tokens
+bool ffn_fwd_takes_tokens(int dtype, int E, int max_rows, int est_rows, int M, int F);
 int ffn_bwd(const void *go, const void *xd, const void *h, const void *a, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
             int max_rows, int est_rows, int M, int F, const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2, void *g_b2,
             void *gx, int accumulate, int gelu_bwd, void *workspace, size_t workspace_bytes, hipStream_t st);

@@ -450,6 +450,7 @@ static int run_gemm(const GemmArgs &g, int max_rows, int tiles_generic, hipStrea
             if (rc != -100) return rc;
         }
     }
+    MOLE_REQUIRE(g.pair_row == nullptr, "grouped GEMM: tokens in place of dispatched rows for a kernel that reads rows");
     if constexpr (sizeof(T) == 2) {
         if (fast_path_enabled()) {
             const int rc = launch_gemm256(g, A_KS, B_KS, WG, EPI, max_rows, ws, ws_bytes, st, kid);
@@ -483,7 +484,7 @@ static int weights_pass_by(int E, int est_rows, int M, int F, size_t elem, int f
 template <typename T>
 static int ffn_fwd_t(const void *xd, const int32_t *offsets, const int32_t *kept, int E, int max_rows, int M, int F,
                      const void *w1, const void *b1, const void *w2, const void *b2, void *h, void *a, void *out,
-                     void *ws, size_t ws_bytes, int est_rows, int forward_only, CombineTail *tail, hipStream_t st) {
+                     void *ws, size_t ws_bytes, int est_rows, int forward_only, const DispatchHead *head, CombineTail *tail, hipStream_t st) {
     const int m_tiles = max_rows / TBM + E;  // every expert may end in a partial tile
     GemmArgs g{};
     g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles; g.est_rows = est_rows;
@@ -492,8 +493,10 @@ static int ffn_fwd_t(const void *xd, const int32_t *offsets, const int32_t *kept
     // (h is for the backward pass alone: a store of R F elements and a turn through LDS less where none follows; 6002 rows,
     // 16 experts, 1024 -> 4096: the pass 188.4 -> 183.0 us, and 49 MB less memory)
     g.C = forward_only ? nullptr : h; g.C2 = a; g.ldc = F; g.bias = b1;
+    if (head != nullptr) { g.pair_row = head->row; g.tokens = head->S; g.pairs = head->S * head->k; }
     if (int rc = run_gemm<T, false, false, false, EPI_BIAS_GELU>(g, max_rows, m_tiles * ceil_div(F, TBN), st, MOLE_K_FFN_FWD1)) return rc;
     // out = a . w2 + b2   (w2 [F,M]: K-strided)
+    g.pair_row = nullptr;
     g.A = a; g.lda = F; g.B = w2; g.ldb = M; g.strideB = (long)F * M; g.N = M; g.K = F;
     g.C = out; g.C2 = nullptr; g.ldc = M; g.bias = b2;
     g.once = weights_pass_by(E, est_rows, M, F, sizeof(T), forward_only);
@@ -575,17 +578,21 @@ size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, 
     return ks > 1 ? (size_t)ks * max_rows * M * sizeof(float) : 0;
 }
 
+bool ffn_fwd_takes_tokens(int dtype, int E, int max_rows, int est_rows, int M, int F) {
+    return fast_path_enabled() && gemm_skinny_takes_tokens(E, max_rows, est_rows, F, M, dtype);
+}
+
 int ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, int est_rows, int M, int F,
             const void *w1, const void *b1, const void *w2, const void *b2, void *h, void *a, void *out, void *workspace,
-            size_t workspace_bytes, int forward_only, CombineTail *tail, hipStream_t st) {
+            size_t workspace_bytes, int forward_only, const DispatchHead *head, CombineTail *tail, hipStream_t st) {
     if (int rc = check_ffn("mole_ffn_fwd", dtype, E, max_rows, M, F)) return rc;
     if (max_rows == 0) return 0;
     MOLE_REQUIRE(xd && offsets && kept_rows && w1 && b1 && w2 && b2 && (h || forward_only) && a && out, "mole_ffn_fwd: null pointer");
     MOLE_REQUIRE(al16(xd) && al16(w1) && al16(w2) && al16(h) && al16(a) && al16(out) && al16(workspace),
                  "mole_ffn_fwd: buffers must be 16-byte aligned");
     if (dtype == MOLE_BF16)
-        return ffn_fwd_t<bf16_t>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes, est_rows, forward_only, tail, st);
-    return ffn_fwd_t<float>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes, est_rows, forward_only, tail, st);
+        return ffn_fwd_t<bf16_t>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes, est_rows, forward_only, head, tail, st);
+    return ffn_fwd_t<float>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes, est_rows, forward_only, head, tail, st);
 }
 
 int ffn_bwd(const void *go, const void *xd, const void *h, const void *a, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
@@ -614,7 +621,7 @@ extern "C" int mole_ffn_fwd_ws(const void *xd, int dtype, const int32_t *offsets
                                int max_rows, int M, int F, const void *w1, const void *b1, const void *w2, const void *b2,
                                void *h, void *a, void *out, void *workspace, size_t workspace_bytes, mole_stream_t stream) {
     return ffn_fwd(xd, dtype, offsets, kept_rows, E, max_rows, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes,
-                   0, nullptr, (hipStream_t)stream);
+                   0, nullptr, nullptr, (hipStream_t)stream);
 }
 
 extern "C" int mole_ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,

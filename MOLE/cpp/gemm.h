@@ -137,6 +137,13 @@ struct CombineTail {
     bool done;
 };
 
+// The dispatch in front of h = xd.w1^T + b1, xd[row[j][i]] = x[i], for the few-row kernel to do as it reads its tokens (layer.hip)
+struct DispatchHead {
+    const int32_t *row;     // [k][S] row of a pair (-1: dropped)
+    int S, k;
+};
+constexpr int HEAD_PAIRS = 512;     // most pairs, one per thread of a block
+
 struct GemmArgs {
     const void *A, *B;      // operands (see A_KS / B_KS for their layout)
     void *C, *C2;           // outputs; C2 = gelu(h) for EPI_BIAS_GELU, whose C may be null (h is then not stored)
@@ -165,6 +172,8 @@ struct GemmArgs {
     int once;               // row-ragged products with K-strided weights: see weights_pass_by()
     int est_rows;           // host's estimate of the rows of all experts together (no more than the launch's bound)
     CombineTail *tail;      // host side only: see CombineTail (null: none)
+    const int32_t *pair_row;    // A is the tokens and not their dispatched rows: [pairs], pair p is token p % tokens (null: it is the rows)
+    int pairs, tokens;
     int m_fastest;          // row-ragged products, 256-wide kernel: number an expert's tiles m-tile first (see gemm256.hip)
 };
 
@@ -187,6 +196,7 @@ inline int planes_allowed(int ks, int max_rows, int est_rows, int N) {
 }
 // Few rows per expert (gemm_skinny.hip): weights streamed straight into fragments; -100 when the shape is not its.
 int launch_gemm_skinny(const GemmArgs &g, int dtype, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
+bool gemm_skinny_takes_tokens(int E, int max_rows, int est_rows, int N, int K, int dtype);    // as dispatched by a DispatchHead
 int gemm_skinny_ksplit(int E, int max_rows, int est_rows, int N, int K, int dtype);    // 0: not its shape
 // fp32 tiles with direct-to-LDS loads (gemm_f32.hip); -100 as above.
 int launch_gemm_f32(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);

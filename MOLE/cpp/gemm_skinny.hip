@@ -24,6 +24,7 @@ namespace mole {
 typedef float sk_f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int SK_WAVES = 8, SK_THREADS = 64 * SK_WAVES;
+static_assert(HEAD_PAIRS <= SK_THREADS, "a thread per pair");
 
 template <typename T> struct SkElem;
 template <> struct SkElem<bf16_t> { static constexpr int EPC = 8; };
@@ -172,8 +173,8 @@ __device__ __forceinline__ void sk_epilogue4(const GemmArgs &g, int e, long row,
 // CU, out of step with each other, keep the memory busier than eight waves with two rounds in flight each (the
 // registers allow one or the other; 256 experts of eight rows, 2048 -> 1024: 215 against 250 us, 1.07 GB of weights).
 template <typename T, int MB, int NA, int EPI>
-__device__ __forceinline__ void skinny_kc_run(const GemmArgs &g, sk_f32x4 (&red)[SK_WAVES][NA][WAVE], int e, int rows, long row0,
-                                              int m0, int n0) {
+__device__ __forceinline__ void skinny_kc_run(const GemmArgs &g, sk_f32x4 (&red)[SK_WAVES][NA][WAVE], const int *token, int e,
+                                              int rows, long row0, int m0, int n0) {
     constexpr int EPC = SkElem<T>::EPC, KSTEP = 4 * EPC, U = 8 / NA;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i16 = lane & 15, kg = lane >> 4;
@@ -183,7 +184,10 @@ __device__ __forceinline__ void skinny_kc_run(const GemmArgs &g, sk_f32x4 (&red)
 #pragma unroll
     for (int a = 0; a < NA; ++a) wp[a] = (const T *)g.B + (long)e * g.strideB + (long)min(n0 + 16 * a + i16, g.N - 1) * g.ldb;
 #pragma unroll
-    for (int b = 0; b < MB; ++b) xp[b] = (const T *)g.A + (row0 + min(m0 + 16 * b + i16, rows - 1)) * g.lda;
+    for (int b = 0; b < MB; ++b) {
+        const int m = min(m0 + 16 * b + i16, rows - 1);
+        xp[b] = (const T *)g.A + (EPI == EPI_BIAS_GELU && g.pair_row != nullptr ? (long)min((unsigned)token[m - m0], (unsigned)g.tokens - 1u) : row0 + m) * g.lda;
+    }
     sk_f32x4 acc[NA][MB];
 #pragma unroll
     for (int a = 0; a < NA; ++a)
@@ -243,17 +247,32 @@ __device__ __forceinline__ void skinny_kc_run(const GemmArgs &g, sk_f32x4 (&red)
     }
 }
 
-// MB: 16-row blocks of a group; a group with fewer live ones runs the code for those
+// MB: 16-row blocks of a group; a group with fewer live ones runs the code for those.  With g.pair_row every block finds the tokens
+// of its rows for itself, a pair per thread: the pairs' rows arrive while the block looks its group up, where a launch in front of
+// this one is 2 us of latency for a few kilobytes.  Passes with a dispatch / without: 1 token, 64 experts of 2048 -> 8192, 47.9 /
+// 45.7 us; 8 tokens, 8 of 1024 -> 4096, 37.4 / 35.5; 256 tokens top-2, 32 of 512 -> 1024, 512 pairs, 39.7 / 37.6; fp32, 1 token, 8 of
+// 1024 -> 4096, 28.9 / 26.3, 128 tokens top-2, 32 of 512 -> 1024, 49.8 / 48.1.
 template <typename T, int MB, int NA, int EPI>
 __global__ __launch_bounds__(SK_THREADS, 4) void skinny_kc_kernel(const GemmArgs g) {
     __shared__ __align__(16) sk_f32x4 red[SK_WAVES][NA][WAVE];
+    __shared__ int token[16 * MB];
     const int chunks = (g.N + 16 * NA - 1) / (16 * NA);
     int e, grp, rows;
     long row0;
+    int pair = -1;
+    if constexpr (EPI == EPI_BIAS_GELU)
+        if (g.pair_row != nullptr && threadIdx.x < (unsigned)g.pairs) pair = g.pair_row[threadIdx.x];
     if (!sk_find_group<16 * MB>(g, blockIdx.x / chunks, e, grp, rows, row0)) return;
+    if constexpr (EPI == EPI_BIAS_GELU) {
+        if (g.pair_row != nullptr) {
+            const long r = pair - (row0 + grp * (16 * MB));
+            if (pair >= 0 && r >= 0 && r < 16 * MB) token[r] = threadIdx.x % (unsigned)g.tokens;
+            __syncthreads();
+        }
+    }
     const int n0 = (blockIdx.x % chunks) * (16 * NA), m0 = grp * (16 * MB), live = rows - m0;
-    if (MB == 1 || live <= 16) skinny_kc_run<T, 1, NA, EPI>(g, red, e, rows, row0, m0, n0);
-    else skinny_kc_run<T, MB, NA, EPI>(g, red, e, rows, row0, m0, n0);
+    if (MB == 1 || live <= 16) skinny_kc_run<T, 1, NA, EPI>(g, red, token, e, rows, row0, m0, n0);
+    else skinny_kc_run<T, MB, NA, EPI>(g, red, token, e, rows, row0, m0, n0);
 }
 
 // ---- weights [K][N] ---------------------------------------------------------------------------------------------
@@ -533,6 +552,12 @@ static bool tiles_split(int dtype, int E, int max_rows, int est_rows, int N, int
     if (dtype != MOLE_BF16) return true;
     const int ks = gemm256_ksplit(E, est_rows, N, K);
     return ks <= 1 || (planes_allowed(ks, max_rows, est_rows, N) == ks && ws_bytes >= (size_t)ks * max_rows * N * sizeof(float));
+}
+
+bool gemm_skinny_takes_tokens(int E, int max_rows, int est_rows, int N, int K, int dtype) {
+    const int epc = dtype == MOLE_BF16 ? 8 : 4;
+    SkinnyPlan p;
+    return max_rows > 0 && N % epc == 0 && K % epc == 0 && skinny_plan(dtype, false, E, est_rows, N, K, true, p);
 }
 
 int gemm_skinny_ksplit(int E, int max_rows, int est_rows, int N, int K, int dtype) {

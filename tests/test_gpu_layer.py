@@ -864,3 +864,33 @@ def test_combine_in_the_reduction(S, M, E, k, Fd, cf, dtype):
     else:                                  # (fewer rows than S k: the layer may split the contraction otherwise)
         assert int((r.row < 0).sum()) > 0 and rel_err(y.float().cpu(), want.float().cpu()) < tol(dtype)
     _run_and_compare(m, x, ref, k, cf, dtype)
+
+
+# Few tokens without a backward pass: the first product reads the tokens themselves.  Bit for bit what dispatched rows give, for one
+# pair, as many as a block has threads and one more; groups of 16 and of 32 rows, many of them in one expert (heavy); widths that
+# end inside a step; dropped pairs.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("S,M,E,k,Fd,cf,heavy", [
+    (1, 256, 8, 1, 512, 0.0, False), (5, 264, 6, 5, 1032, 0.0, False), (512, 256, 64, 1, 512, 0.0, False),
+    (171, 256, 64, 3, 512, 0.0, False), (400, 136, 32, 1, 520, 0.0, True), (400, 136, 64, 1, 520, 0.0, True),
+    (128, 256, 64, 4, 512, 0.0, False), (400, 256, 32, 1, 512, 0.5, True),
+])
+def test_tokens_in_place_of_dispatched_rows(S, M, E, k, Fd, cf, heavy, dtype):
+    from mole_amd import hip_ops as H
+    m, x, _ = _build(S, M, E, k, Fd, dtype, seed=S + E)
+    print(f"tokens in place of rows S={S} M={M} E={E} k={k} F={Fd} cf={cf} heavy={heavy} {dtype}", flush=True)
+    with torch.no_grad():
+        if heavy:                          # about half of the tokens choose expert 1
+            m.gate[0].linear.weight[1] *= 20.0
+        y = m(x, capacity_factor=cf)
+        r = m.last_route
+        if heavy and cf == 0.0:
+            assert int(r.kept_rows.max()) > 100
+        xd = H.dispatch_fwd(x, r.row, S * k)
+        out, _, _ = H.ffn_fwd(xd, r.offsets, r.kept_rows, m.FC1_W_GPU.all_tensors, m.FC1_B_GPU.all_tensors,
+                              m.FC2_W_GPU.all_tensors, m.FC2_B_GPU.all_tensors)
+        want = H.combine_fwd(out, r.row, r.gates)
+    if cf == 0.0:
+        assert torch.equal(y, want)
+    else:                                  # (fewer rows than S k: the layer may split the contraction otherwise)
+        assert int((r.row < 0).sum()) > 0 and rel_err(y.float().cpu(), want.float().cpu()) < tol(dtype)
