@@ -267,7 +267,7 @@ int mole_ffn_bwd_ws(const void *go, const void *xd, const void *h, const void *a
  * caller's; d_l_aux: NULL or the gradient of l_aux. */
 typedef struct mole_layer {
     int32_t dtype, S, M, E, k, F, rows, layout, normalize_gate;
-    int32_t forward_only;              /* no backward pass follows: h is not stored, and may be null */
+    int32_t forward_only;              /* no backward pass follows: h is not stored, and may be null; xd and out are scratch */
     double capacity_factor;
     const void *x;
     const float *wg, *logit_bias;
