@@ -1105,10 +1105,7 @@ static TilePlan tile_plan(int E, int est_rows, int N, int K, bool tall) {
     } else if (few) {
         p.tile = TILE_128;
         const long t128 = (long)active * ceil_div(full, 128) * ceil_div(N, 128);
-        // (a contraction that ends inside a stage walks slower, 0.41 us a stage against 0.31: split until two blocks share a CU, out
-        // and gx of 16 experts of 128 rows, 520 -> 1416, in two planes: the training pass of two micro-batches 367 -> 356 us, of one with
-        // its 1026 tokens 156.7 -> 152.5.  Whole stages lose by it: 8 of 200 rows, 1024 -> 2048, three planes instead of two, 146 -> 153.)
-        const long fit = (K % Q_BK ? 512 : 256) / t128, most = K / 512;
+        const long fit = 256 / t128, most = K / 512;
         p.ksplit = (int)(fit < most ? fit : most);
         p.ksplit = p.ksplit < 1 ? 1 : (p.ksplit > 4 ? 4 : p.ksplit);
     }

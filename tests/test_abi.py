@@ -240,3 +240,13 @@ def test_fp32_products_leave_the_few_row_kernel_at_48_rows():
     from mole_amd import _lib as L
     ws = lambda rows: L.lib().mole_ffn_workspace_bytes(L.MOLE_F32, 16, rows, 1024, 4096)
     assert ws(16 * 48) == 0 and ws(16 * 48 + 1) > 0
+
+
+def test_bf16_planes_of_widths_that_end_inside_a_stage():
+    """A contraction that ends inside a stage is split into as many planes as one of whole stages with the same tiles: its sums
+    keep their order (one plane at 16 experts of 128 rows, 520 -> 1416)."""
+    from mole_amd import _lib as L
+    planes = lambda E, rows, M, F: L.lib().mole_ffn_workspace_bytes(L.MOLE_BF16, E, rows, M, F) / (4 * rows * M)
+    for E, rows, M, F in ((16, 2052, 520, 1416), (16, 4104, 520, 1416), (8, 1600, 1032, 2056), (20, 2600, 264, 1032), (8, 800, 520, 1032)):
+        assert planes(E, rows, M, F) == planes(E, rows, M, F // 32 * 32), (E, rows, M, F)
+    assert planes(16, 2052, 520, 1416) == 0
