@@ -2,18 +2,23 @@
 // (MOLE/cpp/define.hpp:152-155 - fp32 is the only type its kernels are instantiated for; the products are
 // _BatchRecord::bffn_fwd / bffn_bwd, MOLE/cpp/core.cpp:344-356, 381-414).
 //
-// The products run on the bf16 matrix cores.  An fp32 number is the sum of three bf16 numbers (8 + 8 + 8 significand bits), so
-// a product is nine products of parts, of which the three smallest lie below 2^-24 of it: six of v_mfma_f32_32x32x16_bf16, which
-// takes 32 cycles for 16 of k, replace eight of v_mfma_f32_32x32x2_f32 of 64 each.  Nothing is lost by it: 16 of k are summed
-// before a rounding where there were two, and measured against 64 bits the errors are 0.75-0.9 of what fp32 operands gave (8
-// experts of 1000 rows, 512 -> 2048: h 4.05e-7 -> 3.4e-7, out 8.1e-7 -> 7.0e-7, weight gradients 5.6e-7 and 7.0e-7 -> 4.8e-7 and
-// 6.0e-7).  (Parts below 1.2e-38, the smallest normal number, may count as zero.)  The bf16 matrix cores round their sums down,
-// a bias of about 2^-26 a step that a sum over rows or columns would collect: one of a wave's two m-blocks is multiplied with its
-// sign changed, so that neighbouring blocks of rows err in opposite directions (bias gradients: 4.6e-7 with fp32 operands,
-// 8.4e-7 with one sign, 4.1e-7 with both).
-// Bound: the chip's power management, as in bf16 (1.76 GHz with the matrix pipes busy 0.61 of the cycles).  Same-box figures of
-// fp32 operands and of parts, us: 8 experts of 1000 rows, 512 -> 2048: h 163 -> 128, out 143 -> 116, t 165 -> 126, gx 142 -> 112,
-// the weight gradients 145 -> 102 each; 8 of 2000, 1024 -> 4096: 1042, 1008, 1047, 997, 1020 -> 797, 706, 783, 702, 715.
+// The products run on the bf16 matrix cores.  An fp32 number of 2^-110 or more is the sum of three bf16 numbers (8 + 8 + 8
+// significand bits; bf16 ends at 2^-133), so a product is nine products of parts, of which the three smallest, together 2^-24
+// of it at most and 2^-27 in the root mean square, are left out: six of v_mfma_f32_32x32x16_bf16, which takes 32 cycles for 16 of k, replace eight of
+// v_mfma_f32_32x32x2_f32 of 64 each.
+// Accuracy.  The matrix cores round to nearest, eight of k at a time in bf16 and one at a time in fp32, and cut off what lies far
+// below the accumulator: 0.004 units of its last place an instruction, always downwards.  The products hi hi have an accumulator of
+// their own, in which they are near its size; the five smaller ones go into a second, whose last place is 2^-8 of the first's, and
+// the two are added once.  That leaves two roundings for 16 of k where fp32 operands take sixteen and no drift that the
+// roundings do not cover, in one result or in a sum over many.  2-norm errors against 64 bits with fp32 operands / here, in 2^-24:
+// 8 experts of 1000 rows, 512 -> 2048: h 6.8 / 2.2, out 7.9 / 2.8, weight gradients 9.6 and 11.8 / 3.4 and 3.8, bias gradient of
+// b1 7.8 / 4.2; all operands positive: h 5.3 / 2.0, out 3.6 / 1.5, weight gradients 7.8 / 2.9; 2048 -> 4096, 300 rows, positive: h
+// 10.3 / 3.7, mean error 0.04 / 0.03.  Only a sum of a single product is no closer: 0.42 / 0.44.  (One accumulator for all six:
+// 0.75-0.9 of fp32 operands' error, but a drift of 0.02 units a stage.)
+// A tile whose operands include a number below 2^-110 that is not zero, or whose results are not all finite, is computed again
+// from fp32 operands.  All rows of a tile take the same steps, so equal rows give equal results.
+// Time, fp32 operands / parts on one box, us: 8 experts of 1000 rows, 512 -> 2048: h 154 / 128, out 135 / 115, t 154 / 125, gx 133 /
+// 112, the weight gradients 136 / 108 each; 8 of 2000, 1024 -> 4096: 1036, 1004, 1047, 993, 1010 / 838, 756, 833, 750, 788.
 //
 // A block of four waves owns a 128 x 128 tile (2 x 2 waves) or, where that suits the rows better, a 64 x 128 tile (1 x 4); two or
 // three blocks share a CU.  Operand stages of 16 of K come as fp32 from HBM/L2 straight into a ring of four LDS stages
@@ -121,47 +126,51 @@ template <int ROWS, bool KS, int NB> struct FFrag {
     }
 };
 
-// A fragment block (8 k of one row per lane) as three bf16 numbers a value: x = hi + mid + lo exactly, each the rounding of what
-// the ones before leave (8 + 8 + 8 significand bits are the 24 of fp32).  NEG: the parts of -x.  A remainder is taken with
+// A fragment block (8 k of one row per lane) as three bf16 numbers a value: x = hi + mid + lo, each the rounding of what the ones
+// before leave (8 + 8 + 8 significand bits are the 24 of fp32; exact from 2^-110 on).  A remainder is taken with
 // plain additions on the unpacked parts, five instructions for a pair of values and a part: v_dot2_f32_bf16 would take three,
 // but it runs on the matrix pipe (5 of them behind each of 24 MFMAs of 32 x 32 x 16: 357 -> 669 us; additions, shifts, masks
 // and conversions: 331-379).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 struct Planes {
     u32x4 p[3];
-    template <bool NEG> __device__ __forceinline__ void split(const float (&x)[8]) {
+    // least: the smallest of the numbers met so far, as the bits of its magnitude doubled, less one (zero: the largest)
+    __device__ __forceinline__ void split(const float (&x)[8], uint32_t &least) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             float r0 = x[2 * i], r1 = x[2 * i + 1];
+            const uint32_t u0 = (__float_as_uint(r0) << 1) - 1u, u1 = (__float_as_uint(r1) << 1) - 1u;
+            asm("v_min3_u32 %0, %0, %1, %2" : "+v"(least) : "v"(u0), "v"(u1));
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
                 uint32_t h;
-                if constexpr (NEG) asm("v_cvt_pk_bf16_f32 %0, -%1, -%2" : "=v"(h) : "v"(r0), "v"(r1));
-                else asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h) : "v"(r0), "v"(r1));
+                asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h) : "v"(r0), "v"(r1));
                 p[q][i] = h;
                 if (q < 2) {
-                    const float h0 = __uint_as_float(h << 16), h1 = __uint_as_float(h & 0xffff0000u);
-                    r0 = NEG ? r0 + h0 : r0 - h0;
-                    r1 = NEG ? r1 + h1 : r1 - h1;
+                    r0 -= __uint_as_float(h << 16);
+                    r1 -= __uint_as_float(h & 0xffff0000u);
                 }
             }
         }
     }
     __device__ __forceinline__ bf16x8 part(int q) const { return __builtin_bit_cast(bf16x8, p[q]); }
 };
-// the six of the nine products of two triples that fp32 accuracy needs, the smallest first
+// The smallest number whose three parts are sure to be exact: bf16 ends at 2^-133, 23 bits below it.
+constexpr float PARTS_MIN = 0x1p-110f;
+// the six of the nine products of two triples that fp32 accuracy needs, those of the last parts first
 __device__ constexpr int SPLIT_M[6] = {0, 2, 1, 0, 1, 0}, SPLIT_N[6] = {2, 0, 1, 1, 0, 0};
 
-// The K loop of one tile: acc += the products of its nk stages.
+// The K loop of one tile: acc += the products of its nk stages.  SPLIT: by the parts of the operands; returns whether this lane
+// met an operand that has no exact parts.
 template <int BM, int BN, int NSTAGE, bool M_KS, bool N_KS, bool WG, bool SPLIT>
-__device__ __forceinline__ void f32_loop(const GemmArgs &g, const float *Mp, const float *Np, int m0, int n0, int m_ext, int k_ext, char *smem,
+__device__ __forceinline__ bool f32_loop(const GemmArgs &g, const float *Mp, const float *Np, int m0, int n0, int m_ext, int k_ext, char *smem,
                                          int wave, int wm, int wn, f32x16 (&acc)[FTile<BM, BN, NSTAGE>::TMW][FTile<BM, BN, NSTAGE>::TNW], int sum_side,
                                          float (&psum)[4][2]) {
     typedef FTile<BM, BN, NSTAGE> TL;
     constexpr int F_NSTAGE = NSTAGE;
     constexpr int TMW = TL::TMW, TNW = TL::TNW, L = TL::L;
     const int nk = (k_ext + F_BK - 1) / F_BK;
-    if (nk <= 0) return;
+    if (nk <= 0) return false;
     const int kl = k_ext - (nk - 1) * F_BK;     // k-rows of the last stage (a row-ragged product's K is whole stages)
     FOff<BM, M_KS> om, cm;
     FOff<BN, N_KS> on, cn;
@@ -218,12 +227,19 @@ __device__ __forceinline__ void f32_loop(const GemmArgs &g, const float *Mp, con
     if (WG && nk == 1 && kl < F_BK) zero_tail(0);
     if constexpr (SPLIT) {
         Planes pa[TMW + TNW], pb[TMW + TNW];
+        f32x16 low[TMW][TNW];           // the products below hi hi
+#pragma unroll
+        for (int i = 0; i < TMW; ++i)
+#pragma unroll
+            for (int j = 0; j < TNW; ++j)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) low[i][j][q] = 0.f;
+        uint32_t least = 0xffffffffu;
         auto split_block = [&](Planes (&p)[TMW + TNW], int b) __attribute__((always_inline)) {      // m-blocks first
             float x[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) x[i] = b < TMW ? ma.get(b, i >> 2, i & 3) : na.get(b - TMW, i >> 2, i & 3);
-            if (b < TMW && (b & 1)) p[b].template split<true>(x);
-            else p[b].template split<false>(x);
+            p[b].split(x, least);
             // (kept where it stands, among the MFMAs: left alone the compiler moves it to the use, a stage later)
             asm volatile("" : "+v"(p[b].p[0]), "+v"(p[b].p[1]), "+v"(p[b].p[2]));
         };
@@ -244,9 +260,9 @@ __device__ __forceinline__ void f32_loop(const GemmArgs &g, const float *Mp, con
         };
         ma.read(smem, fm0, fm1);
         na.read(smem + TL::M_BYTES, fn0, fn1);
+        add_sums();
 #pragma unroll
         for (int b = 0; b < TMW + TNW; ++b) split_block(pa, b);
-        add_sums();
 #define MOLE_SPLIT_STAGE(S, PC, PN, NEXT)                                                                   \
         {                                                                                                   \
             const int s_ = (S);                                                                             \
@@ -272,41 +288,48 @@ __device__ __forceinline__ void f32_loop(const GemmArgs &g, const float *Mp, con
             }                                                                                               \
             __builtin_amdgcn_sched_barrier(0);                                                              \
             if constexpr (NEXT) {                                                                           \
+                add_sums();                                                                                 \
                 _Pragma("unroll") for (int b = 0; b < TMW + TNW; ++b) split_block(PN, b);                   \
             }                                                                                               \
             _Pragma("unroll") for (int grp = 2; grp < 6; ++grp) { MOLE_SPLIT_MFMAS(PC, grp) }               \
             if constexpr (NEXT) {                                                                           \
                 _Pragma("unroll") for (int u = 0; u < 4 * CELLS_; ++u) {                                    \
                     __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                                        \
-                    __builtin_amdgcn_sched_group_barrier(0x2, (44 * (TMW + TNW)) / (4 * CELLS_), 0);        \
+                    __builtin_amdgcn_sched_group_barrier(0x2, (56 * (TMW + TNW)) / (4 * CELLS_), 0);        \
                 }                                                                                           \
             }                                                                                               \
             __builtin_amdgcn_sched_barrier(0);                                                              \
-            if constexpr (NEXT) add_sums();                                                                 \
         }
 #define MOLE_SPLIT_MFMAS(PC, grp)                                                                           \
         _Pragma("unroll") for (int cell_ = 0; cell_ < CELLS_; ++cell_) {                                    \
             const int tm = cell_ / TNW, tn = cell_ % TNW;                                                   \
-            acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(PC[tm].part(SPLIT_M[grp]), PC[TMW + tn].part(SPLIT_N[grp]), acc[tm][tn], 0, 0, 0); \
+            f32x16 &to_ = SPLIT_M[grp] + SPLIT_N[grp] == 0 ? acc[tm][tn] : low[tm][tn];                     \
+            to_ = __builtin_amdgcn_mfma_f32_32x32x16_bf16(PC[tm].part(SPLIT_M[grp]), PC[TMW + tn].part(SPLIT_N[grp]), to_, 0, 0, 0); \
         }
+        // The loop does two stages, the last one no other follows.  (Peeled at the end, for even and odd numbers, the stages cost the
+        // 128 x 128 tiles 80 spilled registers; a reload waits for the operand loads in flight: 1140 us for 735, the training pass of
+        // 8 experts, 512 -> 2048, 4096 tokens top-2.)
         int s = 0;
-        for (; s + 2 < nk; s += 2) {
+        if ((nk & 1) == 0) {
+            MOLE_SPLIT_STAGE(0, pa, pb, true)
+#pragma unroll
+            for (int b = 0; b < TMW + TNW; ++b) pa[b] = pb[b];
+            s = 1;
+        }
+        for (; s + 1 < nk; s += 2) {
             MOLE_SPLIT_STAGE(s, pa, pb, true)
             MOLE_SPLIT_STAGE(s + 1, pb, pa, true)
         }
-        if (nk - s == 2) {
-            MOLE_SPLIT_STAGE(s, pa, pb, true)
-            MOLE_SPLIT_STAGE(s + 1, pb, pa, false)
-        } else {
-            MOLE_SPLIT_STAGE(s, pa, pb, false)
-        }
+        MOLE_SPLIT_STAGE(s, pa, pb, false)
 #undef MOLE_SPLIT_STAGE
 #undef MOLE_SPLIT_MFMAS
 #pragma unroll
-        for (int j = 0; j < TNW; ++j)
+        for (int i = 0; i < TMW; ++i)
 #pragma unroll
-            for (int q = 0; q < 16; ++q) acc[1][j][q] = -acc[1][j][q];
-        return;
+            for (int j = 0; j < TNW; ++j)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) acc[i][j][q] += low[i][j][q];
+        return least < (__float_as_uint(PARTS_MIN) << 1) - 1u;
     }
     FFrag<BM, M_KS, TMW> mb;
     FFrag<BN, N_KS, TNW> nb;
@@ -364,9 +387,11 @@ __device__ __forceinline__ void f32_loop(const GemmArgs &g, const float *Mp, con
         MOLE_F32_STAGE(s, ma, na, mb, nb, false)
     }
 #undef MOLE_F32_STAGE
+    return false;
 }
 
-template <int BM, int BN, int NSTAGE, int BPC, bool M_KS, bool N_KS, bool WG, int EPI>
+// PARTS: by the parts of the operands, otherwise from fp32 operands throughout.
+template <int BM, int BN, int NSTAGE, int BPC, bool PARTS, bool M_KS, bool N_KS, bool WG, int EPI>
 __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs g) {
     typedef FTile<BM, BN, NSTAGE> TL;
     constexpr int TMW = TL::TMW, TNW = TL::TNW;
@@ -473,31 +498,33 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
 #pragma unroll
         for (int b = 0; b < SB; ++b) psum[j][b] = 0.f;
 
-    f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, true>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, sum_side, psum);
-    // An infinity, a NaN or a value within half a unit of bf16 of the overflow limit has no finite parts: its products with
-    // a part that is zero are NaN.  A tile with any result that is not finite is computed again with fp32 operands.
-    float poison = 0.f;
-#pragma unroll
-    for (int i = 0; i < TMW; ++i)
-#pragma unroll
-        for (int j = 0; j < TNW; ++j)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) poison = fmaf(acc[i][j][q], 0.f, poison);
-    int *flag = reinterpret_cast<int *>(smem);
-    __syncthreads();
-    const bool bad = __ballot(poison != 0.f) != 0;      // (NaN compares unequal)
-    if (lane == 0) flag[wave] = bad;
-    __syncthreads();
-    const bool redo = (flag[0] | flag[1] | flag[2] | flag[3]) != 0;
-    if (__builtin_amdgcn_readfirstlane(redo)) {
-        __syncthreads();
+    const bool inexact = f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, PARTS>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, sum_side, psum);
+    if constexpr (PARTS) {
+        // An infinity, a NaN or a value within half a unit of bf16 of the overflow limit has no finite parts: its products with
+        // a part that is zero are NaN.  A tile with any result that is not finite is computed again with fp32 operands.
+        float poison = 0.f;
 #pragma unroll
         for (int i = 0; i < TMW; ++i)
 #pragma unroll
             for (int j = 0; j < TNW; ++j)
 #pragma unroll
-                for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
-        f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, false>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, 0, psum);
+                for (int q = 0; q < 16; ++q) poison = fmaf(acc[i][j][q], 0.f, poison);
+        int *flag = reinterpret_cast<int *>(smem);
+        __syncthreads();
+        const bool bad = __ballot(poison != 0.f || inexact) != 0;      // (NaN compares unequal)
+        if (lane == 0) flag[wave] = bad;
+        __syncthreads();
+        const bool redo = (flag[0] | flag[1] | flag[2] | flag[3]) != 0;
+        if (__builtin_amdgcn_readfirstlane(redo)) {
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < TMW; ++i)
+#pragma unroll
+                for (int j = 0; j < TNW; ++j)
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
+            f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, false>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, 0, psum);
+        }
     }
 
     if constexpr (WG) {
@@ -613,12 +640,12 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
     }
 }
 
-template <int BM, int BN, int NSTAGE, int BPC, bool M_KS, bool N_KS, bool WG, int EPI>
+template <int BM, int BN, int NSTAGE, int BPC, bool PARTS, bool M_KS, bool N_KS, bool WG, int EPI>
 int launch_f32(GemmArgs g, int tiles, hipStream_t st, int kid) {
     if (tiles <= 0) return 0;
     g.n_blocks = tiles;
     const int grid = (tiles + 7) & ~7;
-    auto kern = gemm_f32_kernel<BM, BN, NSTAGE, BPC, M_KS, N_KS, WG, EPI>;
+    auto kern = gemm_f32_kernel<BM, BN, NSTAGE, BPC, PARTS, M_KS, N_KS, WG, EPI>;
     // the LDS request also caps the blocks a CU takes: with room for more than BPC, the dispatcher fills some CUs
     // and leaves others short, and the launch lasts as long as the fullest
     constexpr int lds_min = 160 * 1024 / (BPC + 1) + 1024;
@@ -633,24 +660,24 @@ int launch_f32(GemmArgs g, int tiles, hipStream_t st, int kid) {
     return 0;
 }
 
-template <int BM, int BN, int NSTAGE, int BPC>
+template <int BM, int BN, int NSTAGE, int BPC, bool PARTS>
 int dispatch_f32(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid) {
     const int n_tiles = ceil_div(g.N, BN);
     if (wg) {
         const int tiles = g.E * ceil_div(g.M, BM) * n_tiles;
         if constexpr (BM == 128)
-            if (epi == EPI_WGRAD) return launch_f32<BM, BN, NSTAGE, BPC, true, true, true, EPI_WGRAD>(g, tiles, st, kid);
+            if (epi == EPI_WGRAD) return launch_f32<BM, BN, NSTAGE, BPC, PARTS, true, true, true, EPI_WGRAD>(g, tiles, st, kid);
         return -100;
     }
     const int rows_bound = g.offsets ? max_rows : g.single_rows;
     const int tiles = (rows_bound / BM + (g.offsets ? g.E : 1)) * n_tiles;     // every expert may end in a partial tile
     if (!b_ks) {
-        if (epi == EPI_BIAS_GELU) return launch_f32<BM, BN, NSTAGE, BPC, false, false, false, EPI_BIAS_GELU>(g, tiles, st, kid);
-        if (epi == EPI_DGELU) return launch_f32<BM, BN, NSTAGE, BPC, false, false, false, EPI_DGELU>(g, tiles, st, kid);
+        if (epi == EPI_BIAS_GELU) return launch_f32<BM, BN, NSTAGE, BPC, PARTS, false, false, false, EPI_BIAS_GELU>(g, tiles, st, kid);
+        if (epi == EPI_DGELU) return launch_f32<BM, BN, NSTAGE, BPC, PARTS, false, false, false, EPI_DGELU>(g, tiles, st, kid);
     } else {
-        if (epi == EPI_BIAS) return launch_f32<BM, BN, NSTAGE, BPC, false, true, false, EPI_BIAS>(g, tiles, st, kid);
-        if (epi == EPI_STORE) return launch_f32<BM, BN, NSTAGE, BPC, false, true, false, EPI_STORE>(g, tiles, st, kid);
-        if (epi == EPI_PART) return launch_f32<BM, BN, NSTAGE, BPC, false, true, false, EPI_PART>(g, tiles * g.ksplit, st, kid);
+        if (epi == EPI_BIAS) return launch_f32<BM, BN, NSTAGE, BPC, PARTS, false, true, false, EPI_BIAS>(g, tiles, st, kid);
+        if (epi == EPI_STORE) return launch_f32<BM, BN, NSTAGE, BPC, PARTS, false, true, false, EPI_STORE>(g, tiles, st, kid);
+        if (epi == EPI_PART) return launch_f32<BM, BN, NSTAGE, BPC, PARTS, false, true, false, EPI_PART>(g, tiles * g.ksplit, st, kid);
     }
     return -100;
 }
@@ -663,19 +690,24 @@ bool gemm_f32_sums_operand(const GemmArgs &g) {
 }
 
 // Tile height and number of planes.  A CU works off its tiles one after the other (those that share it share the pipes), so a
-// launch takes ceil(tiles / 256) walks over K.  A stage of 16 of K costs 0.45 us on a 64 x 128 tile, by itself or with others,
-// and on a 128 x 128 tile, which splits a third fewer values per MFMA, 0.81 us where it has a CU to itself and 0.70 us else; the
-// epilogue comes on top.  Same-box figures, us, of h = xd.w1^T + b1 | out = a.w2 + b2 on 64- and on 128-row tiles:
-//   8 experts of 1000 rows, 512 -> 2048: 136 | 132 and 128 | 116;  8 of 2000, 1024 -> 4096: 887 | 837 and 797 | 706;
-//   16 of 60, 1024 -> 1024: 42 | 32 and 64 | 33;  8 of 194, 512 -> 2048: 40.5 | 38 and 45 | 38.5;  3 of 3000, 256 -> 256: 24 | 20 and 30 | 20.
+// launch takes ceil(tiles / 256) walks over K.  A stage of 16 of K costs 0.47 us on a 64 x 128 tile, and on a 128 x 128 tile,
+// which takes a third fewer values apart per MFMA, 0.88 us where it has a CU to itself and 0.76 us else; the epilogue comes on top.
+// A 64-row tile with a CU to itself keeps fp32 operands, 0.52 us a stage: there one wave to a SIMD takes its operands apart with
+// nothing beside it, 0.58 us (forward passes, fp32 operands / parts: 8 experts of 97 rows, 512 -> 2048, 53.0 / 56.0 us; 32 of 100, 256 ->
+// 1024, 53.1 / 54.2; 16 of 256, 512 -> 1024, 83.4 / 87.7).  Same-box figures, us, of h = xd.w1^T + b1 | out = a.w2 + b2 by parts on 64- and on 128-row tiles: 8 experts of 1000 rows, 512
+// -> 2048: 141 | 133 and 129 | 117;  8 of 2000, 1024 -> 4096: 972 | 930 and 840 | 758;  16 of 60, 1024 -> 1024: 44 | 25 and 64 | 33;
+// 8 of 500, 768 -> 3072: 149 | 138 and 138 | 117;  4 of 4096, 512 -> 512: 73 | 66 and 66 | 56.
 // The K = F products are narrow and long and may also be split over blocks into p planes of partial results, which costs the
 // planes' way through memory at 5 TB/s and the reduction's launch.
-static double f32_cost(int bm, int p, int E, int est_rows, int N, int K, bool heavy) {
+static long f32_rounds(int bm, int p, int E, int est_rows, int N) {
     const int active = E < est_rows ? E : est_rows;
-    const long tiles = (long)p * active * ceil_div(ceil_div(est_rows, active), bm) * ceil_div(N, 128), rounds = (tiles + 255) / 256;
+    return ((long)p * active * ceil_div(ceil_div(est_rows, active), bm) * ceil_div(N, 128) + 255) / 256;
+}
+static double f32_cost(int bm, int p, int E, int est_rows, int N, int K, bool heavy) {
+    const long rounds = f32_rounds(bm, p, E, est_rows, N);
     const double stages = K / F_BK / (double)p, planes = p > 1 ? p * (2.0 * est_rows * N * sizeof(float) / 5.0e6) + 6.0 : 0.0;
-    if (bm == 64) return rounds * (0.45 * stages + (heavy ? 2.0 : 0.0)) + planes;
-    return rounds * ((rounds == 1 ? 0.81 : 0.70) * stages + (heavy ? (rounds == 1 ? 7.0 : 4.0) : 3.0)) + planes;
+    if (bm == 64) return rounds * ((rounds == 1 ? 0.52 : 0.47) * stages + (heavy ? 2.0 : 0.0)) + planes;
+    return rounds * ((rounds == 1 ? 0.88 : 0.76) * stages + (heavy ? (rounds == 1 ? 7.0 : 4.0) : 3.0)) + planes;
 }
 static int f32_tile(int p, int E, int est_rows, int N, int K, bool heavy) {
     if (E <= 0 || est_rows <= 0 || N <= 64) return 64;      // (half of the columns or more are padding: 64 rows pad less)
@@ -699,7 +731,7 @@ int launch_gemm_f32(const GemmArgs &g0, bool a_ks, bool b_ks, bool wg, int epi, 
     if (g.lda % 4 || g.ldb % 4 || g.ldc % 4 || g.N % 4 || g.N < 4) return -100;
     if (!wg && (a_ks || g.K <= 0 || g.K % F_BK)) return -100;
     if (wg && (!a_ks || !b_ks || g.M % 4 || g.M < 4)) return -100;
-    if (wg) return dispatch_f32<128, 128, 4, 2>(g, b_ks, wg, epi, max_rows, st, kid);
+    if (wg) return dispatch_f32<128, 128, 4, 2, true>(g, b_ks, wg, epi, max_rows, st, kid);
     if (b_ks && g.offsets != nullptr && ws != nullptr) {
         const int p = planes_allowed(gemm_f32_ksplit(g.E, g.est_rows, g.N, g.K), max_rows, g.est_rows, g.N);
         if (p > 1 && ws_bytes >= (size_t)p * max_rows * g.N * sizeof(float)) {
@@ -710,9 +742,10 @@ int launch_gemm_f32(const GemmArgs &g0, bool a_ks, bool b_ks, bool wg, int epi, 
     }
     const bool heavy = epi == EPI_BIAS_GELU || epi == EPI_DGELU;
     const int e = g.ksplit > 1 ? (int)EPI_PART : epi;
-    const int rc = f32_tile(g.ksplit, g.E, g.est_rows, g.N, g.K, heavy) == 128
-                       ? dispatch_f32<128, 128, 4, 2>(g, b_ks, wg, e, max_rows, st, kid)
-                       : dispatch_f32<64, 128, 4, 3>(g, b_ks, wg, e, max_rows, st, kid);
+    int rc;
+    if (f32_tile(g.ksplit, g.E, g.est_rows, g.N, g.K, heavy) == 128) rc = dispatch_f32<128, 128, 4, 2, true>(g, b_ks, wg, e, max_rows, st, kid);
+    else if (g.E > 0 && g.est_rows > 0 && f32_rounds(64, g.ksplit, g.E, g.est_rows, g.N) == 1) rc = dispatch_f32<64, 128, 4, 3, false>(g, b_ks, wg, e, max_rows, st, kid);
+    else rc = dispatch_f32<64, 128, 4, 3, true>(g, b_ks, wg, e, max_rows, st, kid);
     return rc != 0 || g.ksplit == 1 ? rc : launch_plane_reduce(g, MOLE_F32, max_rows, st);
 }
 

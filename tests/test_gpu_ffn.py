@@ -668,10 +668,9 @@ def test_ffn_split_contraction_of_more_than_2_to_18_rows():
         assert bool(((got - (ae @ w2[e] + b2[e])).abs() <= 4 * 2.0 ** -24 * 32 * terms).all())
 
 
-# fp32 products on the tiles (64 and 128 rows, whole and with remainders; split contractions), computed from bf16 parts of their
-# operands: as far from 64 bits as a sum of K fp32 terms may be, 2^-24 sqrt(K) in the 2-norm, and with no bias: over whole pairs of
-# 32-row blocks the mean error of n results is within 8 / sqrt(n) of their deviation (the matrix cores round down: with one
-# sign throughout it would be 0.07 of it).
+# fp32 products from fp32 operands on 64-row tiles (whole and with remainders; split contractions; the last case's out on the generic
+# kernel) and weight gradients, by bf16 parts of their operands: as far from 64 bits as a sum of K fp32 terms may be, 2^-24 sqrt(K) in
+# the 2-norm, and with no bias: the mean error of n results is within 8 / sqrt(n) of their deviation.
 @pytest.mark.parametrize("E,M,Fd,rows", [(2, 512, 1024, [1024, 1024]), (3, 272, 1040, [64, 192, 64]), (1, 1040, 132, [3200])])
 def test_ffn_fp32_tiles_against_64_bits(E, M, Fd, rows):
     from mole_amd import hip_ops as H
@@ -696,8 +695,106 @@ def test_ffn_fp32_tiles_against_64_bits(E, M, Fd, rows):
     assert float(err.mean().abs()) <= 8 * float(err.std()) / err.numel() ** 0.5
 
 
+# The same by parts: h and t on 128- and 64-row tiles (F = 4096, 2064), out and gx on them (M = 4096, 2064) and in planes (F = 4096: 128
+# rows, 1024: 64), experts that end in half a tile and in a lone 32-row block; operands around zero and operands of one sign, whose
+# terms all push the sum the same way.  Each of the
+# products sums eight of k before it rounds to nearest, in units of 2^-24 of the result at most: 2^-24 sqrt(K / 8) in the 2-norm.
+# What the matrix cores cut off far below the sum is 0.004 units of its last place (2^-23 at most) for every 16 of k, on a sum that
+# is half of the result on average: 2^-24 times 0.004 K / 16 in the mean, for even and odd blocks of 32 rows alike.
+PARTS_SHAPES = [(2, 272, 4096, [1024, 1000]), (2, 4096, 272, [1024, 1000]), (16, 144, 2064, [65] * 16), (16, 2064, 144, [65] * 16)]
+
+
+@pytest.mark.parametrize("one_sign", [False, True])
+@pytest.mark.parametrize("E,M,Fd,rows", PARTS_SHAPES + [(2, 2048, 1024, [288, 261])])
+def test_ffn_fp32_products_drift_in_no_direction(E, M, Fd, rows, one_sign):
+    from mole_amd import hip_ops as H
+    print(f"ffn fp32 drift E={E} M={M} F={Fd} rows={rows} one_sign={one_sign}", flush=True)
+    d = _make(E, M, Fd, rows, torch.float32, seed=M)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    if one_sign:
+        c = {k: (v.abs() if torch.is_tensor(v) else v) for k, v in c.items()}
+    off, n = torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda()
+    out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+    g = [torch.empty_like(c[k]) for k in ("w1", "b1", "w2", "b2")]
+    flat = torch.full_like(h, 50.0)            # gelu' = 1: t = go w2^T
+    gx = H.ffn_bwd(c["go"], c["xd"], flat, a, off, n, c["w1"], c["w2"], *g)
+
+    def close(got, want, K, by_blocks=True):
+        err, rms = (got.double() - want) * 2.0 ** 24, want.norm() / want.numel() ** 0.5
+        assert float(err.norm() / want.norm()) <= (K / 8) ** 0.5
+        odd = torch.arange(err.shape[0], device="cuda") // 32 % 2 == 1
+        for e in (err[~odd], err[odd]) if by_blocks and bool(odd.any()) else (err,):
+            assert float(e.mean().abs() / rms) <= 0.004 * K / 16 + 8 * float(e.std() / rms) / e.numel() ** 0.5
+
+    for e in range(E):
+        r = slice(int(d["off"][e]), int(d["off"][e]) + rows[e])
+        X, A, G, W1, W2 = (t.double() for t in (c["xd"][r], a[r], c["go"][r], c["w1"][e], c["w2"][e]))
+        close(h[r], X @ W1.t() + c["b1"][e].double(), M)
+        close(out[r], A @ W2 + c["b2"][e].double(), Fd)
+        T = G @ W2.t()
+        close(gx[r], T @ W1, Fd + M)            # (t, a sum of M terms, in a sum of F)
+        if rows[e] >= 128:
+            close(g[2][e], A.t() @ G, rows[e])
+            close(g[0][e], T.t() @ X, rows[e] + M)
+            close(g[1][e][None], T.sum(0)[None], rows[e] + M, False)
+
+
+# Numbers below 2^-110, where bf16 ends before the last part: the tile is computed from fp32 operands, whose error is that of K fp32
+# terms.  All of an operand small; a subnormal number alone in its row, against weights that lift it.
+@pytest.mark.parametrize("E,M,Fd,rows", PARTS_SHAPES)
+def test_ffn_fp32_tiles_with_tiny_operands(E, M, Fd, rows):
+    from mole_amd import hip_ops as H
+    print(f"ffn fp32 tiny operands E={E} M={M} F={Fd}", flush=True)
+    d = _make(E, M, Fd, rows, torch.float32, seed=M)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off, n = torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda()
+    b1, b2 = torch.zeros_like(c["b1"]), torch.zeros_like(c["b2"])
+    g = [torch.empty_like(c[k]) for k in ("w1", "b1", "w2", "b2")]
+    w1, w2, tiny = c["w1"] * 2.0 ** 20, c["w2"] * 2.0 ** 20, 2.0 ** -118
+    _, h, a = H.ffn_fwd(c["xd"] * tiny, off, n, w1, b1, w2, b2)
+    gx = H.ffn_bwd(c["go"] * tiny, c["xd"], torch.full_like(h, 50.0), a, off, n, w1, c["w2"], *g)
+    sub = c["xd"].clone()
+    sub[5] = 0.0
+    sub[5, 7] = 2.0 ** -140
+    lift = c["w1"].clone()
+    lift[:, :, 7] = 2.0 ** 100
+    _, hs, _ = H.ffn_fwd(sub, off, n, lift, b1, c["w2"], b2)
+    assert bool((hs[5] == 2.0 ** -40).all())
+    for e in range(E):
+        r = slice(int(d["off"][e]), int(d["off"][e]) + rows[e])
+        want = (c["xd"][r] * tiny).double() @ w1[e].double().t()
+        assert float((h[r].double() - want).norm() / want.norm()) <= 2.0 ** -24 * M ** 0.5
+        want = (c["go"][r] * tiny).double() @ c["w2"][e].double().t() @ w1[e].double()
+        assert float((gx[r].double() - want).norm() / want.norm()) <= 2.0 ** -24 * (M + Fd) ** 0.5
+
+
+# Where a row lies in its tile makes no difference to it, and a sum of zeros is a positive zero.
+@pytest.mark.parametrize("E,M,Fd,rows", PARTS_SHAPES)
+def test_ffn_fp32_rows_of_a_tile_are_treated_alike(E, M, Fd, rows):
+    from mole_amd import hip_ops as H
+    print(f"ffn fp32 equal rows E={E} M={M} F={Fd}", flush=True)
+    d = _make(E, M, Fd, rows, torch.float32, seed=Fd)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off, n = torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda()
+    for e in range(E):
+        for t in (c["xd"], c["go"]):
+            t[int(d["off"][e]):int(d["off"][e]) + rows[e]] = t[int(d["off"][e])]
+    g = [torch.empty_like(c[k]) for k in ("w1", "b1", "w2", "b2")]
+    out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+    gx = H.ffn_bwd(c["go"], c["xd"], h, a, off, n, c["w1"], c["w2"], *g)
+    for e in range(E):
+        r = slice(int(d["off"][e]), int(d["off"][e]) + rows[e])
+        for t in (h, out, gx):
+            assert bool((t[r] == t[int(d["off"][e])]).all())
+    zero = torch.zeros_like(c["go"])
+    gx = H.ffn_bwd(zero, c["xd"], torch.full_like(h, 50.0), a, off, n, c["w1"], c["w2"], *g)
+    for t in (gx, *g):
+        assert not bool(t.any()) and not bool(t.signbit().any())
+
+
 # ... and where an operand has no finite parts the tile is computed from fp32 operands: infinities and NaNs come out as fp32
-# arithmetic gives them, and a weight above the largest bf16 number gives the finite results that it should.
+# arithmetic gives them, and a weight above the largest bf16 number gives the finite results that it should (weight gradients; the other products of
+# these shapes keep fp32 operands).
 @pytest.mark.parametrize("E,M,Fd,rows", [(2, 144, 272, [130, 65]), (3, 512, 528, [300, 0, 64])])
 def test_ffn_fp32_tiles_with_infinite_and_largest_weights(E, M, Fd, rows):
     from mole_amd import hip_ops as H, _lib as L
@@ -731,6 +828,49 @@ def test_ffn_fp32_tiles_with_infinite_and_largest_weights(E, M, Fd, rows):
     assert float((h.cpu().double() - want)[:, 5].norm() / want[:, 5].norm()) <= 2.0 ** -22
     rest = torch.arange(Fd) != 5
     assert float((h.cpu().double() - want)[:, rest].norm() / want[:, rest].norm()) <= 2.0 ** -24 * M ** 0.5
+
+
+@pytest.mark.parametrize("E,M,Fd,rows", PARTS_SHAPES)
+def test_ffn_fp32_parts_with_infinite_and_largest_weights(E, M, Fd, rows):
+    """... the products by parts, h and t (F = 4096, 2064), out and gx (M = 4096, 2064), and beside them tiles that stay with parts."""
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"fp32 parts, infinite weights E={E} M={M} F={Fd}", flush=True)
+    d = _make(E, M, Fd, rows, torch.float32, seed=M)
+    R = sum(rows)
+    for name in ("xd", "go", "w1", "w2"):
+        d[name] = torch.where(d[name].abs() < 1e-3, torch.full_like(d[name], 1e-3), d[name])
+    c = {q: (v.cuda() if torch.is_tensor(v) else v) for q, v in d.items()}
+    off, n = torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda()
+    g = [torch.empty_like(c[q]) for q in ("w1", "b1", "w2", "b2")]
+    _, h0, a0 = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+    experts = [slice(int(d["off"][e]), int(d["off"][e]) + rows[e]) for e in range(E)]
+    for value in (float("inf"), -float("inf"), float("nan")):
+        w1, w2 = c["w1"].clone(), c["w2"].clone()
+        w1[:, 5, M - 1], w2[:, Fd // 2, 7] = value, value
+        _, h, _ = H.ffn_fwd(c["xd"], off, n, w1, c["b1"], c["w2"], c["b2"])
+        out, _, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], w2, c["b2"])
+        t, gx = torch.empty(R, Fd, device="cuda"), torch.empty(R, M, device="cuda")
+        H.ffn_bwd_into(c["go"], c["xd"], h0, a0, off, n, E, R, M, Fd, c["w1"], w2, t, *g, None, False, L.GELU_BWD_EXACT)
+        t_inf = t.clone()
+        H.ffn_bwd_into(c["go"], c["xd"], h0, a0, off, n, E, R, M, Fd, w1, c["w2"], t, *g, gx, False, L.GELU_BWD_EXACT)
+        for e, r in enumerate(experts):
+            D = lambda q: q.double()
+            assert _same_class(h[r], D(c["xd"][r]) @ D(w1[e]).t() + D(c["b1"][e]))
+            assert _same_class(out[r], D(a[r]) @ D(w2[e]) + D(c["b2"][e]))
+            assert _same_class(t_inf[r], (D(c["go"][r]) @ D(w2[e]).t()).cpu() * O.d_gelu_exact(D(h0[r]).cpu()))
+            assert _same_class(gx[r], D(t[r]) @ D(w1[e]))
+    # a weight above the largest bf16 number (column 5 of h to its own scale, one term carries it)
+    w1 = c["w1"].clone()
+    w1[:, 5, 3] = 3.4e38
+    x = c["xd"].clone()
+    x[:, 3] = 1e-3
+    _, h, _ = H.ffn_fwd(x, off, n, w1, c["b1"], c["w2"], c["b2"])
+    rest = torch.arange(Fd, device="cuda") != 5
+    for e, r in enumerate(experts):
+        want = x[r].double() @ w1[e].double().t() + c["b1"][e].double()
+        err = h[r].double() - want
+        assert float(err[:, 5].norm() / want[:, 5].norm()) <= 2.0 ** -22
+        assert float(err[:, rest].norm() / want[:, rest].norm()) <= 2.0 ** -24 * M ** 0.5
 
 
 # Few-row products with weights [N][K]: blocks of 32 columns (up to 1024 blocks of 64) and of 64, columns that end inside either,
