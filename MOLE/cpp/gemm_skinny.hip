@@ -169,13 +169,15 @@ __device__ __forceinline__ void sk_epilogue4(const GemmArgs &g, int e, long row,
 
 // ---- weights [N][K] ---------------------------------------------------------------------------------------------
 // A block owns 16 NA result columns of one group of up to 16 MB rows; its eight waves split the contraction.  A wave has the
-// weights of 8 / NA steps (eight loads of 1 KiB) in flight and waits for them before it asks for more: sixteen waves to a
+// weights of two steps (2 NA loads of 1 KiB) in flight and waits for them before it asks for more: sixteen waves to a
 // CU, out of step with each other, keep the memory busier than eight waves with two rounds in flight each (the
-// registers allow one or the other; 256 experts of eight rows, 2048 -> 1024: 215 against 250 us, 1.07 GB of weights).
+// registers allow one or the other; 256 experts of eight rows, 2048 -> 1024: 215 against 250 us, 1.07 GB of weights).  Two
+// steps also with 32 columns, where four would keep as many loads in flight: what a wave's share lacks of them is loaded all the
+// same (see launch_kc).
 template <typename T, int MB, int NA, int EPI>
 __device__ __forceinline__ void skinny_kc_run(const GemmArgs &g, sk_f32x4 (&red)[SK_WAVES][NA][WAVE], const int *token, int e,
                                               int rows, long row0, int m0, int n0) {
-    constexpr int EPC = SkElem<T>::EPC, KSTEP = 4 * EPC, U = 8 / NA;
+    constexpr int EPC = SkElem<T>::EPC, KSTEP = 4 * EPC, U = 2;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i16 = lane & 15, kg = lane >> 4;
     const int steps = (g.K + KSTEP - 1) / KSTEP;
@@ -584,15 +586,23 @@ static int launch_kc_na(const GemmArgs &g, int epi, int groups, hipStream_t st, 
     MOLE_LAUNCH_CHECK();
     return 0;
 }
-// 32 columns a block instead of 64 where those give a CU no more than four blocks: two share a CU, so 64 columns leave half of
-// that room empty up to 512 blocks (forward passes, 64 / 32 columns: 1 token, 64 experts of 2048 -> 8192, 256 blocks of 64 columns,
-// 49.5 / 47.7 us; 8 tokens, 8 of 1024 -> 4096, 512 blocks, 39.6 / 37.8; fp32, 1 token, 64 blocks, 31.7 / 27.9, 16 tokens, 1024
-// blocks, 103.3 / 100.7; 2048 blocks 65.7 / 65.6).  Not with groups of 32 rows, whose token loads double (24 tokens, 4 of 4096 ->
-// 4096: 71 / 80 us).
+// 32 columns a block instead of 64: 46 registers and 16 KB of LDS, four blocks to a CU where 64 columns run three, and twice
+// the blocks where those leave CUs without one.  What counts against them is that every block loads its tokens for half of the
+// columns, which shows where a wave has so few steps that its last pair repeats one; there 64 columns keep the launches that fill
+// the chip with them.  h alone, weights in no cache, experts of one to eight rows, us with 64 / 32 columns (64-column blocks):
+//   bf16, K = 2048: 12.5 / 7.5 (32), 18.4 / 18.0 (256), 30.1 / 27.2 (512), 40.6 / 32.9 (640);  K = 512: 5.4 / 4.5 (32), 11.3 / 11.0
+//   (512), 14.5 / 13.3 (640), 14.5 / 14.5 (704);  K = 768, 8 rows: 22.2 / 21.4 (640), 22.4 / 24.3 (704);  K = 128: 4.2 / 4.0 (32), 5.6 /
+//   5.9 (384), 6.6 / 7.1 (512), 9.0 / 9.8 (704).
+//   fp32, K = 1024: 11.9 / 7.4 (32), 32.3 / 28.8 (512), 56 / 50.5 (1024), 230 / 223 (4096);  K = 384, 8 rows: 22.8 / 21.3 (640), 30.6 /
+//   32.3 (1024);  K = 128: 5.3 / 4.2 (32), 9.7 / 10.2 (512), 20.7 / 23.1 (1536).
+// (With four steps of 32 columns in flight a share of fewer steps loads them all the same: K = 512, 12.1 us for 320 blocks of 64
+// columns, 19.4 for 640.)  Not with groups of 32 rows, whose token loads double (24 tokens, 4 of 4096 -> 4096: 71 / 80 us, the pass).
 template <typename T, int MB>
 static int launch_kc(const GemmArgs &g, int epi, int groups, hipStream_t st, int kid) {
     if constexpr (MB == 1) {
-        if ((long)(g.E < g.est_rows ? g.E : g.est_rows) * ceil_div(g.N, 64) <= 1024) return launch_kc_na<T, MB, 2>(g, epi, groups, st, kid);
+        const int steps = ceil_div(g.K, SK_WAVES * 4 * SkElem<T>::EPC);      // a wave's
+        const long blocks = (long)(g.E < g.est_rows ? g.E : g.est_rows) * ceil_div(g.N, 64);
+        if (steps >= 4 || blocks < (steps >= 2 ? 641 : 512)) return launch_kc_na<T, MB, 2>(g, epi, groups, st, kid);
     }
     return launch_kc_na<T, MB, 4>(g, epi, groups, st, kid);
 }

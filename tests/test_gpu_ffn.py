@@ -873,10 +873,12 @@ def test_ffn_fp32_parts_with_infinite_and_largest_weights(E, M, Fd, rows):
         assert float(err[:, rest].norm() / want[:, rest].norm()) <= 2.0 ** -24 * M ** 0.5
 
 
-# Few-row products with weights [N][K]: blocks of 32 columns (up to 1024 blocks of 64) and of 64, columns that end inside either,
-# contractions of fewer steps than a block's waves and of odd numbers of them.
+# Few-row products with weights [N][K]: blocks of 32 columns and, for short contractions in many blocks, of 64 (the last two shapes; the
+# 4096-column one in fp32 only, in bf16 it is the tiles'), columns that end inside either, contractions of fewer steps than a block's
+# waves, of odd numbers of them and of more than a wave has in flight.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("E,M,Fd,rows", [(1, 24, 40, [1]), (3, 264, 72, [2, 0, 7]), (2, 520, 1048, [8, 3]), (20, 136, 4096, [1 + e % 3 for e in range(20)])])
+@pytest.mark.parametrize("E,M,Fd,rows", [(1, 24, 40, [1]), (3, 264, 72, [2, 0, 7]), (2, 520, 1048, [8, 3]), (3, 1176, 72, [2, 0, 7]),
+                                         (20, 136, 4096, [1 + e % 3 for e in range(20)]), (44, 136, 1000, [1 + e % 3 for e in range(44)])])
 def test_ffn_few_rows_by_block_width(E, M, Fd, rows, dtype):
     from mole_amd import hip_ops as H
     print(f"few rows, block widths E={E} M={M} F={Fd} {dtype}", flush=True)

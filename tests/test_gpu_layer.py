@@ -867,12 +867,13 @@ def test_combine_in_the_reduction(S, M, E, k, Fd, cf, dtype):
 
 
 # Few tokens without a backward pass: the first product reads the tokens themselves.  Bit for bit what dispatched rows give, for one
-# pair, as many as a block has threads and one more; groups of 16 and of 32 rows, many of them in one expert (heavy); widths that
-# end inside a step; dropped pairs.
+# pair, as many as a block has threads and one more; groups of 16 and of 32 rows, many of them in one expert (heavy; of 16 rows in bf16
+# at F = 504: 520 columns are a tile more for every expert, with which the tiles take the product); widths that end inside a step; dropped
+# pairs.
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("S,M,E,k,Fd,cf,heavy", [
     (1, 256, 8, 1, 512, 0.0, False), (5, 264, 6, 5, 1032, 0.0, False), (512, 256, 64, 1, 512, 0.0, False),
-    (171, 256, 64, 3, 512, 0.0, False), (400, 136, 32, 1, 520, 0.0, True), (400, 136, 64, 1, 520, 0.0, True),
+    (171, 256, 64, 3, 512, 0.0, False), (400, 136, 32, 1, 520, 0.0, True), (400, 136, 64, 1, 520, 0.0, True), (400, 136, 64, 1, 504, 0.0, True),
     (128, 256, 64, 4, 512, 0.0, False), (400, 256, 32, 1, 512, 0.5, True),
 ])
 def test_tokens_in_place_of_dispatched_rows(S, M, E, k, Fd, cf, heavy, dtype):
@@ -882,7 +883,12 @@ def test_tokens_in_place_of_dispatched_rows(S, M, E, k, Fd, cf, heavy, dtype):
     with torch.no_grad():
         if heavy:                          # about half of the tokens choose expert 1
             m.gate[0].linear.weight[1] *= 20.0
+        L.kernel_timing_enable(True)
+        L.kernel_timing_read()
         y = m(x, capacity_factor=cf)
+        dispatches = L.kernel_timing_read()["dispatch_fwd"][0]
+        L.kernel_timing_enable(False)
+        assert dispatches == (1 if S * k > 512 or (dtype == torch.bfloat16 and E == 64 and Fd == 520) else 0)
         r = m.last_route
         if heavy and cf == 0.0:
             assert int(r.kept_rows.max()) > 100
