@@ -200,12 +200,13 @@ template <int TMB, int WM, int WN, bool M_KS, bool N_KS, int TMC, int TMCW> stru
         for (int i = 0; i < TMCW; ++i)
             acc[H * TMCW + i][P] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(n[P], m[H][i], acc[H * TMCW + i][P], 0, 0, 0);
         if constexpr (SUM != 0) {
+            static_assert(SUM != 1 || TMCW <= WN, "the wave columns share out a wave row's m-blocks");
             const bf16_t one = (bf16_t)1.0f;
             const bf16x8 ones = {one, one, one, one, one, one, one, one};
             if constexpr (SUM == 1 && P == 3) {
 #pragma unroll
                 for (int i = 0; i < TMCW; ++i)
-                    if (wn == (H * TMCW + i) >> 1) sums[i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, m[H][i], sums[i & 1], 0, 0, 0);
+                    if (wn == (H * TMCW + i) >> 1) sums[(H * TMCW + i) & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, m[H][i], sums[(H * TMCW + i) & 1], 0, 0, 0);
             } else if constexpr (SUM == 2 && H == 0) {
                 if (wm == P >> 1) sums[P & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(n[P], ones, sums[P & 1], 0, 0, 0);
             }
