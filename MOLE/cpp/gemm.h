@@ -133,7 +133,7 @@ struct CombineTail {
     const float *gates;         // [k][S]
     void *y;                    // [S][N]
     int S, k;
-    bool keep_out;              // a backward pass will read out
+    bool keep_out;              // out is read after the pass (by a backward pass or the caller)
     bool done;
 };
 

@@ -88,15 +88,16 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
     if (int rc = mole_gate_route(L->x, L->dtype, L->wg, L->logit_bias, L->S, L->E, L->M, L->k, L->capacity_factor, L->normalize_gate, 1,
                                  L->layout, L->scores, L->idx, L->loc, L->gates, L->row, L->counts, L->kept_rows, L->offsets,
                                  L->capacity, L->l_aux, L->workspace, L->workspace_bytes, stream)) return rc;
-    // Few tokens whose first product goes to the few-row kernel: it reads the tokens where they lie, if no backward pass wants xd.
+    const bool scratch = L->forward_only == 2;       // xd and out are read by nobody after this pass
+    // Few tokens whose first product goes to the few-row kernel: it reads the tokens where they lie, if nobody wants xd.
     // (what the dispatch would refuse is left to it)
     const DispatchHead head{L->row, L->S, L->k};
-    const bool head_ok = L->forward_only != 0 && L->k >= 1 && L->k <= 16 && (long)L->S * L->k <= HEAD_PAIRS && ((uintptr_t)L->x & 15) == 0 &&
+    const bool head_ok = scratch && L->k >= 1 && L->k <= 16 && (long)L->S * L->k <= HEAD_PAIRS && ((uintptr_t)L->x & 15) == 0 &&
                          ffn_fwd_takes_tokens(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
     if (!head_ok)
         if (int rc = mole_dispatch_fwd(L->x, L->dtype, L->row, L->S, L->M, L->k, L->xd, stream)) return rc;
     // (what the combine would refuse is left to it)
-    CombineTail tail{L->row, L->idx, L->gates, y, L->S, L->k, L->forward_only == 0, false};
+    CombineTail tail{L->row, L->idx, L->gates, y, L->S, L->k, !scratch, false};
     const bool tail_ok = y != nullptr && ((uintptr_t)y & 15) == 0 && L->k >= 1 && L->k <= 16;
     if (int rc = ffn_fwd(head_ok ? L->x : L->xd, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, est_rows(*L), L->M, L->F, L->w1, L->b1, L->w2, L->b2, L->h,
                                  L->a, L->out, L->workspace, L->workspace_bytes, L->forward_only, head_ok ? &head : nullptr, tail_ok ? &tail : nullptr, (hipStream_t)stream)) return rc;

@@ -160,7 +160,7 @@ Outputs run_forward(Call &c, const Tensor &x, const Tensor &wg, bool forward_onl
                              forward_only ? a + p.act_off[Plan::H] : (char *)ws.data_ptr(), p.ws_fwd);
     L.l_aux = l_aux.data_ptr<float>();
     if (forward_only) {
-        L.forward_only = 1;
+        L.forward_only = 2;
         L.h = nullptr;
     }
     check(mole_layer_fwd(&L, y.data_ptr(), current_stream(x)), "mole_layer_fwd");

@@ -267,7 +267,8 @@ int mole_ffn_bwd_ws(const void *go, const void *xd, const void *h, const void *a
  * caller's; d_l_aux: NULL or the gradient of l_aux. */
 typedef struct mole_layer {
     int32_t dtype, S, M, E, k, F, rows, layout, normalize_gate;
-    int32_t forward_only;              /* no backward pass follows: h is not stored, and may be null; xd and out are scratch */
+    int32_t forward_only;              /* 1: no backward pass follows, h is not stored and may be null; 2: nor does the caller read
+                                        * xd and out, which are scratch then and need not hold anything afterwards */
     double capacity_factor;
     const void *x;
     const float *wg, *logit_bias;

@@ -900,3 +900,46 @@ def test_tokens_in_place_of_dispatched_rows(S, M, E, k, Fd, cf, heavy, dtype):
         assert torch.equal(y, want)
     else:                                  # (fewer rows than S k: the layer may split the contraction otherwise)
         assert int((r.row < 0).sum()) > 0 and rel_err(y.float().cpu(), want.float().cpu()) < tol(dtype)
+
+
+# The C entry point without a backward pass: forward_only 1 leaves the dispatched rows and the experts' outputs in xd and out, as a pass
+# with one does; 2 may skip them.  y is the same.  One token and more whose first product would read them in place, split and
+# unsplit second products, dropped pairs.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("S,M,E,k,Fd,cf", [(1, 512, 8, 2, 2048, 0.0), (40, 264, 9, 3, 512, 0.0), (300, 512, 8, 2, 2048, 0.5)])
+def test_native_forward_only_fills_xd_and_out(S, M, E, k, Fd, cf, dtype):
+    import ctypes
+    from mole_amd import hip_ops as H
+    print(f"forward_only S={S} M={M} E={E} k={k} F={Fd} cf={cf} {dtype}", flush=True)
+    m, x, _ = _build(S, M, E, k, Fd, dtype, seed=S + M)
+    w1, b1, w2, b2 = (p.all_tensors for p in (m.FC1_W_GPU, m.FC1_B_GPU, m.FC2_W_GPU, m.FC2_B_GPU))
+    wg, rows = m.gate[0].linear.weight.detach(), S * k
+
+    class Block(ctypes.Structure):
+        _fields_ = ([(n, ctypes.c_int32) for n in "dtype S M E k F rows layout normalize_gate forward_only".split()] + [("capacity_factor", ctypes.c_double)] +
+                    [(n, ctypes.c_void_p) for n in "x wg logit_bias w1 b1 w2 b2 scores gates l_aux idx loc row counts kept_rows offsets capacity "
+                                                   "xd h a out workspace".split()] + [("workspace_bytes", ctypes.c_size_t)])
+
+    def run(forward_only):
+        i32 = lambda *n: torch.zeros(*n, dtype=torch.int32, device="cuda")
+        f32 = lambda *n: torch.zeros(*n, device="cuda")
+        act = lambda *n: torch.full(n, 7.0, dtype=dtype, device="cuda")
+        t = dict(x=x, wg=wg, w1=w1, b1=b1, w2=w2, b2=b2, scores=f32(S, E), gates=f32(k, S), l_aux=f32(1), idx=i32(k, S), loc=i32(k, S), row=i32(k, S),
+                 counts=i32(k, E), kept_rows=i32(E), offsets=i32(E + 1), capacity=i32(1), xd=act(rows, M), h=act(rows, Fd), a=act(rows, Fd), out=act(rows, M))
+        block = Block(L.dtype_code(dtype), S, M, E, k, Fd, rows, L.LAYOUT_RAGGED, 1, forward_only, cf, **{n: v.data_ptr() for n, v in t.items()})
+        block.workspace_bytes = L.lib().mole_layer_workspace_bytes(ctypes.byref(block), 0)
+        ws, y = torch.empty(max(1, block.workspace_bytes), dtype=torch.uint8, device="cuda"), act(S, M)
+        block.workspace = ws.data_ptr()
+        L.check(L.lib().mole_layer_fwd(ctypes.byref(block), L.ptr(y), L.stream()), "mole_layer_fwd")
+        torch.cuda.synchronize()
+        return y, t
+
+    y0, t0 = run(0)
+    y1, t1 = run(1)
+    y2, _ = run(2)
+    assert torch.equal(y0, y1) and torch.equal(y0, y2)
+    kept = t0["row"][t0["row"] >= 0].long()
+    assert 0 < kept.numel() <= rows and (cf == 0.0) == (kept.numel() == rows)
+    for name in ("xd", "out"):
+        assert torch.equal(t1[name][kept], t0[name][kept])
+    assert torch.equal(t1["xd"][kept], H.dispatch_fwd(x, t1["row"], rows)[kept])
