@@ -768,6 +768,29 @@ def test_ffn_fp32_tiles_with_tiny_operands(E, M, Fd, rows):
         assert float((gx[r].double() - want).norm() / want.norm()) <= 2.0 ** -24 * (M + Fd) ** 0.5
 
 
+# Down to 2^-110 the parts hold: the last part is then a bf16 number below the smallest normal one.  Every operand of one side is between
+# 2^-109 and 2^-101; the bound is that of the products by parts.
+@pytest.mark.parametrize("E,M,Fd,rows", PARTS_SHAPES)
+def test_ffn_fp32_parts_of_small_operands(E, M, Fd, rows):
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"ffn fp32 small operands E={E} M={M} F={Fd}", flush=True)
+    d = _make(E, M, Fd, rows, torch.float32, seed=Fd)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off, n = torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda()
+    small = lambda t: (t / t.abs().max() * 2.0 ** 8).abs().clamp_min(1.0).copysign(t) * 2.0 ** -109
+    xd, go, b1 = small(c["xd"]), small(c["go"]), torch.zeros_like(c["b1"])
+    w1, w2 = c["w1"] * 2.0 ** 20, c["w2"] * 2.0 ** 20
+    g = [torch.empty_like(c[k]) for k in ("w1", "b1", "w2", "b2")]
+    _, h, _ = H.ffn_fwd(xd, off, n, w1, b1, w2, c["b2"])
+    t = torch.empty_like(h)
+    H.ffn_bwd_into(go, xd, torch.full_like(h, 50.0), torch.ones_like(h), off, n, E, sum(rows), M, Fd, c["w1"], w2, t, *g, torch.empty_like(xd), False,
+                   L.GELU_BWD_EXACT)
+    for e in range(E):
+        r = slice(int(d["off"][e]), int(d["off"][e]) + rows[e])
+        for got, want, K in ((h[r], xd[r].double() @ w1[e].double().t(), M), (t[r], go[r].double() @ w2[e].double().t(), M)):
+            assert float((got.double() - want).norm() / want.norm()) <= 2.0 ** -24 * (K / 8) ** 0.5
+
+
 # Where a row lies in its tile makes no difference to it, and a sum of zeros is a positive zero.
 @pytest.mark.parametrize("E,M,Fd,rows", PARTS_SHAPES)
 def test_ffn_fp32_rows_of_a_tile_are_treated_alike(E, M, Fd, rows):
