@@ -129,7 +129,8 @@ template <int ROWS, int THREADS> __device__ __forceinline__ void zero_k_tail(cha
 // ---- MFMA fragments: 8 bf16 of k (8 (lane / 16) on) for row lane % 16 of 16-row block tb; one covers the stage's 32 of k --
 // v_mfma_f32_16x16x32_bf16 and not the 32x32x16 shape of the same rate: the chip runs matrix work against its power limit,
 // and per flop the smaller shape moves half of the accumulator bytes.  Back to back on random operands held in registers
-// (256 blocks of eight waves) it sustains 1985 TFLOP/s against 1665; on zeros both reach 2450-2490.
+// (mole_probe_mfma, 256 blocks of eight waves; the same probe with either shape, in turn on one box) it sustains 1661-1686 TFLOP/s
+// against 1520-1536, on zeros 2274-2298 against 2212-2234; the K loop of h at 16384 x 1024 -> 4096 takes 112-114 us against 121-124.
 __device__ __forceinline__ bf16x8 frag_kc(const char *lds, int tb) {
     const int lane = threadIdx.x & 63;
     const int row = lane & 15;
