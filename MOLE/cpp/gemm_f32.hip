@@ -13,8 +13,8 @@
 // roundings do not cover, in one result or in a sum over many.  2-norm errors against 64 bits with fp32 operands / here, in 2^-24:
 // 8 experts of 1000 rows, 512 -> 2048: h 6.8 / 2.2, out 7.9 / 2.8, weight gradients 9.6 and 11.8 / 3.4 and 3.8, bias gradient of
 // b1 7.8 / 4.2; all operands positive: h 5.3 / 2.0, out 3.6 / 1.5, weight gradients 7.8 / 2.9; 2048 -> 4096, 300 rows, positive: h
-// 10.3 / 3.7, mean error 0.04 / 0.03.  Only a sum of a single product is no closer: 0.42 / 0.44.  (One accumulator for all six:
-// 0.75-0.9 of fp32 operands' error, but a drift of 0.02 units a stage.)
+// 10.3 / 3.7, mean error 0.04 / 0.03.  Only a sum of a single product would be no closer, 0.424 / 0.435: weight gradients of one row
+// keep fp32 operands.  (One accumulator for all six: 0.75-0.9 of fp32 operands' error, but a drift of 0.02 units a stage.)
 // A tile whose operands include a number below 2^-110 that is not zero, or whose results are not all finite, is computed again
 // from fp32 operands.  All rows of a tile take the same steps, so equal rows give equal results.
 // Time, fp32 operands / parts on one box, us: 8 experts of 1000 rows, 512 -> 2048: h 154 / 128, out 135 / 115, t 154 / 125, gx 133 /
@@ -225,6 +225,21 @@ __device__ __forceinline__ bool f32_loop(const GemmArgs &g, const float *Mp, con
     else __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     __builtin_amdgcn_s_barrier();
     if (WG && nk == 1 && kl < F_BK) zero_tail(0);
+    auto add_sums = [&]() __attribute__((always_inline)) {
+        if constexpr (WG) {
+            if (sum_side == 1) {
+#pragma unroll
+                for (int b = 0; b < TMW; ++b)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) psum[i & 3][b] += ma.get(b, i >> 2, i & 3);
+            } else if (sum_side == 2) {
+#pragma unroll
+                for (int b = 0; b < TNW; ++b)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) psum[i & 3][b] += na.get(b, i >> 2, i & 3);
+            }
+        }
+    };
     if constexpr (SPLIT) {
         Planes pa[TMW + TNW], pb[TMW + TNW];
         f32x16 low[TMW][TNW];           // the products below hi hi
@@ -242,21 +257,6 @@ __device__ __forceinline__ bool f32_loop(const GemmArgs &g, const float *Mp, con
             p[b].split(x, least);
             // (kept where it stands, among the MFMAs: left alone the compiler moves it to the use, a stage later)
             asm volatile("" : "+v"(p[b].p[0]), "+v"(p[b].p[1]), "+v"(p[b].p[2]));
-        };
-        auto add_sums = [&]() __attribute__((always_inline)) {
-            if constexpr (WG) {
-                if (sum_side == 1) {
-#pragma unroll
-                    for (int b = 0; b < TMW; ++b)
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) psum[i & 3][b] += ma.get(b, i >> 2, i & 3);
-                } else if (sum_side == 2) {
-#pragma unroll
-                    for (int b = 0; b < TNW; ++b)
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) psum[i & 3][b] += na.get(b, i >> 2, i & 3);
-                }
-            }
         };
         ma.read(smem, fm0, fm1);
         na.read(smem + TL::M_BYTES, fn0, fn1);
@@ -335,6 +335,7 @@ __device__ __forceinline__ bool f32_loop(const GemmArgs &g, const float *Mp, con
     FFrag<BN, N_KS, TNW> nb;
     ma.read(smem, fm0, fm1);
     na.read(smem + TL::M_BYTES, fn0, fn1);
+    add_sums();         // (of the first stage: only contractions of one row ask for sums here)
 
     // One stage: the MFMAs of stage S on the fragments MC / NC.  With NEXT, first the hand-over to stage S + 1: wait
     // until this wave's share of it has landed, barrier; then, dealt out between the MFMAs so that the matrix pipe
@@ -498,23 +499,31 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
 #pragma unroll
         for (int b = 0; b < SB; ++b) psum[j][b] = 0.f;
 
-    const bool inexact = f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, PARTS>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, sum_side, psum);
+    // A weight gradient of one row is products without a sum: exact but for their rounding from fp32 operands, where the products that the
+    // parts leave out add to it (2-norm error in 2^-24: 0.424, by parts 0.435; two rows 0.518 and 0.440).  Its only stage also gives the sums.
+    const bool one_row = PARTS && WG && k_ext <= 1;
+    bool redo = one_row;
+    if (!one_row) {
+        const bool inexact = f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, PARTS>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, sum_side, psum);
+        if constexpr (PARTS) {
+            // An infinity, a NaN or a value within half a unit of bf16 of the overflow limit has no finite parts: its products with
+            // a part that is zero are NaN.  A tile with any result that is not finite is computed again with fp32 operands.
+            float poison = 0.f;
+#pragma unroll
+            for (int i = 0; i < TMW; ++i)
+#pragma unroll
+                for (int j = 0; j < TNW; ++j)
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) poison = fmaf(acc[i][j][q], 0.f, poison);
+            int *flag = reinterpret_cast<int *>(smem);
+            __syncthreads();
+            const bool bad = __ballot(poison != 0.f || inexact) != 0;      // (NaN compares unequal)
+            if (lane == 0) flag[wave] = bad;
+            __syncthreads();
+            redo = (flag[0] | flag[1] | flag[2] | flag[3]) != 0;
+        }
+    }
     if constexpr (PARTS) {
-        // An infinity, a NaN or a value within half a unit of bf16 of the overflow limit has no finite parts: its products with
-        // a part that is zero are NaN.  A tile with any result that is not finite is computed again with fp32 operands.
-        float poison = 0.f;
-#pragma unroll
-        for (int i = 0; i < TMW; ++i)
-#pragma unroll
-            for (int j = 0; j < TNW; ++j)
-#pragma unroll
-                for (int q = 0; q < 16; ++q) poison = fmaf(acc[i][j][q], 0.f, poison);
-        int *flag = reinterpret_cast<int *>(smem);
-        __syncthreads();
-        const bool bad = __ballot(poison != 0.f || inexact) != 0;      // (NaN compares unequal)
-        if (lane == 0) flag[wave] = bad;
-        __syncthreads();
-        const bool redo = (flag[0] | flag[1] | flag[2] | flag[3]) != 0;
         if (__builtin_amdgcn_readfirstlane(redo)) {
             __syncthreads();
 #pragma unroll
@@ -523,7 +532,7 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
                 for (int j = 0; j < TNW; ++j)
 #pragma unroll
                     for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
-            f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, false>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, 0, psum);
+            f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, false>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, one_row ? sum_side : 0, psum);
         }
     }
 

@@ -791,6 +791,28 @@ def test_ffn_fp32_parts_of_small_operands(E, M, Fd, rows):
             assert float((got.double() - want).norm() / want.norm()) <= 2.0 ** -24 * (K / 8) ** 0.5
 
 
+# Weight gradients of experts with one row are products rounded once, those of two rows sums of two; the bias gradients are the row itself.
+@pytest.mark.parametrize("E,M,Fd,rows", [(5, 132, 272, [1, 2, 1, 0, 1]), (1, 512, 140, [1])])
+def test_ffn_fp32_weight_gradients_of_one_row(E, M, Fd, rows):
+    from mole_amd import hip_ops as H
+    print(f"ffn fp32 one row E={E} M={M} F={Fd}", flush=True)
+    d = _make(E, M, Fd, rows, torch.float32, seed=M)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off, n = torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda()
+    a, h = torch.randn(sum(rows), Fd, device="cuda"), torch.zeros(sum(rows), Fd, device="cuda")
+    g = [torch.empty_like(c[k]) for k in ("w1", "b1", "w2", "b2")]
+    H.ffn_bwd(c["go"], c["xd"], h, a, off, n, c["w1"], c["w2"], *g)
+    for e in range(E):
+        r = slice(int(d["off"][e]), int(d["off"][e]) + rows[e])
+        if rows[e] == 1:
+            assert torch.equal(g[2][e], a[r].t() * c["go"][r]) and torch.equal(g[3][e], c["go"][r][0])
+        elif rows[e] == 2:
+            want = a[r].double().t() @ c["go"][r].double()
+            assert float((g[2][e].double() - want).norm() / want.norm()) <= 2.0 ** -24
+        else:
+            assert not bool(g[2][e].any()) and not bool(g[3][e].any())
+
+
 # Where a row lies in its tile makes no difference to it, and a sum of zeros is a positive zero.
 @pytest.mark.parametrize("E,M,Fd,rows", PARTS_SHAPES)
 def test_ffn_fp32_rows_of_a_tile_are_treated_alike(E, M, Fd, rows):
