@@ -17,6 +17,7 @@
 // as whole 128-byte rows.  A ragged m-tile runs only the 32-row blocks it has rows for.
 #include "gemm.h"
 #include "lds_dma.h"
+#include "wgrad_few.h"
 
 #include <stdlib.h>
 
@@ -28,6 +29,9 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int Q_BK = 32;
+// Rows of an expert up to which a weight-gradient tile goes by way of few_rows_tile: two steps of 32, whose fragments fit the registers
+// beside the results' old values.  (Up to 32 / up to 64: 8 experts of 2048 x 4096, 48 rows, 35.4 / 30.1 us; 64 of 1024 x 2048 81 / 75.)
+constexpr int FEW_ROWS = 64;
 
 // Geometry of a BM x BN tile of TMB 32-row m-blocks computed by WM x WN waves: WM wave rows of TMB/WM m-blocks
 // each, WN wave columns of 64 columns each.  Eight waves put two on every SIMD: while one waits for
@@ -906,6 +910,26 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
         }
     }
     const bf16_t *Mp = (const bf16_t *)g.A + row0 * g.lda;
+    if constexpr (WG && EPI == EPI_WGRAD) {
+        // Up to FEW_ROWS rows: every wave by itself, 128 columns by 64 rows of the tile (128-wide tiles: by 32); see wgrad_few.h.
+        if (k_ext <= FEW_ROWS) {
+            constexpr int COLS = Q_BN / 128, VM = Q_BM / 16 / (TL::NW / COLS);     // the block's waves along n; columns of a lane on the m-side
+            const int w = __builtin_amdgcn_readfirstlane(wave), m_few = m0 + w / COLS * (16 * VM), n_few = n0 + w % COLS * 128;
+            const bf16_t *Bp = (const bf16_t *)g.B + row0 * g.ldb;
+            bf16_t *Cb = (bf16_t *)g.C + (long)e * g.strideC, *sums = nullptr;
+            int side = 0;
+            if (g.colsum != nullptr && g.colsum_side == 1 && nt == sum_nt && w % COLS == 0) { side = 1; sums = (bf16_t *)g.colsum + (long)e * g.M; }
+            if (g.colsum != nullptr && g.colsum_side == 2 && mt == sum_mt && w / COLS == 0) { side = 2; sums = (bf16_t *)g.colsum + (long)e * g.N; }
+            if (k_ext <= 32) {
+                if (g.accumulate) few_rows_tile<VM, 8, 1, true>(g, Mp, Bp, Cb, sums, side, m_few, n_few, k_ext);
+                else few_rows_tile<VM, 8, 1, false>(g, Mp, Bp, Cb, sums, side, m_few, n_few, k_ext);
+            } else {
+                if (g.accumulate) few_rows_tile<VM, 8, 2, true>(g, Mp, Bp, Cb, sums, side, m_few, n_few, k_ext);
+                else few_rows_tile<VM, 8, 2, false>(g, Mp, Bp, Cb, sums, side, m_few, n_few, k_ext);
+            }
+            return;
+        }
+    }
     const bf16_t *Np = WG ? (const bf16_t *)g.B + row0 * g.ldb : (const bf16_t *)g.B + (long)e * g.strideB;
     if constexpr (EPI == EPI_PART) {           // this block's whole stages of the contraction (the last plane has the ragged end)
         split_k = __builtin_amdgcn_readfirstlane(split_k);
@@ -1119,8 +1143,15 @@ static TilePlan tile_plan(int E, int est_rows, int N, int K, bool tall) {
 // 256 large tiles costs what 768 small ones do.  128 x 128 against 256 x 256: 16 experts of 520 x 1416, 128 rows, 17 / 22 us;
 // 512 x 512, 1000 rows, 20 / 30; 4 of 512 x 2048, 500 rows, 13 / 19; 63 of 384 x 1536, 344 rows, 55 / 58; on the other
 // side of the line 8 experts of 1024 x 3072, 500 rows, 44 / 41; 123 of 256 x 512, 325 rows, 29 / 27.
-static int wgrad_tile(int E, int M, int N) {
+// Launches of experts with up to 24 rows are a stream of results (see wgrad_few.h), which two 128 x 128 blocks to a CU keep up where
+// one of twice the waves leaves it between blocks: 128 x 128 / 256 x 256, 1 to 24 rows an expert, 200 of 384 x 768, 22 / 24 us; 64 of 1024 x
+// 2048, 58 / 60 and 91 / 98 where the results are added to; 12 of 1344 x 2688, 16 / 19; 16 of 1024 x 4096, 27 / 28.  With more rows skewed
+// loads leave enough to the experts above FEW_ROWS for the large tiles (64 of 1024 x 2048, 32 rows, Zipf(1.2): 71 / 67), and more than
+// 2^15 blocks are slower to hand out (64 of 2048 x 8192: 405 / 385).
+static int wgrad_tile(int E, int est_rows, int M, int N) {
     const long t256 = (long)E * ceil_div(M, 256) * ceil_div(N, 256), t128 = (long)E * ceil_div(M, 128) * ceil_div(N, 128);
+    const int active = E < est_rows ? E : est_rows;
+    if (active > 0 && est_rows <= 24l * active && t128 <= 32768) return TILE_128;
     return t128 < 768 * ((t256 + 255) / 256) ? TILE_128 : TILE_256;
 }
 int gemm256_ksplit(int E, int est_rows, int N, int K) { return tile_plan(E, est_rows, N, K, true).ksplit; }
@@ -1139,7 +1170,7 @@ int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, in
     TilePlan p{TILE_256, 1};
     if (!wg && g.offsets != nullptr && epi < EPI_NONE) p = tile_plan(g.E, g.est_rows, g.N, g.K, b_ks);
     p.ksplit = planes_allowed(p.ksplit, max_rows, g.est_rows, g.N);
-    if (wg && epi == EPI_WGRAD) p.tile = wgrad_tile(g.E, g.M, g.N);
+    if (wg && epi == EPI_WGRAD) p.tile = wgrad_tile(g.E, g.est_rows, g.M, g.N);
     GemmArgs gp = g;
     gp.ksplit = 1;
     if (p.ksplit > 1 && b_ks && ws != nullptr && ws_bytes >= (size_t)p.ksplit * max_rows * g.N * sizeof(float)) {

@@ -522,6 +522,41 @@ def test_ffn_weight_gradients_by_small_tiles(E, M, Fd, rows, gap, accumulate):
 # K-strided weights read past the caches, in a forward pass that no backward follows: from 64 MB of weights of the experts that
 # can have rows, the recorded pass (256 MB) taking the ordinary loads.  Experts of a few rows on the kernel for them, of up
 # to 64 and up to 128 on the tiles, of more (ordinary loads there), and of none.  The loads' cache policy changes no result.
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("E,M,Fd,rows,gap", [
+    (6, 136, 264, [1, 31, 32, 33, 0, 8], 0),                # one and two steps of rows, 128-wide tiles that end in the middle
+    (4, 264, 136, [64, 63, 65, 2], 3),                      # both sides of the limit in one launch
+    (3, 8, 16, [5, 0, 64], 0),                              # less than a lane's columns on one side
+    (40, 520, 1032, [40] * 38 + [64, 0], 0),                # 256-wide tiles
+    (40, 512, 1024, [33 + e % 32 for e in range(39)] + [700], 0),
+])
+def test_ffn_weight_gradients_of_few_rows(E, M, Fd, rows, gap, accumulate):
+    """Experts of up to 64 rows, whose weight gradients are formed without the operand ring: sums of bf16 products in fp32 (64
+    terms: 64 x 2^-24 of the terms' size) and one rounding to bf16, 2^-9 of the result, two where it is added to what is there."""
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"few-row weight gradients E={E} M={M} F={Fd} rows={rows} accumulate={accumulate}", flush=True)
+    d = _make(E, M, Fd, rows, torch.bfloat16, seed=E + M, pad_between=gap)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off = torch.from_numpy(d["off"]).cuda(); n = torch.from_numpy(d["n"]).cuda()
+    R = max(d["R"], 1)
+    h = torch.randn(R, Fd, generator=torch.Generator().manual_seed(3)).bfloat16().cuda()
+    a = torch.nn.functional.gelu(h.float()).bfloat16()
+    t = torch.zeros(R, Fd, dtype=torch.bfloat16, device="cuda")
+    old = 0.5
+    g = [torch.full_like(c[k], old) for k in ("w1", "b1", "w2", "b2")]
+    H.ffn_bwd_into(c["go"], c["xd"], h, a, off, n, E, R, M, Fd, c["w1"], c["w2"], t, *g, None, accumulate, L.GELU_BWD_EXACT)
+    go, xd, a64, t64 = (v.double().cpu() for v in (c["go"], c["xd"], a, t))
+    for e in range(E):
+        lo, hi = int(d["off"][e]), int(d["off"][e]) + int(d["n"][e])
+        want = (t64[lo:hi].t() @ xd[lo:hi], t64[lo:hi].sum(0), a64[lo:hi].t() @ go[lo:hi], go[lo:hi].sum(0))
+        size = (t64[lo:hi].abs().t() @ xd[lo:hi].abs(), t64[lo:hi].abs().sum(0), a64[lo:hi].abs().t() @ go[lo:hi].abs(), go[lo:hi].abs().sum(0))
+        for got, w, s in zip(g, want, size):
+            w = w + old if accumulate else w
+            # (an expert above the limit: its larger tiles keep the same sums)
+            bound = 2.0 ** -8 * w.abs() + max(hi - lo, 64) * 2.0 ** -24 * (s + old)
+            assert bool(((got[e].double().cpu() - w).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("E,M,Fd,k,S", [
     (40, 1024, 1024, 1, 61), (40, 1024, 1024, 2, 120), (23, 512, 3264, 2, 33),      # few rows; the last of 67 / 134 MB
