@@ -5,14 +5,19 @@
 // MOLETopk.forward (MOLE/utils/Ugate.py:13).
 //
 // Up to four launches, all on the caller's stream:
-//   route_tokens    64 tokens per block of 16 waves.  A group of 16 lanes (64 beyond 256 experts) owns one token and holds
+//   route_tokens    64 tokens per block of 16 waves, or 16 or 4 of four waves.  A group of 16 lanes (64 beyond 256 experts, and beyond
+//                   64 where the tokens are few) owns one token and holds
 //                   its scores in registers - softmaxed on the spot when it is given logits; k rounds of a lane-pattern
-//                   arg-max with the (score desc, index asc) order.  Then wave j ranks choice j: a token's rank is the
-//                   number of the block's earlier tokens with the same expert, from one ballot per bit of the index.
+//                   arg-max with the (score desc, index asc) order.
+//   then, up to 8192 pairs,
+//   route_rank      one block: locations, counts, capacity, kept rows, row offsets, l_aux from the chosen experts alone;
+//   otherwise route_tokens goes on: wave j ranks choice j, a token's rank being the
+//                   number of the block's earlier tokens with the same expert, from one ballot per bit of the index; and
 //   route_scan      one wave per (choice, expert): exclusive prefix over the blocks' histograms.
 //   route_finish    one block: per-expert totals, capacity, kept rows, row offsets, l_aux; for small problems also the scan
-//                   and the last stage.  A single block of tokens does all of it itself.
+//                   and the last stage.
 //   route_finalize  loc = base(choice, expert) + block prefix + in-block rank; row = offset + loc.
+// A single block of tokens does all of it itself.
 #include "common.h"
 
 #include <algorithm>
@@ -55,6 +60,21 @@ __device__ __forceinline__ float topk_unkey(uint32_t key) {
 // one crossbar swizzle, the whole wave reads the four row results into scalars.
 template <int CTRL> __device__ __forceinline__ int dpp_lane(int x) {
     return __builtin_amdgcn_update_dpp(x, x, CTRL, 0xf, 0xf, false);
+}
+// the value of lane l ^ M, M = 1, 2, 4 or 8 (xor 4: the mirrored half row, then the reversed quads)
+template <int M> __device__ __forceinline__ float lane_xor(float x) {
+    const int v = __builtin_bit_cast(int, x);
+    if constexpr (M == 1) return __builtin_bit_cast(float, dpp_lane<0xb1>(v));
+    else if constexpr (M == 2) return __builtin_bit_cast(float, dpp_lane<0x4e>(v));
+    else if constexpr (M == 4) return __builtin_bit_cast(float, dpp_lane<0x1b>(dpp_lane<0x141>(v)));
+    else return __builtin_bit_cast(float, dpp_lane<0x128>(v));       // row_ror 8
+}
+// sum over aligned groups of 16 lanes in the order of a butterfly from 8 down, as __shfl_xor would add it
+__device__ __forceinline__ float butterfly16(float x) {
+    x += lane_xor<8>(x);
+    x += lane_xor<4>(x);
+    x += lane_xor<2>(x);
+    return x + lane_xor<1>(x);
 }
 template <typename T, typename Op> __device__ __forceinline__ T group_reduce(T x, int logG, Op op) {
     static_assert(sizeof(T) == 4, "32-bit lanes");
@@ -116,6 +136,7 @@ __device__ __forceinline__ void topk_block_tail(int BT, int S, int E, int k, int
         }
     }
 
+    if (hist == nullptr) return;           // (route_rank takes them from the indices)
     // ---- in-block ranks per choice (lane = token; wave w takes choices w, w + 4, ...) ------
     // Each wave works on a histogram of its own, so the choices proceed side by side without block barriers.
     int *my_hist = s_hist + w * E;
@@ -196,44 +217,58 @@ struct RouteEnd {
     int32_t *idx, *loc, *row;          // loc: in-block ranks in, locations out
 };
 
-// block-wide reductions of FIN_THREADS threads: lane patterns inside a wave, 16 values in LDS between the waves
-__device__ __forceinline__ int block_max(int v, int *s16) {
-    v = group_reduce(v, 6, [](int a, int c) { return max(a, c); });
-    if ((threadIdx.x & 63) == 0) s16[threadIdx.x >> 6] = v;
+// Loads of the experts (s_off [E]) -> capacity, kept rows, offsets (s_off again), l_aux (s_me [E]: column sum of the scores x count of the
+// first choice).  Called by all threads of a block.  What runs over the experts - the largest load, the offsets, the loss's
+// sum - is one wave's work, 64 experts at a time: by all waves of the block each of the three is a reduction between two or three
+// barriers.
+__device__ __forceinline__ void finish_offsets(const RouteEnd &r, const float *s_me, int *s_off, int *s_cap) {
+    const int tid = threadIdx.x, E = r.E;
+    if (tid < WAVE) {
+        int cap = r.cap_bound;
+        if (r.cf_sign <= 0) {              // uniform: the largest load, which only capacity factors <= 0 ask for
+            int most = 0;
+            for (int e = tid; e < E; e += WAVE) most = max(most, s_off[e]);
+            cap = group_reduce(most, 6, [](int a, int c) { return max(a, c); });
+            if (r.cf_sign < 0) cap = min(cap, r.cap_bound);
+        }
+        const int rem = cap % r.alignment;
+        if (rem > 0) cap += r.alignment - rem;
+        int before = 0;
+        float loss = 0.f;
+        for (int e0 = 0; e0 < E; e0 += WAVE) {
+            const int e = e0 + tid, n = e < E ? min(s_off[e], cap) : 0;
+            int off = e * cap;
+            if (r.layout == MOLE_LAYOUT_RAGGED) {
+                const int incl = wave_scan(n);
+                off = before + incl - n;
+                before += wave_total(incl);
+            }
+            if (r.l_aux != nullptr) loss += e < E ? s_me[e] : 0.f;
+            if (e < E) {
+                r.kept_rows[e] = n;
+                r.offsets[e] = off;
+                s_off[e] = off;
+            }
+        }
+        if (r.l_aux != nullptr) loss = wave_sum(loss);
+        if (tid == 0) {
+            r.offsets[E] = r.layout == MOLE_LAYOUT_RAGGED ? before : E * cap;
+            r.capacity[0] = cap;
+            *s_cap = cap;
+            if (r.l_aux != nullptr) r.l_aux[0] = r.S > 0 ? loss * ((float)E / ((float)r.S * (float)r.S)) : 0.f;
+        }
+    }
     __syncthreads();
-    int m = s16[0];
-#pragma unroll
-    for (int w = 1; w < FIN_THREADS / WAVE; ++w) m = max(m, s16[w]);
-    __syncthreads();
-    return m;
-}
-__device__ __forceinline__ float block_sum(float v, float *s16) {
-    v = wave_sum(v);
-    if ((threadIdx.x & 63) == 0) s16[threadIdx.x >> 6] = v;
-    __syncthreads();
-    float m = s16[0];
-#pragma unroll
-    for (int w = 1; w < FIN_THREADS / WAVE; ++w) m += s16[w];
-    __syncthreads();
-    return m;
-}
-__device__ __forceinline__ int block_inclusive(int v, int *s16) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    v = wave_scan(v);
-    if (lane == WAVE - 1) s16[w] = v;
-    __syncthreads();
-    for (int q = 0; q < w; ++q) v += s16[q];
-    __syncthreads();
-    return v;
 }
 
-// Counts -> capacity, kept rows, offsets, l_aux.  Thread e owns expert e (E <= FIN_THREADS).  cnt: [k][E] totals (global or
-// LDS), replaced by base(choice, expert), the rows of the expert's earlier choices; me: the column sum of the scores of
-// the thread's expert.  Returns the capacity; s_off[e] = first row of expert e.
-__device__ __forceinline__ int finish_counts(const RouteEnd &r, int *cnt, float me, int *s_off, int *s16) {
-    const int e = threadIdx.x, E = r.E;
-    int tot = 0, first = 0;
-    if (e < E) {
+// Counts -> capacity, kept rows, offsets, l_aux.  cnt: [k][E] totals (global or LDS), replaced by base(choice, expert), the rows of
+// the expert's earlier choices; s_me [E]: the column sums of the scores (with l_aux).  Returns the capacity; s_off[e] = first row of
+// expert e.
+template <int THREADS>
+__device__ __forceinline__ int finish_counts(const RouteEnd &r, int *cnt, float *s_me, int *s_off, int *s_cap) {
+    const int tid = threadIdx.x, E = r.E;
+    for (int e = tid; e < E; e += THREADS) {
+        int tot = 0, first = 0;
         for (int j = 0; j < r.k; ++j) {
             const int c = cnt[j * E + e];
             if (j == 0) first = c;
@@ -241,31 +276,40 @@ __device__ __forceinline__ int finish_counts(const RouteEnd &r, int *cnt, float 
             cnt[j * E + e] = tot;
             tot += c;
         }
-    }
-    int cap = r.cap_bound;
-    if (r.cf_sign <= 0) {              // uniform: the largest load, which only capacity factors <= 0 ask for
-        cap = block_max(tot, s16);
-        if (r.cf_sign < 0) cap = min(cap, r.cap_bound);
-    }
-    const int rem = cap % r.alignment;
-    if (rem > 0) cap += r.alignment - rem;
-    const int n = min(tot, cap);
-    if (e < E) r.kept_rows[e] = n;
-    if (r.layout == MOLE_LAYOUT_RAGGED) {
-        const int incl = block_inclusive(n, s16);
-        if (e < E) { r.offsets[e] = incl - n; s_off[e] = incl - n; }
-        if (e == E - 1) r.offsets[E] = incl;
-    } else {
-        if (e < E) { r.offsets[e] = e * cap; s_off[e] = e * cap; }
-        if (e == 0) r.offsets[E] = E * cap;
-    }
-    if (e == 0) r.capacity[0] = cap;
-    if (r.l_aux != nullptr) {          // uniform over the grid
-        const float sum = block_sum(e < E ? me * (float)first : 0.f, (float *)s16);
-        if (e == 0) r.l_aux[0] = r.S > 0 ? sum * ((float)E / ((float)r.S * (float)r.S)) : 0.f;
+        s_off[e] = tot;
+        if (r.l_aux != nullptr) s_me[e] *= (float)first;
     }
     __syncthreads();
-    return cap;
+    finish_offsets(r, s_me, s_off, s_cap);
+    return *s_cap;
+}
+// The column sums of the scores (with l_aux): thread (g, e) adds blocks g, g + groups, ... in order; later the groups in order.
+__device__ __forceinline__ float column_part(const RouteEnd &r, const float *__restrict__ colsum, int nb_col) {
+    float me = 0.f;
+    const int E = r.E, groups = FIN_THREADS / E;
+    if ((int)threadIdx.x < groups * E) {
+        const int e = threadIdx.x % E, gq = threadIdx.x / E;
+        for (int b0 = gq; b0 < nb_col; b0 += 8 * groups) {
+            float t[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int b = b0 + u * groups;
+                t[u] = load_or_zero(colsum + (size_t)min(b, nb_col - 1) * E + e, b < nb_col);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (b0 + u * groups < nb_col) me += t[u];
+        }
+    }
+    return me;
+}
+// s_part: the threads' parts; s_part[e], e < E, becomes the sum
+__device__ __forceinline__ void fold_columns(const RouteEnd &r, float *s_part) {
+    const int E = r.E, tid = threadIdx.x;
+    if (r.l_aux == nullptr || tid >= E) return;
+    float me = s_part[tid];
+    for (int gq = 1; gq < FIN_THREADS / E; ++gq) me += s_part[gq * E + tid];
+    s_part[tid] = me;
 }
 
 // One block.  scan_hist == NULL: counts holds the totals already (route_scan ran).  Otherwise the block scans the
@@ -278,29 +322,10 @@ __global__ __launch_bounds__(FIN_THREADS) void route_finish_kernel(const RouteEn
                                                                    int32_t *__restrict__ basej, int32_t *scan_hist, int nb, int bt,
                                                                    int last) {
     __shared__ int s_off[FIN_THREADS];
-    __shared__ int s16[FIN_THREADS / WAVE];
-    __shared__ float s_fred[FIN_THREADS];
+    __shared__ int s_cap;
+    __shared__ float s_part[FIN_THREADS];
     const int tid = threadIdx.x, E = r.E, npairs = r.k * E;
-    // column sums of the scores: thread (g, e) adds blocks g, g + groups, ... in order, thread e then the groups in order
-    float me = 0.f;
-    if (r.l_aux != nullptr) {
-        const int groups = FIN_THREADS / E;
-        if (tid < groups * E) {
-            const int e = tid % E, gq = tid / E;
-            for (int b0 = gq; b0 < nb_col; b0 += 8 * groups) {
-                float t[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const int b = b0 + u * groups;
-                    t[u] = load_or_zero(colsum + (size_t)min(b, nb_col - 1) * E + e, b < nb_col);
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    if (b0 + u * groups < nb_col) me += t[u];
-            }
-        }
-        s_fred[tid] = me;
-    }
+    if (r.l_aux != nullptr) s_part[tid] = column_part(r, colsum, nb_col);
     if (scan_hist != nullptr) {
         if (nb <= FIN_FEW) {
             for (int pair = tid; pair < npairs; pair += FIN_THREADS) {
@@ -324,12 +349,8 @@ __global__ __launch_bounds__(FIN_THREADS) void route_finish_kernel(const RouteEn
     }
     __threadfence_block();
     __syncthreads();
-    if (r.l_aux != nullptr && tid < E) {
-        const int groups = FIN_THREADS / E;
-        me = s_fred[tid];
-        for (int gq = 1; gq < groups; ++gq) me += s_fred[gq * E + tid];
-    }
-    const int cap = finish_counts(r, basej, me, s_off, s16);
+    fold_columns(r, s_part);
+    const int cap = finish_counts<FIN_THREADS>(r, basej, s_part, s_off, &s_cap);
     if (!last) return;
     __threadfence_block();
     for (int p = tid; p < r.k * r.S; p += FIN_THREADS) {
@@ -338,6 +359,85 @@ __global__ __launch_bounds__(FIN_THREADS) void route_finish_kernel(const RouteEn
         const int l = basej[j * E + e] + scan_hist[((size_t)j * E + e) * nb + i / bt] + r.loc[p];
         r.loc[p] = l;
         r.row[p] = l < cap ? s_off[e] + l : -1;
+    }
+}
+
+// The end of the routing from the chosen experts alone, in one block: no histograms through memory, no launch behind it.  The pairs
+// lie in choice-major order, in chunks of 64 tokens of one choice; wave w ranks chunks w, w + 16, ... (P of them) and leaves their
+// counts in LDS, an exclusive prefix over the chunks of every expert is then a pair's location but for its rank.  Bound by latency:
+// one round trip for the indices, the rest is LDS.  Histograms through memory and what goes with them / here: 256 experts, top-8, 256 tokens
+// 17.8 / 13.4 us; 8 experts, top-2, 777 tokens 7.6 / 5.8, 4096 tokens 12.9 / 10.4 (two launches / one); 16 experts, top-2, 2048 tokens 9.5 /
+// 7.4, 3001 tokens 13.7 / 11.8.  A thread's eight pairs are as long as the launch they save: the line lies there.
+constexpr int RANK_PAIRS = 8192, RANK_COUNTS = 16384;       // most pairs (P = 8) and counts (64 KB of LDS)
+static bool rank_in_one_block(int S, int E, int k) {
+    const long chunks = (long)k * ceil_div(S, WAVE);
+    return chunks <= RANK_PAIRS / WAVE && chunks * (E | 1) <= RANK_COUNTS;
+}
+template <int P>
+__global__ __launch_bounds__(FIN_THREADS) void route_rank_kernel(const RouteEnd r, const float *__restrict__ colsum, int nb_col) {
+    constexpr int WAVES = FIN_THREADS / WAVE;
+    extern __shared__ __align__(16) int s_cnt[];            // [chunks][stride]
+    __shared__ int s_off[FIN_THREADS];
+    __shared__ float s_part[FIN_THREADS];
+    __shared__ int s_cap;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, E = r.E, S = r.S, k = r.k;
+    const int per = (S + WAVE - 1) / WAVE, chunks = k * per, stride = E | 1;       // (odd: the scan walks down a column)
+    int e[P], at[P];
+    bool ok[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int c = p * WAVES + w, j = c / per, i = (c - j * per) * WAVE + lane;
+        ok[p] = c < chunks && i < S;
+        at[p] = min(j, k - 1) * S + min(i, S - 1);
+        e[p] = load_or_zero(r.idx + at[p], ok[p]);
+    }
+    if (r.l_aux != nullptr) s_part[tid] = column_part(r, colsum, nb_col);
+    for (int q = tid; q < chunks * stride; q += FIN_THREADS) s_cnt[q] = 0;
+    __syncthreads();
+    fold_columns(r, s_part);
+    int rank[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        int same;
+        rank[p] = rank_in_wave(e[p], ok[p], E, same);
+        if (ok[p] && rank[p] == 0) s_cnt[(p * WAVES + w) * stride + e[p]] = same;
+    }
+    __syncthreads();
+    // exclusive prefix over the chunks, a wave per expert, four at a time
+    for (int e0 = w; e0 < E; e0 += 4 * WAVES) {
+        int run[4] = {0, 0, 0, 0};
+        for (int c0 = 0; c0 < chunks; c0 += WAVE) {
+            const int c = c0 + lane;
+            int n[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) n[u] = load_or_zero(s_cnt + min(c, chunks - 1) * stride + min(e0 + u * WAVES, E - 1), c < chunks);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int incl = wave_scan(n[u]);
+                if (c < chunks && e0 + u * WAVES < E) s_cnt[c * stride + e0 + u * WAVES] = run[u] + incl - n[u];
+                run[u] += wave_total(incl);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (lane == 0 && e0 + u * WAVES < E) s_off[e0 + u * WAVES] = run[u];         // all rows of the expert
+    }
+    __syncthreads();
+    for (int q = tid; q < k * E; q += FIN_THREADS) {         // counts of a choice: where the next one starts less where it does
+        const int j = q / E, ee = q - j * E;
+        const int n = (j + 1 < k ? s_cnt[(j + 1) * per * stride + ee] : s_off[ee]) - s_cnt[j * per * stride + ee];
+        r.counts[q] = n;
+        if (j == 0 && r.l_aux != nullptr) s_part[ee] *= (float)n;
+    }
+    __syncthreads();
+    finish_offsets(r, s_part, s_off, &s_cap);
+    const int cap = s_cap;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        if (!ok[p]) continue;
+        const int l = s_cnt[(p * WAVES + w) * stride + e[p]] + rank[p];
+        r.loc[at[p]] = l;
+        r.row[at[p]] = l < cap ? s_off[e[p]] + l : -1;
     }
 }
 
@@ -357,45 +457,62 @@ __global__ __launch_bounds__(256) void route_finalize_kernel(
 }
 
 // ---- the tokens' own part ------------------------------------------------------------------------------------------
-// 64 tokens per block of 16 waves.  2^LOGG lanes own a token and hold VPL scores each (lane g: experts g, g + G, ...); with
-// 16 lanes per token all 64 tokens go through their rounds at once.  (Four waves on 64 tokens, 16 tokens a wave, four at a
-// time, spent four times the latency of a round: 256 experts, top-8: 42 us for 256 tokens and 58 for 32768, now 9 and 27.)
+// A block of THREADS takes THREADS / 16 tokens.  2^LOGG lanes own a token and hold VPL scores each (lane g: experts g, g + G, ...); with
+// 16 lanes per token all the block's tokens go through their rounds at once.  64 tokens a block where there are many (four waves on 64 tokens, 16 tokens a wave, four at a
+// time, spent four times the latency of a round: 256 experts, top-8: 42 us for 256 tokens and 58 for 32768, now 21 and 45).  Few tokens
+// leave the other CUs idle that way, while the rounds of a block's 16 waves share the four SIMDs of one: they take blocks of four waves
+// and 16 tokens, or, beyond 64 experts, of four tokens with a wave each (256 experts, top-8, 256 tokens: 21 -> 7.8 us).
 // logits != 0: `in` holds logits (without bias if one is given) and the block starts with the softmax (the sums in the order of gate_fwd_kernel's), writing
-// scores.  nb == 1: the block has seen all tokens and goes on to the end of the routing by itself.
-template <int VPL, int LOGG>
-__global__ __launch_bounds__(FIN_THREADS) void route_tokens_kernel(const float *__restrict__ in, const float *__restrict__ bias,
+// scores; LOGITS_PARTS / LOGITS_PAIRS: `in` holds four partial sums of them, [4][S][E], to be added one after the other / in pairs.
+// nb == 1: the block has seen all tokens and goes on to the end of the routing by itself.  hist null: route_rank takes it
+// from the indices.
+enum { LOGITS_NONE, LOGITS_WHOLE, LOGITS_PARTS, LOGITS_PAIRS };
+template <int VPL, int LOGG, int THREADS, int TOK>
+__global__ __launch_bounds__(THREADS) void route_tokens_kernel(const float *__restrict__ in, const float *__restrict__ bias,
                                                                    int logits, int normalize,
                                                                    float *__restrict__ scores, float *__restrict__ gates,
                                                                    int32_t *__restrict__ hist /* [k][E][nb] */,
                                                                    float *__restrict__ colsum /* [nb][E] */, int nb, const RouteEnd r) {
-    constexpr int G = 1 << LOGG, TPP = FIN_THREADS >> LOGG, PASSES = RT_TOKENS > TPP ? RT_TOKENS / TPP : 1;
-    constexpr int WAVES = FIN_THREADS / WAVE;
+    constexpr int G = 1 << LOGG, TPP = THREADS >> LOGG, PASSES = TOK / TPP;
+    constexpr int WAVES = THREADS / WAVE, PER_WAVE = (MOLE_MAX_TOPK + WAVES - 1) / WAVES;
+    constexpr int ROWS = THREADS == 256 ? WAVE / G : 1;      // a small block keeps its waves' token groups' column sums apart
     extern __shared__ __align__(16) char smem[];
     const int S = r.S, E = r.E, k = r.k;
-    int *s_idx = (int *)smem;                          // [k][64]
-    float *s_graw = (float *)(s_idx + k * RT_TOKENS);  // [k][64]
-    int *s_hist = (int *)(s_graw + k * RT_TOKENS);     // [k][E]
-    float *s_col = (float *)(s_hist + k * E);          // [16][E]
-    __shared__ int s_off[FIN_THREADS];
-    __shared__ int s16[WAVES];
+    int *s_idx = (int *)smem;                          // [k][TOK]
+    float *s_graw = (float *)(s_idx + k * TOK);        // [k][TOK]
+    float *s_col = (float *)(s_graw + k * TOK);        // [WAVES ROWS][E]
+    int *s_hist = (int *)(s_col + WAVES * ROWS * E);          // [k][E], with hist or nb == 1
+    int *s_off = s_hist + k * E;                       // [E], nb == 1
+    __shared__ int s_cap;
 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int b = blockIdx.x, tok0 = b * RT_TOKENS;
+    const int b = blockIdx.x, tok0 = b * TOK;
     const int g = lane & (G - 1);
-    for (int i = tid; i < k * E; i += FIN_THREADS) s_hist[i] = 0;
+    const bool count = nb == 1 || hist != nullptr;
+    if (count)
+        for (int i = tid; i < k * E; i += THREADS) s_hist[i] = 0;
     float colacc[VPL];
 #pragma unroll
     for (int q = 0; q < VPL; ++q) colacc[q] = 0.f;
     for (int pass = 0; pass < PASSES; ++pass) {
         const int tl = pass * TPP + (tid >> LOGG);
         const int token = tok0 + tl;
-        const bool tv = tl < RT_TOKENS && token < S;
+        const bool tv = tl < TOK && token < S;
         float v[VPL];
 #pragma unroll
         for (int q = 0; q < VPL; ++q) v[q] = 0.f;
         if (S > 0) {
 #pragma unroll
             for (int q = 0; q < VPL; ++q) v[q] = in[(size_t)min(token, S - 1) * E + min(g + (q << LOGG), E - 1)];
+            if (logits >= LOGITS_PARTS) {
+                float t[3][VPL];
+#pragma unroll
+                for (int u = 0; u < 3; ++u)
+#pragma unroll
+                    for (int q = 0; q < VPL; ++q) t[u][q] = in[((size_t)(u + 1) * S + min(token, S - 1)) * E + min(g + (q << LOGG), E - 1)];
+#pragma unroll
+                for (int q = 0; q < VPL; ++q) v[q] = logits == LOGITS_PARTS ? v[q] + t[0][q] + t[1][q] + t[2][q] : (v[q] + t[0][q]) + (t[1][q] + t[2][q]);
+            }
         }
         if (logits) {
             float mx = -INFINITY;
@@ -405,7 +522,7 @@ __global__ __launch_bounds__(FIN_THREADS) void route_tokens_kernel(const float *
                 v[q] = g + (q << LOGG) < E ? v[q] : -INFINITY;
                 mx = fmaxf(mx, v[q]);
             }
-            for (int m = G / 2; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, WAVE));
+            mx = group_reduce(mx, LOGG, [](float a, float c) { return fmaxf(a, c); });
             float sum = 0.f;
 #pragma unroll
             for (int q = 0; q < VPL; ++q) v[q] = g + (q << LOGG) < E ? expf(v[q] - mx) : 0.f;
@@ -425,7 +542,7 @@ __global__ __launch_bounds__(FIN_THREADS) void route_tokens_kernel(const float *
 #pragma unroll
                 for (int q = 0; q < VPL; ++q) sum += v[q];
                 if constexpr (LOGG == 4) {
-                    for (int m = 8; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, WAVE);
+                    sum = butterfly16(sum);
                 } else {
                     sum = group_reduce(sum, LOGG, [](float a, float d) { return a + d; });
                 }
@@ -462,8 +579,8 @@ __global__ __launch_bounds__(FIN_THREADS) void route_tokens_kernel(const float *
             for (int q = 0; q < VPL; ++q)
                 if (mine && (bi >> LOGG) == q) key[q] = 0u;
             if (g == 0 && tv) {
-                s_idx[j * RT_TOKENS + tl] = bi;
-                s_graw[j * RT_TOKENS + tl] = topk_unkey(top);
+                s_idx[j * TOK + tl] = bi;
+                s_graw[j * TOK + tl] = topk_unkey(top);
             }
         }
     }
@@ -471,47 +588,60 @@ __global__ __launch_bounds__(FIN_THREADS) void route_tokens_kernel(const float *
 #pragma unroll
     for (int q = 0; q < VPL; ++q) {
         float c = colacc[q];
-        for (int m = G; m < WAVE; m <<= 1) c += __shfl_xor(c, m, WAVE);
+        if constexpr (ROWS == 1)
+            for (int m = G; m < WAVE; m <<= 1) c += __shfl_xor(c, m, WAVE);
         const int e = g + (q << LOGG);
-        if (lane < G && e < E) s_col[w * E + e] = c;
+        if ((ROWS > 1 || lane < G) && e < E) s_col[(w * ROWS + (ROWS > 1 ? lane >> LOGG : 0)) * E + e] = c;
     }
     __syncthreads();
-    float me = 0.f;
-    if (tid < E) {
-        for (int q = 0; q < WAVES; ++q) me += s_col[q * E + tid];
-        if (nb > 1) colsum[(size_t)b * E + tid] = me;
+    for (int e = tid; e < E; e += THREADS) {
+        float me = 0.f;
+#pragma unroll
+        for (int q = 0; q < WAVES * ROWS; ++q) me += s_col[q * E + e];
+        if (nb > 1) colsum[(size_t)b * E + e] = me;
+        else s_col[e] = me;
     }
-    // gate values and indices out: thread t < 64 is token t
-    if (tid < RT_TOKENS && tok0 + tid < S) {
+    // gate values and indices out: thread t < TOK is token t
+    if (tid < TOK && tok0 + tid < S) {
         float denom = 0.f;
-        for (int j = 0; j < k; ++j) denom += s_graw[j * RT_TOKENS + tid];  // left to right, fp32
+        for (int j = 0; j < k; ++j) denom += s_graw[j * TOK + tid];  // left to right, fp32
         const float den = denom < FP32_EPS ? FP32_EPS : denom;
         for (int j = 0; j < k; ++j) {
-            float gv = s_graw[j * RT_TOKENS + tid];
+            float gv = s_graw[j * TOK + tid];
             if (k > 1 && normalize) gv = gv / den;
             gates[(size_t)j * S + tok0 + tid] = gv;
-            r.idx[(size_t)j * S + tok0 + tid] = s_idx[j * RT_TOKENS + tid];
+            r.idx[(size_t)j * S + tok0 + tid] = s_idx[j * TOK + tid];
         }
     }
-    // in-block ranks: wave j ranks choice j (k <= 16 = the number of waves), lane = token
+    if (!count) return;
+    // in-block ranks: wave w ranks choices w, w + WAVES, ..., lane = token
     const int token = tok0 + lane;
-    const bool cv = w < k && token < S;
-    const int my_e = cv ? s_idx[w * RT_TOKENS + lane] : 0;
-    int same;
-    const int rank = rank_in_wave(my_e, cv, E, same);
-    if (cv && rank == 0) s_hist[w * E + my_e] = same;
-    if (nb > 1) {
-        if (cv) r.loc[(size_t)w * S + token] = rank;
-        if (w < k)                     // written and read by this wave: program order is enough
-            for (int e = lane; e < E; e += WAVE) hist[((size_t)w * E + e) * nb + b] = s_hist[w * E + e];
-        return;
+    int my_e[PER_WAVE], rank[PER_WAVE];
+#pragma unroll
+    for (int q = 0; q < PER_WAVE; ++q) {
+        const int j = q * WAVES + w;
+        if (j >= k) break;
+        const bool cv = lane < TOK && token < S;
+        my_e[q] = cv ? s_idx[j * TOK + lane] : 0;
+        int same;
+        rank[q] = rank_in_wave(my_e[q], cv, E, same);
+        if (cv && rank[q] == 0) s_hist[j * E + my_e[q]] = same;
+        if (nb > 1) {
+            if (cv) r.loc[(size_t)j * S + token] = rank[q];
+            // written and read by this wave: program order is enough
+            for (int e = lane; e < E; e += WAVE) hist[((size_t)j * E + e) * nb + b] = s_hist[j * E + e];
+        }
     }
+    if (nb > 1) return;
     __syncthreads();
-    const int cap = finish_counts(r, s_hist, me, s_off, s16);
-    if (cv) {
-        const int l = s_hist[w * E + my_e] + rank;
-        r.loc[(size_t)w * S + token] = l;
-        r.row[(size_t)w * S + token] = l < cap ? s_off[my_e] + l : -1;
+    const int cap = finish_counts<THREADS>(r, s_hist, s_col, s_off, &s_cap);
+#pragma unroll
+    for (int q = 0; q < PER_WAVE; ++q) {
+        const int j = q * WAVES + w;
+        if (j >= k || lane >= TOK || token >= S) break;
+        const int l = s_hist[j * E + my_e[q]] + rank[q];
+        r.loc[(size_t)j * S + token] = l;
+        r.row[(size_t)j * S + token] = l < cap ? s_off[my_e[q]] + l : -1;
     }
 }
 
@@ -521,10 +651,15 @@ static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 using namespace mole;
 
+// Up to FEW_TOKENS tokens in small blocks: 16 tokens of up to 64 experts, 16 lanes each, or 4 tokens, a wave each.
+constexpr int FEW_TOKENS = 512;
+static int few_block(int E) { return E <= 64 ? 16 : 4; }
+
 extern "C" size_t mole_route_workspace_bytes(int S, int E, int k) {
     if (S < 0 || E <= 0 || k <= 0) return 0;
     const size_t nb = (size_t)ceil_div(S > 0 ? S : 1, RT_TOKENS);
-    return align256(nb * k * E * sizeof(int32_t)) + align256((size_t)k * E * sizeof(int32_t)) +
+    const size_t few = S <= FEW_TOKENS ? align256((size_t)ceil_div(S, few_block(E)) * E * sizeof(float)) : 0;      // (only their column sums)
+    return few + align256(nb * k * E * sizeof(int32_t)) + align256((size_t)k * E * sizeof(int32_t)) +
            align256(nb * E * sizeof(float)) + align256((size_t)COLSUM_SLICES * E * sizeof(float));
 }
 
@@ -568,16 +703,54 @@ static RouteEnd route_end(int S, int E, int k, double capacity_factor, int align
     return RouteEnd{S, E, k, cf_sign, k * (prod < (double)limit ? (int)prod : limit), alignment, layout, counts, kept_rows, offsets, capacity, l_aux, idx, loc, row};
 }
 
-template <int VPL, int LOGG>
-static int launch_tokens(const float *in, const float *bias, int logits, int normalize, float *scores, float *gates, int32_t *hist, float *colsum,
-                         int nb, const RouteEnd &r, hipStream_t st) {
-    const size_t lds = (size_t)r.k * RT_TOKENS * 8 + (size_t)r.k * r.E * 4 + (size_t)(FIN_THREADS / WAVE) * r.E * 4;
-    auto kern = route_tokens_kernel<VPL, LOGG>;
+template <int VPL, int LOGG, int THREADS, int TOK>
+static int launch_tokens_as(const float *in, const float *bias, int logits, int normalize, float *scores, float *gates, int32_t *hist, float *colsum,
+                            int nb, const RouteEnd &r, hipStream_t st) {
+    constexpr int COLS = THREADS / WAVE * (THREADS == 256 ? WAVE >> LOGG : 1);
+    const size_t lds = (size_t)r.k * TOK * 8 + (size_t)COLS * r.E * 4 + (nb == 1 || hist != nullptr ? (size_t)(r.k + 1) * r.E * 4 : 0);
+    auto kern = route_tokens_kernel<VPL, LOGG, THREADS, TOK>;
     if (lds > 48 * 1024)               // hundreds of experts and a long top-k: beyond the default limit together with the static part
         MOLE_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3(nb), dim3(FIN_THREADS), lds, st, in, bias, logits, normalize, scores, gates, hist, colsum, nb, r);
+    hipLaunchKernelGGL(kern, dim3(nb), dim3(THREADS), lds, st, in, bias, logits, normalize, scores, gates, hist, colsum, nb, r);
     MOLE_LAUNCH_CHECK();
     return 0;
+}
+// few: at most FEW_TOKENS tokens, in blocks of few_block(E)
+static int launch_tokens(bool few, const float *in, const float *bias, int logits, int normalize, float *scores, float *gates, int32_t *hist, float *colsum,
+                         int nb, const RouteEnd &r, hipStream_t st) {
+#define MOLE_LT(VPL, LOGG, THREADS, TOK) launch_tokens_as<VPL, LOGG, THREADS, TOK>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st)
+    const int E = r.E;
+    if (few) {
+        if (E <= 16) return MOLE_LT(1, 4, 256, 16);
+        if (E <= 32) return MOLE_LT(2, 4, 256, 16);
+        if (E <= 64) return MOLE_LT(4, 4, 256, 16);
+        if (E <= 128) return MOLE_LT(2, 6, 256, 4);
+        if (E <= 256) return MOLE_LT(4, 6, 256, 4);
+        return MOLE_LT(16, 6, 256, 4);
+    }
+    // 16 lanes per token; beyond 256 experts a lane would hold more than 16 values, so the whole wave takes a token
+    if (E <= 16) return MOLE_LT(1, 4, 1024, 64);
+    if (E <= 32) return MOLE_LT(2, 4, 1024, 64);
+    if (E <= 64) return MOLE_LT(4, 4, 1024, 64);
+    if (E <= 128) return MOLE_LT(8, 4, 1024, 64);
+    if (E <= 256) return MOLE_LT(16, 4, 1024, 64);
+    return MOLE_LT(16, 6, 1024, 64);
+#undef MOLE_LT
+}
+template <int P> static int launch_rank(const float *colsum, int nb_col, const RouteEnd &r, hipStream_t st) {
+    const size_t lds = (size_t)r.k * ceil_div(r.S, WAVE) * (r.E | 1) * 4;
+    auto kern = route_rank_kernel<P>;
+    if (lds > 48 * 1024) MOLE_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, RANK_COUNTS * 4));
+    hipLaunchKernelGGL(kern, dim3(1), dim3(FIN_THREADS), lds, st, r, colsum, nb_col);
+    MOLE_LAUNCH_CHECK();
+    return 0;
+}
+static int route_rank(const float *colsum, int nb_col, const RouteEnd &r, hipStream_t st) {
+    const int p = ceil_div(r.k * ceil_div(r.S, WAVE), FIN_THREADS / WAVE);
+    if (p <= 1) return launch_rank<1>(colsum, nb_col, r, st);
+    if (p <= 2) return launch_rank<2>(colsum, nb_col, r, st);
+    if (p <= 4) return launch_rank<4>(colsum, nb_col, r, st);
+    return launch_rank<RANK_PAIRS / FIN_THREADS>(colsum, nb_col, r, st);
 }
 
 // The whole routing of scores (or of logits, to which bias is added if given and whose softmax then goes to `scores`).
@@ -585,6 +758,15 @@ static int route_from(const float *in, const float *bias, int logits, int normal
                       hipStream_t st) {
     const int nb = ceil_div(r.S > 0 ? r.S : 1, RT_TOKENS);
     char *ws = (char *)workspace;
+    if (r.S <= few_block(r.E)) return launch_tokens(true, in, bias, logits, normalize, scores, gates, nullptr, nullptr, 1, r, st);
+    const bool few = r.S <= FEW_TOKENS, rank = rank_in_one_block(r.S, r.E, r.k);
+    if (nb == 1 && !(rank && r.E > 64)) return launch_tokens(false, in, bias, logits, normalize, scores, gates, nullptr, nullptr, 1, r, st);
+    if (rank) {
+        float *colsum = (float *)ws;
+        const int blocks = few ? ceil_div(r.S, few_block(r.E)) : nb;
+        if (int rc = launch_tokens(few, in, bias, logits, normalize, scores, gates, nullptr, colsum, blocks, r, st)) return rc;
+        return route_rank(colsum, blocks, r, st);
+    }
     int32_t *hist = (int32_t *)ws;
     ws += align256((size_t)nb * r.k * r.E * sizeof(int32_t));
     int32_t *basej = (int32_t *)ws;
@@ -592,16 +774,7 @@ static int route_from(const float *in, const float *bias, int logits, int normal
     float *colsum = (float *)ws;
     ws += align256((size_t)nb * r.E * sizeof(float));
     float *colpart = (float *)ws;
-    // 16 lanes per token; beyond 256 experts a lane would hold more than 16 values, so the whole wave takes a token
-    const int vpl = ceil_div(r.E, 16);
-    int rc;
-    if (vpl <= 1) rc = launch_tokens<1, 4>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
-    else if (vpl <= 2) rc = launch_tokens<2, 4>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
-    else if (vpl <= 4) rc = launch_tokens<4, 4>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
-    else if (vpl <= 8) rc = launch_tokens<8, 4>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
-    else if (vpl <= 16) rc = launch_tokens<16, 4>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
-    else rc = launch_tokens<16, 6>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st);
-    if (rc || nb == 1) return rc;
+    if (int rc = launch_tokens(false, in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st)) return rc;
     return route_after_topk(r, hist, basej, colsum, colpart, nb, RT_TOKENS, st);
 }
 
@@ -625,7 +798,7 @@ extern "C" int mole_route(const float *scores, int S, int E, int k, double capac
     hipStream_t st = (hipStream_t)stream;
     ScopedTiming timing(MOLE_K_ROUTE, st);
     const RouteEnd r = route_end(S, E, k, capacity_factor, alignment, layout, idx, loc, row, counts, kept_rows, offsets, capacity, l_aux);
-    return route_from(scores, nullptr, 0, normalize_gate, nullptr, gates, r, workspace, st);
+    return route_from(scores, nullptr, LOGITS_NONE, normalize_gate, nullptr, gates, r, workspace, st);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1093,13 +1266,16 @@ __global__ __launch_bounds__(256) void gate_fwd_kernel(const bf16_t *__restrict_
 // the waves'.  A single running sum per wave is a chain of M / 4 additions, which left the logits 1.9 (M = 256) to 3.6 times
 // (M = 4096) as far off as gate_fwd_f32_kernel's 64 lanes do, and with them the gate values; this way they are as close or
 // closer.
-template <typename T, int TG>
-__global__ __launch_bounds__(256, 2) void gate_logits_kernel(const T *__restrict__ x, const float *__restrict__ wg,
+// QUARTERS: a block is one of the four waves and writes its partial logits, [4][S][E], which route_tokens adds up in the same order.  A
+// handful of tokens has so few blocks that each pulls its share of Wg through one CU (1 token, 64 experts of 2048: four blocks
+// of 128 KB, 6.2 us; now 3.6); see gate_quarters.
+template <typename T, int TG, bool QUARTERS>
+__global__ __launch_bounds__(QUARTERS ? 64 : 256, QUARTERS ? 1 : 2) void gate_logits_kernel(const T *__restrict__ x, const float *__restrict__ wg,
                                                           const float *__restrict__ bias, int S, int E, int M,
                                                           float *__restrict__ logits) {
-    constexpr int EPC = 16 / sizeof(T), KSTEP = 4 * EPC, U = TG == 1 ? 8 : 4, NA = sizeof(T) == 2 ? 1 : 4 * U;
+    constexpr int EPC = 16 / sizeof(T), KSTEP = 4 * EPC, U = QUARTERS && sizeof(T) == 2 ? 16 : TG == 1 ? 8 : 4, NA = sizeof(T) == 2 ? 1 : 4 * U;
     __shared__ float part[4][16 * TG][17];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, wave = QUARTERS ? blockIdx.z : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, kq = lane >> 4;
     const int tok0 = blockIdx.x * 16 * TG, e0 = blockIdx.y * 16;
     const int steps = (M + KSTEP - 1) / KSTEP, s_lo = wave * steps / 4, s_hi = (wave + 1) * steps / 4;
@@ -1157,9 +1333,18 @@ __global__ __launch_bounds__(256, 2) void gate_logits_kernel(const T *__restrict
         for (int half = NA / 2; half >= 1; half /= 2)
 #pragma unroll
             for (int i = 0; i < half; ++i) acc[t][i] += acc[t][i + half];
+        if constexpr (QUARTERS) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) part[wave][16 * t + 4 * kq + r][r16] = acc[t][0][r];
+            for (int r = 0; r < 4; ++r) {
+                const int token = tok0 + 16 * t + 4 * kq + r;
+                if (token < S && e0 + r16 < E) logits[((size_t)wave * S + token) * E + e0 + r16] = acc[t][0][r];
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[wave][16 * t + 4 * kq + r][r16] = acc[t][0][r];
+        }
     }
+    if constexpr (QUARTERS) return;
     __syncthreads();
     const int e = e0 + (threadIdx.x & 15);
 #pragma unroll
@@ -1227,6 +1412,8 @@ static size_t gate_route_fused_bytes(int S, int E, int k) {
 //   SCORES  fp32, up to 32 experts: mole_gate_fwd's wave per token, then the routing of the scores
 //   GEMM    logits on the grouped-GEMM tiles, then softmax and routing
 enum { GR_FUSED, GR_FEW, GR_SCORES, GR_GEMM };
+// The logits of FEW by quarters of the model dimension: while four times the blocks are at most one for every CU.
+static bool gate_quarters(int S, int E) { return S <= RT_TOKENS && ceil_div(S, 16) * ceil_div(E, 16) <= 64; }
 static int gate_route_path(int dtype, int S, int E, int M) {
     if (dtype == MOLE_BF16 && M % 128 == 0 && E <= 64 && S > RT_TOKENS) return GR_FUSED;
     if (S <= 2048) return GR_FEW;
@@ -1238,7 +1425,7 @@ extern "C" size_t mole_gate_route_shape_workspace_bytes(int dtype, int S, int E,
     const int path = gate_route_path(dtype, S, E, M);
     if (path == GR_FUSED) return gate_route_fused_bytes(S, E, k);
     size_t n = mole_route_workspace_bytes(S, E, k);
-    if (path != GR_SCORES) n += align256((size_t)S * E * sizeof(float));
+    if (path != GR_SCORES) n += align256((path == GR_FEW && gate_quarters(S, E) ? 4 : 1) * (size_t)S * E * sizeof(float));
     if (path == GR_GEMM && dtype == MOLE_BF16) n += align256((size_t)E * M * sizeof(bf16_t));
     return n;
 }
@@ -1285,22 +1472,30 @@ extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const 
         if (path == GR_SCORES) {
             if (int rc = mole_gate_fwd(x, dtype, wg, logit_bias, S, E, M, scores, stream)) return rc;
             ScopedTiming timing(MOLE_K_ROUTE, st);
-            return route_from(scores, nullptr, 0, normalize_gate, nullptr, gates, r, route_ws, st);
+            return route_from(scores, nullptr, LOGITS_NONE, normalize_gate, nullptr, gates, r, route_ws, st);
         }
         float *logits = (float *)ws;
+        if (path == GR_FEW && gate_quarters(S, E)) {
+            const dim3 grid(ceil_div(S, 16), ceil_div(E, 16), 4);
+            if (dtype == MOLE_BF16) timed_launch(MOLE_K_GATE_FWD, gate_logits_kernel<bf16_t, 1, true>, grid, dim3(64), 0, st, (const bf16_t *)x, wg, nullptr, S, E, M, logits);
+            else timed_launch(MOLE_K_GATE_FWD, gate_logits_kernel<float, 1, true>, grid, dim3(64), 0, st, (const float *)x, wg, nullptr, S, E, M, logits);
+            MOLE_LAUNCH_CHECK();
+            ScopedTiming timing(MOLE_K_ROUTE, st);
+            return route_from(logits, logit_bias, dtype == MOLE_BF16 ? LOGITS_PARTS : LOGITS_PAIRS, normalize_gate, scores, gates, r, route_ws, st);
+        }
         ws += align256((size_t)S * E * sizeof(float));
         if (path == GR_FEW) {
             // Wg is read once for 16 or 32 tokens.  fp32 gates of one or two groups of experts have the blocks to spare
             // (2048 tokens, 16 experts of 4096, with the routing: 32 us in 16s, 38 in 32s); wide ones do not (2000, 256 of 2048: 97 / 86).
             const int tg = S <= 512 || (dtype == MOLE_F32 && E <= 32) ? 1 : 2;
             const dim3 grid(ceil_div(S, 16 * tg), ceil_div(E, 16));
-#define MOLE_GL(T, TG) timed_launch(MOLE_K_GATE_FWD, gate_logits_kernel<T, TG>, grid, dim3(256), 0, st, (const T *)x, wg, logit_bias, S, E, M, logits)
+#define MOLE_GL(T, TG) timed_launch(MOLE_K_GATE_FWD, gate_logits_kernel<T, TG, false>, grid, dim3(256), 0, st, (const T *)x, wg, logit_bias, S, E, M, logits)
             if (dtype == MOLE_BF16) { if (tg == 1) MOLE_GL(bf16_t, 1); else MOLE_GL(bf16_t, 2); }
             else { if (tg == 1) MOLE_GL(float, 1); else MOLE_GL(float, 2); }
 #undef MOLE_GL
             MOLE_LAUNCH_CHECK();
             ScopedTiming timing(MOLE_K_ROUTE, st);
-            return route_from(logits, nullptr, 1, normalize_gate, scores, gates, r, route_ws, st);
+            return route_from(logits, nullptr, LOGITS_WHOLE, normalize_gate, scores, gates, r, route_ws, st);
         }
         const void *w = wg;
         if (dtype == MOLE_BF16) {
@@ -1311,7 +1506,7 @@ extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const 
         }
         if (int rc = mole_gemm_nt(x, w, dtype, S, E, M, logits, stream)) return rc;
         ScopedTiming timing(MOLE_K_ROUTE, st);
-        return route_from(logits, logit_bias, 1, normalize_gate, scores, gates, r, route_ws, st);
+        return route_from(logits, logit_bias, LOGITS_WHOLE, normalize_gate, scores, gates, r, route_ws, st);
     }
     const int nb = ceil_div(S, GATE_ROUTE_TOKENS);
     int32_t *hist = (int32_t *)ws;
@@ -1321,7 +1516,8 @@ extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const 
     float *colsum = (float *)ws;
     ws += align256((size_t)nb * E * sizeof(float));
     float *colpart = (float *)ws;
-    const GateRoute rt{k, normalize_gate, nb, idx, loc, hist, gates, colsum};
+    const bool ranks = rank_in_one_block(S, E, k);
+    const GateRoute rt{k, normalize_gate, nb, idx, loc, ranks ? nullptr : hist, gates, colsum};
     const unsigned route_lds = (unsigned)((size_t)k * GATE_ROUTE_TOKENS * 8 + (size_t)E * 4 * 4 * 2);
     const bf16_t *xb = (const bf16_t *)x;
     if (E <= 16)
@@ -1335,7 +1531,7 @@ extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const 
                      E, M, scores, rt);
     MOLE_LAUNCH_CHECK();
     ScopedTiming timing(MOLE_K_ROUTE, st);
-    return route_after_topk(r, hist, basej, colsum, colpart, nb, GATE_ROUTE_TOKENS, st);
+    return ranks ? route_rank(colsum, nb, r, st) : route_after_topk(r, hist, basej, colsum, colpart, nb, GATE_ROUTE_TOKENS, st);
 }
 
 extern "C" int mole_gate_fwd(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M,

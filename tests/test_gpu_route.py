@@ -63,6 +63,16 @@ def test_route_full_size_configs(name, S, E, k, cf):
     _compare(zipf_scores(S, E, seed=1), k, cf, True)
 
 
+@pytest.mark.parametrize("S,E,k,cf", [
+    # blocks of 16 and of 4 tokens: one block, its edge, many; both ends of the ranking block's pairs (8192) and counts (16384)
+    (4, 65, 3, 0.0), (5, 65, 3, 0.0), (16, 64, 16, 1.0), (17, 64, 16, 0.0), (64, 65, 2, 0.5), (65, 33, 1, 0.0), (512, 256, 4, 0.0), (513, 255, 7, -0.5),
+    (4096, 8, 2, 1.0), (4097, 8, 2, 1.0), (1024, 1024, 1, 0.0), (960, 1023, 1, 0.0), (130, 600, 10, 0.0), (8192, 3, 1, 0.0), (8192, 128, 1, 0.0)])
+@pytest.mark.parametrize("ragged", [True, False])
+def test_route_of_few_tokens_matches_oracle(S, E, k, cf, ragged):
+    print(f"route of few tokens S={S} E={E} k={k} cf={cf} ragged={ragged}", flush=True)
+    _compare(zipf_scores(S, E, seed=S + E + k, ties=E > 4), k, cf, ragged)
+
+
 @pytest.mark.parametrize("S,E", [(100, 8), (513, 16), (64, 100), (300, 256)])
 def test_softmax_and_gate_bwd(S, E):
     from mole_amd import hip_ops as H
