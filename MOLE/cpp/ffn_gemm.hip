@@ -526,12 +526,34 @@ static int ffn_bwd_t(const void *go, const void *xd, const void *h, const void *
         fused_sums = fast_path_enabled() && gemm256_sums_operand(gw2);
     else
         fused_sums = fast_path_enabled() && gemm_f32_sums_operand(gw2);
-    // g_w2[e] = a^T . go          (contract over the expert's rows); g_b2 = sum go
+    // The four products in two pairs that do not need each other: g_w2[e] = a^T . go (contract over the expert's rows; g_b2 = sum go) and
+    // t = (go . w2^T) * gelu'(h) (w2 [F,M]: K = M contiguous), then g_w1[e] = t^T . xd (g_b1 = sum t) and gx = t . w1 (w1 [F,M]: K = F
+    // strided).  Small bf16 layers run a pair as one launch.
     if (fused_sums) { gw2.colsum = g_b2; gw2.colsum_side = 2; }
-    if (int rc = run_gemm<T, true, true, true, EPI_WGRAD>(gw2, max_rows, wg_tiles, st, MOLE_K_FFN_GW2)) return rc;
-    // t = (go . w2^T) * gelu'(h)   (w2 [F,M]: K = M contiguous)
-    g.A = go; g.lda = M; g.B = w2; g.ldb = M; g.strideB = (long)F * M; g.N = F; g.K = M; g.C = t; g.ldc = F; g.H = h;
-    if (int rc = run_gemm<T, false, false, false, EPI_DGELU>(g, max_rows, m_tiles * ceil_div(F, TBN), st, MOLE_K_FFN_DA)) return rc;
+    GemmArgs gda = g, gw1 = g, ggx = g;
+    gda.A = go; gda.lda = M; gda.B = w2; gda.ldb = M; gda.strideB = (long)F * M; gda.N = F; gda.K = M; gda.C = t; gda.ldc = F; gda.H = h;
+    gw1.A = t; gw1.lda = F; gw1.B = xd; gw1.ldb = M; gw1.M = F; gw1.N = M; gw1.C = g_w1; gw1.ldc = M; gw1.strideC = (long)F * M;
+    if (fused_sums) { gw1.colsum = g_b1; gw1.colsum_side = 1; }
+    ggx.A = t; ggx.lda = F; ggx.B = w1; ggx.ldb = M; ggx.strideB = (long)F * M; ggx.N = M; ggx.K = F; ggx.C = gx; ggx.ldc = M;
+    ggx.once = weights_pass_by(E, est_rows, M, F, sizeof(T), 0);
+    // (a result in the place of what the other product reads goes by the order of the two launches)
+    auto overlaps = [&](const void *p, long np, const void *q, long nq) {
+        const uintptr_t a0 = (uintptr_t)p, b0 = (uintptr_t)q, na = (uintptr_t)np * max_rows * sizeof(T), nb = (uintptr_t)nq * max_rows * sizeof(T);
+        return a0 < b0 + nb && b0 < a0 + na;
+    };
+    auto pair = [&](const GemmArgs &r, const GemmArgs &w, bool b_ks, int epi, int kid) {
+        if constexpr (sizeof(T) == 2)
+            if (fast_path_enabled() && fused_sums && max_rows > 0 && !overlaps(r.C, r.N, w.A, w.M) && !overlaps(r.C, r.N, w.B, w.N) &&
+                !gemm_skinny_takes(r, MOLE_BF16, b_ks, max_rows, ws, ws_bytes))
+                return launch_gemm256_pair(r, w, b_ks, epi, max_rows, ws, ws_bytes, st, kid);
+        return -100;
+    };
+    int rc = pair(gda, gw2, false, EPI_DGELU, MOLE_K_FFN_DA);
+    if (rc == -100) {
+        rc = run_gemm<T, true, true, true, EPI_WGRAD>(gw2, max_rows, wg_tiles, st, MOLE_K_FFN_GW2);
+        if (rc == 0) rc = run_gemm<T, false, false, false, EPI_DGELU>(gda, max_rows, m_tiles * ceil_div(F, TBN), st, MOLE_K_FFN_DA);
+    }
+    if (rc) return rc;
     if (!fused_sums) {
         // g_b2 = sum go ; g_b1 = sum t
         ScopedTiming timing(MOLE_K_FFN_GB, st);
@@ -541,17 +563,13 @@ static int ffn_bwd_t(const void *go, const void *xd, const void *h, const void *
                            (const T *)t, F, (T *)g_b1, offsets, kept, accumulate);
         MOLE_LAUNCH_CHECK();
     }
-    // g_w1[e] = t^T . xd ; g_b1 = sum t
-    g.A = t; g.lda = F; g.B = xd; g.ldb = M; g.M = F; g.N = M; g.C = g_w1; g.ldc = M; g.strideC = (long)F * M;
-    if (fused_sums) { g.colsum = g_b1; g.colsum_side = 1; }
-    if (int rc = run_gemm<T, true, true, true, EPI_WGRAD>(g, max_rows, wg_tiles, st, MOLE_K_FFN_GW1)) return rc;
-    g.colsum = nullptr; g.colsum_side = 0;
-    // gx = t . w1                  (w1 [F,M]: K = F strided)
     if (gx != nullptr) {
-        g.A = t; g.lda = F; g.B = w1; g.ldb = M; g.strideB = (long)F * M; g.N = M; g.K = F; g.C = gx; g.ldc = M; g.bias = nullptr;
-        g.once = weights_pass_by(E, est_rows, M, F, sizeof(T), 0);
-        if (int rc = run_gemm<T, false, true, false, EPI_STORE>(g, max_rows, m_tiles * ceil_div(M, TBN), st, MOLE_K_FFN_GX, ws, ws_bytes)) return rc;
+        rc = pair(ggx, gw1, true, EPI_STORE, MOLE_K_FFN_GX);
+        if (rc != -100) return rc;
     }
+    if (int e = run_gemm<T, true, true, true, EPI_WGRAD>(gw1, max_rows, wg_tiles, st, MOLE_K_FFN_GW1)) return e;
+    if (gx != nullptr)
+        return run_gemm<T, false, true, false, EPI_STORE>(ggx, max_rows, m_tiles * ceil_div(M, TBN), st, MOLE_K_FFN_GX, ws, ws_bytes);
     return 0;
 }
 

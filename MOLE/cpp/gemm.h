@@ -181,6 +181,8 @@ struct GemmArgs {
 // 256x256 bf16 tiles with direct-to-LDS loads (gemm256.hip).  Returns -100 when the shape does not
 // meet its alignment requirements; the caller then uses the generic kernel.
 int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
+// ... a row-ragged product of the backward pass and a weight gradient in one launch; -100 where they have no kernel in common.
+int launch_gemm256_pair(const GemmArgs &g, const GemmArgs &w, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
 // planes a K = F product of est_rows rows over E experts would be split into, given the workspace (1: none)
 int gemm256_ksplit(int E, int est_rows, int N, int K);
 // out = sum of the planes (+ bias), for the rows of g's experts (gemm_skinny.hip)
@@ -196,6 +198,7 @@ inline int planes_allowed(int ks, int max_rows, int est_rows, int N) {
 }
 // Few rows per expert (gemm_skinny.hip): weights streamed straight into fragments; -100 when the shape is not its.
 int launch_gemm_skinny(const GemmArgs &g, int dtype, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
+bool gemm_skinny_takes(const GemmArgs &g, int dtype, bool b_ks, int max_rows, void *ws, size_t ws_bytes);
 bool gemm_skinny_takes_tokens(int E, int max_rows, int est_rows, int N, int K, int dtype);    // as dispatched by a DispatchHead
 int gemm_skinny_ksplit(int E, int max_rows, int est_rows, int N, int K, int dtype);    // 0: not its shape
 // fp32 tiles with direct-to-LDS loads (gemm_f32.hip); -100 as above.

@@ -678,12 +678,12 @@ __device__ __forceinline__ void store_sums(const GemmArgs &g, const f32x4 (&sums
 
 // Row-ragged (!WG): C[rows_e, N] = Mop[rows_e, K] . Nop_e ; Mop K-contiguous, Nop_e [N,K] or (N_KS) [K,N].
 // Weight gradient (WG): C_e[M, N] = sum_{r in rows_e} Mop[r, M]^T . Nop[r, N], both K-strided.
+// block: the block's number among those of the product.
 template <int TMB, int WM, int WN, bool N_KS, bool WG, bool KT, int EPI>
-__global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::WAVES_PER_SIMD)) void gemm256_kernel(const GemmArgs g) {
+__device__ __forceinline__ void gemm256_block(const GemmArgs &g, const int block, char *smem) {
     typedef Tile<TMB, WM, WN> TL;
     constexpr bool M_KS = WG;
     constexpr int Q_BM = TL::BM, Q_BN = TL::BN, TMW = TL::TMW;
-    extern __shared__ __align__(16) char smem[];
     // ---- which tile am I?  Blocks are dealt round-robin to the 8 XCDs (block b runs on XCD b mod 8):
     //      give each XCD a contiguous range of the REAL tiles, so that neighbours share operands in
     //      its L2 and every XCD gets the same share.  For row-ragged products the number of real
@@ -756,7 +756,7 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
         if ((n_h + n_l) * n_units > 16 * 256) { split = false; n_h += n_l; n_l = 0; }
         const int total_h = n_h * n_units, total_l = n_l * n_units;
         const int per_h = (total_h + 7) >> 3, per_l = (total_l + 7) >> 3;
-        const int slot = blockIdx.x >> 3, xcd = blockIdx.x & 7;
+        const int slot = block >> 3, xcd = block & 7;
         const bool heavy = slot < per_h;
         const int t = heavy ? xcd * per_h + slot : xcd * per_l + (slot - per_h);
         if (heavy ? t >= total_h : (slot - per_h >= per_l || t >= total_l)) return;
@@ -843,14 +843,14 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
         // on different XCDs each fetch the expert's rows of the n-side operand into their own L2.  Then (wg_expert_major)
         // the experts are dealt round-robin instead, all blocks of one expert on one XCD.
         const int m_tiles = (g.M + Q_BM - 1) / Q_BM;
-        const int slot = blockIdx.x >> 3;
+        const int slot = block >> 3;
         if (g.wg_expert_major) {
             const int u = slot / n_tiles;
-            e = (u / m_tiles) * 8 + (blockIdx.x & 7);
+            e = (u / m_tiles) * 8 + (block & 7);
             mt = u % m_tiles;
             if (e >= g.E) return;
         } else {
-            const int unit = (slot / n_tiles) * 8 + (blockIdx.x & 7);
+            const int unit = (slot / n_tiles) * 8 + (block & 7);
             if (unit >= g.E * m_tiles) return;
             e = unit / m_tiles;
             mt = unit % m_tiles;
@@ -996,6 +996,25 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
 }
 
 template <int TMB, int WM, int WN, bool N_KS, bool WG, bool KT, int EPI>
+__global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::WAVES_PER_SIMD)) void gemm256_kernel(const GemmArgs g) {
+    extern __shared__ __align__(16) char smem[];
+    gemm256_block<TMB, WM, WN, N_KS, WG, KT, EPI>(g, blockIdx.x, smem);
+}
+
+// Two products of the backward pass that do not need each other in one launch, on 128 x 128 tiles: the first `first` blocks a row-ragged
+// one (t = (go.w2^T) gelu'(h), or gx = t.w1), the others a weight gradient (g_w2 beside the former, g_w1 beside the latter).  On
+// their own the row-ragged product of a small layer is a round of tiles that leaves half of the block slots empty and lasts as long as
+// one block's chain of waits, and the weight gradient many short blocks that fill just such holes.  The long blocks start first.
+// Bound by latency.  Training passes, apart / together: 2 x 513 tokens, 16 experts top-4, 520 -> 1416, 366 / 322 us; 2 x 130, 6 of 824 -> 824,
+// top-6, skewed, 300 / 255; 2048 tokens, 16 of 512 -> 1024, top-2, 119 / 113.5.
+template <bool N_KS, bool KT, int EPI>
+__global__ __launch_bounds__((Tile<4, 2, 2>::THREADS), (Tile<4, 2, 2>::WAVES_PER_SIMD)) void gemm256_pair_kernel(const GemmArgs g, const GemmArgs w, int first) {
+    extern __shared__ __align__(16) char smem[];
+    if ((int)blockIdx.x < first) gemm256_block<4, 2, 2, N_KS, false, KT, EPI>(g, blockIdx.x, smem);
+    else gemm256_block<4, 2, 2, true, true, true, EPI_WGRAD>(w, (int)blockIdx.x - first, smem);
+}
+
+template <int TMB, int WM, int WN, bool N_KS, bool WG, bool KT, int EPI>
 static int launch256_kt(GemmArgs g, int tiles, hipStream_t st, int kid) {
     typedef Tile<TMB, WM, WN> TL;
     if (tiles <= 0) return 0;
@@ -1038,6 +1057,15 @@ static int m_fastest_from() { return 8; }
 static bool sums_off() { return false; }
 #endif
 
+// Blocks of a row-ragged launch: the worst-case number of m-tiles (an expert with r rows has ceil(r / BM) of them); + 16, as the heavy
+// and the light tiles of an XCD are rounded up to whole slots separately.  A multiple of 8.
+static int ragged_blocks(const GemmArgs &g, int epi, int rows_bound, int BM, int n_tiles) {
+    const int m_bound = rows_bound / BM + (g.offsets ? min(g.E, rows_bound) : 1);
+    return ((m_bound * n_tiles * (epi == EPI_PART ? g.ksplit : 1) + 7) & ~7) + 16;
+}
+// ... of a weight gradient by whole (expert, m-tile) units per XCD
+static int wgrad_blocks(const GemmArgs &g, int BM, int n_tiles) { return 8 * ceil_div(g.E * ceil_div(g.M, BM), 8) * n_tiles; }
+
 template <int TMB, int WM, int WN>
 static int dispatch256(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_rows, hipStream_t st, int kid) {
     constexpr int BM = Tile<TMB, WM, WN>::BM;
@@ -1050,20 +1078,16 @@ static int dispatch256(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_r
             GemmArgs gw = g;
             gw.wg_expert_major = g.E >= 128 && g.est_rows / g.E >= 768;
             // whole (expert, m-tile) units per XCD, or whole experts
-            const int tiles = gw.wg_expert_major ? 8 * ceil_div(g.E, 8) * ceil_div(g.M, BM) * n_tiles
-                                                 : 8 * ceil_div(g.E * ceil_div(g.M, BM), 8) * n_tiles;
+            const int tiles = gw.wg_expert_major ? 8 * ceil_div(g.E, 8) * ceil_div(g.M, BM) * n_tiles : wgrad_blocks(g, BM, n_tiles);
             if (epi == EPI_WGRAD) return launch256<TMB, WM, WN, true, true, EPI_WGRAD>(gw, tiles, st, kid);
             return -100;
         }
     }
-    // block slots: the worst-case number of m-tiles (an expert with r rows has ceil(r / BM) of them)
     const int rows_bound = g.offsets ? max_rows : g.single_rows;
     GemmArgs gg = g;
     gg.m_fastest = ((m_fastest_mask() >> kid) & 1) ? m_fastest_group() : 0;
     gg.m_fastest_from = m_fastest_from();
-    // (+ 16: the heavy and the light tiles of an XCD are rounded up to whole slots separately)
-    const int m_bound = rows_bound / BM + (g.offsets ? min(g.E, rows_bound) : 1);
-    const int tiles = ((m_bound * n_tiles * (epi == EPI_PART ? g.ksplit : 1) + 7) & ~7) + 16;
+    const int tiles = ragged_blocks(g, epi, rows_bound, BM, n_tiles);
     if (wg) return -100;
     if (!b_ks) {
         if constexpr (TMB != 10) {
@@ -1165,22 +1189,63 @@ bool gemm256_sums_operand(const GemmArgs &g) {
     return !sums_off();
 }
 
-int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid) {
-    // alignment the direct-to-LDS path relies on: 16-byte rows and pieces of K
-    if (g.lda % 8 || g.ldb % 8 || g.ldc % 8 || g.N % 8) return -100;
-    if (!wg && (a_ks || g.K % 8)) return -100;
-    if (wg && (!a_ks || !b_ks || g.M % 8)) return -100;
+// alignment the direct-to-LDS path relies on: 16-byte rows and pieces of K
+static bool aligned256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg) {
+    if (g.lda % 8 || g.ldb % 8 || g.ldc % 8 || g.N % 8) return false;
+    return wg ? a_ks && b_ks && g.M % 8 == 0 : !a_ks && g.K % 8 == 0;
+}
+// the tile of a row-ragged product; where its contraction is split, gp and epi become those of the planes
+static int plan256(GemmArgs &gp, bool b_ks, int &epi, int max_rows, void *ws, size_t ws_bytes) {
     TilePlan p{TILE_256, 1};
-    if (!wg && g.offsets != nullptr && epi < EPI_NONE) p = tile_plan(g.E, g.est_rows, g.N, g.K, b_ks);
-    p.ksplit = planes_allowed(p.ksplit, max_rows, g.est_rows, g.N);
-    if (wg && epi == EPI_WGRAD) p.tile = wgrad_tile(g.E, g.est_rows, g.M, g.N);
-    GemmArgs gp = g;
+    if (gp.offsets != nullptr && epi < EPI_NONE) p = tile_plan(gp.E, gp.est_rows, gp.N, gp.K, b_ks);
+    p.ksplit = planes_allowed(p.ksplit, max_rows, gp.est_rows, gp.N);
     gp.ksplit = 1;
-    if (p.ksplit > 1 && b_ks && ws != nullptr && ws_bytes >= (size_t)p.ksplit * max_rows * g.N * sizeof(float)) {
+    if (p.ksplit > 1 && b_ks && ws != nullptr && ws_bytes >= (size_t)p.ksplit * max_rows * gp.N * sizeof(float)) {
         gp.ksplit = p.ksplit;
         gp.part = (float *)ws;
         gp.part_rows = max_rows;
         epi = EPI_PART;
+    }
+    return p.tile;
+}
+
+template <bool N_KS, bool KT, int EPI> static int launch_pair_kt(const GemmArgs &g, const GemmArgs &w, int max_rows, hipStream_t st, int kid) {
+    typedef Tile<4, 2, 2> TL;
+    const int first = ragged_blocks(g, EPI, max_rows, TL::BM, ceil_div(g.N, TL::BN)), rest = wgrad_blocks(w, TL::BM, ceil_div(w.N, TL::BN));
+    auto kern = gemm256_pair_kernel<N_KS, KT, EPI>;
+    static bool attr_done = false;
+    if (!attr_done) {
+        MOLE_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS_BYTES));
+        attr_done = true;
+    }
+    timed_launch(kid, kern, dim3(first + rest), dim3(TL::THREADS), TL::LDS_BYTES, st, g, w, first);
+    MOLE_LAUNCH_CHECK();
+    return 0;
+}
+template <bool N_KS, int EPI> static int launch_pair(const GemmArgs &g, const GemmArgs &w, int max_rows, hipStream_t st, int kid) {
+    return g.K % Q_BK ? launch_pair_kt<N_KS, true, EPI>(g, w, max_rows, st, kid) : launch_pair_kt<N_KS, false, EPI>(g, w, max_rows, st, kid);
+}
+// The row-ragged product g (EPI_DGELU, or EPI_STORE with K-strided weights) and the weight gradient w together where both take 128 x 128
+// tiles; -100 otherwise, and nothing is launched.
+int launch_gemm256_pair(const GemmArgs &g, const GemmArgs &w, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid) {
+    if (!aligned256(g, false, b_ks, false) || !aligned256(w, true, true, true) || g.offsets == nullptr) return -100;
+    GemmArgs gp = g;
+    if (wgrad_tile(w.E, w.est_rows, w.M, w.N) != TILE_128 || plan256(gp, b_ks, epi, max_rows, ws, ws_bytes) != TILE_128) return -100;
+    int rc;
+    if (epi == EPI_DGELU) rc = launch_pair<false, EPI_DGELU>(gp, w, max_rows, st, kid);
+    else if (epi == EPI_STORE) rc = launch_pair<true, EPI_STORE>(gp, w, max_rows, st, kid);
+    else rc = launch_pair<true, EPI_PART>(gp, w, max_rows, st, kid);
+    return rc != 0 || gp.ksplit == 1 ? rc : launch_plane_reduce(gp, MOLE_BF16, max_rows, st);
+}
+
+int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid) {
+    if (!aligned256(g, a_ks, b_ks, wg)) return -100;
+    GemmArgs gp = g;
+    TilePlan p{TILE_256, 1};
+    if (!wg) p.tile = plan256(gp, b_ks, epi, max_rows, ws, ws_bytes);
+    else {
+        gp.ksplit = 1;
+        if (epi == EPI_WGRAD) p.tile = wgrad_tile(g.E, g.est_rows, g.M, g.N);
     }
     int rc;
     if (p.tile == TILE_128) rc = dispatch256<4, 2, 2>(gp, b_ks, wg, epi, max_rows, st, kid);

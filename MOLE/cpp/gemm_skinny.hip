@@ -618,15 +618,23 @@ static int launch_ks(const GemmArgs &g, int epi, int groups, int max_rows, hipSt
     return 0;
 }
 
+static bool plan_launch(const GemmArgs &g, int dtype, bool b_ks, int max_rows, void *ws, size_t ws_bytes, SkinnyPlan &p) {
+    const int epc = dtype == MOLE_BF16 ? 8 : 4;
+    if (max_rows <= 0 || g.offsets == nullptr || g.kept == nullptr) return false;
+    const bool split = !b_ks || tiles_split(dtype, g.E, max_rows, g.est_rows, g.N, g.K, ws != nullptr ? ws_bytes : 0);
+    if (!skinny_plan(dtype, b_ks, g.E, g.est_rows, g.N, g.K, split, p)) return false;
+    return !(g.K % epc || g.N % epc || g.lda % epc || g.ldb % epc || g.ldc % epc || g.strideB % epc);
+}
+bool gemm_skinny_takes(const GemmArgs &g, int dtype, bool b_ks, int max_rows, void *ws, size_t ws_bytes) {
+    SkinnyPlan p;
+    return plan_launch(g, dtype, b_ks, max_rows, ws, ws_bytes, p);
+}
+
 int launch_gemm_skinny(const GemmArgs &g0, int dtype, bool b_ks, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid) {
     GemmArgs g = g0;
-    const int epc = dtype == MOLE_BF16 ? 8 : 4;
     SkinnyPlan p;
-    if (max_rows <= 0 || g.offsets == nullptr || g.kept == nullptr) return -100;
-    const bool split = !b_ks || tiles_split(dtype, g.E, max_rows, g.est_rows, g.N, g.K, ws != nullptr ? ws_bytes : 0);
-    if (!skinny_plan(dtype, b_ks, g.E, g.est_rows, g.N, g.K, split, p)) return -100;
+    if (!plan_launch(g, dtype, b_ks, max_rows, ws, ws_bytes, p)) return -100;
     const int groups = (g.E < max_rows ? g.E : max_rows) + max_rows / (16 * p.mb);     // as many as max_rows rows can need
-    if (g.K % epc || g.N % epc || g.lda % epc || g.ldb % epc || g.ldc % epc || g.strideB % epc) return -100;
     g.ksplit = 1;
     p.ksplit = planes_allowed(p.ksplit, max_rows, g.est_rows, g.N);
     if (p.ksplit > 1 && ws != nullptr && ws_bytes >= (size_t)p.ksplit * max_rows * g.N * sizeof(float)) {

@@ -519,6 +519,42 @@ def test_ffn_weight_gradients_by_small_tiles(E, M, Fd, rows, gap, accumulate):
         assert rel_err(got, want + 0.5 if accumulate else want) < tol(dtype)
 
 
+# Layers whose backward products all take 128 x 128 tiles run them in two launches, each a row-ragged product beside a weight gradient.
+# A result in the place of an operand of the other product (t in a's place, gx in xd's) is not such a pair: the same launches one
+# after the other give the same bits.  Whole stages and contractions that end inside one; planes; empty and skewed experts.
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("E,M,Fd,rows,gap", [
+    (16, 520, 1416, [128, 97, 131, 0, 161] + [120] * 11, 0), (4, 512, 1024, [257, 228, 0, 255], 3), (2, 256, 1536, [200, 130], 0),
+    (1, 136, 1032, [700], 0), (9, 320, 640, [30, 1, 400, 33, 64, 0, 65, 128, 129], 1)])
+def test_ffn_backward_products_in_pairs(E, M, Fd, rows, gap, accumulate):
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"ffn pairs E={E} M={M} F={Fd} accumulate={accumulate}", flush=True)
+    d = _make(E, M, Fd, rows, torch.bfloat16, seed=E + M, pad_between=gap)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off = torch.from_numpy(d["off"]).cuda(); n = torch.from_numpy(d["n"]).cuda()
+    R = d["R"]
+    out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+    ws = torch.empty(max(1, L.lib().mole_ffn_workspace_bytes(L.MOLE_BF16, E, R, M, Fd)), dtype=torch.uint8, device="cuda")
+    res = []
+    for in_place in (False, True):
+        xd, a_ = c["xd"].clone(), a.clone()
+        t = a_ if in_place else torch.zeros_like(a)
+        gx = xd if in_place else torch.zeros_like(xd)
+        g = [torch.full_like(c[k], 0.5) for k in ("w1", "b1", "w2", "b2")]
+        L.kernel_timing_enable(True)
+        L.kernel_timing_read()
+        L.check(L.lib().mole_ffn_bwd_ws(L.ptr(c["go"]), L.ptr(xd), L.ptr(h), L.ptr(a_), L.MOLE_BF16, L.ptr(off), L.ptr(n), E, R, M, Fd, L.ptr(c["w1"]),
+                                        L.ptr(c["w2"]), L.ptr(t), *[L.ptr(q) for q in g], L.ptr(gx), int(accumulate), L.GELU_BWD_TANH, L.ptr(ws), ws.numel(),
+                                        L.stream()), "mole_ffn_bwd_ws")
+        torch.cuda.synchronize()
+        launches = {k: v[0] for k, v in L.kernel_timing_read().items() if k in ("ffn_gw1", "ffn_gw2")}
+        L.kernel_timing_enable(False)
+        assert sum(launches.values()) == (2 if in_place else 0)
+        live = torch.cat([torch.arange(int(d["off"][e]), int(d["off"][e]) + int(d["n"][e])) for e in range(E)]).cuda()
+        res.append([t[live], gx[live]] + g)
+    assert all(torch.equal(x, y) for x, y in zip(*res))
+
+
 # K-strided weights read past the caches, in a forward pass that no backward follows: from 64 MB of weights of the experts that
 # can have rows, the recorded pass (256 MB) taking the ordinary loads.  Experts of a few rows on the kernel for them, of up
 # to 64 and up to 128 on the tiles, of more (ordinary loads there), and of none.  The loads' cache policy changes no result.
