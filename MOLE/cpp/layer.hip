@@ -23,11 +23,6 @@ __global__ __launch_bounds__(256) void pad_convert_kernel(const float *__restric
     const int y = (int)(i / co), x = (int)(i % co);
     out[i] = y < r && x < c ? from_f32<T>(in[(size_t)y * c + x]) : from_f32<T>(0.f);
 }
-template <typename T>
-__global__ __launch_bounds__(256) void to_f32_kernel(const T *__restrict__ in, float *__restrict__ out, size_t n) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) out[i] = to_f32(in[i]);
-}
 static int pad_convert(const float *in, int r, int c, void *out, int ro, int co, int dtype, hipStream_t st) {
     const dim3 grid((unsigned)(((size_t)ro * co + 255) / 256));
     if (dtype == MOLE_BF16) hipLaunchKernelGGL(pad_convert_kernel<bf16_t>, grid, dim3(256), 0, st, in, r, c, (bf16_t *)out, ro, co);
@@ -36,10 +31,9 @@ static int pad_convert(const float *in, int r, int c, void *out, int ro, int co,
     return 0;
 }
 
-// Scratch of the backward's gate part, and which way its two products go.
+// Scratch of the backward's gate part, and which way its input gradient goes.
 struct GateBwdPlan {
     bool fold;           // dlogits . Wg inside the dispatch backward (up to 32 experts)
-    bool wgrad_kernel;   // dlogits^T . x on the gate's own kernel, otherwise on the grouped-GEMM tiles
     int e_pad;           // experts rounded up to the tiles' granule
     size_t dgates, dl_t, wg_t, dx_add, wgrad, total;     // bytes
 };
@@ -48,13 +42,12 @@ static GateBwdPlan gate_bwd_plan(const mole_layer &L) {
     const size_t es = L.dtype == MOLE_BF16 ? 2 : 4;
     const int epc = L.dtype == MOLE_BF16 ? 8 : 4;
     p.fold = L.E <= 32;
-    p.wgrad_kernel = (L.dtype == MOLE_BF16 && L.E <= 256 && L.M % 64 == 0) || L.E <= 32;
     p.e_pad = (L.E + epc - 1) / epc * epc;
     p.dgates = L.E > 256 ? up256((size_t)L.k * L.S * 4) : 0;
-    p.dl_t = p.fold && p.wgrad_kernel ? 0 : up256((size_t)L.S * p.e_pad * es);
+    p.dl_t = p.fold ? 0 : up256((size_t)L.S * p.e_pad * es);
     p.wg_t = p.fold ? 0 : up256((size_t)p.e_pad * L.M * es);
     p.dx_add = p.fold ? 0 : up256((size_t)L.S * L.M * es);
-    p.wgrad = up256(p.wgrad_kernel ? mole_gate_wgrad_workspace_bytes(L.S, L.E, L.M) : (size_t)p.e_pad * L.M * es);
+    p.wgrad = up256(mole_gate_wgrad_workspace_bytes(L.S, L.E, L.M));
     p.total = p.dgates + p.dl_t + p.wg_t + p.dx_add + p.wgrad;
     return p;
 }
@@ -132,21 +125,13 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
                                  G->t, G->g_w1, G->g_b1, G->g_w2, G->g_b2, G->gxd, G->accumulate, G->gelu_bwd, L->workspace,
                                  L->workspace_bytes, st)) return rc;
     char *dl_t = ws + p.dgates, *wg_t = dl_t + p.dl_t, *dx_add = wg_t + p.wg_t, *wgrad = dx_add + p.dx_add;
-    if (p.dl_t)
-        if (int rc = pad_convert(G->dlogits, L->S, L->E, dl_t, L->S, p.e_pad, L->dtype, st)) return rc;
     if (p.fold) {
         if (int rc = mole_dispatch_bwd(G->gxd, L->dtype, L->row, L->S, L->M, L->k, G->dlogits, L->wg, L->E, nullptr, G->dx, stream)) return rc;
     } else {
+        if (int rc = pad_convert(G->dlogits, L->S, L->E, dl_t, L->S, p.e_pad, L->dtype, st)) return rc;
         if (int rc = pad_convert(L->wg, L->E, L->M, wg_t, p.e_pad, L->M, L->dtype, st)) return rc;
         if (int rc = mole_gemm_nn(dl_t, wg_t, L->dtype, L->S, L->M, p.e_pad, dx_add, stream)) return rc;
         if (int rc = mole_dispatch_bwd(G->gxd, L->dtype, L->row, L->S, L->M, L->k, nullptr, nullptr, 0, dx_add, G->dx, stream)) return rc;
     }
-    if (p.wgrad_kernel) return mole_gate_wgrad(G->dlogits, L->x, L->dtype, L->S, L->E, L->M, G->dwg, wgrad, p.wgrad, stream);
-    if (int rc = mole_gemm_tn(dl_t, L->x, L->dtype, L->S, p.e_pad, L->M, wgrad, stream)) return rc;
-    const size_t n = (size_t)L->E * L->M;
-    const dim3 grid((unsigned)((n + 255) / 256));
-    if (L->dtype == MOLE_BF16) hipLaunchKernelGGL(to_f32_kernel<bf16_t>, grid, dim3(256), 0, st, (const bf16_t *)wgrad, G->dwg, n);
-    else hipLaunchKernelGGL(to_f32_kernel<float>, grid, dim3(256), 0, st, (const float *)wgrad, G->dwg, n);
-    MOLE_LAUNCH_CHECK();
-    return 0;
+    return gate_wgrad(G->dlogits, L->x, L->dtype, L->S, L->E, L->M, G->dwg, wgrad, p.wgrad, st);
 }

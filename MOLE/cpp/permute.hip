@@ -513,66 +513,78 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
 // gw_tokens() tokens write partial [E, M] sums, a second kernel adds the partials in order.
 constexpr int GW_TOKENS = 64, GW_TOKENS_FEW = 16;
 // A block walks its tokens in batches of eight, one round trip to memory each: short blocks where long ones leave CUs
-// idle (513 tokens x 520, 16 experts: 11.5 -> 4.9 us; 110 x 384 fp32, 29 experts: 17.3 -> 7.0).
-static int gw_tokens(int S, int M) { return (long)ceil_div(S, GW_TOKENS) * ceil_div(M, 512) < 192 ? GW_TOKENS_FEW : GW_TOKENS; }
+// idle (513 tokens x 520, 16 experts: 11.5 -> 4.9 us; 110 x 384 fp32, 29 experts: 17.3 -> 7.0).  Gates of more than 32 experts take
+// a block per 32 of them, and chunks of more tokens while the partial sums would fill more than 32 MB.
+static int gw_tokens(int S, int E, int M) {
+    const int zs = ceil_div(E, 32);
+    int t = (long)ceil_div(S, GW_TOKENS) * ceil_div(M, 512) * zs < 192 ? GW_TOKENS_FEW : GW_TOKENS;
+    if (zs > 1)
+        while ((size_t)ceil_div(S, t) * E * M * sizeof(float) > (32u << 20) && t < S) t *= 2;
+    return t;
+}
 template <typename T, int EB>
 __global__ __launch_bounds__(256) void gate_wgrad_partial_kernel(const float *__restrict__ dlogits,
                                                                  const T *__restrict__ x, int S, int E, int M, int tokens,
                                                                  float *__restrict__ part) {
     __shared__ __align__(16) float s_dl[GW_TOKENS][EB];
-    const int i0 = blockIdx.x * tokens;
-    const int nt = min(tokens, S - i0);
-    for (int idx = threadIdx.x; idx < tokens * EB; idx += 256) {
-        const int t = idx / EB, e = idx % EB;
-        s_dl[t][e] = (t < nt && e < E) ? dlogits[(size_t)(i0 + t) * E + e] : 0.f;
-    }
-    __syncthreads();
     const int m = (blockIdx.y * 256 + threadIdx.x) * 2;    // two columns per thread
-    if (m >= M) return;
+    const int e0 = blockIdx.z * EB;
+    const bool col_ok = m < M;
     float acc[EB][2];
 #pragma unroll
     for (int e = 0; e < EB; ++e) acc[e][0] = acc[e][1] = 0.f;
-    const T *px = x + (size_t)i0 * M + m;
-    // eight rows per batch, the next batch's loads in flight while the current one is used
-    auto load8 = [&](float (&xv)[8][2], int t0) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int t = min(t0 + u, nt - 1);
-            if constexpr (sizeof(T) == 2) {
-                const uint32_t v = *reinterpret_cast<const uint32_t *>(px + (size_t)t * M);
-                xv[u][0] = __uint_as_float(v << 16); xv[u][1] = __uint_as_float(v & 0xffff0000u);
-            } else {
-                const float2 v = *reinterpret_cast<const float2 *>(px + (size_t)t * M);
-                xv[u][0] = v.x; xv[u][1] = v.y;
-            }
+    const int last = min((int)(blockIdx.x + 1) * tokens, S);
+    for (int i0 = blockIdx.x * tokens; i0 < last; i0 += GW_TOKENS) {       // up to 64 of the chunk's tokens at a time
+        const int nt = min(GW_TOKENS, last - i0);
+        if (i0 != (int)blockIdx.x * tokens) __syncthreads();
+        for (int idx = threadIdx.x; idx < nt * EB; idx += 256) {
+            const int t = idx / EB, e = idx % EB;
+            s_dl[t][e] = e0 + e < E ? dlogits[(size_t)(i0 + t) * E + e0 + e] : 0.f;
         }
-    };
-    auto use8 = [&](const float (&xv)[8][2], int t0) __attribute__((always_inline)) {
+        __syncthreads();
+        const T *px = x + (size_t)i0 * M + (col_ok ? m : 0);
+        // eight rows per batch, the next batch's loads in flight while the current one is used
+        auto load8 = [&](float (&xv)[8][2], int t0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            if (t0 + u >= nt) break;
-#pragma unroll
-            for (int e = 0; e < EB; e += 4) {
-                const float4 d = *reinterpret_cast<const float4 *>(&s_dl[t0 + u][e]);   // same address in every lane
-                acc[e][0] += d.x * xv[u][0]; acc[e][1] += d.x * xv[u][1];
-                acc[e + 1][0] += d.y * xv[u][0]; acc[e + 1][1] += d.y * xv[u][1];
-                acc[e + 2][0] += d.z * xv[u][0]; acc[e + 2][1] += d.z * xv[u][1];
-                acc[e + 3][0] += d.w * xv[u][0]; acc[e + 3][1] += d.w * xv[u][1];
+            for (int u = 0; u < 8; ++u) {
+                const int t = min(t0 + u, nt - 1);
+                if constexpr (sizeof(T) == 2) {
+                    const uint32_t v = *reinterpret_cast<const uint32_t *>(px + (size_t)t * M);
+                    xv[u][0] = __uint_as_float(v << 16); xv[u][1] = __uint_as_float(v & 0xffff0000u);
+                } else {
+                    const float2 v = *reinterpret_cast<const float2 *>(px + (size_t)t * M);
+                    xv[u][0] = v.x; xv[u][1] = v.y;
+                }
             }
+        };
+        auto use8 = [&](const float (&xv)[8][2], int t0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (t0 + u >= nt) break;
+#pragma unroll
+                for (int e = 0; e < EB; e += 4) {
+                    const float4 d = *reinterpret_cast<const float4 *>(&s_dl[t0 + u][e]);   // same address in every lane
+                    acc[e][0] += d.x * xv[u][0]; acc[e][1] += d.x * xv[u][1];
+                    acc[e + 1][0] += d.y * xv[u][0]; acc[e + 1][1] += d.y * xv[u][1];
+                    acc[e + 2][0] += d.z * xv[u][0]; acc[e + 2][1] += d.z * xv[u][1];
+                    acc[e + 3][0] += d.w * xv[u][0]; acc[e + 3][1] += d.w * xv[u][1];
+                }
+            }
+        };
+        float xa[8][2], xb[8][2];
+        load8(xa, 0);
+        for (int t0 = 0; t0 < nt; t0 += 16) {
+            load8(xb, t0 + 8);
+            use8(xa, t0);
+            load8(xa, t0 + 16);
+            use8(xb, t0 + 8);
         }
-    };
-    float xa[8][2], xb[8][2];
-    load8(xa, 0);
-    for (int t0 = 0; t0 < nt; t0 += 16) {
-        load8(xb, t0 + 8);
-        use8(xa, t0);
-        load8(xa, t0 + 16);
-        use8(xb, t0 + 8);
     }
+    if (!col_ok) return;
 #pragma unroll
     for (int e = 0; e < EB; ++e)
-        if (e < E)
-            *reinterpret_cast<float2 *>(part + ((size_t)blockIdx.x * E + e) * M + m) = make_float2(acc[e][0], acc[e][1]);
+        if (e0 + e < E)
+            *reinterpret_cast<float2 *>(part + ((size_t)blockIdx.x * E + e0 + e) * M + m) = make_float2(acc[e][0], acc[e][1]);
 }
 // The partial sums on the matrix cores, for bf16 tokens and gates of up to 256 experts:
 // part[chunk][e][m] = sum over the chunk's tokens of dlogits[t][e] x[t][m], a [E x tokens] by [tokens x M]
@@ -1117,12 +1129,60 @@ extern "C" int mole_dispatch_bwd(const void *dxd, int dtype, const int32_t *row,
 
 extern "C" size_t mole_gate_wgrad_workspace_bytes(int S, int E, int M) {
     if (S <= 0 || E <= 0 || M <= 0) return 0;
-    // enough for either kernel: the caller does not say the dtype here (small gates: the VALU kernel's
-    // partials; large gates only run on the matrix cores, with their own chunking)
+    // enough for either kernel: the caller does not say the dtype here
     const size_t mfma = (size_t)ceil_div(S, gate_wgrad_mfma_chunk(S, E, M)) * E * M * sizeof(float);
-    const size_t valu = E <= 32 ? (size_t)ceil_div(S, gw_tokens(S, M)) * E * M * sizeof(float) : 0;
+    const size_t valu = (size_t)ceil_div(S, gw_tokens(S, E, M)) * E * M * sizeof(float);
     return mfma > valu ? mfma : valu;
 }
+
+namespace mole {
+// Any number of experts.  A single chunk of tokens writes the result itself, without the reduction's launch.  Gates that neither kernel took
+// before went through the grouped-GEMM tiles, a block's walk over all tokens for 128 x 128 results, in the tokens' type: fp32, 3380 tokens, 79
+// experts of 448: 254 us; training passes, before / now: 8 tokens, 172 experts of 920 -> 456, 157 / 124; 4041 fp32 tokens, 245 of 704 -> 2112, 3127 /
+// 2833.
+int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int M, float *dwg, void *workspace, size_t workspace_bytes, hipStream_t st) {
+    ScopedTiming timing(MOLE_K_GATE_WGRAD, st);
+    MOLE_REQUIRE(dlogits && x && dwg && workspace && aligned16(x) && aligned16(dwg) && aligned16(workspace), "mole_gate_wgrad: null or misaligned pointer");
+    if (workspace_bytes < mole_gate_wgrad_workspace_bytes(S, E, M)) {
+        set_error("mole_gate_wgrad: workspace of %zu bytes, need %zu", workspace_bytes, mole_gate_wgrad_workspace_bytes(S, E, M));
+        return MOLE_E_WORKSPACE;
+    }
+    int nb;
+    float *part;
+    if (gate_wgrad_mfma_ok(dtype, S, E, M)) {
+        const int chunk = gate_wgrad_mfma_chunk(S, E, M);
+        nb = ceil_div(S, chunk);
+        part = nb == 1 ? dwg : (float *)workspace;
+        const int eg = E <= 16 ? 1 : (E <= 32 ? 2 : 4);
+        const int nz = ceil_div(E, 16 * eg), nunits = nb * ceil_div(M, 256);
+        const dim3 grid((unsigned)(ceil_div(nunits, 8) * 8 * nz));
+#define MOLE_GM(EG, V) hipLaunchKernelGGL((gate_wgrad_mfma_kernel<EG, V>), grid, dim3(256), 0, st, dlogits, (const bf16_t *)x, S, E, M, chunk, nb, nz, part)
+        if (E % 4 == 0 && aligned16(dlogits)) {
+            if (eg == 1) MOLE_GM(1, true); else if (eg == 2) MOLE_GM(2, true); else MOLE_GM(4, true);
+        } else {
+            if (eg == 1) MOLE_GM(1, false); else if (eg == 2) MOLE_GM(2, false); else MOLE_GM(4, false);
+        }
+#undef MOLE_GM
+    } else {
+        const int tokens = gw_tokens(S, E, M);
+        nb = ceil_div(S, tokens);
+        part = nb == 1 ? dwg : (float *)workspace;
+        const dim3 grid(nb, ceil_div(M, 512), ceil_div(E, 32));
+#define MOLE_GW(T, EB) hipLaunchKernelGGL((gate_wgrad_partial_kernel<T, EB>), grid, dim3(256), 0, st, dlogits, (const T *)x, S, E, M, tokens, part)
+        if (dtype == MOLE_BF16) {
+            if (E <= 8) MOLE_GW(bf16_t, 8); else if (E <= 16) MOLE_GW(bf16_t, 16); else MOLE_GW(bf16_t, 32);
+        } else {
+            if (E <= 8) MOLE_GW(float, 8); else if (E <= 16) MOLE_GW(float, 16); else MOLE_GW(float, 32);
+        }
+#undef MOLE_GW
+    }
+    MOLE_LAUNCH_CHECK();
+    if (nb == 1) return 0;
+    hipLaunchKernelGGL(gate_wgrad_reduce_kernel, dim3(ceil_div(E * M, 64)), dim3(256), 0, st, part, nb, E * M, dwg);
+    MOLE_LAUNCH_CHECK();
+    return 0;
+}
+}  // namespace mole
 
 extern "C" int mole_gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int M, float *dwg,
                                void *workspace, size_t workspace_bytes, mole_stream_t stream) {
@@ -1131,49 +1191,12 @@ extern "C" int mole_gate_wgrad(const float *dlogits, const void *x, int dtype, i
                  "mole_gate_wgrad: need E <= 32, or bf16 tokens with E <= 256 and M %% 64 == 0 (S=%d E=%d M=%d dtype=%d)", S, E, M, dtype);
     MOLE_REQUIRE(dwg != nullptr, "mole_gate_wgrad: null output");
     hipStream_t st = (hipStream_t)stream;
+    if (S > 0) return gate_wgrad(dlogits, x, dtype, S, E, M, dwg, workspace, workspace_bytes, st);
+    // no tokens: the reduction over zero partials writes the zeros (a kernel, not a memset, so that a
+    // caller may capture the call in a graph)
     ScopedTiming timing(MOLE_K_GATE_WGRAD, st);
-    if (S == 0) {
-        // no tokens: the reduction over zero partials writes the zeros (a kernel, not a memset, so that a
-        // caller may capture the call in a graph)
-        MOLE_REQUIRE(aligned16(dwg), "mole_gate_wgrad: misaligned output");
-        hipLaunchKernelGGL(gate_wgrad_reduce_kernel, dim3(ceil_div(E * M, 64)), dim3(256), 0, st, (const float *)dwg, 0, E * M, dwg);
-        MOLE_LAUNCH_CHECK();
-        return 0;
-    }
-    MOLE_REQUIRE(dlogits && x && workspace && aligned16(x) && aligned16(dwg) && aligned16(workspace), "mole_gate_wgrad: null or misaligned pointer");
-    if (workspace_bytes < mole_gate_wgrad_workspace_bytes(S, E, M)) {
-        set_error("mole_gate_wgrad: workspace of %zu bytes, need %zu", workspace_bytes, mole_gate_wgrad_workspace_bytes(S, E, M));
-        return MOLE_E_WORKSPACE;
-    }
-    float *part = (float *)workspace;
-    if (gate_wgrad_mfma_ok(dtype, S, E, M)) {
-        const int chunk = gate_wgrad_mfma_chunk(S, E, M), nchunks = ceil_div(S, chunk);
-        const int eg = E <= 16 ? 1 : (E <= 32 ? 2 : 4);
-        const int nz = ceil_div(E, 16 * eg), nunits = nchunks * ceil_div(M, 256);
-        const dim3 grid((unsigned)(ceil_div(nunits, 8) * 8 * nz));
-#define MOLE_GM(EG, V) hipLaunchKernelGGL((gate_wgrad_mfma_kernel<EG, V>), grid, dim3(256), 0, st, dlogits, (const bf16_t *)x, S, E, M, chunk, nchunks, nz, part)
-        if (E % 4 == 0 && aligned16(dlogits)) {
-            if (eg == 1) MOLE_GM(1, true); else if (eg == 2) MOLE_GM(2, true); else MOLE_GM(4, true);
-        } else {
-            if (eg == 1) MOLE_GM(1, false); else if (eg == 2) MOLE_GM(2, false); else MOLE_GM(4, false);
-        }
-#undef MOLE_GM
-        MOLE_LAUNCH_CHECK();
-        hipLaunchKernelGGL(gate_wgrad_reduce_kernel, dim3(ceil_div(E * M, 64)), dim3(256), 0, st, part, nchunks, E * M, dwg);
-        MOLE_LAUNCH_CHECK();
-        return 0;
-    }
-    const int tokens = gw_tokens(S, M), nb = ceil_div(S, tokens);
-    const dim3 grid(nb, ceil_div(M, 512));
-#define MOLE_GW(T, EB) hipLaunchKernelGGL((gate_wgrad_partial_kernel<T, EB>), grid, dim3(256), 0, st, dlogits, (const T *)x, S, E, M, tokens, part)
-    if (dtype == MOLE_BF16) {
-        if (E <= 8) MOLE_GW(bf16_t, 8); else if (E <= 16) MOLE_GW(bf16_t, 16); else MOLE_GW(bf16_t, 32);
-    } else {
-        if (E <= 8) MOLE_GW(float, 8); else if (E <= 16) MOLE_GW(float, 16); else MOLE_GW(float, 32);
-    }
-#undef MOLE_GW
-    MOLE_LAUNCH_CHECK();
-    hipLaunchKernelGGL(gate_wgrad_reduce_kernel, dim3(ceil_div(E * M, 64)), dim3(256), 0, st, part, nb, E * M, dwg);
+    MOLE_REQUIRE(aligned16(dwg), "mole_gate_wgrad: misaligned output");
+    hipLaunchKernelGGL(gate_wgrad_reduce_kernel, dim3(ceil_div(E * M, 64)), dim3(256), 0, st, (const float *)dwg, 0, E * M, dwg);
     MOLE_LAUNCH_CHECK();
     return 0;
 }

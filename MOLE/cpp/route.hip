@@ -1408,7 +1408,9 @@ static size_t gate_route_fused_bytes(int S, int E, int k) {
 //           (a block of 32 tokens reads all of Wg, so with few tokens few blocks read it one after the other:
 //           1 token, 64 experts of 2048: 21 + 17 + 4 us in three kernels against 4 + 7 us)
 //   FEW     logits by 16 x 16 tiles, then softmax and routing: up to 2048 tokens (2048 blocks at 256 experts; beyond, the
-//           re-reads of x and Wg by the tiles cost more than the GEMM's tiles)
+//           re-reads of x and Wg by the tiles cost more than the GEMM's tiles), in fp32, whose GEMM tiles are 128 x 128 of one
+//           block's walk over M, up to 3072 blocks (2977 tokens, 200 experts of 1536: 139 / 69 us; 8192, 40 of 2048: 167 / 52; 16384, 64
+//           of 1032: 97 / 66; 16384, 128 of 512, 4096 blocks: 64 / 71; 32768, 80 of 1032: 111 / 137)
 //   SCORES  fp32, up to 32 experts: mole_gate_fwd's wave per token, then the routing of the scores
 //   GEMM    logits on the grouped-GEMM tiles, then softmax and routing
 enum { GR_FUSED, GR_FEW, GR_SCORES, GR_GEMM };
@@ -1416,7 +1418,7 @@ enum { GR_FUSED, GR_FEW, GR_SCORES, GR_GEMM };
 static bool gate_quarters(int S, int E) { return S <= RT_TOKENS && ceil_div(S, 16) * ceil_div(E, 16) <= 64; }
 static int gate_route_path(int dtype, int S, int E, int M) {
     if (dtype == MOLE_BF16 && M % 128 == 0 && E <= 64 && S > RT_TOKENS) return GR_FUSED;
-    if (S <= 2048) return GR_FEW;
+    if (S <= 2048 || (dtype == MOLE_F32 && E > 32 && (long)ceil_div(S, 32) * ceil_div(E, 16) <= 3072)) return GR_FEW;
     return dtype == MOLE_F32 && E <= 32 ? GR_SCORES : GR_GEMM;
 }
 

@@ -87,6 +87,16 @@ def _run_and_compare(m, x, ref, k, cf, dtype, gelu_bwd="tanh", normalize=True, a
     return res
 
 
+# gates of more than 32 experts whose weight gradient does not go through the matrix cores (fp32, widths that are no multiple of 64, more
+# than 256 experts): the last group of 32 short, one chunk of tokens (16 or fewer) and many, chunks of more than 64 tokens
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("S,M,E,k,Fd,cf", [(12, 72, 40, 2, 64, 0.0), (17, 520, 33, 1, 32, 0.0), (1300, 136, 70, 4, 32, 1.25), (300, 64, 300, 2, 16, 0.0), (9000, 1032, 100, 1, 8, 0.0)])
+def test_layer_with_a_large_gate(S, M, E, k, Fd, cf, dtype):
+    print(f"layer with a large gate S={S} M={M} E={E} k={k} F={Fd} {dtype}", flush=True)
+    m, x, ref = _build(S, M, E, k, Fd, dtype)
+    _run_and_compare(m, x, ref, k, cf, dtype, aux_w=0.5)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("reference_layout", [False, True])
 @pytest.mark.parametrize("S,M,E,k,Fd,cf", [(300, 64, 4, 2, 128, 1.0), (1000, 128, 8, 1, 256, 1.25), (513, 64, 16, 4, 128, 0.0)])
