@@ -462,6 +462,7 @@ static int run_gemm(const GemmArgs &g, int max_rows, int tiles_generic, hipStrea
             if (rc != -100) return rc;
         }
     }
+    MOLE_REQUIRE(g.token_of == nullptr, "grouped GEMM: tokens in place of dispatched rows for a kernel that reads rows");
     // only the direct-to-LDS kernels sum an operand on the side: the caller asks gemm*_sums_operand() first
     MOLE_REQUIRE(g.colsum == nullptr, "grouped GEMM: operand sums requested from a kernel that does not produce them");
     return launch_gemm<T, A_KS, B_KS, WG, TBM, TBN, EPI>(g, tiles_generic, st, kid);
@@ -493,10 +494,11 @@ static int ffn_fwd_t(const void *xd, const int32_t *offsets, const int32_t *kept
     // (h is for the backward pass alone: a store of R F elements and a turn through LDS less where none follows; 6002 rows,
     // 16 experts, 1024 -> 4096: the pass 188.4 -> 183.0 us, and 49 MB less memory)
     g.C = forward_only ? nullptr : h; g.C2 = a; g.ldc = F; g.bias = b1;
-    if (head != nullptr) { g.pair_row = head->row; g.tokens = head->S; g.pairs = head->S * head->k; }
+    if (head != nullptr && head->token_of != nullptr) { g.token_of = head->token_of; g.tokens = head->S; }
+    else if (head != nullptr) { g.pair_row = head->row; g.tokens = head->S; g.pairs = head->S * head->k; }
     if (int rc = run_gemm<T, false, false, false, EPI_BIAS_GELU>(g, max_rows, m_tiles * ceil_div(F, TBN), st, MOLE_K_FFN_FWD1)) return rc;
     // out = a . w2 + b2   (w2 [F,M]: K-strided)
-    g.pair_row = nullptr;
+    g.pair_row = g.token_of = nullptr;
     g.A = a; g.lda = F; g.B = w2; g.ldb = M; g.strideB = (long)F * M; g.N = M; g.K = F;
     g.C = out; g.C2 = nullptr; g.ldc = M; g.bias = b2;
     g.once = weights_pass_by(E, est_rows, M, F, sizeof(T), forward_only);
@@ -596,8 +598,10 @@ size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, 
     return ks > 1 ? (size_t)ks * max_rows * M * sizeof(float) : 0;
 }
 
-bool ffn_fwd_takes_tokens(int dtype, int E, int max_rows, int est_rows, int M, int F) {
-    return fast_path_enabled() && gemm_skinny_takes_tokens(E, max_rows, est_rows, F, M, dtype);
+FwdTokens ffn_fwd_takes_tokens(int dtype, int E, int max_rows, int est_rows, int M, int F) {
+    if (!fast_path_enabled()) return TOKENS_NO;
+    if (gemm_skinny_takes_tokens(E, max_rows, est_rows, F, M, dtype)) return TOKENS_PAIRS;
+    return max_rows > 0 && (dtype == MOLE_BF16 ? M % 8 == 0 && F % 8 == 0 : gemm_f32_takes(F, M)) ? TOKENS_LIST : TOKENS_NO;
 }
 
 int ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, int est_rows, int M, int F,

@@ -137,9 +137,11 @@ struct CombineTail {
     bool done;
 };
 
-// The dispatch in front of h = xd.w1^T + b1, xd[row[j][i]] = x[i], for the few-row kernel to do as it reads its tokens (layer.hip)
+// The dispatch in front of h = xd.w1^T + b1, xd[row[j][i]] = x[i], for the product to do as it reads its rows (layer.hip): the few-row
+// kernel turns row round by itself, the tiles take the routing's list.
 struct DispatchHead {
     const int32_t *row;     // [k][S] row of a pair (-1: dropped)
+    const int32_t *token_of;    // token of a row (tiles; null: few-row kernel)
     int S, k;
 };
 constexpr int HEAD_PAIRS = 512;     // most pairs, one per thread of a block
@@ -174,6 +176,7 @@ struct GemmArgs {
     CombineTail *tail;      // host side only: see CombineTail (null: none)
     const int32_t *pair_row;    // A is the tokens and not their dispatched rows: [pairs], pair p is token p % tokens (null: it is the rows)
     int pairs, tokens;
+    const int32_t *token_of;    // A is the tokens and its row r token token_of[r] (null: A is the rows); EPI_BIAS_GELU by tiles
     int m_fastest;          // row-ragged products, 256-wide kernel: number an expert's tiles m-tile first (see gemm256.hip)
 };
 
@@ -204,6 +207,7 @@ int gemm_skinny_ksplit(int E, int max_rows, int est_rows, int N, int K, int dtyp
 // fp32 tiles with direct-to-LDS loads (gemm_f32.hip); -100 as above.
 int launch_gemm_f32(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
 int gemm_f32_ksplit(int E, int est_rows, int N, int K);
+bool gemm_f32_takes(int N, int K);      // the widths of a row-ragged product
 bool gemm_f32_sums_operand(const GemmArgs &g);
 
 }  // namespace mole

@@ -83,15 +83,22 @@ template <int TMB, int WM, int WN, bool M_KS, int TMC> struct Stage {
 // operand from the tile's first row on, k_left = k-rows from the stage's first k on (only the last stage
 // of a ragged contraction has fewer than 32).
 __device__ __forceinline__ int swz16(int row) { return ((row >> 3) & 1) | (((row >> 1) ^ (row >> 2)) & 2); }
+// src: the operand's rows are those of a matrix of n_src rows that src names, and the base is that matrix (null: they lie there in order).
 template <int ROWS, int NW> struct OffKC {
     uint32_t off[ROWS / (16 * NW)];
-    __device__ __forceinline__ void init(long ld, int r_left, int k_left) {
+    __device__ __forceinline__ void init(long ld, int r_left, int k_left, const int32_t *src, int n_src) {
+        uint32_t at[ROWS / (16 * NW)];
+#pragma unroll
+        for (int i = 0; i < ROWS / (16 * NW); ++i) {
+            at[i] = (uint32_t)min((NW * i + (int)(threadIdx.x >> 6)) * 16 + ((int)threadIdx.x >> 2 & 15), r_left - 1);
+            if (src != nullptr) at[i] = min((uint32_t)src[at[i]], (uint32_t)n_src - 1u);
+        }
         const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
         for (int i = 0; i < ROWS / (16 * NW); ++i) {
             const int row = (NW * i + w) * 16 + (lane >> 2);
             const int c = min((lane & 3) ^ swz16(row), (k_left >> 3) - 1);     // (k_left is a multiple of 8)
-            off[i] = (uint32_t)(min(row, r_left - 1) * ld * 2 + c * 16);
+            off[i] = (uint32_t)(at[i] * ld * 2 + c * 16);
         }
     }
 };
@@ -101,7 +108,7 @@ template <int ROWS, int NW> struct OffKC {
 __device__ __forceinline__ int swz_ks(int k) { return ((k & 3) << 1) | ((k >> 3) & 1); }
 template <int ROWS, int NW> struct OffKS {
     uint32_t off[ROWS / (16 * NW)];
-    __device__ __forceinline__ void init(long ld, int r_left, int k_left) {
+    __device__ __forceinline__ void init(long ld, int r_left, int k_left, const int32_t *, int) {
         constexpr int SPR = ROWS / 8;          // 16-byte slots per k-row
         constexpr int KPL = 64 / SPR;          // k-rows per wave load
         const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -239,15 +246,15 @@ template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC, bool 
     int nk;
     bool ragged_k;
     __device__ __forceinline__ void init(const bf16_t *Mp, long ldm, int m0, int m_ext, const bf16_t *Np, long ldn, int n0,
-                                         int n_ext, int k_ext, char *smem, int wave) {
-        om.init(ldm, m_ext - m0, Q_BK);
-        on.init(ldn, n_ext - n0, Q_BK);
+                                         int n_ext, int k_ext, char *smem, int wave, const int32_t *src, int n_src) {
+        om.init(ldm, m_ext - m0, Q_BK, src, n_src);
+        on.init(ldn, n_ext - n0, Q_BK, nullptr, 0);
         ragged_k = KT && (k_ext & (Q_BK - 1));
         if constexpr (KT) {   // last stage of a ragged contraction: k past the end is clamped to the last k-row / 16-byte piece
-            cm.init(ldm, m_ext - m0, ragged_k ? (k_ext & (Q_BK - 1)) : Q_BK);
-            cn.init(ldn, n_ext - n0, ragged_k ? (k_ext & (Q_BK - 1)) : Q_BK);
+            cm.init(ldm, m_ext - m0, ragged_k ? (k_ext & (Q_BK - 1)) : Q_BK, src, n_src);
+            cn.init(ldn, n_ext - n0, ragged_k ? (k_ext & (Q_BK - 1)) : Q_BK, nullptr, 0);
         }
-        bm = uniform_ptr(M_KS ? Mp + m0 : Mp + (long)m0 * ldm);
+        bm = uniform_ptr(src != nullptr ? Mp : M_KS ? Mp + m0 : Mp + (long)m0 * ldm);
         bn = uniform_ptr(N_KS ? Np + n0 : Np + (long)n0 * ldn);
         step_m = M_KS ? ldm * (Q_BK * 2) : Q_BK * 2;
         step_n = N_KS ? ldn * (Q_BK * 2) : Q_BK * 2;
@@ -318,7 +325,7 @@ template <int B, int L, int X> __device__ __forceinline__ void wait_stages_behin
 template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC, int TMCW, int SUM, bool ONCE = false, int PART = 0, bool BIAS = false>
 __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, int m_ext, const bf16_t *Np, long ldn,
                                           int n0, int n_ext, int k_ext, char *smem, int wave, int wm, int wn,
-                                          f32x4 (&acc)[2 * Tile<TMB, WM, WN>::TMW][4], f32x4 (&sums)[2], const uint2 (&bias_raw)[4]) {
+                                          f32x4 (&acc)[2 * Tile<TMB, WM, WN>::TMW][4], f32x4 (&sums)[2], const uint2 (&bias_raw)[4], const int32_t *src, int n_src) {
     typedef Tile<TMB, WM, WN> TL;
     typedef Stage<TMB, WM, WN, M_KS, TMC> SG;
     constexpr int AHEAD = SG::NSTAGE - 1, NP = 4;
@@ -327,7 +334,7 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
     const int nk = __builtin_amdgcn_readfirstlane((k_ext + Q_BK - 1) / Q_BK);
     if (nk == 0) return;
     FD fd;
-    fd.init(Mp, ldm, m0, m_ext, Np, ldn, n0, n_ext, k_ext, smem, wave);
+    fd.init(Mp, ldm, m0, m_ext, Np, ldn, n0, n_ext, k_ext, smem, wave, src, n_src);
     auto fix_tail = [&](int s, int buf) __attribute__((always_inline)) {   // ragged contraction: zero what lies past it in the last stage
         if (KT && s == nk - 1 && (k_ext & (Q_BK - 1))) {
             char *b = smem + buf * SG::BYTES;
@@ -912,7 +919,11 @@ __device__ __forceinline__ void gemm256_block(const GemmArgs &g, const int block
             return;
         }
     }
-    const bf16_t *Mp = (const bf16_t *)g.A + row0 * g.lda;
+    // h = xd.w1^T + b1 may read its rows where the tokens lie (a forward pass that nobody asks for xd)
+    constexpr bool MAY_GATHER = EPI == EPI_BIAS_GELU;
+    const int32_t *src = nullptr;
+    if constexpr (MAY_GATHER) { if (g.token_of != nullptr) src = g.token_of + row0 + m0; }
+    const bf16_t *Mp = (const bf16_t *)g.A + (src != nullptr ? 0 : row0 * g.lda);
     if constexpr (WG && EPI == EPI_WGRAD) {
         // Up to FEW_ROWS rows: every wave by itself, 128 columns by 64 rows of the tile (128-wide tiles: by 32); see wgrad_few.h.
         if (k_ext <= FEW_ROWS) {
@@ -969,7 +980,7 @@ __device__ __forceinline__ void gemm256_block(const GemmArgs &g, const int block
     f32x4 sums[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #define MOLE_RUN_TILE_AS(C, SUM, ONCE)                                                                                         \
     {                                                                                                                     \
-        main_loop<TMB, WM, WN, M_KS, N_KS, KT, WM *(C), (C), SUM, ONCE, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw); \
+        main_loop<TMB, WM, WN, M_KS, N_KS, KT, WM *(C), (C), SUM, ONCE, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw, src, g.tokens); \
         if constexpr (SUM != 0) store_sums<SUM, (C)>(g, sums, e, m0, n0, m_ext, wm, wn, lane);                            \
         epilogue<TMB, WM, WN, WG, EPI, (C), KT && !WG>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, split_k);      \
     }

@@ -57,17 +57,26 @@ template <int BM, int BN, int NSTAGE> struct FTile {
 // element at the stage's first k.  Wave w's load i fills LDS bytes [(4 i + w) 1024, +1024) of the tile.  Rows
 // (k-rows) past the operand's end are clamped to the last valid one: what lands for them is finite data that only
 // reaches results which are not stored - except along a ragged contraction, whose tail is zeroed in LDS.
+// src: the operand's rows are those of a matrix of n_src rows that src names, and the base is that matrix (null: they lie there in order).
 template <int ROWS, bool KS> struct FOff {
     static constexpr int NL = ROWS / 64;
     uint32_t off[NL];
-    __device__ __forceinline__ void init(long ld, int r_left, int k_left) {
+    __device__ __forceinline__ void init(long ld, int r_left, int k_left, const int32_t *src = nullptr, int n_src = 0) {
         const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+        uint32_t at[NL];
+        if constexpr (!KS) {
+#pragma unroll
+            for (int i = 0; i < NL; ++i) {
+                at[i] = (uint32_t)min((4 * i + w) * 16 + (lane >> 2), r_left - 1);
+                if (src != nullptr) at[i] = min((uint32_t)src[at[i]], (uint32_t)n_src - 1u);
+            }
+        }
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
             if constexpr (!KS) {
                 const int row = (4 * i + w) * 16 + (lane >> 2);
                 const int c = (lane & 3) ^ swz4(row);
-                off[i] = (uint32_t)(min(row, r_left - 1) * ld * 4 + c * 16);
+                off[i] = (uint32_t)(at[i] * ld * 4 + c * 16);
             } else {
                 constexpr int SPR = ROWS / 4, KPL = 64 / SPR;      // 16-byte pieces per k-row, k-rows per load
                 const int kr = (4 * i + w) * KPL + lane / SPR;
@@ -165,7 +174,7 @@ __device__ constexpr int SPLIT_M[6] = {0, 2, 1, 0, 1, 0}, SPLIT_N[6] = {2, 0, 1,
 template <int BM, int BN, int NSTAGE, bool M_KS, bool N_KS, bool WG, bool SPLIT>
 __device__ __forceinline__ bool f32_loop(const GemmArgs &g, const float *Mp, const float *Np, int m0, int n0, int m_ext, int k_ext, char *smem,
                                          int wave, int wm, int wn, f32x16 (&acc)[FTile<BM, BN, NSTAGE>::TMW][FTile<BM, BN, NSTAGE>::TNW], int sum_side,
-                                         float (&psum)[4][2]) {
+                                         float (&psum)[4][2], const int32_t *src) {
     typedef FTile<BM, BN, NSTAGE> TL;
     constexpr int F_NSTAGE = NSTAGE;
     constexpr int TMW = TL::TMW, TNW = TL::TNW, L = TL::L;
@@ -174,10 +183,10 @@ __device__ __forceinline__ bool f32_loop(const GemmArgs &g, const float *Mp, con
     const int kl = k_ext - (nk - 1) * F_BK;     // k-rows of the last stage (a row-ragged product's K is whole stages)
     FOff<BM, M_KS> om, cm;
     FOff<BN, N_KS> on, cn;
-    om.init(g.lda, m_ext - m0, F_BK);
+    om.init(g.lda, m_ext - m0, F_BK, src, g.tokens);
     on.init(g.ldb, g.N - n0, F_BK);
     if constexpr (WG) { cm.init(g.lda, m_ext - m0, kl); cn.init(g.ldb, g.N - n0, kl); }
-    const char *bm = uniform_ptr(M_KS ? Mp + m0 : Mp + (long)m0 * g.lda);
+    const char *bm = uniform_ptr(src != nullptr ? Mp : M_KS ? Mp + m0 : Mp + (long)m0 * g.lda);
     const char *bn = uniform_ptr(N_KS ? Np + n0 : Np + (long)n0 * g.ldb);
     const long step_m = M_KS ? g.lda * (F_BK * 4) : F_BK * 4;
     const long step_n = N_KS ? g.ldb * (F_BK * 4) : F_BK * 4;
@@ -461,7 +470,10 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
     k_ext = __builtin_amdgcn_readfirstlane(k_ext);
     row0 = ((long)__builtin_amdgcn_readfirstlane((int)(row0 >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)row0);
     const int m0 = mt * BM, n0 = nt * BN;
-    const float *Mp = (const float *)g.A + row0 * g.lda;
+    // h = xd.w1^T + b1 may read its rows where the tokens lie (a forward pass that nobody asks for xd)
+    const int32_t *src = nullptr;
+    if constexpr (EPI == EPI_BIAS_GELU) { if (g.token_of != nullptr) src = g.token_of + row0 + m0; }
+    const float *Mp = (const float *)g.A + (src != nullptr ? 0 : row0 * g.lda);
     const float *Np = WG ? (const float *)g.B + row0 * g.ldb : (const float *)g.B + (long)e * g.strideB;
     if constexpr (EPI == EPI_PART) {           // this block's stages of the contraction (which is whole stages)
         split_k = __builtin_amdgcn_readfirstlane(split_k);
@@ -504,7 +516,7 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
     const bool one_row = PARTS && WG && k_ext <= 1;
     bool redo = one_row;
     if (!one_row) {
-        const bool inexact = f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, PARTS>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, sum_side, psum);
+        const bool inexact = f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, PARTS>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, sum_side, psum, src);
         if constexpr (PARTS) {
             // An infinity, a NaN or a value within half a unit of bf16 of the overflow limit has no finite parts: its products with
             // a part that is zero are NaN.  A tile with any result that is not finite is computed again with fp32 operands.
@@ -532,7 +544,7 @@ __global__ __launch_bounds__(F_THREADS, BPC) void gemm_f32_kernel(const GemmArgs
                 for (int j = 0; j < TNW; ++j)
 #pragma unroll
                     for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
-            f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, false>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, one_row ? sum_side : 0, psum);
+            f32_loop<BM, BN, NSTAGE, M_KS, N_KS, WG, false>(g, Mp, Np, m0, n0, m_ext, k_ext, smem, wave, wm, wn, acc, one_row ? sum_side : 0, psum, src);
         }
     }
 
@@ -733,12 +745,14 @@ int gemm_f32_ksplit(int E, int est_rows, int N, int K) {
     return best;
 }
 
+bool gemm_f32_takes(int N, int K) { return N >= 4 && N % 4 == 0 && K > 0 && K % F_BK == 0; }
+
 int launch_gemm_f32(const GemmArgs &g0, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid) {
     GemmArgs g = g0;
     g.ksplit = 1;
     // what the direct-to-LDS path relies on: 16-byte rows, whole stages of K for row-ragged products
     if (g.lda % 4 || g.ldb % 4 || g.ldc % 4 || g.N % 4 || g.N < 4) return -100;
-    if (!wg && (a_ks || g.K <= 0 || g.K % F_BK)) return -100;
+    if (!wg && (a_ks || !gemm_f32_takes(g.N, g.K))) return -100;
     if (wg && (!a_ks || !b_ks || g.M % 4 || g.M < 4)) return -100;
     if (wg) return dispatch_f32<128, 128, 4, 2, true>(g, b_ks, wg, epi, max_rows, st, kid);
     if (b_ks && g.offsets != nullptr && ws != nullptr) {

@@ -620,7 +620,7 @@ static int launch_ks(const GemmArgs &g, int epi, int groups, int max_rows, hipSt
 
 static bool plan_launch(const GemmArgs &g, int dtype, bool b_ks, int max_rows, void *ws, size_t ws_bytes, SkinnyPlan &p) {
     const int epc = dtype == MOLE_BF16 ? 8 : 4;
-    if (max_rows <= 0 || g.offsets == nullptr || g.kept == nullptr) return false;
+    if (max_rows <= 0 || g.offsets == nullptr || g.kept == nullptr || g.token_of != nullptr) return false;
     const bool split = !b_ks || tiles_split(dtype, g.E, max_rows, g.est_rows, g.N, g.K, ws != nullptr ? ws_bytes : 0);
     if (!skinny_plan(dtype, b_ks, g.E, g.est_rows, g.N, g.K, split, p)) return false;
     return !(g.K % epc || g.N % epc || g.lda % epc || g.ldb % epc || g.ldc % epc || g.strideB % epc);

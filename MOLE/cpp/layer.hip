@@ -78,15 +78,27 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
         set_error("mole_layer_fwd: workspace of %zu bytes, need %zu", L->workspace_bytes, need);
         return MOLE_E_WORKSPACE;
     }
-    if (int rc = mole_gate_route(L->x, L->dtype, L->wg, L->logit_bias, L->S, L->E, L->M, L->k, L->capacity_factor, L->normalize_gate, 1,
-                                 L->layout, L->scores, L->idx, L->loc, L->gates, L->row, L->counts, L->kept_rows, L->offsets,
-                                 L->capacity, L->l_aux, L->workspace, L->workspace_bytes, stream)) return rc;
     const bool scratch = L->forward_only == 2;       // xd and out are read by nobody after this pass
-    // Few tokens whose first product goes to the few-row kernel: it reads the tokens where they lie, if nobody wants xd.
-    // (what the dispatch would refuse is left to it)
-    const DispatchHead head{L->row, L->S, L->k};
-    const bool head_ok = scratch && L->k >= 1 && L->k <= 16 && (long)L->S * L->k <= HEAD_PAIRS && ((uintptr_t)L->x & 15) == 0 &&
-                         ffn_fwd_takes_tokens(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
+    // Where nobody wants xd the first product reads the tokens where they lie: the few-row kernel, which turns the pairs' rows round by
+    // itself, up to HEAD_PAIRS; the tiles from a list that the routing leaves in xd's place.  A tile's start then waits for memory once
+    // more, about 0.5 us; a dispatch is a launch, writes R M elements and has them read from memory instead of the tokens from the
+    // caches.  Forward passes, dispatched / from the list, us: 61 tokens, 16 experts top-1, 1024 -> 4096, 63.5 / 61.8; 3001, 16 top-2, 1024 ->
+    // 4096, 169.5 / 166.5; 4000, 8 top-2, 4096 -> 2048, 341 / 328; 32768, 64 top-8, 2048 -> 1024, 2640 / 2382; 30000, 64 top-8, 1000 -> 1000, whose
+    // rows share their 128-byte lines, 1712 / 1446; fp32 777, 8 top-2, 520 -> 2048, 102.6 / 100.5; fp32 10000, 16 top-2, 1024 -> 1024, 661 / 641.
+    // Nothing measured lost.  (Up to HEAD_PAIRS pairs of narrow tokens are dispatched as ever, and the kernels' timings show it: 400 tokens, 64
+    // experts, 136 -> 520, 35.7 / 33.8.  What the dispatch would refuse, and tokens that 32-bit offsets do not reach, are left to it.)
+    FwdTokens takes = TOKENS_NO;
+    if (scratch && L->k >= 1 && L->k <= 16 && ((uintptr_t)L->x & 15) == 0)
+        takes = ffn_fwd_takes_tokens(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
+    if (takes == TOKENS_PAIRS && (long)L->S * L->k > HEAD_PAIRS) takes = TOKENS_NO;
+    if (takes == TOKENS_LIST && ((size_t)L->S * L->M * (L->dtype == MOLE_BF16 ? 2 : 4) >= (size_t)1 << 31 ||
+                                 (L->M < 256 && (long)L->S * L->k <= HEAD_PAIRS))) takes = TOKENS_NO;
+    int32_t *const token_of = takes == TOKENS_LIST ? (int32_t *)L->xd : nullptr;
+    if (int rc = gate_route(L->x, L->dtype, L->wg, L->logit_bias, L->S, L->E, L->M, L->k, L->capacity_factor, L->normalize_gate, 1,
+                            L->layout, L->scores, L->idx, L->loc, L->gates, L->row, L->counts, L->kept_rows, L->offsets,
+                            L->capacity, L->l_aux, token_of, L->workspace, L->workspace_bytes, stream)) return rc;
+    const DispatchHead head{L->row, token_of, L->S, L->k};
+    const bool head_ok = takes != TOKENS_NO;
     if (!head_ok)
         if (int rc = mole_dispatch_fwd(L->x, L->dtype, L->row, L->S, L->M, L->k, L->xd, stream)) return rc;
     // (what the combine would refuse is left to it)

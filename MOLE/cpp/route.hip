@@ -215,6 +215,14 @@ struct RouteEnd {
     int32_t *counts, *kept_rows, *offsets, *capacity;
     float *l_aux;
     int32_t *idx, *loc, *row;          // loc: in-block ranks in, locations out
+    int32_t *token_of;                 // token of every row that is kept (null: nobody asks)
+    // location l of pair p (token i) of an expert whose rows start at off
+    __device__ __forceinline__ void place(size_t p, int i, int l, int cap, int off) const {
+        const int at = l < cap ? off + l : -1;
+        loc[p] = l;
+        row[p] = at;
+        if (token_of != nullptr && at >= 0) token_of[at] = i;
+    }
 };
 
 // Loads of the experts (s_off [E]) -> capacity, kept rows, offsets (s_off again), l_aux (s_me [E]: column sum of the scores x count of the
@@ -356,9 +364,7 @@ __global__ __launch_bounds__(FIN_THREADS) void route_finish_kernel(const RouteEn
     for (int p = tid; p < r.k * r.S; p += FIN_THREADS) {
         const int j = p / r.S, i = p % r.S;
         const int e = r.idx[p];
-        const int l = basej[j * E + e] + scan_hist[((size_t)j * E + e) * nb + i / bt] + r.loc[p];
-        r.loc[p] = l;
-        r.row[p] = l < cap ? s_off[e] + l : -1;
+        r.place(p, i, basej[j * E + e] + scan_hist[((size_t)j * E + e) * nb + i / bt] + r.loc[p], cap, s_off[e]);
     }
 }
 
@@ -435,25 +441,19 @@ __global__ __launch_bounds__(FIN_THREADS) void route_rank_kernel(const RouteEnd 
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         if (!ok[p]) continue;
-        const int l = s_cnt[(p * WAVES + w) * stride + e[p]] + rank[p];
-        r.loc[at[p]] = l;
-        r.row[at[p]] = l < cap ? s_off[e[p]] + l : -1;
+        const int c = p * WAVES + w;
+        r.place(at[p], c % per * WAVE + lane, s_cnt[c * stride + e[p]] + rank[p], cap, s_off[e[p]]);
     }
 }
 
-__global__ __launch_bounds__(256) void route_finalize_kernel(
-    const int32_t *__restrict__ idx, const int32_t *__restrict__ hist, const int32_t *__restrict__ basej,
-    const int32_t *__restrict__ offsets, const int32_t *__restrict__ capacity, int S, int E, int k, int nb,
-    int bt /* tokens per histogram block */, int32_t *__restrict__ loc /* in: in-block rank, out: location */,
-    int32_t *__restrict__ row) {
+__global__ __launch_bounds__(256) void route_finalize_kernel(const RouteEnd r, const int32_t *__restrict__ hist, const int32_t *__restrict__ basej,
+                                                             int nb, int bt /* tokens per histogram block */) {
     const size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (size_t)k * S) return;
-    const int j = (int)(p / S), i = (int)(p % S);
-    const int e = idx[p];
+    if (p >= (size_t)r.k * r.S) return;
+    const int j = (int)(p / r.S), i = (int)(p % r.S);
+    const int e = r.idx[p];
     const int b = i / bt;
-    const int l = basej[j * E + e] + hist[((size_t)j * E + e) * nb + b] + loc[p];
-    loc[p] = l;
-    row[p] = l < capacity[0] ? offsets[e] + l : -1;
+    r.place(p, i, basej[j * r.E + e] + hist[((size_t)j * r.E + e) * nb + b] + r.loc[p], r.capacity[0], r.offsets[e]);
 }
 
 // ---- the tokens' own part ------------------------------------------------------------------------------------------
@@ -639,9 +639,7 @@ __global__ __launch_bounds__(THREADS) void route_tokens_kernel(const float *__re
     for (int q = 0; q < PER_WAVE; ++q) {
         const int j = q * WAVES + w;
         if (j >= k || lane >= TOK || token >= S) break;
-        const int l = s_hist[j * E + my_e[q]] + rank[q];
-        r.loc[(size_t)j * S + token] = l;
-        r.row[(size_t)j * S + token] = l < cap ? s_off[my_e[q]] + l : -1;
+        r.place((size_t)j * S + token, token, s_hist[j * E + my_e[q]] + rank[q], cap, s_off[my_e[q]]);
     }
 }
 
@@ -685,22 +683,22 @@ static int route_after_topk(const RouteEnd &r, int32_t *hist, int32_t *basej, fl
     MOLE_LAUNCH_CHECK();
     if (r.S > 0 && !last_in_finish) {
         const size_t n = (size_t)r.k * r.S;
-        hipLaunchKernelGGL(route_finalize_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, r.idx, hist,
-                           basej, r.offsets, r.capacity, r.S, r.E, r.k, nb, bt, r.loc, r.row);
+        hipLaunchKernelGGL(route_finalize_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, r, hist, basej, nb, bt);
         MOLE_LAUNCH_CHECK();
     }
     return 0;
 }
 
 static RouteEnd route_end(int S, int E, int k, double capacity_factor, int alignment, int layout, int32_t *idx, int32_t *loc,
-                          int32_t *row, int32_t *counts, int32_t *kept_rows, int32_t *offsets, int32_t *capacity, float *l_aux) {
+                          int32_t *row, int32_t *counts, int32_t *kept_rows, int32_t *offsets, int32_t *capacity, float *l_aux,
+                          int32_t *token_of = nullptr) {
     const int spe = (S + E - 1) / E;
     const int cf_sign = capacity_factor > 0. ? 1 : (capacity_factor < 0. ? -1 : 0);
     // int(cf * spe) of the Python reference: the product is taken in double precision
     const double prod = (capacity_factor < 0. ? -capacity_factor : capacity_factor) * (double)spe;
     // (held to what leaves room for the alignment in 32 bits: a factor that overflowed them made the capacity negative)
     const int limit = (INT_MAX - alignment) / k;
-    return RouteEnd{S, E, k, cf_sign, k * (prod < (double)limit ? (int)prod : limit), alignment, layout, counts, kept_rows, offsets, capacity, l_aux, idx, loc, row};
+    return RouteEnd{S, E, k, cf_sign, k * (prod < (double)limit ? (int)prod : limit), alignment, layout, counts, kept_rows, offsets, capacity, l_aux, idx, loc, row, token_of};
 }
 
 template <int VPL, int LOGG, int THREADS, int TOK>
@@ -1438,11 +1436,12 @@ extern "C" size_t mole_gate_route_workspace_bytes(int S, int E, int k) {
                          : std::max(gate_route_fused_bytes(S, E, k), mole_gate_route_shape_workspace_bytes(MOLE_BF16, S, E, 128, k));
 }
 
-extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M,
-                               int k, double capacity_factor, int normalize_gate, int alignment, int layout, float *scores,
-                               int32_t *idx, int32_t *loc, float *gates, int32_t *row, int32_t *counts,
-                               int32_t *kept_rows, int32_t *offsets, int32_t *capacity, float *l_aux, void *workspace,
-                               size_t workspace_bytes, mole_stream_t stream) {
+namespace mole {
+// mole_gate_route, which also writes down the token of every kept row (null: it does not)
+int gate_route(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M, int k, double capacity_factor,
+               int normalize_gate, int alignment, int layout, float *scores, int32_t *idx, int32_t *loc, float *gates, int32_t *row, int32_t *counts,
+               int32_t *kept_rows, int32_t *offsets, int32_t *capacity, float *l_aux, int32_t *token_of, void *workspace, size_t workspace_bytes,
+               mole_stream_t stream) {
     MOLE_REQUIRE(dtype == MOLE_BF16 || dtype == MOLE_F32, "mole_gate_route: bad dtype %d", dtype);
     const int epc = dtype == MOLE_BF16 ? 8 : 4;
     MOLE_REQUIRE(S >= 1 && E >= 1 && E <= MOLE_MAX_EXPERTS && M >= epc && M % epc == 0,
@@ -1465,7 +1464,7 @@ extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const 
         return MOLE_E_WORKSPACE;
     }
     hipStream_t st = (hipStream_t)stream;
-    const RouteEnd r = route_end(S, E, k, capacity_factor, alignment, layout, idx, loc, row, counts, kept_rows, offsets, capacity, l_aux);
+    const RouteEnd r = route_end(S, E, k, capacity_factor, alignment, layout, idx, loc, row, counts, kept_rows, offsets, capacity, l_aux, token_of);
     const int path = gate_route_path(dtype, S, E, M);
     char *ws = (char *)workspace;
     if (path != GR_FUSED) {
@@ -1534,6 +1533,16 @@ extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const 
     MOLE_LAUNCH_CHECK();
     ScopedTiming timing(MOLE_K_ROUTE, st);
     return ranks ? route_rank(colsum, nb, r, st) : route_after_topk(r, hist, basej, colsum, colpart, nb, GATE_ROUTE_TOKENS, st);
+}
+}  // namespace mole
+
+extern "C" int mole_gate_route(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M,
+                               int k, double capacity_factor, int normalize_gate, int alignment, int layout, float *scores,
+                               int32_t *idx, int32_t *loc, float *gates, int32_t *row, int32_t *counts,
+                               int32_t *kept_rows, int32_t *offsets, int32_t *capacity, float *l_aux, void *workspace,
+                               size_t workspace_bytes, mole_stream_t stream) {
+    return gate_route(x, dtype, wg, logit_bias, S, E, M, k, capacity_factor, normalize_gate, alignment, layout, scores, idx, loc, gates, row, counts,
+                      kept_rows, offsets, capacity, l_aux, nullptr, workspace, workspace_bytes, stream);
 }
 
 extern "C" int mole_gate_fwd(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M,

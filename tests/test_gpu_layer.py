@@ -614,6 +614,28 @@ def test_forward_without_autograd_gives_the_same_bits(S, M, E, k, Fd, dtype):
         assert torch.equal(m(x, capacity_factor=0.0), y)
 
 
+# Tiles that read the tokens where they lie instead of dispatched rows (no backward pass), by every routing kernel that lists the rows' tokens:
+# one block of tokens, the ranking block, the finishing block with and without its last stage, the gate's own top-k; tiles of 64 to 256 rows,
+# one row to whole tiles an expert, contractions that end inside a stage, dropped pairs, experts without rows, numbers that fp32 parts do not hold.
+@pytest.mark.parametrize("S,M,E,k,Fd,cf,dtype,scale", [
+    (64, 1024, 4, 1, 256, 0.0, torch.bfloat16, 1.0), (64, 520, 2, 2, 264, 1.0, torch.bfloat16, 1.0),
+    (257, 256, 40, 4, 128, 0.5, torch.bfloat16, 1.0), (3001, 256, 16, 2, 2048, 0.0, torch.bfloat16, 1.0),
+    (5003, 136, 70, 2, 1032, 1.25, torch.bfloat16, 1.0), (20001, 128, 9, 3, 256, 0.0, torch.bfloat16, 1.0), (1100, 64, 600, 8, 64, 0.0, torch.bfloat16, 1.0),
+    (700, 128, 300, 8, 64, 2.0, torch.float32, 1.0), (777, 512, 8, 2, 256, 1.0, torch.float32, 1.0), (9001, 144, 8, 1, 260, 0.5, torch.float32, 1.0),
+    (777, 128, 8, 2, 256, 0.0, torch.float32, 1e-36), (4500, 256, 4, 2, 512, 0.0, torch.float32, 1e-36)])
+@pytest.mark.parametrize("padded", [False, True])
+def test_forward_from_the_tokens_gives_the_bits_of_dispatched_rows(S, M, E, k, Fd, cf, dtype, scale, padded):
+    if padded and cf == 0.0:
+        cf = 1.25
+    print(f"forward from the tokens S={S} M={M} E={E} k={k} F={Fd} cf={cf} {dtype} padded={padded} scale={scale}", flush=True)
+    m, x, _ = _build(S, M, E, k, Fd, dtype, reference_layout=padded)
+    x = (x.detach() * scale).requires_grad_(True)
+    y = m(x, capacity_factor=cf).detach()
+    with torch.no_grad():
+        for _ in range(2):
+            assert torch.equal(m(x, capacity_factor=cf), y)
+
+
 @pytest.mark.parametrize("padded", [False, True])
 def test_last_route_holds_the_loss_term(padded):
     """last_route.l_aux is the l_aux of the pass, recorded by autograd or not, whatever the memory held before; both are
