@@ -15,18 +15,27 @@ static int est_rows(const mole_layer &L) { return L.rows < L.S * L.k ? L.rows : 
 
 static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// out [ro][co] in T = in [r][c] fp32, zeros beyond
+// out [ro][co] in T = in [r][c] fp32, zeros beyond, for two matrices in one launch: `first` blocks for the first.  Bound by the launch: training
+// passes, a launch each / one for both, 300 tokens, 100 experts of 512 133.3 / 130.9 us; 3000, 128 of 1024 487.6 / 483.6.
+struct PadConvert {
+    const float *in;
+    void *out;
+    int r, c, ro, co;
+    unsigned blocks() const { return (unsigned)(((size_t)ro * co + 255) / 256); }
+};
 template <typename T>
-__global__ __launch_bounds__(256) void pad_convert_kernel(const float *__restrict__ in, int r, int c, T *__restrict__ out, int ro, int co) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= (size_t)ro * co) return;
-    const int y = (int)(i / co), x = (int)(i % co);
-    out[i] = y < r && x < c ? from_f32<T>(in[(size_t)y * c + x]) : from_f32<T>(0.f);
+__global__ __launch_bounds__(256) void pad_convert_kernel(const PadConvert a, const PadConvert b, unsigned first) {
+    const bool second = blockIdx.x >= first;
+    const PadConvert &p = second ? b : a;
+    const size_t i = (size_t)(blockIdx.x - (second ? first : 0)) * 256 + threadIdx.x;
+    if (i >= (size_t)p.ro * p.co) return;
+    const int y = (int)(i / p.co), x = (int)(i % p.co);
+    ((T *)p.out)[i] = y < p.r && x < p.c ? from_f32<T>(p.in[(size_t)y * p.c + x]) : from_f32<T>(0.f);
 }
-static int pad_convert(const float *in, int r, int c, void *out, int ro, int co, int dtype, hipStream_t st) {
-    const dim3 grid((unsigned)(((size_t)ro * co + 255) / 256));
-    if (dtype == MOLE_BF16) hipLaunchKernelGGL(pad_convert_kernel<bf16_t>, grid, dim3(256), 0, st, in, r, c, (bf16_t *)out, ro, co);
-    else hipLaunchKernelGGL(pad_convert_kernel<float>, grid, dim3(256), 0, st, in, r, c, (float *)out, ro, co);
+static int pad_convert(const PadConvert &a, const PadConvert &b, int dtype, hipStream_t st) {
+    const dim3 grid(a.blocks() + b.blocks());
+    if (dtype == MOLE_BF16) hipLaunchKernelGGL(pad_convert_kernel<bf16_t>, grid, dim3(256), 0, st, a, b, a.blocks());
+    else hipLaunchKernelGGL(pad_convert_kernel<float>, grid, dim3(256), 0, st, a, b, a.blocks());
     MOLE_LAUNCH_CHECK();
     return 0;
 }
@@ -140,8 +149,7 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
     if (p.fold) {
         if (int rc = mole_dispatch_bwd(G->gxd, L->dtype, L->row, L->S, L->M, L->k, G->dlogits, L->wg, L->E, nullptr, G->dx, stream)) return rc;
     } else {
-        if (int rc = pad_convert(G->dlogits, L->S, L->E, dl_t, L->S, p.e_pad, L->dtype, st)) return rc;
-        if (int rc = pad_convert(L->wg, L->E, L->M, wg_t, p.e_pad, L->M, L->dtype, st)) return rc;
+        if (int rc = pad_convert({G->dlogits, dl_t, L->S, L->E, L->S, p.e_pad}, {L->wg, wg_t, L->E, L->M, p.e_pad, L->M}, L->dtype, st)) return rc;
         if (int rc = mole_gemm_nn(dl_t, wg_t, L->dtype, L->S, L->M, p.e_pad, dx_add, stream)) return rc;
         if (int rc = mole_dispatch_bwd(G->gxd, L->dtype, L->row, L->S, L->M, L->k, nullptr, nullptr, 0, dx_add, G->dx, stream)) return rc;
     }
