@@ -108,6 +108,10 @@ inline void timed_launch(int id, void (*kernel)(KArgs...), dim3 grid, dim3 block
 // dWg = dlogits^T . x of a gate of any size (permute.hip); workspace of mole_gate_wgrad_workspace_bytes
 int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int M, float *dwg, void *workspace, size_t workspace_bytes, hipStream_t st);
 
+// the dispatch's backward with the gate's input gradient from bf16 operands, beyond the 32 experts of mole_dispatch_bwd's own (permute.hip)
+bool dispatch_bwd_folds(int dtype, int E);
+int dispatch_bwd_fold(const void *dxd, const int32_t *row, int S, int M, int k, const float *dlogits, const float *wg, int E, void *dx, hipStream_t st);
+
 struct CombineTail;     // gemm.h
 struct DispatchHead;
 // the FFN's entry points with the caller's estimate of the rows beside their bound (ffn_gemm.hip)

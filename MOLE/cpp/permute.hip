@@ -315,7 +315,8 @@ typedef float perm_f32x4 __attribute__((ext_vector_type(4)));
 // last wave's columns past it read the row's last ones and are not stored.  SPLIT: gradients and weights enter as the sum of
 // three bf16 numbers each (24 bits; six products, what is left out is below 2^-23 of a term), which keeps the gate's part at
 // fp32 accuracy before it is rounded to bf16: widths that are not whole 128-column pieces take it.
-template <bool E8, int TOK, bool SPLIT>
+// NH: 32s of experts (two: not split).
+template <bool E8, int TOK, bool SPLIT, int NH>
 __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_t *__restrict__ dxd,
                                                                      const int32_t *__restrict__ row, int S, int M, int k,
                                                                      const float *__restrict__ dlogits,
@@ -352,25 +353,29 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
     gather(src, src_ok, blockIdx.x * TOK);
     // A fragment of a group of 16 tokens: dlogits[tok0 + r16][8 kq .. 8 kq + 7], fetched one group ahead like the rows
     // (fetched where it is used, the product waited for it in every group: 15.0 -> 14.2 us at 16384 x 1024)
-    auto load_d = [&](float (&d)[8], int tok0) __attribute__((always_inline)) {
-        if constexpr (E8) {
-            const float4 *dp = reinterpret_cast<const float4 *>(dlogits + (size_t)min(tok0 + r16, S - 1) * E + min(8 * kq, E - 8));
-            const float4 d0 = dp[0], d1 = dp[1];
-            d[0] = d0.x; d[1] = d0.y; d[2] = d0.z; d[3] = d0.w;
-            d[4] = d1.x; d[5] = d1.y; d[6] = d1.z; d[7] = d1.w;
-        } else {
+    auto load_d = [&](float (&d)[NH][8], int tok0) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) d[i] = dlogits[(size_t)min(tok0 + r16, S - 1) * E + min(8 * kq + i, E - 1)];
+        for (int h = 0; h < NH; ++h) {
+            if constexpr (E8) {
+                const float4 *dp = reinterpret_cast<const float4 *>(dlogits + (size_t)min(tok0 + r16, S - 1) * E + min(32 * h + 8 * kq, E - 8));
+                const float4 d0 = dp[0], d1 = dp[1];
+                d[h][0] = d0.x; d[h][1] = d0.y; d[h][2] = d0.z; d[h][3] = d0.w;
+                d[h][4] = d1.x; d[h][5] = d1.y; d[h][6] = d1.z; d[h][7] = d1.w;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) d[h][i] = dlogits[(size_t)min(tok0 + r16, S - 1) * E + min(32 * h + 8 * kq + i, E - 1)];
+            }
         }
     };
-    float d[8];
+    float d[NH][8];
     load_d(d, blockIdx.x * TOK);
     // B fragments: Wg[8 kq + i][col0 + 16 cb + r16], i = 0..7, for the wave's 8 column blocks.  Fetched row by row
     // with 16-byte loads (a lane takes 4 columns of the 8 experts of one group) and turned by way of the LDS
     // buffer, [expert group][column] with a group's 8 experts as one bf16x8 entry: picking them out of global
     // memory one float at a time took longer than the rest of the kernel.  Two expert groups per pass.
     constexpr int P = SPLIT ? 3 : 1;
-    perm_bf16x8 bfrag[P][8];
+    static_assert(NH == 1 || !SPLIT, "the parts of one 32 of experts fit the registers");
+    perm_bf16x8 bfrag[P][NH][8];
     // the value rounded to bf16, of which the remainder stays behind for the next part
     auto part_of = [](float &v) __attribute__((always_inline)) {
         const bf16_t b = (bf16_t)v;
@@ -381,12 +386,16 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
         perm_bf16x8 *wt = reinterpret_cast<perm_bf16x8 *>(buf);      // [2][DM_COLS]
         const int c4 = (lane & 31) * 4, half = lane >> 5;
 #pragma unroll
-        for (int pass = 0; pass < 2; ++pass) {
+        for (int pass = 0; pass < 2 * NH; ++pass) {
             if (pass * 16 >= E) break;
             const int eg = 2 * pass + half;
+            struct __attribute__((packed, aligned(4))) AnyFloat4 { float x, y, z, w; };        // (a gate's weight may start anywhere in a buffer)
             float4 w[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) w[i] = *reinterpret_cast<const float4 *>(wg + (size_t)min(8 * eg + i, E - 1) * M + min(col0 + c4, M - 4));
+            for (int i = 0; i < 8; ++i) {
+                const AnyFloat4 v = *reinterpret_cast<const AnyFloat4 *>(wg + (size_t)min(8 * eg + i, E - 1) * M + min(col0 + c4, M - 4));
+                w[i] = make_float4(v.x, v.y, v.z, v.w);
+            }
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 if (8 * eg + i >= E) w[i] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -402,18 +411,20 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
 #pragma unroll
                 for (int c = 0; c < 4; ++c) dst[c] = t[c];
                 // the lanes whose expert group (kq) this pass staged pick up their fragments
-                if ((kq >> 1) == pass) {
+                if ((kq >> 1) == (pass & 1)) {
 #pragma unroll
-                    for (int cb = 0; cb < 8; ++cb) bfrag[p][cb] = wt[(kq & 1) * DM_COLS + 16 * cb + r16];
+                    for (int cb = 0; cb < 8; ++cb) bfrag[p][pass >> 1][cb] = wt[(kq & 1) * DM_COLS + 16 * cb + r16];
                 }
             }
         }
-        if (8 * kq >= E) {        // expert groups past the gate's size contribute nothing
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            if (32 * h + 8 * kq < E) continue;        // expert groups past the gate's size contribute nothing
             const bf16_t z = (bf16_t)0.0f;
 #pragma unroll
             for (int p = 0; p < P; ++p)
 #pragma unroll
-                for (int cb = 0; cb < 8; ++cb) bfrag[p][cb] = perm_bf16x8{z, z, z, z, z, z, z, z};
+                for (int cb = 0; cb < 8; ++cb) bfrag[p][h][cb] = perm_bf16x8{z, z, z, z, z, z, z, z};
         }
     }
 #pragma unroll
@@ -422,19 +433,23 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
         if (tok0 >= S) return;
         uint4 nxt[4];
         uint32_t nxt_ok[4];
-        float d_nxt[8];
+        float d_nxt[NH][8];
         if (g0 + 16 < TOK) {
             gather(nxt, nxt_ok, tok0 + 16);
             load_d(d_nxt, tok0 + 16);
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (tok0 + r16 >= S || 8 * kq + i >= E) d[i] = 0.f;
-        perm_bf16x8 afrag[P];
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (tok0 + r16 >= S || 32 * h + 8 * kq + i >= E) d[h][i] = 0.f;
+        perm_bf16x8 afrag[P][NH];
 #pragma unroll
         for (int p = 0; p < P; ++p)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) afrag[p][i] = part_of(d[i]);
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) afrag[p][h][i] = part_of(d[h][i]);
         // product tiles into LDS.  The gate's weights go into the first operand slot, so the four results of a lane
         // are four consecutive columns of one token (acc[r] = column 16 cb + 4 kq + r of token r16) and leave with
         // one 16-byte LDS write (a quarter wave's 16 rows are 16 banks-of-four apart: see DM_ROW)
@@ -445,10 +460,12 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
             for (int order = P - 1; order >= 0; --order)       // the smallest products first
 #pragma unroll
                 for (int p = 0; p <= order; ++p)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfrag[p][cb], afrag[order - p], acc, 0, 0, 0);
+#pragma unroll
+                    for (int h = 0; h < NH; ++h)
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfrag[p][h][cb], afrag[order - p][h], acc, 0, 0, 0);
             if constexpr (SPLIT) {
                 // the parts of an infinity are the infinity and NaN: where the leading product is not finite, it is the result
-                const perm_f32x4 lead = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfrag[0][cb], afrag[0], perm_f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                const perm_f32x4 lead = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfrag[0][0][cb], afrag[0][0], perm_f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) acc[r] = fabsf(lead[r]) < INFINITY ? acc[r] : lead[r];
             }
@@ -503,7 +520,9 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
 #pragma unroll
             for (int u = 0; u < 4; ++u) { src[u] = nxt[u]; src_ok[u] = nxt_ok[u]; }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) d[i] = d_nxt[i];
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) d[h][i] = d_nxt[h][i];
         }
     }
 }
@@ -1084,6 +1103,28 @@ extern "C" int mole_dispatch_fwd(const void *x, int dtype, const int32_t *row, i
     return 0;
 }
 
+namespace mole {
+// dx = dispatch backward + dlogits . Wg by dispatch_bwd_gate_mfma_kernel
+template <bool SPLIT, int NH>
+static int launch_fold(const void *dxd, const int32_t *row, int S, int M, int k, const float *dlogits, const float *wg, int E, void *dx, hipStream_t st) {
+    const int tok = (long)ceil_div(S, DM_TOKENS) * ceil_div(M, 8 * DM_COLS) < DM_FEW_BLOCKS ? DM_TOKENS_FEW : DM_TOKENS;
+    const dim3 grid(ceil_div(S, tok), ceil_div(M, 8 * DM_COLS));
+    const bool e8 = E % 8 == 0 && ((uintptr_t)dlogits & 15) == 0;
+#define MOLE_DM(E8, TOK) timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_mfma_kernel<E8, TOK, SPLIT, NH>, grid, dim3(512), 0, st, (const bf16_t *)dxd, row, S, M, k, dlogits, wg, E, (bf16_t *)dx)
+    if (tok == DM_TOKENS) { if (e8) MOLE_DM(true, DM_TOKENS); else MOLE_DM(false, DM_TOKENS); }
+    else { if (e8) MOLE_DM(true, DM_TOKENS_FEW); else MOLE_DM(false, DM_TOKENS_FEW); }
+#undef MOLE_DM
+    MOLE_LAUNCH_CHECK();
+    return 0;
+}
+bool dispatch_bwd_folds(int dtype, int E) { return dtype == MOLE_BF16 && E <= 64; }
+int dispatch_bwd_fold(const void *dxd, const int32_t *row, int S, int M, int k, const float *dlogits, const float *wg, int E, void *dx, hipStream_t st) {
+    if (int rc = check_perm("mole_dispatch_bwd", MOLE_BF16, S, M, k)) return rc;
+    MOLE_REQUIRE(dxd && row && dx && dlogits && aligned16(dxd) && aligned16(dx) && wg && dispatch_bwd_folds(MOLE_BF16, E), "mole_dispatch_bwd: null or misaligned pointer");
+    return launch_fold<false, 2>(dxd, row, S, M, k, dlogits, wg, E, dx, st);
+}
+}  // namespace mole
+
 extern "C" int mole_dispatch_bwd(const void *dxd, int dtype, const int32_t *row, int S, int M, int k,
                                  const float *dlogits, const float *wg, int E, const void *dx_add, void *dx,
                                  mole_stream_t stream) {
@@ -1094,19 +1135,8 @@ extern "C" int mole_dispatch_bwd(const void *dxd, int dtype, const int32_t *row,
                  "mole_dispatch_bwd: dlogits given without a valid wg/E");
     MOLE_REQUIRE(dx_add == nullptr || aligned16(dx_add), "mole_dispatch_bwd: misaligned dx_add");
     if (dlogits != nullptr && dx_add == nullptr && E <= 32 && dtype == MOLE_BF16) {
-        const int tok = (long)ceil_div(S, DM_TOKENS) * ceil_div(M, 8 * DM_COLS) < DM_FEW_BLOCKS ? DM_TOKENS_FEW : DM_TOKENS;
-        const dim3 grid(ceil_div(S, tok), ceil_div(M, 8 * DM_COLS));
-        const bool e8 = E % 8 == 0 && ((uintptr_t)dlogits & 15) == 0;
-        const bool split = M % DM_COLS != 0;
-#define MOLE_DM_(E8, TOK, SPLIT) timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_mfma_kernel<E8, TOK, SPLIT>, grid, dim3(512), 0, (hipStream_t)stream, \
-                                              (const bf16_t *)dxd, row, S, M, k, dlogits, wg, E, (bf16_t *)dx)
-#define MOLE_DM(E8, TOK) if (split) MOLE_DM_(E8, TOK, true); else MOLE_DM_(E8, TOK, false)
-        if (tok == DM_TOKENS) { if (e8) { MOLE_DM(true, DM_TOKENS); } else { MOLE_DM(false, DM_TOKENS); } }
-        else { if (e8) { MOLE_DM(true, DM_TOKENS_FEW); } else { MOLE_DM(false, DM_TOKENS_FEW); } }
-#undef MOLE_DM
-#undef MOLE_DM_
-        MOLE_LAUNCH_CHECK();
-        return 0;
+        return M % DM_COLS != 0 ? launch_fold<true, 1>(dxd, row, S, M, k, dlogits, wg, E, dx, (hipStream_t)stream)
+                                : launch_fold<false, 1>(dxd, row, S, M, k, dlogits, wg, E, dx, (hipStream_t)stream);
     }
     if (dlogits != nullptr && dx_add == nullptr && E <= 32 && M % 4 == 0) {
         const int db_tokens = (long)ceil_div(S, DB_TOKENS) * ceil_div(M, 1024) < 1024 ? DB_TOKENS_FEW : DB_TOKENS;

@@ -97,6 +97,16 @@ def test_layer_with_a_large_gate(S, M, E, k, Fd, cf, dtype):
     _run_and_compare(m, x, ref, k, cf, dtype, aux_w=0.5)
 
 
+# 33 to 64 experts in bf16: the gate's input gradient inside the dispatch's backward, 32 experts and a rest.  Blocks of 16 and of 64 tokens, both ends of
+# the experts, gradients that lie on 16 bytes and not, rows that end inside a wave's columns and a block's, dropped pairs.
+@pytest.mark.parametrize("S,M,E,k,Fd,cf", [(1, 8, 64, 2, 8, 0.0), (65, 136, 33, 3, 16, 0.0), (515, 1032, 48, 8, 16, 0.5), (100, 128, 63, 1, 16, 1.0),
+                                           (6150, 1160, 64, 2, 16, 0.0), (12353, 72, 57, 4, 16, 1.25)])
+def test_layer_with_a_gate_of_up_to_64(S, M, E, k, Fd, cf):
+    print(f"layer with a gate of up to 64 S={S} M={M} E={E} k={k} F={Fd}", flush=True)
+    m, x, ref = _build(S, M, E, k, Fd, torch.bfloat16)
+    _run_and_compare(m, x, ref, k, cf, torch.bfloat16, aux_w=0.5)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("reference_layout", [False, True])
 @pytest.mark.parametrize("S,M,E,k,Fd,cf", [(300, 64, 4, 2, 128, 1.0), (1000, 128, 8, 1, 256, 1.25), (513, 64, 16, 4, 128, 0.0)])
@@ -614,7 +624,7 @@ def test_forward_without_autograd_gives_the_same_bits(S, M, E, k, Fd, dtype):
         assert torch.equal(m(x, capacity_factor=0.0), y)
 
 
-# Tiles that read the tokens where they lie instead of dispatched rows (no backward pass), by every routing kernel that lists the rows' tokens:
+# Tiles that read the tokens where they lie instead of dispatched rows, by every routing kernel that lists the rows' tokens:
 # one block of tokens, the ranking block, the finishing block with and without its last stage, the gate's own top-k; tiles of 64 to 256 rows,
 # one row to whole tiles an expert, contractions that end inside a stage, dropped pairs, experts without rows, numbers that fp32 parts do not hold.
 @pytest.mark.parametrize("S,M,E,k,Fd,cf,dtype,scale", [
@@ -625,6 +635,7 @@ def test_forward_without_autograd_gives_the_same_bits(S, M, E, k, Fd, dtype):
     (777, 128, 8, 2, 256, 0.0, torch.float32, 1e-36), (4500, 256, 4, 2, 512, 0.0, torch.float32, 1e-36)])
 @pytest.mark.parametrize("padded", [False, True])
 def test_forward_from_the_tokens_gives_the_bits_of_dispatched_rows(S, M, E, k, Fd, cf, dtype, scale, padded):
+    from mole_amd import hip_ops as H
     if padded and cf == 0.0:
         cf = 1.25
     print(f"forward from the tokens S={S} M={M} E={E} k={k} F={Fd} cf={cf} {dtype} padded={padded} scale={scale}", flush=True)
@@ -634,6 +645,15 @@ def test_forward_from_the_tokens_gives_the_bits_of_dispatched_rows(S, M, E, k, F
     with torch.no_grad():
         for _ in range(2):
             assert torch.equal(m(x, capacity_factor=cf), y)
+        r = m.last_route
+        xd = H.dispatch_fwd(x, r.row, int(r.offsets[-1]))
+        out, _, _ = H.ffn_fwd(xd, r.offsets, r.kept_rows, m.FC1_W_GPU.all_tensors, m.FC1_B_GPU.all_tensors,
+                              m.FC2_W_GPU.all_tensors, m.FC2_B_GPU.all_tensors)
+        want = H.combine_fwd(out, r.row, r.gates)
+    if cf == 0.0:
+        assert torch.equal(y, want)
+    else:                                  # (fewer rows than S k: the layer may split the contraction otherwise)
+        assert rel_err(y.float().cpu(), want.float().cpu()) < tol(dtype)
 
 
 @pytest.mark.parametrize("padded", [False, True])
