@@ -42,7 +42,7 @@ static int pad_convert(const PadConvert &a, const PadConvert &b, int dtype, hipS
 
 // Scratch of the backward's gate part, and which way its input gradient goes.
 struct GateBwdPlan {
-    bool fold;           // dlogits . Wg inside mole_dispatch_bwd (up to 32 experts)
+    bool fold, fold_wide;    // dlogits . Wg inside mole_dispatch_bwd (up to 32 experts) / inside dispatch_bwd_fold
     int e_pad;           // experts rounded up to the tiles' granule
     size_t dgates, dl_t, wg_t, dx_add, wgrad, total;     // bytes
 };
@@ -51,11 +51,13 @@ static GateBwdPlan gate_bwd_plan(const mole_layer &L) {
     const size_t es = L.dtype == MOLE_BF16 ? 2 : 4;
     const int epc = L.dtype == MOLE_BF16 ? 8 : 4;
     p.fold = L.E <= 32;
+    p.fold_wide = !p.fold && dispatch_bwd_folds(L.dtype, L.E);
+    const bool product = !p.fold && !p.fold_wide;
     p.e_pad = (L.E + epc - 1) / epc * epc;
     p.dgates = L.E > 256 ? up256((size_t)L.k * L.S * 4) : 0;
-    p.dl_t = p.fold ? 0 : up256((size_t)L.S * p.e_pad * es);
-    p.wg_t = p.fold ? 0 : up256((size_t)p.e_pad * L.M * es);
-    p.dx_add = p.fold ? 0 : up256((size_t)L.S * L.M * es);
+    p.dl_t = !product ? 0 : up256((size_t)L.S * p.e_pad * es);
+    p.wg_t = !product ? 0 : up256((size_t)p.e_pad * L.M * es);
+    p.dx_add = !product ? 0 : up256((size_t)L.S * L.M * es);
     p.wgrad = up256(mole_gate_wgrad_workspace_bytes(L.S, L.E, L.M));
     p.total = p.dgates + p.dl_t + p.wg_t + p.dx_add + p.wgrad;
     return p;
@@ -148,7 +150,7 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
     char *dl_t = ws + p.dgates, *wg_t = dl_t + p.dl_t, *dx_add = wg_t + p.wg_t, *wgrad = dx_add + p.dx_add;
     if (p.fold) {
         if (int rc = mole_dispatch_bwd(G->gxd, L->dtype, L->row, L->S, L->M, L->k, G->dlogits, L->wg, L->E, nullptr, G->dx, stream)) return rc;
-    } else if (dispatch_bwd_folds(L->dtype, L->E)) {
+    } else if (p.fold_wide) {
         // 33 to 64 experts: the operands in bf16 like those of the product below, its sum in fp32 and without a way through memory, three
         // launches less.  Training passes, by the product / folded, us: 8 tokens, 64 experts of 1024 top-2, 123.5 / 117.8; 300, 40 of 1024, 175.1 /
         // 166.9; 3000, 64 of 1024, 319.5 / 309.8; 8192, 64 of 2048, 857 / 838; 30000, 64 of 1000 top-8, 4838 / 4813; 2000, 64 of 4096, 924.8 / 916.
