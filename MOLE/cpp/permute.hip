@@ -325,8 +325,8 @@ typedef float perm_f32x4 __attribute__((ext_vector_type(4)));
 // last wave's columns past it read the row's last ones and are not stored.  SPLIT: gradients and weights enter as the sum of
 // three bf16 numbers each (24 bits; six products, what is left out is below 2^-23 of a term), which keeps the gate's part at
 // fp32 accuracy before it is rounded to bf16: widths that are not whole 128-column pieces take it.
-// NH: 32s of experts (two: not split).
-template <bool E8, int TOK, bool SPLIT, int NH>
+// NH: 32s of experts (two: not split).  MORE: several choices.
+template <bool E8, int TOK, bool SPLIT, int NH, bool MORE>
 __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_t *__restrict__ dxd,
                                                                      const int32_t *__restrict__ row, int S, int M, int k,
                                                                      const float *__restrict__ dlogits,
@@ -456,7 +456,7 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
             gather(nxt, nxt_ok, tok0 + 16);
             load_d(d_nxt, tok0 + 16);
         }
-        if (k > 1) rows_of(1);
+        if constexpr (MORE) rows_of(1);
 #pragma unroll
         for (int h = 0; h < NH; ++h)
 #pragma unroll
@@ -507,7 +507,7 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
 #pragma unroll
             for (int q = 0; q < 8; ++q) acc[u][q] += f[q];
         }
-        for (int j = 1; j < k; ++j) {          // a choice's four gathers are in flight together
+        for (int j = 1; MORE && j < k; ++j) {          // a choice's four gathers are in flight together
             uint4 more[4];
             uint32_t ok[4];
 #pragma unroll
@@ -1127,10 +1127,12 @@ static int launch_fold(const void *dxd, const int32_t *row, int S, int M, int k,
     const int tok = (long)ceil_div(S, DM_TOKENS) * ceil_div(M, 8 * DM_COLS) < DM_FEW_BLOCKS ? DM_TOKENS_FEW : DM_TOKENS;
     const dim3 grid(ceil_div(S, tok), ceil_div(M, 8 * DM_COLS));
     const bool e8 = E % 8 == 0 && ((uintptr_t)dlogits & 15) == 0;
-#define MOLE_DM(E8, TOK) timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_mfma_kernel<E8, TOK, SPLIT, NH>, grid, dim3(512), 0, st, (const bf16_t *)dxd, row, S, M, k, dlogits, wg, E, (bf16_t *)dx)
+#define MOLE_DM_(E8, TOK, MORE) timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_mfma_kernel<E8, TOK, SPLIT, NH, MORE>, grid, dim3(512), 0, st, (const bf16_t *)dxd, row, S, M, k, dlogits, wg, E, (bf16_t *)dx)
+#define MOLE_DM(E8, TOK) do { if (k > 1) MOLE_DM_(E8, TOK, true); else MOLE_DM_(E8, TOK, false); } while (0)
     if (tok == DM_TOKENS) { if (e8) MOLE_DM(true, DM_TOKENS); else MOLE_DM(false, DM_TOKENS); }
     else { if (e8) MOLE_DM(true, DM_TOKENS_FEW); else MOLE_DM(false, DM_TOKENS_FEW); }
 #undef MOLE_DM
+#undef MOLE_DM_
     MOLE_LAUNCH_CHECK();
     return 0;
 }
