@@ -304,7 +304,7 @@ __global__ __launch_bounds__(256) void dispatch_bwd_gate_kernel(const float *__r
 }
 
 // The same for bf16 tokens with the gate product on the matrix cores.  dlogits . Wg is a [tokens x E] by
-// [E x M] product with E <= 32: one v_mfma_f32_16x16x32_bf16 per 16 tokens x 16 columns, both operands rounded
+// [E x M] product with E <= 32 (NH 2: 64): one v_mfma_f32_16x16x32_bf16 (two) per 16 tokens x 16 columns, both operands rounded
 // to bf16 (the sum is rounded to bf16 on the way out anyway).  The fp32 kernel above spends 2 E VALU
 // instructions per pair of output elements on it, which is what bounds it; here the VALU work is the
 // unpack / add / pack of a copy.
