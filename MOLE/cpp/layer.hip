@@ -7,11 +7,22 @@
 // longer than the kernels (61 tokens, 16 experts of 1024 -> 4096: 95 us of host time for 75 us of kernels).
 #include "gemm.h"
 
+#include <algorithm>
+
 namespace mole {
 
 // rows the experts hold in all likelihood: every pair, or the capacity's bound where that is less (the padded layout's
 // buffers have a row for every slot)
 static int est_rows(const mole_layer &L) { return L.rows < L.S * L.k ? L.rows : L.S * L.k; }
+
+// Whether the first product reads the tokens through the list although their rows are written for later: where the rows of several choices are
+// more than the last-level cache holds and the tokens are well below it.  Training passes, from the rows / from the tokens, us: 30000 tokens,
+// 64 experts top-8, 1000 -> 1000, 4720 / 4585; 32768, 16 top-8, 1024 -> 512, skewed, 3059 / 3040; 20000, 32 top-4, 2048 -> 1024, 2480 / 2459; on the
+// other side of the line, tokens of 134 and 268 MB, 32768, 256 top-8, 2048 -> 1024, 8292 / 8315; 32768, 8 top-2, 4096 -> 2048, 6434 / 6479.
+static bool tokens_beside_rows(const mole_layer &L) {
+    const size_t width = (size_t)L.M * (L.dtype == MOLE_BF16 ? 2 : 4);
+    return L.k >= 2 && est_rows(L) * width >= (size_t)256 << 20 && L.S * width <= (size_t)96 << 20;
+}
 
 static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
@@ -70,7 +81,8 @@ using namespace mole;
 extern "C" size_t mole_layer_workspace_bytes(const mole_layer *L, int backward) {
     if (L == nullptr || L->S <= 0 || L->E <= 0) return 0;
     const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
-    const size_t other = backward ? gate_bwd_plan(*L).total : mole_gate_route_shape_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
+    size_t other = backward ? gate_bwd_plan(*L).total : mole_gate_route_shape_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
+    if (!backward && tokens_beside_rows(*L)) other = up256(other) + (size_t)L->rows * 4;
     return ffn > other ? ffn : other;        // the two are never in use at the same time
 }
 
@@ -84,7 +96,8 @@ static int check_layer(const char *fn, const mole_layer *L, mole_stream_t) {
 
 extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream) {
     if (int rc = check_layer("mole_layer_fwd", L, stream)) return rc;
-    const size_t need = mole_layer_workspace_bytes(L, 0);
+    const size_t route_bytes = mole_gate_route_shape_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
+    const size_t need = std::max(route_bytes, ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F));
     if (L->workspace_bytes < need) {
         set_error("mole_layer_fwd: workspace of %zu bytes, need %zu", L->workspace_bytes, need);
         return MOLE_E_WORKSPACE;
@@ -96,21 +109,22 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
     // caches.  Forward passes, dispatched / from the list, us: 61 tokens, 16 experts top-1, 1024 -> 4096, 63.5 / 61.8; 3001, 16 top-2, 1024 ->
     // 4096, 169.5 / 166.5; 4000, 8 top-2, 4096 -> 2048, 341 / 328; 32768, 64 top-8, 2048 -> 1024, 2640 / 2382; 30000, 64 top-8, 1000 -> 1000, whose
     // rows share their 128-byte lines, 1712 / 1446; fp32 777, 8 top-2, 520 -> 2048, 102.6 / 100.5; fp32 10000, 16 top-2, 1024 -> 1024, 661 / 641.
-    // Nothing measured lost.  (Up to HEAD_PAIRS pairs of narrow tokens are dispatched as ever, and the kernels' timings show it: 400 tokens, 64
+    // Nothing measured lost.  Where tokens_beside_rows, they are read so beside a dispatch, from a list in the workspace.  (Up to HEAD_PAIRS pairs of narrow tokens are dispatched as ever, and the kernels' timings show it: 400 tokens, 64
     // experts, 136 -> 520, 35.7 / 33.8.  What the dispatch would refuse, and tokens that 32-bit offsets do not reach, are left to it.)
     FwdTokens takes = TOKENS_NO;
-    if (scratch && L->k >= 1 && L->k <= 16 && ((uintptr_t)L->x & 15) == 0)
+    const bool beside = !scratch && tokens_beside_rows(*L) && L->workspace_bytes >= up256(route_bytes) + (size_t)L->rows * 4;
+    if ((scratch || beside) && L->k >= 1 && L->k <= 16 && ((uintptr_t)L->x & 15) == 0)
         takes = ffn_fwd_takes_tokens(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
-    if (takes == TOKENS_PAIRS && (long)L->S * L->k > HEAD_PAIRS) takes = TOKENS_NO;
+    if (takes == TOKENS_PAIRS && (beside || (long)L->S * L->k > HEAD_PAIRS)) takes = TOKENS_NO;
     if (takes == TOKENS_LIST && ((size_t)L->S * L->M * (L->dtype == MOLE_BF16 ? 2 : 4) >= (size_t)1 << 31 ||
                                  (L->M < 256 && (long)L->S * L->k <= HEAD_PAIRS))) takes = TOKENS_NO;
-    int32_t *const token_of = takes == TOKENS_LIST ? (int32_t *)L->xd : nullptr;
+    int32_t *const token_of = takes != TOKENS_LIST ? nullptr : beside ? (int32_t *)((char *)L->workspace + up256(route_bytes)) : (int32_t *)L->xd;
     if (int rc = gate_route(L->x, L->dtype, L->wg, L->logit_bias, L->S, L->E, L->M, L->k, L->capacity_factor, L->normalize_gate, 1,
                             L->layout, L->scores, L->idx, L->loc, L->gates, L->row, L->counts, L->kept_rows, L->offsets,
                             L->capacity, L->l_aux, token_of, L->workspace, L->workspace_bytes, stream)) return rc;
     const DispatchHead head{L->row, token_of, L->S, L->k};
     const bool head_ok = takes != TOKENS_NO;
-    if (!head_ok)
+    if (!head_ok || beside)
         if (int rc = mole_dispatch_fwd(L->x, L->dtype, L->row, L->S, L->M, L->k, L->xd, stream)) return rc;
     // (what the combine would refuse is left to it)
     CombineTail tail{L->row, L->idx, L->gates, y, L->S, L->k, !scratch, false};

@@ -632,6 +632,7 @@ def test_forward_without_autograd_gives_the_same_bits(S, M, E, k, Fd, dtype):
     (257, 256, 40, 4, 128, 0.5, torch.bfloat16, 1.0), (3001, 256, 16, 2, 2048, 0.0, torch.bfloat16, 1.0),
     (5003, 136, 70, 2, 1032, 1.25, torch.bfloat16, 1.0), (20001, 128, 9, 3, 256, 0.0, torch.bfloat16, 1.0), (1100, 64, 600, 8, 64, 0.0, torch.bfloat16, 1.0),
     (700, 128, 300, 8, 64, 2.0, torch.float32, 1.0), (777, 512, 8, 2, 256, 1.0, torch.float32, 1.0), (9001, 144, 8, 1, 260, 0.5, torch.float32, 1.0),
+    (33000, 1024, 8, 4, 16, 0.0, torch.bfloat16, 1.0), (17000, 1024, 8, 4, 16, 0.0, torch.float32, 1.0),      # (more rows than a cache holds)
     (777, 128, 8, 2, 256, 0.0, torch.float32, 1e-36), (4500, 256, 4, 2, 512, 0.0, torch.float32, 1e-36)])
 @pytest.mark.parametrize("padded", [False, True])
 def test_forward_from_the_tokens_gives_the_bits_of_dispatched_rows(S, M, E, k, Fd, cf, dtype, scale, padded):
