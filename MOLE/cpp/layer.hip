@@ -165,10 +165,10 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
     if (p.fold) {
         if (int rc = mole_dispatch_bwd(G->gxd, L->dtype, L->row, L->S, L->M, L->k, G->dlogits, L->wg, L->E, nullptr, G->dx, stream)) return rc;
     } else if (p.fold_wide) {
-        // 33 to 64 experts: the operands in bf16 like those of the product below, its sum in fp32 and without a way through memory, three
-        // launches less.  Training passes, by the product / folded, us: 8 tokens, 64 experts of 1024 top-2, 123.5 / 117.8; 300, 40 of 1024, 175.1 /
-        // 166.9; 3000, 64 of 1024, 319.5 / 309.8; 8192, 64 of 2048, 857 / 838; 30000, 64 of 1000 top-8, 4838 / 4813; 2000, 64 of 4096, 924.8 / 916.
-        // Beyond, a wave would hold more than 64 registers of weights or read them again for every 16 tokens.
+        // 33 to 64 experts: operands and result in bf16 like those of the product below, bit for bit, without the result's way through
+        // memory and three launches less.  Training passes, by the product / folded, us: 8 tokens, 64 experts of 1024 top-2, 123.5 / 117.8;
+        // 300, 40 of 1024, 175.1 / 166.9; 3000, 64 of 1024, 319.5 / 309.8; 8192, 64 of 2048, 857 / 838; 30000, 64 of 1000 top-8, 4838 / 4813;
+        // 2000, 64 of 4096, 924.8 / 916.  Beyond, a wave would hold more than 64 registers of weights or read them again for every 16 tokens.
         if (int rc = dispatch_bwd_fold(G->gxd, L->row, L->S, L->M, L->k, G->dlogits, L->wg, L->E, G->dx, st)) return rc;
     } else {
         if (int rc = pad_convert({G->dlogits, dl_t, L->S, L->E, L->S, p.e_pad}, {L->wg, wg_t, L->E, L->M, p.e_pad, L->M}, L->dtype, st)) return rc;

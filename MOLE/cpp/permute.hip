@@ -325,7 +325,8 @@ typedef float perm_f32x4 __attribute__((ext_vector_type(4)));
 // last wave's columns past it read the row's last ones and are not stored.  SPLIT: gradients and weights enter as the sum of
 // three bf16 numbers each (24 bits; six products, what is left out is below 2^-23 of a term), which keeps the gate's part at
 // fp32 accuracy before it is rounded to bf16: widths that are not whole 128-column pieces take it.
-// NH: 32s of experts (two: not split).  MORE: several choices.
+// NH: 32s of experts (two: not split; the product is rounded to bf16 and added behind the rows, bit for bit what mole_gemm_nn and
+// the dispatch backward with its result as dx_add give).  MORE: several choices.
 template <bool E8, int TOK, bool SPLIT, int NH, bool MORE>
 __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_t *__restrict__ dxd,
                                                                      const int32_t *__restrict__ row, int S, int M, int k,
@@ -494,13 +495,20 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
         float acc[4][8];
         Vec<bf16_t> v;
         float f[8];
+        auto product = [&](float (&p)[8], int u) __attribute__((always_inline)) {
+            const float *src_p = buf + (4 * u + tsel) * DM_ROW + c8;
+            const float4 p0 = *reinterpret_cast<const float4 *>(src_p), p1 = *reinterpret_cast<const float4 *>(src_p + 4);
+            p[0] = p0.x; p[1] = p0.y; p[2] = p0.z; p[3] = p0.w;
+            p[4] = p1.x; p[5] = p1.y; p[6] = p1.z; p[7] = p1.w;
+        };
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const int tl = 4 * u + tsel;
-            const float4 p0 = *reinterpret_cast<const float4 *>(buf + tl * DM_ROW + c8);
-            const float4 p1 = *reinterpret_cast<const float4 *>(buf + tl * DM_ROW + c8 + 4);
-            acc[u][0] = p0.x; acc[u][1] = p0.y; acc[u][2] = p0.z; acc[u][3] = p0.w;
-            acc[u][4] = p1.x; acc[u][5] = p1.y; acc[u][6] = p1.z; acc[u][7] = p1.w;
+            if constexpr (NH == 1) {
+                product(acc[u], u);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) acc[u][q] = 0.f;
+            }
             v.raw = src[u];
             v.mask(src_ok[u]);
             v.unpack(f);
@@ -528,6 +536,11 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int t = tok0 + 4 * u + tsel;
+            if constexpr (NH == 2) {
+                product(f, u);
+#pragma unroll
+                for (int q = 0; q < 8; ++q) acc[u][q] += (float)(bf16_t)f[q];
+            }
             if (t < S && col_ok) {
                 v.pack(acc[u]);
                 v.store(dx + (size_t)t * M + at);

@@ -1,5 +1,7 @@
 """The MoE layer module end to end (forward + backward) against the CPU oracle's layer, for
 GPU-resident and host-offloaded experts, in both execution shapes of MOLEModule."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -996,3 +998,53 @@ def test_native_forward_only_fills_xd_and_out(S, M, E, k, Fd, cf, dtype):
     for name in ("xd", "out"):
         assert torch.equal(t1[name][kept], t0[name][kept])
     assert torch.equal(t1["xd"][kept], H.dispatch_fwd(x, t1["row"], rows)[kept])
+
+
+class _Grads(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("accumulate", "gelu_bwd")] + [(n, ctypes.c_void_p) for n in "dy d_l_aux dlogits d_o t gxd g_w1 g_b1 g_w2 g_b2 dx dwg".split()]
+
+
+class _Layer(ctypes.Structure):
+    _fields_ = ([(n, ctypes.c_int32) for n in "dtype S M E k F rows layout normalize_gate forward_only".split()] + [("capacity_factor", ctypes.c_double)] +
+                [(n, ctypes.c_void_p) for n in "x wg logit_bias w1 b1 w2 b2 scores gates l_aux idx loc row counts kept_rows offsets capacity "
+                                               "xd h a out workspace".split()] + [("workspace_bytes", ctypes.c_size_t)])
+
+
+def _native_training_pass(m, x, E, k, Fd, cf, dwg=None):
+    """mole_layer_fwd and mole_layer_bwd on buffers of the test's own: every tensor of both blocks, and y."""
+    S, M = x.shape
+    dtype, rows, wg = x.dtype, S * k, m.gate[0].linear.weight.detach()
+    w = dict(zip(("w1", "b1", "w2", "b2"), (p.all_tensors for p in (m.FC1_W_GPU, m.FC1_B_GPU, m.FC2_W_GPU, m.FC2_B_GPU))))
+    i32 = lambda *n: torch.zeros(*n, dtype=torch.int32, device="cuda")
+    f32 = lambda *n: torch.zeros(*n, device="cuda")
+    act = lambda *n: torch.full(n, 7.0, dtype=dtype, device="cuda")
+    t = dict(x=x, wg=wg, **w, scores=f32(S, E), gates=f32(k, S), l_aux=f32(1), idx=i32(k, S), loc=i32(k, S), row=i32(k, S), counts=i32(k, E), kept_rows=i32(E),
+             offsets=i32(E + 1), capacity=i32(1), xd=act(rows, M), h=act(rows, Fd), a=act(rows, Fd), out=act(rows, M))
+    block = _Layer(L.dtype_code(dtype), S, M, E, k, Fd, rows, L.LAYOUT_RAGGED, 1, 0, cf, **{n: v.data_ptr() for n, v in t.items()})
+    y = act(S, M)
+    dy = (torch.randn(S, M, generator=torch.Generator().manual_seed(S)) * 1e-2).to(dtype).cuda()
+    g = dict(dy=dy, dlogits=f32(S, E), d_o=act(rows, M), t=act(rows, Fd), gxd=act(rows, M), dx=act(S, M), dwg=f32(E, M) if dwg is None else dwg,
+             **{"g_" + n: torch.empty_like(v) for n, v in w.items()})
+    grads = _Grads(0, L.GELU_BWD_TANH, **{n: v.data_ptr() for n, v in g.items()})
+    for backward in (0, 1):
+        block.workspace_bytes = L.lib().mole_layer_workspace_bytes(ctypes.byref(block), backward)
+        ws = torch.empty(max(1, block.workspace_bytes), dtype=torch.uint8, device="cuda")
+        block.workspace = ws.data_ptr()
+        if backward:
+            L.check(L.lib().mole_layer_bwd(ctypes.byref(block), ctypes.byref(grads), L.stream()), "mole_layer_bwd")
+        else:
+            L.check(L.lib().mole_layer_fwd(ctypes.byref(block), L.ptr(y), L.stream()), "mole_layer_fwd")
+        torch.cuda.synchronize()
+    return dict(t, **g, y=y)
+
+
+# Where the dispatch's backward takes the gate's input gradient in, the sum is that of the two entry points, bit for bit: the product from
+# bf16 operands, rounded to bf16, behind the rows.  One 32 of experts and a rest, whole and broken pieces of columns, dropped pairs.
+@pytest.mark.parametrize("S,M,E,k,Fd,cf", [(300, 1024, 40, 2, 64, 0.0), (3000, 1000, 64, 4, 64, 0.0), (8, 1024, 64, 1, 64, 0.0), (515, 136, 57, 8, 16, 0.5), (9000, 256, 33, 1, 16, 1.0)])
+def test_input_gradient_of_a_gate_of_up_to_64_is_that_of_its_product(S, M, E, k, Fd, cf):
+    from mole_amd import hip_ops as H
+    print(f"input gradient of a gate of up to 64 S={S} M={M} E={E} k={k} F={Fd} cf={cf}", flush=True)
+    m, x, _ = _build(S, M, E, k, Fd, torch.bfloat16, seed=S + E)
+    t = _native_training_pass(m, x, E, k, Fd, cf)
+    want = H.dispatch_bwd(t["gxd"], t["row"], t["dlogits"], t["wg"])
+    assert float(t["dlogits"].abs().max()) > 0 and torch.equal(t["dx"], want)
