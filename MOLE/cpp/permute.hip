@@ -837,7 +837,11 @@ __global__ __launch_bounds__(256) void gate_wgrad_reduce_kernel(const float *__r
         float4 r = s_acc[0][o];
 #pragma unroll
         for (int sl = 1; sl < 16; ++sl) { r.x += s_acc[sl][o].x; r.y += s_acc[sl][o].y; r.z += s_acc[sl][o].z; r.w += s_acc[sl][o].w; }
-        *reinterpret_cast<float4 *>(dwg + idx) = r;
+        if (((uintptr_t)dwg & 15) == 0) {
+            *reinterpret_cast<float4 *>(dwg + idx) = r;
+        } else {
+            dwg[idx] = r.x; dwg[idx + 1] = r.y; dwg[idx + 2] = r.z; dwg[idx + 3] = r.w;
+        }
     }
 }
 
@@ -1204,7 +1208,10 @@ namespace mole {
 // 2833.
 int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int M, float *dwg, void *workspace, size_t workspace_bytes, hipStream_t st) {
     ScopedTiming timing(MOLE_K_GATE_WGRAD, st);
-    MOLE_REQUIRE(dlogits && x && dwg && workspace && aligned16(x) && aligned16(dwg) && aligned16(workspace), "mole_gate_wgrad: null or misaligned pointer");
+    // (the layer's gates beyond mole_gate_wgrad's own may have their result at any alignment of its elements, a view into a flat buffer of
+    // gradients: it is then the reduction's to write)
+    const bool any_dwg = E > 32 && !gate_wgrad_mfma_ok(dtype, S, E, M), direct = aligned16(dwg);
+    MOLE_REQUIRE(dlogits && x && dwg && workspace && aligned16(x) && (any_dwg || aligned16(dwg)) && aligned16(workspace), "mole_gate_wgrad: null or misaligned pointer");
     if (workspace_bytes < mole_gate_wgrad_workspace_bytes(S, E, M)) {
         set_error("mole_gate_wgrad: workspace of %zu bytes, need %zu", workspace_bytes, mole_gate_wgrad_workspace_bytes(S, E, M));
         return MOLE_E_WORKSPACE;
@@ -1228,7 +1235,7 @@ int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int
     } else {
         const int tokens = gw_tokens(S, E, M);
         nb = ceil_div(S, tokens);
-        part = nb == 1 ? dwg : (float *)workspace;
+        part = nb == 1 && direct ? dwg : (float *)workspace;
         const dim3 grid(nb, ceil_div(M, 512), ceil_div(E, 32));
 #define MOLE_GW(T, EB) hipLaunchKernelGGL((gate_wgrad_partial_kernel<T, EB>), grid, dim3(256), 0, st, dlogits, (const T *)x, S, E, M, tokens, part)
         if (dtype == MOLE_BF16) {
@@ -1239,7 +1246,7 @@ int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int
 #undef MOLE_GW
     }
     MOLE_LAUNCH_CHECK();
-    if (nb == 1) return 0;
+    if (part == dwg) return 0;
     hipLaunchKernelGGL(gate_wgrad_reduce_kernel, dim3(ceil_div(E * M, 64)), dim3(256), 0, st, part, nb, E * M, dwg);
     MOLE_LAUNCH_CHECK();
     return 0;

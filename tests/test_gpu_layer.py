@@ -1048,3 +1048,18 @@ def test_input_gradient_of_a_gate_of_up_to_64_is_that_of_its_product(S, M, E, k,
     t = _native_training_pass(m, x, E, k, Fd, cf)
     want = H.dispatch_bwd(t["gxd"], t["row"], t["dlogits"], t["wg"])
     assert float(t["dlogits"].abs().max()) > 0 and torch.equal(t["dx"], want)
+
+
+# A large gate's weight gradient at any alignment of its elements (a view into a flat buffer of gradients): fp32 tokens, widths that are no
+# multiple of 64, more than 256 experts; one chunk of tokens, which an aligned result gets without a reduction, and several.
+@pytest.mark.parametrize("S,M,E,k,Fd,dtype", [(12, 72, 40, 2, 64, torch.float32), (700, 132, 70, 2, 32, torch.float32), (15, 520, 33, 1, 32, torch.bfloat16),
+                                              (1300, 136, 70, 4, 32, torch.bfloat16), (300, 64, 300, 2, 16, torch.bfloat16)])
+def test_gate_weight_gradient_at_any_alignment(S, M, E, k, Fd, dtype):
+    print(f"gate weight gradient at any alignment S={S} M={M} E={E} k={k} F={Fd} {dtype}", flush=True)
+    m, x, _ = _build(S, M, E, k, Fd, dtype, seed=S + E)
+    want = _native_training_pass(m, x, E, k, Fd, 0.0)["dwg"]
+    for off in (1, 2, 3):
+        flat = torch.full((E * M + 8,), 3.0, device="cuda")
+        _native_training_pass(m, x, E, k, Fd, 0.0, dwg=flat[off:off + E * M].view(E, M))
+        assert float(want.abs().max()) > 0 and torch.equal(flat[off:off + E * M].view(E, M), want)
+        assert bool((flat[:off] == 3.0).all()) and bool((flat[off + E * M:] == 3.0).all())
