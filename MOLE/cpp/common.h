@@ -105,7 +105,8 @@ inline void timed_launch(int id, void (*kernel)(KArgs...), dim3 grid, dim3 block
     }
 }
 
-// dWg = dlogits^T . x of a gate of any size (permute.hip); workspace of mole_gate_wgrad_workspace_bytes
+// dWg = dlogits^T . x of a gate of any size, with a workspace of gate_wgrad_bytes (permute.hip)
+size_t gate_wgrad_bytes(int dtype, int S, int E, int M);
 int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int M, float *dwg, void *workspace, size_t workspace_bytes, hipStream_t st);
 
 // the dispatch's backward with the gate's input gradient from bf16 operands, beyond the 32 experts of mole_dispatch_bwd's own (permute.hip)

@@ -69,7 +69,7 @@ static GateBwdPlan gate_bwd_plan(const mole_layer &L) {
     p.dl_t = !product ? 0 : up256((size_t)L.S * p.e_pad * es);
     p.wg_t = !product ? 0 : up256((size_t)p.e_pad * L.M * es);
     p.dx_add = !product ? 0 : up256((size_t)L.S * L.M * es);
-    p.wgrad = up256(mole_gate_wgrad_workspace_bytes(L.S, L.E, L.M));
+    p.wgrad = up256(gate_wgrad_bytes(L.dtype, L.S, L.E, L.M));
     p.total = p.dgates + p.dl_t + p.wg_t + p.dx_add + p.wgrad;
     return p;
 }

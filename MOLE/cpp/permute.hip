@@ -1193,15 +1193,21 @@ extern "C" int mole_dispatch_bwd(const void *dxd, int dtype, const int32_t *row,
     return 0;
 }
 
+static size_t gate_wgrad_valu_bytes(int S, int E, int M) { return (size_t)ceil_div(S, gw_tokens(S, E, M)) * E * M * sizeof(float); }
 extern "C" size_t mole_gate_wgrad_workspace_bytes(int S, int E, int M) {
     if (S <= 0 || E <= 0 || M <= 0) return 0;
-    // enough for either kernel: the caller does not say the dtype here
+    // enough for either kernel: the caller does not say the dtype here (small gates: the VALU kernel's
+    // partials; large gates only run on the matrix cores, with their own chunking)
     const size_t mfma = (size_t)ceil_div(S, gate_wgrad_mfma_chunk(S, E, M)) * E * M * sizeof(float);
-    const size_t valu = (size_t)ceil_div(S, gw_tokens(S, E, M)) * E * M * sizeof(float);
+    const size_t valu = E <= 32 ? gate_wgrad_valu_bytes(S, E, M) : 0;
     return mfma > valu ? mfma : valu;
 }
 
 namespace mole {
+// the need of gate_wgrad: that of mole_gate_wgrad for the gates it takes, the VALU kernel's partials beyond
+size_t gate_wgrad_bytes(int dtype, int S, int E, int M) {
+    return E <= 32 || gate_wgrad_mfma_ok(dtype, S, E, M) ? mole_gate_wgrad_workspace_bytes(S, E, M) : gate_wgrad_valu_bytes(S, E, M);
+}
 // Any number of experts.  A single chunk of tokens writes the result itself, without the reduction's launch.  Gates that neither kernel took
 // before went through the grouped-GEMM tiles, a block's walk over all tokens for 128 x 128 results, in the tokens' type: fp32, 3380 tokens, 79
 // experts of 448: 254 us; training passes, before / now: 8 tokens, 172 experts of 920 -> 456, 157 / 124; 4041 fp32 tokens, 245 of 704 -> 2112, 3127 /
@@ -1212,8 +1218,9 @@ int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int
     // gradients: it is then the reduction's to write)
     const bool any_dwg = E > 32 && !gate_wgrad_mfma_ok(dtype, S, E, M), direct = aligned16(dwg);
     MOLE_REQUIRE(dlogits && x && dwg && workspace && aligned16(x) && (any_dwg || aligned16(dwg)) && aligned16(workspace), "mole_gate_wgrad: null or misaligned pointer");
-    if (workspace_bytes < mole_gate_wgrad_workspace_bytes(S, E, M)) {
-        set_error("mole_gate_wgrad: workspace of %zu bytes, need %zu", workspace_bytes, mole_gate_wgrad_workspace_bytes(S, E, M));
+    const size_t need = gate_wgrad_bytes(dtype, S, E, M);
+    if (workspace_bytes < need) {
+        set_error("mole_gate_wgrad: workspace of %zu bytes, need %zu", workspace_bytes, need);
         return MOLE_E_WORKSPACE;
     }
     int nb;

@@ -234,6 +234,26 @@ def test_planes_of_a_padded_layout_stay_bounded():
     assert ragged > 32 << 20 and ragged * 7520 == padded * 6002
 
 
+def test_gate_weight_gradient_scratch_is_what_its_kernel_uses():
+    """mole_gate_wgrad: the matrix-core kernel's chunks of 128 tokens for gates that only that kernel takes (no more than 32 MB or
+    eight chunks).  The layer's: what the gate's own kernel needs, not the partial sums of one that does not take it."""
+    import ctypes
+    import struct
+    from mole_amd import _lib as L
+    lib = L.lib()
+    for S, E, M in ((2048, 64, 1024), (300, 40, 1024), (1, 33, 64), (5000, 200, 128)):
+        assert lib.mole_gate_wgrad_workspace_bytes(S, E, M) == (S + 127) // 128 * E * M * 4, (S, E, M)
+    assert lib.mole_gate_wgrad_workspace_bytes(16384, 256, 4096) == 8 * 256 * 4096 * 4
+
+    def backward(S, M, E, dtype):
+        block = ctypes.create_string_buffer(struct.pack("10id", dtype, S, M, E, 1, 64, S, L.LAYOUT_RAGGED, 1, 0, 1.0), 512)
+        return lib.mole_layer_workspace_bytes(ctypes.cast(block, ctypes.c_void_p), 1)
+
+    # 1024 experts of 8192: gradients of the gates, operands and result of the input gradient's product, and one [E, M] in fp32
+    S, E, M = 4096, 1024, 8192
+    assert backward(S, M, E, L.MOLE_BF16) <= 4 * S + 2 * (S * E + E * M + S * M) + 4 * E * M + 4096
+
+
 def test_fp32_products_leave_the_few_row_kernel_at_48_rows():
     """Beyond 48 rows per expert the tiles with split contractions are the faster ones; the few-row kernel has blocks enough
     there without a split, and no workspace."""
