@@ -43,6 +43,11 @@ __global__ __launch_bounds__(256) void pad_convert_kernel(const PadConvert a, co
     const int y = (int)(i / p.co), x = (int)(i % p.co);
     ((T *)p.out)[i] = y < p.r && x < p.c ? from_f32<T>(p.in[(size_t)y * p.c + x]) : from_f32<T>(0.f);
 }
+template <typename T>
+__global__ __launch_bounds__(256) void to_f32_kernel(const T *__restrict__ in, float *__restrict__ out, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) out[i] = to_f32(in[i]);
+}
 static int pad_convert(const PadConvert &a, const PadConvert &b, int dtype, hipStream_t st) {
     const dim3 grid(a.blocks() + b.blocks());
     if (dtype == MOLE_BF16) hipLaunchKernelGGL(pad_convert_kernel<bf16_t>, grid, dim3(256), 0, st, a, b, a.blocks());
@@ -51,9 +56,20 @@ static int pad_convert(const PadConvert &a, const PadConvert &b, int dtype, hipS
     return 0;
 }
 
-// Scratch of the backward's gate part, and which way its input gradient goes.
+// Whether dlogits^T . x of a gate that the matrix-core kernel does not take goes by the grouped-GEMM tiles, with the result in the tokens'
+// type, and not by gate_wgrad's VALU kernel, whose work grows with E M where a tile's walk over the tokens does not.  Training passes, tiles / VALU
+// kernel, us: bf16, 16384 tokens, 256 experts of 1800 871 / 802, 600 of 1024 875 / 855, 1024 of 1024 1172 / 1247, 256 of 4088 1354 / 1449; 2000
+// tokens of the last 533 / 533, 1000 464 / 450; fp32, 8192 tokens, 512 of 4096 2541 / 2436, 700 of 4096 3172 / 3280.
+static bool gate_wgrad_by_tiles(const mole_layer &L) {
+    if (L.E <= 32 || (L.dtype == MOLE_BF16 && L.E <= 256 && L.M % 64 == 0)) return false;
+    const size_t em = (size_t)L.E * L.M;
+    return L.dtype == MOLE_BF16 ? em > 5 << 17 && L.S > 1024 : em > 1 << 21;
+}
+
+// Scratch of the backward's gate part, and which way its two products go.
 struct GateBwdPlan {
     bool fold, fold_wide;    // dlogits . Wg inside mole_dispatch_bwd (up to 32 experts) / inside dispatch_bwd_fold
+    bool wgrad_tiles;        // dlogits^T . x on the grouped-GEMM tiles
     int e_pad;           // experts rounded up to the tiles' granule
     size_t dgates, dl_t, wg_t, dx_add, wgrad, total;     // bytes
 };
@@ -66,10 +82,11 @@ static GateBwdPlan gate_bwd_plan(const mole_layer &L) {
     const bool product = !p.fold && !p.fold_wide;
     p.e_pad = (L.E + epc - 1) / epc * epc;
     p.dgates = L.E > 256 ? up256((size_t)L.k * L.S * 4) : 0;
-    p.dl_t = !product ? 0 : up256((size_t)L.S * p.e_pad * es);
+    p.wgrad_tiles = gate_wgrad_by_tiles(L);
+    p.dl_t = !product && !p.wgrad_tiles ? 0 : up256((size_t)L.S * p.e_pad * es);
     p.wg_t = !product ? 0 : up256((size_t)p.e_pad * L.M * es);
     p.dx_add = !product ? 0 : up256((size_t)L.S * L.M * es);
-    p.wgrad = up256(gate_wgrad_bytes(L.dtype, L.S, L.E, L.M));
+    p.wgrad = up256(p.wgrad_tiles ? (size_t)p.e_pad * L.M * es : gate_wgrad_bytes(L.dtype, L.S, L.E, L.M));
     p.total = p.dgates + p.dl_t + p.wg_t + p.dx_add + p.wgrad;
     return p;
 }
@@ -175,5 +192,14 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
         if (int rc = mole_gemm_nn(dl_t, wg_t, L->dtype, L->S, L->M, p.e_pad, dx_add, stream)) return rc;
         if (int rc = mole_dispatch_bwd(G->gxd, L->dtype, L->row, L->S, L->M, L->k, nullptr, nullptr, 0, dx_add, G->dx, stream)) return rc;
     }
-    return gate_wgrad(G->dlogits, L->x, L->dtype, L->S, L->E, L->M, G->dwg, wgrad, p.wgrad, st);
+    if (!p.wgrad_tiles) return gate_wgrad(G->dlogits, L->x, L->dtype, L->S, L->E, L->M, G->dwg, wgrad, p.wgrad, st);
+    if (p.fold_wide)
+        if (int rc = pad_convert({G->dlogits, dl_t, L->S, L->E, L->S, p.e_pad}, {}, L->dtype, st)) return rc;
+    if (int rc = mole_gemm_tn(dl_t, L->x, L->dtype, L->S, p.e_pad, L->M, wgrad, stream)) return rc;
+    const size_t n = (size_t)L->E * L->M;
+    const dim3 grid((unsigned)((n + 255) / 256));
+    if (L->dtype == MOLE_BF16) hipLaunchKernelGGL(to_f32_kernel<bf16_t>, grid, dim3(256), 0, st, (const bf16_t *)wgrad, G->dwg, n);
+    else hipLaunchKernelGGL(to_f32_kernel<float>, grid, dim3(256), 0, st, (const float *)wgrad, G->dwg, n);
+    MOLE_LAUNCH_CHECK();
+    return 0;
 }

@@ -563,12 +563,14 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
 constexpr int GW_TOKENS = 64, GW_TOKENS_FEW = 16;
 // A block walks its tokens in batches of eight, one round trip to memory each: short blocks where long ones leave CUs
 // idle (513 tokens x 520, 16 experts: 11.5 -> 4.9 us; 110 x 384 fp32, 29 experts: 17.3 -> 7.0).  Gates of more than 32 experts take
-// a block per 32 of them, and chunks of more tokens while the partial sums would fill more than 32 MB.
+// a block per 32 of them, and chunks of more tokens while the partial sums would fill more than 40 MB: 16 chunks of the largest bf16 gates of
+// many tokens that come here (layer.hip), which eight leave short of blocks (training passes of 16384 tokens, eight / 16 chunks, us: 140
+// experts of 4088 1341 / 1133, 256 of 2056 1119 / 910).
 static int gw_tokens(int S, int E, int M) {
     const int zs = ceil_div(E, 32);
     int t = (long)ceil_div(S, GW_TOKENS) * ceil_div(M, 512) * zs < 192 ? GW_TOKENS_FEW : GW_TOKENS;
     if (zs > 1)
-        while ((size_t)ceil_div(S, t) * E * M * sizeof(float) > (32u << 20) && t < S) t *= 2;
+        while ((size_t)ceil_div(S, t) * E * M * sizeof(float) > (40u << 20) && t < S) t *= 2;
     return t;
 }
 template <typename T, int EB>
@@ -1208,10 +1210,9 @@ namespace mole {
 size_t gate_wgrad_bytes(int dtype, int S, int E, int M) {
     return E <= 32 || gate_wgrad_mfma_ok(dtype, S, E, M) ? mole_gate_wgrad_workspace_bytes(S, E, M) : gate_wgrad_valu_bytes(S, E, M);
 }
-// Any number of experts.  A single chunk of tokens writes the result itself, without the reduction's launch.  Gates that neither kernel took
-// before went through the grouped-GEMM tiles, a block's walk over all tokens for 128 x 128 results, in the tokens' type: fp32, 3380 tokens, 79
-// experts of 448: 254 us; training passes, before / now: 8 tokens, 172 experts of 920 -> 456, 157 / 124; 4041 fp32 tokens, 245 of 704 -> 2112, 3127 /
-// 2833.
+// Any number of experts.  A single chunk of tokens writes the result itself, without the reduction's launch.  Gates that neither kernel of
+// mole_gate_wgrad takes, by the grouped-GEMM tiles (a block's walk over all tokens for 128 x 128 results, in the tokens' type) / here, us: training
+// passes of 8 tokens, 172 experts of 920 -> 456, 157 / 124; 4041 fp32 tokens, 245 of 704 -> 2112, 3127 / 2833; the largest stay there (layer.hip).
 int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int M, float *dwg, void *workspace, size_t workspace_bytes, hipStream_t st) {
     ScopedTiming timing(MOLE_K_GATE_WGRAD, st);
     // (the layer's gates beyond mole_gate_wgrad's own may have their result at any alignment of its elements, a view into a flat buffer of

@@ -1063,3 +1063,20 @@ def test_gate_weight_gradient_at_any_alignment(S, M, E, k, Fd, dtype):
         _native_training_pass(m, x, E, k, Fd, 0.0, dwg=flat[off:off + E * M].view(E, M))
         assert float(want.abs().max()) > 0 and torch.equal(flat[off:off + E * M].view(E, M), want)
         assert bool((flat[:off] == 3.0).all()) and bool((flat[off + E * M:] == 3.0).all())
+
+
+# Both sides of the line between the two ways of a large gate's weight gradient: by tiles beyond it, bit for bit what mole_gemm_tn gives from
+# operands in the tokens' type; before it fp32 sums of at most 16 x 128 tokens a chunk and 16 chunks (2^-24 of the terms' size a step of either).
+@pytest.mark.parametrize("S,M,E,Fd,dtype,tiles", [(1030, 2192, 300, 8, torch.bfloat16, True), (1030, 2184, 300, 8, torch.bfloat16, False), (1024, 2192, 300, 8, torch.bfloat16, False),
+                                                  (1100, 10248, 64, 8, torch.bfloat16, True), (130, 2100, 1000, 4, torch.float32, True), (130, 2096, 1000, 4, torch.float32, False)])
+def test_gate_weight_gradient_on_either_side_of_the_tiles(S, M, E, Fd, dtype, tiles):
+    from mole_amd import hip_ops as H
+    print(f"gate weight gradient, tiles={tiles} S={S} M={M} E={E} F={Fd} {dtype}", flush=True)
+    m, x, _ = _build(S, M, E, 1, Fd, dtype, seed=S + M)
+    t = _native_training_pass(m, x, E, 1, Fd, 0.0)
+    by_tiles = H.gemm_tn(H._pad_cols(t["dlogits"].to(dtype), 8 if dtype == torch.bfloat16 else 4), x)[:E].float()
+    assert float(t["dwg"].abs().max()) > 0 and torch.equal(t["dwg"], by_tiles) == tiles
+    if not tiles:
+        dl, x64 = t["dlogits"].double().cpu(), x.double().cpu()
+        bound = (16 * 128 + 16) * 2.0 ** -24 * (dl.abs().t() @ x64.abs())
+        assert bool(((t["dwg"].double().cpu() - dl.t() @ x64).abs() <= bound).all())
