@@ -467,7 +467,10 @@ __global__ __launch_bounds__(256) void route_finalize_kernel(const RouteEnd r, c
 // nb == 1: the block has seen all tokens and goes on to the end of the routing by itself.  hist null: route_rank takes it
 // from the indices.
 enum { LOGITS_NONE, LOGITS_WHOLE, LOGITS_PARTS, LOGITS_PAIRS };
-template <int VPL, int LOGG, int THREADS, int TOK>
+// PARTS: partial sums may come (up to 64 tokens).  Their registers are not for the blocks of 64 tokens beyond 64 experts: three parts beside 16
+// values a lane, and 54 registers instead of 18 are spilled (routing of 512 tokens, 300 experts top-8, with / without, 80.6 / 75.1 us; 16384, 512
+// top-8, 91.2 / 78.9; that pass 274 / 261).
+template <int VPL, int LOGG, int THREADS, int TOK, bool PARTS>
 __global__ __launch_bounds__(THREADS) void route_tokens_kernel(const float *__restrict__ in, const float *__restrict__ bias,
                                                                    int logits, int normalize,
                                                                    float *__restrict__ scores, float *__restrict__ gates,
@@ -504,7 +507,7 @@ __global__ __launch_bounds__(THREADS) void route_tokens_kernel(const float *__re
         if (S > 0) {
 #pragma unroll
             for (int q = 0; q < VPL; ++q) v[q] = in[(size_t)min(token, S - 1) * E + min(g + (q << LOGG), E - 1)];
-            if (logits >= LOGITS_PARTS) {
+            if (PARTS && logits >= LOGITS_PARTS) {
                 float t[3][VPL];
 #pragma unroll
                 for (int u = 0; u < 3; ++u)
@@ -701,12 +704,13 @@ static RouteEnd route_end(int S, int E, int k, double capacity_factor, int align
     return RouteEnd{S, E, k, cf_sign, k * (prod < (double)limit ? (int)prod : limit), alignment, layout, counts, kept_rows, offsets, capacity, l_aux, idx, loc, row, token_of};
 }
 
-template <int VPL, int LOGG, int THREADS, int TOK>
+template <int VPL, int LOGG, int THREADS, int TOK, bool PARTS>
 static int launch_tokens_as(const float *in, const float *bias, int logits, int normalize, float *scores, float *gates, int32_t *hist, float *colsum,
                             int nb, const RouteEnd &r, hipStream_t st) {
     constexpr int COLS = THREADS / WAVE * (THREADS == 256 ? WAVE >> LOGG : 1);
     const size_t lds = (size_t)r.k * TOK * 8 + (size_t)COLS * r.E * 4 + (nb == 1 || hist != nullptr ? (size_t)(r.k + 1) * r.E * 4 : 0);
-    auto kern = route_tokens_kernel<VPL, LOGG, THREADS, TOK>;
+    auto kern = route_tokens_kernel<VPL, LOGG, THREADS, TOK, PARTS>;
+    MOLE_REQUIRE(PARTS || logits < LOGITS_PARTS, "routing: partial logits for a kernel that takes whole ones (S=%d E=%d k=%d)", r.S, r.E, r.k);
     if (lds > 48 * 1024)               // hundreds of experts and a long top-k: beyond the default limit together with the static part
         MOLE_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(kern, dim3(nb), dim3(THREADS), lds, st, in, bias, logits, normalize, scores, gates, hist, colsum, nb, r);
@@ -716,23 +720,23 @@ static int launch_tokens_as(const float *in, const float *bias, int logits, int 
 // few: at most FEW_TOKENS tokens, in blocks of few_block(E)
 static int launch_tokens(bool few, const float *in, const float *bias, int logits, int normalize, float *scores, float *gates, int32_t *hist, float *colsum,
                          int nb, const RouteEnd &r, hipStream_t st) {
-#define MOLE_LT(VPL, LOGG, THREADS, TOK) launch_tokens_as<VPL, LOGG, THREADS, TOK>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st)
+#define MOLE_LT(VPL, LOGG, THREADS, TOK, PARTS) launch_tokens_as<VPL, LOGG, THREADS, TOK, PARTS>(in, bias, logits, normalize, scores, gates, hist, colsum, nb, r, st)
     const int E = r.E;
     if (few) {
-        if (E <= 16) return MOLE_LT(1, 4, 256, 16);
-        if (E <= 32) return MOLE_LT(2, 4, 256, 16);
-        if (E <= 64) return MOLE_LT(4, 4, 256, 16);
-        if (E <= 128) return MOLE_LT(2, 6, 256, 4);
-        if (E <= 256) return MOLE_LT(4, 6, 256, 4);
-        return MOLE_LT(16, 6, 256, 4);
+        if (E <= 16) return MOLE_LT(1, 4, 256, 16, true);
+        if (E <= 32) return MOLE_LT(2, 4, 256, 16, true);
+        if (E <= 64) return MOLE_LT(4, 4, 256, 16, true);
+        if (E <= 128) return MOLE_LT(2, 6, 256, 4, true);
+        if (E <= 256) return MOLE_LT(4, 6, 256, 4, true);
+        return MOLE_LT(16, 6, 256, 4, true);
     }
     // 16 lanes per token; beyond 256 experts a lane would hold more than 16 values, so the whole wave takes a token
-    if (E <= 16) return MOLE_LT(1, 4, 1024, 64);
-    if (E <= 32) return MOLE_LT(2, 4, 1024, 64);
-    if (E <= 64) return MOLE_LT(4, 4, 1024, 64);
-    if (E <= 128) return MOLE_LT(8, 4, 1024, 64);
-    if (E <= 256) return MOLE_LT(16, 4, 1024, 64);
-    return MOLE_LT(16, 6, 1024, 64);
+    if (E <= 16) return MOLE_LT(1, 4, 1024, 64, true);
+    if (E <= 32) return MOLE_LT(2, 4, 1024, 64, true);
+    if (E <= 64) return MOLE_LT(4, 4, 1024, 64, true);
+    if (E <= 128) return MOLE_LT(8, 4, 1024, 64, false);
+    if (E <= 256) return MOLE_LT(16, 4, 1024, 64, false);
+    return MOLE_LT(16, 6, 1024, 64, false);
 #undef MOLE_LT
 }
 template <int P> static int launch_rank(const float *colsum, int nb_col, const RouteEnd &r, hipStream_t st) {
@@ -1412,8 +1416,11 @@ static size_t gate_route_fused_bytes(int S, int E, int k) {
 //   SCORES  fp32, up to 32 experts: mole_gate_fwd's wave per token, then the routing of the scores
 //   GEMM    logits on the grouped-GEMM tiles, then softmax and routing
 enum { GR_FUSED, GR_FEW, GR_SCORES, GR_GEMM };
-// The logits of FEW by quarters of the model dimension: while four times the blocks are at most one for every CU.
-static bool gate_quarters(int S, int E) { return S <= RT_TOKENS && ceil_div(S, 16) * ceil_div(E, 16) <= 64; }
+// The logits of FEW by quarters of the model dimension: while four times the blocks are at most one for every CU, and where the routing adds
+// them up (all but 5 to 64 tokens over 1024 experts, top-16, whose pairs route_rank does not hold: see route_from).
+static bool gate_quarters(int S, int E, int k) {
+    return S <= RT_TOKENS && ceil_div(S, 16) * ceil_div(E, 16) <= 64 && (E <= 64 || S <= few_block(E) || rank_in_one_block(S, E, k));
+}
 static int gate_route_path(int dtype, int S, int E, int M) {
     if (dtype == MOLE_BF16 && M % 128 == 0 && E <= 64 && S > RT_TOKENS) return GR_FUSED;
     if (S <= 2048 || (dtype == MOLE_F32 && E > 32 && (long)ceil_div(S, 32) * ceil_div(E, 16) <= 3072)) return GR_FEW;
@@ -1425,7 +1432,7 @@ extern "C" size_t mole_gate_route_shape_workspace_bytes(int dtype, int S, int E,
     const int path = gate_route_path(dtype, S, E, M);
     if (path == GR_FUSED) return gate_route_fused_bytes(S, E, k);
     size_t n = mole_route_workspace_bytes(S, E, k);
-    if (path != GR_SCORES) n += align256((path == GR_FEW && gate_quarters(S, E) ? 4 : 1) * (size_t)S * E * sizeof(float));
+    if (path != GR_SCORES) n += align256((path == GR_FEW && gate_quarters(S, E, k) ? 4 : 1) * (size_t)S * E * sizeof(float));
     if (path == GR_GEMM && dtype == MOLE_BF16) n += align256((size_t)E * M * sizeof(bf16_t));
     return n;
 }
@@ -1476,7 +1483,7 @@ int gate_route(const void *x, int dtype, const float *wg, const float *logit_bia
             return route_from(scores, nullptr, LOGITS_NONE, normalize_gate, nullptr, gates, r, route_ws, st);
         }
         float *logits = (float *)ws;
-        if (path == GR_FEW && gate_quarters(S, E)) {
+        if (path == GR_FEW && gate_quarters(S, E, k)) {
             const dim3 grid(ceil_div(S, 16), ceil_div(E, 16), 4);
             if (dtype == MOLE_BF16) timed_launch(MOLE_K_GATE_FWD, gate_logits_kernel<bf16_t, 1, true>, grid, dim3(64), 0, st, (const bf16_t *)x, wg, nullptr, S, E, M, logits);
             else timed_launch(MOLE_K_GATE_FWD, gate_logits_kernel<float, 1, true>, grid, dim3(64), 0, st, (const float *)x, wg, nullptr, S, E, M, logits);

@@ -254,6 +254,35 @@ def test_gate_weight_gradient_scratch_is_what_its_kernel_uses():
     assert backward(S, M, E, L.MOLE_BF16) <= 4 * S + 2 * (S * E + E * M + S * M) + 4 * E * M + 4096
 
 
+def _kernel_metadata():
+    """What the built library's code objects say about their kernels: name -> metadata map of the AMDGPU note."""
+    import struct
+    import msgpack
+    from mole_amd import _lib as L
+    blob, out, at = open(L.LIB_PATH, "rb").read(), {}, 0
+    while (at := blob.find(b"\x7fELF", at + 1)) >= 0:
+        if struct.unpack_from("<H", blob, at + 18)[0] != 224:                      # EM_AMDGPU
+            continue
+        shoff, (shentsize, shnum) = struct.unpack_from("<Q", blob, at + 40)[0], struct.unpack_from("<HH", blob, at + 58)
+        for i in range(shnum):
+            kind, _, _, off = struct.unpack_from("<IQQQ", blob, at + shoff + i * shentsize + 4)
+            if kind == 7:                                                          # SHT_NOTE
+                name, desc = struct.unpack_from("<II", blob, at + off)
+                start = at + off + 12 + (name + 3) // 4 * 4
+                for k in msgpack.unpackb(blob[start:start + desc])["amdhsa.kernels"]:
+                    out[k[".name"]] = k
+    return out
+
+
+def test_routing_of_many_tokens_keeps_its_registers():
+    """The top-k kernel of many tokens holds 16 scores a lane and no partial sums of them beside: it spills a few registers beyond 256 experts
+    (18, with the sums 54) and none below."""
+    spills = {n: k[".vgpr_spill_count"] for n, k in _kernel_metadata().items() if "route_tokens_kernel" in n}
+    wide = [n for n in spills if "ILi16ELi6ELi1024E" in n]
+    assert len(spills) >= 12 and len(wide) == 1
+    assert all(v <= (24 if n in wide else 0) for n, v in spills.items()), spills
+
+
 def test_fp32_products_leave_the_few_row_kernel_at_48_rows():
     """Beyond 48 rows per expert the tiles with split contractions are the faster ones; the few-row kernel has blocks enough
     there without a split, and no workspace."""
