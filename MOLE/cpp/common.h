@@ -117,6 +117,7 @@ struct CombineTail;     // gemm.h
 struct DispatchHead;
 // the FFN's entry points with the caller's estimate of the rows beside their bound (ffn_gemm.hip)
 size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, int F);
+size_t gate_route_least_bytes(int dtype, int S, int E, int M, int k);     // gate_route's without small blocks
 int gate_route(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M, int k, double capacity_factor,
                int normalize_gate, int alignment, int layout, float *scores, int32_t *idx, int32_t *loc, float *gates, int32_t *row, int32_t *counts,
                int32_t *kept_rows, int32_t *offsets, int32_t *capacity, float *l_aux, int32_t *token_of, void *workspace, size_t workspace_bytes,

@@ -60,10 +60,10 @@ static int pad_convert(const PadConvert &a, const PadConvert &b, int dtype, hipS
 // type, and not by gate_wgrad's VALU kernel, whose work grows with E M where a tile's walk over the tokens does not.  Training passes, tiles / VALU
 // kernel, us: bf16, 16384 tokens, 256 experts of 1800 871 / 802, 600 of 1024 875 / 855, 1024 of 1024 1172 / 1247, 256 of 4088 1354 / 1449; 2000
 // tokens of the last 533 / 533, 1000 464 / 450; fp32, 8192 tokens, 512 of 4096 2541 / 2436, 700 of 4096 3172 / 3280.
+static bool gate_wgrad_may_go_by_tiles(const mole_layer &L) { return L.E > 32 && !(L.dtype == MOLE_BF16 && L.E <= 256 && L.M % 64 == 0); }
 static bool gate_wgrad_by_tiles(const mole_layer &L) {
-    if (L.E <= 32 || (L.dtype == MOLE_BF16 && L.E <= 256 && L.M % 64 == 0)) return false;
     const size_t em = (size_t)L.E * L.M;
-    return L.dtype == MOLE_BF16 ? em > 5 << 17 && L.S > 1024 : em > 1 << 21;
+    return gate_wgrad_may_go_by_tiles(L) && (L.dtype == MOLE_BF16 ? em > 5 << 17 && L.S > 1024 : em > 1 << 21);
 }
 
 // Scratch of the backward's gate part, and which way its two products go.
@@ -73,7 +73,7 @@ struct GateBwdPlan {
     int e_pad;           // experts rounded up to the tiles' granule
     size_t dgates, dl_t, wg_t, dx_add, wgrad, total;     // bytes
 };
-static GateBwdPlan gate_bwd_plan(const mole_layer &L) {
+static GateBwdPlan gate_bwd_plan(const mole_layer &L, bool wgrad_tiles) {
     GateBwdPlan p{};
     const size_t es = L.dtype == MOLE_BF16 ? 2 : 4;
     const int epc = L.dtype == MOLE_BF16 ? 8 : 4;
@@ -82,7 +82,7 @@ static GateBwdPlan gate_bwd_plan(const mole_layer &L) {
     const bool product = !p.fold && !p.fold_wide;
     p.e_pad = (L.E + epc - 1) / epc * epc;
     p.dgates = L.E > 256 ? up256((size_t)L.k * L.S * 4) : 0;
-    p.wgrad_tiles = gate_wgrad_by_tiles(L);
+    p.wgrad_tiles = wgrad_tiles;
     p.dl_t = !product && !p.wgrad_tiles ? 0 : up256((size_t)L.S * p.e_pad * es);
     p.wg_t = !product ? 0 : up256((size_t)p.e_pad * L.M * es);
     p.dx_add = !product ? 0 : up256((size_t)L.S * L.M * es);
@@ -98,7 +98,7 @@ using namespace mole;
 extern "C" size_t mole_layer_workspace_bytes(const mole_layer *L, int backward) {
     if (L == nullptr || L->S <= 0 || L->E <= 0) return 0;
     const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
-    size_t other = backward ? gate_bwd_plan(*L).total : mole_gate_route_shape_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
+    size_t other = backward ? gate_bwd_plan(*L, gate_wgrad_by_tiles(*L)).total : mole_gate_route_shape_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
     if (!backward && tokens_beside_rows(*L)) other = up256(other) + (size_t)L->rows * 4;
     return ffn > other ? ffn : other;        // the two are never in use at the same time
 }
@@ -114,8 +114,8 @@ static int check_layer(const char *fn, const mole_layer *L, mole_stream_t) {
 extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream) {
     if (int rc = check_layer("mole_layer_fwd", L, stream)) return rc;
     const size_t route_bytes = mole_gate_route_shape_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
-    const size_t need = std::max(route_bytes, ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F));
-    if (L->workspace_bytes < need) {
+    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F), need = std::max(route_bytes, ffn);
+    if (L->workspace_bytes < std::max(gate_route_least_bytes(L->dtype, L->S, L->E, L->M, L->k), ffn)) {
         set_error("mole_layer_fwd: workspace of %zu bytes, need %zu", L->workspace_bytes, need);
         return MOLE_E_WORKSPACE;
     }
@@ -156,12 +156,14 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
     if (int rc = check_layer("mole_layer_bwd", L, stream)) return rc;
     MOLE_REQUIRE(!L->forward_only, "mole_layer_bwd: the forward pass was a forward_only one");
     MOLE_REQUIRE(G && G->dy && G->dlogits && G->d_o && G->t && G->gxd && G->dx && G->dwg, "mole_layer_bwd: null gradient pointer");
-    const size_t need = mole_layer_workspace_bytes(L, 1);
-    if (L->workspace_bytes < need) {
+    const size_t need = mole_layer_workspace_bytes(L, 1), ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
+    GateBwdPlan p = gate_bwd_plan(*L, gate_wgrad_by_tiles(*L));
+    // (a workspace that does not hold the partial sums of a large gate has its weight gradient by the tiles)
+    if (L->workspace_bytes < need && gate_wgrad_may_go_by_tiles(*L)) p = gate_bwd_plan(*L, true);
+    if (L->workspace_bytes < std::max(ffn, p.total)) {
         set_error("mole_layer_bwd: workspace of %zu bytes, need %zu", L->workspace_bytes, need);
         return MOLE_E_WORKSPACE;
     }
-    const GateBwdPlan p = gate_bwd_plan(*L);
     hipStream_t st = (hipStream_t)stream;
     char *ws = (char *)L->workspace;
     const int32_t *counts0 = G->d_l_aux ? L->counts : nullptr;

@@ -656,12 +656,17 @@ using namespace mole;
 constexpr int FEW_TOKENS = 512;
 static int few_block(int E) { return E <= 64 ? 16 : 4; }
 
+// Scratch of the routing by histograms, with which mole_route does any call, and the column sums of small blocks, which are more where the blocks are
+// many and the choices few: mole_route takes small blocks where the workspace holds them.
+static size_t route_hist_bytes(int S, int E, int k) {
+    const size_t nb = (size_t)ceil_div(S > 0 ? S : 1, RT_TOKENS);
+    return align256(nb * k * E * sizeof(int32_t)) + align256((size_t)k * E * sizeof(int32_t)) +
+           align256(nb * E * sizeof(float)) + align256((size_t)COLSUM_SLICES * E * sizeof(float));
+}
+static size_t few_bytes(int S, int E) { return S <= FEW_TOKENS ? align256((size_t)ceil_div(S, few_block(E)) * E * sizeof(float)) : 0; }
 extern "C" size_t mole_route_workspace_bytes(int S, int E, int k) {
     if (S < 0 || E <= 0 || k <= 0) return 0;
-    const size_t nb = (size_t)ceil_div(S > 0 ? S : 1, RT_TOKENS);
-    const size_t few = S <= FEW_TOKENS ? align256((size_t)ceil_div(S, few_block(E)) * E * sizeof(float)) : 0;      // (only their column sums)
-    return few + align256(nb * k * E * sizeof(int32_t)) + align256((size_t)k * E * sizeof(int32_t)) +
-           align256(nb * E * sizeof(float)) + align256((size_t)COLSUM_SLICES * E * sizeof(float));
+    return std::max(route_hist_bytes(S, E, k), few_bytes(S, E));
 }
 
 // The stages of the routing behind the tokens' own: scan of the histograms over blocks, counts / capacity / offsets /
@@ -757,12 +762,12 @@ static int route_rank(const float *colsum, int nb_col, const RouteEnd &r, hipStr
 
 // The whole routing of scores (or of logits, to which bias is added if given and whose softmax then goes to `scores`).
 static int route_from(const float *in, const float *bias, int logits, int normalize, float *scores, float *gates, const RouteEnd &r, void *workspace,
-                      hipStream_t st) {
+                      size_t workspace_bytes, hipStream_t st) {
     const int nb = ceil_div(r.S > 0 ? r.S : 1, RT_TOKENS);
     char *ws = (char *)workspace;
     if (r.S <= few_block(r.E)) return launch_tokens(true, in, bias, logits, normalize, scores, gates, nullptr, nullptr, 1, r, st);
-    const bool few = r.S <= FEW_TOKENS, rank = rank_in_one_block(r.S, r.E, r.k);
-    if (nb == 1 && !(rank && r.E > 64)) return launch_tokens(false, in, bias, logits, normalize, scores, gates, nullptr, nullptr, 1, r, st);
+    const bool few = r.S <= FEW_TOKENS && workspace_bytes >= few_bytes(r.S, r.E), rank = rank_in_one_block(r.S, r.E, r.k);
+    if (nb == 1 && !(few && rank && r.E > 64)) return launch_tokens(false, in, bias, logits, normalize, scores, gates, nullptr, nullptr, 1, r, st);
     if (rank) {
         float *colsum = (float *)ws;
         const int blocks = few ? ceil_div(r.S, few_block(r.E)) : nb;
@@ -793,14 +798,14 @@ extern "C" int mole_route(const float *scores, int S, int E, int k, double capac
     MOLE_REQUIRE(counts && kept_rows && offsets && capacity && workspace, "mole_route: null output pointer");
     MOLE_REQUIRE(S == 0 || (scores && idx && loc && gates && row), "mole_route: null token buffer");
     MOLE_REQUIRE((long long)S * k < INT_MAX && (long long)S * E < (1ll << 40), "mole_route: S*k too large");
-    if (workspace_bytes < mole_route_workspace_bytes(S, E, k)) {
+    if (workspace_bytes < route_hist_bytes(S, E, k)) {
         set_error("mole_route: workspace of %zu bytes, need %zu", workspace_bytes, mole_route_workspace_bytes(S, E, k));
         return MOLE_E_WORKSPACE;
     }
     hipStream_t st = (hipStream_t)stream;
     ScopedTiming timing(MOLE_K_ROUTE, st);
     const RouteEnd r = route_end(S, E, k, capacity_factor, alignment, layout, idx, loc, row, counts, kept_rows, offsets, capacity, l_aux);
-    return route_from(scores, nullptr, LOGITS_NONE, normalize_gate, nullptr, gates, r, workspace, st);
+    return route_from(scores, nullptr, LOGITS_NONE, normalize_gate, nullptr, gates, r, workspace, workspace_bytes, st);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1427,14 +1432,20 @@ static int gate_route_path(int dtype, int S, int E, int M) {
     return dtype == MOLE_F32 && E <= 32 ? GR_SCORES : GR_GEMM;
 }
 
-extern "C" size_t mole_gate_route_shape_workspace_bytes(int dtype, int S, int E, int M, int k) {
-    if (S < 0 || E <= 0 || M <= 0 || k <= 0) return 0;
+// small: with the routing's small blocks and the logits by quarters; otherwise the least that the call does with
+static size_t gate_route_bytes(int dtype, int S, int E, int M, int k, bool small) {
     const int path = gate_route_path(dtype, S, E, M);
     if (path == GR_FUSED) return gate_route_fused_bytes(S, E, k);
-    size_t n = mole_route_workspace_bytes(S, E, k);
-    if (path != GR_SCORES) n += align256((path == GR_FEW && gate_quarters(S, E, k) ? 4 : 1) * (size_t)S * E * sizeof(float));
+    size_t n = small ? mole_route_workspace_bytes(S, E, k) : route_hist_bytes(S, E, k);
+    if (path != GR_SCORES) n += align256((small && path == GR_FEW && gate_quarters(S, E, k) ? 4 : 1) * (size_t)S * E * sizeof(float));
     if (path == GR_GEMM && dtype == MOLE_BF16) n += align256((size_t)E * M * sizeof(bf16_t));
     return n;
+}
+extern "C" size_t mole_gate_route_shape_workspace_bytes(int dtype, int S, int E, int M, int k) {
+    return S < 0 || E <= 0 || M <= 0 || k <= 0 ? 0 : gate_route_bytes(dtype, S, E, M, k, true);
+}
+namespace mole {
+size_t gate_route_least_bytes(int dtype, int S, int E, int M, int k) { return gate_route_bytes(dtype, S, E, M, k, false); }
 }
 
 extern "C" size_t mole_gate_route_workspace_bytes(int S, int E, int k) {
@@ -1466,7 +1477,8 @@ int gate_route(const void *x, int dtype, const float *wg, const float *logit_bia
                  "mole_gate_route: x and wg must be 16-byte aligned");
     MOLE_REQUIRE((long long)S * k < INT_MAX, "mole_gate_route: S*k too large");
     const size_t need = mole_gate_route_shape_workspace_bytes(dtype, S, E, M, k);
-    if (workspace_bytes < need) {
+    const bool small = workspace_bytes >= need;
+    if (workspace_bytes < gate_route_least_bytes(dtype, S, E, M, k)) {
         set_error("mole_gate_route: workspace of %zu bytes, need %zu", workspace_bytes, need);
         return MOLE_E_WORKSPACE;
     }
@@ -1476,20 +1488,21 @@ int gate_route(const void *x, int dtype, const float *wg, const float *logit_bia
     char *ws = (char *)workspace;
     if (path != GR_FUSED) {
         void *route_ws = ws;
-        ws += mole_route_workspace_bytes(S, E, k);
+        const size_t route_bytes = small ? mole_route_workspace_bytes(S, E, k) : route_hist_bytes(S, E, k);
+        ws += route_bytes;
         if (path == GR_SCORES) {
             if (int rc = mole_gate_fwd(x, dtype, wg, logit_bias, S, E, M, scores, stream)) return rc;
             ScopedTiming timing(MOLE_K_ROUTE, st);
-            return route_from(scores, nullptr, LOGITS_NONE, normalize_gate, nullptr, gates, r, route_ws, st);
+            return route_from(scores, nullptr, LOGITS_NONE, normalize_gate, nullptr, gates, r, route_ws, route_bytes, st);
         }
         float *logits = (float *)ws;
-        if (path == GR_FEW && gate_quarters(S, E, k)) {
+        if (small && path == GR_FEW && gate_quarters(S, E, k)) {
             const dim3 grid(ceil_div(S, 16), ceil_div(E, 16), 4);
             if (dtype == MOLE_BF16) timed_launch(MOLE_K_GATE_FWD, gate_logits_kernel<bf16_t, 1, true>, grid, dim3(64), 0, st, (const bf16_t *)x, wg, nullptr, S, E, M, logits);
             else timed_launch(MOLE_K_GATE_FWD, gate_logits_kernel<float, 1, true>, grid, dim3(64), 0, st, (const float *)x, wg, nullptr, S, E, M, logits);
             MOLE_LAUNCH_CHECK();
             ScopedTiming timing(MOLE_K_ROUTE, st);
-            return route_from(logits, logit_bias, dtype == MOLE_BF16 ? LOGITS_PARTS : LOGITS_PAIRS, normalize_gate, scores, gates, r, route_ws, st);
+            return route_from(logits, logit_bias, dtype == MOLE_BF16 ? LOGITS_PARTS : LOGITS_PAIRS, normalize_gate, scores, gates, r, route_ws, route_bytes, st);
         }
         ws += align256((size_t)S * E * sizeof(float));
         if (path == GR_FEW) {
@@ -1503,7 +1516,7 @@ int gate_route(const void *x, int dtype, const float *wg, const float *logit_bia
 #undef MOLE_GL
             MOLE_LAUNCH_CHECK();
             ScopedTiming timing(MOLE_K_ROUTE, st);
-            return route_from(logits, nullptr, LOGITS_WHOLE, normalize_gate, scores, gates, r, route_ws, st);
+            return route_from(logits, nullptr, LOGITS_WHOLE, normalize_gate, scores, gates, r, route_ws, route_bytes, st);
         }
         const void *w = wg;
         if (dtype == MOLE_BF16) {
@@ -1514,7 +1527,7 @@ int gate_route(const void *x, int dtype, const float *wg, const float *logit_bia
         }
         if (int rc = mole_gemm_nt(x, w, dtype, S, E, M, logits, stream)) return rc;
         ScopedTiming timing(MOLE_K_ROUTE, st);
-        return route_from(logits, logit_bias, LOGITS_WHOLE, normalize_gate, scores, gates, r, route_ws, st);
+        return route_from(logits, logit_bias, LOGITS_WHOLE, normalize_gate, scores, gates, r, route_ws, route_bytes, st);
     }
     const int nb = ceil_div(S, GATE_ROUTE_TOKENS);
     int32_t *hist = (int32_t *)ws;

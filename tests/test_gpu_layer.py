@@ -1010,8 +1010,8 @@ class _Layer(ctypes.Structure):
                                                "xd h a out workspace".split()] + [("workspace_bytes", ctypes.c_size_t)])
 
 
-def _native_training_pass(m, x, E, k, Fd, cf, dwg=None):
-    """mole_layer_fwd and mole_layer_bwd on buffers of the test's own: every tensor of both blocks, and y."""
+def _native_training_pass(m, x, E, k, Fd, cf, dwg=None, sizes=None):
+    """mole_layer_fwd and mole_layer_bwd on buffers of the test's own: every tensor of both blocks, and y.  sizes: bytes of the two workspaces."""
     S, M = x.shape
     dtype, rows, wg = x.dtype, S * k, m.gate[0].linear.weight.detach()
     w = dict(zip(("w1", "b1", "w2", "b2"), (p.all_tensors for p in (m.FC1_W_GPU, m.FC1_B_GPU, m.FC2_W_GPU, m.FC2_B_GPU))))
@@ -1028,14 +1028,18 @@ def _native_training_pass(m, x, E, k, Fd, cf, dwg=None):
     grads = _Grads(0, L.GELU_BWD_TANH, **{n: v.data_ptr() for n, v in g.items()})
     for backward in (0, 1):
         block.workspace_bytes = L.lib().mole_layer_workspace_bytes(ctypes.byref(block), backward)
-        ws = torch.empty(max(1, block.workspace_bytes), dtype=torch.uint8, device="cuda")
+        if sizes is not None:
+            assert sizes[backward] <= block.workspace_bytes
+            block.workspace_bytes = sizes[backward]
+        ws = torch.full((max(1, block.workspace_bytes) + 256,), 77, dtype=torch.uint8, device="cuda")
         block.workspace = ws.data_ptr()
         if backward:
             L.check(L.lib().mole_layer_bwd(ctypes.byref(block), ctypes.byref(grads), L.stream()), "mole_layer_bwd")
         else:
             L.check(L.lib().mole_layer_fwd(ctypes.byref(block), L.ptr(y), L.stream()), "mole_layer_fwd")
         torch.cuda.synchronize()
-    return dict(t, **g, y=y)
+        assert bool((ws[block.workspace_bytes:] == 77).all())
+    return dict(t, **g, y=y, block=block)
 
 
 # Where the dispatch's backward takes the gate's input gradient in, the sum is that of the two entry points, bit for bit: the product from
@@ -1080,3 +1084,32 @@ def test_gate_weight_gradient_on_either_side_of_the_tiles(S, M, E, Fd, dtype, ti
         dl, x64 = t["dlogits"].double().cpu(), x.double().cpu()
         bound = (16 * 128 + 16) * 2.0 ** -24 * (dl.abs().t() @ x64.abs())
         assert bool(((t["dwg"].double().cpu() - dl.t() @ x64).abs() <= bound).all())
+
+
+# Workspaces of the least sizes: histograms of blocks of 64 tokens and whole logits for the forward pass, operands and results of the gate's two products
+# for the backward one.  The pass is the same but for the order of the loss term's sums and a large gate's weight gradient, which is then the tiles'.
+@pytest.mark.parametrize("S,M,E,k,Fd,dtype", [(40, 128, 70, 1, 16, torch.bfloat16), (500, 64, 256, 1, 16, torch.bfloat16), (60, 136, 20, 2, 32, torch.bfloat16),
+                                              (2000, 72, 100, 2, 8, torch.float32), (700, 136, 70, 4, 16, torch.bfloat16), (50, 64, 1000, 2, 4, torch.float32)])
+def test_layer_with_the_least_workspaces(S, M, E, k, Fd, dtype):
+    from mole_amd import hip_ops as H
+    print(f"least workspaces S={S} M={M} E={E} k={k} F={Fd} {dtype}", flush=True)
+    m, x, _ = _build(S, M, E, k, Fd, dtype, seed=S + E)
+    up = lambda n: (n + 255) // 256 * 256
+    nb, es, ep = (S + 63) // 64, x.element_size(), 8 if dtype == torch.bfloat16 else 4
+    e_pad = (E + ep - 1) // ep * ep
+    ffn = L.lib().mole_ffn_workspace_bytes(L.dtype_code(dtype), E, S * k, M, Fd)
+    fwd = up(nb * k * E * 4) + up(k * E * 4) + up(nb * E * 4) + up(16 * E * 4) + up(S * E * 4)
+    bwd = (up(k * S * 4) if E > 256 else 0) + up(S * e_pad * es) + up(e_pad * M * es) + up(S * M * es) + up(e_pad * M * es)
+    whole = _native_training_pass(m, x, E, k, Fd, 0.0)
+    if E <= 32 or (dtype == torch.bfloat16 and E <= 256 and M % 64 == 0):
+        bwd = 1 << 40                      # (the gate's own kernels' scratch, which is no matter here)
+    full = [L.lib().mole_gate_route_shape_workspace_bytes(L.dtype_code(dtype), S, E, M, k), L.lib().mole_layer_workspace_bytes(ctypes.byref(whole["block"]), 1)]
+    t = _native_training_pass(m, x, E, k, Fd, 0.0, sizes=(max(ffn, min(fwd, full[0])), min(max(ffn, bwd), full[1])))
+    for name in ("scores", "gates", "idx", "loc", "row", "counts", "kept_rows", "offsets", "capacity", "xd", "h", "a", "out", "y", "dlogits", "dx", "g_w1", "g_b1", "g_w2", "g_b2"):
+        assert torch.equal(t[name], whole[name]), name
+    assert rel_err(t["l_aux"], whole["l_aux"]) < 1e-6
+    if bwd < full[1]:
+        by_tiles = H.gemm_tn(H._pad_cols(t["dlogits"].to(dtype), ep), x)[:E].float()
+        assert torch.equal(t["dwg"], by_tiles) and rel_err(whole["dwg"], by_tiles) < tol(dtype)
+    else:
+        assert torch.equal(t["dwg"], whole["dwg"])

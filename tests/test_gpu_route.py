@@ -73,6 +73,26 @@ def test_route_of_few_tokens_matches_oracle(S, E, k, cf, ragged):
     _compare(zipf_scores(S, E, seed=S + E + k, ties=E > 4), k, cf, ragged)
 
 
+@pytest.mark.parametrize("S,E,k", [(512, 256, 1), (130, 70, 2), (40, 65, 1), (64, 1024, 1), (512, 33, 1)])
+def test_route_with_the_workspace_of_its_histograms(S, E, k):
+    """mole_route does every call with the scratch of blocks of 64 tokens, also where small blocks, which it is asked for, leave more column sums."""
+    from mole_amd import _lib as L, hip_ops as H
+    print(f"route with the least workspace S={S} E={E} k={k}", flush=True)
+    up = lambda n: (n + 255) // 256 * 256
+    nb = (S + 63) // 64
+    least = up(nb * k * E * 4) + up(k * E * 4) + up(nb * E * 4) + up(16 * E * 4)
+    assert least <= L.lib().mole_route_workspace_bytes(S, E, k)
+    scores = zipf_scores(S, E, seed=S + E).cuda()
+    want = H.route(scores, k, 0.5, True, 1, L.LAYOUT_RAGGED)
+    t = {n: torch.full_like(getattr(want, n), -7) for n in ("idx", "loc", "gates", "row", "counts", "kept_rows", "offsets", "capacity", "l_aux")}
+    ws = torch.full((least + 256,), 77, dtype=torch.uint8, device="cuda")
+    L.check(L.lib().mole_route(L.ptr(scores), S, E, k, 0.5, 1, 1, L.LAYOUT_RAGGED, *[L.ptr(v) for v in t.values()], L.ptr(ws), least, L.stream()), "mole_route")
+    torch.cuda.synchronize()
+    assert bool((ws[least:] == 77).all())
+    for n, v in t.items():
+        assert rel_err(v, want.l_aux) < 1e-6 if n == "l_aux" else torch.equal(v, getattr(want, n)), n
+
+
 @pytest.mark.parametrize("S,E", [(100, 8), (513, 16), (64, 100), (300, 256)])
 def test_softmax_and_gate_bwd(S, E):
     from mole_amd import hip_ops as H
