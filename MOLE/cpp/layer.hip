@@ -135,6 +135,7 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
     if (takes == TOKENS_PAIRS && (beside || (long)L->S * L->k > HEAD_PAIRS)) takes = TOKENS_NO;
     if (takes == TOKENS_LIST && ((size_t)L->S * L->M * (L->dtype == MOLE_BF16 ? 2 : 4) >= (size_t)1 << 31 ||
                                  (L->M < 256 && (long)L->S * L->k <= HEAD_PAIRS))) takes = TOKENS_NO;
+    if (takes == TOKENS_LIST && !beside && ((uintptr_t)L->xd & 15) != 0) takes = TOKENS_NO;
     int32_t *const token_of = takes != TOKENS_LIST ? nullptr : beside ? (int32_t *)((char *)L->workspace + up256(route_bytes)) : (int32_t *)L->xd;
     if (int rc = gate_route(L->x, L->dtype, L->wg, L->logit_bias, L->S, L->E, L->M, L->k, L->capacity_factor, L->normalize_gate, 1,
                             L->layout, L->scores, L->idx, L->loc, L->gates, L->row, L->counts, L->kept_rows, L->offsets,

@@ -1113,3 +1113,28 @@ def test_layer_with_the_least_workspaces(S, M, E, k, Fd, dtype):
         assert torch.equal(t["dwg"], by_tiles) and rel_err(whole["dwg"], by_tiles) < tol(dtype)
     else:
         assert torch.equal(t["dwg"], whole["dwg"])
+
+
+@pytest.mark.parametrize("S,k", [(700, 1), (300, 2)])
+def test_forward_only_refuses_rows_off_their_alignment(S, k):
+    """xd is scratch for the routing's list in a pass that nobody asks for the rows, and has to lie on 16 bytes as it has to for the rows."""
+    M, E, Fd = 256, 2, 256
+    print(f"forward only, xd off its alignment S={S} k={k}", flush=True)
+    m, x, _ = _build(S, M, E, k, Fd, torch.bfloat16, seed=S)
+    block = _native_training_pass(m, x, E, k, Fd, 0.0)["block"]
+    # (the pass's buffers are gone; new ones for what this call touches before it is refused, or would)
+    bufs = {n: torch.zeros(c, device="cuda") for n, c in (("scores", S * E), ("gates", k * S), ("l_aux", 1), ("idx", k * S), ("loc", k * S), ("row", k * S), ("counts", k * E),
+                                                          ("kept_rows", E), ("offsets", E + 1), ("capacity", 1), ("xd", S * k * M), ("h", S * k * Fd), ("a", S * k * Fd), ("out", S * k * M))}
+    block.forward_only = 2
+    for n, v in bufs.items():
+        setattr(block, n, v.data_ptr())
+    block.x, block.wg = x.data_ptr(), m.gate[0].linear.weight.data_ptr()
+    block.workspace_bytes = L.lib().mole_layer_workspace_bytes(ctypes.byref(block), 0)
+    ws, y = torch.empty(max(1, block.workspace_bytes), dtype=torch.uint8, device="cuda"), torch.zeros(S, M, dtype=torch.bfloat16, device="cuda")
+    block.workspace = ws.data_ptr()
+    L.check(L.lib().mole_layer_fwd(ctypes.byref(block), L.ptr(y), L.stream()), "mole_layer_fwd")
+    for off in (2, 4, 8):
+        block.xd = bufs["xd"].data_ptr() + off
+        assert L.lib().mole_layer_fwd(ctypes.byref(block), L.ptr(y), L.stream()) == -1
+        assert b"misaligned" in L.lib().mole_last_error_string()
+    torch.cuda.synchronize()
