@@ -16,9 +16,12 @@ namespace mole {
 static int est_rows(const mole_layer &L) { return L.rows < L.S * L.k ? L.rows : L.S * L.k; }
 
 // Whether the first product reads the tokens through the list although their rows are written for later: where the rows of several choices are
-// more than the last-level cache holds and the tokens are well below it.  Training passes, from the rows / from the tokens, us: 30000 tokens,
-// 64 experts top-8, 1000 -> 1000, 4720 / 4585; 32768, 16 top-8, 1024 -> 512, skewed, 3059 / 3040; 20000, 32 top-4, 2048 -> 1024, 2480 / 2459; on the
-// other side of the line, tokens of 134 and 268 MB, 32768, 256 top-8, 2048 -> 1024, 8292 / 8315; 32768, 8 top-2, 4096 -> 2048, 6434 / 6479.
+// more than the last-level cache holds and the tokens are well below it, so that the tokens come from the cache and the rows do not.  Training
+// passes and their first product, from the rows / from the tokens, us (two runs of one side differ by 0.4 % at most): rows of whole lines, 20000
+// tokens, 32 experts top-4, 2048 -> 1024, 2474 / 2442 and 384 / 352; 32768, 64 top-8, 1024 -> 512, 2611 / 2587 and 394 / 359; 32768, 16 top-8, 1024 -> 512,
+// skewed, 3058 / 3035 and 348 / 315; rows that share theirs with others, 30000, 64 top-8, 1000 -> 1000, 4702 / 4568 and 949 / 794; 32768, 16 top-4,
+// 1400 -> 704, 2955 / 2873 and 481 / 386; fp32 16384, 32 top-8, 1008 -> 1008, 10650 / 10619 and 1759 / 1749.  On the other side of the line, tokens of
+// 134 and 268 MB, passes of 32768, 256 top-8, 2048 -> 1024, 8292 / 8315; 32768, 8 top-2, 4096 -> 2048, 6434 / 6479.
 static bool tokens_beside_rows(const mole_layer &L) {
     const size_t width = (size_t)L.M * (L.dtype == MOLE_BF16 ? 2 : 4);
     return L.k >= 2 && est_rows(L) * width >= (size_t)256 << 20 && L.S * width <= (size_t)96 << 20;
@@ -123,11 +126,14 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
     // Where nobody wants xd the first product reads the tokens where they lie: the few-row kernel, which turns the pairs' rows round by
     // itself, up to HEAD_PAIRS; the tiles from a list that the routing leaves in xd's place.  A tile's start then waits for memory once
     // more, about 0.5 us; a dispatch is a launch, writes R M elements and has them read from memory instead of the tokens from the
-    // caches.  Forward passes, dispatched / from the list, us: 61 tokens, 16 experts top-1, 1024 -> 4096, 63.5 / 61.8; 3001, 16 top-2, 1024 ->
-    // 4096, 169.5 / 166.5; 4000, 8 top-2, 4096 -> 2048, 341 / 328; 32768, 64 top-8, 2048 -> 1024, 2640 / 2382; 30000, 64 top-8, 1000 -> 1000, whose
-    // rows share their 128-byte lines, 1712 / 1446; fp32 777, 8 top-2, 520 -> 2048, 102.6 / 100.5; fp32 10000, 16 top-2, 1024 -> 1024, 661 / 641.
-    // Nothing measured lost.  Where tokens_beside_rows, they are read so beside a dispatch, from a list in the workspace.  (Up to HEAD_PAIRS pairs of narrow tokens are dispatched as ever, and the kernels' timings show it: 400 tokens, 64
-    // experts, 136 -> 520, 35.7 / 33.8.  What the dispatch would refuse, and tokens that 32-bit offsets do not reach, are left to it.)
+    // caches.  Forward passes, dispatched / from the list, us: 61 tokens, 16 experts top-1, 1024 -> 4096, 63.5 / 61.8; 3001, 16 top-2,
+    // 1024 -> 4096, 169.5 / 166.5; 4000, 8 top-2, 4096 -> 2048, 341 / 328; 32768, 64 top-8, 2048 -> 1024, 2640 / 2382; 30000, 64 top-8,
+    // 1000 -> 1000, whose rows share their 128-byte lines, 1712 / 1446; fp32 10000, 16 top-2, 1024 -> 1024, 661 / 641.
+    // Where tokens_beside_rows, they are read so beside a dispatch, from a list in the workspace.
+    // Up to HEAD_PAIRS pairs of tokens narrower than 256 keep their dispatch, which test_tokens_in_place_of_dispatched_rows counts, and not for
+    // speed: dispatched / from the list, us, 400 tokens, 64 experts, 136 -> 520, 33.7 / 31.8; 512, 16, 136 -> 544, 30.7 / 28.7; fp32 512, 4, 128 -> 512,
+    // 44.3 / 42.5.
+    // What the dispatch would refuse, and tokens that 32-bit offsets do not reach, are left to it.
     FwdTokens takes = TOKENS_NO;
     const bool beside = !scratch && tokens_beside_rows(*L) && L->workspace_bytes >= up256(route_bytes) + (size_t)L->rows * 4;
     if ((scratch || beside) && L->k >= 1 && L->k <= 16 && ((uintptr_t)L->x & 15) == 0)
