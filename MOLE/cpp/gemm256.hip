@@ -896,15 +896,8 @@ __device__ __forceinline__ void gemm256_block(const GemmArgs &g, const int block
             if (g.accumulate) return;
             typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
             bf16_t *Cz = (bf16_t *)g.C + (long)e * g.strideC + (long)m0 * g.ldc;
-            if (g.ldc == g.N) {
-                const long pieces = (long)min(Q_BM, m_ext - m0) * (g.N >> 3), lo = pieces * nt / n_tiles, hi = pieces * (nt + 1) / n_tiles;
-                for (long u = lo + threadIdx.x; u < hi; u += TL::THREADS) __builtin_nontemporal_store(u32x4{0u, 0u, 0u, 0u}, reinterpret_cast<u32x4 *>(Cz) + u);
-            } else {
-                constexpr int LPR = Q_BN / 8, RPW = WAVE / LPR;        // lanes per row piece, rows per wave and store
-                const int col = n0 + (lane % LPR) * 8;
-                for (int r = wave * RPW + lane / LPR; r < min(Q_BM, m_ext - m0); r += RPW * TL::NW)
-                    if (col < g.N) __builtin_nontemporal_store(u32x4{0u, 0u, 0u, 0u}, reinterpret_cast<u32x4 *>(Cz + (long)r * g.ldc + col));
-            }
+            const long pieces = (long)min(Q_BM, m_ext - m0) * (g.N >> 3), lo = pieces * nt / n_tiles, hi = pieces * (nt + 1) / n_tiles;
+            for (long u = lo + threadIdx.x; u < hi; u += TL::THREADS) __builtin_nontemporal_store(u32x4{0u, 0u, 0u, 0u}, reinterpret_cast<u32x4 *>(Cz) + u);
             if (g.colsum != nullptr) {
                 bf16_t *out = (bf16_t *)g.colsum;
                 const bf16_t z = (bf16_t)0.0f;
@@ -1196,14 +1189,14 @@ int gemm256_ksplit(int E, int est_rows, int N, int K) { return tile_plan(E, est_
 
 // Whether the weight-gradient launch for g will also produce the operand sums asked for in g.colsum.
 bool gemm256_sums_operand(const GemmArgs &g) {
-    if (g.lda % 8 || g.ldb % 8 || g.ldc % 8 || g.N % 8 || g.M % 8) return false;
+    if (g.lda % 8 || g.ldb % 8 || g.ldc != g.N || g.N % 8 || g.M % 8) return false;
     return !sums_off();
 }
 
-// alignment the direct-to-LDS path relies on: 16-byte rows and pieces of K
+// alignment the direct-to-LDS path relies on: 16-byte rows and pieces of K; weight gradients whose rows follow one another
 static bool aligned256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg) {
     if (g.lda % 8 || g.ldb % 8 || g.ldc % 8 || g.N % 8) return false;
-    return wg ? a_ks && b_ks && g.M % 8 == 0 : !a_ks && g.K % 8 == 0;
+    return wg ? a_ks && b_ks && g.M % 8 == 0 && g.ldc == g.N : !a_ks && g.K % 8 == 0;
 }
 // the tile of a row-ragged product; where its contraction is split, gp and epi become those of the planes
 static int plan256(GemmArgs &gp, bool b_ks, int &epi, int max_rows, void *ws, size_t ws_bytes) {

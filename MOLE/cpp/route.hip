@@ -457,11 +457,12 @@ __global__ __launch_bounds__(256) void route_finalize_kernel(const RouteEnd r, c
 }
 
 // ---- the tokens' own part ------------------------------------------------------------------------------------------
-// A block of THREADS takes THREADS / 16 tokens.  2^LOGG lanes own a token and hold VPL scores each (lane g: experts g, g + G, ...); with
-// 16 lanes per token all the block's tokens go through their rounds at once.  64 tokens a block where there are many (four waves on 64 tokens, 16 tokens a wave, four at a
-// time, spent four times the latency of a round: 256 experts, top-8: 42 us for 256 tokens and 58 for 32768, now 21 and 45).  Few tokens
-// leave the other CUs idle that way, while the rounds of a block's 16 waves share the four SIMDs of one: they take blocks of four waves
-// and 16 tokens, or, beyond 64 experts, of four tokens with a wave each (256 experts, top-8, 256 tokens: 21 -> 7.8 us).
+// A block of THREADS takes TOK tokens.  2^LOGG lanes own a token and hold VPL scores each (lane g: experts g, g + G, ...); with 16 lanes per token
+// all the block's tokens go through their rounds at once, with a wave per token THREADS / 64 of them.  64 tokens
+// a block where there are many (four waves on 64 tokens, 16 tokens a wave, four at a time, spent four times the latency of a round: 256 experts,
+// top-8: 42 us for 256 tokens and 58 for 32768, now 21 and 45).  Few tokens leave the other CUs idle that way, while the rounds of a block's 16
+// waves share the four SIMDs of one: they take blocks of four waves and 16 tokens, or, beyond 64 experts, of four tokens with a wave each (256
+// experts, top-8, 256 tokens: 21 -> 7.8 us).
 // logits != 0: `in` holds logits (without bias if one is given) and the block starts with the softmax (the sums in the order of gate_fwd_kernel's), writing
 // scores; LOGITS_PARTS / LOGITS_PAIRS: `in` holds four partial sums of them, [4][S][E], to be added one after the other / in pairs.
 // nb == 1: the block has seen all tokens and goes on to the end of the routing by itself.  hist null: route_rank takes it
