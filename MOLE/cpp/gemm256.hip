@@ -17,6 +17,7 @@
 // as whole 128-byte rows.  A ragged m-tile runs only the 32-row blocks it has rows for.
 #include "gemm.h"
 #include "lds_dma.h"
+#include "mole_hip_probe.h"
 #include "wgrad_few.h"
 
 #include <stdlib.h>
@@ -1259,3 +1260,5 @@ int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, in
 }
 
 }  // namespace mole
+
+extern "C" int mole_probe_wgrad_tile(int E, int est_rows, int M, int N) { return mole::wgrad_tile(E, est_rows, M, N) == mole::TILE_128 ? 128 : 256; }

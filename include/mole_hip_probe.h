@@ -28,6 +28,9 @@ int mole_probe_kloop(const void *a, const void *b, const int32_t *offsets, const
 int mole_probe_kloop_part(const void *a, const void *b, const int32_t *offsets, const int32_t *kept_rows, int E,
                           int max_rows, int N, int K, int part, float *sink, mole_stream_t stream);
 
+/* mole_probe_wgrad_tile: columns of the bf16 tile that the weight gradients [M,N] of E experts, est_rows rows together, take (128 or 256). */
+int mole_probe_wgrad_tile(int E, int est_rows, int M, int N);
+
 #ifdef __cplusplus
 }
 #endif

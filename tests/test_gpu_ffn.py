@@ -555,18 +555,19 @@ def test_ffn_backward_products_in_pairs(E, M, Fd, rows, gap, accumulate):
     assert all(torch.equal(x, y) for x, y in zip(*res))
 
 
-# K-strided weights read past the caches, in a forward pass that no backward follows: from 64 MB of weights of the experts that
-# can have rows, the recorded pass (256 MB) taking the ordinary loads.  Experts of a few rows on the kernel for them, of up
-# to 64 and up to 128 on the tiles, of more (ordinary loads there), and of none.  The loads' cache policy changes no result.
+# Weight gradients of experts with a few rows, on both tiles (every wave by itself: 128 columns by 32 rows of a 128 x 128 tile, by 64 of a 256 x 256 one).
 @pytest.mark.parametrize("accumulate", [False, True])
-@pytest.mark.parametrize("E,M,Fd,rows,gap", [
-    (6, 136, 264, [1, 31, 32, 33, 0, 8], 0),                # one and two steps of rows, 128-wide tiles that end in the middle
-    (4, 264, 136, [64, 63, 65, 2], 3),                      # both sides of the limit in one launch
-    (3, 8, 16, [5, 0, 64], 0),                              # less than a lane's columns on one side
-    (40, 520, 1032, [40] * 38 + [64, 0], 0),                # 256-wide tiles
-    (40, 512, 1024, [33 + e % 32 for e in range(39)] + [700], 0),
+@pytest.mark.parametrize("E,M,Fd,rows,gap,tile", [
+    (6, 136, 264, [1, 31, 32, 33, 0, 8], 0, 128),           # one and two steps of rows, tiles that end in the middle
+    (4, 264, 136, [64, 63, 65, 2], 3, 128),                 # both sides of the limit in one launch
+    (3, 8, 16, [5, 0, 64], 0, 128),                         # less than a lane's columns on one side
+    (40, 520, 1032, [40] * 38 + [64, 0], 0, 128),           # many tiles
+    (40, 512, 1024, [33 + e % 32 for e in range(39)] + [700], 0, 128),
+    (64, 520, 1000, [1, 31, 32, 33, 63, 64, 65, 0] * 8, 0, 256),        # tiles that end in the middle on both sides
+    (64, 1000, 520, [40, 64, 0, 65, 1, 8, 33, 90] * 8, 1, 256),
+    (64, 512, 1024, [48] * 63 + [0], 0, 256),               # whole tiles
 ])
-def test_ffn_weight_gradients_of_few_rows(E, M, Fd, rows, gap, accumulate):
+def test_ffn_weight_gradients_of_few_rows(E, M, Fd, rows, gap, tile, accumulate):
     """Experts of up to 64 rows, whose weight gradients are formed without the operand ring: sums of bf16 products in fp32 (64
     terms: 64 x 2^-24 of the terms' size) and one rounding to bf16, 2^-9 of the result, two where it is added to what is there."""
     from mole_amd import hip_ops as H, _lib as L
@@ -575,6 +576,7 @@ def test_ffn_weight_gradients_of_few_rows(E, M, Fd, rows, gap, accumulate):
     c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
     off = torch.from_numpy(d["off"]).cuda(); n = torch.from_numpy(d["n"]).cuda()
     R = max(d["R"], 1)
+    assert L.lib().mole_probe_wgrad_tile(E, R, Fd, M) == tile
     h = torch.randn(R, Fd, generator=torch.Generator().manual_seed(3)).bfloat16().cuda()
     a = torch.nn.functional.gelu(h.float()).bfloat16()
     t = torch.zeros(R, Fd, dtype=torch.bfloat16, device="cuda")
@@ -593,6 +595,9 @@ def test_ffn_weight_gradients_of_few_rows(E, M, Fd, rows, gap, accumulate):
             assert bool(((got[e].double().cpu() - w).abs() <= bound).all())
 
 
+# K-strided weights read past the caches, in a forward pass that no backward follows: from 64 MB of weights of the experts that
+# can have rows, the recorded pass (256 MB) taking the ordinary loads.  Experts of a few rows on the kernel for them, of up
+# to 64 and up to 128 on the tiles, of more (ordinary loads there), and of none.  The loads' cache policy changes no result.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("E,M,Fd,k,S", [
     (40, 1024, 1024, 1, 61), (40, 1024, 1024, 2, 120), (23, 512, 3264, 2, 33),      # few rows; the last of 67 / 134 MB

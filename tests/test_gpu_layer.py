@@ -13,6 +13,16 @@ from tests.util import expert_rel_err, rel_err, row_rel_err, tol
 pytestmark = pytest.mark.gpu
 
 
+class _Grads(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("accumulate", "gelu_bwd")] + [(n, ctypes.c_void_p) for n in "dy d_l_aux dlogits d_o t gxd g_w1 g_b1 g_w2 g_b2 dx dwg".split()]
+
+
+class _Layer(ctypes.Structure):
+    _fields_ = ([(n, ctypes.c_int32) for n in "dtype S M E k F rows layout normalize_gate forward_only".split()] + [("capacity_factor", ctypes.c_double)] +
+                [(n, ctypes.c_void_p) for n in "x wg logit_bias w1 b1 w2 b2 scores gates l_aux idx loc row counts kept_rows offsets capacity "
+                                               "xd h a out workspace".split()] + [("workspace_bytes", ctypes.c_size_t)])
+
+
 def _build(S, M, E, k, Fd, dtype, d_experts=0, pool=0, ebatch=4, seed=0, acc_step=1, adv_adam=False, **kw):
     from mole_amd.moe.layer import MOLEModule
     MOLEModule.reset_instances()
@@ -629,15 +639,18 @@ def test_forward_without_autograd_gives_the_same_bits(S, M, E, k, Fd, dtype):
 # Tiles that read the tokens where they lie instead of dispatched rows, by every routing kernel that lists the rows' tokens:
 # one block of tokens, the ranking block, the finishing block with and without its last stage, the gate's own top-k; tiles of 64 to 256 rows,
 # one row to whole tiles an expert, contractions that end inside a stage, dropped pairs, experts without rows, numbers that fp32 parts do not hold.
-@pytest.mark.parametrize("S,M,E,k,Fd,cf,dtype,scale", [
-    (64, 1024, 4, 1, 256, 0.0, torch.bfloat16, 1.0), (64, 520, 2, 2, 264, 1.0, torch.bfloat16, 1.0),
-    (257, 256, 40, 4, 128, 0.5, torch.bfloat16, 1.0), (3001, 256, 16, 2, 2048, 0.0, torch.bfloat16, 1.0),
-    (5003, 136, 70, 2, 1032, 1.25, torch.bfloat16, 1.0), (20001, 128, 9, 3, 256, 0.0, torch.bfloat16, 1.0), (1100, 64, 600, 8, 64, 0.0, torch.bfloat16, 1.0),
-    (700, 128, 300, 8, 64, 2.0, torch.float32, 1.0), (777, 512, 8, 2, 256, 1.0, torch.float32, 1.0), (9001, 144, 8, 1, 260, 0.5, torch.float32, 1.0),
-    (33000, 1024, 8, 4, 16, 0.0, torch.bfloat16, 1.0), (17000, 1024, 8, 4, 16, 0.0, torch.float32, 1.0),      # (more rows than a cache holds)
-    (777, 128, 8, 2, 256, 0.0, torch.float32, 1e-36), (4500, 256, 4, 2, 512, 0.0, torch.float32, 1e-36)])
+# (listed: not 0, the passes without a backward have no dispatch, and 2, the recorded one lists its rows' tokens beside one; 0, the few-row kernel
+# has the product, whose rows are dispatched beyond 512 pairs)
+@pytest.mark.parametrize("S,M,E,k,Fd,cf,dtype,scale,listed", [
+    (64, 1024, 4, 1, 256, 0.0, torch.bfloat16, 1.0, 1), (64, 520, 2, 2, 264, 1.0, torch.bfloat16, 1.0, 1), (64, 256, 16, 16, 128, 0.0, torch.bfloat16, 1.0, 1),
+    (257, 256, 40, 4, 128, 0.5, torch.bfloat16, 1.0, 0), (512, 256, 12, 4, 128, 0.5, torch.bfloat16, 1.0, 1), (3001, 256, 16, 2, 2048, 0.0, torch.bfloat16, 1.0, 1),
+    (5003, 136, 70, 2, 1032, 1.25, torch.bfloat16, 1.0, 1), (20001, 128, 9, 3, 256, 0.0, torch.bfloat16, 1.0, 1), (1100, 64, 600, 8, 64, 0.0, torch.bfloat16, 1.0, 1),
+    (700, 128, 300, 8, 64, 2.0, torch.float32, 1.0, 0), (4000, 128, 300, 8, 64, 2.0, torch.float32, 1.0, 1), (777, 512, 8, 2, 256, 1.0, torch.float32, 1.0, 1),
+    (9001, 144, 8, 1, 260, 0.5, torch.float32, 1.0, 1),
+    (33000, 1024, 8, 4, 16, 0.0, torch.bfloat16, 1.0, 2), (17000, 1024, 8, 4, 16, 0.0, torch.float32, 1.0, 2),      # (more rows than a cache holds)
+    (777, 128, 8, 2, 256, 0.0, torch.float32, 1e-36, 1), (4500, 256, 4, 2, 512, 0.0, torch.float32, 1e-36, 1)])
 @pytest.mark.parametrize("padded", [False, True])
-def test_forward_from_the_tokens_gives_the_bits_of_dispatched_rows(S, M, E, k, Fd, cf, dtype, scale, padded):
+def test_forward_from_the_tokens_gives_the_bits_of_dispatched_rows(S, M, E, k, Fd, cf, dtype, scale, listed, padded):
     from mole_amd import hip_ops as H
     if padded and cf == 0.0:
         cf = 1.25
@@ -646,8 +659,18 @@ def test_forward_from_the_tokens_gives_the_bits_of_dispatched_rows(S, M, E, k, F
     x = (x.detach() * scale).requires_grad_(True)
     y = m(x, capacity_factor=cf).detach()
     with torch.no_grad():
+        L.kernel_timing_enable(True)
+        L.kernel_timing_read()
         for _ in range(2):
             assert torch.equal(m(x, capacity_factor=cf), y)
+        dispatches = L.kernel_timing_read()["dispatch_fwd"][0]
+        L.kernel_timing_enable(False)
+        assert dispatches == (0 if listed else 2)
+        if not padded:                     # (the list of a recorded pass has its room behind the routing's scratch)
+            block = _Layer(L.dtype_code(dtype), S, M, E, k, Fd, S * k, L.LAYOUT_RAGGED, 1, 0, cf)
+            route, ffn = L.lib().mole_gate_route_shape_workspace_bytes(block.dtype, S, E, M, k), L.lib().mole_ffn_workspace_bytes(block.dtype, E, S * k, M, Fd)
+            want = max(ffn, (route + 255) // 256 * 256 + 4 * S * k if listed == 2 else route)
+            assert L.lib().mole_layer_workspace_bytes(ctypes.byref(block), 0) == want > (max(ffn, route) if listed == 2 else 0)
         r = m.last_route
         xd = H.dispatch_fwd(x, r.row, int(r.offsets[-1]))
         out, _, _ = H.ffn_fwd(xd, r.offsets, r.kept_rows, m.FC1_W_GPU.all_tensors, m.FC1_B_GPU.all_tensors,
@@ -998,16 +1021,6 @@ def test_native_forward_only_fills_xd_and_out(S, M, E, k, Fd, cf, dtype):
     for name in ("xd", "out"):
         assert torch.equal(t1[name][kept], t0[name][kept])
     assert torch.equal(t1["xd"][kept], H.dispatch_fwd(x, t1["row"], rows)[kept])
-
-
-class _Grads(ctypes.Structure):
-    _fields_ = [(n, ctypes.c_int32) for n in ("accumulate", "gelu_bwd")] + [(n, ctypes.c_void_p) for n in "dy d_l_aux dlogits d_o t gxd g_w1 g_b1 g_w2 g_b2 dx dwg".split()]
-
-
-class _Layer(ctypes.Structure):
-    _fields_ = ([(n, ctypes.c_int32) for n in "dtype S M E k F rows layout normalize_gate forward_only".split()] + [("capacity_factor", ctypes.c_double)] +
-                [(n, ctypes.c_void_p) for n in "x wg logit_bias w1 b1 w2 b2 scores gates l_aux idx loc row counts kept_rows offsets capacity "
-                                               "xd h a out workspace".split()] + [("workspace_bytes", ctypes.c_size_t)])
 
 
 def _native_training_pass(m, x, E, k, Fd, cf, dwg=None, sizes=None):
