@@ -60,16 +60,16 @@ const char *mole_last_error_string(void);
 enum {
     MOLE_K_FFN_FWD1 = 0,  /* h = xd.w1^T + b1, a = gelu(h) */
     MOLE_K_FFN_FWD2 = 1,  /* out = a.w2 + b2 */
-    MOLE_K_FFN_GW2 = 2,   /* g_w2 = a^T.go */
-    MOLE_K_FFN_DA = 3,    /* t = (go.w2^T) * gelu'(h) */
-    MOLE_K_FFN_GW1 = 4,   /* g_w1 = t^T.xd */
-    MOLE_K_FFN_GX = 5,    /* gx = t.w1 */
+    MOLE_K_FFN_GW2 = 2,   /* g_w2 = a^T.go; no launch of its own where it runs beside t (small bf16 layers) */
+    MOLE_K_FFN_DA = 3,    /* t = (go.w2^T) * gelu'(h), there together with g_w2: the time is that of both products */
+    MOLE_K_FFN_GW1 = 4,   /* g_w1 = t^T.xd; no launch of its own where it runs beside gx */
+    MOLE_K_FFN_GX = 5,    /* gx = t.w1, there together with g_w1 */
     MOLE_K_FFN_GB = 6,    /* bias gradients */
     MOLE_K_DISPATCH_FWD = 7,
     MOLE_K_DISPATCH_BWD = 8,
     MOLE_K_COMBINE_FWD = 9,
     MOLE_K_COMBINE_BWD = 10,
-    MOLE_K_ROUTE = 11,    /* the four routing kernels together */
+    MOLE_K_ROUTE = 11,    /* the routing kernels together */
     MOLE_K_GEMM_NT = 12,
     MOLE_K_ADAM = 13,
     MOLE_K_GATE_FWD = 14,   /* gate logits + softmax in one kernel, or the softmax kernel alone */
