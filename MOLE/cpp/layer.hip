@@ -153,8 +153,9 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
     // (what the combine would refuse is left to it)
     CombineTail tail{L->row, L->idx, L->gates, y, L->S, L->k, !scratch, false};
     const bool tail_ok = y != nullptr && ((uintptr_t)y & 15) == 0 && L->k >= 1 && L->k <= 16;
-    if (int rc = ffn_fwd(head_ok ? L->x : L->xd, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, est_rows(*L), L->M, L->F, L->w1, L->b1, L->w2, L->b2, L->h,
-                                 L->a, L->out, L->workspace, L->workspace_bytes, L->forward_only, head_ok ? &head : nullptr, tail_ok ? &tail : nullptr, (hipStream_t)stream)) return rc;
+    if (int rc = ffn_fwd(head_ok ? L->x : L->xd, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, est_rows(*L), L->M, L->F, L->w1, L->b1, L->w2,
+                         L->b2, L->h, L->a, L->out, L->workspace, L->workspace_bytes, L->forward_only, head_ok ? &head : nullptr,
+                         tail_ok ? &tail : nullptr, (hipStream_t)stream)) return rc;
     if (tail.done) return 0;
     return mole_combine_fwd(L->out, L->dtype, L->row, L->gates, L->S, L->M, L->k, y, stream);
 }
@@ -163,8 +164,9 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
     if (int rc = check_layer("mole_layer_bwd", L, stream)) return rc;
     MOLE_REQUIRE(!L->forward_only, "mole_layer_bwd: the forward pass was a forward_only one");
     MOLE_REQUIRE(G && G->dy && G->dlogits && G->d_o && G->t && G->gxd && G->dx && G->dwg, "mole_layer_bwd: null gradient pointer");
-    const size_t need = mole_layer_workspace_bytes(L, 1), ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
+    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
     GateBwdPlan p = gate_bwd_plan(*L, gate_wgrad_by_tiles(*L));
+    const size_t need = std::max(ffn, p.total);
     // (a workspace that does not hold the partial sums of a large gate has its weight gradient by the tiles)
     if (L->workspace_bytes < need && gate_wgrad_may_go_by_tiles(*L)) p = gate_bwd_plan(*L, true);
     if (L->workspace_bytes < std::max(ffn, p.total)) {

@@ -1146,7 +1146,8 @@ static int launch_fold(const void *dxd, const int32_t *row, int S, int M, int k,
     const int tok = (long)ceil_div(S, DM_TOKENS) * ceil_div(M, 8 * DM_COLS) < DM_FEW_BLOCKS ? DM_TOKENS_FEW : DM_TOKENS;
     const dim3 grid(ceil_div(S, tok), ceil_div(M, 8 * DM_COLS));
     const bool e8 = E % 8 == 0 && ((uintptr_t)dlogits & 15) == 0;
-#define MOLE_DM_(E8, TOK, MORE) timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_mfma_kernel<E8, TOK, SPLIT, NH, MORE>, grid, dim3(512), 0, st, (const bf16_t *)dxd, row, S, M, k, dlogits, wg, E, (bf16_t *)dx)
+#define MOLE_DM_(E8, TOK, MORE) timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_mfma_kernel<E8, TOK, SPLIT, NH, MORE>, grid, dim3(512), 0, st, \
+                                             (const bf16_t *)dxd, row, S, M, k, dlogits, wg, E, (bf16_t *)dx)
 #define MOLE_DM(E8, TOK) do { if (k > 1) MOLE_DM_(E8, TOK, true); else MOLE_DM_(E8, TOK, false); } while (0)
     if (tok == DM_TOKENS) { if (e8) MOLE_DM(true, DM_TOKENS); else MOLE_DM(false, DM_TOKENS); }
     else { if (e8) MOLE_DM(true, DM_TOKENS_FEW); else MOLE_DM(false, DM_TOKENS_FEW); }
@@ -1158,7 +1159,8 @@ static int launch_fold(const void *dxd, const int32_t *row, int S, int M, int k,
 bool dispatch_bwd_folds(int dtype, int E) { return dtype == MOLE_BF16 && E <= 64; }
 int dispatch_bwd_fold(const void *dxd, const int32_t *row, int S, int M, int k, const float *dlogits, const float *wg, int E, void *dx, hipStream_t st) {
     if (int rc = check_perm("mole_dispatch_bwd", MOLE_BF16, S, M, k)) return rc;
-    MOLE_REQUIRE(dxd && row && dx && dlogits && aligned16(dxd) && aligned16(dx) && wg && dispatch_bwd_folds(MOLE_BF16, E), "mole_dispatch_bwd: null or misaligned pointer");
+    MOLE_REQUIRE(dxd && row && dx && dlogits && aligned16(dxd) && aligned16(dx) && wg && dispatch_bwd_folds(MOLE_BF16, E),
+                 "mole_dispatch_bwd: null or misaligned pointer");
     return launch_fold<false, 2>(dxd, row, S, M, k, dlogits, wg, E, dx, st);
 }
 }  // namespace mole
