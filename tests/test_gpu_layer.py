@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 
 class _Grads(ctypes.Structure):
-    _fields_ = [(n, ctypes.c_int32) for n in ("accumulate", "gelu_bwd")] + [(n, ctypes.c_void_p) for n in "dy d_l_aux dlogits d_o t gxd g_w1 g_b1 g_w2 g_b2 dx dwg".split()]
+    _fields_ = ([(n, ctypes.c_int32) for n in ("accumulate", "gelu_bwd")] +
+                [(n, ctypes.c_void_p) for n in "dy d_l_aux dlogits d_o t gxd g_w1 g_b1 g_w2 g_b2 dx dwg".split()])
 
 
 class _Layer(ctypes.Structure):
@@ -1057,7 +1058,8 @@ def _native_training_pass(m, x, E, k, Fd, cf, dwg=None, sizes=None):
 
 # Where the dispatch's backward takes the gate's input gradient in, the sum is that of the two entry points, bit for bit: the product from
 # bf16 operands, rounded to bf16, behind the rows.  One 32 of experts and a rest, whole and broken pieces of columns, dropped pairs.
-@pytest.mark.parametrize("S,M,E,k,Fd,cf", [(300, 1024, 40, 2, 64, 0.0), (3000, 1000, 64, 4, 64, 0.0), (8, 1024, 64, 1, 64, 0.0), (515, 136, 57, 8, 16, 0.5), (9000, 256, 33, 1, 16, 1.0)])
+@pytest.mark.parametrize("S,M,E,k,Fd,cf", [(300, 1024, 40, 2, 64, 0.0), (3000, 1000, 64, 4, 64, 0.0), (8, 1024, 64, 1, 64, 0.0), (515, 136, 57, 8, 16, 0.5),
+                                           (9000, 256, 33, 1, 16, 1.0)])
 def test_input_gradient_of_a_gate_of_up_to_64_is_that_of_its_product(S, M, E, k, Fd, cf):
     from mole_amd import hip_ops as H
     print(f"input gradient of a gate of up to 64 S={S} M={M} E={E} k={k} F={Fd} cf={cf}", flush=True)
@@ -1084,8 +1086,9 @@ def test_gate_weight_gradient_at_any_alignment(S, M, E, k, Fd, dtype):
 
 # Both sides of the line between the two ways of a large gate's weight gradient: by tiles beyond it, bit for bit what mole_gemm_tn gives from
 # operands in the tokens' type; before it fp32 sums of at most 16 x 128 tokens a chunk and 16 chunks (2^-24 of the terms' size a step of either).
-@pytest.mark.parametrize("S,M,E,Fd,dtype,tiles", [(1030, 2192, 300, 8, torch.bfloat16, True), (1030, 2184, 300, 8, torch.bfloat16, False), (1024, 2192, 300, 8, torch.bfloat16, False),
-                                                  (1100, 10248, 64, 8, torch.bfloat16, True), (130, 2100, 1000, 4, torch.float32, True), (130, 2096, 1000, 4, torch.float32, False)])
+@pytest.mark.parametrize("S,M,E,Fd,dtype,tiles", [
+    (1030, 2192, 300, 8, torch.bfloat16, True), (1030, 2184, 300, 8, torch.bfloat16, False), (1024, 2192, 300, 8, torch.bfloat16, False),
+    (1100, 10248, 64, 8, torch.bfloat16, True), (130, 2100, 1000, 4, torch.float32, True), (130, 2096, 1000, 4, torch.float32, False)])
 def test_gate_weight_gradient_on_either_side_of_the_tiles(S, M, E, Fd, dtype, tiles):
     from mole_amd import hip_ops as H
     print(f"gate weight gradient, tiles={tiles} S={S} M={M} E={E} F={Fd} {dtype}", flush=True)
@@ -1118,7 +1121,7 @@ def test_layer_with_the_least_workspaces(S, M, E, k, Fd, dtype):
         bwd = 1 << 40                      # (the gate's own kernels' scratch, which is no matter here)
     full = [L.lib().mole_gate_route_shape_workspace_bytes(L.dtype_code(dtype), S, E, M, k), L.lib().mole_layer_workspace_bytes(ctypes.byref(whole["block"]), 1)]
     t = _native_training_pass(m, x, E, k, Fd, 0.0, sizes=(max(ffn, min(fwd, full[0])), min(max(ffn, bwd), full[1])))
-    for name in ("scores", "gates", "idx", "loc", "row", "counts", "kept_rows", "offsets", "capacity", "xd", "h", "a", "out", "y", "dlogits", "dx", "g_w1", "g_b1", "g_w2", "g_b2"):
+    for name in "scores gates idx loc row counts kept_rows offsets capacity xd h a out y dlogits dx g_w1 g_b1 g_w2 g_b2".split():
         assert torch.equal(t[name], whole[name]), name
     assert rel_err(t["l_aux"], whole["l_aux"]) < 1e-6
     if bwd < full[1]:
@@ -1136,8 +1139,9 @@ def test_forward_only_refuses_rows_off_their_alignment(S, k):
     m, x, _ = _build(S, M, E, k, Fd, torch.bfloat16, seed=S)
     block = _native_training_pass(m, x, E, k, Fd, 0.0)["block"]
     # (the pass's buffers are gone; new ones for what this call touches before it is refused, or would)
-    bufs = {n: torch.zeros(c, device="cuda") for n, c in (("scores", S * E), ("gates", k * S), ("l_aux", 1), ("idx", k * S), ("loc", k * S), ("row", k * S), ("counts", k * E),
-                                                          ("kept_rows", E), ("offsets", E + 1), ("capacity", 1), ("xd", S * k * M), ("h", S * k * Fd), ("a", S * k * Fd), ("out", S * k * M))}
+    sizes = dict(scores=S * E, gates=k * S, l_aux=1, idx=k * S, loc=k * S, row=k * S, counts=k * E, kept_rows=E, offsets=E + 1, capacity=1,
+                 xd=S * k * M, h=S * k * Fd, a=S * k * Fd, out=S * k * M)
+    bufs = {n: torch.zeros(c, device="cuda") for n, c in sizes.items()}
     block.forward_only = 2
     for n, v in bufs.items():
         setattr(block, n, v.data_ptr())
