@@ -72,7 +72,7 @@ template <int TMB, int WM, int WN, bool M_KS, int TMC> struct Stage {
 // A stage holds 32 of K.  Every lane always issues its load (no divergent branches in the K loop):
 // rows past the operand's extent are clamped to the last valid row / 16-byte piece.  What lands in
 // LDS for them is real, finite data that only contributes to output rows or columns the epilogue
-// does not store - except along a ragged contraction length, which zero_k_tail() repairs.
+// does not store - except along a ragged contraction length, which the zero_*_tail functions repair.
 //
 // K-contiguous operand, element (r, k) at p[r*ld + k]: LDS [ROWS][4 x 16 B], the chunk index XORed
 // with swz16(row).  A fragment read has lane l at row l % 16, chunk l / 16; one pass of ds_read_b128 serves 16 lanes, either
@@ -81,8 +81,7 @@ template <int TMB, int WM, int WN, bool M_KS, int TMC> struct Stage {
 // With NW waves, wave w's load i fills LDS bytes [(NW i + w)*1024, +1024) = rows 16(NW i + w) .. +16.
 // Per-lane byte offsets of the ROWS/(16 NW) loads a wave issues for one stage of an operand tile, relative to
 // the tile's first element at the stage's first k (what the scalar base points at).  r_left = rows of the
-// operand from the tile's first row on, k_left = k-rows from the stage's first k on (only the last stage
-// of a ragged contraction has fewer than 32).
+// operand from the tile's first row on, k_left = k of the stage (only stage 0 of a ragged contraction has fewer than 32).
 __device__ __forceinline__ int swz16(int row) { return ((row >> 3) & 1) | (((row >> 1) ^ (row >> 2)) & 2); }
 // src: the operand's rows are those of a matrix of n_src rows that src names, and the base is that matrix (null: they lie there in order).
 template <int ROWS, int NW> struct OffKC {
@@ -132,7 +131,7 @@ template <int ROWS, int THREADS> __device__ __forceinline__ void zero_kc_tail(ch
         if (c * 8 >= k_valid) *reinterpret_cast<uint4 *>(lds + row * 64 + ((c ^ swz16(row)) << 4)) = make_uint4(0, 0, 0, 0);
     }
 }
-// zero the k-rows [k_valid, 32) of a K-strided tile (the last, partial stage of a ragged contraction)
+// zero the k-rows [k_valid, 32) of a K-strided tile
 template <int ROWS, int THREADS> __device__ __forceinline__ void zero_k_tail(char *lds, int k_valid) {
     for (int idx = threadIdx.x; idx < (Q_BK - k_valid) * (ROWS / 8); idx += THREADS)
         *reinterpret_cast<uint4 *>(lds + k_valid * (ROWS * 2) + idx * 16) = make_uint4(0, 0, 0, 0);
@@ -229,31 +228,33 @@ template <int TMB, int WM, int WN, bool M_KS, bool N_KS, int TMC, int TMCW> stru
 
 // Issues the asynchronous loads of the operand stages of one tile.  The two operand tiles are addressed
 // by a scalar base (advanced by one stage of K after a stage's last load) plus per-lane offsets that stay
-// fixed for the whole K loop.  Stages are fetched in order; past the last one the last is fetched again,
-// harmlessly: it keeps the number of loads per stage, which the vmcnt arithmetic of the loop relies on.
+// fixed for the whole K loop.  Stages are fetched in order.
 // Of a K-contiguous m-side tile only the 64-row groups that hold live 32-row blocks (the first TMC) are fetched.
-// KT: the contraction may end inside a stage (weight gradients always may; row-ragged products when K is not a multiple of
-// 32).  The last stage's loads are then clamped to what exists and main_loop zeroes what lies past it.
+// KT: the contraction may not be whole stages (weight gradients; row-ragged products when K is not a multiple of 32).  What is
+// left over at its end comes first, as stage 0, whose loads are clamped to what exists and of which main_loop zeroes the rest; the
+// loop then meets whole stages only.  As the last stage it had every iteration choose between two sets of offsets and ask
+// whether its stage was that one, 47 ns of a stage's 230 on 128 x 128 tiles.  us, left over last / first: weight gradients, 64
+// experts of 1024 x 2048, 100 rows, 78.8 / 73.4, 200 rows 98 / 95, 500 rows 167 / 164; 16 of 1024 x 4096, 500 rows, 80.1 / 78.0;
+// 59 of 568 x 2272, 100 rows, 53.0 / 50.4; out of 128 rows, 16 experts of 1408 -> 512 by the kernel for any K, 17.3 / 15.2.
 // ONCE: no other tile reads this tile's n-side panel (the weights of an expert with a single m-tile).
 template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC, bool ONCE> struct Feeder {
     typedef Tile<TMB, WM, WN> TL;
     typedef Stage<TMB, WM, WN, M_KS, TMC> SG;
     static constexpr int LM = SG::LM, L = SG::L;
-    Off<TL::M_ROWS, TL::NW, M_KS> om, cm;
+    Off<TL::M_ROWS, TL::NW, M_KS> om, cm;      // cm, cn: of stage 0
     Off<TL::BN, TL::NW, N_KS> on, cn;
     const char *bm, *bn;
     long step_m, step_n;
     uint32_t lds_w;      // LDS address of ring buffer 0 + this wave's 1 KiB lane
-    int nk;
-    bool ragged_k;
+    int nk, left;        // stages; k of stage 0 where that is not a whole one, otherwise 0
     __device__ __forceinline__ void init(const bf16_t *Mp, long ldm, int m0, int m_ext, const bf16_t *Np, long ldn, int n0,
                                          int n_ext, int k_ext, char *smem, int wave, const int32_t *src, int n_src) {
         om.init(ldm, m_ext - m0, Q_BK, src, n_src);
         on.init(ldn, n_ext - n0, Q_BK, nullptr, 0);
-        ragged_k = KT && (k_ext & (Q_BK - 1));
-        if constexpr (KT) {   // last stage of a ragged contraction: k past the end is clamped to the last k-row / 16-byte piece
-            cm.init(ldm, m_ext - m0, ragged_k ? (k_ext & (Q_BK - 1)) : Q_BK, src, n_src);
-            cn.init(ldn, n_ext - n0, ragged_k ? (k_ext & (Q_BK - 1)) : Q_BK, nullptr, 0);
+        left = KT ? k_ext & (Q_BK - 1) : 0;
+        if constexpr (KT) {   // k past the end is clamped to the last k-row / 16-byte piece
+            cm.init(ldm, m_ext - m0, left ? left : Q_BK, src, n_src);
+            cn.init(ldn, n_ext - n0, left ? left : Q_BK, nullptr, 0);
         }
         bm = uniform_ptr(src != nullptr ? Mp : M_KS ? Mp + m0 : Mp + (long)m0 * ldm);
         bn = uniform_ptr(N_KS ? Np + n0 : Np + (long)n0 * ldn);
@@ -262,23 +263,30 @@ template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC, bool 
         lds_w = lds_offset_of(smem) + __builtin_amdgcn_readfirstlane(wave * 1024);
         nk = (k_ext + Q_BK - 1) / Q_BK;
     }
-    // loads [J0, J1) of stage s (the m-side tile's loads come first) into ring buffer buf
+    __device__ __forceinline__ void load(int j, uint32_t o, uint32_t dst) const {
+        if (j < LM) dma16s(bm, o, dst + j * (TL::NW * 1024));
+        else if constexpr (ONCE) dma16s_nt(bn, o, dst + SG::M_OPERAND + (j - LM) * (TL::NW * 1024));
+        else dma16s(bn, o, dst + SG::M_OPERAND + (j - LM) * (TL::NW * 1024));
+    }
+    // the loads of stage 0, into ring buffer 0
+    __device__ __forceinline__ void issue_first() {
+        if constexpr (!KT) return issue<0, L>(0, 0);
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_w);
+        const long ahead = left ? nk - 1 : 0;         // stages before what is left over
+        bm += ahead * step_m;
+        bn += ahead * step_n;
+#pragma unroll
+        for (int j = 0; j < L; ++j) load(j, j < LM ? cm.off[j < LM ? j : 0] : cn.off[j < LM ? 0 : j - LM], dst);
+        if (nk > 1) {
+            bm += (left ? -ahead : 1) * step_m;
+            bn += (left ? -ahead : 1) * step_n;
+        }
+    }
+    // loads [J0, J1) of stage s (the m-side tile's loads come first) into ring buffer buf; past the last stage that one's again
     template <int J0, int J1> __device__ __forceinline__ void issue(int s, int buf) {
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_w + buf * SG::BYTES);
-        const bool clamp_k = KT && ragged_k && s >= nk - 1;
 #pragma unroll
-        for (int j = J0; j < J1; ++j) {
-            if (j < LM) {
-                uint32_t o = om.off[j];
-                if constexpr (KT) o = clamp_k ? cm.off[j] : o;
-                dma16s(bm, o, dst + j * (TL::NW * 1024));
-            } else {
-                uint32_t o = on.off[j - LM];
-                if constexpr (KT) o = clamp_k ? cn.off[j - LM] : o;
-                if constexpr (ONCE) dma16s_nt(bn, o, dst + SG::M_OPERAND + (j - LM) * (TL::NW * 1024));
-                else dma16s(bn, o, dst + SG::M_OPERAND + (j - LM) * (TL::NW * 1024));
-            }
-        }
+        for (int j = J0; j < J1; ++j) load(j, j < LM ? om.off[j < LM ? j : 0] : on.off[j < LM ? 0 : j - LM], dst);
         if (J1 == L && s + 1 < nk) { bm += step_m; bn += step_n; }
     }
 };
@@ -336,16 +344,6 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
     if (nk == 0) return;
     FD fd;
     fd.init(Mp, ldm, m0, m_ext, Np, ldn, n0, n_ext, k_ext, smem, wave, src, n_src);
-    auto fix_tail = [&](int s, int buf) __attribute__((always_inline)) {   // ragged contraction: zero what lies past it in the last stage
-        if (KT && s == nk - 1 && (k_ext & (Q_BK - 1))) {
-            char *b = smem + buf * SG::BYTES;
-            if constexpr (M_KS) zero_k_tail<TL::BM, TL::THREADS>(b, k_ext & (Q_BK - 1));
-            else zero_kc_tail<SG::M_OPERAND / 64, TL::THREADS>(b, k_ext & (Q_BK - 1));
-            if constexpr (N_KS) zero_k_tail<TL::BN, TL::THREADS>(b + SG::M_OPERAND, k_ext & (Q_BK - 1));
-            else zero_kc_tail<TL::BN, TL::THREADS>(b + SG::M_OPERAND, k_ext & (Q_BK - 1));
-            __syncthreads();
-        }
-    };
     // SPLIT: with three or more stages in flight a stage's loads are spread over two halves (one iteration
     // of look-ahead is lost for the later half); with two, all of them go into the half after the barrier.
     constexpr bool SPLIT = AHEAD >= 3;
@@ -359,8 +357,10 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
     // iteration in between made the register allocator spill.
     constexpr int LX = SPLIT ? LH : L;        // loads of stage AHEAD - 1 that the prologue issues
     if constexpr (!NO_LOADS) {
+        static_assert(AHEAD >= 2, "the prologue issues all of stage 0");
+        fd.issue_first();
 #pragma unroll
-        for (int s = 0; s < AHEAD - 1; ++s)
+        for (int s = 1; s < AHEAD - 1; ++s)
             if (s < nk) fd.template issue<0, L>(s, s);
         if (AHEAD - 1 < nk) fd.template issue<0, LX>(AHEAD - 1, AHEAD - 1);
     }
@@ -379,7 +379,17 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
                 for (int j = 0; j < 4; ++j) acc[tm][c][j] = b4[j];
         }
     }
-    fix_tail(0, 0);
+    if constexpr (KT) {
+        if (fd.left) {       // stage 0 is what whole stages leave over
+            if constexpr (M_KS) zero_k_tail<TL::BM, TL::THREADS>(smem, fd.left);
+            else zero_kc_tail<SG::M_OPERAND / 64, TL::THREADS>(smem, fd.left);
+            if constexpr (N_KS) zero_k_tail<TL::BN, TL::THREADS>(smem + SG::M_OPERAND, fd.left);
+            else zero_kc_tail<TL::BN, TL::THREADS>(smem + SG::M_OPERAND, fd.left);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (and not for the loads of the stages behind it)
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
+    }
     Frags<TMB, WM, WN, M_KS, N_KS, TMC, TMCW> fr;
     fr.read_first(smem, wm, wn);
     if constexpr (NO_READS) {
@@ -409,7 +419,6 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
         WAIT;                                                                                             \
         if constexpr (!NO_BARRIERS) __builtin_amdgcn_s_barrier();                                         \
         __builtin_amdgcn_sched_barrier(0);                                                                \
-        fix_tail(s + 1, nxt_b);                                                                           \
         MOLE_PART(ISSUE, 1, 0, 0, SPLIT ? LH : L, s + AHEAD, free_b, nxt)                                  \
         MOLE_PART(ISSUE, 1, 1, 0, SPLIT ? LH : L, s + AHEAD, free_b, nxt)                                  \
         MOLE_PART(ISSUE, 1, 2, 0, SPLIT ? LH : L, s + AHEAD, free_b, nxt)                                  \

@@ -441,6 +441,34 @@ def test_ffn_contraction_ends_inside_a_stage(E, M, Fd, rows, gap):
         assert rel_err(got, want) < tol(dtype)
 
 
+# What whole stages of 32 leave of a contraction comes first: every such rest, alone, before one stage, two, and more than the ring holds.  Small
+# whole numbers, whose sums are exact in any order: the results are the nearest bf16 numbers.
+@pytest.mark.parametrize("E,M,Fd,rows,tile", [
+    (6, 520, 264, [65, 71, 95, 96, 97, 127], 128), (5, 136, 256, [129, 159, 161, 191, 223], 128), (64, 512, 1024, [65 + (31 * e) % 260 for e in range(64)], 256)])
+def test_ffn_contraction_with_its_rest_first(E, M, Fd, rows, tile):
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"ffn rest first E={E} M={M} F={Fd} rows={rows[:6]}", flush=True)
+    g = torch.Generator().manual_seed(E + M)
+    whole = lambda *s: torch.randint(-3, 4, s, generator=g).bfloat16().cuda()
+    off = torch.tensor([0] + list(np.cumsum(rows)), dtype=torch.int32).cuda(); n = torch.tensor(rows, dtype=torch.int32).cuda()
+    R = sum(rows)
+    assert L.lib().mole_probe_wgrad_tile(E, R, Fd, M) == tile
+    a, go = whole(R, Fd), whole(R, M)
+    w = whole(E, Fd, M)
+    t = torch.zeros(R, Fd, dtype=torch.bfloat16, device="cuda")
+    grads = [torch.full_like(q, 9.0) for q in (w, w[:, :, 0].contiguous(), w, w[:, 0].contiguous())]
+    H.ffn_bwd_into(go, whole(R, M), a, a, off, n, E, R, M, Fd, w, w, t, *grads, None, False, L.GELU_BWD_EXACT)
+    o = np.cumsum([0] + rows)
+    for e in range(E):
+        want = a[o[e]:o[e + 1]].double().t() @ go[o[e]:o[e + 1]].double()
+        assert torch.equal(grads[2][e], want.bfloat16()) and torch.equal(grads[3][e], go[o[e]:o[e + 1]].double().sum(0).bfloat16())
+    for K in (8, 40, 64, 72, 136, 248):
+        p, q = whole(300, K), whole(72, K)
+        want = p.double() @ q.double().t()
+        assert torch.equal(H.gemm_nt(p, q).double(), want)
+        assert torch.equal(H.gemm_nn(p, q.t().contiguous()), want.bfloat16())
+
+
 # K = F products whose contraction is split into planes: 256- and 320-row tiles in two to four planes, 128 x 128 tiles in two to
 # four, planes of unequal and of ragged length, columns that are not whole tiles, an expert with no rows; the two results
 # with a workspace (split) and without one.
