@@ -327,18 +327,17 @@ typedef float perm_f32x4 __attribute__((ext_vector_type(4)));
 // fp32 accuracy before it is rounded to bf16: widths that are not whole 128-column pieces take it.
 // NH: 32s of experts (two: not split; the product is rounded to bf16 and added behind the rows, bit for bit what mole_gemm_nn and
 // the dispatch backward with its result as dx_add give).  MORE: several choices.
+// block, col_block: the block's tokens and 1024 columns; s_t: its LDS.
+constexpr int DM_LDS = 8 * 16 * DM_ROW;       // floats
 template <bool E8, int TOK, bool SPLIT, int NH, bool MORE>
-__global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_t *__restrict__ dxd,
-                                                                     const int32_t *__restrict__ row, int S, int M, int k,
-                                                                     const float *__restrict__ dlogits,
-                                                                     const float *__restrict__ wg, int E,
-                                                                     bf16_t *__restrict__ dx) {
-    __shared__ __align__(16) float s_t[8][16 * DM_ROW];
+__device__ __forceinline__ void dispatch_bwd_gate_mfma_block(const int block, const int col_block, float *s_t, const bf16_t *__restrict__ dxd,
+                                                             const int32_t *__restrict__ row, int S, int M, int k, const float *__restrict__ dlogits,
+                                                             const float *__restrict__ wg, int E, bf16_t *__restrict__ dx) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, kq = lane >> 4;
-    const int col0 = (blockIdx.y * 8 + wave) * DM_COLS;      // this wave's first column
+    const int col0 = (col_block * 8 + wave) * DM_COLS;       // this wave's first column
     if (col0 >= M) return;                                   // (no barrier below)
-    float *buf = s_t[wave];
+    float *buf = s_t + wave * (16 * DM_ROW);
     const bool rest_first = (((E + 7) & ~7) & 31) != 0;      // NH 2: the order in which mole_gemm_nn takes a contraction over E (in whole eights)
     const int tsel = lane >> 4, c8 = (lane & 15) * 8;        // row-major side: token within a quartet, first of 8 columns
     const bool col_ok = col0 + c8 < M;
@@ -349,11 +348,11 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
     // (the first-choice rows of the block's tokens come with one load, lane l holding token l's, and are handed
     // round between lanes: the gathers' addresses then wait for no load of their own)
     static_assert(TOK <= WAVE, "one first-choice row per lane");
-    const int my_row = row[min((int)blockIdx.x * TOK + lane, S - 1)];
+    const int my_row = row[min(block * TOK + lane, S - 1)];
     auto gather = [&](uint4 (&v)[4], uint32_t (&ok)[4], int tok0) __attribute__((always_inline)) {
         int r[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) r[u] = __shfl(my_row, (tok0 - (int)blockIdx.x * TOK + 4 * u + tsel) & (WAVE - 1), WAVE);
+        for (int u = 0; u < 4; ++u) r[u] = __shfl(my_row, (tok0 - block * TOK + 4 * u + tsel) & (WAVE - 1), WAVE);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             ok[u] = (tok0 + 4 * u + tsel < S && r[u] >= 0) ? 0xffffffffu : 0u;
@@ -362,7 +361,7 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
     };
     uint4 src[4];
     uint32_t src_ok[4];
-    gather(src, src_ok, blockIdx.x * TOK);
+    gather(src, src_ok, block * TOK);
     // A fragment of a group of 16 tokens: dlogits[tok0 + r16][8 kq .. 8 kq + 7], fetched one group ahead like the rows
     // (fetched where it is used, the product waited for it in every group: 15.0 -> 14.2 us at 16384 x 1024)
     auto load_d = [&](float (&d)[NH][8], int tok0) __attribute__((always_inline)) {
@@ -380,7 +379,7 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
         }
     };
     float d[NH][8];
-    load_d(d, blockIdx.x * TOK);
+    load_d(d, block * TOK);
     // B fragments: Wg[8 kq + i][col0 + 16 cb + r16], i = 0..7, for the wave's 8 column blocks.  Fetched row by row
     // with 16-byte loads (a lane takes 4 columns of the 8 experts of one group) and turned by way of the LDS
     // buffer, [expert group][column] with a group's 8 experts as one bf16x8 entry: picking them out of global
@@ -441,7 +440,7 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
     }
 #pragma unroll
     for (int g0 = 0; g0 < TOK; g0 += 16) {
-        const int tok0 = blockIdx.x * TOK + g0;
+        const int tok0 = block * TOK + g0;
         if (tok0 >= S) return;
         uint4 nxt[4];
         uint32_t nxt_ok[4];
@@ -564,6 +563,13 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
                 for (int i = 0; i < 8; ++i) d[h][i] = d_nxt[h][i];
         }
     }
+}
+
+template <bool E8, int TOK, bool SPLIT, int NH, bool MORE>
+__global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_t *__restrict__ dxd, const int32_t *__restrict__ row, int S, int M, int k,
+                                                                     const float *__restrict__ dlogits, const float *__restrict__ wg, int E, bf16_t *__restrict__ dx) {
+    __shared__ __align__(16) float s_t[DM_LDS];
+    dispatch_bwd_gate_mfma_block<E8, TOK, SPLIT, NH, MORE>(blockIdx.x, blockIdx.y, s_t, dxd, row, S, M, k, dlogits, wg, E, dx);
 }
 
 // Gate weight gradient dWg[e, m] = sum_i dlogits[i, e] * x[i, m] (the Linear backward that
@@ -798,6 +804,149 @@ __global__ __launch_bounds__(256, 2) void gate_wgrad_mfma_kernel(const float *__
             for (int cb = 0; cb < 4; ++cb) out[(size_t)e * M + col0 + 16 * cb + r16] = acc[g][cb][r];
         }
 }
+
+// dWg of few tokens in one launch: a block has 32 columns and 16 experts, its NW waves share out the tokens, 32 at a time, and their
+// sums meet in LDS in the waves' order.  Bound by latency: a wave's walk over its share, one step's loads in flight while the one before
+// it is multiplied; partial sums in memory and a second launch for them cost more up to the lines of gate_wgrad_direct_ok.
+// Neither operand is contiguous along the tokens that are summed over, and there is no LDS on the way in:
+//   bf16 tokens: a lane loads two columns of eight tokens and one expert's gradient of each, and turns them in registers for
+//       v_mfma_f32_16x16x32_bf16.  The gradients enter as three bf16 numbers each, 24 bits.  The first ones' products have an accumulator
+//       of their own, and where that is not finite it is the result: the later parts of an infinity, or times one, are NaN.
+//   fp32 tokens: v_mfma_f32_16x16x4_f32 on the values as they come, four tokens an instruction, in four accumulators in turn: the fewer
+//       roundings a sum has in a row, the closer it is (513 tokens, 2-norm error 1.27e-7 with one, 1.01e-7 with four).
+// cols, group: the block's 32 columns and 16 experts; s_sum: its LDS, GD_LDS floats.
+template <int NW> constexpr int GD_LDS = NW * 16 * 32;
+template <typename T, int NW>
+__device__ __forceinline__ void gate_wgrad_direct_block(const int cols, const int group, float *s_sum, const float *__restrict__ dlogits, const T *__restrict__ x, int S, int E, int M,
+                                                        float *__restrict__ dwg) {
+    constexpr bool BF = sizeof(T) == 2;
+    constexpr int COLS = 32, ROWS = 16;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, kg = lane >> 4;
+    const int c0 = cols * COLS, e0 = group * ROWS;
+    const T *xc = x + min(c0 + 2 * i, M - 2);
+    const float *dc = dlogits + min(e0 + i, E - 1);
+    struct Step {
+        uint32_t x[8][BF ? 1 : 2];
+        float d[8];
+    };
+    // u-th token of this lane in the step that begins at t0
+    auto token = [&](int t0, int u) { return BF ? t0 + 8 * kg + u : t0 + 4 * u + kg; };
+    auto fetch = [&](Step &p, int t0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const size_t t = min(token(t0, u), S - 1);
+            if constexpr (BF) {
+                p.x[u][0] = *reinterpret_cast<const uint32_t *>(xc + t * M);
+            } else {
+                const uint2 v = *reinterpret_cast<const uint2 *>(xc + t * M);
+                p.x[u][0] = v.x; p.x[u][1] = v.y;
+            }
+            p.d[u] = dc[t * E];
+        }
+    };
+    constexpr int NA = BF ? 2 : 4;           // bf16: the first parts' products and the others'
+    perm_f32x4 acc[NA][2];
+#pragma unroll
+    for (int n = 0; n < NA; ++n)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[n][j] = perm_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](Step &p, int t0) __attribute__((always_inline)) {
+        if (t0 + 32 > S) {               // tokens past the end count nothing
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (token(t0, u) >= S) {
+#pragma unroll
+                    for (int c = 0; c < (BF ? 1 : 2); ++c) p.x[u][c] = 0;
+                    p.d[u] = 0.f;
+                }
+        }
+        if constexpr (BF) {
+            perm_bf16x8 col[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const uint32_t sel = j ? 0x07060302u : 0x05040100u;
+                uint32_t w[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) w[q] = __builtin_amdgcn_perm(p.x[2 * q + 1][0], p.x[2 * q][0], sel);
+                col[j] = __builtin_bit_cast(perm_bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+            }
+            perm_bf16x8 part[3];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                float r = p.d[u];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    const bf16_t b = (bf16_t)r;
+                    part[q][u] = b;
+                    r = fabsf((float)b) < INFINITY ? r - (float)b : 0.f;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                acc[1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[2], col[j], acc[1][j], 0, 0, 0);
+                acc[1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[1], col[j], acc[1][j], 0, 0, 0);
+                acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part[0], col[j], acc[0][j], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[u % NA][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p.d[u], __uint_as_float(p.x[u][j]), acc[u % NA][j], 0, 0, 0);
+        }
+    };
+    // Two steps' loads are in flight (four are no faster).  They come from clamped addresses without a condition: the steps past a wave's last
+    // one are fetched for nobody.
+    Step a, b;
+    constexpr int STEP = NW * 32;
+    const int first = wave * 32;
+    fetch(a, first);
+    for (int t0 = first; t0 < S; t0 += 2 * STEP) {
+        fetch(b, t0 + STEP);
+        multiply(a, t0);
+        fetch(a, t0 + 2 * STEP);
+        if (t0 + STEP < S) multiply(b, t0 + STEP);
+    }
+    // acc[.][j][r] = expert e0 + 4 kg + r, column c0 + 2 i + j
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        float v[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if constexpr (BF) v[j] = fabsf(acc[0][j][r]) < INFINITY ? acc[0][j][r] + acc[1][j][r] : acc[0][j][r];
+            else v[j] = (acc[0][j][r] + acc[1][j][r]) + (acc[2][j][r] + acc[3][j][r]);
+        }
+        *reinterpret_cast<float2 *>(s_sum + (wave * ROWS + 4 * kg + r) * COLS + 2 * i) = make_float2(v[0], v[1]);
+    }
+    __syncthreads();
+    for (int o = threadIdx.x; o < ROWS * COLS; o += 64 * NW) {
+        float v = s_sum[o];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += s_sum[w * ROWS * COLS + o];
+        const int e = e0 + o / COLS, c = c0 + o % COLS;
+        if (e < E && c < M) dwg[(size_t)e * M + c] = v;
+    }
+}
+template <typename T>
+__global__ __launch_bounds__(1024) void gate_wgrad_direct_kernel(const float *__restrict__ dlogits, const T *__restrict__ x, int S, int E, int M, float *__restrict__ dwg) {
+    __shared__ __align__(16) float s_sum[GD_LDS<16>];
+    gate_wgrad_direct_block<T, 16>(blockIdx.x, blockIdx.y, s_sum, dlogits, x, S, E, M, dwg);
+}
+// ... in the dispatch's backward's launch, as its first `first` blocks: neither needs the other, and both are a few waves' walk.
+template <bool E8, bool SPLIT, int NH, bool MORE>
+__global__ __launch_bounds__(512) void dispatch_bwd_wgrad_kernel(const bf16_t *__restrict__ dxd, const int32_t *__restrict__ row, int S, int M, int k,
+                                                                 const float *__restrict__ dlogits, const float *__restrict__ wg, int E, bf16_t *__restrict__ dx,
+                                                                 const bf16_t *__restrict__ x, float *__restrict__ dwg, int first, int groups, int token_blocks) {
+    static_assert(GD_LDS<8> <= DM_LDS, "one block of LDS for either");
+    __shared__ __align__(16) float s_t[DM_LDS];
+    const int b = (int)blockIdx.x - first;
+    if (b < 0) gate_wgrad_direct_block<bf16_t, 8>((int)blockIdx.x / groups, (int)blockIdx.x % groups, s_t, dlogits, x, S, E, M, dwg);
+    else dispatch_bwd_gate_mfma_block<E8, DM_TOKENS_FEW, SPLIT, NH, MORE>(b % token_blocks, b / token_blocks, s_t, dxd, row, S, M, k, dlogits, wg, E, dx);
+}
+// Up to 1536 bf16 tokens and 512 fp32 ones.  Partial sums and their reduction / here, us with an event pair around them: bf16, 256 tokens x 1024, 8
+// experts 9.0 / 6.4, 100 11.9 / 6.4, 256 13.8 / 7.9; 1024 tokens, 8 experts 9.2 / 7.3, 256 17.7 / 12.9; x 520, 32 experts 13.2 / 7.4; 2048 x 512, 8
+// experts 8.9 / 10.3.  fp32, 256 x 1024, 8 experts 9.5 / 6.2, 32 13.0 / 7.0; 512 10.0 / 7.7.  Error against 64 bits (2-norm, 1e-7), before / here:
+// bf16, 256 tokens x 1024 24 / 0.68, x 520 1.05 / 0.67; fp32 256 tokens 1.06 / 0.86, 513 1.04 / 1.01, 700 1.11 / 1.12: the line of fp32.
+static bool gate_wgrad_direct_ok(int dtype, int S, int E) { return E <= 256 && S <= (dtype == MOLE_BF16 ? 1536 : 512); }
 
 // tokens per chunk of the kernel above: chunks of 128 tokens while the partials stay within 32 MB (or 8
 // chunks), twice as long as often as needed beyond
@@ -1149,12 +1298,23 @@ extern "C" int mole_dispatch_fwd(const void *x, int dtype, const int32_t *row, i
 }
 
 namespace mole {
-// dx = dispatch backward + dlogits . Wg by dispatch_bwd_gate_mfma_kernel
+// dx = dispatch backward + dlogits . Wg by dispatch_bwd_gate_mfma_kernel; with a dwg also dlogits^T . x in the same launch, where
+// gate_wgrad_beside says so
 template <bool SPLIT, int NH>
-static int launch_fold(const void *dxd, const int32_t *row, int S, int M, int k, const float *dlogits, const float *wg, int E, void *dx, hipStream_t st) {
+static int launch_fold(const void *dxd, const int32_t *row, int S, int M, int k, const float *dlogits, const float *wg, int E, void *dx, const void *x, float *dwg, hipStream_t st) {
     const int tok = (long)ceil_div(S, DM_TOKENS) * ceil_div(M, 8 * DM_COLS) < DM_FEW_BLOCKS ? DM_TOKENS_FEW : DM_TOKENS;
     const dim3 grid(ceil_div(S, tok), ceil_div(M, 8 * DM_COLS));
     const bool e8 = E % 8 == 0 && ((uintptr_t)dlogits & 15) == 0;
+    if (dwg != nullptr) {
+        const int groups = ceil_div(E, 16), first = ceil_div(M, 32) * groups, token_blocks = ceil_div(S, DM_TOKENS_FEW);
+#define MOLE_DW(E8, MORE) timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_wgrad_kernel<E8, SPLIT, NH, MORE>, dim3(first + token_blocks * ceil_div(M, 8 * DM_COLS)), dim3(512), 0, st, \
+                                       (const bf16_t *)dxd, row, S, M, k, dlogits, wg, E, (bf16_t *)dx, (const bf16_t *)x, dwg, first, groups, token_blocks)
+        if (e8) { if (k > 1) MOLE_DW(true, true); else MOLE_DW(true, false); }
+        else { if (k > 1) MOLE_DW(false, true); else MOLE_DW(false, false); }
+#undef MOLE_DW
+        MOLE_LAUNCH_CHECK();
+        return 0;
+    }
 #define MOLE_DM_(E8, TOK, MORE) timed_launch(MOLE_K_DISPATCH_BWD, dispatch_bwd_gate_mfma_kernel<E8, TOK, SPLIT, NH, MORE>, grid, dim3(512), 0, st, \
                                              (const bf16_t *)dxd, row, S, M, k, dlogits, wg, E, (bf16_t *)dx)
 #define MOLE_DM(E8, TOK) do { if (k > 1) MOLE_DM_(E8, TOK, true); else MOLE_DM_(E8, TOK, false); } while (0)
@@ -1165,12 +1325,18 @@ static int launch_fold(const void *dxd, const int32_t *row, int S, int M, int k,
     MOLE_LAUNCH_CHECK();
     return 0;
 }
+// Up to 2560 tokens, where the dispatch's backward takes blocks of 16 tokens.  Training passes, three launches / one, us: 513 tokens x 520, 16 experts
+// top-4, 140 / 133; 2048 x 512, 16 top-2, 114.5 / 111; 1000 x 1024, 64 top-2, 165 / 156; 2000 x 1024, 64, 187 / 178.5; 300 x 1024, 40, 167 / 158; 3000 x 768,
+// 16, 176 / 175; 4000 x 512, 8, 160 / 162.5.
+bool gate_wgrad_beside(int dtype, int S, int E, int M) {
+    return dispatch_bwd_folds(dtype, E) && S <= 2560 && (long)ceil_div(S, DM_TOKENS) * ceil_div(M, 8 * DM_COLS) < DM_FEW_BLOCKS;
+}
 bool dispatch_bwd_folds(int dtype, int E) { return dtype == MOLE_BF16 && E <= 64; }
 int dispatch_bwd_fold(const void *dxd, const int32_t *row, int S, int M, int k, const float *dlogits, const float *wg, int E, void *dx, hipStream_t st) {
     if (int rc = check_perm("mole_dispatch_bwd", MOLE_BF16, S, M, k)) return rc;
     MOLE_REQUIRE(dxd && row && dx && dlogits && aligned16(dxd) && aligned16(dx) && wg && dispatch_bwd_folds(MOLE_BF16, E),
                  "mole_dispatch_bwd: null or misaligned pointer");
-    return launch_fold<false, 2>(dxd, row, S, M, k, dlogits, wg, E, dx, st);
+    return launch_fold<false, 2>(dxd, row, S, M, k, dlogits, wg, E, dx, nullptr, nullptr, st);
 }
 }  // namespace mole
 
@@ -1184,8 +1350,8 @@ extern "C" int mole_dispatch_bwd(const void *dxd, int dtype, const int32_t *row,
                  "mole_dispatch_bwd: dlogits given without a valid wg/E");
     MOLE_REQUIRE(dx_add == nullptr || aligned16(dx_add), "mole_dispatch_bwd: misaligned dx_add");
     if (dlogits != nullptr && dx_add == nullptr && E <= 32 && dtype == MOLE_BF16) {
-        return M % DM_COLS != 0 ? launch_fold<true, 1>(dxd, row, S, M, k, dlogits, wg, E, dx, (hipStream_t)stream)
-                                : launch_fold<false, 1>(dxd, row, S, M, k, dlogits, wg, E, dx, (hipStream_t)stream);
+        return M % DM_COLS != 0 ? launch_fold<true, 1>(dxd, row, S, M, k, dlogits, wg, E, dx, nullptr, nullptr, (hipStream_t)stream)
+                                : launch_fold<false, 1>(dxd, row, S, M, k, dlogits, wg, E, dx, nullptr, nullptr, (hipStream_t)stream);
     }
     if (dlogits != nullptr && dx_add == nullptr && E <= 32 && M % 4 == 0) {
         const int db_tokens = (long)ceil_div(S, DB_TOKENS) * ceil_div(M, 1024) < 1024 ? DB_TOKENS_FEW : DB_TOKENS;
@@ -1224,23 +1390,34 @@ size_t gate_wgrad_bytes(int dtype, int S, int E, int M) {
 // Any number of experts.  A single chunk of tokens writes the result itself, without the reduction's launch.  Gates that neither kernel of
 // mole_gate_wgrad takes, by the grouped-GEMM tiles (a block's walk over all tokens for 128 x 128 results, in the tokens' type) / here, us: training
 // passes of 8 tokens, 172 experts of 920 -> 456, 157 / 124; 4041 fp32 tokens, 245 of 704 -> 2112, 3127 / 2833; the largest stay there (layer.hip).
-int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int M, float *dwg, void *workspace, size_t workspace_bytes, hipStream_t st) {
-    ScopedTiming timing(MOLE_K_GATE_WGRAD, st);
+static int check_gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int M, const float *dwg, const void *workspace, size_t workspace_bytes) {
     // (the layer's gates beyond mole_gate_wgrad's own may have their result at any alignment of its elements, a view into a flat buffer of
     // gradients: it is then the reduction's to write)
-    const bool any_dwg = E > 32 && !gate_wgrad_mfma_ok(dtype, S, E, M), direct = aligned16(dwg);
+    const bool any_dwg = E > 32 && !gate_wgrad_mfma_ok(dtype, S, E, M);
     MOLE_REQUIRE(dlogits && x && dwg && workspace && aligned16(x) && (any_dwg || aligned16(dwg)) && aligned16(workspace), "mole_gate_wgrad: null or misaligned pointer");
     const size_t need = gate_wgrad_bytes(dtype, S, E, M);
     if (workspace_bytes < need) {
         set_error("mole_gate_wgrad: workspace of %zu bytes, need %zu", workspace_bytes, need);
         return MOLE_E_WORKSPACE;
     }
+    return 0;
+}
+int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int M, float *dwg, void *workspace, size_t workspace_bytes, hipStream_t st) {
+    ScopedTiming timing(MOLE_K_GATE_WGRAD, st);
+    if (int rc = check_gate_wgrad(dlogits, x, dtype, S, E, M, dwg, workspace, workspace_bytes)) return rc;
+    if (gate_wgrad_direct_ok(dtype, S, E)) {
+        const dim3 grid(ceil_div(M, 32), ceil_div(E, 16));
+        if (dtype == MOLE_BF16) hipLaunchKernelGGL(gate_wgrad_direct_kernel<bf16_t>, grid, dim3(1024), 0, st, dlogits, (const bf16_t *)x, S, E, M, dwg);
+        else hipLaunchKernelGGL(gate_wgrad_direct_kernel<float>, grid, dim3(1024), 0, st, dlogits, (const float *)x, S, E, M, dwg);
+        MOLE_LAUNCH_CHECK();
+        return 0;
+    }
     int nb;
     float *part;
     if (gate_wgrad_mfma_ok(dtype, S, E, M)) {
         const int chunk = gate_wgrad_mfma_chunk(S, E, M);
         nb = ceil_div(S, chunk);
-        part = nb == 1 ? dwg : (float *)workspace;
+        part = (float *)workspace;
         const int eg = E <= 16 ? 1 : (E <= 32 ? 2 : 4);
         const int nz = ceil_div(E, 16 * eg), nunits = nb * ceil_div(M, 256);
         const dim3 grid((unsigned)(ceil_div(nunits, 8) * 8 * nz));
@@ -1254,7 +1431,7 @@ int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int
     } else {
         const int tokens = gw_tokens(S, E, M);
         nb = ceil_div(S, tokens);
-        part = nb == 1 && direct ? dwg : (float *)workspace;
+        part = nb == 1 && aligned16(dwg) ? dwg : (float *)workspace;
         const dim3 grid(nb, ceil_div(M, 512), ceil_div(E, 32));
 #define MOLE_GW(T, EB) hipLaunchKernelGGL((gate_wgrad_partial_kernel<T, EB>), grid, dim3(256), 0, st, dlogits, (const T *)x, S, E, M, tokens, part)
         if (dtype == MOLE_BF16) {
@@ -1269,6 +1446,16 @@ int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int
     hipLaunchKernelGGL(gate_wgrad_reduce_kernel, dim3(ceil_div(E * M, 64)), dim3(256), 0, st, part, nb, E * M, dwg);
     MOLE_LAUNCH_CHECK();
     return 0;
+}
+// The dispatch's backward with the gate's input gradient and gate_wgrad in one launch, where gate_wgrad_beside says so; what either refuses is refused.
+int dispatch_bwd_gate_wgrad(const void *dxd, const int32_t *row, int S, int M, int k, const float *dlogits, const float *wg, int E, void *dx, const void *x, float *dwg, void *workspace,
+                            size_t workspace_bytes, hipStream_t st) {
+    if (int rc = check_perm("mole_dispatch_bwd", MOLE_BF16, S, M, k)) return rc;
+    MOLE_REQUIRE(dxd && row && dx && dlogits && aligned16(dxd) && aligned16(dx) && wg && (E > 32 || aligned16(wg)) && gate_wgrad_beside(MOLE_BF16, S, E, M),
+                 "mole_dispatch_bwd: null or misaligned pointer");
+    if (int rc = check_gate_wgrad(dlogits, x, MOLE_BF16, S, E, M, dwg, workspace, workspace_bytes)) return rc;
+    if (E > 32) return launch_fold<false, 2>(dxd, row, S, M, k, dlogits, wg, E, dx, x, dwg, st);
+    return M % DM_COLS != 0 ? launch_fold<true, 1>(dxd, row, S, M, k, dlogits, wg, E, dx, x, dwg, st) : launch_fold<false, 1>(dxd, row, S, M, k, dlogits, wg, E, dx, x, dwg, st);
 }
 }  // namespace mole
 

@@ -1099,6 +1099,48 @@ def test_input_gradient_of_a_gate_of_up_to_64_is_that_of_its_product(S, M, E, k,
     assert float(t["dlogits"].abs().max()) > 0 and torch.equal(t["dx"], want)
 
 
+# A gate's weight gradient of few tokens, in the dispatch's backward's launch and in one of its own: both sides of the lines, one token, steps of 32 and their
+# rests, groups of experts and columns that are not whole ones.  fp32 sums of exact products (bf16 tokens: of 24 bits, rounded once more):
+# S + 32 steps of 2^-24 of the terms' size at most, and dx of the separate launches bit for bit.
+@pytest.mark.parametrize("S,M,E,k,dtype,beside", [
+    (1, 8, 1, 1, torch.bfloat16, True), (33, 520, 16, 4, torch.bfloat16, True), (513, 128, 17, 2, torch.bfloat16, True), (255, 24, 64, 1, torch.bfloat16, True),
+    (2560, 264, 33, 1, torch.bfloat16, True), (2561, 256, 8, 2, torch.bfloat16, False), (1536, 72, 70, 2, torch.bfloat16, False), (1537, 64, 256, 1, torch.bfloat16, False),
+    (31, 136, 255, 8, torch.bfloat16, False), (1, 4, 3, 1, torch.float32, False), (512, 132, 33, 2, torch.float32, False), (513, 64, 8, 2, torch.float32, False)])
+def test_gate_weight_gradient_of_few_tokens(S, M, E, k, dtype, beside):
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"gate weight gradient of few tokens S={S} M={M} E={E} k={k} {dtype}", flush=True)
+    m, x, _ = _build(S, M, E, k, 16, dtype, seed=S + E)
+    L.kernel_timing_enable(True)
+    L.kernel_timing_read()
+    t = _native_training_pass(m, x, E, k, 16, 0.0)
+    launches = L.kernel_timing_read()["gate_wgrad"][0]
+    L.kernel_timing_enable(False)
+    assert launches == (0 if beside else 1)
+    dl, x64 = t["dlogits"].double().cpu(), x.double().cpu()
+    bound = (S + 32) * 2.0 ** -24 * (dl.abs().t() @ x64.abs())
+    assert float(dl.abs().max()) > 0 or E == 1
+    assert bool(((t["dwg"].double().cpu() - dl.t() @ x64).abs() <= bound).all())
+    if beside:
+        assert torch.equal(t["dx"], H.dispatch_bwd(t["gxd"], t["row"], t["dlogits"], t["wg"]))
+
+
+# Infinities and NaN among the gradients and the tokens come out where the sums of products have them.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gate_weight_gradient_of_few_tokens_with_infinities(dtype):
+    from mole_amd import hip_ops as H
+    S, M, E = 70, 40, 20
+    print(f"gate weight gradient with infinities {dtype}", flush=True)
+    g = torch.Generator().manual_seed(1)
+    x = (torch.randn(S, M, generator=g) + 3.0).to(dtype)
+    dl = torch.randn(S, E, generator=g).abs() + 0.1
+    x[3, 5], x[69, 39], x[40, 7] = float("inf"), float("-inf"), float("nan")
+    dl[2, 4], dl[69, 19], dl[33, 0] = float("inf"), float("-inf"), float("nan")
+    got, want = H.gate_wgrad(dl.cuda(), x.cuda()).double().cpu(), dl.double().t() @ x.double()
+    finite = torch.isfinite(want)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+    assert torch.equal(torch.isfinite(got), finite) and float((got - want)[finite].abs().max() / want[finite].abs().max()) < 1e-5
+
+
 # A large gate's weight gradient at any alignment of its elements (a view into a flat buffer of gradients): fp32 tokens, widths that are no
 # multiple of 64, more than 256 experts; one chunk of tokens, which an aligned result gets without a reduction, and several.
 @pytest.mark.parametrize("S,M,E,k,Fd,dtype", [(12, 72, 40, 2, 64, torch.float32), (700, 132, 70, 2, 32, torch.float32), (15, 520, 33, 1, 32, torch.bfloat16),
