@@ -118,21 +118,23 @@ int dispatch_bwd_fold(const void *dxd, const int32_t *row, int S, int M, int k, 
 
 struct CombineTail;     // gemm.h
 struct DispatchHead;
-// the FFN's entry points with the caller's estimate of the rows beside their bound (ffn_gemm.hip)
-size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, int F);
+// what the caller knows of the rows beside their bound: how many all experts hold in all likelihood, and the most that one can hold
+struct Rows { int est, most; };
+// the FFN's entry points with these (ffn_gemm.hip)
+size_t ffn_workspace_bytes(int dtype, int E, int max_rows, Rows rows, int M, int F);
 size_t gate_route_least_bytes(int dtype, int S, int E, int M, int k);     // gate_route's without small blocks
 int gate_route(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M, int k, double capacity_factor,
                int normalize_gate, int alignment, int layout, float *scores, int32_t *idx, int32_t *loc, float *gates, int32_t *row, int32_t *counts,
                int32_t *kept_rows, int32_t *offsets, int32_t *capacity, float *l_aux, int32_t *token_of, void *workspace, size_t workspace_bytes,
                mole_stream_t stream);
-int ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, int est_rows, int M, int F,
+int ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, Rows rows, int M, int F,
             const void *w1, const void *b1, const void *w2, const void *b2, void *h, void *a, void *out, void *workspace,
             size_t workspace_bytes, int forward_only, const DispatchHead *head, CombineTail *tail, hipStream_t st);     // head: xd is the tokens
 // Whether h = xd.w1^T + b1 can read the tokens where they lie: not at all, from the pairs' rows or from the list of the rows' tokens
 enum FwdTokens { TOKENS_NO, TOKENS_PAIRS, TOKENS_LIST };
-FwdTokens ffn_fwd_takes_tokens(int dtype, int E, int max_rows, int est_rows, int M, int F);
+FwdTokens ffn_fwd_takes_tokens(int dtype, int E, int max_rows, Rows rows, int M, int F);
 int ffn_bwd(const void *go, const void *xd, const void *h, const void *a, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
-            int max_rows, int est_rows, int M, int F, const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2, void *g_b2,
+            int max_rows, Rows rows, int M, int F, const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2, void *g_b2,
             void *gx, int accumulate, int gelu_bwd, void *workspace, size_t workspace_bytes, hipStream_t st);
 
 }  // namespace mole

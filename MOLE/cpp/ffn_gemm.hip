@@ -485,10 +485,10 @@ static int weights_pass_by(int E, int est_rows, int M, int F, size_t elem, int f
 template <typename T>
 static int ffn_fwd_t(const void *xd, const int32_t *offsets, const int32_t *kept, int E, int max_rows, int M, int F,
                      const void *w1, const void *b1, const void *w2, const void *b2, void *h, void *a, void *out,
-                     void *ws, size_t ws_bytes, int est_rows, int forward_only, const DispatchHead *head, CombineTail *tail, hipStream_t st) {
+                     void *ws, size_t ws_bytes, Rows rows, int forward_only, const DispatchHead *head, CombineTail *tail, hipStream_t st) {
     const int m_tiles = max_rows / TBM + E;  // every expert may end in a partial tile
     GemmArgs g{};
-    g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles; g.est_rows = est_rows;
+    g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles; g.est_rows = rows.est; g.most_rows = rows.most;
     // h = xd . w1^T + b1, a = gelu(h)
     g.A = xd; g.lda = M; g.B = w1; g.ldb = M; g.strideB = (long)F * M; g.N = F; g.K = M;
     // (h is for the backward pass alone: a store of R F elements and a turn through LDS less where none follows; 6002 rows,
@@ -501,7 +501,7 @@ static int ffn_fwd_t(const void *xd, const int32_t *offsets, const int32_t *kept
     g.pair_row = g.token_of = nullptr;
     g.A = a; g.lda = F; g.B = w2; g.ldb = M; g.strideB = (long)F * M; g.N = M; g.K = F;
     g.C = out; g.C2 = nullptr; g.ldc = M; g.bias = b2;
-    g.once = weights_pass_by(E, est_rows, M, F, sizeof(T), forward_only);
+    g.once = weights_pass_by(E, rows.est, M, F, sizeof(T), forward_only);
     g.tail = tail;
     return run_gemm<T, false, true, false, EPI_BIAS>(g, max_rows, m_tiles * ceil_div(M, TBN), st, MOLE_K_FFN_FWD2, ws, ws_bytes);
 }
@@ -510,10 +510,10 @@ template <typename T>
 static int ffn_bwd_t(const void *go, const void *xd, const void *h, const void *a, const int32_t *offsets,
                      const int32_t *kept, int E, int max_rows, int M, int F, const void *w1, const void *w2, void *t,
                      void *g_w1, void *g_b1, void *g_w2, void *g_b2, void *gx, int accumulate, int gelu_bwd,
-                     void *ws, size_t ws_bytes, int est_rows, hipStream_t st) {
+                     void *ws, size_t ws_bytes, Rows rows, hipStream_t st) {
     const int m_tiles = max_rows / TBM + E;
     GemmArgs g{};
-    g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles; g.est_rows = est_rows;
+    g.offsets = offsets; g.kept = kept; g.E = E; g.m_tiles_bound = m_tiles; g.est_rows = rows.est; g.most_rows = rows.most;
     g.accumulate = accumulate; g.gelu_bwd = gelu_bwd;
     const int wg_tiles = E * ceil_div(F, TBM) * ceil_div(M, TBN);
     // The bias gradients are sums of go and of t over every expert's rows: go and t are operands of the two
@@ -537,7 +537,7 @@ static int ffn_bwd_t(const void *go, const void *xd, const void *h, const void *
     gw1.A = t; gw1.lda = F; gw1.B = xd; gw1.ldb = M; gw1.M = F; gw1.N = M; gw1.C = g_w1; gw1.ldc = M; gw1.strideC = (long)F * M;
     if (fused_sums) { gw1.colsum = g_b1; gw1.colsum_side = 1; }
     ggx.A = t; ggx.lda = F; ggx.B = w1; ggx.ldb = M; ggx.strideB = (long)F * M; ggx.N = M; ggx.K = F; ggx.C = gx; ggx.ldc = M;
-    ggx.once = weights_pass_by(E, est_rows, M, F, sizeof(T), 0);
+    ggx.once = weights_pass_by(E, rows.est, M, F, sizeof(T), 0);
     // (a result in the place of what the other product reads goes by the order of the two launches)
     auto overlaps = [&](const void *p, long np, const void *q, long nq) {
         const uintptr_t a0 = (uintptr_t)p, b0 = (uintptr_t)q, na = (uintptr_t)np * max_rows * sizeof(T), nb = (uintptr_t)nq * max_rows * sizeof(T);
@@ -590,21 +590,21 @@ using namespace mole;
 
 namespace mole {
 
-size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, int F) {
+size_t ffn_workspace_bytes(int dtype, int E, int max_rows, Rows rows, int M, int F) {
     if (E <= 0 || max_rows <= 0 || M <= 0 || F <= 0) return 0;
-    int ks = gemm_skinny_ksplit(E, max_rows, est_rows, M, F, dtype);
-    if (ks == 0) ks = dtype == MOLE_BF16 ? gemm256_ksplit(E, est_rows, M, F) : gemm_f32_ksplit(E, est_rows, M, F);
-    ks = planes_allowed(ks, max_rows, est_rows, M);
+    int ks = gemm_skinny_ksplit(E, max_rows, rows.est, M, F, dtype);
+    if (ks == 0) ks = dtype == MOLE_BF16 ? gemm256_ksplit(E, rows.est, M, F) : gemm_f32_ksplit(E, rows, M, F);
+    ks = planes_allowed(ks, max_rows, rows.est, M);
     return ks > 1 ? (size_t)ks * max_rows * M * sizeof(float) : 0;
 }
 
-FwdTokens ffn_fwd_takes_tokens(int dtype, int E, int max_rows, int est_rows, int M, int F) {
+FwdTokens ffn_fwd_takes_tokens(int dtype, int E, int max_rows, Rows rows, int M, int F) {
     if (!fast_path_enabled()) return TOKENS_NO;
-    if (gemm_skinny_takes_tokens(E, max_rows, est_rows, F, M, dtype)) return TOKENS_PAIRS;
+    if (gemm_skinny_takes_tokens(E, max_rows, rows.est, F, M, dtype)) return TOKENS_PAIRS;
     return max_rows > 0 && (dtype == MOLE_BF16 ? M % 8 == 0 && F % 8 == 0 : gemm_f32_takes(F, M)) ? TOKENS_LIST : TOKENS_NO;
 }
 
-int ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, int est_rows, int M, int F,
+int ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E, int max_rows, Rows rows, int M, int F,
             const void *w1, const void *b1, const void *w2, const void *b2, void *h, void *a, void *out, void *workspace,
             size_t workspace_bytes, int forward_only, const DispatchHead *head, CombineTail *tail, hipStream_t st) {
     if (int rc = check_ffn("mole_ffn_fwd", dtype, E, max_rows, M, F)) return rc;
@@ -613,12 +613,12 @@ int ffn_fwd(const void *xd, int dtype, const int32_t *offsets, const int32_t *ke
     MOLE_REQUIRE(al16(xd) && al16(w1) && al16(w2) && al16(h) && al16(a) && al16(out) && al16(workspace),
                  "mole_ffn_fwd: buffers must be 16-byte aligned");
     if (dtype == MOLE_BF16)
-        return ffn_fwd_t<bf16_t>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes, est_rows, forward_only, head, tail, st);
-    return ffn_fwd_t<float>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes, est_rows, forward_only, head, tail, st);
+        return ffn_fwd_t<bf16_t>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes, rows, forward_only, head, tail, st);
+    return ffn_fwd_t<float>(xd, offsets, kept_rows, E, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes, rows, forward_only, head, tail, st);
 }
 
 int ffn_bwd(const void *go, const void *xd, const void *h, const void *a, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
-            int max_rows, int est_rows, int M, int F, const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2, void *g_b2,
+            int max_rows, Rows rows, int M, int F, const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2, void *g_b2,
             void *gx, int accumulate, int gelu_bwd, void *workspace, size_t workspace_bytes, hipStream_t st) {
     if (int rc = check_ffn("mole_ffn_bwd", dtype, E, max_rows, M, F)) return rc;
     MOLE_REQUIRE(gelu_bwd == MOLE_GELU_BWD_TANH || gelu_bwd == MOLE_GELU_BWD_EXACT, "mole_ffn_bwd: bad gelu_bwd %d", gelu_bwd);
@@ -628,21 +628,21 @@ int ffn_bwd(const void *go, const void *xd, const void *h, const void *a, int dt
                  "mole_ffn_bwd: buffers must be 16-byte aligned");
     if (dtype == MOLE_BF16)
         return ffn_bwd_t<bf16_t>(go, xd, h, a, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx, accumulate,
-                                 gelu_bwd, workspace, workspace_bytes, est_rows, st);
+                                 gelu_bwd, workspace, workspace_bytes, rows, st);
     return ffn_bwd_t<float>(go, xd, h, a, offsets, kept_rows, E, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx, accumulate, gelu_bwd,
-                            workspace, workspace_bytes, est_rows, st);
+                            workspace, workspace_bytes, rows, st);
 }
 
 }  // namespace mole
 
 extern "C" size_t mole_ffn_workspace_bytes(int dtype, int E, int max_rows, int M, int F) {
-    return ffn_workspace_bytes(dtype, E, max_rows, max_rows, M, F);
+    return ffn_workspace_bytes(dtype, E, max_rows, Rows{max_rows, max_rows}, M, F);
 }
 
 extern "C" int mole_ffn_fwd_ws(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
                                int max_rows, int M, int F, const void *w1, const void *b1, const void *w2, const void *b2,
                                void *h, void *a, void *out, void *workspace, size_t workspace_bytes, mole_stream_t stream) {
-    return ffn_fwd(xd, dtype, offsets, kept_rows, E, max_rows, max_rows, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes,
+    return ffn_fwd(xd, dtype, offsets, kept_rows, E, max_rows, Rows{max_rows, max_rows}, M, F, w1, b1, w2, b2, h, a, out, workspace, workspace_bytes,
                    0, nullptr, nullptr, (hipStream_t)stream);
 }
 
@@ -657,7 +657,7 @@ extern "C" int mole_ffn_bwd_ws(const void *go, const void *xd, const void *h, co
                                const void *w1, const void *w2, void *t, void *g_w1, void *g_b1, void *g_w2, void *g_b2,
                                void *gx, int accumulate, int gelu_bwd, void *workspace, size_t workspace_bytes,
                                mole_stream_t stream) {
-    return ffn_bwd(go, xd, h, a, dtype, offsets, kept_rows, E, max_rows, max_rows, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx, accumulate,
+    return ffn_bwd(go, xd, h, a, dtype, offsets, kept_rows, E, max_rows, Rows{max_rows, max_rows}, M, F, w1, w2, t, g_w1, g_b1, g_w2, g_b2, gx, accumulate,
                    gelu_bwd, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
@@ -676,7 +676,7 @@ extern "C" int mole_gemm_nt(const void *a, const void *b, int dtype, int rows, i
     if (rows == 0) return 0;
     MOLE_REQUIRE(a && b && c && al16(a) && al16(b), "mole_gemm_nt: null or misaligned pointer");
     GemmArgs g{};
-    g.single_rows = rows; g.E = 1; g.est_rows = rows;
+    g.single_rows = rows; g.E = 1; g.est_rows = g.most_rows = rows;
     g.A = a; g.lda = K; g.B = b; g.ldb = K; g.N = N; g.K = K; g.C = c; g.ldc = N;
     const int tiles = ceil_div(rows, TBM) * ceil_div(N, TBN);
     if (dtype == MOLE_BF16) return run_gemm<bf16_t, false, false, false, EPI_F32>(g, rows, tiles, (hipStream_t)stream, MOLE_K_GEMM_NT);
@@ -691,7 +691,7 @@ extern "C" int mole_gemm_nn(const void *a, const void *b, int dtype, int rows, i
     if (rows == 0) return 0;
     MOLE_REQUIRE(a && b && c && al16(a) && al16(b) && al16(c), "mole_gemm_nn: null or misaligned pointer");
     GemmArgs g{};
-    g.single_rows = rows; g.E = 1; g.est_rows = rows;
+    g.single_rows = rows; g.E = 1; g.est_rows = g.most_rows = rows;
     g.A = a; g.lda = K; g.B = b; g.ldb = N; g.N = N; g.K = K; g.C = c; g.ldc = N;
     const int tiles = ceil_div(rows, TBM) * ceil_div(N, TBN);
     if (dtype == MOLE_BF16) return run_gemm<bf16_t, false, true, false, EPI_STORE>(g, rows, tiles, (hipStream_t)stream, MOLE_K_GEMM_NT);
@@ -705,7 +705,7 @@ extern "C" int mole_gemm_tn(const void *a, const void *b, int dtype, int rows, i
     MOLE_REQUIRE(rows >= 0 && N > 0 && Mo > 0 && Mo % epc == 0 && N % epc == 0, "mole_gemm_tn: bad sizes rows=%d Mo=%d N=%d", rows, Mo, N);
     MOLE_REQUIRE(c && al16(c) && (rows == 0 || (a && b && al16(a) && al16(b))), "mole_gemm_tn: null or misaligned pointer");
     GemmArgs g{};
-    g.single_rows = rows; g.E = 1; g.est_rows = rows;      // one group whose contraction runs over all rows (zero rows: c = 0)
+    g.single_rows = rows; g.E = 1; g.est_rows = g.most_rows = rows;      // one group whose contraction runs over all rows (zero rows: c = 0)
     g.A = a; g.lda = Mo; g.B = b; g.ldb = N; g.M = Mo; g.N = N; g.C = c; g.ldc = N; g.strideC = (long)Mo * N;
     const int tiles = ceil_div(Mo, TBM) * ceil_div(N, TBN);
     if (dtype == MOLE_BF16) return launch_gemm<bf16_t, true, true, true, TBM, TBN, EPI_WGRAD>(g, tiles, (hipStream_t)stream, MOLE_K_GEMM_NT);

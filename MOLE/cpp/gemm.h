@@ -173,6 +173,7 @@ struct GemmArgs {
     int ksplit;
     int once;               // row-ragged products with K-strided weights: see weights_pass_by()
     int est_rows;           // host's estimate of the rows of all experts together (no more than the launch's bound)
+    int most_rows;          // the most rows that one expert can have
     CombineTail *tail;      // host side only: see CombineTail (null: none)
     const int32_t *pair_row;    // A is the tokens and not their dispatched rows: [pairs], pair p is token p % tokens (null: it is the rows)
     int pairs, tokens;
@@ -206,7 +207,7 @@ bool gemm_skinny_takes_tokens(int E, int max_rows, int est_rows, int N, int K, i
 int gemm_skinny_ksplit(int E, int max_rows, int est_rows, int N, int K, int dtype);    // 0: not its shape
 // fp32 tiles with direct-to-LDS loads (gemm_f32.hip); -100 as above.
 int launch_gemm_f32(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
-int gemm_f32_ksplit(int E, int est_rows, int N, int K);
+int gemm_f32_ksplit(int E, Rows rows, int N, int K);
 bool gemm_f32_takes(int N, int K);      // the widths of a row-ragged product
 bool gemm_f32_sums_operand(const GemmArgs &g);
 

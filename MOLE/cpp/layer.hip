@@ -8,12 +8,18 @@
 #include "gemm.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace mole {
 
 // rows the experts hold in all likelihood: every pair, or the capacity's bound where that is less (the padded layout's
 // buffers have a row for every slot)
 static int est_rows(const mole_layer &L) { return L.rows < L.S * L.k ? L.rows : L.S * L.k; }
+static Rows rows_of(const mole_layer &L) {
+    // an expert takes a token once, and of those no more than the capacity
+    const double capacity = L.capacity_factor > 0. ? (double)L.k * std::floor(L.capacity_factor * ((L.S + L.E - 1) / L.E)) : (double)L.S;
+    return Rows{est_rows(L), capacity < L.S ? (int)capacity : L.S};
+}
 
 // Whether the first product reads the tokens through the list although their rows are written for later: where the rows of several choices are
 // more than the last-level cache holds and the tokens are well below it, so that the tokens come from the cache and the rows do not.  Training
@@ -100,7 +106,7 @@ using namespace mole;
 
 extern "C" size_t mole_layer_workspace_bytes(const mole_layer *L, int backward) {
     if (L == nullptr || L->S <= 0 || L->E <= 0) return 0;
-    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
+    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, rows_of(*L), L->M, L->F);
     size_t other = backward ? gate_bwd_plan(*L, gate_wgrad_by_tiles(*L)).total : mole_gate_route_shape_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
     if (!backward && tokens_beside_rows(*L)) other = up256(other) + (size_t)L->rows * 4;
     return ffn > other ? ffn : other;        // the two are never in use at the same time
@@ -117,7 +123,7 @@ static int check_layer(const char *fn, const mole_layer *L, mole_stream_t) {
 extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream) {
     if (int rc = check_layer("mole_layer_fwd", L, stream)) return rc;
     const size_t route_bytes = mole_gate_route_shape_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
-    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F), need = std::max(route_bytes, ffn);
+    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, rows_of(*L), L->M, L->F), need = std::max(route_bytes, ffn);
     if (L->workspace_bytes < std::max(gate_route_least_bytes(L->dtype, L->S, L->E, L->M, L->k), ffn)) {
         set_error("mole_layer_fwd: workspace of %zu bytes, need %zu", L->workspace_bytes, need);
         return MOLE_E_WORKSPACE;
@@ -137,7 +143,7 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
     FwdTokens takes = TOKENS_NO;
     const bool beside = !scratch && tokens_beside_rows(*L) && L->workspace_bytes >= up256(route_bytes) + (size_t)L->rows * 4;
     if ((scratch || beside) && L->k >= 1 && L->k <= 16 && ((uintptr_t)L->x & 15) == 0)
-        takes = ffn_fwd_takes_tokens(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
+        takes = ffn_fwd_takes_tokens(L->dtype, L->E, L->rows, rows_of(*L), L->M, L->F);
     if (takes == TOKENS_PAIRS && (beside || (long)L->S * L->k > HEAD_PAIRS)) takes = TOKENS_NO;
     if (takes == TOKENS_LIST && ((size_t)L->S * L->M * (L->dtype == MOLE_BF16 ? 2 : 4) >= (size_t)1 << 31 ||
                                  (L->M < 256 && (long)L->S * L->k <= HEAD_PAIRS))) takes = TOKENS_NO;
@@ -153,7 +159,7 @@ extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream
     // (what the combine would refuse is left to it)
     CombineTail tail{L->row, L->idx, L->gates, y, L->S, L->k, !scratch, false};
     const bool tail_ok = y != nullptr && ((uintptr_t)y & 15) == 0 && L->k >= 1 && L->k <= 16;
-    if (int rc = ffn_fwd(head_ok ? L->x : L->xd, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, est_rows(*L), L->M, L->F, L->w1, L->b1, L->w2,
+    if (int rc = ffn_fwd(head_ok ? L->x : L->xd, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, rows_of(*L), L->M, L->F, L->w1, L->b1, L->w2,
                          L->b2, L->h, L->a, L->out, L->workspace, L->workspace_bytes, L->forward_only, head_ok ? &head : nullptr,
                          tail_ok ? &tail : nullptr, (hipStream_t)stream)) return rc;
     if (tail.done) return 0;
@@ -164,7 +170,7 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
     if (int rc = check_layer("mole_layer_bwd", L, stream)) return rc;
     MOLE_REQUIRE(!L->forward_only, "mole_layer_bwd: the forward pass was a forward_only one");
     MOLE_REQUIRE(G && G->dy && G->dlogits && G->d_o && G->t && G->gxd && G->dx && G->dwg, "mole_layer_bwd: null gradient pointer");
-    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, est_rows(*L), L->M, L->F);
+    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, rows_of(*L), L->M, L->F);
     GateBwdPlan p = gate_bwd_plan(*L, gate_wgrad_by_tiles(*L));
     const size_t need = std::max(ffn, p.total);
     // (a workspace that does not hold the partial sums of a large gate has its weight gradient by the tiles)
@@ -186,7 +192,7 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
                                    stream)) return rc;
     }
     // (the FFN's scratch takes the place of dgates and makes room for the gate's products, in stream order)
-    if (int rc = ffn_bwd(G->d_o, L->xd, L->h, L->a, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, est_rows(*L), L->M, L->F, L->w1, L->w2,
+    if (int rc = ffn_bwd(G->d_o, L->xd, L->h, L->a, L->dtype, L->offsets, L->kept_rows, L->E, L->rows, rows_of(*L), L->M, L->F, L->w1, L->w2,
                                  G->t, G->g_w1, G->g_b1, G->g_w2, G->g_b2, G->gxd, G->accumulate, G->gelu_bwd, L->workspace,
                                  L->workspace_bytes, st)) return rc;
     char *dl_t = ws + p.dgates, *wg_t = dl_t + p.dl_t, *dx_add = wg_t + p.wg_t, *wgrad = dx_add + p.dx_add;

@@ -772,6 +772,44 @@ def test_ffn_split_contraction_of_more_than_2_to_18_rows():
         assert bool(((got - (ae @ w2[e] + b2[e])).abs() <= 4 * 2.0 ** -24 * 32 * terms).all())
 
 
+# fp32 tiles whose parts a block makes once: h and t (K = M: 12.5, 13 and 13.5 stages of 32 k, which the loop takes in pairs), columns that end 16
+# into a tile, rows that end anywhere in one; out and gx of the last case are split into planes of 16 and 17 such stages.  Eight of k are summed
+# before a rounding to nearest: 2^-24 sqrt(K / 8) in the 2-norm, as of all products by parts.  A tile that an infinite weight reaches
+# is formed from fp32 operands instead, 2^-24 sqrt(K), and no other tile changes.
+@pytest.mark.parametrize("E,M,Fd,rows", [(6, 400, 2064, [190, 201, 129, 128, 255, 237]), (6, 416, 2064, [190, 201, 129, 128, 255, 237]),
+                                         (6, 432, 2064, [190, 201, 129, 128, 255, 237]), (8, 512, 2064, [194, 256, 130, 192, 255, 193, 129, 196])])
+def test_ffn_fp32_parts_that_a_block_shares(E, M, Fd, rows):
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"ffn fp32 shared parts E={E} M={M} F={Fd}", flush=True)
+    d = _make(E, M, Fd, rows, torch.float32, seed=M)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    off, n, R = torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda(), sum(rows)
+    out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+    g = [torch.empty_like(c[k]) for k in ("w1", "b1", "w2", "b2")]
+    t, gx = torch.empty(R, Fd, device="cuda"), torch.empty(R, M, device="cuda")
+    H.ffn_bwd_into(c["go"], c["xd"], h, a, off, n, E, R, M, Fd, c["w1"], c["w2"], t, *g, gx, False, L.GELU_BWD_EXACT)
+    w1 = c["w1"].clone()
+    w1[1, 5, M - 1] = float("inf")
+    _, h_inf, _ = H.ffn_fwd(c["xd"], off, n, w1, c["b1"], c["w2"], c["b2"])
+    def close(got, want, terms):
+        assert float((got.double() - want).norm() / want.norm()) <= 2.0 ** -24 * terms ** 0.5
+    rest = torch.arange(Fd, device="cuda") != 5
+    for e in range(E):
+        r = slice(int(d["off"][e]), int(d["off"][e]) + rows[e])
+        D = lambda q: q.double()
+        want = D(c["xd"][r]) @ D(c["w1"][e]).t() + D(c["b1"][e])
+        close(h[r], want, M / 8)
+        close(out[r], D(a[r]) @ D(c["w2"][e]) + D(c["b2"][e]), Fd / 8)
+        # (GELU' takes h to a few units of fp32 of its largest value: its share of t's error is that of as many terms)
+        close(t[r], (D(c["go"][r]) @ D(c["w2"][e]).t()) * O.d_gelu_exact(D(h[r]).cpu()).cuda(), M / 8 + 16)
+        close(gx[r], D(t[r]) @ D(c["w1"][e]), Fd / 8)
+        if e != 1:
+            assert torch.equal(h_inf[r], h[r])
+        else:
+            assert torch.equal(h_inf[r, 5], c["xd"][r, M - 1].sign() * float("inf"))
+            close(h_inf[r][:, rest], want[:, rest], M)
+
+
 # fp32 products from fp32 operands on 64-row tiles (whole and with remainders; split contractions; the last case's out on the generic
 # kernel) and weight gradients, by bf16 parts of their operands: as far from 64 bits as a sum of K fp32 terms may be, 2^-24 sqrt(K) in
 # the 2-norm, and with no bias: the mean error of n results is within 8 / sqrt(n) of their deviation.
