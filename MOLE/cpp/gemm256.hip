@@ -341,6 +341,13 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
     typedef Feeder<TMB, WM, WN, M_KS, N_KS, KT, TMC, ONCE> FD;
     constexpr int L = FD::L, LH = L / 2;      // loads per wave per stage; the halves are LH and L - LH
     const int nk = __builtin_amdgcn_readfirstlane((k_ext + Q_BK - 1) / Q_BK);
+    auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2 * Tile<TMB, WM, WN>::TMW; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    if (M_KS || nk == 0) clear();
     if (nk == 0) return;
     FD fd;
     fd.init(Mp, ldm, m0, m_ext, Np, ldn, n0, n_ext, k_ext, smem, wave, src, n_src);
@@ -364,6 +371,7 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
             if (s < nk) fd.template issue<0, L>(s, s);
         if (AHEAD - 1 < nk) fd.template issue<0, LX>(AHEAD - 1, AHEAD - 1);
     }
+    if constexpr (!M_KS) clear();       // (while the loads are on their way; weight gradients are 1 % slower for it)
     // stage 0 has landed when no more is in flight than what was issued after it
     if (nk >= AHEAD) __builtin_amdgcn_s_waitcnt(waitcnt_vm((AHEAD - 2) * L + LX));
     else wait_stages_behind<AHEAD - 2, L, 0>(nk - 1, false);
@@ -725,23 +733,34 @@ __device__ __forceinline__ void gemm256_block(const GemmArgs &g, const int block
         const bool single = g.offsets == nullptr;
         auto rows_of = [&](int ee) { return single ? g.single_rows : g.kept[ee]; };
         const int nE = single ? 1 : g.E;
-        // rows and first row of the first 256 experts, fetched together (lane l holds experts l, l + 64, l + 128,
+        // Rows and first row of the first 256 experts, fetched together (lane l holds experts l, l + 64, l + 128,
         // l + 192): the lookups below then need no further loads.  Fetched where they were needed, each pass of the
         // search below and the two lookups after it waited for memory in turn - four to five dependent round trips
         // per tile for experts past the 64th, half of a tile's fixed cost with 256 experts and a contraction of 1024.
         // (Beyond 256 experts the rest is read through the cache as before.)
+        // A block has nothing to run beside this search: its time is the tile's.  What up to 64 experts need stands first and straight: one
+        // scan a class that serves the totals and the search, one division.  On tiles of 128 x 128, 16 experts, the search 1.65 -> 1.15 us of a
+        // block's 10 to 16: h of 128 rows, 512 -> 1408 11.9 -> 11.2 us, out 15.3 -> 14.8; h of 256, 512 -> 1024 12.4 -> 11.8; passes of 3001
+        // tokens, top-2 of 16, 1024 -> 4096 -1 %, of 256, top-8 of 256, -1.5 %.
         constexpr int RC = 4;
+        const bool many = nE > WAVE;
         int rows_c[RC], off_c[RC];
+        rows_c[0] = lane < nE ? rows_of(lane) : 0;
+        off_c[0] = !single && lane < nE ? g.offsets[lane] : 0;
 #pragma unroll
-        for (int c = 0; c < RC; ++c) {
-            const int ee = lane + WAVE * c;
-            rows_c[c] = ee < nE ? rows_of(min(ee, nE - 1)) : 0;
-            off_c[c] = (!single && ee < nE) ? g.offsets[min(ee, nE - 1)] : 0;
+        for (int c = 1; c < RC; ++c) rows_c[c] = off_c[c] = 0;
+        if (many) {
+#pragma unroll
+            for (int c = 1; c < RC; ++c) {
+                const int ee = lane + WAVE * c;
+                rows_c[c] = ee < nE ? rows_of(ee) : 0;
+                off_c[c] = !single && ee < nE ? g.offsets[ee] : 0;
+            }
         }
-        auto rows_at = [&](int ee) {            // rows of expert ee = base + lane of the caller's pass (ee uniform in ee / 64)
+        auto rows_at = [&](int ee) {            // rows of expert ee = base + lane of the caller's pass (ee uniform in ee / 64), from the 65th on
             int r = 0;
 #pragma unroll
-            for (int c = 0; c < RC; ++c)
+            for (int c = 1; c < RC; ++c)
                 if ((ee >> 6) == c) r = rows_c[c];
             return (ee >> 6) < RC ? r : (ee < nE ? rows_of(ee) : 0);
         };
@@ -758,18 +777,23 @@ __device__ __forceinline__ void gemm256_block(const GemmArgs &g, const int block
         auto heavy_of = [&](int r) {
             const int cnt = tiles_of(r);
             if (cnt == 0 || !split) return cnt;
-            if (TMB == 10) return ((((r + cnt - 1) / cnt) + 31) & ~31) > Q_BM / 2 ? cnt : 0;
+            if (TMB == 10) return cnt > 1 || r > Q_BM / 2 ? cnt : 0;      // (two or more of equal height are above half a tile each)
             return cnt - 1 + ((r - (cnt - 1) * Q_BM) > Q_BM / 2 ? 1 : 0);
         };
-        int n_h = 0, n_l = 0;
-        for (int ee = lane; ee < nE; ee += WAVE) {
-            const int r = rows_at(ee);
-            const int hv = heavy_of(r);
-            n_h += hv;
-            n_l += tiles_of(r) - hv;
+        const int hv_0 = heavy_of(rows_c[0]), lt_0 = tiles_of(rows_c[0]) - hv_0;
+        int incl_h = wave_scan(hv_0), incl_l = wave_scan(lt_0);
+        int n_h = wave_total(incl_h), n_l = wave_total(incl_l);
+        if (many) {
+            int more_h = 0, more_l = 0;
+            for (int ee = lane + WAVE; ee < nE; ee += WAVE) {
+                const int r = rows_at(ee);
+                const int hv = heavy_of(r);
+                more_h += hv;
+                more_l += tiles_of(r) - hv;
+            }
+            n_h += wave_total(wave_scan(more_h));
+            n_l += wave_total(wave_scan(more_l));
         }
-        n_h = wave_total(wave_scan(n_h));
-        n_l = wave_total(wave_scan(n_l));
         if ((n_h + n_l) * n_units > 16 * 256) { split = false; n_h += n_l; n_l = 0; }
         const int total_h = n_h * n_units, total_l = n_l * n_units;
         const int per_h = (total_h + 7) >> 3, per_l = (total_l + 7) >> 3;
@@ -791,43 +815,45 @@ __device__ __forceinline__ void gemm256_block(const GemmArgs &g, const int block
         const bool mf = g.m_fastest != 0;
         const int unit = mf ? n_tiles : 1;       // tiles per counted m-tile
         const int target = mf ? t : t / n_units;
-        nt = t % n_units;
+        nt = t - target * n_units;               // (m-tile first: found below)
         // the expert whose running count (of the class) passes `target`
-        int run = 0, found = -1, before = 0, cnt_found = 1;
-        for (int base = 0; base < nE && found < 0; base += WAVE) {
-            const int ee = base + lane;
-            const int r = rows_at(ee);
-            const int hv = heavy_of(r);
-            const int cnt = (heavy ? hv : tiles_of(r) - hv) * unit;
-            const int incl = wave_scan(cnt);
-            const unsigned long long hit = __ballot(run + incl > target);
-            if (hit) {
-                const int src = __ffsll(hit) - 1;
-                found = base + src;
-                before = run + __builtin_amdgcn_readlane(incl - cnt, src);
-                cnt_found = __builtin_amdgcn_readlane(cnt, src);
+        int run = 0, base = 0;
+        int cnt = heavy ? (split ? hv_0 : hv_0 + lt_0) : lt_0, incl = heavy ? (split ? incl_h : incl_h + incl_l) : incl_l;
+        unsigned long long hit = __ballot(incl * unit > target);
+        if (many) {
+            while (!hit) {
+                run += wave_total(incl);
+                base += WAVE;
+                if (base >= nE) break;
+                const int r = rows_at(base + lane);
+                const int hv = heavy_of(r);
+                cnt = heavy ? hv : tiles_of(r) - hv;
+                incl = wave_scan(cnt);
+                hit = __ballot((run + incl) * unit > target);
             }
-            run += wave_total(incl);
         }
-        if (found < 0) return;
-        e = found;
-        // (found is the same in every lane: the expert's chunk register, then the lane that holds it)
-        {
-            int mv = 0;
+        if (!hit) return;
+        const int src = __ffsll(hit) - 1;
+        e = base + src;
+        const int c_e = __builtin_amdgcn_readlane(cnt, src);      // the expert's m-tiles of this class
+        int mt_class = target - (run + __builtin_amdgcn_readlane(incl - cnt, src)) * unit;
+        m_ext = __builtin_amdgcn_readlane(rows_c[0], src);
+        int first_row = __builtin_amdgcn_readlane(off_c[0], src);
+        if (many && base > 0) {
 #pragma unroll
-            for (int c = 0; c < RC; ++c)
-                if ((found >> 6) == c) mv = __builtin_amdgcn_readlane(rows_c[c], found & 63);
-            m_ext = (found >> 6) < RC ? mv : rows_of(e);
+            for (int c = 1; c < RC; ++c)
+                if (base == WAVE * c) { m_ext = __builtin_amdgcn_readlane(rows_c[c], src); first_row = __builtin_amdgcn_readlane(off_c[c], src); }
+            if (base >= WAVE * RC) { m_ext = rows_of(e); first_row = g.offsets[e]; }
         }
-        int mt_class = target - before;
-        if (mf && cnt_found / n_tiles < g.m_fastest_from) {
+        row0 = first_row;
+        if (mf && c_e < g.m_fastest_from) {
             // an expert with few m-tiles keeps the n-tile-first order (its tiles are counted one by one here)
-            nt = mt_class % n_tiles;
-            mt_class /= n_tiles;
+            const int m = mt_class / n_tiles;
+            nt = mt_class - m * n_tiles;
+            mt_class = m;
         } else if (mf) {
             // groups of G n-tiles, an expert's m-tiles of the class inside a group, the group's n-tiles innermost
             // (G = 1: m-tile first; the last group may be short)
-            const int c_e = cnt_found / n_tiles;      // the expert's m-tiles of this class
             const int G = g.m_fastest;
             const int n_groups = (n_tiles + G - 1) / G;
             const int grp = min(mt_class / (c_e * G), n_groups - 1);
@@ -839,13 +865,6 @@ __device__ __forceinline__ void gemm256_block(const GemmArgs &g, const int block
         mt = mt_class + (heavy ? 0 : heavy_of(m_ext));   // an expert's light tiles follow its heavy ones
         const int t_e = (m_ext + Q_BM - 1) / Q_BM;
         tile_h = TMB == 10 ? ((((m_ext + t_e - 1) / t_e) + 31) & ~31) : Q_BM;
-        {
-            int ov = 0;
-#pragma unroll
-            for (int c = 0; c < RC; ++c)
-                if ((found >> 6) == c) ov = __builtin_amdgcn_readlane(off_c[c], found & 63);
-            row0 = single ? 0 : ((found >> 6) < RC ? ov : g.offsets[e]);
-        }
         k_ext = g.K;
         if constexpr (EPI == EPI_PART) {
             split_k = nt / n_tiles;
@@ -958,11 +977,6 @@ __device__ __forceinline__ void gemm256_block(const GemmArgs &g, const int block
     }
 
     f32x4 acc[2 * TMW][4];
-#pragma unroll
-    for (int i = 0; i < 2 * TMW; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
     const int live = min(tile_h, m_ext - m0);
     const int tmc = (live + 31) >> 5;
     const int wu = __builtin_amdgcn_readfirstlane(wave);

@@ -730,34 +730,44 @@ __global__ __launch_bounds__(64 * NW, BPC * NW / 4) void gemm_f32_kernel(const G
     int e, mt, nt, m_ext, k_ext, split_k = 0;
     long row0;
     if constexpr (!WG) {
+        // (Nothing runs beside this search on a CU with one block: 777 tokens, top-2 of 8, 79.6 -> 78 us for it and its loads in one.  Lane l holds the rows and the first row of expert l, of later 64 if
+        // those do not reach this tile.)
         const bool single = g.offsets == nullptr;
         const int nE = single ? 1 : g.E;
-        int part = 0;
-        for (int ee = lane; ee < nE; ee += WAVE) part += ((single ? g.single_rows : g.kept[ee]) + BM - 1) / BM;
-        const int total = wave_total(wave_scan(part)) * n_units;
+        auto fetch = [&](int ee, int &rows, int &first) {
+            rows = ee < nE ? (single ? g.single_rows : g.kept[ee]) : 0;
+            first = !single && ee < nE ? g.offsets[ee] : 0;
+        };
+        int rows, first, base = 0, run = 0;
+        fetch(lane, rows, first);
+        int cnt = (rows + BM - 1) / BM, incl = wave_scan(cnt), total = wave_total(incl);
+        if (nE > WAVE) {
+            int more = 0;
+            for (int ee = lane + WAVE; ee < nE; ee += WAVE) more += (g.kept[ee] + BM - 1) / BM;
+            total += wave_total(wave_scan(more));
+        }
+        total *= n_units;
         const int per_xcd = (total + 7) >> 3;
         const int slot = blockIdx.x >> 3;
         const int t = (blockIdx.x & 7) * per_xcd + slot;
         if (slot >= per_xcd || t >= total) return;
         const int mtg = t / n_units;
-        nt = t % n_units;
-        int run = 0, found = -1, fmt = 0;
-        for (int base = 0; base < nE && found < 0; base += WAVE) {
-            const int ee = base + lane;
-            const int tiles = ee < nE ? ((single ? g.single_rows : g.kept[ee]) + BM - 1) / BM : 0;
-            const int incl = wave_scan(tiles);
-            const unsigned long long hit = __ballot(run + incl > mtg);
-            if (hit) {
-                const int src = __ffsll(hit) - 1;
-                found = base + src;
-                fmt = mtg - (run + __builtin_amdgcn_readlane(incl - tiles, src));
-            }
+        nt = t - mtg * n_units;
+        unsigned long long hit = __ballot(incl > mtg);
+        while (!hit) {
             run += wave_total(incl);
+            base += WAVE;
+            if (base >= nE) return;
+            fetch(base + lane, rows, first);
+            cnt = (rows + BM - 1) / BM;
+            incl = wave_scan(cnt);
+            hit = __ballot(run + incl > mtg);
         }
-        if (found < 0) return;
-        e = found; mt = fmt;
-        m_ext = single ? g.single_rows : g.kept[e];
-        row0 = single ? 0 : g.offsets[e];
+        const int at = __ffsll(hit) - 1;
+        e = base + at;
+        mt = mtg - (run + __builtin_amdgcn_readlane(incl - cnt, at));
+        m_ext = __builtin_amdgcn_readlane(rows, at);
+        row0 = __builtin_amdgcn_readlane(first, at);
         k_ext = g.K;
         if constexpr (EPI == EPI_PART) {
             split_k = nt / n_tiles;

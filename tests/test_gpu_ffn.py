@@ -97,6 +97,24 @@ def test_ffn_fwd_bwd_matches_oracle(E, M, Fd, rows, gap, gelu_bwd, dtype):
     assert rel_err(g_w2, 2 * w_gw2) < t and rel_err(g_b1, 2 * w_gb1) < t
 
 
+# The tile search: as many experts as a wave has lanes, one more, and more than the 256 whose rows a block holds; the last expert has rows, many
+# have none, and an expert's last tile is full, above half a tile or below.  Every row against fp32 products of its own expert.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("E", [64, 65, 257, 321])
+def test_ffn_tiles_of_many_experts(E, dtype):
+    from mole_amd import hip_ops as H
+    print(f"ffn tiles of {E} experts {dtype}", flush=True)
+    rows = [(0, 70, 128, 129, 200)[e % 5] for e in range(E - 1)] + [391]
+    d = _make(E, 64, 136, rows, dtype, seed=E)
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    out, h, a = H.ffn_fwd(c["xd"], torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda(), c["w1"], c["b1"], c["w2"], c["b2"])
+    for e in range(E):
+        r = slice(int(d["off"][e]), int(d["off"][e]) + rows[e])
+        if rows[e]:
+            assert rel_err(h[r], c["xd"][r].float() @ c["w1"][e].float().t() + c["b1"][e].float()) < tol(dtype)
+            assert rel_err(out[r], a[r].float() @ c["w2"][e].float() + c["b2"][e].float()) < tol(dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_gemm_nt_gate_logits(dtype):
     from mole_amd import hip_ops as H
