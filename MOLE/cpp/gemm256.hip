@@ -55,7 +55,8 @@ template <int TMB, int WM, int WN> struct Tile {
 // m-side tile only the 64-row groups that hold live blocks are fetched and stored, so a light tile has
 // smaller stages and its ring, in the same LDS, is deeper: light tiles do little arithmetic per stage and
 // run at the memory latency divided by the stages in flight.
-template <int TMB, int WM, int WN, bool M_KS, int TMC> struct Stage {
+// NS: stages of a full tile that the ring has room for.
+template <int TMB, int WM, int WN, bool M_KS, int TMC, int NS = Tile<TMB, WM, WN>::NSTAGE> struct Stage {
     typedef Tile<TMB, WM, WN> TL;
     static constexpr int RPL = 16 * TL::NW;                                       // rows (or 16-byte slot groups) one load of every wave covers
     static_assert(!M_KS || TL::BM % RPL == 0, "a K-strided m-side tile must be whole load rounds wide");
@@ -64,7 +65,7 @@ template <int TMB, int WM, int WN, bool M_KS, int TMC> struct Stage {
     static constexpr int L = LM + LN;                                             // loads per wave
     static constexpr int M_OPERAND = LM * RPL * Q_BK * 2;
     static constexpr int BYTES = M_OPERAND + TL::N_OPERAND;
-    static constexpr int FIT = TL::NSTAGE * TL::STAGE / BYTES;
+    static constexpr int FIT = NS * TL::STAGE / BYTES;
     static constexpr int NSTAGE = FIT > 6 ? 6 : FIT;
 };
 
@@ -331,12 +332,12 @@ template <int B, int L, int X> __device__ __forceinline__ void wait_stages_behin
 // BIAS: the accumulators start from the bias of their columns instead of zero (bias_raw: the 4 x 4 columns a lane
 // holds, fetched before the operand loads and therefore landed when the first stage has), so that the epilogue adds
 // nothing.
-template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC, int TMCW, int SUM, bool ONCE = false, int PART = 0, bool BIAS = false>
+template <int TMB, int WM, int WN, int NS, bool M_KS, bool N_KS, bool KT, int TMC, int TMCW, int SUM, bool ONCE = false, int PART = 0, bool BIAS = false>
 __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, int m_ext, const bf16_t *Np, long ldn,
                                           int n0, int n_ext, int k_ext, char *smem, int wave, int wm, int wn,
                                           f32x4 (&acc)[2 * Tile<TMB, WM, WN>::TMW][4], f32x4 (&sums)[2], const uint2 (&bias_raw)[4], const int32_t *src, int n_src) {
     typedef Tile<TMB, WM, WN> TL;
-    typedef Stage<TMB, WM, WN, M_KS, TMC> SG;
+    typedef Stage<TMB, WM, WN, M_KS, TMC, NS> SG;
     constexpr int AHEAD = SG::NSTAGE - 1, NP = 4;
     typedef Feeder<TMB, WM, WN, M_KS, N_KS, KT, TMC, ONCE> FD;
     constexpr int L = FD::L, LH = L / 2;      // loads per wave per stage; the halves are LH and L - LH
@@ -704,7 +705,7 @@ __device__ __forceinline__ void store_sums(const GemmArgs &g, const f32x4 (&sums
 // Row-ragged (!WG): C[rows_e, N] = Mop[rows_e, K] . Nop_e ; Mop K-contiguous, Nop_e [N,K] or (N_KS) [K,N].
 // Weight gradient (WG): C_e[M, N] = sum_{r in rows_e} Mop[r, M]^T . Nop[r, N], both K-strided.
 // block: the block's number among those of the product.
-template <int TMB, int WM, int WN, bool N_KS, bool WG, bool KT, int EPI>
+template <int TMB, int WM, int WN, bool N_KS, bool WG, bool KT, int EPI, int NS = Tile<TMB, WM, WN>::NSTAGE>
 __device__ __forceinline__ void gemm256_block(const GemmArgs &g, const int block, char *smem) {
     typedef Tile<TMB, WM, WN> TL;
     constexpr bool M_KS = WG;
@@ -997,7 +998,7 @@ __device__ __forceinline__ void gemm256_block(const GemmArgs &g, const int block
     f32x4 sums[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #define MOLE_RUN_TILE_AS(C, SUM, ONCE)                                                                                         \
     {                                                                                                                     \
-        main_loop<TMB, WM, WN, M_KS, N_KS, KT, WM *(C), (C), SUM, ONCE, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw, src, g.tokens); \
+        main_loop<TMB, WM, WN, NS, M_KS, N_KS, KT, WM *(C), (C), SUM, ONCE, (EPI > EPI_NONE ? EPI - EPI_NONE : 0), (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU)>(Mp, g.lda, m0, m_ext, Np, g.ldb, n0, g.N, k_ext, smem, wu, wm, wn, acc, sums, bias_raw, src, g.tokens); \
         if constexpr (SUM != 0) store_sums<SUM, (C)>(g, sums, e, m0, n0, m_ext, wm, wn, lane);                            \
         epilogue<TMB, WM, WN, WG, EPI, (C), KT && !WG>(g, acc, smem, lane, wu, wn, e, row0, m0w, n0, m_ext, live_w, split_k);      \
     }
@@ -1035,11 +1036,12 @@ __global__ __launch_bounds__((Tile<TMB, WM, WN>::THREADS), (Tile<TMB, WM, WN>::W
 // one block's chain of waits, and the weight gradient many short blocks that fill just such holes.  The long blocks start first.
 // Bound by latency.  Training passes, apart / together: 2 x 513 tokens, 16 experts top-4, 520 -> 1416, 366 / 322 us; 2 x 130, 6 of 824 -> 824,
 // top-6, skewed, 300 / 255; 2048 tokens, 16 of 512 -> 1024, top-2, 119 / 113.5.
-template <bool N_KS, bool KT, int EPI>
-__global__ __launch_bounds__((Tile<4, 2, 2>::THREADS), (Tile<4, 2, 2>::WAVES_PER_SIMD)) void gemm256_pair_kernel(const GemmArgs g, const GemmArgs w, int first) {
+// NS: stages of the ring, five in two blocks to a CU or three in three.
+template <bool N_KS, bool KT, int EPI, int NS>
+__global__ __launch_bounds__((Tile<4, 2, 2>::THREADS), (NS == 3 ? 3 : Tile<4, 2, 2>::WAVES_PER_SIMD)) void gemm256_pair_kernel(const GemmArgs g, const GemmArgs w, int first) {
     extern __shared__ __align__(16) char smem[];
-    if ((int)blockIdx.x < first) gemm256_block<4, 2, 2, N_KS, false, KT, EPI>(g, blockIdx.x, smem);
-    else gemm256_block<4, 2, 2, true, true, true, EPI_WGRAD>(w, (int)blockIdx.x - first, smem);
+    if ((int)blockIdx.x < first) gemm256_block<4, 2, 2, N_KS, false, KT, EPI, NS>(g, blockIdx.x, smem);
+    else gemm256_block<4, 2, 2, true, true, true, EPI_WGRAD, NS>(w, (int)blockIdx.x - first, smem);
 }
 
 template <int TMB, int WM, int WN, bool N_KS, bool WG, bool KT, int EPI>
@@ -1248,20 +1250,31 @@ static int plan256(GemmArgs &gp, bool b_ks, int &epi, int max_rows, void *ws, si
     return p.tile;
 }
 
-template <bool N_KS, bool KT, int EPI> static int launch_pair_kt(const GemmArgs &g, const GemmArgs &w, int max_rows, hipStream_t st, int kid) {
+template <bool N_KS, bool KT, int EPI, int NS = Tile<4, 2, 2>::NSTAGE> static int launch_pair_kt(const GemmArgs &g, const GemmArgs &w, int max_rows, hipStream_t st, int kid) {
     typedef Tile<4, 2, 2> TL;
     const int first = ragged_blocks(g, EPI, max_rows, TL::BM, ceil_div(g.N, TL::BN)), rest = wgrad_blocks(w, TL::BM, ceil_div(w.N, TL::BN));
-    auto kern = gemm256_pair_kernel<N_KS, KT, EPI>;
+    auto kern = gemm256_pair_kernel<N_KS, KT, EPI, NS>;
+    constexpr int lds = NS * TL::STAGE > TL::SLABS ? NS * TL::STAGE : TL::SLABS;
     static bool attr_done = false;
     if (!attr_done) {
-        MOLE_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS_BYTES));
+        MOLE_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         attr_done = true;
     }
-    timed_launch(kid, kern, dim3(first + rest), dim3(TL::THREADS), TL::LDS_BYTES, st, g, w, first);
+    timed_launch(kid, kern, dim3(first + rest), dim3(TL::THREADS), lds, st, g, w, first);
     MOLE_LAUNCH_CHECK();
     return 0;
 }
 template <bool N_KS, int EPI> static int launch_pair(const GemmArgs &g, const GemmArgs &w, int max_rows, hipStream_t st, int kid) {
+    // t walks over K = M, few stages beside gx's K = F.  Where its tiles are an eighth more than the CUs and all of them more than two a CU,
+    // a third block counts for more than stages in flight (19 of 24 launches of random sizes beyond the line 1 to 15 % faster, two 5 % slower; us, two blocks / three: 2 x 513 tokens, top-4 of 16, 520 -> 1416 33.6 / 32.1; 2048 of the
+    // padded layout, 16 of 512 -> 1024 24.4 / 21.4; 571, top-8 of 22, 384 -> 768 22.0 / 19.2; 1587, 10 of 704 -> 2816 34.1 / 29.5; fewer tiles: 654,
+    // top-2 of 13, 520 -> 1560 21.4 / 24.8; 1825, 17 of 1016 -> 1016 30.3 / 36.9; gx of the first two 31.4 / 37.2, 19.7 / 23.0).
+    if constexpr (EPI == EPI_DGELU) {
+        const int active = g.E < g.est_rows ? g.E : g.est_rows;
+        const double tiles = (g.est_rows / 128.0 + 0.5 * active) * ceil_div(g.N, 128);      // (an expert's last one is half full in the mean)
+        if (tiles >= 288.0 && tiles + (double)w.E * ceil_div(w.M, 128) * ceil_div(w.N, 128) >= 640)
+            return g.K % Q_BK ? launch_pair_kt<N_KS, true, EPI, 3>(g, w, max_rows, st, kid) : launch_pair_kt<N_KS, false, EPI, 3>(g, w, max_rows, st, kid);
+    }
     return g.K % Q_BK ? launch_pair_kt<N_KS, true, EPI>(g, w, max_rows, st, kid) : launch_pair_kt<N_KS, false, EPI>(g, w, max_rows, st, kid);
 }
 // The row-ragged product g (EPI_DGELU, or EPI_STORE with K-strided weights) and the weight gradient w together where both take 128 x 128

@@ -458,8 +458,8 @@ __device__ __forceinline__ bool f32_loop(const GemmArgs &g, const float *Mp, con
 }
 
 // A stage of 32 of k of an operand tile of ROWS rows, as parts in LDS: the 16 bytes at ((4 part + h) ROWS + (row ^ X(h))) 16 hold the eight k
-// of eighth h of a row.  A fragment read (lane l: row l % 32, eighth l / 32 of a half stage) is two stretches of 512 bytes; X keeps the
-// eighths that the lanes of a wave write together on different banks, whichever 32 of them a pass takes.
+// of eighth h of a row.  A fragment read (lane l: row l % 16, eighth l / 16) is four stretches of 256 bytes; X, 12 for odd h, keeps what a
+// pass of it takes of two stretches on different banks (X = 4 h, which the writes would like better: 6 % slower in all).
 template <int ROWS> struct Parts {
     static constexpr int PLANE = 4 * ROWS * 16, BYTES = 3 * PLANE;
     static __device__ __forceinline__ uint32_t at(int h, int row) { return (uint32_t)((h * ROWS + (row ^ ((h & 1) * 12))) * 16); }

@@ -115,6 +115,14 @@ def test_ffn_tiles_of_many_experts(E, dtype):
             assert rel_err(out[r], a[r].float() @ c["w2"][e].float() + c["b2"][e].float()) < tol(dtype)
 
 
+# t and g_w2 in one launch with a ring of three stages (many tiles of few rows): contractions of one stage, of one and a rest, of three and of a rest
+# and three, which fill the ring and go round it.
+@pytest.mark.parametrize("M", [32, 40, 96, 104])
+def test_ffn_backward_pair_with_three_stages(M):
+    rows = [(30, 70, 128, 129, 1, 0, 100, 140)[e % 8] for e in range(32)]
+    test_ffn_fwd_bwd_matches_oracle(32, M, 1416, rows, 0, "exact", torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_gemm_nt_gate_logits(dtype):
     from mole_amd import hip_ops as H
