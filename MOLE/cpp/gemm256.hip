@@ -1161,9 +1161,9 @@ static int dispatch256(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_r
 //     512 -> 1024: h 20.9 -> 14.7 us, out 26 -> 14); with more, their operand bytes per flop cost more than the idle CUs
 //     (16 experts of 375 rows, 1024 -> 4096: h 109 against 83 us).  Their K = F products are split as well while the tiles
 //     leave CUs idle (8 experts of 194 rows, 512 -> 2048: out 25 -> 16 us).  out, which runs alone (gx shares its launch with a weight gradient),
-//     goes on to the CUs' second blocks where experts have more than one m-tile and the shorter walk, 0.4 us for 32 of K (where rows are not whole pieces 0.48), saves more than the planes
-//     cost: forward passes of 513 tokens, top-4 of 16, 520 -> 1416 57.8 -> 51.9 us; 1480, top-2 of 24, 448 -> 1792 56.0 -> 51.9; 641, top-4 of 22,
-//     512 -> 1536 57.1 -> 52.9.  On the other side of the line: 748, top-6 of 6, 512 -> 1024 48.6 / 53.8; 3854, top-1 of 22, 512 -> 2048
+//     goes on to the CUs' second blocks where experts have more than one m-tile and the shorter walk, 0.4 us for 32 of K, saves more than the planes
+//     cost: forward passes of 1480 tokens, top-2 of 24, 448 -> 1792 56.0 -> 51.9 us; 601, top-4 of 8, 704 -> 2816 74.5 -> 67.1; 799, top-2 of 9,
+//     904 -> 2712 82.0 -> 71.1.  On the other side of the line: 748, top-6 of 6, 512 -> 1024 48.6 / 53.8; 3854, top-1 of 22, 512 -> 2048
 //     (training) 171 / 173; one m-tile an expert, whose weights' stream bounds it: 304, top-8 of 33, 480 -> 1920 69.0 / 73.5.
 enum { TILE_256, TILE_320, TILE_128 };
 struct TilePlan { int tile, ksplit; };
@@ -1195,8 +1195,8 @@ static TilePlan tile_plan(int E, int est_rows, int N, int K, bool tall, bool alo
         const long fit = 256 / t128, most = K / 512;
         p.ksplit = (int)(fit < most ? fit : most);
         p.ksplit = p.ksplit < 1 ? 1 : (p.ksplit > 4 ? 4 : p.ksplit);
-        auto us = [&](int q) {       // a plane's element is written and read in fp32 instead of once in bf16
-            const double walk = K / 32 * (K % 32 ? 0.48 : 0.4) / q * (t128 * q > 256 ? 1.15 : 1.0), stream = 2.0 * active * N * K / 4.0e6;
+        auto us = [&](int q) {       // a plane's element is written and read in fp32 instead of once in bf16; whole stages only, so that all widths of the same tiles go alike
+            const double walk = K / 32 * 0.4 / q * (t128 * q > 256 ? 1.15 : 1.0), stream = 2.0 * active * N * (K / 32 * 32) / 4.0e6;
             return (walk > stream ? walk : stream) + (q > 1 ? (8.0 * q - 4.0) * est_rows * N / 2.7e6 + 1.0 : 0.0);
         };
         if (alone && full > 128)
