@@ -1160,14 +1160,10 @@ static int dispatch256(const GemmArgs &g, bool b_ks, bool wg, int epi, int max_r
 //   * the others run 128 x 128 tiles of four waves, two blocks to a CU, up to 112 large tiles (16 experts of 256 rows,
 //     512 -> 1024: h 20.9 -> 14.7 us, out 26 -> 14); with more, their operand bytes per flop cost more than the idle CUs
 //     (16 experts of 375 rows, 1024 -> 4096: h 109 against 83 us).  Their K = F products are split as well while the tiles
-//     leave CUs idle (8 experts of 194 rows, 512 -> 2048: out 25 -> 16 us).  out, which runs alone (gx shares its launch with a weight gradient),
-//     goes on to the CUs' second blocks where experts have more than one m-tile and the shorter walk, 0.4 us for 32 of K, saves more than the planes
-//     cost: forward passes of 1480 tokens, top-2 of 24, 448 -> 1792 56.0 -> 51.9 us; 601, top-4 of 8, 704 -> 2816 74.5 -> 67.1; 799, top-2 of 9,
-//     904 -> 2712 82.0 -> 71.1.  On the other side of the line: 748, top-6 of 6, 512 -> 1024 48.6 / 53.8; 3854, top-1 of 22, 512 -> 2048
-//     (training) 171 / 173; one m-tile an expert, whose weights' stream bounds it: 304, top-8 of 33, 480 -> 1920 69.0 / 73.5.
+//     leave CUs idle (8 experts of 194 rows, 512 -> 2048: out 25 -> 16 us).
 enum { TILE_256, TILE_320, TILE_128 };
 struct TilePlan { int tile, ksplit; };
-static TilePlan tile_plan(int E, int est_rows, int N, int K, bool tall, bool alone) {
+static TilePlan tile_plan(int E, int est_rows, int N, int K, bool tall) {
     TilePlan p{TILE_256, 1};
     const int active = E < est_rows ? E : est_rows;
     if (active <= 0) return p;
@@ -1195,13 +1191,6 @@ static TilePlan tile_plan(int E, int est_rows, int N, int K, bool tall, bool alo
         const long fit = 256 / t128, most = K / 512;
         p.ksplit = (int)(fit < most ? fit : most);
         p.ksplit = p.ksplit < 1 ? 1 : (p.ksplit > 4 ? 4 : p.ksplit);
-        auto us = [&](int q) {       // a plane's element is written and read in fp32 instead of once in bf16; whole stages only, so that all widths of the same tiles go alike
-            const double walk = K / 32 * 0.4 / q * (t128 * q > 256 ? 1.15 : 1.0), stream = 2.0 * active * N * (K / 32 * 32) / 4.0e6;
-            return (walk > stream ? walk : stream) + (q > 1 ? (8.0 * q - 4.0) * est_rows * N / 2.7e6 + 1.0 : 0.0);
-        };
-        if (alone && full > 128)
-            for (int q = p.ksplit + 1; q <= 4 && q * t128 <= 512 && q <= most; ++q)
-                if (us(q) < 0.9 * us(p.ksplit)) p.ksplit = q;
     }
     return p;
 }
@@ -1222,7 +1211,7 @@ static int wgrad_tile(int E, int est_rows, int M, int N) {
     if (active > 0 && est_rows <= 24l * active && t128 <= 32768) return TILE_128;
     return t128 < 768 * ((t256 + 255) / 256) ? TILE_128 : TILE_256;
 }
-int gemm256_ksplit(int E, int est_rows, int N, int K) { return tile_plan(E, est_rows, N, K, true, true).ksplit; }
+int gemm256_ksplit(int E, int est_rows, int N, int K) { return tile_plan(E, est_rows, N, K, true).ksplit; }
 
 // Whether the weight-gradient launch for g will also produce the operand sums asked for in g.colsum.
 bool gemm256_sums_operand(const GemmArgs &g) {
@@ -1238,7 +1227,7 @@ static bool aligned256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg) {
 // the tile of a row-ragged product; where its contraction is split, gp and epi become those of the planes
 static int plan256(GemmArgs &gp, bool b_ks, int &epi, int max_rows, void *ws, size_t ws_bytes) {
     TilePlan p{TILE_256, 1};
-    if (gp.offsets != nullptr && epi < EPI_NONE) p = tile_plan(gp.E, gp.est_rows, gp.N, gp.K, b_ks, epi == EPI_BIAS);
+    if (gp.offsets != nullptr && epi < EPI_NONE) p = tile_plan(gp.E, gp.est_rows, gp.N, gp.K, b_ks);
     p.ksplit = planes_allowed(p.ksplit, max_rows, gp.est_rows, gp.N);
     gp.ksplit = 1;
     if (p.ksplit > 1 && b_ks && ws != nullptr && ws_bytes >= (size_t)p.ksplit * max_rows * gp.N * sizeof(float)) {

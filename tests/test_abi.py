@@ -299,3 +299,11 @@ def test_bf16_planes_of_widths_that_end_inside_a_stage():
     for E, rows, M, F in ((16, 2052, 520, 1416), (16, 4104, 520, 1416), (8, 1600, 1032, 2056), (20, 2600, 264, 1032), (8, 800, 520, 1032)):
         assert planes(E, rows, M, F) == planes(E, rows, M, F // 32 * 32), (E, rows, M, F)
     assert planes(16, 2052, 520, 1416) == 0
+
+
+def test_bf16_scratch_is_no_more_than_both_directions_use():
+    """A layer's scratch is laid out once for its two narrow products: out is split into no more planes than gx, which shares a launch
+    (layers of several 128-row tiles an expert that leave half of the CUs' block slots idle)."""
+    from mole_amd import _lib as L
+    for E, rows, M, F in ((9, 1609, 904, 2712), (9, 2384, 640, 1920), (24, 2976, 448, 1792)):
+        assert L.lib().mole_ffn_workspace_bytes(L.MOLE_BF16, E, rows, M, F) == 0, (E, rows, M, F)

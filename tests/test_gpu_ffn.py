@@ -777,21 +777,6 @@ def test_ffn_few_rows_with_infinite_weights(E, M, Fd, rows, dtype):
             assert _same_class(gx, want)
 
 
-# out of 128 x 128 tiles that leave the CUs' second blocks idle, in two planes: contractions of 84.75, 60 and 56 stages of 32, experts of one and of two
-# m-tiles, columns that end in a tile.  bf16 results of fp32 sums in another order: the tolerance of every FFN test.
-@pytest.mark.parametrize("E,M,Fd,rows", [(9, 904, 2712, [129, 256, 97, 128, 257, 200, 192, 150, 190]), (10, 640, 1920, [131, 172, 150, 129, 200] * 2), (24, 448, 1792, [140, 97, 160, 129, 90, 128] * 4)])
-def test_ffn_split_contraction_of_second_blocks(E, M, Fd, rows):
-    from mole_amd import hip_ops as H, _lib as L
-    print(f"split contraction of second blocks E={E} M={M} F={Fd}", flush=True)
-    d = _make(E, M, Fd, rows, torch.bfloat16, seed=E + M)
-    assert L.lib().mole_ffn_workspace_bytes(L.MOLE_BF16, E, d["R"], M, Fd) == 2 * d["R"] * M * 4
-    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
-    out, _, a = H.ffn_fwd(c["xd"], torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda(), c["w1"], c["b1"], c["w2"], c["b2"])
-    for e in range(E):
-        r = slice(int(d["off"][e]), int(d["off"][e]) + rows[e])
-        assert rel_err(out[r], a[r].float() @ c["w2"][e].float() + c["b2"][e].float()) < tol(torch.bfloat16)
-
-
 def test_ffn_split_contraction_of_more_than_2_to_18_rows():
     """The reduction of a split contraction has a block for every four rows: more of them than a grid has in y.  fp32, rows of
     eight columns; out against torch's fp32 products of the same activations (two orders of 1024 terms: 2^-24 sqrt(1024) of
