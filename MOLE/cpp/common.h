@@ -121,7 +121,7 @@ struct DispatchHead;
 // what the caller knows of the rows beside their bound: how many all experts hold in all likelihood, and the most that one can hold
 struct Rows { int est, most; };
 // the FFN's entry points with these (ffn_gemm.hip)
-size_t ffn_workspace_bytes(int dtype, int E, int max_rows, Rows rows, int M, int F);
+size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, int F, bool least);     // least: what a call needs at least
 size_t gate_route_least_bytes(int dtype, int S, int E, int M, int k);     // gate_route's without small blocks
 int gate_route(const void *x, int dtype, const float *wg, const float *logit_bias, int S, int E, int M, int k, double capacity_factor,
                int normalize_gate, int alignment, int layout, float *scores, int32_t *idx, int32_t *loc, float *gates, int32_t *row, int32_t *counts,

@@ -22,6 +22,8 @@
 
 #include <stdlib.h>
 
+#include <algorithm>
+
 namespace mole {
 
 // ---------------------------------------------------------------------------------------------
@@ -590,11 +592,17 @@ using namespace mole;
 
 namespace mole {
 
-size_t ffn_workspace_bytes(int dtype, int E, int max_rows, Rows rows, int M, int F) {
+size_t ffn_workspace_bytes(int dtype, int E, int max_rows, int est_rows, int M, int F, bool least) {
     if (E <= 0 || max_rows <= 0 || M <= 0 || F <= 0) return 0;
-    int ks = gemm_skinny_ksplit(E, max_rows, rows.est, M, F, dtype);
-    if (ks == 0) ks = dtype == MOLE_BF16 ? gemm256_ksplit(E, rows.est, M, F) : gemm_f32_ksplit(E, rows, M, F);
-    ks = planes_allowed(ks, max_rows, rows.est, M);
+    int ks = gemm_skinny_ksplit(E, max_rows, est_rows, M, F, dtype);
+    if (ks == 0 && dtype == MOLE_BF16) ks = gemm256_ksplit(E, est_rows, M, F);
+    else if (ks == 0) {
+        // (whatever the most rows of an expert, which come from the capacity factor: a caller may set it after its scratch was laid out)
+        const int bounded = gemm_f32_ksplit(E, Rows{est_rows, 0}, M, F, 4), unbounded = gemm_f32_ksplit(E, Rows{est_rows, max_rows}, M, F, 4);
+        const int laid_out = gemm_f32_planes_laid_out(E, est_rows, M, F);
+        ks = least ? std::min({bounded, unbounded, laid_out}) : std::max({bounded, unbounded, laid_out});
+    }
+    ks = planes_allowed(ks, max_rows, est_rows, M);
     return ks > 1 ? (size_t)ks * max_rows * M * sizeof(float) : 0;
 }
 
@@ -636,7 +644,7 @@ int ffn_bwd(const void *go, const void *xd, const void *h, const void *a, int dt
 }  // namespace mole
 
 extern "C" size_t mole_ffn_workspace_bytes(int dtype, int E, int max_rows, int M, int F) {
-    return ffn_workspace_bytes(dtype, E, max_rows, Rows{max_rows, max_rows}, M, F);
+    return ffn_workspace_bytes(dtype, E, max_rows, max_rows, M, F, false);
 }
 
 extern "C" int mole_ffn_fwd_ws(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,

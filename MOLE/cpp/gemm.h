@@ -207,7 +207,8 @@ bool gemm_skinny_takes_tokens(int E, int max_rows, int est_rows, int N, int K, i
 int gemm_skinny_ksplit(int E, int max_rows, int est_rows, int N, int K, int dtype);    // 0: not its shape
 // fp32 tiles with direct-to-LDS loads (gemm_f32.hip); -100 as above.
 int launch_gemm_f32(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, int max_rows, void *ws, size_t ws_bytes, hipStream_t st, int kid);
-int gemm_f32_ksplit(int E, Rows rows, int N, int K);
+int gemm_f32_ksplit(int E, Rows rows, int N, int K, int room);      // of at most `room` planes
+int gemm_f32_planes_laid_out(int E, int est_rows, int N, int K);
 bool gemm_f32_takes(int N, int K);      // the widths of a row-ragged product
 bool gemm_f32_sums_operand(const GemmArgs &g);
 

@@ -1127,16 +1127,33 @@ static int f32_tile(int p, int E, Rows rows, int N, int K, bool heavy) {
     if (E <= 0 || rows.est <= 0 || N <= 64) return 64;      // (half of the columns or more are padding: 64 rows pad less)
     return f32_cost(128, p, E, rows, N, K, heavy) < f32_cost(64, p, E, rows, N, K, heavy) ? 128 : 64;
 }
-int gemm_f32_ksplit(int E, Rows rows, int N, int K) {
+int gemm_f32_ksplit(int E, Rows rows, int N, int K, int room) {
     if (E <= 0 || rows.est <= 0 || K % F_BK) return 1;
     int best = 1;
     double least = 0.0;
-    for (int p = 1; p <= 4 && (p == 1 || K / p >= 16 * F_BK); ++p) {
+    for (int p = 1; p <= room && (p == 1 || K / p >= 16 * F_BK); ++p) {
         const int bm = f32_tile(p, E, rows, N, K, false);
         double us = f32_cost(bm, p, E, rows, N, K, false);
         if (bm == 64 && f32_tiles(64, p, E, rows, N) <= 256.0) us += 0.1 * K / F_BK / p;      // of near equals the one with parts, whose results are closer
         if (p == 1 || us < least) { least = us; best = p; }
     }
+    return best;
+}
+
+// The planes that callers laid scratch out for when a launch had tiles of own parts or fp32 operands alone, of either height, and its rows were taken to
+// lie evenly: scratch of that size stays enough.  It has no say in which way a launch goes.
+int gemm_f32_planes_laid_out(int E, int est_rows, int N, int K) {
+    if (E <= 0 || est_rows <= 0 || K % F_BK) return 1;
+    const int active = E < est_rows ? E : est_rows;
+    auto us = [&](int bm, int p) {
+        const long rounds = ((long)p * active * ceil_div(ceil_div(est_rows, active), bm) * ceil_div(N, 128) + 255) / 256;
+        const double stages = K / F_BK / (double)p, planes = p > 1 ? p * (2.0 * est_rows * N * sizeof(float) / 5.0e6) + 6.0 : 0.0;
+        return bm == 64 ? rounds * (rounds == 1 ? 0.52 : 0.47) * stages + planes : rounds * ((rounds == 1 ? 0.88 : 0.76) * stages + 3.0) + planes;
+    };
+    auto least = [&](int p) { return N <= 64 ? us(64, p) : std::min(us(64, p), us(128, p)); };
+    int best = 1;
+    for (int p = 2; p <= 4 && K / p >= 16 * F_BK; ++p)
+        if (least(p) < least(best)) best = p;
     return best;
 }
 
@@ -1151,9 +1168,11 @@ int launch_gemm_f32(const GemmArgs &g0, bool a_ks, bool b_ks, bool wg, int epi, 
     if (!wg && (a_ks || !gemm_f32_takes(g.N, g.K))) return -100;
     if (wg && (!a_ks || !b_ks || g.M % 4 || g.M < 4)) return -100;
     if (wg) return dispatch_f32<128, 128, 4, 4, 2, OWN_PARTS>(g, b_ks, wg, epi, max_rows, st, kid);
-    if (b_ks && g.offsets != nullptr && ws != nullptr) {
-        const int p = planes_allowed(gemm_f32_ksplit(g.E, rows, g.N, g.K), max_rows, g.est_rows, g.N);
-        if (p > 1 && ws_bytes >= (size_t)p * max_rows * g.N * sizeof(float)) {
+    if (b_ks && g.offsets != nullptr && ws != nullptr && max_rows > 0) {
+        // as many planes as the scratch has room for, at most
+        const int room = planes_allowed((int)std::min<size_t>(4, ws_bytes / ((size_t)max_rows * g.N * sizeof(float))), max_rows, g.est_rows, g.N);
+        const int p = gemm_f32_ksplit(g.E, rows, g.N, g.K, room);
+        if (p > 1) {
             g.ksplit = p;
             g.part = (float *)ws;
             g.part_rows = max_rows;

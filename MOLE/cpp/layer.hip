@@ -20,6 +20,7 @@ static Rows rows_of(const mole_layer &L) {
     const double capacity = L.capacity_factor > 0. ? (double)L.k * std::floor(L.capacity_factor * ((L.S + L.E - 1) / L.E)) : (double)L.S;
     return Rows{est_rows(L), capacity < L.S ? (int)capacity : L.S};
 }
+static size_t planes_bytes(const mole_layer &L, bool least) { return ffn_workspace_bytes(L.dtype, L.E, L.rows, est_rows(L), L.M, L.F, least); }
 
 // Whether the first product reads the tokens through the list although their rows are written for later: where the rows of several choices are
 // more than the last-level cache holds and the tokens are well below it, so that the tokens come from the cache and the rows do not.  Training
@@ -106,7 +107,7 @@ using namespace mole;
 
 extern "C" size_t mole_layer_workspace_bytes(const mole_layer *L, int backward) {
     if (L == nullptr || L->S <= 0 || L->E <= 0) return 0;
-    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, rows_of(*L), L->M, L->F);
+    const size_t ffn = planes_bytes(*L, false);
     size_t other = backward ? gate_bwd_plan(*L, gate_wgrad_by_tiles(*L)).total : mole_gate_route_shape_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
     if (!backward && tokens_beside_rows(*L)) other = up256(other) + (size_t)L->rows * 4;
     return ffn > other ? ffn : other;        // the two are never in use at the same time
@@ -123,8 +124,8 @@ static int check_layer(const char *fn, const mole_layer *L, mole_stream_t) {
 extern "C" int mole_layer_fwd(const mole_layer *L, void *y, mole_stream_t stream) {
     if (int rc = check_layer("mole_layer_fwd", L, stream)) return rc;
     const size_t route_bytes = mole_gate_route_shape_workspace_bytes(L->dtype, L->S, L->E, L->M, L->k);
-    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, rows_of(*L), L->M, L->F), need = std::max(route_bytes, ffn);
-    if (L->workspace_bytes < std::max(gate_route_least_bytes(L->dtype, L->S, L->E, L->M, L->k), ffn)) {
+    const size_t need = std::max(route_bytes, planes_bytes(*L, false));
+    if (L->workspace_bytes < std::max(gate_route_least_bytes(L->dtype, L->S, L->E, L->M, L->k), planes_bytes(*L, true))) {
         set_error("mole_layer_fwd: workspace of %zu bytes, need %zu", L->workspace_bytes, need);
         return MOLE_E_WORKSPACE;
     }
@@ -170,11 +171,11 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
     if (int rc = check_layer("mole_layer_bwd", L, stream)) return rc;
     MOLE_REQUIRE(!L->forward_only, "mole_layer_bwd: the forward pass was a forward_only one");
     MOLE_REQUIRE(G && G->dy && G->dlogits && G->d_o && G->t && G->gxd && G->dx && G->dwg, "mole_layer_bwd: null gradient pointer");
-    const size_t ffn = ffn_workspace_bytes(L->dtype, L->E, L->rows, rows_of(*L), L->M, L->F);
+    const size_t ffn = planes_bytes(*L, true);
     GateBwdPlan p = gate_bwd_plan(*L, gate_wgrad_by_tiles(*L));
-    const size_t need = std::max(ffn, p.total);
+    const size_t need = std::max(planes_bytes(*L, false), p.total);
     // (a workspace that does not hold the partial sums of a large gate has its weight gradient by the tiles)
-    if (L->workspace_bytes < need && gate_wgrad_may_go_by_tiles(*L)) p = gate_bwd_plan(*L, true);
+    if (L->workspace_bytes < p.total && gate_wgrad_may_go_by_tiles(*L)) p = gate_bwd_plan(*L, true);
     if (L->workspace_bytes < std::max(ffn, p.total)) {
         set_error("mole_layer_bwd: workspace of %zu bytes, need %zu", L->workspace_bytes, need);
         return MOLE_E_WORKSPACE;

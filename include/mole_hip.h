@@ -244,7 +244,7 @@ int mole_ffn_bwd(const void *go, const void *xd, const void *h, const void *a, i
 /* The same two calls with a workspace.  With few rows per expert the two products whose contraction runs over F are
  * narrow (M columns) and long; given mole_ffn_workspace_bytes() bytes (0: none needed) the library splits the
  * contraction over several blocks and adds the fp32 partial results in a fixed order.  A smaller or NULL workspace is
- * allowed: the contraction is then not split. */
+ * allowed: the contraction is then split less (fp32) or not at all. */
 size_t mole_ffn_workspace_bytes(int dtype, int E, int max_rows, int M, int F);
 int mole_ffn_fwd_ws(const void *xd, int dtype, const int32_t *offsets, const int32_t *kept_rows, int E,
                     int max_rows, int M, int F, const void *w1, const void *b1, const void *w2,

@@ -307,3 +307,25 @@ def test_bf16_scratch_is_no_more_than_both_directions_use():
     from mole_amd import _lib as L
     for E, rows, M, F in ((9, 1609, 904, 2712), (9, 2384, 640, 1920), (24, 2976, 448, 1792)):
         assert L.lib().mole_ffn_workspace_bytes(L.MOLE_BF16, E, rows, M, F) == 0, (E, rows, M, F)
+
+
+def test_layer_scratch_is_told_from_the_sizes_alone():
+    """mole_layer_workspace_bytes reads the sizes of the block: the capacity factor, which a caller may set after it has laid the scratch out,
+    changes nothing at equal sizes."""
+    import ctypes
+    import random
+    import struct
+    from mole_amd import _lib as L
+    rng = random.Random(2)
+    sizes = [(L.MOLE_F32, 757, 512, 32, 4, 1024)]
+    for _ in range(4000):
+        E, grain = rng.randint(2, 64), rng.choice([64, 16, 8])
+        M = grain * rng.randint(1, 1024 // grain)
+        sizes.append((rng.choice([L.MOLE_F32, L.MOLE_F32, L.MOLE_BF16]), int(2 ** rng.uniform(0, 14)), M, E, rng.randint(1, min(E, 8)), rng.choice([1, 2, 4]) * M))
+    for dtype, S, M, E, k, F in sizes:
+        for backward in (0, 1):
+            need = set()
+            for cf in (0.0, 0.5, 1.0, 1.25, 2.0):
+                block = ctypes.create_string_buffer(struct.pack("10id", dtype, S, M, E, k, F, S * k, L.LAYOUT_RAGGED, 1, 0, cf), 512)
+                need.add(L.lib().mole_layer_workspace_bytes(ctypes.cast(block, ctypes.c_void_p), backward))
+            assert len(need) == 1, (dtype, S, M, E, k, F, need)

@@ -1174,6 +1174,24 @@ def test_gate_weight_gradient_on_either_side_of_the_tiles(S, M, E, Fd, dtype, ti
         assert bool(((t["dwg"].double().cpu() - dl.t() @ x64).abs() <= bound).all())
 
 
+# fp32 layers whose scratch was laid out for fewer planes of out and gx than the present rule takes (none of two, two of three, two of four):
+# they run in the planes that it holds.  Two orders of a sum of Fd fp32 products: 2^-24 sqrt(Fd) each in the 2-norm.
+@pytest.mark.parametrize("S,M,E,k,Fd,planes", [(203, 1024, 14, 4, 512, 0), (888, 320, 15, 2, 960, 2), (285, 2048, 3, 1, 1024, 2)])
+def test_layer_with_scratch_of_fewer_planes(S, M, E, k, Fd, planes):
+    print(f"scratch of fewer planes S={S} M={M} E={E} k={k} F={Fd}", flush=True)
+    m, x, _ = _build(S, M, E, k, Fd, torch.float32, seed=S)
+    whole = _native_training_pass(m, x, E, k, Fd, 0.0)
+    sizes = []
+    for backward in (0, 1):
+        need = [L.lib().mole_layer_workspace_bytes(ctypes.byref(_Layer(L.MOLE_F32, S, M, E, k, width, S * k, L.LAYOUT_RAGGED, 1, 0, 0.0)), backward) for width in (16, Fd)]
+        sizes.append(max(need[0], planes * S * k * M * 4))
+        assert sizes[backward] < need[1]
+    t = _native_training_pass(m, x, E, k, Fd, 0.0, sizes=sizes)
+    for n in ("out", "gxd"):
+        assert float((t[n] - whole[n]).double().norm() / whole[n].double().norm()) <= 2 * 2.0 ** -24 * Fd ** 0.5
+    assert torch.equal(t["a"], whole["a"]) and torch.equal(t["idx"], whole["idx"])
+
+
 # Workspaces of the least sizes: histograms of blocks of 64 tokens and whole logits for the forward pass, operands and results of the gate's two products
 # for the backward one.  The pass is the same but for the order of the loss term's sums and a large gate's weight gradient, which is then the tiles'.
 @pytest.mark.parametrize("S,M,E,k,Fd,dtype", [(40, 128, 70, 1, 16, torch.bfloat16), (500, 64, 256, 1, 16, torch.bfloat16), (60, 136, 20, 2, 32, torch.bfloat16),
