@@ -810,12 +810,13 @@ __global__ __launch_bounds__(256, 2) void gate_wgrad_mfma_kernel(const float *__
 // it is multiplied; partial sums in memory and a second launch for them cost more up to the lines of gate_wgrad_direct_ok.
 // Neither operand is contiguous along the tokens that are summed over, and there is no LDS on the way in:
 //   bf16 tokens: a lane loads two columns of eight tokens and one expert's gradient of each, and turns them in registers for
-//       v_mfma_f32_16x16x32_bf16.  The gradients enter as three bf16 numbers each, 24 bits.  The first ones' products have an accumulator
-//       of their own, and where that is not finite it is the result: the later parts of an infinity, or times one, are NaN.
+//       v_mfma_f32_16x16x32_bf16.  The gradients enter as three bf16 numbers each, 24 bits, and the first ones' products have an accumulator
+//       of their own.  Results of a block that met a gradient below 2^-110 that is not zero, whose last part may be below the smallest bf16
+//       number, and results that are not finite (an infinity has no parts, nor has a gradient that bf16 rounds to one) are formed again in fp32.
 //   fp32 tokens: v_mfma_f32_16x16x4_f32 on the values as they come, four tokens an instruction, in four accumulators in turn: the fewer
 //       roundings a sum has in a row, the closer it is (513 tokens, 2-norm error 1.27e-7 with one, 1.01e-7 with four).
 // cols, group: the block's 32 columns and 16 experts; s_sum: its LDS, GD_LDS floats.
-template <int NW> constexpr int GD_LDS = NW * 16 * 32;
+template <int NW> constexpr int GD_LDS = NW * 16 * 32 + NW;
 template <typename T, int NW>
 __device__ __forceinline__ void gate_wgrad_direct_block(const int cols, const int group, float *s_sum, const float *__restrict__ dlogits, const T *__restrict__ x, int S, int E, int M,
                                                         float *__restrict__ dwg) {
@@ -844,6 +845,7 @@ __device__ __forceinline__ void gate_wgrad_direct_block(const int cols, const in
             p.d[u] = dc[t * E];
         }
     };
+    uint32_t least = 0xffffffffu;            // of the gradients' magnitudes: their bits doubled, less one (zero: the largest)
     constexpr int NA = BF ? 2 : 4;           // bf16: the first parts' products and the others'
     perm_f32x4 acc[NA][2];
 #pragma unroll
@@ -874,11 +876,12 @@ __device__ __forceinline__ void gate_wgrad_direct_block(const int cols, const in
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 float r = p.d[u];
+                least = min(least, (__float_as_uint(r) << 1) - 1u);
 #pragma unroll
                 for (int q = 0; q < 3; ++q) {
                     const bf16_t b = (bf16_t)r;
                     part[q][u] = b;
-                    r = fabsf((float)b) < INFINITY ? r - (float)b : 0.f;
+                    r -= (float)b;
                 }
             }
 #pragma unroll
@@ -912,18 +915,33 @@ __device__ __forceinline__ void gate_wgrad_direct_block(const int cols, const in
         float v[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            if constexpr (BF) v[j] = fabsf(acc[0][j][r]) < INFINITY ? acc[0][j][r] + acc[1][j][r] : acc[0][j][r];
+            if constexpr (BF) v[j] = acc[0][j][r] + acc[1][j][r];
             else v[j] = (acc[0][j][r] + acc[1][j][r]) + (acc[2][j][r] + acc[3][j][r]);
         }
         *reinterpret_cast<float2 *>(s_sum + (wave * ROWS + 4 * kg + r) * COLS + 2 * i) = make_float2(v[0], v[1]);
     }
+    uint32_t *const flag = reinterpret_cast<uint32_t *>(s_sum + NW * ROWS * COLS);
+    const bool inexact = BF && __ballot(least < (0x08800000u << 1) - 1u) != 0;      // 2^-110
+    if (lane == 0) flag[wave] = inexact;
     __syncthreads();
+    bool again = false;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) again |= flag[w] != 0;
     for (int o = threadIdx.x; o < ROWS * COLS; o += 64 * NW) {
         float v = s_sum[o];
 #pragma unroll
         for (int w = 1; w < NW; ++w) v += s_sum[w * ROWS * COLS + o];
         const int e = e0 + o / COLS, c = c0 + o % COLS;
-        if (e < E && c < M) dwg[(size_t)e * M + c] = v;
+        if (e >= E || c >= M) continue;
+        if (BF && (again || !(fabsf(v) < INFINITY))) {
+            v = 0.f;
+            for (int t0 = 0; t0 < S; t0 += 64) {       // sums of 64 tokens, added in turn
+                float s = 0.f;
+                for (int t = t0; t < min(t0 + 64, S); ++t) s = fmaf(dlogits[(size_t)t * E + e], (float)x[(size_t)t * M + c], s);
+                v += s;
+            }
+        }
+        dwg[(size_t)e * M + c] = v;
     }
 }
 template <typename T>

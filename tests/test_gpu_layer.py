@@ -1054,7 +1054,7 @@ def test_native_forward_only_fills_xd_and_out(S, M, E, k, Fd, cf, dtype):
     assert torch.equal(t1["xd"][kept], H.dispatch_fwd(x, t1["row"], rows)[kept])
 
 
-def _native_training_pass(m, x, E, k, Fd, cf, dwg=None, sizes=None):
+def _native_training_pass(m, x, E, k, Fd, cf, dwg=None, sizes=None, dy_scale=1e-2):
     """mole_layer_fwd and mole_layer_bwd on buffers of the test's own: every tensor of both blocks, and y.  sizes: bytes of the two workspaces."""
     S, M = x.shape
     dtype, rows, wg = x.dtype, S * k, m.gate[0].linear.weight.detach()
@@ -1066,7 +1066,7 @@ def _native_training_pass(m, x, E, k, Fd, cf, dwg=None, sizes=None):
              offsets=i32(E + 1), capacity=i32(1), xd=act(rows, M), h=act(rows, Fd), a=act(rows, Fd), out=act(rows, M))
     block = _Layer(L.dtype_code(dtype), S, M, E, k, Fd, rows, L.LAYOUT_RAGGED, 1, 0, cf, **{n: v.data_ptr() for n, v in t.items()})
     y = act(S, M)
-    dy = (torch.randn(S, M, generator=torch.Generator().manual_seed(S)) * 1e-2).to(dtype).cuda()
+    dy = (torch.randn(S, M, generator=torch.Generator().manual_seed(S)) * dy_scale).to(dtype).cuda()
     g = dict(dy=dy, dlogits=f32(S, E), d_o=act(rows, M), t=act(rows, Fd), gxd=act(rows, M), dx=act(S, M), dwg=f32(E, M) if dwg is None else dwg,
              **{"g_" + n: torch.empty_like(v) for n, v in w.items()})
     grads = _Grads(0, L.GELU_BWD_TANH, **{n: v.data_ptr() for n, v in g.items()})
@@ -1139,6 +1139,31 @@ def test_gate_weight_gradient_of_few_tokens_with_infinities(dtype):
     finite = torch.isfinite(want)
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
     assert torch.equal(torch.isfinite(got), finite) and float((got - want)[finite].abs().max() / want[finite].abs().max()) < 1e-5
+
+
+# Gradients that three bf16 numbers do not hold: below 2^-110, where the last of them is below the smallest bf16 number, and within half a unit of bf16 of
+# the largest fp32 number, where the first is infinite.  bf16 tokens of widths that are no multiple of 64, in a launch of their own and (few tokens of the
+# layer) in the dispatch's backward's: the bound of test_gate_weight_gradient_of_few_tokens.
+@pytest.mark.parametrize("S,M,E", [(70, 40, 20), (300, 520, 16)])
+def test_gate_weight_gradient_of_gradients_without_parts(S, M, E):
+    from mole_amd import hip_ops as H
+    print(f"gate weight gradient of gradients without parts S={S} M={M} E={E}", flush=True)
+    g = torch.Generator().manual_seed(S)
+    x = torch.randn(S, M, generator=g).bfloat16()
+    def check(got, d, x):
+        want = d.double().t() @ x.double()
+        assert bool(((got.double().cpu() - want).abs() <= (S + 32) * 2.0 ** -24 * (d.double().abs().t() @ x.double().abs())).all())
+    small = torch.randn(S, E, generator=g) * 2.0 ** -122
+    check(H.gate_wgrad(small.cuda(), x.cuda()), small, x)
+    large = torch.randn(S, E, generator=g)
+    large[S - 1, 3] = 3.4e38
+    x_tiny = (x.float() * 2.0 ** -9).bfloat16()
+    check(H.gate_wgrad(large.cuda(), x_tiny.cuda()), large, x_tiny)
+    m, xl, _ = _build(S, M, E, 2, 16, torch.bfloat16, seed=S)
+    t = _native_training_pass(m, xl, E, 2, 16, 0.0, dy_scale=2.0 ** -118)
+    d = t["dlogits"].cpu()
+    assert 0 < float(d.abs().max()) < 2.0 ** -110
+    check(t["dwg"], d, xl.cpu())
 
 
 # A large gate's weight gradient at any alignment of its elements (a view into a flat buffer of gradients): fp32 tokens, widths that are no
