@@ -112,6 +112,9 @@ int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int
 // the dispatch's backward with the gate's input gradient from bf16 operands, beyond the 32 experts of mole_dispatch_bwd's own (permute.hip)
 bool dispatch_bwd_folds(int dtype, int E);
 bool gate_wgrad_beside(int dtype, int S, int E, int M);      // dispatch_bwd_gate_wgrad takes the two in one launch
+inline bool overlap(const void *p, size_t np, const void *q, size_t nq) {      // of np bytes at p and nq at q
+    return p != nullptr && q != nullptr && (uintptr_t)p < (uintptr_t)q + nq && (uintptr_t)q < (uintptr_t)p + np;
+}
 int dispatch_bwd_gate_wgrad(const void *dxd, const int32_t *row, int S, int M, int k, const float *dlogits, const float *wg, int E, void *dx, const void *x, float *dwg, void *workspace,
                             size_t workspace_bytes, hipStream_t st);
 int dispatch_bwd_fold(const void *dxd, const int32_t *row, int S, int M, int k, const float *dlogits, const float *wg, int E, void *dx, hipStream_t st);

@@ -197,7 +197,12 @@ extern "C" int mole_layer_bwd(const mole_layer *L, const mole_layer_grads *G, mo
                                  G->t, G->g_w1, G->g_b1, G->g_w2, G->g_b2, G->gxd, G->accumulate, G->gelu_bwd, L->workspace,
                                  L->workspace_bytes, st)) return rc;
     char *dl_t = ws + p.dgates, *wg_t = dl_t + p.dl_t, *dx_add = wg_t + p.wg_t, *wgrad = dx_add + p.dx_add;
-    if (!p.wgrad_tiles && gate_wgrad_beside(L->dtype, L->S, L->E, L->M))
+    // (not where dwg lies on what the dispatch's backward or other blocks of its own still read: the launches' order then keeps them apart)
+    const size_t dwg_bytes = (size_t)L->E * L->M * 4, token_bytes = (size_t)L->M * (L->dtype == MOLE_BF16 ? 2 : 4), pairs = (size_t)L->S * L->k;
+    const bool dwg_apart = !overlap(G->dwg, dwg_bytes, L->wg, dwg_bytes) && !overlap(G->dwg, dwg_bytes, G->gxd, L->rows * token_bytes) &&
+                           !overlap(G->dwg, dwg_bytes, L->row, pairs * 4) && !overlap(G->dwg, dwg_bytes, G->dlogits, (size_t)L->S * L->E * 4) &&
+                           !overlap(G->dwg, dwg_bytes, L->x, L->S * token_bytes);
+    if (!p.wgrad_tiles && dwg_apart && gate_wgrad_beside(L->dtype, L->S, L->E, L->M))
         return dispatch_bwd_gate_wgrad(G->gxd, L->row, L->S, L->M, L->k, G->dlogits, L->wg, L->E, G->dx, L->x, G->dwg, wgrad, p.wgrad, st);
     if (p.fold) {
         if (int rc = mole_dispatch_bwd(G->gxd, L->dtype, L->row, L->S, L->M, L->k, G->dlogits, L->wg, L->E, nullptr, G->dx, stream)) return rc;

@@ -1423,7 +1423,9 @@ static int check_gate_wgrad(const float *dlogits, const void *x, int dtype, int 
 int gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int M, float *dwg, void *workspace, size_t workspace_bytes, hipStream_t st) {
     ScopedTiming timing(MOLE_K_GATE_WGRAD, st);
     if (int rc = check_gate_wgrad(dlogits, x, dtype, S, E, M, dwg, workspace, workspace_bytes)) return rc;
-    if (gate_wgrad_direct_ok(dtype, S, E)) {
+    // (a result in the place of an operand is written when the partial sums have read it)
+    const size_t result = (size_t)E * M * sizeof(float), tokens_bytes = (size_t)S * M * (dtype == MOLE_BF16 ? 2 : 4);
+    if (gate_wgrad_direct_ok(dtype, S, E) && !overlap(dwg, result, dlogits, (size_t)S * E * sizeof(float)) && !overlap(dwg, result, x, tokens_bytes)) {
         const dim3 grid(ceil_div(M, 32), ceil_div(E, 16));
         if (dtype == MOLE_BF16) hipLaunchKernelGGL(gate_wgrad_direct_kernel<bf16_t>, grid, dim3(1024), 0, st, dlogits, (const bf16_t *)x, S, E, M, dwg);
         else hipLaunchKernelGGL(gate_wgrad_direct_kernel<float>, grid, dim3(1024), 0, st, dlogits, (const float *)x, S, E, M, dwg);

@@ -1141,6 +1141,22 @@ def test_gate_weight_gradient_of_few_tokens_with_infinities(dtype):
     assert torch.equal(torch.isfinite(got), finite) and float((got - want)[finite].abs().max() / want[finite].abs().max()) < 1e-5
 
 
+# dwg in the memory of the gate's weights, which the dispatch's backward reads, and of the tokens' gradients: as from memory of its own.
+def test_gate_weight_gradient_in_the_place_of_an_operand():
+    from mole_amd import hip_ops as H
+    S, M, E = 300, 264, 16
+    print(f"gate weight gradient in the place of an operand S={S} M={M} E={E}", flush=True)
+    m, x, _ = _build(S, M, E, 2, 16, torch.bfloat16, seed=S)
+    apart = _native_training_pass(m, x, E, 2, 16, 0.0)
+    t = _native_training_pass(m, x, E, 2, 16, 0.0, dwg=m.gate[0].linear.weight.detach())
+    assert torch.equal(t["dx"], apart["dx"]) and rel_err(t["dwg"], apart["dwg"]) < 1e-5
+    dl = torch.randn(S, 16, generator=torch.Generator().manual_seed(1)).cuda()
+    want = dl.double().t() @ x.double()
+    ws = torch.empty(L.lib().mole_gate_wgrad_workspace_bytes(S, E, M), dtype=torch.uint8, device="cuda")
+    L.check(L.lib().mole_gate_wgrad(L.ptr(dl), L.ptr(x), L.MOLE_BF16, S, E, M, L.ptr(dl), L.ptr(ws), ws.numel(), L.stream()), "mole_gate_wgrad")
+    assert rel_err(dl.flatten()[:E * M].view(E, M), want) < 1e-5
+
+
 # Gradients that three bf16 numbers do not hold: below 2^-110, where the last of them is below the smallest bf16 number, and within half a unit of bf16 of
 # the largest fp32 number, where the first is infinite.  bf16 tokens of widths that are no multiple of 64, in a launch of their own and (few tokens of the
 # layer) in the dispatch's backward's: the bound of test_gate_weight_gradient_of_few_tokens.
