@@ -1253,15 +1253,22 @@ template <bool N_KS, bool KT, int EPI, int NS = Tile<4, 2, 2>::NSTAGE> static in
     MOLE_LAUNCH_CHECK();
     return 0;
 }
+// Whether t and g_w2 take three blocks to a CU, with rings of three stages.  t walks over K = M, few stages beside gx's K = F: a third block counts for more
+// than stages in flight where t's tiles are more than the CUs (256) and all of them at least two and a half a CU (640).  Of 25 such launches in training
+// passes of random sizes 22 were 1 to 17 % faster and three 2 to 4 % slower; of 14 with fewer tiles of t eleven up to 21 % slower, of 16 with fewer
+// in all twelve 5 to 18 %.  us, two blocks / three, t's tiles and all: 2 x 470 tokens, top-4 of 16, 520 -> 1416 (272, 1232) 31.1 / 32.5, 2 x 490 (280, 1240) 31.7 / 32.2, 2 x
+// 513 (288, 1248) 32.4 / 31.5, 2 x 560 (306, 1266) 36.0 / 33.6; 2048 of the padded layout, 16 of 512 -> 1024 (320, 832) 23.4 / 21.4; 571, top-8 of 22, 384 -> 768 (280,
+// 676) 18.1 / 17.7; 2333, 12 of 448 -> 1344 (266, 794) 20.1 / 18.6; 4 of 640 -> 2560, 429 top-4 (308, 708) 27.1 / 23.2.  Fewer of t's: 654, top-2 of 13, 520 -> 1560 (217,
+// 1062) 21.3 / 25.0; 2589, 26 of 896 -> 896 (233, 1507) 25.3 / 28.0; 287, top-8 of 10, 304 -> 1216 (229, 529) 17.4 / 18.4; fewer in all: 728, top-8 of 13, 256 -> 768 (312, 468)
+// 15.0 / 17.5; 10649, top-2 of 12, 512 -> 256 (345, 441) 30.8 / 33.6.  gx of the first case 31.4 / 37.2.
+static bool three_blocks(int E, int est_rows, int F, int M) {
+    const int active = E < est_rows ? E : est_rows, n_tiles = ceil_div(F, 128);
+    const double tiles = (est_rows / 128.0 + 0.5 * active) * n_tiles;      // (an expert's last one is half full in the mean)
+    return tiles > 256.0 && tiles + (double)E * n_tiles * ceil_div(M, 128) >= 640.0;
+}
 template <bool N_KS, int EPI> static int launch_pair(const GemmArgs &g, const GemmArgs &w, int max_rows, hipStream_t st, int kid) {
-    // t walks over K = M, few stages beside gx's K = F.  Where its tiles are an eighth more than the CUs and all of them more than two a CU,
-    // a third block counts for more than stages in flight (19 of 24 launches of random sizes beyond the line 1 to 15 % faster, two 5 % slower; us, two blocks / three: 2 x 513 tokens, top-4 of 16, 520 -> 1416 33.6 / 32.1; 2048 of the
-    // padded layout, 16 of 512 -> 1024 24.4 / 21.4; 571, top-8 of 22, 384 -> 768 22.0 / 19.2; 1587, 10 of 704 -> 2816 34.1 / 29.5; fewer tiles: 654,
-    // top-2 of 13, 520 -> 1560 21.4 / 24.8; 1825, 17 of 1016 -> 1016 30.3 / 36.9; gx of the first two 31.4 / 37.2, 19.7 / 23.0).
     if constexpr (EPI == EPI_DGELU) {
-        const int active = g.E < g.est_rows ? g.E : g.est_rows;
-        const double tiles = (g.est_rows / 128.0 + 0.5 * active) * ceil_div(g.N, 128);      // (an expert's last one is half full in the mean)
-        if (tiles >= 288.0 && tiles + (double)w.E * ceil_div(w.M, 128) * ceil_div(w.N, 128) >= 640)
+        if (three_blocks(g.E, g.est_rows, g.N, g.K))
             return g.K % Q_BK ? launch_pair_kt<N_KS, true, EPI, 3>(g, w, max_rows, st, kid) : launch_pair_kt<N_KS, false, EPI, 3>(g, w, max_rows, st, kid);
     }
     return g.K % Q_BK ? launch_pair_kt<N_KS, true, EPI>(g, w, max_rows, st, kid) : launch_pair_kt<N_KS, false, EPI>(g, w, max_rows, st, kid);
@@ -1298,3 +1305,8 @@ int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, in
 }  // namespace mole
 
 extern "C" int mole_probe_wgrad_tile(int E, int est_rows, int M, int N) { return mole::wgrad_tile(E, est_rows, M, N) == mole::TILE_128 ? 128 : 256; }
+
+extern "C" int mole_probe_pair_stages(int E, int est_rows, int M, int F) {
+    if (mole::wgrad_tile(E, est_rows, F, M) != mole::TILE_128 || mole::tile_plan(E, est_rows, F, M, false).tile != mole::TILE_128) return 0;
+    return mole::three_blocks(E, est_rows, F, M) ? 3 : mole::Tile<4, 2, 2>::NSTAGE;
+}

@@ -119,8 +119,10 @@ def test_ffn_tiles_of_many_experts(E, dtype):
 # and three, which fill the ring and go round it.
 @pytest.mark.parametrize("M", [32, 40, 96, 104])
 def test_ffn_backward_pair_with_three_stages(M):
-    rows = [(30, 70, 128, 129, 1, 0, 100, 140)[e % 8] for e in range(32)]
-    test_ffn_fwd_bwd_matches_oracle(32, M, 1416, rows, 0, "exact", torch.bfloat16)
+    from mole_amd import _lib as L
+    rows = [(300, 70, 256, 129, 1, 0, 512, 652)[e % 8] for e in range(32)]
+    assert L.lib().mole_probe_pair_stages(32, sum(rows), M, 760) == 3
+    test_ffn_fwd_bwd_matches_oracle(32, M, 760, rows, 0, "exact", torch.bfloat16)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
