@@ -1183,9 +1183,11 @@ def test_gate_weight_gradient_of_gradients_without_parts(S, M, E):
 
 
 # A large gate's weight gradient at any alignment of its elements (a view into a flat buffer of gradients): fp32 tokens, widths that are no
-# multiple of 64, more than 256 experts; one chunk of tokens, which an aligned result gets without a reduction, and several.
+# multiple of 64, more than 256 experts.  Few tokens of up to 256 experts, whose kernel has no partial sums; beyond either line one chunk of tokens, which an
+# aligned result gets without a reduction, and several.
 @pytest.mark.parametrize("S,M,E,k,Fd,dtype", [(12, 72, 40, 2, 64, torch.float32), (700, 132, 70, 2, 32, torch.float32), (15, 520, 33, 1, 32, torch.bfloat16),
-                                              (1300, 136, 70, 4, 32, torch.bfloat16), (300, 64, 300, 2, 16, torch.bfloat16)])
+                                              (1300, 136, 70, 4, 32, torch.bfloat16), (300, 64, 300, 2, 16, torch.bfloat16), (12, 72, 300, 2, 16, torch.float32),
+                                              (15, 520, 270, 1, 16, torch.bfloat16), (1600, 136, 70, 4, 32, torch.bfloat16)])
 def test_gate_weight_gradient_at_any_alignment(S, M, E, k, Fd, dtype):
     print(f"gate weight gradient at any alignment S={S} M={M} E={E} k={k} F={Fd} {dtype}", flush=True)
     m, x, _ = _build(S, M, E, k, Fd, dtype, seed=S + E)

@@ -194,10 +194,12 @@ def test_dispatch_bwd_with_gate_bf16_ragged_widths(S, E, k, M):
     assert rel_err(got, want) < tol(torch.bfloat16)
 
 
-# The gate's weight gradient where its blocks take 16 tokens (few of them) and 64, around the batch of eight.  fp32 sums of up
-# to 12300 terms (2^-24 sqrt(12300) = 7e-6 at worst); the matrix cores' variant splits dlogits in two parts (2^-17 = 8e-6).
+# The gate's weight gradient where its blocks take 16 tokens (few of them) and 64, around the batch of eight: beyond 512 fp32 and 1536 bf16 tokens; few
+# tokens by the kernel without partial sums.  fp32 sums of up to 12300 terms (2^-24 sqrt(12300) = 7e-6 at worst); the matrix cores' variant splits
+# dlogits in two parts (2^-17 = 8e-6).
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("S,E,M", [(1, 3, 72), (15, 8, 520), (17, 16, 8), (513, 32, 520), (12300, 8, 72), (6200, 9, 1032)])
+@pytest.mark.parametrize("S,E,M", [(1, 3, 72), (15, 8, 520), (17, 16, 8), (513, 32, 520), (12300, 8, 72), (6200, 9, 1032),
+                                   (1537, 8, 72), (1700, 16, 520), (2009, 32, 136)])
 def test_gate_wgrad_short_blocks(S, E, M, dtype):
     from mole_amd import hip_ops as H
     print(f"gate_wgrad S={S} E={E} M={M} {dtype}", flush=True)

@@ -129,7 +129,8 @@ def test_softmax_and_gate_bwd(S, E):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("S,E,M", [(1, 1, 4), (100, 8, 64), (1000, 16, 1024), (333, 32, 520), (70, 5, 2048),
-                                   (16384, 16, 1024), (700, 64, 192), (4100, 256, 2048), (129, 100, 320)])
+                                   (16384, 16, 1024), (700, 64, 192), (4100, 256, 2048), (129, 100, 320),
+                                   (1601, 5, 64), (1600, 24, 128), (1700, 30, 192), (2000, 70, 128)])
 def test_gate_wgrad(S, E, M, dtype):
     from mole_amd import hip_ops as H
     print(f"gate_wgrad S={S} E={E} M={M} {dtype}", flush=True)
@@ -138,8 +139,8 @@ def test_gate_wgrad(S, E, M, dtype):
     x = torch.randn(S, M, generator=g).to(dtype)
     got = H.gate_wgrad(dl.cuda(), x.cuda())
     want = dl.double().t() @ x.double()
-    # fp32 sums of exact products (VALU kernel) or of products with dlogits split into two bf16 parts (matrix
-    # cores, bf16 tokens); fp32 tokens with a large gate take the transposed product of the grouped-GEMM tiles
+    # fp32 sums of exact products (VALU kernel, few tokens) or of products with dlogits split into two bf16 parts (matrix
+    # cores, bf16 beyond 1536 tokens); fp32 tokens with a large gate take the transposed product of the grouped-GEMM tiles
     assert got.shape == (E, M)
     assert rel_err(got, want) < 2e-5
 
