@@ -573,8 +573,8 @@ __global__ __launch_bounds__(512) void dispatch_bwd_gate_mfma_kernel(const bf16_
 }
 
 // Gate weight gradient dWg[e, m] = sum_i dlogits[i, e] * x[i, m] (the Linear backward that
-// autograd runs for MOLETopk, MOLE/utils/Ugate.py:12), in two deterministic passes: blocks of
-// gw_tokens() tokens write partial [E, M] sums, a second kernel adds the partials in order.
+// autograd runs for MOLETopk, MOLE/utils/Ugate.py:12), in a fixed order of sums.  Few tokens: gate_wgrad_direct_block below, one pass.  More:
+// two passes, blocks of gw_tokens() tokens (or of a chunk on the matrix cores) write partial [E, M] sums, a second kernel adds the partials in order.
 constexpr int GW_TOKENS = 64, GW_TOKENS_FEW = 16;
 // A block walks its tokens in batches of eight, one round trip to memory each: short blocks where long ones leave CUs
 // idle (513 tokens x 520, 16 experts: 11.5 -> 4.9 us; 110 x 384 fp32, 29 experts: 17.3 -> 7.0).  Gates of more than 32 experts take

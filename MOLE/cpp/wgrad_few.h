@@ -13,6 +13,8 @@
 // V i + j for lane i of 16.  The m-side (VM columns) feeds the instruction's first slot, so that a lane ends up with VN consecutive
 // columns of row VM (4 kg + r) + j in the VN products of m-fragment j: with VN = 8 a store writes whole 256-byte pieces of four rows
 // (128-byte pieces, VN = 4: 440 -> 530 us for 2.1 GB).
+// The first 32 rows are summed first and the rest follows; the large tiles begin with what whole stages of 32 leave over, so with 33 to 63 rows their
+// results may be the neighbouring ones.
 #pragma once
 #include "gemm.h"
 

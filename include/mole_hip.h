@@ -110,11 +110,14 @@ int mole_gate_bwd(const float *dgates, const float *scores, const int32_t *idx, 
                   int k, int normalize_gate, int through_softmax, const int32_t *counts0, const float *d_l_aux,
                   float *dout, mole_stream_t stream);
 /* Gradient of the gate's Linear (MOLE/utils/Ugate.py:12, run by autograd in the reference):
- * dwg[E,M] = dlogits[S,E]^T . x[S,M], fp32, summed in a fixed order (partial sums per chunk of tokens in the
- * workspace, then a reduction).  bf16 tokens: E <= 256 and M a multiple of 64 on the matrix cores (dlogits
- * enters as the sum of two bf16 numbers, so the result keeps fp32-level accuracy); either dtype: E <= 32 and
- * M a multiple of 4 on the VALU.  Other shapes are rejected (a library GEMM serves them on the host side).
- * workspace of mole_gate_wgrad_workspace_bytes(S, E, M) bytes. */
+ * dwg[E,M] = dlogits[S,E]^T . x[S,M], fp32, summed in a fixed order.  Taken are bf16 tokens with E <= 256 and M a
+ * multiple of 64, and either dtype with E <= 32 and M a multiple of 4; other shapes are rejected (a library GEMM serves
+ * them on the host side).  Up to 1536 bf16 or 512 fp32 tokens: one launch on the matrix cores, without partial sums in
+ * memory (bf16: dlogits enters as the sum of three bf16 numbers, 24 bits; fp32 as it is).  More tokens: partial sums
+ * per chunk of tokens in the workspace, then a reduction; the first shapes on the matrix cores (dlogits as the sum of
+ * two bf16 numbers, 16 bits), the others on the VALU in fp32.
+ * workspace of mole_gate_wgrad_workspace_bytes(S, E, M) bytes, which is asked for with few tokens as well but not
+ * touched there (except where dwg lies on an operand: then partial sums are taken). */
 size_t mole_gate_wgrad_workspace_bytes(int S, int E, int M);
 int mole_gate_wgrad(const float *dlogits, const void *x, int dtype, int S, int E, int M, float *dwg,
                     void *workspace, size_t workspace_bytes, mole_stream_t stream);
