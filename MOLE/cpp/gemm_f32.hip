@@ -47,7 +47,6 @@
 // of a row and bias, GELU and stores go by 16 bytes (fp32 operands, one 64-row tile to a CU, against 32 x 32 x 2 with the slots the other way:
 // h of 64 rows x 8, 512 -> 2048 27.0 -> 24.1 us, 256 x 1, 256 -> 1024 17.6 -> 14.3, 128 x 16, 1024 -> 1024 47.2 -> 43.2, 27 x 6, 4096 -> 1216 129 -> 130).
 #include "gemm.h"
-#include "mole_hip_probe.h"
 #include "lds_dma.h"
 
 #include <algorithm>
@@ -1117,16 +1116,6 @@ static double f32_pairs(double stages) { return std::ceil(stages * F_BK / (2 * P
 static bool f32_shares(double walks, double stages, bool heavy, int p) {
     return walks <= 1.0 || (p == 1 && (heavy ? f32_pairs(stages) <= 1.1 * stages : stages > 64.0));
 }
-// h and t of many walks are as fast by own parts, and read less: a shared block's loads go by the registers, its next tile's wait for the end of this one.
-// Inside training passes, own / shared, us, h + t, walks: 1024 rows x 8, 512 -> 2048 (4 walks) 265 / 266, with 130 MB and 198 MB read instead of 151 and 217;
-// -> 2560 (5) 317 / 319, -> 3072 (6) 378 / 386; 2048 x 8, 512 -> 2048 (8) 493 / 511; 512 x 16, 768 -> 2048 (4) 361 / 361.  Fewer walks: 768 x 8, 512 -> 2048 (3) 201 /
-// 195, 512 x 8 (2) 139 / 130; a longer K: 1024 x 8, 1024 -> 2048 (4) 452 / 435.  Of 25 products of random sizes: up to 3.5 walks shared ones 1 to 11 % faster, beyond 6 from
-// 5 % slower to even, one 4 % faster.  (The cost rule takes the two for one.)
-static bool f32_launch_shares(int E, Rows rows, int N, int K, bool heavy, int p) {
-    const double walks = f32_tiles(128, p, E, rows, N) / 256.0, stages = K / F_BK;
-    if (heavy && walks >= 4.0 && (walks > 6.0 || stages < 64.0)) return false;
-    return f32_shares(walks, stages, heavy, p);
-}
 static double f32_cost(int bm, int p, int E, Rows rows, int N, int K, bool heavy) {
     const double walks = f32_tiles(bm, p, E, rows, N) / 256.0, whole = std::ceil(walks);
     const double stages = K / F_BK / (double)p, planes = p > 1 ? p * (2.0 * rows.est * N * sizeof(float) / 5.0e6) + 6.0 : 0.0;
@@ -1193,7 +1182,7 @@ int launch_gemm_f32(const GemmArgs &g0, bool a_ks, bool b_ks, bool wg, int epi, 
     const int e = g.ksplit > 1 ? (int)EPI_PART : epi;
     int rc;
     if (f32_tile(g.ksplit, g.E, rows, g.N, g.K, heavy) == 128) {
-        if (f32_launch_shares(g.E, rows, g.N, g.K, heavy, g.ksplit)) rc = dispatch_f32<128, 128, 4, 8, 1, SHARED_PARTS>(g, b_ks, wg, e, max_rows, st, kid);
+        if (f32_shares(f32_tiles(128, g.ksplit, g.E, rows, g.N) / 256.0, g.K / F_BK, heavy, g.ksplit)) rc = dispatch_f32<128, 128, 4, 8, 1, SHARED_PARTS>(g, b_ks, wg, e, max_rows, st, kid);
         else rc = dispatch_f32<128, 128, 4, 4, 2, OWN_PARTS>(g, b_ks, wg, e, max_rows, st, kid);
     }
     else if (g.E > 0 && g.est_rows > 0 && f32_tiles(64, g.ksplit, g.E, rows, g.N) <= 256.0) rc = dispatch_f32<64, 128, 4, 4, 3, OPERANDS>(g, b_ks, wg, e, max_rows, st, kid);
@@ -1202,8 +1191,3 @@ int launch_gemm_f32(const GemmArgs &g0, bool a_ks, bool b_ks, bool wg, int epi, 
 }
 
 }  // namespace mole
-
-extern "C" int mole_probe_f32_waves(int E, int est_rows, int most_rows, int N, int K) {
-    const mole::Rows rows{est_rows, most_rows};
-    return mole::f32_tile(1, E, rows, N, K, true) == 64 ? 0 : mole::f32_launch_shares(E, rows, N, K, true, 1) ? 8 : 4;
-}

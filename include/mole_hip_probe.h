@@ -32,9 +32,6 @@ int mole_probe_kloop_part(const void *a, const void *b, const int32_t *offsets, 
 int mole_probe_wgrad_tile(int E, int est_rows, int M, int N);
 /* mole_probe_pair_stages: stages of the ring that t and g_w2 of a bf16 FFN share a launch with, by its tiles (0: a launch each). */
 int mole_probe_pair_stages(int E, int est_rows, int M, int F);
-/* mole_probe_f32_waves: waves of the 128-row tiles that the fp32 products h and t [rows,N] over K take, est_rows rows together and most_rows of one expert
- * at most: 8 (parts that a block shares), 4 (parts of every wave's own) or 0 (64-row tiles). */
-int mole_probe_f32_waves(int E, int est_rows, int most_rows, int N, int K);
 
 #ifdef __cplusplus
 }

@@ -34,7 +34,6 @@ _SIGNATURES = {
     "mole_probe_kloop": (c_int, [_P, _P, _P, _P, c_int, c_int, c_int, c_int, _P, _P]),
     "mole_probe_wgrad_tile": (c_int, [c_int, c_int, c_int, c_int]),
     "mole_probe_pair_stages": (c_int, [c_int, c_int, c_int, c_int]),
-    "mole_probe_f32_waves": (c_int, [c_int, c_int, c_int, c_int, c_int]),
     "mole_probe_kloop_part": (c_int, [_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P, _P]),
     "mole_softmax_fwd": (c_int, [_P, _P, c_int, c_int, _P, _P]),
     "mole_gate_fwd": (c_int, [_P, c_int, _P, _P, c_int, c_int, c_int, _P, _P]),

@@ -838,30 +838,6 @@ def test_ffn_fp32_parts_that_a_block_shares(E, M, Fd, rows):
             close(h_inf[r][:, rest], want[:, rest], M)
 
 
-# fp32 h and t on either side of the lines between shared and own parts: 3.9 and 4 walks over 32 stages of 16 of K, 6 and 6.1 over 64; columns that
-# end in a tile, rows that end anywhere in one.  Eight of K are summed before a rounding: 2^-24 sqrt(K / 8) in the 2-norm (t: and the share of GELU', as above).
-@pytest.mark.parametrize("M,Fd,waves", [(512, 8048, 8), (512, 8080, 4), (1024, 12288, 8), (1024, 12304, 4)])
-def test_ffn_fp32_first_products_of_many_walks(M, Fd, waves):
-    from mole_amd import hip_ops as H, _lib as L
-    E, rows = 8, [194, 256, 130, 192, 255, 193, 129, 196]
-    print(f"ffn fp32 many walks M={M} F={Fd}", flush=True)
-    R = sum(rows)
-    assert L.lib().mole_probe_f32_waves(E, R, R, Fd, M) == waves
-    g = torch.Generator(device="cuda").manual_seed(Fd)
-    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
-    xd, go, w1, w2, b1, b2 = rand(R, M), rand(R, M), rand(E, Fd, M) * 0.05, rand(E, Fd, M) * 0.05, rand(E, Fd), rand(E, M)
-    off = torch.tensor([0] + list(np.cumsum(rows)), dtype=torch.int32, device="cuda")
-    n = torch.tensor(rows, dtype=torch.int32, device="cuda")
-    _, h, a = H.ffn_fwd(xd, off, n, w1, b1, w2, b2)
-    t = torch.empty_like(h)
-    H.ffn_bwd_into(go, xd, h, a, off, n, E, R, M, Fd, w1, w2, t, *[torch.empty_like(q) for q in (w1, b1, w2, b2)], None, False, L.GELU_BWD_EXACT)
-    for e in range(E):
-        r = slice(int(off[e]), int(off[e]) + rows[e])
-        for got, want, terms in ((h, xd[r].double() @ w1[e].double().t() + b1[e].double(), M / 8),
-                                 (t, (go[r].double() @ w2[e].double().t()) * O.d_gelu_exact(h[r].double().cpu()).cuda(), M / 8 + 16)):
-            assert float((got[r].double() - want).norm() / want.norm()) <= 2.0 ** -24 * terms ** 0.5
-
-
 # fp32 products from fp32 operands on 64-row tiles (whole and with remainders; split contractions; the last case's out on the generic
 # kernel) and weight gradients, by bf16 parts of their operands: as far from 64 bits as a sum of K fp32 terms may be, 2^-24 sqrt(K) in
 # the 2-norm, and with no bias: the mean error of n results is within 8 / sqrt(n) of their deviation.
