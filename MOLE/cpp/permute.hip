@@ -935,9 +935,9 @@ __device__ __forceinline__ void gate_wgrad_direct_block(const int cols, const in
         if (e >= E || c >= M) continue;
         if (BF && (again || !(fabsf(v) < INFINITY))) {
             v = 0.f;
-            for (int t0 = 0; t0 < S; t0 += 64) {       // sums of 64 tokens, added in turn
+            for (int t0 = 0; t0 < S; t0 += GW_TOKENS_FEW) {       // the partial sums of few tokens, added in turn
                 float s = 0.f;
-                for (int t = t0; t < min(t0 + 64, S); ++t) s = fmaf(dlogits[(size_t)t * E + e], (float)x[(size_t)t * M + c], s);
+                for (int t = t0; t < min(t0 + GW_TOKENS_FEW, S); ++t) s = fmaf(dlogits[(size_t)t * E + e], (float)x[(size_t)t * M + c], s);
                 v += s;
             }
         }
