@@ -1253,23 +1253,24 @@ template <bool N_KS, bool KT, int EPI, int NS = Tile<4, 2, 2>::NSTAGE> static in
     MOLE_LAUNCH_CHECK();
     return 0;
 }
-// Whether t and g_w2 take three blocks to a CU, with rings of three stages.  t walks over K = M, few stages beside gx's K = F: a third block counts for more
-// than stages in flight where t's tiles are more than the CUs (256) and all of them at least two and a half a CU (640).  Of 25 such launches in training
-// passes of random sizes 22 were 1 to 17 % faster and three 2 to 4 % slower; of 14 with fewer tiles of t eleven up to 21 % slower, of 16 with fewer
-// in all twelve 5 to 18 %.  us, two blocks / three, t's tiles and all: 2 x 470 tokens, top-4 of 16, 520 -> 1416 (272, 1232) 31.1 / 32.5, 2 x 490 (280, 1240) 31.7 / 32.2, 2 x
-// 513 (288, 1248) 32.4 / 31.5, 2 x 560 (306, 1266) 36.0 / 33.6; 2048 of the padded layout, 16 of 512 -> 1024 (320, 832) 23.4 / 21.4; 571, top-8 of 22, 384 -> 768 (280,
-// 676) 18.1 / 17.7; 2333, 12 of 448 -> 1344 (266, 794) 20.1 / 18.6; 4 of 640 -> 2560, 429 top-4 (308, 708) 27.1 / 23.2.  Fewer of t's: 654, top-2 of 13, 520 -> 1560 (217,
-// 1062) 21.3 / 25.0; 2589, 26 of 896 -> 896 (233, 1507) 25.3 / 28.0; 287, top-8 of 10, 304 -> 1216 (229, 529) 17.4 / 18.4; fewer in all: 728, top-8 of 13, 256 -> 768 (312, 468)
-// 15.0 / 17.5; 10649, top-2 of 12, 512 -> 256 (345, 441) 30.8 / 33.6.  gx of the first case 31.4 / 37.2.
+// Whether t and g_w2 take three blocks to a CU, with rings of three stages: t walks over K = M, few stages beside gx's K = F, and a third block can
+// count for more than stages in flight.  It does where M is whole stages, t's tiles are more than the CUs (256) and all of them at least two and a half a CU
+// (640): of 51 such training passes of random sizes 36 were 0.2 to 4 % faster with it and seven up to 0.7 % slower, 1 % in the mean.  us, two blocks / three, t's
+// tiles and all: 2048 tokens of the padded layout, 16 experts of 512 -> 1024 (320, 832) 102.6 / 101.4; 429, top-4 of 4, 640 -> 2560 (308, 708) 120.0 / 117.2; 2 x 3923,
+// top-2 of 14, 1024 -> 512 (273, 721) 339.1 / 329.5; 1361, top-4 of 12, 320 -> 960 (388, 676) 105.9 / 103.7; near the first bound 571, top-8 of 22, 384 -> 768 (280, 676)
+// 99.1 / 99.8, 2333, 12 of 448 -> 1344 (266, 794) 109.5 / 108.7.  Not with fewer tiles of t (eight passes up to 2 % faster or slower, as often) or fewer than 540 in all (ten
+// passes, 2.8 % slower in the mean: 12871, top-2 of 8, 512 -> 256 (410, 474) 193.3 / 200.1), and not where M ends inside a stage: below 288 tiles of t 26 of 28 slower, 1.7 %
+// in the mean (373, top-8 of 15, 264 -> 1056 (277, 682) 102.2 / 104.3), above as many faster as slower (2 x 513, top-4 of 16, 520 -> 1416 (288, 1248) 294.4 / 293.1; 2 x 490
+// (280, 1240) 270.5 / 272.9; 442, top-8 of 23, 496 -> 992 (313, 1049) 122.1 / 122.5).  gx, whose walk is longer: 31.4 / 37.2 the launch of 2 x 513.
 static bool three_blocks(int E, int est_rows, int F, int M) {
+    if (M % Q_BK != 0) return false;
     const int active = E < est_rows ? E : est_rows, n_tiles = ceil_div(F, 128);
     const double tiles = (est_rows / 128.0 + 0.5 * active) * n_tiles;      // (an expert's last one is half full in the mean)
     return tiles > 256.0 && tiles + (double)E * n_tiles * ceil_div(M, 128) >= 640.0;
 }
 template <bool N_KS, int EPI> static int launch_pair(const GemmArgs &g, const GemmArgs &w, int max_rows, hipStream_t st, int kid) {
     if constexpr (EPI == EPI_DGELU) {
-        if (three_blocks(g.E, g.est_rows, g.N, g.K))
-            return g.K % Q_BK ? launch_pair_kt<N_KS, true, EPI, 3>(g, w, max_rows, st, kid) : launch_pair_kt<N_KS, false, EPI, 3>(g, w, max_rows, st, kid);
+        if (three_blocks(g.E, g.est_rows, g.N, g.K)) return launch_pair_kt<N_KS, false, EPI, 3>(g, w, max_rows, st, kid);
     }
     return g.K % Q_BK ? launch_pair_kt<N_KS, true, EPI>(g, w, max_rows, st, kid) : launch_pair_kt<N_KS, false, EPI>(g, w, max_rows, st, kid);
 }
