@@ -17,7 +17,7 @@
 // keep fp32 operands.  (One accumulator for all six: 0.75-0.9 of fp32 operands' error, but a drift of 0.02 units a stage.)
 // A tile whose operands include a number below 2^-110 that is not zero, or whose results are not all finite, is computed again
 // from fp32 operands.  All rows of a tile take the same steps, so equal rows give equal results.
-// Time, fp32 operands / parts that every wave makes / parts that a block shares, on one box, us: 8 experts of 1000 rows, 512 -> 2048: h 154 / 128 / 128,
+// Time of launches one by one, fp32 operands / parts that every wave makes / parts that a block shares, on one box, us: 8 experts of 1000 rows, 512 -> 2048: h 154 / 128 / 128,
 // out 135 / 115 / 106, t 154 / 125 / 127, gx 133 / 112 / 104, the weight gradients 136 / 108 each; 8 of 2000, 1024 -> 4096: 1036, 1004,
 // 1047, 993, 1010 / 838, 756, 833, 750, 788.
 //
@@ -1112,6 +1112,10 @@ static double f32_tiles(int bm, int p, int E, Rows rows, int N) {
 // own parts, two to a CU, hide each other's ends, and that counts where a CU walks more than once over a short K (shared / own, us, out:
 // 1636 rows x 23, 576 -> 576 193 / 172; 528 x 64, 320 -> 320 85 / 73; 1238 x 20, 768 -> 320 128 / 120; 1570 x 20, 512 -> 832 238 / 227; K = 1664,
 // 1160 x 8 241 / 240, K = 2880, 391 x 20 620 / 634), over a K in planes (two, of the same: 337 / 291, 248 / 230, 688 / 639) and where an eighth of h's walk over K would be padding (7911 x 7, 336 -> 1008 347 / 320).
+// h and t of many walks take the same time either way when launches are timed one by one (1024 x 8, 512 -> 2048: 265 / 266 for both, and shared ones read 151
+// and 217 MB instead of 130 and 198); passes that follow each other run into the power limit, and there shared ones are ahead, shared / own, us: 4096 tokens, 8 experts top-2,
+// 512 -> 2048 704 / 714, 16384 2660 / 2680, 16 of 768 -> 2048 1048 / 1067, 8 of 1024 -> 2048 1269 / 1301; 8192, 8 of 1024 -> 4096 4855 / 4977; 7548, 46 of 1600 -> 1600 3693 /
+// 3764; 10617, 14 of 544 -> 1088 1375 / 1376.  Of 19 passes with 4 to 33 walks 13 were 0.4 to 2.7 % faster, six within 0.3 % of even.
 static double f32_pairs(double stages) { return std::ceil(stages * F_BK / (2 * P_BK)) * (2 * P_BK / F_BK); }
 static bool f32_shares(double walks, double stages, bool heavy, int p) {
     return walks <= 1.0 || (p == 1 && (heavy ? f32_pairs(stages) <= 1.1 * stages : stages > 64.0));
