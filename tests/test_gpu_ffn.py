@@ -115,10 +115,18 @@ def test_ffn_tiles_of_many_experts(E, dtype):
             assert rel_err(out[r], a[r].float() @ c["w2"][e].float() + c["b2"][e].float()) < tol(dtype)
 
 
+# Backward products of many experts of few rows: contractions of one stage, of one and a rest, of three and of a rest and three.  (F = 1416 gives t more
+# rows of tiles than 128 x 128 ones are taken for; the next test has the launches with rings of three stages.)
+@pytest.mark.parametrize("M", [32, 40, 96, 104])
+def test_ffn_backward_pair_with_three_stages(M):
+    rows = [(30, 70, 128, 129, 1, 0, 100, 140)[e % 8] for e in range(32)]
+    test_ffn_fwd_bwd_matches_oracle(32, M, 1416, rows, 0, "exact", torch.bfloat16)
+
+
 # t and g_w2 in one launch with a ring of three stages (many tiles of few rows): contractions of one to four stages, which fill the ring and go
 # round it; weight gradients of rows that end anywhere in a stage.
 @pytest.mark.parametrize("M", [32, 64, 96, 128])
-def test_ffn_backward_pair_with_three_stages(M):
+def test_ffn_backward_pair_on_the_ring_of_three_stages(M):
     from mole_amd import _lib as L
     rows = [(300, 70, 256, 129, 1, 0, 512, 652)[e % 8] for e in range(32)]
     assert L.lib().mole_probe_pair_stages(32, sum(rows), M, 760) == 3
@@ -777,6 +785,21 @@ def test_ffn_few_rows_with_infinite_weights(E, M, Fd, rows, dtype):
             H.ffn_bwd_into(c["go"], c["xd"], h, a, off, n, E, R, M, Fd, w1.cuda(), c["w2"], t, *g, gx, False, L.GELU_BWD_EXACT)
             want = torch.einsum("rf,rfm->rm", t.double().cpu(), w1.double()[owner])
             assert _same_class(gx, want)
+
+
+# out of 128 x 128 tiles that leave the CUs' second blocks idle: contractions of 84.75, 60 and 56 stages of 32, in one piece or in two planes, experts of one and of two
+# m-tiles, columns that end in a tile.  bf16 results of fp32 sums in another order: the tolerance of every FFN test.
+@pytest.mark.parametrize("E,M,Fd,rows", [(9, 904, 2712, [129, 256, 97, 128, 257, 200, 192, 150, 190]), (10, 640, 1920, [131, 172, 150, 129, 200] * 2), (24, 448, 1792, [140, 97, 160, 129, 90, 128] * 4)])
+def test_ffn_split_contraction_of_second_blocks(E, M, Fd, rows):
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"split contraction of second blocks E={E} M={M} F={Fd}", flush=True)
+    d = _make(E, M, Fd, rows, torch.bfloat16, seed=E + M)
+    assert L.lib().mole_ffn_workspace_bytes(L.MOLE_BF16, E, d["R"], M, Fd) == {9: 0, 10: 2, 24: 0}[E] * d["R"] * M * 4
+    c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+    out, _, a = H.ffn_fwd(c["xd"], torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda(), c["w1"], c["b1"], c["w2"], c["b2"])
+    for e in range(E):
+        r = slice(int(d["off"][e]), int(d["off"][e]) + rows[e])
+        assert rel_err(out[r], a[r].float() @ c["w2"][e].float() + c["b2"][e].float()) < tol(torch.bfloat16)
 
 
 def test_ffn_split_contraction_of_more_than_2_to_18_rows():
