@@ -1254,23 +1254,26 @@ template <bool N_KS, bool KT, int EPI, int NS = Tile<4, 2, 2>::NSTAGE> static in
     return 0;
 }
 // Whether t and g_w2 take three blocks to a CU, with rings of three stages: t walks over K = M, few stages beside gx's K = F, and a third block can
-// count for more than stages in flight.  It does where M is whole stages, t's tiles are more than the CUs (256) and all of them at least two and a half a CU
-// (640): of 51 such training passes of random sizes 36 were 0.2 to 4 % faster with it and seven up to 0.7 % slower, 1 % in the mean.  us, two blocks / three, t's
+// count for more than stages in flight.  It does where t's tiles are more than the CUs (256) and all of them at least two and a half a CU (640).
+// M of whole stages: of 51 such training passes of random sizes 36 were 0.2 to 4 % faster with it and seven up to 0.7 % slower, 1 % in the mean.  us, two blocks / three, t's
 // tiles and all: 2048 tokens of the padded layout, 16 experts of 512 -> 1024 (320, 832) 102.6 / 101.4; 429, top-4 of 4, 640 -> 2560 (308, 708) 120.0 / 117.2; 2 x 3923,
 // top-2 of 14, 1024 -> 512 (273, 721) 339.1 / 329.5; 1361, top-4 of 12, 320 -> 960 (388, 676) 105.9 / 103.7; near the first bound 571, top-8 of 22, 384 -> 768 (280, 676)
 // 99.1 / 99.8, 2333, 12 of 448 -> 1344 (266, 794) 109.5 / 108.7.  Not with fewer tiles of t (eight passes up to 2 % faster or slower, as often) or fewer than 540 in all (ten
-// passes, 2.8 % slower in the mean: 12871, top-2 of 8, 512 -> 256 (410, 474) 193.3 / 200.1), and not where M ends inside a stage: below 288 tiles of t 26 of 28 slower, 1.7 %
-// in the mean (373, top-8 of 15, 264 -> 1056 (277, 682) 102.2 / 104.3), above as many faster as slower (2 x 513, top-4 of 16, 520 -> 1416 (288, 1248) 294.4 / 293.1; 2 x 490
-// (280, 1240) 270.5 / 272.9; 442, top-8 of 23, 496 -> 992 (313, 1049) 122.1 / 122.5).  gx, whose walk is longer: 31.4 / 37.2 the launch of 2 x 513.
-static bool three_blocks(int E, int est_rows, int F, int M) {
-    if (M % Q_BK != 0) return false;
+// passes, 2.8 % slower in the mean: 12871, top-2 of 8, 512 -> 256 (410, 474) 193.3 / 200.1).
+// M that ends inside a stage, whose stages take a third longer: where the weight gradient is added to what is there, for its blocks wait for the old values as well (27 passes of two micro-
+// batches, 256 to 394 tiles of t: 23 are 0.3 to 5 % faster, four up to 1.5 % slower, 0.9 % in the mean; 2 x 490, 513 and 540 tokens, top-4 of 16, 520 -> 1416 (280, 288, 298) 286.5 / 285.6,
+// 296.1 / 294.1, 304.6 / 297.3), and without that from 370 tiles of t on: 26 of 26 passes up to 487 are 0.3 to 5 % faster, 1.6 % in the mean (1522, top-8 of 16, 408 -> 408 (413, 669) 143.1 /
+// 136.6; 404, 1052 in all, M = 328 144.5 / 141.0; 372, 980, M = 440 142.9 / 142.4).  From 300 to 370 eight of 25 are faster (345, 778, M = 712 166.2 / 163.8; 349, 1629, M = 904 188.3 / 191.9),
+// below 300 three of 44 (261, 1661, M = 1264 187.1 / 191.9).  gx, whose walk is longer: 31.4 / 37.2 the launch of 2 x 513.
+static bool three_blocks(int E, int est_rows, int F, int M, bool accumulate) {
     const int active = E < est_rows ? E : est_rows, n_tiles = ceil_div(F, 128);
     const double tiles = (est_rows / 128.0 + 0.5 * active) * n_tiles;      // (an expert's last one is half full in the mean)
-    return tiles > 256.0 && tiles + (double)E * n_tiles * ceil_div(M, 128) >= 640.0;
+    return tiles > 256.0 && (M % Q_BK == 0 || accumulate || tiles >= 370.0) && tiles + (double)E * n_tiles * ceil_div(M, 128) >= 640.0;
 }
 template <bool N_KS, int EPI> static int launch_pair(const GemmArgs &g, const GemmArgs &w, int max_rows, hipStream_t st, int kid) {
     if constexpr (EPI == EPI_DGELU) {
-        if (three_blocks(g.E, g.est_rows, g.N, g.K)) return launch_pair_kt<N_KS, false, EPI, 3>(g, w, max_rows, st, kid);
+        if (three_blocks(g.E, g.est_rows, g.N, g.K, w.accumulate != 0))
+            return g.K % Q_BK ? launch_pair_kt<N_KS, true, EPI, 3>(g, w, max_rows, st, kid) : launch_pair_kt<N_KS, false, EPI, 3>(g, w, max_rows, st, kid);
     }
     return g.K % Q_BK ? launch_pair_kt<N_KS, true, EPI>(g, w, max_rows, st, kid) : launch_pair_kt<N_KS, false, EPI>(g, w, max_rows, st, kid);
 }
@@ -1307,7 +1310,7 @@ int launch_gemm256(const GemmArgs &g, bool a_ks, bool b_ks, bool wg, int epi, in
 
 extern "C" int mole_probe_wgrad_tile(int E, int est_rows, int M, int N) { return mole::wgrad_tile(E, est_rows, M, N) == mole::TILE_128 ? 128 : 256; }
 
-extern "C" int mole_probe_pair_stages(int E, int est_rows, int M, int F) {
+extern "C" int mole_probe_pair_stages(int E, int est_rows, int M, int F, int accumulate) {
     if (mole::wgrad_tile(E, est_rows, F, M) != mole::TILE_128 || mole::tile_plan(E, est_rows, F, M, false).tile != mole::TILE_128) return 0;
-    return mole::three_blocks(E, est_rows, F, M) ? 3 : mole::Tile<4, 2, 2>::NSTAGE;
+    return mole::three_blocks(E, est_rows, F, M, accumulate != 0) ? 3 : mole::Tile<4, 2, 2>::NSTAGE;
 }

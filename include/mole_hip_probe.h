@@ -30,8 +30,9 @@ int mole_probe_kloop_part(const void *a, const void *b, const int32_t *offsets, 
 
 /* mole_probe_wgrad_tile: columns of the bf16 tile that the weight gradients [M,N] of E experts, est_rows rows together, take (128 or 256). */
 int mole_probe_wgrad_tile(int E, int est_rows, int M, int N);
-/* mole_probe_pair_stages: stages of the ring that t and g_w2 of a bf16 FFN share a launch with, by its tiles (0: a launch each). */
-int mole_probe_pair_stages(int E, int est_rows, int M, int F);
+/* mole_probe_pair_stages: stages of the ring that t and g_w2 (accumulate: added to what is there) of a bf16 FFN share a launch with, by its tiles
+ * (0: a launch each). */
+int mole_probe_pair_stages(int E, int est_rows, int M, int F, int accumulate);
 
 #ifdef __cplusplus
 }

@@ -329,3 +329,12 @@ def test_layer_scratch_is_told_from_the_sizes_alone():
                 block = ctypes.create_string_buffer(struct.pack("10id", dtype, S, M, E, k, F, S * k, L.LAYOUT_RAGGED, 1, 0, cf), 512)
                 need.add(L.lib().mole_layer_workspace_bytes(ctypes.cast(block, ctypes.c_void_p), backward))
             assert len(need) == 1, (dtype, S, M, E, k, F, need)
+
+
+def test_rings_of_three_stages_lie_where_they_were_measured():
+    """t and g_w2 in one launch: sizes on either side of each line of the rule (rings of three stages, of five, or a launch each)."""
+    from mole_amd import _lib as L
+    ring = L.lib().mole_probe_pair_stages
+    for (E, rows, M, F), stored, added in (((22, 571 * 8, 384, 768), 3, 3), ((16, 2052, 520, 1416), 5, 3), ((16, 1522 * 8, 408, 408), 3, 3), ((10, 2260, 984, 1968), 5, 3),
+                                           ((8, 12871 * 2, 512, 256), 5, 5), ((13, 654 * 2, 520, 1560), 5, 5), ((32, 3616, 32, 1416), 0, 0)):
+        assert (ring(E, rows, M, F, 0), ring(E, rows, M, F, 1)) == (stored, added), (E, rows, M, F)

@@ -123,13 +123,13 @@ def test_ffn_backward_pair_with_three_stages(M):
     test_ffn_fwd_bwd_matches_oracle(32, M, 1416, rows, 0, "exact", torch.bfloat16)
 
 
-# t and g_w2 in one launch with a ring of three stages (many tiles of few rows): contractions of one to four stages, which fill the ring and go
-# round it; weight gradients of rows that end anywhere in a stage.
-@pytest.mark.parametrize("M", [32, 64, 96, 128])
+# t and g_w2 in one launch with a ring of three stages (many tiles of few rows), results stored and added: contractions of one to four stages, which fill
+# the ring and go round it, of one and a rest and of a rest and three; weight gradients of rows that end anywhere in a stage.
+@pytest.mark.parametrize("M", [32, 40, 64, 96, 104, 128])
 def test_ffn_backward_pair_on_the_ring_of_three_stages(M):
     from mole_amd import _lib as L
     rows = [(300, 70, 256, 129, 1, 0, 512, 652)[e % 8] for e in range(32)]
-    assert L.lib().mole_probe_pair_stages(32, sum(rows), M, 760) == 3
+    assert [L.lib().mole_probe_pair_stages(32, sum(rows), M, 760, accumulate) for accumulate in (0, 1)] == [3, 3]
     test_ffn_fwd_bwd_matches_oracle(32, M, 760, rows, 0, "exact", torch.bfloat16)
 
 
