@@ -811,10 +811,11 @@ __global__ __launch_bounds__(256, 2) void gate_wgrad_mfma_kernel(const float *__
 // Neither operand is contiguous along the tokens that are summed over, and there is no LDS on the way in:
 //   bf16 tokens: a lane loads two columns of eight tokens and one expert's gradient of each, and turns them in registers for
 //       v_mfma_f32_16x16x32_bf16.  The gradients enter as three bf16 numbers each, 24 bits, and the first ones' products have an accumulator
-//       of their own.  Results of a block that met a gradient below 2^-110 that is not zero, whose last part may be below the smallest bf16
-//       number, and results that are not finite (an infinity has no parts, nor has a gradient that bf16 rounds to one) are formed again in fp32.
+//       of their own.  A block that met a gradient below 2^-110 that is not zero, whose last part may be below the smallest bf16 number, or whose
+//       sums are not all finite (an infinity has no parts, nor has a gradient that bf16 rounds to one) forms its results again as fp32 tokens'.
 //   fp32 tokens: v_mfma_f32_16x16x4_f32 on the values as they come, four tokens an instruction, in four accumulators in turn: the fewer
-//       roundings a sum has in a row, the closer it is (513 tokens, 2-norm error 1.27e-7 with one, 1.01e-7 with four).
+//       roundings a sum has in a row, the closer it is (513 tokens, 2-norm error 1.27e-7 with one, 1.01e-7 with four).  It keeps numbers below
+//       the normal ones, in operands and sums.
 // cols, group: the block's 32 columns and 16 experts; s_sum: its LDS, GD_LDS floats.
 template <int NW> constexpr int GD_LDS = NW * 16 * 32 + NW;
 template <typename T, int NW>
@@ -846,13 +847,8 @@ __device__ __forceinline__ void gate_wgrad_direct_block(const int cols, const in
         }
     };
     uint32_t least = 0xffffffffu;            // of the gradients' magnitudes: their bits doubled, less one (zero: the largest)
-    constexpr int NA = BF ? 2 : 4;           // bf16: the first parts' products and the others'
-    perm_f32x4 acc[NA][2];
-#pragma unroll
-    for (int n = 0; n < NA; ++n)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[n][j] = perm_f32x4{0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](Step &p, int t0) __attribute__((always_inline)) {
+    // by_parts: acc[0] the first parts' products, acc[1] the others'; otherwise four sums of fp32 products
+    auto multiply = [&](auto by_parts, auto &acc, Step &p, int t0) __attribute__((always_inline)) {
         if (t0 + 32 > S) {               // tokens past the end count nothing
 #pragma unroll
             for (int u = 0; u < 8; ++u)
@@ -862,7 +858,7 @@ __device__ __forceinline__ void gate_wgrad_direct_block(const int cols, const in
                     p.d[u] = 0.f;
                 }
         }
-        if constexpr (BF) {
+        if constexpr (by_parts) {
             perm_bf16x8 col[2];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
@@ -894,54 +890,71 @@ __device__ __forceinline__ void gate_wgrad_direct_block(const int cols, const in
 #pragma unroll
             for (int u = 0; u < 8; ++u)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[u % NA][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p.d[u], __uint_as_float(p.x[u][j]), acc[u % NA][j], 0, 0, 0);
+                for (int j = 0; j < 2; ++j) {
+                    const uint32_t xv = !BF ? p.x[u][BF ? 0 : j] : j ? p.x[u][0] & 0xffff0000u : p.x[u][0] << 16;
+                    acc[u % 4][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p.d[u], __uint_as_float(xv), acc[u % 4][j], 0, 0, 0);
+                }
         }
     };
     // Two steps' loads are in flight (four are no faster).  They come from clamped addresses without a condition: the steps past a wave's last
     // one are fetched for nobody.
-    Step a, b;
     constexpr int STEP = NW * 32;
     const int first = wave * 32;
-    fetch(a, first);
-    for (int t0 = first; t0 < S; t0 += 2 * STEP) {
-        fetch(b, t0 + STEP);
-        multiply(a, t0);
-        fetch(a, t0 + 2 * STEP);
-        if (t0 + STEP < S) multiply(b, t0 + STEP);
-    }
-    // acc[.][j][r] = expert e0 + 4 kg + r, column c0 + 2 i + j
+    auto walk = [&](auto by_parts, auto &acc) __attribute__((always_inline)) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        float v[2];
+        for (auto &n : acc)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            if constexpr (BF) v[j] = acc[0][j][r] + acc[1][j][r];
-            else v[j] = (acc[0][j][r] + acc[1][j][r]) + (acc[2][j][r] + acc[3][j][r]);
+            for (auto &sum : n) sum = perm_f32x4{0.f, 0.f, 0.f, 0.f};
+        Step a, b;
+        fetch(a, first);
+        for (int t0 = first; t0 < S; t0 += 2 * STEP) {
+            fetch(b, t0 + STEP);
+            multiply(by_parts, acc, a, t0);
+            fetch(a, t0 + 2 * STEP);
+            if (t0 + STEP < S) multiply(by_parts, acc, b, t0 + STEP);
         }
+    };
+    // acc[.][j][r] = expert e0 + 4 kg + r, column c0 + 2 i + j
+    auto put = [&](int r, const float (&v)[2]) __attribute__((always_inline)) {
         *reinterpret_cast<float2 *>(s_sum + (wave * ROWS + 4 * kg + r) * COLS + 2 * i) = make_float2(v[0], v[1]);
-    }
-    uint32_t *const flag = reinterpret_cast<uint32_t *>(s_sum + NW * ROWS * COLS);
-    const bool inexact = BF && __ballot(least < (0x08800000u << 1) - 1u) != 0;      // 2^-110
-    if (lane == 0) flag[wave] = inexact;
-    __syncthreads();
-    bool again = false;
+    };
+    auto in_fp32 = [&]() __attribute__((always_inline)) {
+        perm_f32x4 acc[4][2];
+        walk(std::false_type{}, acc);
 #pragma unroll
-    for (int w = 0; w < NW; ++w) again |= flag[w] != 0;
+        for (int r = 0; r < 4; ++r) put(r, {(acc[0][0][r] + acc[1][0][r]) + (acc[2][0][r] + acc[3][0][r]), (acc[0][1][r] + acc[1][1][r]) + (acc[2][1][r] + acc[3][1][r])});
+    };
+    if constexpr (BF) {
+        perm_f32x4 acc[2][2];
+        walk(std::true_type{}, acc);
+        bool inexact = least < (0x08800000u << 1) - 1u;      // 2^-110
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float v[2] = {acc[0][0][r] + acc[1][0][r], acc[0][1][r] + acc[1][1][r]};
+            inexact |= !(fabsf(v[0]) < INFINITY && fabsf(v[1]) < INFINITY);
+            put(r, v);
+        }
+        uint32_t *const flag = reinterpret_cast<uint32_t *>(s_sum + NW * ROWS * COLS);
+        inexact = __ballot(inexact) != 0;
+        if (lane == 0) flag[wave] = inexact;
+        __syncthreads();
+        bool again = false;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) again |= flag[w] != 0;
+        if (again) {                                         // (every wave overwrites what it has put there itself)
+            in_fp32();
+            __syncthreads();
+        }
+    } else {
+        in_fp32();
+        __syncthreads();
+    }
     for (int o = threadIdx.x; o < ROWS * COLS; o += 64 * NW) {
         float v = s_sum[o];
 #pragma unroll
         for (int w = 1; w < NW; ++w) v += s_sum[w * ROWS * COLS + o];
         const int e = e0 + o / COLS, c = c0 + o % COLS;
-        if (e >= E || c >= M) continue;
-        if (BF && (again || !(fabsf(v) < INFINITY))) {
-            v = 0.f;
-            for (int t0 = 0; t0 < S; t0 += GW_TOKENS_FEW) {       // the partial sums of few tokens, added in turn
-                float s = 0.f;
-                for (int t = t0; t < min(t0 + GW_TOKENS_FEW, S); ++t) s = fmaf(dlogits[(size_t)t * E + e], (float)x[(size_t)t * M + c], s);
-                v += s;
-            }
-        }
-        dwg[(size_t)e * M + c] = v;
+        if (e < E && c < M) dwg[(size_t)e * M + c] = v;
     }
 }
 template <typename T>

@@ -113,7 +113,8 @@ int mole_gate_bwd(const float *dgates, const float *scores, const int32_t *idx, 
  * dwg[E,M] = dlogits[S,E]^T . x[S,M], fp32, summed in a fixed order.  Taken are bf16 tokens with E <= 256 and M a
  * multiple of 64, and either dtype with E <= 32 and M a multiple of 4; other shapes are rejected (a library GEMM serves
  * them on the host side).  Up to 1536 bf16 or 512 fp32 tokens: one launch on the matrix cores, without partial sums in
- * memory (bf16: dlogits enters as the sum of three bf16 numbers, 24 bits; fp32 as it is).  More tokens: partial sums
+ * memory (bf16: dlogits enters as the sum of three bf16 numbers, 24 bits, or as it is where these do not hold it; fp32
+ * as it is).  More tokens: partial sums
  * per chunk of tokens in the workspace, then a reduction; the first shapes on the matrix cores (dlogits as the sum of
  * two bf16 numbers, 16 bits), the others on the VALU in fp32.
  * workspace of mole_gate_wgrad_workspace_bytes(S, E, M) bytes, which is asked for with few tokens as well but not

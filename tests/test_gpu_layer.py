@@ -1160,7 +1160,7 @@ def test_gate_weight_gradient_in_the_place_of_an_operand():
 # Gradients that three bf16 numbers do not hold: below 2^-110, where the last of them is below the smallest bf16 number, and within half a unit of bf16 of
 # the largest fp32 number, where the first is infinite.  bf16 tokens of widths that are no multiple of 64, in a launch of their own and (few tokens of the
 # layer) in the dispatch's backward's: the bound of test_gate_weight_gradient_of_few_tokens.
-@pytest.mark.parametrize("S,M,E", [(70, 40, 20), (300, 520, 16)])
+@pytest.mark.parametrize("S,M,E", [(70, 40, 20), (300, 520, 16), (1500, 72, 27)])
 def test_gate_weight_gradient_of_gradients_without_parts(S, M, E):
     from mole_amd import hip_ops as H
     print(f"gate weight gradient of gradients without parts S={S} M={M} E={E}", flush=True)
@@ -1171,6 +1171,8 @@ def test_gate_weight_gradient_of_gradients_without_parts(S, M, E):
         assert bool(((got.double().cpu() - want).abs() <= (S + 32) * 2.0 ** -24 * (d.double().abs().t() @ x.double().abs())).all())
     small = torch.randn(S, E, generator=g) * 2.0 ** -122
     check(H.gate_wgrad(small.cuda(), x.cuda()), small, x)
+    below, x_large = (torch.randn(S, E, generator=g).double() * 2.0 ** -136).float(), (x.float() * 2.0 ** 20).bfloat16()      # below the normal numbers
+    check(H.gate_wgrad(below.cuda(), x_large.cuda()), below, x_large)
     large = torch.randn(S, E, generator=g)
     large[S - 1, 3] = 3.4e38
     x_tiny = (x.float() * 2.0 ** -9).bfloat16()
