@@ -82,12 +82,12 @@ template <int TMB, int WM, int WN, bool M_KS, int TMC, int NS = Tile<TMB, WM, WN
 // With NW waves, wave w's load i fills LDS bytes [(NW i + w)*1024, +1024) = rows 16(NW i + w) .. +16.
 // Per-lane byte offsets of the ROWS/(16 NW) loads a wave issues for one stage of an operand tile, relative to
 // the tile's first element at the stage's first k (what the scalar base points at).  r_left = rows of the
-// operand from the tile's first row on, k_left = k of the stage (only stage 0 of a ragged contraction has fewer than 32).
+// operand from the tile's first row on.
 __device__ __forceinline__ int swz16(int row) { return ((row >> 3) & 1) | (((row >> 1) ^ (row >> 2)) & 2); }
 // src: the operand's rows are those of a matrix of n_src rows that src names, and the base is that matrix (null: they lie there in order).
 template <int ROWS, int NW> struct OffKC {
     uint32_t off[ROWS / (16 * NW)];
-    __device__ __forceinline__ void init(long ld, int r_left, int k_left, const int32_t *src, int n_src) {
+    __device__ __forceinline__ void init(long ld, int r_left, const int32_t *src, int n_src) {
         uint32_t at[ROWS / (16 * NW)];
 #pragma unroll
         for (int i = 0; i < ROWS / (16 * NW); ++i) {
@@ -98,9 +98,15 @@ template <int ROWS, int NW> struct OffKC {
 #pragma unroll
         for (int i = 0; i < ROWS / (16 * NW); ++i) {
             const int row = (NW * i + w) * 16 + (lane >> 2);
-            const int c = min((lane & 3) ^ swz16(row), (k_left >> 3) - 1);     // (k_left is a multiple of 8)
-            off[i] = (uint32_t)(at[i] * ld * 2 + c * 16);
+            off[i] = (uint32_t)(at[i] * ld * 2 + ((lane & 3) ^ swz16(row)) * 16);
         }
+    }
+    // of a stage with k_left (a multiple of 8) of k: the last 16-byte piece instead of those past it
+    __device__ __forceinline__ void clamp(int k_left, long) {
+        const int lane = threadIdx.x & 63;
+        const uint32_t past = (uint32_t)max(((lane & 3) ^ swz16(lane >> 2)) - ((k_left >> 3) - 1), 0) * 16;      // (the swizzle goes by the row's place among 16)
+#pragma unroll
+        for (int i = 0; i < ROWS / (16 * NW); ++i) off[i] -= past;
     }
 };
 // K-strided operand, element (r, k) at p[k*ld + r]: LDS [32 k][ROWS x 2 B] as it lies in HBM, the
@@ -109,17 +115,23 @@ template <int ROWS, int NW> struct OffKC {
 __device__ __forceinline__ int swz_ks(int k) { return ((k & 3) << 1) | ((k >> 3) & 1); }
 template <int ROWS, int NW> struct OffKS {
     uint32_t off[ROWS / (16 * NW)];
-    __device__ __forceinline__ void init(long ld, int r_left, int k_left, const int32_t *, int) {
-        constexpr int SPR = ROWS / 8;          // 16-byte slots per k-row
-        constexpr int KPL = 64 / SPR;          // k-rows per wave load
+    static constexpr int SPR = ROWS / 8;          // 16-byte slots per k-row
+    static constexpr int KPL = 64 / SPR;          // k-rows per wave load
+    __device__ __forceinline__ void init(long ld, int r_left, const int32_t *, int) {
         const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
         for (int i = 0; i < ROWS / (16 * NW); ++i) {
             const int kr = (NW * i + w) * KPL + lane / SPR;
             const int pc = lane % SPR;                                        // physical 16-byte slot in the k-row
             const int c = ((((pc >> 1) ^ swz_ks(kr)) << 1) | (pc & 1));  // logical 16-byte chunk
-            off[i] = (uint32_t)(min(kr, k_left - 1) * ld * 2 + min(c * 8, r_left - 8) * 2);
+            off[i] = (uint32_t)(kr * ld * 2 + min(c * 8, r_left - 8) * 2);
         }
+    }
+    // of a stage with k_left k-rows: the last one instead of those past it
+    __device__ __forceinline__ void clamp(int k_left, long ld) {
+#pragma unroll
+        for (int i = 0; i < ROWS / (16 * NW); ++i)
+            off[i] -= (uint32_t)(max((NW * i + (int)(threadIdx.x >> 6)) * KPL + (int)(threadIdx.x & 63) / SPR - (k_left - 1), 0) * ld * 2);
     }
 };
 template <int ROWS, int NW, bool KS> struct Off;
@@ -231,57 +243,60 @@ template <int TMB, int WM, int WN, bool M_KS, bool N_KS, int TMC, int TMCW> stru
 // by a scalar base (advanced by one stage of K after a stage's last load) plus per-lane offsets that stay
 // fixed for the whole K loop.  Stages are fetched in order.
 // Of a K-contiguous m-side tile only the 64-row groups that hold live 32-row blocks (the first TMC) are fetched.
-// KT: the contraction may not be whole stages (weight gradients; row-ragged products when K is not a multiple of 32).  What is
-// left over at its end comes first, as stage 0, whose loads are clamped to what exists and of which main_loop zeroes the rest; the
-// loop then meets whole stages only.  As the last stage it had every iteration choose between two sets of offsets and ask
-// whether its stage was that one, 47 ns of a stage's 230 on 128 x 128 tiles.  us, left over last / first: weight gradients, 64
+// KT: the contraction may not be whole stages (weight gradients; row-ragged products when K is not a multiple of 32).  The loads of what is
+// left over are clamped to what exists, and main_loop zeroes the rest of its stage.  A weight gradient takes it first, as stage 0, and its loop then
+// meets whole stages only.  As the last stage it had every iteration choose between two sets of offsets and ask
+// whether its stage was that one, 47 ns of a stage's 230 on 128 x 128 tiles.  us, left over last / first: 64
 // experts of 1024 x 2048, 100 rows, 78.8 / 73.4, 200 rows 98 / 95, 500 rows 167 / 164; 16 of 1024 x 4096, 500 rows, 80.1 / 78.0;
-// 59 of 568 x 2272, 100 rows, 53.0 / 50.4; out of 128 rows, 16 experts of 1408 -> 512 by the kernel for any K, 17.3 / 15.2.
+// 59 of 568 x 2272, 100 rows, 53.0 / 50.4.  A row-ragged product takes it last, so that its sums are in the order of k whatever the
+// width: the offsets are changed once, in the iteration that issues the first of that stage's loads (first: 0.6 % of a training pass less, 19 passes of such
+// widths; loops that stop between iterations for it: no faster).
 // ONCE: no other tile reads this tile's n-side panel (the weights of an expert with a single m-tile).
 template <int TMB, int WM, int WN, bool M_KS, bool N_KS, bool KT, int TMC, bool ONCE> struct Feeder {
     typedef Tile<TMB, WM, WN> TL;
     typedef Stage<TMB, WM, WN, M_KS, TMC> SG;
     static constexpr int LM = SG::LM, L = SG::L;
-    Off<TL::M_ROWS, TL::NW, M_KS> om, cm;      // cm, cn: of stage 0
-    Off<TL::BN, TL::NW, N_KS> on, cn;
+    Off<TL::M_ROWS, TL::NW, M_KS> om;
+    Off<TL::BN, TL::NW, N_KS> on;
     const char *bm, *bn;
     long step_m, step_n;
     uint32_t lds_w;      // LDS address of ring buffer 0 + this wave's 1 KiB lane
-    int nk, left;        // stages; k of stage 0 where that is not a whole one, otherwise 0
+    int nk;
+    int left, tail;      // KT: k of the stage that is not a whole one (0: there is none), and its number (otherwise one that no stage has)
     __device__ __forceinline__ void init(const bf16_t *Mp, long ldm, int m0, int m_ext, const bf16_t *Np, long ldn, int n0,
                                          int n_ext, int k_ext, char *smem, int wave, const int32_t *src, int n_src) {
-        om.init(ldm, m_ext - m0, Q_BK, src, n_src);
-        on.init(ldn, n_ext - n0, Q_BK, nullptr, 0);
-        left = KT ? k_ext & (Q_BK - 1) : 0;
-        if constexpr (KT) {   // k past the end is clamped to the last k-row / 16-byte piece
-            cm.init(ldm, m_ext - m0, left ? left : Q_BK, src, n_src);
-            cn.init(ldn, n_ext - n0, left ? left : Q_BK, nullptr, 0);
-        }
+        om.init(ldm, m_ext - m0, src, n_src);
+        on.init(ldn, n_ext - n0, nullptr, 0);
         bm = uniform_ptr(src != nullptr ? Mp : M_KS ? Mp + m0 : Mp + (long)m0 * ldm);
         bn = uniform_ptr(N_KS ? Np + n0 : Np + (long)n0 * ldn);
         step_m = M_KS ? ldm * (Q_BK * 2) : Q_BK * 2;
         step_n = N_KS ? ldn * (Q_BK * 2) : Q_BK * 2;
         lds_w = lds_offset_of(smem) + __builtin_amdgcn_readfirstlane(wave * 1024);
         nk = (k_ext + Q_BK - 1) / Q_BK;
+        left = KT ? __builtin_amdgcn_readfirstlane(k_ext & (Q_BK - 1)) : 0;
+        tail = __builtin_amdgcn_readfirstlane(!left ? -1 : M_KS ? 0 : nk - 1);
+    }
+    // the loads are those of the stage that is not a whole one from here on
+    __device__ __forceinline__ void clamp() {
+        om.clamp(left, step_m / (Q_BK * 2));
+        on.clamp(left, step_n / (Q_BK * 2));
     }
     __device__ __forceinline__ void load(int j, uint32_t o, uint32_t dst) const {
         if (j < LM) dma16s(bm, o, dst + j * (TL::NW * 1024));
         else if constexpr (ONCE) dma16s_nt(bn, o, dst + SG::M_OPERAND + (j - LM) * (TL::NW * 1024));
         else dma16s(bn, o, dst + SG::M_OPERAND + (j - LM) * (TL::NW * 1024));
     }
-    // the loads of stage 0, into ring buffer 0
+    // weight gradients: the loads of stage 0, into ring buffer 0
     __device__ __forceinline__ void issue_first() {
-        if constexpr (!KT) return issue<0, L>(0, 0);
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_w);
+        Feeder f = *this;
         const long ahead = left ? nk - 1 : 0;         // stages before what is left over
-        bm += ahead * step_m;
-        bn += ahead * step_n;
+        f.bm += ahead * step_m;
+        f.bn += ahead * step_n;
+        if (left) f.clamp();
 #pragma unroll
-        for (int j = 0; j < L; ++j) load(j, j < LM ? cm.off[j < LM ? j : 0] : cn.off[j < LM ? 0 : j - LM], dst);
-        if (nk > 1) {
-            bm += (left ? -ahead : 1) * step_m;
-            bn += (left ? -ahead : 1) * step_n;
-        }
+        for (int j = 0; j < L; ++j) f.load(j, j < LM ? f.om.off[j < LM ? j : 0] : f.on.off[j < LM ? 0 : j - LM], dst);
+        if (!left && nk > 1) { bm += step_m; bn += step_n; }
     }
     // loads [J0, J1) of stage s (the m-side tile's loads come first) into ring buffer buf; past the last stage that one's again
     template <int J0, int J1> __device__ __forceinline__ void issue(int s, int buf) {
@@ -341,6 +356,7 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
     constexpr int AHEAD = SG::NSTAGE - 1, NP = 4;
     typedef Feeder<TMB, WM, WN, M_KS, N_KS, KT, TMC, ONCE> FD;
     constexpr int L = FD::L, LH = L / 2;      // loads per wave per stage; the halves are LH and L - LH
+    constexpr bool LAST = KT && !M_KS;        // what whole stages leave of the contraction comes last (weight gradients: first)
     const int nk = __builtin_amdgcn_readfirstlane((k_ext + Q_BK - 1) / Q_BK);
     auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -366,11 +382,17 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
     constexpr int LX = SPLIT ? LH : L;        // loads of stage AHEAD - 1 that the prologue issues
     if constexpr (!NO_LOADS) {
         static_assert(AHEAD >= 2, "the prologue issues all of stage 0");
-        fd.issue_first();
+        if constexpr (M_KS) fd.issue_first();
 #pragma unroll
-        for (int s = 1; s < AHEAD - 1; ++s)
-            if (s < nk) fd.template issue<0, L>(s, s);
-        if (AHEAD - 1 < nk) fd.template issue<0, LX>(AHEAD - 1, AHEAD - 1);
+        for (int s = M_KS ? 1 : 0; s < AHEAD - 1; ++s)
+            if (s < nk) {
+                if (LAST && s == fd.tail) fd.clamp();
+                fd.template issue<0, L>(s, s);
+            }
+        if (AHEAD - 1 < nk) {
+            if (LAST && AHEAD - 1 == fd.tail) fd.clamp();
+            fd.template issue<0, LX>(AHEAD - 1, AHEAD - 1);
+        }
     }
     if constexpr (!M_KS) clear();       // (while the loads are on their way; weight gradients are 1 % slower for it)
     // stage 0 has landed when no more is in flight than what was issued after it
@@ -388,17 +410,17 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
                 for (int j = 0; j < 4; ++j) acc[tm][c][j] = b4[j];
         }
     }
-    if constexpr (KT) {
-        if (fd.left) {       // stage 0 is what whole stages leave over
-            if constexpr (M_KS) zero_k_tail<TL::BM, TL::THREADS>(smem, fd.left);
-            else zero_kc_tail<SG::M_OPERAND / 64, TL::THREADS>(smem, fd.left);
-            if constexpr (N_KS) zero_k_tail<TL::BN, TL::THREADS>(smem + SG::M_OPERAND, fd.left);
-            else zero_kc_tail<TL::BN, TL::THREADS>(smem + SG::M_OPERAND, fd.left);
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (and not for the loads of the stages behind it)
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-        }
-    }
+    // zeroes what lies past the contraction's end in the stage that is not a whole one, which has landed in buf
+    auto zero_rest = [&](char *buf) __attribute__((always_inline)) {
+        if constexpr (M_KS) zero_k_tail<TL::BM, TL::THREADS>(buf, fd.left);
+        else zero_kc_tail<SG::M_OPERAND / 64, TL::THREADS>(buf, fd.left);
+        if constexpr (N_KS) zero_k_tail<TL::BN, TL::THREADS>(buf + SG::M_OPERAND, fd.left);
+        else zero_kc_tail<TL::BN, TL::THREADS>(buf + SG::M_OPERAND, fd.left);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (and not for loads that are in flight)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (KT && fd.tail == 0) zero_rest(smem);
     Frags<TMB, WM, WN, M_KS, N_KS, TMC, TMCW> fr;
     fr.read_first(smem, wm, wn);
     if constexpr (NO_READS) {
@@ -420,7 +442,7 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
         const int free_b = cur_b == 0 ? SG::NSTAGE - 1 : cur_b - 1;     /* held stage s-1, takes stage s+AHEAD */ \
         const int fill_b = free_b == 0 ? SG::NSTAGE - 1 : free_b - 1;   /* takes the rest of stage s+AHEAD-1 */   \
         const char *cur = smem + cur_b * SG::BYTES;                                                       \
-        const char *nxt = smem + nxt_b * SG::BYTES;                                                       \
+        char *nxt = smem + nxt_b * SG::BYTES;                                                       \
         MOLE_PART(ISSUE, 0, 0, SPLIT ? LH : 0, SPLIT ? L - LH : 0, s + AHEAD - 1, fill_b, cur)             \
         MOLE_PART(ISSUE, 0, 1, SPLIT ? LH : 0, SPLIT ? L - LH : 0, s + AHEAD - 1, fill_b, cur)             \
         MOLE_PART(ISSUE, 0, 2, SPLIT ? LH : 0, SPLIT ? L - LH : 0, s + AHEAD - 1, fill_b, cur)             \
@@ -428,6 +450,8 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
         WAIT;                                                                                             \
         if constexpr (!NO_BARRIERS) __builtin_amdgcn_s_barrier();                                         \
         __builtin_amdgcn_sched_barrier(0);                                                                \
+        if constexpr (LAST && (AHEAD < 3 || !(ISSUE))) { if (s + 1 == fd.tail) zero_rest(nxt); }  /* (the last iteration but one) */ \
+        if constexpr (LAST && (ISSUE)) { if (s + AHEAD == fd.tail) fd.clamp(); }                          \
         MOLE_PART(ISSUE, 1, 0, 0, SPLIT ? LH : L, s + AHEAD, free_b, nxt)                                  \
         MOLE_PART(ISSUE, 1, 1, 0, SPLIT ? LH : L, s + AHEAD, free_b, nxt)                                  \
         MOLE_PART(ISSUE, 1, 2, 0, SPLIT ? LH : L, s + AHEAD, free_b, nxt)                                  \
@@ -437,9 +461,9 @@ __device__ __forceinline__ void main_loop(const bf16_t *Mp, long ldm, int m0, in
     int s = 0;
     // while stage s + AHEAD - 1 exists: its rest is issued, then the first loads of stage s + AHEAD (in the last of
     // these iterations that stage does not exist: LX loads that nothing reads, the only ones of a tile)
-    for (; s + AHEAD - 1 < nk; ++s) MOLE_ITER(true, __builtin_amdgcn_s_waitcnt(waitcnt_vm((AHEAD - 2) * L)))
     // the last AHEAD - 1 iterations issue nothing; in flight behind stage s + 1: the stages after it and those LX loads
     const bool extra = nk >= AHEAD;
+    for (; s + AHEAD - 1 < nk; ++s) MOLE_ITER(true, __builtin_amdgcn_s_waitcnt(waitcnt_vm((AHEAD - 2) * L)))
     for (; s < nk; ++s) MOLE_ITER(false, (wait_stages_behind<AHEAD - 2, L, LX>(nk - 2 - s, extra)))
 #undef MOLE_ITER
 #undef MOLE_PART

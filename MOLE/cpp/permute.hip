@@ -338,7 +338,6 @@ __device__ __forceinline__ void dispatch_bwd_gate_mfma_block(const int block, co
     const int col0 = (col_block * 8 + wave) * DM_COLS;       // this wave's first column
     if (col0 >= M) return;                                   // (no barrier below)
     float *buf = s_t + wave * (16 * DM_ROW);
-    const bool rest_first = (((E + 7) & ~7) & 31) != 0;      // NH 2: the order in which mole_gemm_nn takes a contraction over E (in whole eights)
     const int tsel = lane >> 4, c8 = (lane & 15) * 8;        // row-major side: token within a quartet, first of 8 columns
     const bool col_ok = col0 + c8 < M;
     const int at = min(col0 + c8, M - 8);
@@ -479,18 +478,10 @@ __device__ __forceinline__ void dispatch_bwd_gate_mfma_block(const int block, co
 #pragma unroll
             for (int order = P - 1; order >= 0; --order)       // the smallest products first
 #pragma unroll
-                for (int p = 0; p <= order; ++p) {
-                    auto mma = [&](int h) __attribute__((always_inline)) {
+                for (int p = 0; p <= order; ++p)
+#pragma unroll
+                    for (int h = 0; h < NH; ++h)
                         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfrag[p][h][cb], afrag[order - p][h], acc, 0, 0, 0);
-                    };
-                    if constexpr (NH == 2) {
-                        if (rest_first) mma(1);
-                        mma(0);
-                        if (!rest_first) mma(1);
-                    } else {
-                        mma(0);
-                    }
-                }
             if constexpr (SPLIT) {
                 // the parts of an infinity are the infinity and NaN: where the leading product is not finite, it is the result
                 const perm_f32x4 lead = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfrag[0][0][cb], afrag[0][0], perm_f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);

@@ -133,6 +133,30 @@ def test_ffn_backward_pair_on_the_ring_of_three_stages(M):
     test_ffn_fwd_bwd_matches_oracle(32, M, 760, rows, 0, "exact", torch.bfloat16)
 
 
+# bf16 contractions that end inside a stage of 32 are summed in the order of k, those of whole stages as well: zeros behind them change no bit of h (K = M), out
+# and gx (K = F).  One stage to eight, which every depth of a ring meets before and behind its end; tiles of 128 x 128 and of 256 columns, full and light ones.
+@pytest.mark.parametrize("K", [8, 40, 72, 104, 136, 168, 200, 232])
+@pytest.mark.parametrize("rows,N", [([130, 128, 70, 255, 100, 129, 200, 90] * 2, 512), ([1030, 1000, 700, 999, 1023, 900, 801, 1280] * 2, 1024)])
+def test_ffn_zeros_behind_a_contraction_change_nothing(rows, N, K):
+    from mole_amd import hip_ops as H, _lib as L
+    print(f"zeros behind a contraction rows={sum(rows)} N={N} K={K}", flush=True)
+    E, pad = 16, -K % 32
+    def run(d, M, Fd):
+        c = {k: (v.cuda() if torch.is_tensor(v) else v) for k, v in d.items()}
+        off, n = torch.from_numpy(d["off"]).cuda(), torch.from_numpy(d["n"]).cuda()
+        out, h, a = H.ffn_fwd(c["xd"], off, n, c["w1"], c["b1"], c["w2"], c["b2"])
+        g = [torch.empty_like(c[k]) for k in ("w1", "b1", "w2", "b2")]
+        return h, out, H.ffn_bwd(c["go"], c["xd"], h, a, off, n, c["w1"], c["w2"], *g, True, False, L.GELU_BWD_TANH)
+    behind = lambda t, dim: torch.cat([t, t.new_zeros(*[pad if i == dim % t.dim() else s for i, s in enumerate(t.shape)])], dim)
+    d = _make(E, K, N, rows, torch.bfloat16, seed=K)
+    wide = dict(d, **{k: behind(d[k], -1) for k in ("xd", "w1", "w2", "b2", "go")})
+    assert torch.equal(run(d, K, N)[0], run(wide, K + pad, N)[0])
+    d = _make(E, N, K, rows, torch.bfloat16, seed=K + 1)
+    wide = dict(d, w1=behind(d["w1"], 1), w2=behind(d["w2"], 1), b1=behind(d["b1"], 1))
+    for got, want in zip(run(d, N, K)[1:], run(wide, N, K + pad)[1:]):
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_gemm_nt_gate_logits(dtype):
     from mole_amd import hip_ops as H
